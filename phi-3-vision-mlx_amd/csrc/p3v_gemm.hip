@@ -318,7 +318,7 @@ static int launch_gemm_v(const GemmP& p, hipStream_t s) {
 template <int EPI>
 static int launch_gemm(const GemmP& p, hipStream_t s) { return launch_gemm_v<EPI, 0>(p, s); }
 
-int p3v_gemm256_try(const p3v_gemm_args_t* a, hipStream_t s);   // p3v_gemm256.hip: 256x256 tiles, P3V_ERR_UNSUPPORTED if the shape does not fit
+int p3v_gemm256_try(const p3v_gemm_args_t* a, int mb, int nb, hipStream_t s);   // p3v_gemm256.hip: tiles of 32 mb x 64 nb, P3V_ERR_UNSUPPORTED if the shape does not fit
 static int gemm128(const p3v_gemm_args_t* a, hipStream_t s);
 
 // How many leading rows go to the 256x256 kernel (a multiple of 256, or M for all of them); the rest runs on the
@@ -347,6 +347,41 @@ static int gemm_big_rows(const p3v_gemm_args_t* a) {
     if (c < best - 1e-4f) { best = c; best_rows = rows_big; }
   }
   return best_rows;
+}
+
+// Which tile runs the whole problem in one launch (*mb, *nb: a tile of 32 mb x 64 nb), or false: the packing above (or 128 x 128 tiles).
+// A launch lasts whole rounds of the chip's workgroups, so what counts is how a tile height divides the rows: 2531 x 3072 is 120
+// tiles of 256 x 256 (half the chip idle) but 240 of 128 x 256.  Times of one round in us, K-tiles of 64 = t, fitted to M = 1100 .. 9809 x
+// the decoder's and the vision tower's projections (every choice within 4 % of the best tile there): the flat tiles of
+// p3v_gemm_pc.hip 6.6 + 0.69 t (128 x 256), 7.9 + 0.79 t (160 x 256), 5.5 + 0.61 t (128 x 192); the tall ones of p3v_gemm256.hip
+// 9.5 + 1.28 t (256 x 256), 8.2 + 1.20 t (224 x 256), 8.1 + 1.11 t (256 x 192), a twentieth more per K-tile from the second round on (power);
+// 512 tiles of 128 x 128 6.0 + 0.785 t, up to 256 of them 4.4 + 0.635 t.  A tile has to promise 5 %; short K loops (< 1024) stay.
+// Measured (us, before -> now): 2531 x 3072 x 8192 117 -> 105, 2048 x 9472 x 3072 114 -> 97, 9809 x 1024 x 4096 (+ fp32 residual) 95 -> 73,
+// 4096 x 3072 x 8192 174 -> 163, 640 x 16384 x 3072 (gate | up) 103 -> 58.
+static bool gemm_tile_plan(const p3v_gemm_args_t* a, int rows_big, int* mb, int* nb) {
+  const bool gated = P3V_GATED(a->epilogue);
+  if (a->M <= 256 || a->K < 1024 || a->epilogue == P3V_EPI_PATCH || p3v_tuning().gemm_128 || p3v_tuning().gemm_big_rows >= 0) return false;
+  struct Tile { int mb, nb; float f, c, more; };
+  static const Tile tiles[] = {{8, 4, 9.5f, 1.285f, 0.07f}, {7, 4, 8.2f, 1.20f, 0.03f}, {8, 3, 8.1f, 1.106f, 0.f},
+                               {5, 4, 7.9f, 0.79f, 0.05f},  {4, 4, 6.6f, 0.69f, 0.05f}, {4, 3, 5.5f, 0.61f, 0.f}};
+  const float kt = (float)(a->K / BK);
+  auto time = [&](const Tile& t, int M) {
+    const int rounds = p3v_cdiv((long)p3v_cdiv(M, 32 * t.mb) * (a->N / (gated ? 32 * t.nb : 64 * t.nb)), 256);
+    return rounds * (t.f + t.c * kt) + (rounds > 1 ? (rounds - 1) * t.more * kt : 0.f);
+  };
+  float best = rows_big ? time(tiles[0], rows_big) : 0.f;
+  if (rows_big < a->M) {
+    const long small = (long)p3v_cdiv(a->M - rows_big, BM) * p3v_cdiv(a->N, gated ? BN / 2 : BN), rest = small % 512;
+    best += (small / 512 + (rest > 256)) * (6.0f + 0.785f * kt) + (rest > 0 && rest <= 256 ? 4.4f + 0.635f * kt : 0.f) + (rows_big ? 3.8f : 0.f);
+  }
+  best *= 0.95f;
+  bool found = false;
+  for (const Tile& t : tiles) {
+    if (a->N % (gated ? 32 * t.nb : 64 * t.nb) || (gated && t.nb != 4)) continue;
+    const float c = time(t, a->M);
+    if (c < best) { best = c; *mb = t.mb; *nb = t.nb; found = true; }
+  }
+  return found;
 }
 
 // ---- split-K for prompt-sized-but-small M (17 .. 256 rows: short chat prompts, the text group of a mixed batch).  One
@@ -547,6 +582,7 @@ extern "C" int p3v_gemm(const p3v_gemm_args_t* a, void* stream) {
     if ((size_t)a->M * a->lda * 2 >= (1ull << 32) || w_rows * a->ldw * 2 >= (1ull << 32)) return P3V_ERR_UNSUPPORTED;
   }
   hipStream_t s = (hipStream_t)stream;
+  if (const int t = p3v_tuning().gemm_tile; t > 0) return p3v_gemm256_try(a, t / 10, t % 10, s);
   if (!a->bias) {                                              // 17 .. 256 rows: the weight-streaming kernel (p3v_gemm_skinny.hip)
     const int rc = p3v_gemm_skinny_try(a, s);
     if (rc != P3V_ERR_UNSUPPORTED) return rc;
@@ -557,10 +593,14 @@ extern "C" int p3v_gemm(const p3v_gemm_args_t* a, void* stream) {
   }
   const bool big_tiles = !p3v_tuning().gemm_128;
   const int rows_big = big_tiles ? gemm_big_rows(a) : 0;
+  if (int mb, nb; gemm_tile_plan(a, rows_big, &mb, &nb)) {
+    const int rc = p3v_gemm256_try(a, mb, nb, s);
+    if (rc != P3V_ERR_UNSUPPORTED) return rc;
+  }
   if (rows_big > 0) {
     p3v_gemm_args_t top = *a;
     top.M = rows_big;
-    const int rc = p3v_gemm256_try(&top, s);
+    const int rc = p3v_gemm256_try(&top, 8, 4, s);
     if (rc == P3V_OK && rows_big < a->M) {
       const bool f32_out = a->epilogue == P3V_EPI_BIAS_RESID_F32 || a->epilogue == P3V_EPI_F32 || a->epilogue == P3V_EPI_SCALE_RESID_F32;
       const size_t out_row = (size_t)a->ldo * (f32_out ? 4 : 2);

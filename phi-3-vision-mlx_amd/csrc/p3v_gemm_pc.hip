@@ -1,0 +1,208 @@
+// Flat-tile variant of the dense projection for prefill-sized problems (p3v_gemm's tile plan decides): 128 x 256, 160 x 256 or 128 x 192
+// outputs x 64 of K, for the shapes whose 256 x 256 tiles leave a round of the chip half empty.
+//   waves    12: eight CONSUMERS as 2(M) x 4(N), each 64 .. 80 x 48 .. 64 outputs, and four PRODUCERS (one per SIMD) that only issue the
+//            LDS-DMA and wait for it.  A K-tile of a flat tile has half the MFMAs of a 256 x 256 one but three quarters of its bytes: with
+//            the MFMA waves issuing the DMA themselves (p3v_gemm256.hip's form) a 128 x 256 K-tile takes 1.14 us with two LDS buffers and
+//            0.85 with three, most of it DMA issue in front of the MFMAs; here 0.81 (0.65 with 192 workgroups).
+//   staging  S = 3 (128 x 192: 4) LDS buffers; one barrier per K-tile, in the middle of it: the fragments of one 32-wide half are
+//            multiplied while those of the other are read, so a K-tile's buffer is free, and refilled, half a K-tile before its last MFMA.
+//   bound    the LDS-DMA: 88 - 98 KB/us and CU in pieces of 8 rows x 128 B, i.e. 0.5 us for the 48 KB of a 128 x 256 K-tile against 0.45 of
+//            MFMAs; larger tiles do not fit the 168 registers that twelve waves leave each other.
+// 2531 x 3072 x 8192 (+ residual) 117 -> 105 us (1.21 PFLOP/s), 9809 x 1024 x 4096 (+ fp32 residual) 95 -> 73, 2048 x 9472 x 3072 114 -> 97.
+// Same K order and epilogue as the other tiles: bit-identical results.
+// (Tried and left out: touching the lines of later K-tiles ahead of the DMA, one dword per line -- 64 lines cost the address path as
+//  much as four pieces: 105 -> 137 us; 4 consumers of twice the size without producers: 121 us.)
+#include "p3v_gemm256_epi.h"
+
+struct TilePc {                        // where the requests of an output tile's K-tiles come from
+  int a_off[8], b_off[8]; __amdgpu_buffer_rsrc_t rs_a;
+};
+
+#define GPC_BUF(mb, nb) ((32 * (mb) + 64 * (nb)) * TK * 2)
+#define GPC_STAGES(mb, nb) (160 * 1024 / GPC_BUF(mb, nb) < 4 ? 160 * 1024 / GPC_BUF(mb, nb) : 4)
+
+// MB, NB: 16-row / 16-column blocks of a consumer wave (2 x 4 waves: a tile of 32 MB rows x 64 NB columns)
+template <int EPI, int MB, int NB>
+__global__ void __launch_bounds__(768, 1) k_gemm_pc(Gemm256P p) {
+  constexpr bool SILU = P3V_GATED(EPI);
+  static_assert(NB == 4 || (NB == 3 && !SILU), "");
+  constexpr int TM = 32 * MB, TN = 64 * NB, A_BYTES = TM * TK * 2, BUF_BYTES = A_BYTES + TN * TK * 2;
+  constexpr int S = GPC_STAGES(MB, NB), PER = MB + 2 * NB;        // LDS buffers; requests of a producer wave per K-tile
+  static_assert(S >= 3 && (S - 1) * PER < 64, "");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform: LDS-DMA bases stay in SGPRs
+  constexpr int n_out_tile = SILU ? TN / 2 : TN;
+  const int gx = (p.N + n_out_tile - 1) / n_out_tile, gy = (p.M + TM - 1) / TM, nwg = gx * gy;
+  const int nk = p.K / TK;
+
+  // ---- PERSISTENT over output tiles: workgroup b takes tiles b, b + G, b + 2G, ... (G = gridDim.x, a multiple of 8, so a
+  // workgroup's tiles keep its XCD in the XCD-aware order below), one stream of K-tiles across all of them.
+  auto place = [&](int wid, int& m0, int& n0) {
+    const int q = nwg >> 3, r = nwg & 7, xcd = wid & 7, loc = wid >> 3;
+    const int id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + loc;
+    constexpr int BAND = 4;
+    const int band = id / (BAND * gx), in_band = id % (BAND * gx);
+    const int rows = min(BAND, gy - band * BAND);
+    m0 = (band * BAND + in_band % rows) * TM, n0 = in_band / rows * n_out_tile;
+  };
+  if ((int)blockIdx.x >= nwg) return;
+  const int n_mine = (nwg - 1 - (int)blockIdx.x) / (int)gridDim.x + 1, total = n_mine * nk;      // output tiles, K-tiles of this workgroup
+
+  if (wave >= 8) {
+    // ---- PRODUCERS.  A request = 8 tile rows x 128 B (1 KiB) by LDS-DMA; the 16-byte chunks of a row are swizzled on the source side.
+    // Buffer addressing (SGPR descriptor + 32-bit per-lane byte offset + SGPR K offset): no vector ALU work at all.
+    const int pw = wave - 8, srow = pw * 8 + (lane >> 3), sw = ((lane & 7) ^ (lane >> 3)) * 8;
+    const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, 0xffffffff, 0x00020000);
+    TilePc dt;   // (declared outside the template: a builtin called with a member of a DEPENDENT type is only checked at
+                  //  instantiation, fails there in the HOST pass -- no such builtin -- and hipcc silently drops the host stub)
+    auto aim = [&](int wid) {
+      int m0, n0;
+      place(wid, m0, n0);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int rr = q * 32 + srow;
+        int br = n0 + rr;
+        if (SILU)                                     // a group of 64 tile columns = 32 gate rows + the 32 up rows of the same outputs
+          br = min(n0 + (rr >> 6) * 32 + ((rr >> 4) & 1) * 16 + (rr & 15), p.N - 1) + ((rr & 63) >> 5) * p.N;
+        else
+          br = min(br, p.N - 1);
+        dt.a_off[q] = ((min(m0 + rr, p.M - 1) - m0) * p.lda + sw) * 2;
+        dt.b_off[q] = (int)(((unsigned)br * (unsigned)p.ldw + (unsigned)sw) * 2u);   // < 2^32: checked by the launcher
+      }
+      dt.rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + (size_t)m0 * p.lda), 0, 0xffffffff, 0x00020000);
+    };
+    int dwid = blockIdx.x, dk = 0, slot = 0;                      // the next K-tile to request, and its buffer
+    aim(dwid);
+    auto request = [&]() {
+      unsigned char* base = smem + slot * (int)BUF_BYTES + pw * 1024;
+      const int na = MB, nb = 2 * NB, a_bytes = A_BYTES;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        if (q < na) {
+          lptr_t dst = (lptr_t)(base + q * 4096);
+          const int vo = dt.a_off[q];
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(dt.rs_a, dst, 16, vo, dk * (TK * 2), 0, 0);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        if (q < nb) {
+          lptr_t dst = (lptr_t)(base + a_bytes + q * 4096);
+          const int vo = dt.b_off[q];
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, dst, 16, vo, dk * (TK * 2), 0, 0);
+        }
+      }
+      slot = slot == S - 1 ? 0 : slot + 1;
+      if (++dk == nk) {
+        dk = 0;
+        dwid += gridDim.x;
+        if (dwid < nwg) aim(dwid);
+      }
+    };
+    for (int g = 0; g < min(S, total); ++g) request();
+    for (int g = 0; g < total; ++g) {
+      // K-tile g has landed when only the younger ones' requests are out: S - 1 of them at first, then S - 2, fewer at the end
+      const int young = min(g == 0 ? S - 1 : S - 2, total - 1 - g);
+      if (young >= 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S > 3 ? 3 : 0) * PER) : "memory");
+      else if (young == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER) : "memory");
+      else if (young == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();                               // K-tile g is there; K-tile g - 1 is in the consumers' registers
+      if (g > 0 && g - 1 + S < total) request();
+    }
+    return;
+  }
+
+  // ---- CONSUMERS: the fragments of one 32-wide half of a K-tile are multiplied while those of the next are fetched
+  const int wr = wave >> 2, wc = wave & 3;
+  const int frow = lane & 15, fchunk = lane >> 4;
+  const int fo0 = frow * 128 + ((fchunk ^ (frow & 7)) << 4), fo1 = frow * 128 + (((4 + fchunk) ^ (frow & 7)) << 4);
+  f32x4_t acc[MB][NB];
+  bf16x8_t fa[2][MB], fb[2][NB];                                  // the fragments of the two halves
+  auto fetch = [&](int n, int kk, int buf) {                      // fragment n: the columns' first, then the rows' (the MFMAs walk row by row)
+    const unsigned char* t = smem + buf * BUF_BYTES + (kk ? fo1 : fo0);
+    if (n < NB) fb[kk][n] = *(const bf16x8_t*)(t + A_BYTES + (wc * NB + n) * 2048);
+    else fa[kk][n - NB] = *(const bf16x8_t*)(t + (wr * MB + n - NB) * 2048);
+  };
+  auto half = [&](int kk, bool fetches, int fbuf) {               // all MFMAs of one half, between them (early) the fetches of the other
+    constexpr int C = (MB * NB + 3) / 4;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      if (2 * c < C && (kk == 0 || fetches)) {
+#pragma unroll
+        for (int n = 0; n < MB + NB; ++n)
+          if (n >= 2 * (MB + NB) * c / C && n < 2 * (MB + NB) * (c + 1) / C) fetch(n, kk ^ 1, fbuf);
+      }
+#pragma unroll
+      for (int m = 4 * c; m < 4 * c + 4 && m < MB * NB; ++m)
+        acc[m / NB][m % NB] =                                    // (W fragment first: the block comes out TRANSPOSED, see the epilogue)
+            __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[kk][m % NB], fa[kk][m / NB], acc[m / NB][m % NB], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  int slot = 0;                                                   // LDS buffer of the K-tile in hand
+  __builtin_amdgcn_s_barrier();
+  for (int wid = blockIdx.x; wid < nwg; wid += gridDim.x) {
+    int m0, n0;
+    place(wid, m0, n0);
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int n = 0; n < MB + NB; ++n) fetch(n, 0, slot);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+    for (int kt = 0; kt < nk; ++kt) {
+      const int nslot = slot == S - 1 ? 0 : slot + 1;
+      const bool last = kt + 1 == nk;                              // (nothing is fetched behind a tile's last K-tile: the epilogue needs the registers)
+      half(0, true, slot);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");           // the K-tile in hand is in registers: its buffer is given back
+      if (!last || wid + (int)gridDim.x < nwg) __builtin_amdgcn_s_barrier();
+      half(1, !last, nslot);
+      slot = nslot;
+    }
+    gemm256_epilogue<EPI, MB, NB>(p, acc, m0 + wr * MB * 16, n0 + wc * (n_out_tile / 4), lane);   // straight from the accumulators: p3v_gemm256_epi.h
+  }
+}
+
+int p3v_gemm256_cus();                                             // p3v_gemm256.hip
+
+template <int EPI, int MB, int NB>
+static int launch_pc_v(const Gemm256P& p, hipStream_t s) {
+  constexpr int LDS = GPC_STAGES(MB, NB) * GPC_BUF(MB, NB);
+  static bool attr_set = false;
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)k_gemm_pc<EPI, MB, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return P3V_ERR_HIP;
+    attr_set = true;
+  }
+  const int n_cu = p3v_gemm256_cus();
+  if (!n_cu) return P3V_ERR_HIP;
+  const int tiles = p3v_cdiv(p.N, P3V_GATED(EPI) ? 32 * NB : 64 * NB) * p3v_cdiv(p.M, 32 * MB);
+  hipLaunchKernelGGL((k_gemm_pc<EPI, MB, NB>), dim3(min(tiles, n_cu)), dim3(768), LDS, s, p);
+  P3V_CHECK_LAUNCH();
+  return P3V_OK;
+}
+
+template <int EPI>
+static int launch_pc(const Gemm256P& p, int mb, int nb, hipStream_t s) {
+  if constexpr (!P3V_GATED(EPI))
+    if (nb == 3) return launch_pc_v<EPI, 4, 3>(p, s);
+  return mb == 4 ? launch_pc_v<EPI, 4, 4>(p, s) : launch_pc_v<EPI, 5, 4>(p, s);
+}
+
+int p3v_gemm_pc(const Gemm256P& p, int epi, int mb, int nb, hipStream_t s) {
+  switch (epi) {
+    case P3V_EPI_NONE: return launch_pc<P3V_EPI_NONE>(p, mb, nb, s);
+    case P3V_EPI_BIAS: return launch_pc<P3V_EPI_BIAS>(p, mb, nb, s);
+    case P3V_EPI_BIAS_QGELU: return launch_pc<P3V_EPI_BIAS_QGELU>(p, mb, nb, s);
+    case P3V_EPI_BIAS_GELU: return launch_pc<P3V_EPI_BIAS_GELU>(p, mb, nb, s);
+    case P3V_EPI_BIAS_RESID_F32: return launch_pc<P3V_EPI_BIAS_RESID_F32>(p, mb, nb, s);
+    case P3V_EPI_RESID_BF16: return launch_pc<P3V_EPI_RESID_BF16>(p, mb, nb, s);
+    case P3V_EPI_SILU_MUL: return launch_pc<P3V_EPI_SILU_MUL>(p, mb, nb, s);
+    case P3V_EPI_GELU_MUL: return launch_pc<P3V_EPI_GELU_MUL>(p, mb, nb, s);
+    case P3V_EPI_F32: return launch_pc<P3V_EPI_F32>(p, mb, nb, s);
+    case P3V_EPI_SCALE_RESID_F32: return launch_pc<P3V_EPI_SCALE_RESID_F32>(p, mb, nb, s);
+    default: return P3V_ERR_UNSUPPORTED;
+  }
+}

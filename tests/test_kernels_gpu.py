@@ -817,6 +817,30 @@ def test_merge_launch_with_fused_oproj_under_grouped_queries(ops):
     test_merge_launch_with_fused_oproj_is_bit_identical_to_three_launches(ops, 300, 384, 3, False, True, nkv=8)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 768, 64), (129, 768, 128), (257, 3072, 1024), (1111, 768, 192), (4001, 3072, 128), (2300, 9216, 64)])
+@pytest.mark.parametrize("epi", ["none", "silu", "gelu", "resid_bf16", "resid_f32", "scale"])
+def test_gemm_tiles_agree(ops, epi, M, N, K):
+    """Every tile of the large GEMM kernels (one and several rounds of the chip, fewer K-tiles than LDS buffers, ragged last rows) against
+    the 128 x 128 tiles: the same products in the same order, bit for bit."""
+    gated = epi in ("silu", "gelu")
+    a, w = g((M, K), 40).cuda(), g((2 * N if gated else N, K), 41, 1.0 / math.sqrt(K)).cuda()
+    v, r = g((N,), 42, 0.5).cuda(), g((M, N), 43, 1.0, BF16 if epi == "resid_bf16" else F32).cuda()
+    kw = {"none": {}, "silu": dict(epilogue=ops.EPI_SILU_MUL), "gelu": dict(epilogue=ops.EPI_GELU_MUL), "resid_bf16": dict(epilogue=ops.EPI_RESID_BF16, resid=r),
+          "resid_f32": dict(epilogue=ops.EPI_BIAS_RESID_F32, resid=r, bias=v), "scale": dict(epilogue=ops.EPI_SCALE_RESID_F32, resid=r, col_scale=v)}[epi]
+    names = ("gemm_tile", "gemm_128", "gemm_no_skinny", "gemm_no_splitk")
+    saved = [ops.set_tuning(n, x) for n, x in zip(names, (-1, 1, 1, 1))]
+    try:
+        want = ops.gemm(a, w, **kw)
+        for tile in (84, 74, 83, 54, 44, 43):
+            if tile % 10 == 3 and gated:
+                continue
+            ops.set_tuning("gemm_tile", tile)
+            assert torch.equal(ops.gemm(a, w, **kw), want), f"tile {tile}"
+    finally:
+        for n, x in zip(names, saved):
+            ops.set_tuning(n, x)
+
+
 @pytest.mark.parametrize("B,L,nh,nkv,hd,K,past,rot,bias,big", [
     (1, 2531, 32, 32, 96, 256, 0, True, False, -1),      # the bench prompt's shape (short K): big tiles + remainder rows, ragged end
     (1, 2531, 32, 32, 96, 256, 0, True, False, 1000000),  # all rows on the 256 x 256 kernel
