@@ -1,4 +1,4 @@
-// BASELINE config 5, prefill: W8A8 projection on the gfx950 fp8 matrix cores.
+// Prompts of the fp8 weight format: W8A8 projection on the gfx950 fp8 matrix cores.
 //
 //   C[M,N] = (sa[m] * sw[n]) * sum_k A8[m,k] * W8[n,k]        A8, W8 = OCP e4m3 bytes, K contiguous
 //
@@ -11,23 +11,24 @@
 //             twice the bf16 rate on this chip (the unscaled 16x16x32 fp8 MFMA runs at the bf16 rate).  A lane holds 32
 //             k bytes of its row (lane & 15) for k-block lane >> 4 -- the SAME bytes for A and B, so which k they are
 //             does not matter (the kernel takes 16-byte chunks fchunk and fchunk + 4: bank-conflict-free reads).
-//   tile      256(M) x 256(N) x 128(K) per K step, 512 threads = 8 waves as 2(M) x 4(N), wave tile 128 x 64 = 8 x 4
-//             accumulators; ONE MFMA per accumulator and K step.  The LDS image is the bf16 kernel's (p3v_gemm256.hip):
-//             rows of 128 BYTES, 16-byte chunk c of row r stored at chunk c ^ (r & 7), staged by LDS-DMA with the swizzle
-//             on the source address, two 64-KiB buffers, half-tiles of K-step t+1 requested in the first two phases of t.
-//             Same bytes per K step as the bf16 kernel, twice the k: the step costs the same, the flops double.
-//   epilogue  scales, then none / residual add / SiLU(gate) * up, bf16 out (wave-private LDS tile -> 16-byte stores).
+//   tile      128 or 160(M) x 256 / 192 / 128(N) x 128(K), chosen by how the tiles fill the chip's rounds (f8_tile_plan).  768
+//             threads: 8 CONSUMER waves as 2(M) x 4(N), ONE MFMA per 16 x 16 block and K-tile, and 4 PRODUCER waves that only
+//             request K-tiles by LDS-DMA (as p3v_gemm_pc.hip): rows of 128 BYTES, 16-byte chunk c of row r stored at chunk
+//             c ^ (r & 7), swizzled on the source address; three buffers of a K-tile (four from 128 x 192 down: what 160 KiB
+//             hold), so a request has two or three K-tiles' time to land.
+//             What bounds it: the producers' requests, ~60 ns per round of four 1-KiB pieces (a K-tile of 128 x 256 takes 0.69 us
+//             where its MFMAs take 0.43), and, with all CUs at it, the chip's power: the same launches on all-zero operands are
+//             20-25 % faster.  Against the form it replaced (256-row tiles, eight waves that request and multiply, two buffers and a
+//             full wait per K-tile, one tile per workgroup, outputs staged through LDS), us at M = 2531 / 1024 / 256:
+//               gate_up 131 / 51 / 44 -> 112 / 50 / 18    qkv 79 / 52 / 26 -> 64 / 30 / 16 (K = 3072)
+//               o 29.2 / 27.7 / 25.5 -> 28.2 / 17.4 / 15.4   down 63 / 58 / 57 -> 56 / 32 / 30 (K = 8192)
+//             2.2-2.4 PFLOP/s from 2500 rows on.
+//   epilogue  scales, then none / residual add / SiLU(gate) * up, bf16 out, straight from the accumulators (p3v_gemm256_epi.h).
 #include <stdlib.h>
 
 #include "p3v_common.h"
 
-#define TM 256
-#define TN 256
-#define TKB 128                        // K bytes (= fp8 elements) per step
-#define HALF_BYTES (128 * TKB)         // 16 KiB: 128 rows x 128 B
-#define BUF_BYTES (4 * HALF_BYTES)     // A0 A1 B0 B1
-#define CT_LD 68
-#define GEMMF8_LDS (2 * BUF_BYTES)     // 128 KiB
+#define TKB 128                        // K bytes (= fp8 elements) per K-tile
 
 typedef __attribute__((address_space(3))) void* lptr_t;
 typedef __attribute__((ext_vector_type(8))) int i32x8_t;
@@ -37,259 +38,275 @@ struct GemmF8P {
   int M, N, K, lda, ldw, ldo;
 };
 
-// NJ = 16-column blocks per wave: 4 -> 256 x 256 tile; 2 -> 256 x 128 tile (one B half-tile, 96 KiB of LDS in use): the
-// N = 3072 projections (o_proj, down_proj) have only 120 tiles of 256 x 256 for 256 CUs -- 240 narrower tiles fill the chip.
-template <int EPI, int NJ = 4>
-__global__ void __launch_bounds__(512, 1) k_gemm256_f8(GemmF8P p) {
+struct TileF8 { int a_off[8], b_off[8]; __amdgpu_buffer_rsrc_t rs_a; };   // where the requests of an output tile's K-tiles come from
+
+#define F8_BUF(mb, nb) ((32 * (mb) + 64 * (nb)) * TKB)
+#define F8_STAGES(mb, nb) (160 * 1024 / F8_BUF(mb, nb) < 4 ? 160 * 1024 / F8_BUF(mb, nb) : 4)
+
+// MB, NB: 16-row / 16-column blocks of a consumer wave (2 x 4 waves: a tile of 32 MB rows x 64 NB columns)
+template <int EPI, int MB, int NB>
+__global__ void __launch_bounds__(768, 1) k_gemm_f8(GemmF8P p) {
   constexpr bool SILU = EPI == P3V_EPI_SILU_MUL;
-  static_assert(NJ == 4 || (NJ == 2 && !SILU), "narrow tiles: plain epilogues only");
-  constexpr int TNW = NJ * 64;                       // tile width in W rows
+  static_assert(NB % 2 == 0 || !SILU, "a wave's column blocks: gate, then up of the same outputs");
+  constexpr int HB = SILU ? NB / 2 : NB;                           // column blocks of outputs of a wave
+  constexpr int TM = 32 * MB, TN = 64 * NB, A_BYTES = TM * TKB, BUF_BYTES = F8_BUF(MB, NB);
+  constexpr int S = F8_STAGES(MB, NB), PER = MB + 2 * NB;          // LDS buffers; requests of a producer wave per K-tile
+  static_assert(S >= 3 && (S - 1) * PER < 64, "");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wr = wave >> 2, wc = wave & 3;
-  constexpr int n_out_tile = SILU ? TNW / 2 : TNW;
-  int m_t, n_t;
-  {   // XCD-aware tile order (as p3v_gemm256.hip): each XCD gets a contiguous run of tiles, bands of 4 M tiles
-    const int gx = gridDim.x, gy = gridDim.y, nwg = gx * gy, wid = blockIdx.y * gx + blockIdx.x;
+  constexpr int n_out_tile = SILU ? TN / 2 : TN;
+  const int gx = p.N / n_out_tile, gy = (p.M + TM - 1) / TM, nwg = gx * gy;
+  const int nk = p.K / TKB;
+
+  // persistent over output tiles, XCD-aware order (as p3v_gemm_pc.hip): each XCD gets a contiguous run of tiles, bands of 4 M tiles
+  auto place = [&](int wid, int& m0, int& n0) {
     const int q = nwg >> 3, r = nwg & 7, xcd = wid & 7, loc = wid >> 3;
     const int id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + loc;
     constexpr int BAND = 4;
     const int band = id / (BAND * gx), in_band = id % (BAND * gx);
     const int rows = min(BAND, gy - band * BAND);
-    m_t = band * BAND + in_band % rows;
-    n_t = in_band / rows;
-  }
-  const int m0 = m_t * TM, n0 = n_t * n_out_tile;
-
-  const int srow = tid >> 3, schunk = tid & 7;
-  int a_off[2][2], b_off[2][2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int r = h * 128 + q * 64 + srow;
-      const int sw = (schunk ^ (r & 7)) * 16;
-      const int ar = min(m0 + r, p.M - 1) - m0;
-      a_off[h][q] = ar * p.lda + sw;
-      int br;
-      if (SILU) {                                   // wave column group wcol (64 tile rows) = 32 gate + 32 up rows
-        const int wcol = r >> 6, ni = (r & 63) >> 4, c = r & 15;
-        br = min(n0 + wcol * 32 + (ni & 1) * 16 + c, p.N - 1) + (ni >> 1) * p.N;
-      } else {
-        br = min(n0 + r, p.N - 1);
-      }
-      b_off[h][q] = (int)((unsigned)br * (unsigned)p.ldw + (unsigned)sw);
-    }
-  const __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + (size_t)m0 * p.lda), 0, 0xffffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, 0xffffffff, 0x00020000);
-  auto dma_half = [&](int which, int kt, int buf) {   // which: 0 A0, 1 A1, 2 B0, 3 B1
-    unsigned char* base = smem + buf * BUF_BYTES + which * HALF_BYTES + wave * 1024;
-    const int h = which & 1;
-#pragma unroll
-    for (int q = 0; q < 2; ++q)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(which < 2 ? rs_a : rs_w, (lptr_t)(base + q * 8192), 16,
-                                               which < 2 ? a_off[h][q] : b_off[h][q], kt * TKB, 0, 0);
+    m0 = (band * BAND + in_band % rows) * TM, n0 = in_band / rows * n_out_tile;
   };
+  if ((int)blockIdx.x >= nwg) return;
+  const int n_mine = (nwg - 1 - (int)blockIdx.x) / (int)gridDim.x + 1, total = n_mine * nk;      // output tiles, K-tiles of this workgroup
 
-  f32x4_t acc[8][NJ];
+  if (wave >= 8) {
+    // ---- PRODUCERS (p3v_gemm_pc.hip)
+    const int pw = wave - 8, srow = pw * 8 + (lane >> 3), sw = ((lane & 7) ^ (lane >> 3)) * 16;
+    const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, 0xffffffff, 0x00020000);
+    TileF8 dt;    // (declared outside the template: a builtin called with a member of a DEPENDENT type is only checked at
+                  //  instantiation, fails there in the HOST pass -- no such builtin -- and hipcc silently drops the host stub)
+    auto aim = [&](int wid) {
+      int m0, n0;
+      place(wid, m0, n0);
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-
-  const int frow = lane & 15, fchunk = lane >> 4;
-  const int nk = p.K / TKB;
-#pragma unroll
-  for (int w4 = 0; w4 < (NJ == 4 ? 4 : 3); ++w4) dma_half(w4, 0, 0);
-
-  for (int kt = 0; kt < nk; ++kt) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    const bool more = kt + 1 < nk;
-    const int nb = (kt + 1) & 1;
-    const unsigned char* ta = smem + (kt & 1) * BUF_BYTES + wr * HALF_BYTES;
-    const unsigned char* tb = smem + (kt & 1) * BUF_BYTES + (2 + (wc >> 1)) * HALF_BYTES + (wc & 1) * 64 * 128;
-    if (NJ == 2) tb = smem + (kt & 1) * BUF_BYTES + 2 * HALF_BYTES + wc * 32 * 128;                   // 32 B rows per wave
-    u32x4_t af[4][2], af1[4][2], bf0[2][2], bf1[2][2];
-    // lane (row frow, k-block fchunk) owns the 16-byte chunks fchunk and fchunk + 4 of its 128-byte row (A and B alike, so the
-    // k permutation cancels).  Contiguous chunks 2*fchunk, 2*fchunk + 1 -- the obvious choice -- put the 16 lanes of a
-    // ds_read_b128 group on 8 bank slots, two-way conflicts on every fragment read (PMC: SQ_LDS_BANK_CONFLICT 48 % of the
-    // LDS-active cycles); with chunks (kk * 4 + fchunk) the group covers all 16 slots, as in the bf16 kernel
-    auto read_a_to = [&](int sub, u32x4_t (&dst)[4][2]) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          const int r = sub * 64 + i * 16 + frow;
-          dst[i][kk] = *(const u32x4_t*)(ta + r * 128 + (((fchunk + 4 * kk) ^ (r & 7)) << 4));
+      for (int q = 0; q < 8; ++q) {
+        const int rr = q * 32 + srow;
+        int br = min(n0 + rr, p.N - 1);
+        if (SILU) {                                               // a wave's 16 HB gate rows + the 16 HB up rows of the same outputs
+          const int in = rr % (NB * 16);
+          br = n0 + rr / (NB * 16) * (HB * 16) + in % (HB * 16) + in / (HB * 16) * p.N;
         }
+        dt.a_off[q] = (min(m0 + rr, p.M - 1) - m0) * p.lda + sw;
+        dt.b_off[q] = (int)((unsigned)br * (unsigned)p.ldw + (unsigned)sw);
+      }
+      dt.rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + (size_t)m0 * p.lda), 0, 0xffffffff, 0x00020000);
     };
-    auto read_b = [&](int sub, u32x4_t (&bf)[2][2]) {
+    int dwid = blockIdx.x, dk = 0, slot = 0;                      // the next K-tile to request, and its buffer
+    aim(dwid);
+    auto request = [&]() {
+      unsigned char* base = smem + slot * (int)BUF_BYTES + pw * 1024;
+      const int na = MB, nb = 2 * NB, a_bytes = A_BYTES;
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          const int r = sub * 32 + j * 16 + frow;
-          bf[j][kk] = *(const u32x4_t*)(tb + r * 128 + (((fchunk + 4 * kk) ^ (r & 7)) << 4));
+      for (int q = 0; q < 8; ++q) {
+        if (q < na) {
+          lptr_t dst = (lptr_t)(base + q * 4096);
+          const int vo = dt.a_off[q];
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(dt.rs_a, dst, 16, vo, dk * TKB, 0, 0);
         }
-    };
-    auto quad_from = [&](int asub, int bsub, u32x4_t (&a)[4][2], u32x4_t (&bf)[2][2]) {
-      __builtin_amdgcn_s_setprio(1);
+      }
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const i32x8_t av = {(int)a[i][0][0], (int)a[i][0][1], (int)a[i][0][2], (int)a[i][0][3],
-                              (int)a[i][1][0], (int)a[i][1][1], (int)a[i][1][2], (int)a[i][1][3]};
-          const i32x8_t bv = {(int)bf[j][0][0], (int)bf[j][0][1], (int)bf[j][0][2], (int)bf[j][0][3],
-                              (int)bf[j][1][0], (int)bf[j][1][1], (int)bf[j][1][2], (int)bf[j][1][3]};
-          acc[asub * 4 + i][bsub * 2 + j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-              av, bv, acc[asub * 4 + i][bsub * 2 + j], 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
+      for (int q = 0; q < 8; ++q) {
+        if (q < nb) {
+          lptr_t dst = (lptr_t)(base + a_bytes + q * 4096);
+          const int vo = dt.b_off[q];
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, dst, 16, vo, dk * TKB, 0, 0);
         }
-      __builtin_amdgcn_s_setprio(0);
-    };
-    auto dma_phase = [&](int ph) {                    // half-tiles A0 A1 in phase 0, B0 B1 in phase 1 (SCHED 0x50 of the bf16 kernel)
-      if (more) {
-        if (ph == 0) { dma_half(0, kt + 1, nb); dma_half(1, kt + 1, nb); }
-        else { dma_half(2, kt + 1, nb); if (NJ == 4) dma_half(3, kt + 1, nb); }
+      }
+      slot = slot == S - 1 ? 0 : slot + 1;
+      if (++dk == nk) {
+        dk = 0;
+        dwid += gridDim.x;
+        if (dwid < nwg) aim(dwid);
       }
     };
-    if (NJ == 4) {
-      read_b(0, bf0);
-      read_a_to(0, af);
-      dma_phase(0);
-      read_b(1, bf1);
-      __builtin_amdgcn_sched_barrier(0);
-      quad_from(0, 0, af, bf0);
-      __builtin_amdgcn_sched_barrier(0);
-      read_a_to(1, af1);
-      dma_phase(1);
-      __builtin_amdgcn_sched_barrier(0);
-      quad_from(0, 1, af, bf1);
-      __builtin_amdgcn_sched_barrier(0);
-      quad_from(1, 1, af1, bf1);
-      quad_from(1, 0, af1, bf0);
-    } else {
-      read_b(0, bf0);
-      read_a_to(0, af);
-      dma_phase(0);
-      read_a_to(1, af1);
-      dma_phase(1);
-      __builtin_amdgcn_sched_barrier(0);
-      quad_from(0, 0, af, bf0);
-      quad_from(1, 0, af1, bf0);
+    for (int g = 0; g < min(S, total); ++g) request();
+    for (int g = 0; g < total; ++g) {
+      // K-tile g has landed when only the younger ones' requests are out: S - 1 of them at first, then S - 2, fewer at the end
+      const int young = min(g == 0 ? S - 1 : S - 2, total - 1 - g);
+      if (young >= 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S > 3 ? 3 : 0) * PER) : "memory");
+      else if (young == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER) : "memory");
+      else if (young == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();                               // K-tile g is there; K-tile g - 1 is in the consumers' registers
+      if (g > 0 && g - 1 + S < total) request();
     }
+    return;
   }
 
-  // ---- epilogue: 128 x 64 per wave, four passes of 32 rows through a wave-private [32][68] fp32 LDS tile
-  __syncthreads();
-  float* ct = (float*)smem + wave * (32 * CT_LD);
-  const int ccol = lane & 15, crow = (lane >> 4) * 4;
+  // ---- CONSUMERS.  One MFMA takes a whole K-tile of a 16 x 16 block, so a K-tile is cut by rows: while the first M0 row blocks are
+  // multiplied the other M1 are fetched (then all of it is in registers and its buffer is given back), while those are multiplied
+  // column by column the next K-tile's first row blocks and, behind each column, its new fragment are.
+  constexpr int M0 = (MB + 1) / 2, M1 = MB - M0;
+  const int wr = wave >> 2, wc = wave & 3;
+  const int frow = lane & 15, fchunk = lane >> 4;
+  // lane (row frow, k-block fchunk) owns the 16-byte chunks fchunk and fchunk + 4 of its 128-byte row (A and B alike, so the k
+  // permutation cancels; contiguous chunks would put the 16 lanes of a ds_read_b128 group on 8 bank slots)
+  const int fo0 = frow * 128 + ((fchunk ^ (frow & 7)) << 4), fo1 = frow * 128 + (((4 + fchunk) ^ (frow & 7)) << 4);
+  f32x4_t acc[MB][NB];
+  i32x8_t fa[MB], fb[NB];
+  auto fetch = [&](i32x8_t& f, const unsigned char* t) {
+    const u32x4_t lo = *(const u32x4_t*)(t + fo0), hi = *(const u32x4_t*)(t + fo1);
+    f = (i32x8_t){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+  };
+  auto fetch_a = [&](int i, int buf) { fetch(fa[i], smem + buf * BUF_BYTES + (wr * MB + i) * 2048); };
+  auto fetch_b = [&](int j, int buf) { fetch(fb[j], smem + buf * BUF_BYTES + A_BYTES + (wc * NB + j) * 2048); };
+  auto mma = [&](int i, int j) {                                  // (W fragment first: the block comes out TRANSPOSED, see the epilogue)
+    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[j], fa[i], acc[i][j], 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
+  };
+  int slot = 0;                                                   // LDS buffer of the K-tile in hand
+  __builtin_amdgcn_s_barrier();
+  for (int wid = blockIdx.x; wid < nwg; wid += gridDim.x) {
+    int m0, n0;
+    place(wid, m0, n0);
 #pragma unroll
-  for (int pass = 0; pass < 4; ++pass) {
+    for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+      for (int j = 0; j < NB; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < NJ; ++j)
+    for (int i = 0; i < M0; ++i) fetch_a(i, slot);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) ct[(i * 16 + crow + r) * CT_LD + j * 16 + ccol] = acc[pass * 2 + i][j][r];
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (SILU) {
-      const int c8 = (lane & 3) * 8, n = n0 + wc * 32 + c8;
-      float sg[8], su[8];
-      if (n < p.N) {
+    for (int j = 0; j < NB; ++j) fetch_b(j, slot);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+    for (int kt = 0; kt < nk; ++kt) {
+      const int nslot = slot == S - 1 ? 0 : slot + 1;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) { sg[e] = p.sw[n + e]; su[e] = p.sw[p.N + n + e]; }
-      }
+      for (int j = 0; j < NB; ++j) {
 #pragma unroll
-      for (int it = 0; it < 2; ++it) {
-        const int row = it * 16 + (lane >> 2);
-        const int m = m0 + wr * 128 + pass * 32 + row;
-        if (m < p.M && n < p.N) {
-          const float s = p.sa[m];
-          const float4 g0 = *(const float4*)(ct + row * CT_LD + c8), g1 = *(const float4*)(ct + row * CT_LD + c8 + 4);
-          const float4 u0 = *(const float4*)(ct + row * CT_LD + 32 + c8), u1 = *(const float4*)(ct + row * CT_LD + 36 + c8);
-          const float gs[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-          const float us[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-          u32x4_t w;
+        for (int i = 0; i < M0; ++i) mma(i, j);
+        if (j == 0) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            float o2[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              // gate / up are bf16 Linear outputs, every elementwise op after them rounds to bf16 (phi.py:469-471)
-              const float g = bf16_round(gs[2 * e + h] * (s * sg[2 * e + h])), u = bf16_round(us[2 * e + h] * (s * su[2 * e + h]));
-              o2[h] = bf16_round(g * bf16_round(1.f / (1.f + __expf(-g)))) * u;
-            }
-            w[e] = pack_bf16x2(o2[0], o2[1]);
-          }
-          *(u32x4_t*)(p.out + (size_t)m * p.ldo + n) = w;
+          for (int i = 0; i < M1; ++i) fetch_a(M0 + i, slot);
         }
+        __builtin_amdgcn_sched_barrier(0);
       }
-    } else {
-      // a row of the wave tile is NJ * 16 columns = NJ * 2 lanes of 8 columns: 8 (4) rows per pass of the 64 lanes
-      constexpr int LPR = NJ * 2, RPI = 64 / LPR;
-      const int c8 = (lane % LPR) * 8, n = n0 + wc * (NJ * 16) + c8;
-      const bool ncol_ok = n < p.N;
-      float sc[8];
-      if (ncol_ok) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");           // the K-tile in hand is in registers: its buffer is given back
+      if (kt + 1 < nk || wid + (int)gridDim.x < nwg) __builtin_amdgcn_s_barrier();
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sc[e] = p.sw[n + e];
+      for (int j = 0; j < NB; ++j) {
+        if (j == 0) {
+#pragma unroll
+          for (int i = 0; i < M0; ++i) fetch_a(i, nslot);
+        }
+#pragma unroll
+        for (int i = 0; i < M1; ++i) mma(M0 + i, j);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_b(j, nslot);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      slot = nslot;
+    }
+
+    // ---- epilogue, straight from the accumulators: lane (fc = lane & 15, fq = lane >> 4) holds columns 4 fq .. 4 fq + 3 of block row fc;
+    // lanes q and q ^ 1 trade packed halves of two neighbouring column blocks: 16-byte stores (p3v_gemm256_epi.h)
+    const int fc = lane & 15, fq = lane >> 4;
+    const int mrow0 = m0 + wr * MB * 16 + fc, nw = n0 + wc * (n_out_tile / 4);
+    float sc[NB][4];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int n = SILU ? nw + j % HB * 16 + fq * 4 + j / HB * p.N : nw + j * 16 + fq * 4;
+      const float4 c = *(const float4*)(p.sw + n);
+      sc[j][0] = c.x, sc[j][1] = c.y, sc[j][2] = c.z, sc[j][3] = c.w;
+    }
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      const int m = mrow0 + i * 16;
+      const float s = p.sa[min(m, p.M - 1)];
+      uint32_t pk[HB][2];
+#pragma unroll
+      for (int j = 0; j < HB; ++j) {
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          v[r] = acc[i][j][r] * (s * sc[j][r]);
+          if (SILU) {
+            // gate / up are bf16 Linear outputs, every elementwise op after them rounds to bf16 (phi.py:469-471)
+            const float g = bf16_round(v[r]), u = bf16_round(acc[i][(HB + j) % NB][r] * (s * sc[(HB + j) % NB][r]));
+            v[r] = bf16_round(g * bf16_round(1.f / (1.f + __expf(-g)))) * u;
+          }
+        }
+        pk[j][0] = pack_bf16x2(v[0], v[1]), pk[j][1] = pack_bf16x2(v[2], v[3]);
       }
 #pragma unroll
-      for (int it = 0; it < 32 / RPI; ++it) {
-        const int row = it * RPI + lane / LPR;
-        const int m = m0 + wr * 128 + pass * 32 + row;
-        if (m < p.M && ncol_ok) {
-          const float s = p.sa[m];
-          const float4 a0 = *(const float4*)(ct + row * CT_LD + c8), a1 = *(const float4*)(ct + row * CT_LD + c8 + 4);
-          float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+      for (int jp = 0; jp < HB / 2; ++jp) {
+        u32x4_t w;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] *= s * sc[e];
+        for (int k = 0; k < 2; ++k) {
+          auto sw = __builtin_amdgcn_permlane16_swap(pk[2 * jp][k], pk[2 * jp + 1][k], false, false);
+          w[k] = sw[0], w[2 + k] = sw[1];
+        }
+        const int n = nw + (2 * jp + (fq & 1)) * 16 + (fq >> 1) * 8;
+        if (m < p.M) {
           const size_t o = (size_t)m * p.ldo + n;
           if (EPI == P3V_EPI_RESID_BF16) {
             const u32x4_t rw = *(const u32x4_t*)(p.resid + o);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) { v[2 * j] = bf16lo(rw[j]) + bf16_round(v[2 * j]); v[2 * j + 1] = bf16hi(rw[j]) + bf16_round(v[2 * j + 1]); }
+            for (int k = 0; k < 4; ++k) w[k] = pack_bf16x2(bf16lo(rw[k]) + bf16lo(w[k]), bf16hi(rw[k]) + bf16hi(w[k]));
           }
-          u32x4_t w;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) w[j] = pack_bf16x2(v[2 * j], v[2 * j + 1]);
           *(u32x4_t*)(p.out + o) = w;
         }
       }
+      if (HB & 1) {                                     // the block without a partner: four columns, 8 bytes
+        const int n = nw + (HB - 1) * 16 + fq * 4;
+        if (m < p.M) {
+          const size_t o = (size_t)m * p.ldo + n;
+          u32x2_t w = {pk[HB - 1][0], pk[HB - 1][1]};
+          if (EPI == P3V_EPI_RESID_BF16) {
+            const u32x2_t rw = *(const u32x2_t*)(p.resid + o);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) w[k] = pack_bf16x2(bf16lo(rw[k]) + bf16lo(w[k]), bf16hi(rw[k]) + bf16hi(w[k]));
+          }
+          *(u32x2_t*)(p.out + o) = w;
+        }
+      }
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
 }
 
-template <int EPI, int NJ>
-static int launch_gemm_f8_v(const GemmF8P& p, hipStream_t s) {
+int p3v_gemm256_cus();                                             // p3v_gemm256.hip
+
+template <int EPI, int MB, int NB>
+static int launch_f8_v(const GemmF8P& p, hipStream_t s) {
+  constexpr int LDS = F8_STAGES(MB, NB) * F8_BUF(MB, NB);
   static bool attr_set = false;
   if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)k_gemm256_f8<EPI, NJ>, hipFuncAttributeMaxDynamicSharedMemorySize, GEMMF8_LDS) != hipSuccess)
-      return P3V_ERR_HIP;
+    if (hipFuncSetAttribute((const void*)k_gemm_f8<EPI, MB, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return P3V_ERR_HIP;
     attr_set = true;
   }
-  const int n_tile = EPI == P3V_EPI_SILU_MUL ? TN / 2 : NJ * 64;
-  dim3 grid(p3v_cdiv(p.N, n_tile), p3v_cdiv(p.M, TM));
-  hipLaunchKernelGGL((k_gemm256_f8<EPI, NJ>), grid, dim3(512), GEMMF8_LDS, s, p);
+  const int n_cu = p3v_gemm256_cus();
+  if (!n_cu) return P3V_ERR_HIP;
+  const int tiles = p.N / (EPI == P3V_EPI_SILU_MUL ? 32 * NB : 64 * NB) * p3v_cdiv(p.M, 32 * MB);
+  hipLaunchKernelGGL((k_gemm_f8<EPI, MB, NB>), dim3(min(tiles, n_cu)), dim3(768), LDS, s, p);
   P3V_CHECK_LAUNCH();
   return P3V_OK;
 }
 
-// tile width: the wide tile unless it leaves most of the chip idle (fewer wide tiles than ~0.6 x 256 CUs, or a last round
-// that narrow tiles fill better); P3V_GEMM_F8_NARROW=0/1 pins the choice (kernel tests run both)
-template <int EPI>
-static int launch_gemm_f8(const GemmF8P& p, hipStream_t s) {
-  if constexpr (EPI == P3V_EPI_SILU_MUL) {
-    return launch_gemm_f8_v<EPI, 4>(p, s);
-  } else {
-    const long mt = p3v_cdiv(p.M, TM), wide = mt * p3v_cdiv(p.N, 256), narrow = mt * p3v_cdiv(p.N, 128);
-    bool use_narrow = p.N % 256 != 0 || wide <= 160 || (wide % 256 != 0 && wide % 256 <= 64 && narrow % 256 > 128);
-    if (const int f = p3v_tuning().gemm_f8_narrow; f >= 0) use_narrow = p.N % 256 != 0 || f != 0;
-    return use_narrow ? launch_gemm_f8_v<EPI, 2>(p, s) : launch_gemm_f8_v<EPI, 4>(p, s);
+// the tile whose rounds over the chip cost least.  A round's cost by tile, 128 x 256 = 100, measured over M 256 .. 8192 and the
+// decoder's four projections: 160 x 256 takes 1.02-1.18 of it (least where the chip's power is the limit), 128 x 192 0.87,
+// 128 x 128 0.69.  So 2531 rows x 3072 go in one round of 240 wide tiles (28.2 us; 480 narrow ones 30.4), 2048 in 256 of 192 columns
+// (23.8; wide 25.2), 1024 in 192 narrow ones (17.4; wide 23.5), 2531 x 16384 in 4 rounds of 160 rows (112; 5 of 128 rows 118).
+static void f8_tile_plan(const GemmF8P& p, bool silu, int& mb, int& nb) {
+  static const struct { int mb, nb, cost; } tiles[] = {{4, 4, 100}, {5, 4, 110}, {4, 3, 87}, {4, 2, 69}};
+  const int n_cu = p3v_gemm256_cus(), pin = p3v_tuning().gemm_f8_narrow;
+  long best = -1;
+  for (const auto& t : tiles) {
+    const int n_tile = silu ? 32 * t.nb : 64 * t.nb;
+    if (p.N % n_tile || (silu && t.nb % 2)) continue;
+    long c = (p3v_cdiv((long)(p.N / n_tile) * p3v_cdiv(p.M, 32 * t.mb), (long)max(n_cu, 1))) * t.cost;
+    if (pin == 10 * t.mb + t.nb || (pin == 0 && t.mb == 4 && t.nb == 4) || (pin == 1 && t.nb == 2)) c = 0;
+    if (best < 0 || c < best) best = c, mb = t.mb, nb = t.nb;
   }
+}
+
+template <int EPI>
+static int launch_f8(const GemmF8P& p, hipStream_t s) {
+  int mb = 0, nb = 0;
+  f8_tile_plan(p, EPI == P3V_EPI_SILU_MUL, mb, nb);
+  if constexpr (EPI != P3V_EPI_SILU_MUL)
+    if (nb == 3) return launch_f8_v<EPI, 4, 3>(p, s);
+  if (nb == 2) return launch_f8_v<EPI, 4, 2>(p, s);
+  return mb == 5 ? launch_f8_v<EPI, 5, 4>(p, s) : launch_f8_v<EPI, 4, 4>(p, s);
 }
 
 extern "C" int p3v_gemm_fp8(const p3v_gemm_fp8_args_t* a, void* stream) {
@@ -305,9 +322,9 @@ extern "C" int p3v_gemm_fp8(const p3v_gemm_fp8_args_t* a, void* stream) {
   const GemmF8P p = {a->A, a->a_scale, a->W, a->w_scale, a->out, a->resid, a->M, a->N, a->K, a->lda, a->ldw, a->ldo};
   hipStream_t s = (hipStream_t)stream;
   switch (a->epilogue) {
-    case P3V_EPI_NONE: return launch_gemm_f8<P3V_EPI_NONE>(p, s);
-    case P3V_EPI_RESID_BF16: return launch_gemm_f8<P3V_EPI_RESID_BF16>(p, s);
-    case P3V_EPI_SILU_MUL: return launch_gemm_f8<P3V_EPI_SILU_MUL>(p, s);
+    case P3V_EPI_NONE: return launch_f8<P3V_EPI_NONE>(p, s);
+    case P3V_EPI_RESID_BF16: return launch_f8<P3V_EPI_RESID_BF16>(p, s);
+    case P3V_EPI_SILU_MUL: return launch_f8<P3V_EPI_SILU_MUL>(p, s);
     default: return P3V_ERR_ARG;
   }
 }

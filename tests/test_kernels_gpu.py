@@ -1573,6 +1573,39 @@ def test_gemm_fp8(ops, request, epi, M, N, K, narrow):
     close(out, ref, rtol=2 ** -6, atol=2e-2 * ref.float().abs().max().item() / 16)
 
 
+@pytest.mark.parametrize("epi", ["none", "resid", "silu"])
+@pytest.mark.parametrize("M,N,K", [(1, 768, 128), (129, 768, 256), (160, 3072, 384), (161, 768, 640), (2049, 3072, 512), (321, 384, 1152)])
+def test_gemm_fp8_tiles_agree(ops, request, epi, M, N, K):
+    """Every tile of the fp8 GEMM sums an output's K-tiles in the same order, so all of them give the SAME bits: 1 .. 9 K-tiles
+    against three and four LDS buffers, row counts at and past the 128- and 160-row tiles, more output tiles than CUs (2049 x 3072:
+    the K-tile stream crosses from one output tile to the next), and against the products in float64."""
+    EPI = {"none": ops.EPI_NONE, "resid": ops.EPI_RESID_BF16, "silu": ops.EPI_SILU_MUL}[epi]
+    rows = 2 * N if epi == "silu" else N
+    a8, w8 = _e4m3(g((M, K), 50, 1.0, F32)).view(torch.uint8), _e4m3(g((rows, K), 51, 1.0, F32)).view(torch.uint8)
+    sa, sw = torch.rand((M,), generator=torch.Generator().manual_seed(52)) + 0.5, (torch.rand((rows,), generator=torch.Generator().manual_seed(53)) + 0.5) / K
+    resid = g((M, N), 54, 1.0) if epi == "resid" else None
+    dev = [t.cuda() for t in (a8, sa, w8, sw)]
+    old = ops.set_tuning("gemm_f8_narrow", -1)
+    request.addfinalizer(lambda: ops.set_tuning("gemm_f8_narrow", old))
+    outs = []
+    for tile in (-1, 44, 54, 43, 42):                            # (a tile that does not divide N falls back to the choice by shape)
+        ops.set_tuning("gemm_f8_narrow", tile)
+        out = torch.full((M + 1, N), float("nan"), dtype=BF16).cuda()                # (a guard row behind the last one)
+        ops.gemm_fp8(*dev, EPI, resid=None if resid is None else resid.cuda(), out=out)
+        assert torch.isnan(out[M].float()).all(), tile
+        outs.append(out[:M].clone())
+    for tile, out in zip((44, 54, 43, 42), outs[1:]):
+        assert torch.equal(out.view(torch.int16), outs[0].view(torch.int16)), tile
+    y = (a8.view(torch.float8_e4m3fn).double() * sa[:, None].double()) @ (w8.view(torch.float8_e4m3fn).double() * sw[:, None].double()).t()
+    if epi == "silu":
+        gate, up = y[:, :N], y[:, N:]
+        ref = gate / (1 + torch.exp(-gate)) * up
+    else:
+        ref = y if resid is None else y + resid.double()
+    # products are exact in fp32; K / 128 partial sums, then at most five bf16 roundings (2^-9 each, relative to the largest factor)
+    close(outs[0], ref.float(), rtol=5 * 2 ** -9, atol=5 * 2 ** -9 * y.abs().max().item())
+
+
 def test_gemm_fp8_asymmetric_identity(ops):
     """A = I (scaled), asymmetric W: catches a transposed / permuted C write and a wrong lane -> k mapping."""
     K = N = 256
