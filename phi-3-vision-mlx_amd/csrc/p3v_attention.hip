@@ -2543,6 +2543,185 @@ __global__ void __launch_bounds__(64) k_attn_decode_stream(AttnDecP p) {
   }
 }
 
+// One workgroup of four waves per (row, head): the whole key range of the pair, 32-key tiles dealt to its waves in turn, merged in LDS --
+// no split partials, no waiting for another workgroup.  For batches whose pairs fill the chip by themselves (attn_rows_fit).
+// A wave's tile goes registers -> its own LDS (no barrier); the key a lane takes from there is chosen so that its V^T piece is one
+// 16-byte read: key row i of the S^T product's block h is key 8 (i >> 2) + 4 h + (i & 3) of the tile, so lane group g ends up with the
+// scores of keys 8 g .. 8 g + 7, the k-slots its piece of a V^T row holds.
+// Two tiles of 12 KB per wave in flight, requested by buffer loads that are issued for dead tiles too, with an offset past the
+// buffer (the descriptor's bound turns them into zeros without traffic): a branch around them would turn the counted waits into
+// full ones.  K goes past the caches' replacement (whole lines, read once: -4 %), V^T does not: a 32-key piece is half a line.
+// What bounds it: ~6 us that do not depend on the length (launch, the new rows, the first tiles' latency, the merge), then one CU's
+// share of the keys at 28-30 KB/us, 5.7 TB/s when all CUs have one.  Fragments loaded straight from the caches, 16 pieces of 64
+// bytes per instruction and no LDS at all, ran at the same rate; eight waves a pair 0.5-4 us slower.
+__global__ void __launch_bounds__(256, 2) k_attn_decode_rows(AttnDecP p) {
+  constexpr int NW = 4, HD = 96, TK = 32, NKS = 3, NDT = 6, CPR = 12, ROWB = HD * 2 + 16, LQ = P3V_DECODE_MAX_L;
+  __shared__ __attribute__((aligned(16))) unsigned char Qs[16 * ROWB], Kn[LQ * ROWB];      // rotated queries, rotated new keys
+  __shared__ __attribute__((aligned(16))) bf16_t Vn[LQ * HD];                              // new values
+  constexpr int KSTR = HD * 2 + 16, VSTR = TK * 2 + 16, TILE = TK * KSTR + HD * VSTR, PSTR = HD + 4;
+  __shared__ __attribute__((aligned(16))) unsigned char tiles[NW][TILE];                   // per wave: K rows, V^T rows; at the end O, m, l of its queries
+  static_assert(16 * PSTR * 4 <= TILE, "");
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, qi = lane & 15, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int b = blockIdx.y, head = blockIdx.x, kvh = (head * p.grp_magic) >> 16;
+  const bool kv_writer = head == kvh * p.grp;
+  const float sc2 = p.scale * 1.4426950408889634f;            // softmax on exp2
+  const int row_w = (p.nh + 2 * p.nkv) * HD;
+  bf16_t* kc = p.k_cache + ((size_t)b * p.nkv + kvh) * (size_t)p.cache_t * HD;
+  bf16_t* vc = p.v_cache + ((size_t)b * p.nkv + kvh) * (size_t)HD * p.cache_t;             // V^T: [hd][cache_t]
+  const int past = p.d_past ? *p.d_past : p.past, pad = p.pad_len ? p.pad_len[b] : 0;
+
+  // ---- the new rows of the qkv projection: requested ahead of the tiles (memory returns in order)
+  const int tr = tid / CPR, tc = tid - tr * CPR;
+  const float* cos_b = p.cos_t + (size_t)b * p.rope_bstride * (HD / 2);
+  const float* sin_b = p.sin_t + (size_t)b * p.rope_bstride * (HD / 2);
+  const bf16_t* qkv_b = p.qkv + (size_t)b * p.L * row_w;
+  const bool rtask = tr < p.L;
+  RopeRaw qraw = {}, kraw = {};
+  u32x4_t vnew = {0, 0, 0, 0};
+  if (rtask) {
+    const bf16_t* row = qkv_b + (size_t)tr * row_w;
+    qraw = rope_fetch(row + head * HD, tc, cos_b + tr * (HD / 2), sin_b + tr * (HD / 2));
+    kraw = qraw;
+    const bf16_t* krow = row + (p.nh + kvh) * HD;
+    kraw.x0 = *(const u32x4_t*)(krow + tc * 8);
+    kraw.x1 = *(const u32x4_t*)(krow + (tc < 6 ? tc * 8 + 48 : tc * 8 - 48));
+    vnew = *(const u32x4_t*)(row + (p.nh + p.nkv + kvh) * HD + tc * 8);
+  }
+
+  // ---- this wave's tiles: kv_first, kv_first + 32 NW, ...
+  const int total = min(past + p.L, p.cache_t), kv_first = (pad & ~(TK - 1)) + TK * wave;
+  const __amdgpu_buffer_rsrc_t rs_k = __builtin_amdgcn_make_buffer_rsrc((void*)kc, 0, p.cache_t * HD * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs_v = __builtin_amdgcn_make_buffer_rsrc((void*)vc, 0, p.cache_t * HD * 2, 0x00020000);
+  const int k_lane = lane * 16, v_lane = ((lane >> 2) * p.cache_t + 8 * (lane & 3)) * 2, v_step = 16 * p.cache_t * 2;
+  struct Tile { u32x4_t k[6], v[6]; };                        // pieces 64 j + lane: 12 of a K row, 4 of a V^T row
+  auto load_tile = [&](Tile& t, int kv0) {
+    const bool live = kv0 < total;                             // (past the caches' bytes: nothing is fetched)
+    const int ko = live ? k_lane + kv0 * (HD * 2) : (int)0x80000000, vo = live ? v_lane + kv0 * 2 : (int)0x80000000;
+#pragma unroll
+    for (int j = 0; j < 6; ++j) t.k[j] = __builtin_amdgcn_raw_buffer_load_b128(rs_k, ko + j * 1024, 0, 2);
+#pragma unroll
+    for (int j = 0; j < 6; ++j) t.v[j] = __builtin_amdgcn_raw_buffer_load_b128(rs_v, vo, j * v_step, 0);
+  };
+  Tile ta, tb;
+  load_tile(ta, kv_first);
+  load_tile(tb, kv_first + TK * NW);
+
+  if (tid < 16 * CPR) {
+    u32x4_t v = {0, 0, 0, 0};
+    if (rtask) v = rope_apply(qraw, tc);
+    *(u32x4_t*)(Qs + tr * ROWB + tc * 16) = v;
+  }
+  if (rtask) {
+    const u32x4_t kn = rope_apply(kraw, tc);
+    *(u32x4_t*)(Kn + tr * ROWB + tc * 16) = kn;
+    *(u32x4_t*)(Vn + tr * HD + tc * 8) = vnew;
+    const int t = past + tr;
+    if (kv_writer && t < p.cache_t) {
+      *(u32x4_t*)(kc + (size_t)t * HD + tc * 8) = kn;                                      // phi.py:545
+#pragma unroll
+      for (int e = 0; e < 8; ++e) vc[(size_t)(tc * 8 + e) * p.cache_t + t] = (bf16_t)(vnew[e >> 1] >> (16 * (e & 1)));   // phi.py:546
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // (__syncthreads would wait for the tiles as well)
+  bf16x8_t qf[NKS];
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks) qf[ks] = *(const bf16x8_t*)(Qs + qi * ROWB + ks * 64 + g * 16);
+
+  const int qpos = past + qi;
+  float m_run = -INFINITY, l_run = 0.f;
+  f32x4_t o[NDT];
+#pragma unroll
+  for (int d = 0; d < NDT; ++d) o[d] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  unsigned char *Kt = tiles[wave], *Vt = Kt + TK * KSTR;
+  auto process = [&](Tile& t, int kv0, int kv_next) {
+    asm volatile("" ::: "memory");                             // (the reads of the tile before come first; a wave's LDS accesses stay in order)
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      const int i = j * 64 + lane;
+      *(u32x4_t*)(Kt + i / CPR * KSTR + i % CPR * 16) = t.k[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 6; ++j) *(u32x4_t*)(Vt + (j * 16 + (lane >> 2)) * VSTR + (lane & 3) * 16) = t.v[j];
+    load_tile(t, kv_next);
+    if (kv0 + TK > past) {                                     // wave-uniform: the tile holds new positions, which are not in the caches yet
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      const int r0 = max(kv0 - past, 0), n = min(kv0 + TK - past, p.L) - r0;
+#pragma unroll 1
+      for (int w = lane; w < n * CPR; w += 64) {
+        const int r = r0 + w / CPR, c = w % CPR, key = past + r - kv0;
+        *(u32x4_t*)(Kt + key * KSTR + c * 16) = *(const u32x4_t*)(Kn + r * ROWB + c * 16);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) *(bf16_t*)(Vt + (c * 8 + e) * VSTR + key * 2) = Vn[r * HD + c * 8 + e];
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    f32x4_t s[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      s[h] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks)
+        s[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)(Kt + (8 * (qi >> 2) + 4 * h + (qi & 3)) * KSTR + ks * 64 + g * 16), qf[ks], s[h], 0, 0, 0);
+    }
+    float m_t = -INFINITY;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int key = kv0 + 8 * g + 4 * h + r;
+        const bool vis = key < total && key >= pad && key <= qpos && qpos >= pad;
+        s[h][r] = vis ? s[h][r] * sc2 : -INFINITY;
+        m_t = fmaxf(m_t, s[h][r]);
+      }
+    m_t = rows_max(m_t);
+    const float m_new = fmaxf(m_run, m_t), m_use = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+    float l_t = 0.f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        s[h][r] = __builtin_amdgcn_exp2f(s[h][r] - m_use);
+        l_t += s[h][r];
+      }
+    l_run = l_run * alpha + rows_sum(l_t);
+    m_run = m_new;
+    const u32x4_t pw = {pack_bf16x2(s[0][0], s[0][1]), pack_bf16x2(s[0][2], s[0][3]), pack_bf16x2(s[1][0], s[1][1]), pack_bf16x2(s[1][2], s[1][3])};
+#pragma unroll
+    for (int d = 0; d < NDT; ++d) {
+      o[d] *= alpha;
+      o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)(Vt + (16 * d + qi) * VSTR + g * 16), __builtin_bit_cast(bf16x8_t, pw), o[d], 0, 0, 0);
+    }
+  };
+  for (int kv0 = kv_first; kv0 < total; kv0 += 2 * TK * NW) {
+    process(ta, kv0, kv0 + 2 * TK * NW);
+    if (kv0 + TK * NW < total) process(tb, kv0 + TK * NW, kv0 + 3 * TK * NW);
+  }
+
+  asm volatile("" ::: "memory");
+  if (qi < p.L) {
+    float* w = (float*)Kt + qi * PSTR;
+#pragma unroll
+    for (int d = 0; d < NDT; ++d) *(f32x4_t*)(w + 16 * d + 4 * g) = o[d];
+    if (g == 0) { w[HD] = m_run; w[HD + 1] = l_run; }
+  }
+  __syncthreads();
+  for (int idx = tid; idx < p.L * (HD / 2); idx += 64 * NW) {
+    const int q = idx / (HD / 2), d = (idx - q * (HD / 2)) * 2;
+    float M = -INFINITY, a0 = 0.f, a1 = 0.f, l = 0.f;
+    auto part = [&](int k) { return (const float*)tiles[k] + q * PSTR; };
+#pragma unroll
+    for (int k = 0; k < NW; ++k) M = fmaxf(M, part(k)[HD]);
+    const float Mu = M == -INFINITY ? 0.f : M;
+#pragma unroll
+    for (int k = 0; k < NW; ++k) {
+      const float c = __builtin_amdgcn_exp2f(part(k)[HD] - Mu);
+      a0 += c * part(k)[d], a1 += c * part(k)[d + 1], l += c * part(k)[HD + 1];
+    }
+    *(uint32_t*)(p.out + ((size_t)b * p.L + q) * (p.nh * HD) + head * HD + d) = pack_bf16x2(l > 0.f ? a0 / l : 0.f, l > 0.f ? a1 / l : 0.f);
+  }
+}
+
 // merge split-KV partials: one block of G = 4 or 8 64-lane groups per (b, head, query): thread (grp, d) loads
 // (m, l, o[d]) of its share of the splits (batches of 4 independent loads), reduces them against its own
 // running max, and the groups are merged through LDS.
@@ -2718,6 +2897,17 @@ extern "C" int p3v_attention_decode_fused_role(int wg, int n_heads, int n_split,
   return P3V_OK;
 }
 
+// (row, head) pairs that go one to a workgroup (k_attn_decode_rows), by pairs and cache capacity.  us against the split forms, 32 heads:
+//   short caches, from half a chip of pairs on: 4 rows x 128 5.4 : 6.0, 8 x 256 9.1 : 10.9, 16 x 256 14.9 : 17.9
+//   longer ones only where every CU gets the same number of pairs, a CU's share being what it waits for: 8 rows x 576 14.4 : 15.7,
+//   16 x 576 25.8 : 26.6, but 12 x 576 22.7 : 20.8; past ~640 keys the split forms' 64-key lines win (16 x 832 34.9 : 33.9)
+static bool attn_rows_fit(int pairs, int cache_t) {
+  const int pin = p3v_tuning().attn_rows;
+  if (pin >= 0) return pin != 0;
+  const int idle = (pairs + 255) / 256 * 256 - pairs;           // CUs without a pair in the last round over the chip's 256
+  return pairs >= 128 && pairs <= 512 && (cache_t <= 256 || (cache_t <= 640 && idle <= 64));
+}
+
 extern "C" int p3v_attention_decode(const p3v_attn_decode_args_t* a, void* stream) {
   if (!a || !a->qkv || !a->cos_t || !a->sin_t || !a->k_cache || !a->v_cache || !a->out || !a->ws) return P3V_ERR_ARG;
   if (a->hd != 96) return P3V_ERR_UNSUPPORTED;
@@ -2747,6 +2937,11 @@ extern "C" int p3v_attention_decode(const p3v_attn_decode_args_t* a, void* strea
     } else {
       hipLaunchKernelGGL(k_attn_decode128_o, grid, dim3(256), 0, s, p);
     }
+    P3V_CHECK_LAUNCH();
+    return P3V_OK;
+  }
+  if (!a->o_proj_w && attn_rows_fit(a->B * a->n_heads, a->cache_t)) {
+    hipLaunchKernelGGL(k_attn_decode_rows, dim3(a->n_heads, a->B), dim3(256), 0, s, p);
     P3V_CHECK_LAUNCH();
     return P3V_OK;
   }

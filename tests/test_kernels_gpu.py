@@ -961,6 +961,35 @@ def test_kv_quantize_mlx4_keys_from_exact_fp32_rotation(ops):
     assert torch.equal(kc.cpu()[:, :, :L], mlx_dequantize(pw, ps, pb, 32, 4).to(BF16).reshape(B, nkv, L, hd))
 
 
+@pytest.mark.parametrize("B,L,past,T,nh,nkv,pads", [(1, 1, 0, 64, 2, 2, None), (2, 1, 31, 64, 4, 2, [0, 31]), (3, 1, 32, 64, 2, 2, [0, 32, 33]),
+                                                    (1, 16, 120, 192, 2, 1, None), (2, 5, 251, 256, 4, 1, [0, 250]), (2, 3, 509, 512, 2, 2, [3, 255]),
+                                                    (4, 1, 700, 832, 2, 2, [0, 64, 699, 700])])
+@pytest.mark.parametrize("dev_past", [False, True])
+def test_attention_decode_rows(ops, request, B, L, past, T, nh, nkv, pads, dev_past):
+    """One workgroup per (row, head) against the split form: lengths at and next to a 32-key tile and a wave's turn (128 keys), new
+    rows on both sides of a tile and up to the capacity's last key, shared kv heads, padding that ends inside, at and one short of the
+    last key; the caches must come out with the same bits.  Both round P to bf16 (2^-9) against different maxima, then the output."""
+    hd = 96
+    qkv, kc, vc = g((B * L, (nh + 2 * nkv) * hd), 70), g((B, nkv, T, hd), 71), g((B, nkv, hd, T), 72)
+    torch.manual_seed(7)
+    cos, sin = torch.rand((B, L, hd // 2)).cuda(), torch.rand((B, L, hd // 2)).cuda()
+    pad = None if pads is None else torch.tensor(pads, dtype=torch.int32).cuda()
+    d_past = torch.tensor([past], dtype=torch.int32).cuda() if dev_past else None
+    ws = ops.attention_ws(B, L, nh, hd, 1, "cuda")
+    old = ops.set_tuning("attn_rows", -1)
+    request.addfinalizer(lambda: ops.set_tuning("attn_rows", old))
+    res = []
+    for rows in (0, 1):
+        ops.set_tuning("attn_rows", rows)
+        k, v, out = kc.cuda(), vc.cuda(), torch.full((B, L, nh * hd), float("nan"), dtype=BF16).cuda()
+        ops.attention_decode(qkv.cuda(), cos, sin, L, k, v, out, B, L, nh, nkv, hd, hd ** -0.5, 0 if dev_past else past, T, ws, 1,
+                             pad_len=pad, d_past=d_past, merge_in_launch=False)
+        assert (ws.view(torch.int32) == -1).all()
+        res.append((out, k, v))
+    assert torch.equal(res[0][1], res[1][1]) and torch.equal(res[0][2], res[1][2])
+    close(res[1][0], res[0][0], rtol=2 ** -8, atol=2 * 2 ** -9 * vc.float().abs().max().item())
+
+
 @pytest.mark.parametrize("seed", range(4))
 def test_attention_decode_random_shapes_merge_modes_agree(ops, seed):
     """Fuzz of the decode attention: random (B, L, past, heads, pads) on the 64-key, 128-key and streaming plans; the
