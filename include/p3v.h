@@ -483,8 +483,9 @@ int64_t p3v_attn_mix_ws_bytes(int B, int L, int H, int vdim, int n_split);
 
 /* RMS norm of fp32 rows: out = x / sqrt(mean x^2 + eps) * w * gain, one rounding (out bf16, or fp32 with out_f32) */
 int p3v_rms_rows(const float* x, const uint16_t* w, void* out, int out_f32, int rows, int H, float eps, float gain, void* stream);
-/* p3v_gemv whose input row is p3v_rms_rows of the fp32 row x with args->norm_w, args->norm_eps (args->x unused).  M = 1, K in {1024, 2048,
- * 3072, 4096, 8192}, epilogue NONE, SILU_MUL or GELU_MUL: otherwise P3V_ERR_UNSUPPORTED and the caller runs the two calls. */
+/* p3v_gemv whose input rows are p3v_rms_rows of the fp32 rows x with args->norm_w, args->norm_eps (args->x unused; from two rows on
+ * x w is what is rounded to bf16, the row's factor is applied to the sums).  M <= 8, K in {1024, 2048, 3072, 4096} or M = 1 and 8192,
+ * epilogue NONE, SILU_MUL or GELU_MUL: otherwise P3V_ERR_UNSUPPORTED and the caller runs the two calls. */
 int p3v_gemv_rms(const p3v_gemv_args_t* args /* host */, const float* x, float gain, void* stream);
 
 /* Gated linear attention of B x L new tokens.  y rows [B*L, ld]: H*dim query, H*dim key, H*vdim value, H*vdim gate, rank low-rank

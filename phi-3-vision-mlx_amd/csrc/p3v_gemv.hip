@@ -347,7 +347,10 @@ extern "C" int p3v_gemv_timing_read(long long* out, int n) {
 // first MFMA (that pass took 3 us; the sums are exchanged by the barrier the partials need anyway).  (Two slices in
 // flight per wave -- tried: the 32 extra load instructions block the wave in issue while the queues are full and the
 // prologue behind them gets later, not earlier.)
-template <bool SILU, int NW, int NST, bool SCALED = false>
+// XF32: x is fp32 rows (dyt.x), normalised by p3v_rms_rows' formula: r = gain / sqrt(mean x^2 + eps), gain = dyt.alpha.  The rows are
+// re-read by every workgroup (61 KB at five of 3072) instead of by a launch of their own in front (3.75 us): 564 -> 518 us for a step of 17 such projections.
+// As loads of 8 elements a lane, like the bf16 rows', half of what each one touches is fetched by the next: 544.
+template <bool SILU, int NW, int NST, bool SCALED = false, bool XF32 = false>
 __global__ void __launch_bounds__(NW * 64) k_gemv_mfma8(GemvP p, int n_sets) {
   constexpr int KQ = NST * 256, K = KQ * NW, XS = K * 2 + 64, NCH = KQ / 8;     // slice elements, LDS row stride (bytes), slice chunks
   constexpr int ROWS = SILU ? 8 : 16;                                            // output columns per set
@@ -383,10 +386,34 @@ __global__ void __launch_bounds__(NW * 64) k_gemv_mfma8(GemvP p, int n_sets) {
   // ---- x slice (8 rows x NCH chunks, lanes over chunks) first, then the weight stages of the first set
   GMARK(0);
   unsigned char* xslice = smem + k_lo * 2;
-  u32x4_t gv[2];
   float ss[8];
-  {
-    u32x4_t xv[8][2];
+  if constexpr (XF32) {                                                          // 4 elements a lane and load: NST whole kilobytes of a row's slice
+    float4 xv[8][NST];
+    u32x2_t gw[NST];
+    const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc((void*)p.dyt.x, 0, p.M * K * 4, 0x00020000);
+#pragma unroll
+    for (int k = 0; k < NST; ++k) {
+      const int c = k_lo + 4 * (lane + 64 * k);
+#pragma unroll
+      for (int m = 0; m < 8; ++m)                                                // (a row past M is past the buffer: zeros, no traffic)
+        xv[m][k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs_x, c * 4 + m * (K * 4), 0, 0));
+      gw[k] = *(const u32x2_t*)(p.norm_w + c);
+    }
+    issue(w0, w1, IC0{}, IC0{});
+    if constexpr (NST > 1) issue(w0, w1, IC1{}, IC0{});
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      ss[m] = 0.f;
+#pragma unroll
+      for (int k = 0; k < NST; ++k) {
+        const float4 v = xv[m][k];
+        ss[m] += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
+        *(u32x2_t*)(xslice + m * XS + (lane + 64 * k) * 8) =
+            (u32x2_t){pack_bf16x2(v.x * bf16lo(gw[k][0]), v.y * bf16hi(gw[k][0])), pack_bf16x2(v.z * bf16lo(gw[k][1]), v.w * bf16hi(gw[k][1]))};
+      }
+    }
+  } else {
+    u32x4_t xv[8][2], gv[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int c = min(lane + 64 * k, NCH - 1);
@@ -464,7 +491,7 @@ __global__ void __launch_bounds__(NW * 64) k_gemv_mfma8(GemvP p, int n_sets) {
       e_rf = ((const float*)p.resid)[e_live ? e_o : 0];
       e_ls = bf16_to_f32(p.col_scale[e_live ? e_n : 0]);
     }
-    uint32_t e_res = (e_has ? p.resid : p.x)[e_has && e_live ? e_o : 0];
+    uint32_t e_res = (e_has ? p.resid : XF32 ? p.W : p.x)[e_has && e_live ? e_o : 0];
     f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
     auto step = [&](auto stc) {
       constexpr int st = decltype(stc)::value;
@@ -510,7 +537,7 @@ __global__ void __launch_bounds__(NW * 64) k_gemv_mfma8(GemvP p, int n_sets) {
           t += red[w][m];
         }
         if (p.norm_w) {
-          const float r = rsqrtf(t / (float)K + p.eps);
+          const float r = XF32 ? p.dyt.alpha / sqrtf(t / (float)K + p.eps) : rsqrtf(t / (float)K + p.eps);
           v0 *= r;
           v1 *= r;
         }
@@ -536,12 +563,12 @@ __global__ void __launch_bounds__(NW * 64) k_gemv_mfma8(GemvP p, int n_sets) {
   do_set(IC0{}, std::false_type{});
 }
 
-template <bool SILU, int NW, int NST, bool SCALED = false>
+template <bool SILU, int NW, int NST, bool SCALED = false, bool XF32 = false>
 static int launch_gemv_mfma8(const GemvP& p, hipStream_t s) {
   const size_t lds = (size_t)8 * (p.K * 2 + 64);
   static bool attr_set = false;
   if (!attr_set && lds > 40 * 1024) {
-    if (hipFuncSetAttribute((const void*)k_gemv_mfma8<SILU, NW, NST, SCALED>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 8704) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)k_gemv_mfma8<SILU, NW, NST, SCALED, XF32>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 8704) != hipSuccess)
       return P3V_ERR_HIP;
     attr_set = true;
   }
@@ -549,7 +576,7 @@ static int launch_gemv_mfma8(const GemvP& p, hipStream_t s) {
   // (576 sets -> 192 x 3, 1024 -> 256 x 4, 2004 -> 251 x 8, 192 -> 192 x 1)
   const int max_wg = p3v_tuning().gemv8_wgs;
   const int n_sets = p3v_cdiv(p.N, SILU ? 8 : 16), per = p3v_cdiv(n_sets, max_wg), grid = p3v_cdiv(n_sets, per);
-  hipLaunchKernelGGL((k_gemv_mfma8<SILU, NW, NST, SCALED>), dim3(grid), dim3(NW * 64), lds, s, p, n_sets);
+  hipLaunchKernelGGL((k_gemv_mfma8<SILU, NW, NST, SCALED, XF32>), dim3(grid), dim3(NW * 64), lds, s, p, n_sets);
   P3V_CHECK_LAUNCH();
   return P3V_OK;
 }
@@ -617,11 +644,23 @@ extern "C" int p3v_gemv_dyt(const p3v_gemv_args_t* a, const p3v_dyt_args_t* d, v
 
 extern "C" int p3v_gemv_rms(const p3v_gemv_args_t* a, const float* x, float gain, void* stream) {
   if (!a || !x || !a->norm_w || !a->W || !a->out || a->M <= 0 || a->N <= 0 || a->K <= 0) return P3V_ERR_ARG;
-  if (a->M != 1 || (a->epilogue != P3V_EPI_NONE && !P3V_GATED(a->epilogue))) return P3V_ERR_UNSUPPORTED;
+  if (a->M > 8 || (a->epilogue != P3V_EPI_NONE && !P3V_GATED(a->epilogue))) return P3V_ERR_UNSUPPORTED;
   if (((uintptr_t)x | (uintptr_t)a->norm_w | (uintptr_t)a->W) & 15) return P3V_ERR_UNSUPPORTED;
   GemvP p = {nullptr, a->W, a->out, nullptr, nullptr, a->norm_eps, a->M, a->N, a->K, a->epilogue,
              P3V_GATED(a->epilogue) ? a->N : (a->N + 1) / 2, nullptr, {}};
   p.dyt.x = x, p.dyt.w = a->norm_w, p.dyt.alpha = gain;
+  if (a->M > 1) {
+    if (!p3v_tuning().gemv_mfma8 || a->M < p3v_tuning().gemv8_min) return P3V_ERR_UNSUPPORTED;
+    p.norm_w = a->norm_w;
+    const bool gated = P3V_GATED(a->epilogue);
+    switch (a->K) {                                    // (8192: rows and weights of a wave do not fit its registers)
+      case 1024: return gated ? launch_gemv_mfma8<true, 4, 1, false, true>(p, (hipStream_t)stream) : launch_gemv_mfma8<false, 4, 1, false, true>(p, (hipStream_t)stream);
+      case 2048: return gated ? launch_gemv_mfma8<true, 4, 2, false, true>(p, (hipStream_t)stream) : launch_gemv_mfma8<false, 4, 2, false, true>(p, (hipStream_t)stream);
+      case 3072: return gated ? launch_gemv_mfma8<true, 4, 3, false, true>(p, (hipStream_t)stream) : launch_gemv_mfma8<false, 4, 3, false, true>(p, (hipStream_t)stream);
+      case 4096: return gated ? launch_gemv_mfma8<true, 8, 2, false, true>(p, (hipStream_t)stream) : launch_gemv_mfma8<false, 8, 2, false, true>(p, (hipStream_t)stream);
+      default: return P3V_ERR_UNSUPPORTED;
+    }
+  }
   return gemv3_layered<GEMV_RMS>(p, (hipStream_t)stream);
 }
 

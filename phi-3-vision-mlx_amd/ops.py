@@ -669,14 +669,14 @@ def rms_rows(x, norm, out):
 
 
 def project_rms(x, norm, w, h, epilogue=EPI_NONE, out=None):
-    """project(rms_rows(x)): one launch for a single bf16 row of a width the streaming kernel takes, else the two (h: their scratch rows)."""
+    """project(rms_rows(x)): one launch for up to 8 bf16 rows of a width the streaming kernels take, else the two (h: their scratch rows)."""
     M, H = x.shape
-    if M == 1 and h.dtype == BF16 and out is not None:
+    if M <= 8 and h.dtype == BF16 and out is not None:
         _chk(x, F32, "x"), _chk(w, BF16, "w"), _chk(out, BF16, "out"), _chk(norm[0], BF16, "norm")
         N = w.shape[0] // 2 if epilogue in GATED else w.shape[0]
-        if w.shape[1] != H or out.numel() != N or norm[0].numel() != H:
+        if w.shape[1] != H or out.numel() != M * N or (M > 1 and tuple(out.shape) != (M, N)) or norm[0].numel() != H:
             raise ValueError(f"project_rms: {tuple(w.shape)} on rows of {H} -> {tuple(out.shape)}")
-        args = L.GemvArgs(0, _p(w), _p(out), 0, _p(norm[0]), float(norm[1]), 1, N, H, epilogue, 0)
+        args = L.GemvArgs(0, _p(w), _p(out), 0, _p(norm[0]), float(norm[1]), M, N, H, epilogue, 0)
         rc = L.lib().p3v_gemv_rms(C.byref(args), _p(x), float(norm[2]), _stream())
         if rc != L.ERR_UNSUPPORTED:
             L.check(rc, "gemv_rms")

@@ -69,6 +69,30 @@ def test_rms_norm_in_the_projection_prologue(K, gelu):
     close(host(out), orc.gelu_tanh(y[:, :N]) * y[:, N:] if gelu else y, BF16)
 
 
+@pytest.mark.parametrize("M,N,K", [(2, 33, 1024), (3, 4120, 2048), (5, 96, 3072), (8, 40, 4096), (7, 72, 8192), (8, 8200, 1024)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_rms_norm_in_the_projection_prologue_of_a_batch(M, N, K, gelu):
+    """2 .. 8 rows of very different sizes: the fused launch (8192: the two launches) = norm, then the projection; a partial last set of
+    columns, more sets than workgroups; a row behind the last one stays as it was."""
+    from phi_3_vision_mlx_amd import ops
+    r = np.random.default_rng(K + M)
+    x, w, nw = r.normal(0, 3, (M, K)) * 10.0 ** r.uniform(-4, 3, (M, 1)), bf(r.normal(0, K ** -0.5, (2 * N if gelu else N, K))), bf(r.normal(1, 0.3, K))
+    xd, scratch, out = dev(x, F32), torch.empty((M, K), dtype=BF16, device=DEV), torch.full((M + 1, N), float("nan"), dtype=BF16, device=DEV)
+    y = orc.rms(host(xd), nw, 0.2) * -0.7 @ w.T
+    ops.project_rms(xd, (dev(nw), 0.2, -0.7), dev(w), scratch, ops.EPI_GELU_MUL if gelu else ops.EPI_NONE, out=out[:M])
+    close(host(out[:M]), orc.gelu_tanh(y[:, :N]) * y[:, N:] if gelu else y, BF16)
+    assert torch.isnan(out[M].float()).all()
+
+
+@pytest.mark.parametrize("hidden,off", [(8, 0), (3072, 0), (3072, 1), (2049, 0), (4104, 0)])
+def test_embedding_rows_of_every_width_and_alignment(hidden, off):
+    from phi_3_vision_mlx_amd import ops
+    ids = torch.tensor([3, -1, 9, 99], dtype=torch.int32, device=DEV)
+    table = torch.randn(10 * hidden + off, device=DEV).to(BF16)[off:].view(10, hidden)
+    out = ops.embed_scale(ids, table, 0.37)
+    assert torch.equal(out, table[[3, 0, 9, 9]].float() * 0.37)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 64, 128), (1, 96, 3072), (2, 50, 136), (3, 40, 1024), (5, 96, 2048), (8, 64, 3072), (8, 40, 8192), (12, 128, 3072),
                                    (16, 192, 512), (20, 256, 3072), (60, 128, 1024), (100, 256, 1024), (300, 3072, 512), (1100, 512, 256), (7, 33, 72)])
 @pytest.mark.parametrize("dt", [F32, BF16])
