@@ -61,6 +61,41 @@ template <int HW> struct MixCfg {
   static constexpr int LDS = S_BYTES + P_BYTES + 2 * A_BYTES + HM * 1024 + (HW == 4 ? 8 * 4096 : 0);
 };
 
+// A run = the key tiles [split * per, ..) of one query tile.  first query tile that sees 32-key tile T - 1, and how many do
+__host__ __device__ static inline int mix_q_first(int past, int T) { const int d = 32 * (T - 1) - 15 - past; return d <= 0 ? 0 : (d + 15) >> 4; }
+__host__ __device__ static inline int mix_q_count(int past, int L, int T) {
+  return T > ((past + L - 1) >> 5) + 1 ? 0 : ((L + 15) >> 4) - mix_q_first(past, T);
+}
+// Run number `wid` in the order of the runs' lengths: the full ones split by split, then the partial ones by decreasing length -- with a
+// workgroup per CU, long runs that start late are what the last CUs wait for (2048 rows: 18 tiles' time instead of 23 - 27).
+struct MixRun { int qt, split, b; };
+__device__ __forceinline__ MixRun mix_run(int wid, const AttnMixP& p) {
+  const int per = p.tiles_per_split, n_qt = (p.L + 15) >> 4;
+  for (int s = 0; s < p.n_split; ++s) {
+    const int n = p.B * mix_q_count(p.past, p.L, (s + 1) * per);
+    if (wid < n) return {n_qt - 1 - wid / p.B, s, wid % p.B};
+    wid -= n;
+  }
+  const int lane = threadIdx.x & 63;
+  for (int o0 = 0; o0 < (per - 1) * p.n_split; o0 += 64) {               // (length, split) pairs, a lane each
+    const int o = o0 + lane, len = per - 1 - o / p.n_split, T = o % p.n_split * per + len;
+    const int n = len > 0 ? p.B * (mix_q_count(p.past, p.L, T) - mix_q_count(p.past, p.L, T + 1)) : 0;
+    int sum = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(sum, d);
+      sum += lane >= d ? v : 0;
+    }
+    const unsigned long long hit = __ballot(wid < sum);
+    if (hit) {
+      const int l = __builtin_ctzll(hit), r = wid - __shfl(sum - n, l), q = __shfl(mix_q_first(p.past, T), l), sp = __shfl(o % p.n_split, l);
+      return {__builtin_amdgcn_readfirstlane(q + r / p.B), __builtin_amdgcn_readfirstlane(sp), __builtin_amdgcn_readfirstlane(r % p.B)};
+    }
+    wid -= __shfl(sum, 63);
+  }
+  return {-1, 0, 0};
+}
+
 template <int HW, int DC, int VC, bool SHARED>
 __global__ void __launch_bounds__(512, 1) k_attn_mix_prefill(AttnMixP p) {
   typedef MixCfg<HW> C;
@@ -74,7 +109,10 @@ __global__ void __launch_bounds__(512, 1) k_attn_mix_prefill(AttnMixP p) {
   float* AL = (float*)(smem + C::S_BYTES + C::P_BYTES);
   float* MM = AL + C::HM * 256;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lc = lane & 15, lg = lane >> 4;
-  const int n_qt = (p.L + 15) >> 4, qt = n_qt - 1 - (int)blockIdx.x, split = blockIdx.y, b = blockIdx.z;   // longest rows first
+  MixRun run = {((p.L + 15) >> 4) - 1 - (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z};             // longest rows first
+  if (p.by_size) run = mix_run(blockIdx.x, p);
+  if (run.qt < 0) return;
+  const int qt = run.qt, split = run.split, b = run.b;
   const int q0 = qt * 16, per = p.H / p.G, past = p.d_past ? *p.d_past : p.past, first = p.pad_len ? p.pad_len[b] : 0;
   const int last = past + min(q0 + 15, p.L - 1);                         // last key any query of the tile sees
   // key tiles of this split: the same for every query tile, so that the workgroups an XCD runs together walk the same keys (its L2
@@ -604,6 +642,18 @@ static bool mix_fast(int H, int G, int dim, int vdim, int f32) {
   return !f32 && H <= MIX_MAX_H && dim <= 128 && vdim <= 128;
 }
 
+// Prompts: key tiles of a run.  A CU's share of all of them: with the runs in order of length the launch then lasts about that long.
+// Not below 4 (what a run costs besides its tiles), at most MIX_MAX_ROW_SPLIT runs a query tile.
+// A prompt in 8 layers, us, against equal parts for about 320 workgroups in their plain order: 2048 tokens 5168 -> 5110, 2500 7340 -> 6685,
+// 3000 7999 -> 7770, 4096 11797 -> 11300, 512 and 1500 alike.  (At 2048 the attention itself 184 -> 170 us, where the longest CU's tiles
+// go from 22 to 17: with every CU busy a tile takes longer, its 393 KB of keys and values come out of the L2s at 10.7 TB/s.)
+static int mix_run_tiles(int B, int L, int past) {
+  long sum = 0;
+  for (int q = 0; q < L; q += 16) sum += ((past + min(q + 15, L - 1)) >> 5) + 1;
+  const int want = p3v_tuning().mix_wgs;
+  return max(max(4, p3v_cdiv(sum * B, want > 0 ? want : 256)), p3v_cdiv(((past + L - 1) >> 5) + 1, MIX_MAX_ROW_SPLIT));
+}
+
 extern "C" int p3v_attn_mix_plan(int B, int L, int H, int G, int dim, int vdim, int n_keys, int f32) {
   if (B <= 0 || L <= 0 || H <= 0 || G <= 0 || n_keys <= 0 || !mix_fast(H, G, dim, vdim, f32)) return 0;
   const int want = p3v_tuning().mix_wgs;
@@ -611,8 +661,7 @@ extern "C" int p3v_attn_mix_plan(int B, int L, int H, int G, int dim, int vdim, 
     const int tiles = p3v_cdiv(n_keys, 16), per = p3v_cdiv(tiles, max(1, (want > 0 ? want : 256) / B));
     return min(p3v_cdiv(tiles, per), MIX_MAX_SPLIT);
   }
-  const int qt = p3v_cdiv(L, 16) * B, tiles = p3v_cdiv(n_keys, 32);
-  return max(1, min(min(MIX_MAX_ROW_SPLIT, p3v_cdiv(want > 0 ? want : 320, qt)), tiles / 4));
+  return p3v_cdiv(p3v_cdiv(n_keys, 32), mix_run_tiles(B, L, n_keys - L));
 }
 
 extern "C" int64_t p3v_attn_mix_ws_bytes(int B, int L, int H, int vdim, int n_split) {
@@ -634,7 +683,13 @@ static int launch_prefill(const AttnMixP& p, hipStream_t s) {
     if (hipFuncSetAttribute((const void*)k_attn_mix_prefill<HW, DC, VC, SHARED>, hipFuncAttributeMaxDynamicSharedMemorySize, MixCfg<HW>::LDS) != hipSuccess) return P3V_ERR_HIP;
     attr_set = true;
   }
-  hipLaunchKernelGGL((k_attn_mix_prefill<HW, DC, VC, SHARED>), dim3(p3v_cdiv(p.L, 16), p.n_split, p.B), dim3(512), MixCfg<HW>::LDS, s, p);
+  dim3 grid(p3v_cdiv(p.L, 16), p.n_split, p.B);
+  if (p.by_size) {
+    int runs = 0;
+    for (int sp = 0; sp < p.n_split; ++sp) runs += p.B * mix_q_count(p.past, p.L, sp * p.tiles_per_split + 1);
+    grid = dim3(runs);
+  }
+  hipLaunchKernelGGL((k_attn_mix_prefill<HW, DC, VC, SHARED>), grid, dim3(512), MixCfg<HW>::LDS, s, p);
   P3V_CHECK_LAUNCH();
   return p.n_split > 1 ? mix_combine(p, s) : P3V_OK;
 }
@@ -666,7 +721,10 @@ extern "C" int p3v_attn_mix(const p3v_mix_args_t* a, void* stream) {
   if (a->n_split > 1 && (!a->ws || a->n_split > MIX_MAX_ROW_SPLIT)) return P3V_ERR_ARG;
   AttnMixP p = attn_mix_params(a);
   // (the position may be a device value: the splits then cover the capacity)
-  p.tiles_per_split = p3v_cdiv(p3v_cdiv(a->d_past ? a->Tp : a->past + a->L, 32), a->n_split);
+  const int tiles = p3v_cdiv(a->d_past ? a->Tp : a->past + a->L, 32);
+  p.tiles_per_split = p3v_cdiv(tiles, a->n_split);
+  p.by_size = !a->d_past && a->n_split > 1;
+  if (const int per = mix_run_tiles(a->B, a->L, a->past); p.by_size && p3v_cdiv(tiles, per) == a->n_split) p.tiles_per_split = per;   // as planned
   if (p.n_split > 1 && p.L == 1) return P3V_ERR_ARG;                     // (k_attn_mix_combine's splits are 16-key tiles)
   const int per = p.H / p.G;                                             // query heads of a key / value head
   if (p.H <= 8) return prefill_dc<1, true>(p, s);

@@ -305,6 +305,25 @@ def test_mixed_attention_key_splits(H, G, dim, vdim, n_split):
         close(got[:, 0], np.stack(want), BF16)
 
 
+@pytest.mark.parametrize("B,L,past,pads", [(1, 16, 300, None), (1, 700, 0, None), (2, 333, 31, [0, 40]), (3, 1025, 0, [0, 64, 1000]), (1, 1500, 545, [7])])
+def test_mixed_attention_runs_by_length(B, L, past, pads):
+    """The planned runs, in their order of length (whole and partial ones, several rows, a position inside a tile), give the rows of one
+    run per query tile; the same runs in their plain order (the position on the device) too.  All three sum the same fp32 terms."""
+    from phi_3_vision_mlx_amd import ops
+    m = Mix(4, 2, 64, 64, B, (past + L + 31) // 32 * 32, BF16, seed=L)
+    raw = dev(m.r.normal(0, 1, (B, past + L, m.ld)), BF16)
+    if past:
+        m.run(raw[:, :past].contiguous().view(B * past, -1), past, 0, pads, plan=1)
+    x = raw[:, past:].contiguous().view(B * L, -1)
+    plan = ops.mix_plan(B, L, 4, 2, 64, 64, past + L, BF16)
+    assert plan > 1
+    want = m.run(x, L, past, pads, plan=1)
+    for got in (m.run(x, L, past, pads), m.run(x, L, past, pads, d_past=True)):
+        for b in range(B):
+            lo = max(0, (pads[b] if pads else 0) - past)
+            close(got[b, lo:], want[b, lo:], BF16)
+
+
 @pytest.mark.parametrize("dt", [F32, BF16])
 @pytest.mark.parametrize("far", [0, 1, 15, 16, 31, 32, 255, 256, 399])
 def test_one_far_key_decides(far, dt):
