@@ -202,6 +202,10 @@ typedef struct {
   float q_scale;
 } p3v_qkv_split_t;
 int p3v_gemm_qkv(const p3v_gemm_args_t* gemm /* host */, const p3v_qkv_split_t* split /* host */, void* stream);
+/* ... for p3v_gemm_fp8 (epilogue NONE; out / resid unused), any number of rows.  P3V_ERR_UNSUPPORTED (nothing launched) unless hd % 32 == 0,
+ * (hd / 2) % 16 == 0, whole 256-column tiles per region, an 8-aligned append offset and dst_t. */
+int p3v_gemm_qkv_fp8(const p3v_gemm_fp8_args_t* gemm /* host */, const p3v_qkv_split_t* split /* host */, void* stream);
+int p3v_gemm_qkv_fp8_pays(int M, int n_q, int n_kv, int K);      /* 1: faster than the two calls (n_q, n_kv: rows of W per region) */
 
 /* ---- attention, phi.py:454-457 (decoder, causal + left-pad, Mask4D phi.py:550-563)
  * and phi.py:148 (CLIP, no mask).  q [B, nh, L, hd]; keys/values come from two

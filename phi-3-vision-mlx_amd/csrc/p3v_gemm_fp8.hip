@@ -26,8 +26,9 @@
 //   epilogue  scales, then none / residual add / SiLU(gate) * up, bf16 out, straight from the accumulators (p3v_gemm256_epi.h).
 #include <stdlib.h>
 
-#include "p3v_common.h"
+#include "p3v_gemm_qkv.h"
 
+#define P3V_EPI_QKV 100                // internal: the qkv projection with split + RoPE + KV append in the epilogue (p3v_gemm_qkv.h)
 #define TKB 128                        // K bytes (= fp8 elements) per K-tile
 
 typedef __attribute__((address_space(3))) void* lptr_t;
@@ -36,9 +37,12 @@ typedef __attribute__((ext_vector_type(8))) int i32x8_t;
 struct GemmF8P {
   const uint8_t* A; const float* sa; const uint8_t* W; const float* sw; bf16_t* out; const bf16_t* resid;
   int M, N, K, lda, ldw, ldo;
+  QkvP q;                              // P3V_EPI_QKV only
 };
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));   // (scales: any float address)
 
-struct TileF8 { int a_off[8], b_off[8]; __amdgpu_buffer_rsrc_t rs_a; };   // where the requests of an output tile's K-tiles come from
+struct PlaceF8 { int m0, n0, swapped, is_k, row0; };             // P3V_EPI_QKV: V tile (operand roles swapped) / K region / first W row of the region
+struct TileF8 { int a_off[8], b_off[8]; __amdgpu_buffer_rsrc_t rs_a, rs_b; };   // where the requests of an output tile's K-tiles come from
 
 #define F8_BUF(mb, nb) ((32 * (mb) + 64 * (nb)) * TKB)
 #define F8_STAGES(mb, nb) (160 * 1024 / F8_BUF(mb, nb) < 4 ? 160 * 1024 / F8_BUF(mb, nb) : 4)
@@ -46,7 +50,8 @@ struct TileF8 { int a_off[8], b_off[8]; __amdgpu_buffer_rsrc_t rs_a; };   // whe
 // MB, NB: 16-row / 16-column blocks of a consumer wave (2 x 4 waves: a tile of 32 MB rows x 64 NB columns)
 template <int EPI, int MB, int NB>
 __global__ void __launch_bounds__(768, 1) k_gemm_f8(GemmF8P p) {
-  constexpr bool SILU = EPI == P3V_EPI_SILU_MUL;
+  constexpr bool SILU = EPI == P3V_EPI_SILU_MUL, QKV = EPI == P3V_EPI_QKV;
+  static_assert(!QKV || NB == 4, "both halves of 32 rotation pairs in a wave");
   static_assert(NB % 2 == 0 || !SILU, "a wave's column blocks: gate, then up of the same outputs");
   constexpr int HB = SILU ? NB / 2 : NB;                           // column blocks of outputs of a wave
   constexpr int TM = 32 * MB, TN = 64 * NB, A_BYTES = TM * TKB, BUF_BYTES = F8_BUF(MB, NB);
@@ -55,17 +60,27 @@ __global__ void __launch_bounds__(768, 1) k_gemm_f8(GemmF8P p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr int n_out_tile = SILU ? TN / 2 : TN;
-  const int gx = p.N / n_out_tile, gy = (p.M + TM - 1) / TM, nwg = gx * gy;
+  // (QKV: column tiles 0 .. nq - 1 are Q, the others K; behind them the V tiles, TM rows of W_v by TN tokens)
+  const int nq = QKV ? p.q.nh * p.q.hd / TN : 0;
+  const int gx = QKV ? nq + p.q.nkv * p.q.hd / TN : p.N / n_out_tile, gy = (p.M + TM - 1) / TM;
+  const int vx = QKV ? (p.M + TN - 1) / TN : 0, vy = QKV ? p.q.nkv * p.q.hd / TM : 0, nwg = gx * gy + vx * vy;
   const int nk = p.K / TKB;
 
   // persistent over output tiles, XCD-aware order (as p3v_gemm_pc.hip): each XCD gets a contiguous run of tiles, bands of 4 M tiles
-  auto place = [&](int wid, int& m0, int& n0) {
+  auto place = [&](int wid) {
     const int q = nwg >> 3, r = nwg & 7, xcd = wid & 7, loc = wid >> 3;
-    const int id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + loc;
+    int id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + loc;
+    const bool v = QKV && id >= gx * gy;
+    if (v) id -= gx * gy;
+    const int cx = v ? vx : gx, cy = v ? vy : gy;
     constexpr int BAND = 4;
-    const int band = id / (BAND * gx), in_band = id % (BAND * gx);
-    const int rows = min(BAND, gy - band * BAND);
-    m0 = (band * BAND + in_band % rows) * TM, n0 = in_band / rows * n_out_tile;
+    const int band = id / (BAND * cx), in_band = id % (BAND * cx);
+    const int rows = min(BAND, cy - band * BAND);
+    const int y = band * BAND + in_band % rows, x = in_band / rows;
+    PlaceF8 t = {y * TM, x * n_out_tile, 0, 0, 0};
+    if (v) t = {x * TN, y * TM, 1, 0, (p.q.nh + p.q.nkv) * p.q.hd};          // first token, first row of the V region
+    else if (QKV && x >= nq) t.is_k = 1, t.n0 -= nq * TN, t.row0 = p.q.nh * p.q.hd;
+    return t;
   };
   if ((int)blockIdx.x >= nwg) return;
   const int n_mine = (nwg - 1 - (int)blockIdx.x) / (int)gridDim.x + 1, total = n_mine * nk;      // output tiles, K-tiles of this workgroup
@@ -73,24 +88,30 @@ __global__ void __launch_bounds__(768, 1) k_gemm_f8(GemmF8P p) {
   if (wave >= 8) {
     // ---- PRODUCERS (p3v_gemm_pc.hip)
     const int pw = wave - 8, srow = pw * 8 + (lane >> 3), sw = ((lane & 7) ^ (lane >> 3)) * 16;
-    const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, 0xffffffff, 0x00020000);
     TileF8 dt;    // (declared outside the template: a builtin called with a member of a DEPENDENT type is only checked at
                   //  instantiation, fails there in the HOST pass -- no such builtin -- and hipcc silently drops the host stub)
     auto aim = [&](int wid) {
-      int m0, n0;
-      place(wid, m0, n0);
+      const PlaceF8 t = place(wid);
+      const int m0 = t.m0, n0 = t.n0;
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const int rr = q * 32 + srow;
-        int br = min(n0 + rr, p.N - 1);
+        int br = QKV ? qkv_pair_row(p.q, t.row0, n0 >> 1, rr) : min(n0 + rr, p.N - 1);
         if (SILU) {                                               // a wave's 16 HB gate rows + the 16 HB up rows of the same outputs
           const int in = rr % (NB * 16);
           br = n0 + rr / (NB * 16) * (HB * 16) + in % (HB * 16) + in / (HB * 16) * p.N;
         }
         dt.a_off[q] = (min(m0 + rr, p.M - 1) - m0) * p.lda + sw;
         dt.b_off[q] = (int)((unsigned)br * (unsigned)p.ldw + (unsigned)sw);
+        if (QKV && t.swapped) {                                   // W rows fill the A side, tokens the B side
+          dt.a_off[q] = rr * p.ldw + sw;
+          dt.b_off[q] = (int)((unsigned)min(m0 + rr, p.M - 1) * (unsigned)p.lda + (unsigned)sw);
+        }
       }
-      dt.rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + (size_t)m0 * p.lda), 0, 0xffffffff, 0x00020000);
+      const uint8_t* pa = QKV && t.swapped ? p.W + (size_t)(t.row0 + n0) * p.ldw : p.A + (size_t)m0 * p.lda;
+      const uint8_t* pb = QKV && t.swapped ? p.A : p.W;
+      dt.rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)pa, 0, 0xffffffff, 0x00020000);
+      dt.rs_b = __builtin_amdgcn_make_buffer_rsrc((void*)pb, 0, 0xffffffff, 0x00020000);
     };
     int dwid = blockIdx.x, dk = 0, slot = 0;                      // the next K-tile to request, and its buffer
     aim(dwid);
@@ -110,7 +131,7 @@ __global__ void __launch_bounds__(768, 1) k_gemm_f8(GemmF8P p) {
         if (q < nb) {
           lptr_t dst = (lptr_t)(base + a_bytes + q * 4096);
           const int vo = dt.b_off[q];
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, dst, 16, vo, dk * TKB, 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(dt.rs_b, dst, 16, vo, dk * TKB, 0, 0);
         }
       }
       slot = slot == S - 1 ? 0 : slot + 1;
@@ -157,8 +178,8 @@ __global__ void __launch_bounds__(768, 1) k_gemm_f8(GemmF8P p) {
   int slot = 0;                                                   // LDS buffer of the K-tile in hand
   __builtin_amdgcn_s_barrier();
   for (int wid = blockIdx.x; wid < nwg; wid += gridDim.x) {
-    int m0, n0;
-    place(wid, m0, n0);
+    const PlaceF8 at = place(wid);
+    const int m0 = at.m0, n0 = at.n0;
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -201,13 +222,53 @@ __global__ void __launch_bounds__(768, 1) k_gemm_f8(GemmF8P p) {
     // ---- epilogue, straight from the accumulators: lane (fc = lane & 15, fq = lane >> 4) holds columns 4 fq .. 4 fq + 3 of block row fc;
     // lanes q and q ^ 1 trade packed halves of two neighbouring column blocks: 16-byte stores (p3v_gemm256_epi.h)
     const int fc = lane & 15, fq = lane >> 4;
+    if constexpr (QKV) {                                           // the same products of sum and scales, then p3v_gemm_qkv's epilogues
+      if (at.swapped) {
+        float st[4][4], sr[MB];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) st[j][r] = p.sa[min(m0 + wc * 64 + j * 16 + fq * 4 + r, p.M - 1)];
+#pragma unroll
+        for (int i = 0; i < MB; ++i) sr[i] = p.sw[at.row0 + n0 + (wr * MB + i) * 16 + fc];
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][j][r] *= st[j][r] * sr[i];
+        qkv_epilogue_vt<MB>(p.q, acc, nullptr, n0 + wr * MB * 16, m0 + wc * 64, p.M, lane);
+      } else {
+        f32x4_a4 sc[4];
+        float st[MB];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sc[j] = *(const f32x4_a4*)(p.sw + qkv_pair_row(p.q, at.row0, n0 >> 1, wc * 64 + j * 16 + fq * 4));
+#pragma unroll
+        for (int i = 0; i < MB; ++i) st[i] = p.sa[min(m0 + (wr * MB + i) * 16 + fc, p.M - 1)];
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][j][r] *= st[i] * sc[j][r];
+        static_assert(!QKV || MB % 2 == 0, "");
+#pragma unroll
+        for (int i = 0; i < MB; i += 2) {                          // (two block rows' table values at a time: the registers of twelve waves)
+          f32x4_t part[2][4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) part[0][j] = acc[i][j], part[1][j] = acc[i + 1][j];
+          qkv_epilogue_rot<2>(p.q, part, nullptr, at.is_k, at.row0, (n0 >> 1) + wc * 32, m0 + (wr * MB + i) * 16, p.M, lane);
+        }
+      }
+      continue;
+    }
     const int mrow0 = m0 + wr * MB * 16 + fc, nw = n0 + wc * (n_out_tile / 4);
     float sc[NB][4];
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
       const int n = SILU ? nw + j % HB * 16 + fq * 4 + j / HB * p.N : nw + j * 16 + fq * 4;
-      const float4 c = *(const float4*)(p.sw + n);
-      sc[j][0] = c.x, sc[j][1] = c.y, sc[j][2] = c.z, sc[j][3] = c.w;
+      const f32x4_a4 c = *(const f32x4_a4*)(p.sw + n);
+      sc[j][0] = c[0], sc[j][1] = c[1], sc[j][2] = c[2], sc[j][3] = c[3];
     }
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
@@ -276,7 +337,8 @@ static int launch_f8_v(const GemmF8P& p, hipStream_t s) {
   }
   const int n_cu = p3v_gemm256_cus();
   if (!n_cu) return P3V_ERR_HIP;
-  const int tiles = p.N / (EPI == P3V_EPI_SILU_MUL ? 32 * NB : 64 * NB) * p3v_cdiv(p.M, 32 * MB);
+  int tiles = p.N / (EPI == P3V_EPI_SILU_MUL ? 32 * NB : 64 * NB) * p3v_cdiv(p.M, 32 * MB);
+  if (EPI == P3V_EPI_QKV) tiles = (p.q.nh + p.q.nkv) * p.q.hd / (64 * NB) * p3v_cdiv(p.M, 32 * MB) + p.q.nkv * p.q.hd / (32 * MB) * p3v_cdiv(p.M, 64 * NB);
   hipLaunchKernelGGL((k_gemm_f8<EPI, MB, NB>), dim3(min(tiles, n_cu)), dim3(768), LDS, s, p);
   P3V_CHECK_LAUNCH();
   return P3V_OK;
@@ -286,23 +348,24 @@ static int launch_f8_v(const GemmF8P& p, hipStream_t s) {
 // decoder's four projections: 160 x 256 takes 1.02-1.18 of it (least where the chip's power is the limit), 128 x 192 0.87,
 // 128 x 128 0.69.  So 2531 rows x 3072 go in one round of 240 wide tiles (28.2 us; 480 narrow ones 30.4), 2048 in 256 of 192 columns
 // (23.8; wide 25.2), 1024 in 192 narrow ones (17.4; wide 23.5), 2531 x 16384 in 4 rounds of 160 rows (112; 5 of 128 rows 118).
-static void f8_tile_plan(const GemmF8P& p, bool silu, int& mb, int& nb) {
+static long f8_tile_plan(int M, int N, bool silu, int& mb, int& nb) {
   static const struct { int mb, nb, cost; } tiles[] = {{4, 4, 100}, {5, 4, 110}, {4, 3, 87}, {4, 2, 69}};
   const int n_cu = p3v_gemm256_cus(), pin = p3v_tuning().gemm_f8_narrow;
   long best = -1;
   for (const auto& t : tiles) {
     const int n_tile = silu ? 32 * t.nb : 64 * t.nb;
-    if (p.N % n_tile || (silu && t.nb % 2)) continue;
-    long c = (p3v_cdiv((long)(p.N / n_tile) * p3v_cdiv(p.M, 32 * t.mb), (long)max(n_cu, 1))) * t.cost;
+    if (N % n_tile || (silu && t.nb % 2)) continue;
+    long c = (p3v_cdiv((long)(N / n_tile) * p3v_cdiv(M, 32 * t.mb), (long)max(n_cu, 1))) * t.cost;
     if (pin == 10 * t.mb + t.nb || (pin == 0 && t.mb == 4 && t.nb == 4) || (pin == 1 && t.nb == 2)) c = 0;
     if (best < 0 || c < best) best = c, mb = t.mb, nb = t.nb;
   }
+  return best;
 }
 
 template <int EPI>
 static int launch_f8(const GemmF8P& p, hipStream_t s) {
   int mb = 0, nb = 0;
-  f8_tile_plan(p, EPI == P3V_EPI_SILU_MUL, mb, nb);
+  f8_tile_plan(p.M, p.N, EPI == P3V_EPI_SILU_MUL, mb, nb);
   if constexpr (EPI != P3V_EPI_SILU_MUL)
     if (nb == 3) return launch_f8_v<EPI, 4, 3>(p, s);
   if (nb == 2) return launch_f8_v<EPI, 4, 2>(p, s);
@@ -319,7 +382,7 @@ extern "C" int p3v_gemm_fp8(const p3v_gemm_fp8_args_t* a, void* stream) {
   const size_t w_rows = (size_t)a->N * (a->epilogue == P3V_EPI_SILU_MUL ? 2 : 1);
   if (w_rows * a->ldw >= ((size_t)1 << 32) || (size_t)256 * a->lda >= ((size_t)1 << 31)) return P3V_ERR_UNSUPPORTED;   // 32-bit buffer offsets
   if (a->M == 0) return P3V_OK;
-  const GemmF8P p = {a->A, a->a_scale, a->W, a->w_scale, a->out, a->resid, a->M, a->N, a->K, a->lda, a->ldw, a->ldo};
+  const GemmF8P p = {a->A, a->a_scale, a->W, a->w_scale, a->out, a->resid, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, {}};
   hipStream_t s = (hipStream_t)stream;
   switch (a->epilogue) {
     case P3V_EPI_NONE: return launch_f8<P3V_EPI_NONE>(p, s);
@@ -327,6 +390,36 @@ extern "C" int p3v_gemm_fp8(const p3v_gemm_fp8_args_t* a, void* stream) {
     case P3V_EPI_SILU_MUL: return launch_f8<P3V_EPI_SILU_MUL>(p, s);
     default: return P3V_ERR_ARG;
   }
+}
+
+// Whether one launch beats the two.  It writes and reads 47 MB less (2531 rows), but runs on 128 x 256 tiles alone and each of their rounds
+// is 4.1 us longer; rounds of 128 x 256 from f8_tile_plan's measurements, the split + rotation 2.5 us + 7.8 ns a row of 9216.  us, two :
+// one at K = 3072: 640 rows 29.2 : 27.0, 1300 53.3 : 48.4, 2531 85.6 : 77.2, 4096 130.7 : 123.0, 8192 273 : 226, but 256 20.4 : 23.7,
+// 1024 38.8 : 46.2 and 2048 68.6 : 72.3, where tiles of 160 rows fill their rounds.
+extern "C" int p3v_gemm_qkv_fp8_pays(int M, int n_q, int n_kv, int K) {
+  if (M <= 0 || K <= 0 || n_q <= 0 || n_kv <= 0 || n_q % 256 || n_kv % 256) return 0;
+  int mb, nb;
+  const int N = n_q + 2 * n_kv, n_cu = max(p3v_gemm256_cus(), 1);
+  const float round = 7.6f + 0.575f * (float)(K / TKB), rows = (float)M * (float)N;
+  const long tiles = (long)(n_q + n_kv) / 256 * p3v_cdiv(M, 128) + (long)n_kv / 128 * p3v_cdiv(M, 256);
+  return p3v_cdiv(tiles, (long)n_cu) * (round + 4.1f) < 0.01f * (float)f8_tile_plan(M, N, false, mb, nb) * round + 2.5f + 8.5e-7f * rows;
+}
+
+// p3v_gemm_fp8 (epilogue NONE) + p3v_rope_kv_append in one launch, bit for bit, on 128 x 256 tiles: the projection's 47 MB (2531 rows) are
+// neither written nor read again.
+extern "C" int p3v_gemm_qkv_fp8(const p3v_gemm_fp8_args_t* a, const p3v_qkv_split_t* sp, void* stream) {
+  if (!a || !sp || !a->A || !a->a_scale || !a->W || !a->w_scale || !sp->q_out || !sp->k_dst || !sp->v_dst || (!sp->cos_t) != (!sp->sin_t)) return P3V_ERR_ARG;
+  const int nh = sp->n_heads, nkv = sp->n_kv, hd = sp->hd;
+  if (sp->B <= 0 || sp->L <= 0 || nh <= 0 || nkv <= 0 || hd <= 0 || sp->tab_div <= 0 || !(sp->q_scale > 0.f) || a->epilogue != P3V_EPI_NONE) return P3V_ERR_ARG;
+  if (a->M != sp->B * sp->L || a->N != (nh + 2 * nkv) * hd || a->K <= 0 || a->K % TKB || a->lda < a->K || a->ldw < a->K || a->lda % 16 || a->ldw % 16) return P3V_ERR_ARG;
+  if (((uintptr_t)a->A | (uintptr_t)a->W | (uintptr_t)sp->q_out | (uintptr_t)sp->k_dst | (uintptr_t)sp->v_dst | (uintptr_t)sp->cos_t | (uintptr_t)sp->sin_t) & 15) return P3V_ERR_ARG;
+  const int dpos0 = sp->dst_off_is_past ? sp->past : 0;
+  if (hd % 32 || (hd / 2) % 16 || (nh * hd) % 256 || (nkv * hd) % 256 || dpos0 % 8 || sp->dst_t % 8 || p3v_tuning().gemm_no_qkv_fuse) return P3V_ERR_UNSUPPORTED;
+  if ((size_t)a->N * a->ldw >= ((size_t)1 << 32) || (size_t)a->M * a->lda >= ((size_t)1 << 32) || (size_t)256 * a->lda >= ((size_t)1 << 31) ||
+      (size_t)256 * a->ldw >= ((size_t)1 << 31)) return P3V_ERR_UNSUPPORTED;                                  // 32-bit buffer offsets
+  const GemmF8P p = {a->A, a->a_scale, a->W, a->w_scale, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0,
+                     {sp->cos_t, sp->sin_t, sp->q_out, sp->k_dst, sp->v_dst, sp->L, nh, nkv, hd, sp->past, dpos0, sp->dst_t, sp->tab_t, sp->tab_div, 0, sp->q_scale}};
+  return launch_f8_v<P3V_EPI_QKV, 4, 4>(p, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------- activation quantiser (one wave per token row)

@@ -503,6 +503,18 @@ class Phi3VModel(DecoderModel):
                     normed_in = True                            # (`h` holds the normalised input now, whatever the fused call answers)
                     fused_qkv = ops.gemm_qkv(hn, w[k_w], st.cos, st.sin, q, kd, vd, B, L, nh, nkv, hd, past, st.Tp, True, st.T, 1,
                                              q_scale=scale * ops.Q_PRESCALE)
+            f8_w = self.w8.get(k_w)                             # the same on e4m3 weights and quantised rows
+            if (f8_w is not None and L > ops.L.DECODE_MAX_L and n_beam == 1 and k_w not in self.adapters and not mlx4_first and self.fp8_act
+                    and ops.gemm_fp8_ok(M, f8_w[0].shape[0], cfg.hidden_size, EPI_NONE) and os.environ.get("P3V_QKV_FUSE", "1") != "0"
+                    and ops.gemm_qkv_fp8_pays(M, nh * hd, nkv * hd, cfg.hidden_size)
+                    and not (st.quantized and past > 0 and not getattr(st, "fresh_rows", False))):
+                kd, vd = (st.k_tmp, st.v_tmp) if st.quantized else (st.k[i], st.v[i])
+                a8, sa = ops.quant_fp8_rows(h if normed_in else x, None if normed_in else w[p + "input_layernorm.weight"], eps)
+                fused_qkv = True
+                if not ops.gemm_qkv_fp8(a8, sa, *f8_w, st.cos, st.sin, q, kd, vd, B, L, nh, nkv, hd, past, st.Tp, True, st.T, 1,
+                                        q_scale=scale * ops.Q_PRESCALE):
+                    ops.gemm_fp8(a8, sa, *f8_w, out=qkv)
+                    ops.rope_kv_append(qkv, st.cos, st.sin, q, kd, vd, B, L, nh, nkv, hd, past, st.Tp, True, st.T, 1, q_scale=scale * ops.Q_PRESCALE)
             if i == 0 and step_begin is not None:               # replayed greedy step: the embedding gather + rotation-row staging
                 sb = step_begin                                 # ride in this projection's prologue when the library takes the shape
                 w_fold = w.get(k_w) if k_w in w else (self.w8.get(k_w) or self.w4.get(k_w))   # bf16, (e4m3, row scales) or (4-bit, scale | bias)

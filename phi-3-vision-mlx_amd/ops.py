@@ -348,6 +348,29 @@ def gemm_qkv(a, w, cos_t, sin_t, q_out, k_dst, v_dst, B, Lq, nh, nkv, hd, past, 
     return True
 
 
+def gemm_qkv_fp8(a8, a_scale, w8, w_scale, cos_t, sin_t, q_out, k_dst, v_dst, B, Lq, nh, nkv, hd, past, dst_t, dst_off_is_past, tab_t=0,
+                 tab_div=1, q_scale=1.0):
+    """gemm_qkv on quantised rows and weights: gemm_fp8 + rope_kv_append in one launch, bit for bit.  Returns False -- nothing launched --
+    when the library does not take the shape: the caller then runs the two calls."""
+    _chk(a8, torch.uint8, "a8"), _chk(w8, torch.uint8, "w8"), _chk(a_scale, F32, "a_scale"), _chk(w_scale, F32, "w_scale")
+    M, K = a8.shape
+    if w8.shape[1] != K or a_scale.numel() < M or w_scale.numel() < w8.shape[0]:
+        raise ValueError(f"gemm_qkv_fp8: {tuple(a8.shape)} x {tuple(w8.shape)}, scales {a_scale.numel()} and {w_scale.numel()}")
+    g = L.GemmF8Args(_p(a8), _p(a_scale), _p(w8), _p(w_scale), 0, 0, M, w8.shape[0], K, a8.stride(0), w8.stride(0), w8.shape[0], EPI_NONE)
+    sp = L.QkvSplit(_p(cos_t), _p(sin_t), _p(q_out), _p(k_dst), _p(v_dst), B, Lq, nh, nkv, hd, int(past), dst_t, int(dst_off_is_past),
+                    tab_t, tab_div, float(q_scale))
+    rc = L.lib().p3v_gemm_qkv_fp8(C.byref(g), C.byref(sp), _stream())
+    if rc == L.ERR_UNSUPPORTED:
+        return False
+    L.check(rc, "gemm_qkv_fp8")
+    return True
+
+
+def gemm_qkv_fp8_pays(M, n_q, n_kv, K):
+    """Whether gemm_qkv_fp8 is faster than the two calls it stands for (n_q, n_kv: weight rows per region)."""
+    return bool(L.lib().p3v_gemm_qkv_fp8_pays(M, n_q, n_kv, K))
+
+
 Q_PRESCALE = 1.4426950408889634          # log2(e): q_scale = Q_PRESCALE * softmax scale for q_prescaled attention
 
 

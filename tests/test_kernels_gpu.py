@@ -887,6 +887,28 @@ def test_gemm_qkv_fused(ops, B, L, nh, nkv, hd, K, past, rot, bias, big):
     assert not torch.equal(k1, k0) and not torch.equal(v1, v0)
 
 
+@pytest.mark.parametrize("B,L,nh,nkv,hd,K,past,rot", [(1, 2531, 32, 32, 96, 256, 0, True), (1, 17, 8, 8, 96, 384, 64, True), (2, 128, 16, 4, 64, 128, 0, True),
+                                                     (3, 333, 16, 8, 96, 640, 8, True), (1, 257, 16, 16, 64, 128, 0, False), (5, 577, 8, 8, 96, 128, 0, True)])
+def test_gemm_qkv_fp8_fused(ops, B, L, nh, nkv, hd, K, past, rot):
+    """p3v_gemm_qkv_fp8 against p3v_gemm_fp8, then p3v_rope_kv_append: queries, K rows and V^T columns with the same bits, the rest of the
+    caches untouched; row counts at and next to the 128-row Q / K tiles and the 256-token V tiles, regions of different widths."""
+    M, N, T = B * L, (nh + 2 * nkv) * hd, past + L + 5
+    Tp = (T + 127) // 128 * 128
+    a8, sa = ops.quant_fp8_rows(g((M, K), 420).cuda(), None, 1e-5)
+    w8, sw = ops.quantize_fp8_rows(g((N, K), 421, 1.0 / math.sqrt(K)).cuda())
+    cos, sin = ((torch.rand((B, T, hd // 2), device="cuda"), torch.rand((B, T, hd // 2), device="cuda")) if rot else (None, None))
+    k0, v0 = g((B, nkv, Tp, hd), 423).cuda(), g((B, nkv, hd, Tp), 424).cuda()
+    q1, k1, v1 = torch.empty((B, nh, L, hd), dtype=BF16, device="cuda"), k0.clone(), v0.clone()
+    ops.rope_kv_append(ops.gemm_fp8(a8, sa, w8, sw), cos, sin, q1, k1, v1, B, L, nh, nkv, hd, past, Tp, True, T, 1, q_scale=1.3)
+    q2, k2, v2 = torch.full((B, nh, L, hd), 7.0, dtype=BF16, device="cuda"), k0.clone(), v0.clone()
+    assert ops.gemm_qkv_fp8(a8, sa, w8, sw, cos, sin, q2, k2, v2, B, L, nh, nkv, hd, past, Tp, True, T, 1, q_scale=1.3)
+    assert torch.equal(q2, q1) and torch.equal(k2, k1) and torch.equal(v2, v1)
+    assert not torch.equal(k1, k0) and not torch.equal(v1, v0)
+    # what the epilogue cannot place is declined, nothing written: an append offset that is not a multiple of 8
+    assert not ops.gemm_qkv_fp8(a8, sa, w8, sw, cos, sin, q2, k2, v2, B, L, nh, nkv, hd, past + 3, Tp, True, T, 1)
+    assert torch.equal(k2, k1) and torch.equal(v2, v1)
+
+
 def test_gemm_qkv_declines_what_it_cannot_fuse(ops):
     """Decode-sized inputs (<= 8 rows) and unaligned append offsets: P3V_ERR_UNSUPPORTED, nothing written."""
     nh, hd, K = 16, 64, 128
