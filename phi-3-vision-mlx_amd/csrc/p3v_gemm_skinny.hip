@@ -5,10 +5,9 @@
 // K-tile -- gate_up 34 us + 5 us for the reduction of the split it needs to reach 256 workgroups, 2.9 TB/s.  Here:
 //   tile      128(M) x 64(N) x 64(K): twice the workgroups per weight matrix, so gate_up (256 tiles) and qkv (144) run in one pass
 //             and the others with a smaller split over K (o_proj 4, down 4 slices: one workgroup per CU, partials <= a quarter of
-//             the weight bytes).  Every workgroup re-reads the A panel from L2: a launch stages W x 3 bytes, and the chip delivers
-//             ~9.7 TB/s of staged bytes in this pattern whether the weights are hot in L2 or not (144 and 256 workgroups both settle
-//             there) -- the kernel's bound; 128 x 128 tiles (W x 2 staged, half the workgroups) ran into the ~50 GB/s a single
-//             CU's DMA path takes instead and were not faster on any shape (the template keeps the variant).
+//             the weight bytes).  The kernel's bound: every workgroup re-reads the A panel from L2 beside its weight stream from
+//             HBM, and in one CU the two add up -- the same requests without any compute take 27.7 of gate_up's 30 us at 128 rows.
+//             128 x 128 tiles (W x 2 staged, half the workgroups) were not faster on any shape (the template keeps the variant).
 //   staging   LDS-DMA into a ring of 6 stages (A 16 KiB + W 8 KiB each), 5 in flight behind a counted vmcnt; one workgroup per CU
 //             (<= 64 rows: 64-row tiles, A 8 KiB per stage -- a third less staged per K-tile, the same sums bit for bit: 60 -> 53 us
 //             per decoder layer at 17 rows)
