@@ -301,6 +301,9 @@ int p3v_gemm256_qkv(const p3v_gemm_args_t* a, const QkvP& q, hipStream_t s) {
 
 // called by p3v_gemm (which decides how many rows get the big tile); returns P3V_ERR_UNSUPPORTED to fall back
 int p3v_gemm256_try(const p3v_gemm_args_t* a, int mb, int nb, hipStream_t s) {
+  // the tiles there are (the knob "gemm_tile" may ask for any); a gated epilogue needs whole gate / up pairs of a wave's four column blocks
+  const int tile = 10 * mb + nb;
+  if (tile != 84 && tile != 74 && tile != 54 && tile != 44 && (P3V_GATED(a->epilogue) || (tile != 83 && tile != 43))) return P3V_ERR_UNSUPPORTED;
   const int n_tile = P3V_GATED(a->epilogue) ? 32 * nb : 64 * nb;
   if (a->N % n_tile || a->K % TK || a->epilogue == P3V_EPI_PATCH) return P3V_ERR_UNSUPPORTED;
   const size_t w_rows = (size_t)a->N * (P3V_GATED(a->epilogue) ? 2 : 1);

@@ -138,6 +138,32 @@ def test_fused_decode_attention_role_placement_is_a_bijection(n_split, mode):
     assert l.p3v_attention_decode_fused_role(G, nh, n_split, o_n, mode, out) == -22
 
 
+@pytest.mark.parametrize("tile", [1, 4, 40, 53, 64, 73, 80, 82, 94, 99, 844, -84])
+def test_a_pinned_gemm_tile_that_does_not_exist_is_refused(tile):
+    """The knob "gemm_tile" takes any number: one that names no tile of the large GEMM kernels (or, gated, the 192-column ones) is an
+    error code, not a division by zero and not another tile.  Negative: no pin.  A process of its own, since the fault would end it."""
+    import subprocess
+    import sys
+    code = f"""
+import ctypes as C
+from phi_3_vision_mlx_amd import _lib as L, ops
+l, buf = L.lib(), C.create_string_buffer(4096)
+p = (C.addressof(buf) + 15) // 16 * 16
+def gemm(M, epilogue):
+    return l.p3v_gemm(C.byref(L.GemmArgs(p, p, p, 0, 0, 0, M, 768, 64, 64, 64, 768, epilogue, 0, 0, 0, 0)), None)
+for t, M in (({tile}, 64), (43, 64), (83, 64)):
+    assert l.p3v_set_tuning(b"gemm_tile", t) == 0
+    if t < 0:
+        assert gemm(0, ops.EPI_NONE) == 0
+    elif t not in (43, 83):
+        assert gemm(M, ops.EPI_NONE) == L.ERR_UNSUPPORTED, (t, gemm(M, ops.EPI_NONE))
+    if t > 0:
+        assert gemm(M, ops.EPI_SILU_MUL) == L.ERR_UNSUPPORTED and gemm(M, ops.EPI_GELU_MUL) == L.ERR_UNSUPPORTED, t
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.returncode, r.stderr[-1500:])
+
+
 def test_product_never_imports_the_oracle():
     pkg = os.path.join(ROOT, "phi-3-vision-mlx_amd")
     for dirpath, _, files in os.walk(pkg):
