@@ -692,9 +692,10 @@ def rms_rows(x, norm, out):
 
 
 def project_rms(x, norm, w, h, epilogue=EPI_NONE, out=None):
-    """project(rms_rows(x)): one launch for up to 8 bf16 rows of a width the streaming kernels take, else the two (h: their scratch rows)."""
+    """project(rms_rows(x)): one launch for up to 8 bf16 rows of a width the streaming kernels take, else the two (h: their scratch rows).
+    2 .. 8 rows: outputs that the one launch does not write (fp32, rows of a wider matrix) go through the two."""
     M, H = x.shape
-    if M <= 8 and h.dtype == BF16 and out is not None:
+    if h.dtype == BF16 and out is not None and (M == 1 or (M <= 8 and out.dtype == BF16 and out.is_contiguous())):
         _chk(x, F32, "x"), _chk(w, BF16, "w"), _chk(out, BF16, "out"), _chk(norm[0], BF16, "norm")
         N = w.shape[0] // 2 if epilogue in GATED else w.shape[0]
         if w.shape[1] != H or out.numel() != M * N or (M > 1 and tuple(out.shape) != (M, N)) or norm[0].numel() != H:

@@ -84,6 +84,20 @@ def test_rms_norm_in_the_projection_prologue_of_a_batch(M, N, K, gelu):
     assert torch.isnan(out[M].float()).all()
 
 
+@pytest.mark.parametrize("form", ["fp32", "rows of a wider matrix"])
+@pytest.mark.parametrize("M,N,K", [(2, 40, 1024), (8, 96, 3072)])
+def test_rms_norm_and_projection_into_outputs_of_the_two_launches(M, N, K, form):
+    """2 .. 8 rows into an output that the fused launch does not write: norm, then the projection; columns beside the output stay."""
+    from phi_3_vision_mlx_amd import ops
+    r, wide = np.random.default_rng(N), form != "fp32"
+    x, w, nw = r.normal(0, 3, (M, K)), bf(r.normal(0, K ** -0.5, (N, K))), bf(r.normal(1, 0.3, K))
+    xd, scratch = dev(x, F32), torch.empty((M, K), dtype=BF16, device=DEV)
+    out = torch.full((M, N + 8 if wide else N), float("nan"), dtype=BF16 if wide else F32, device=DEV)
+    ops.project_rms(xd, (dev(nw), 0.2, -0.7), dev(w), scratch, ops.EPI_NONE if wide else ops.EPI_F32, out=out[:, :N])
+    close(host(out[:, :N]), orc.rms(host(xd), nw, 0.2) * -0.7 @ w.T, BF16)
+    assert torch.isnan(out[:, N:].float()).all()
+
+
 @pytest.mark.parametrize("hidden,off", [(8, 0), (3072, 0), (3072, 1), (2049, 0), (4104, 0)])
 def test_embedding_rows_of_every_width_and_alignment(hidden, off):
     from phi_3_vision_mlx_amd import ops
