@@ -414,7 +414,8 @@ extern "C" int p3v_gemm_qkv_fp8(const p3v_gemm_fp8_args_t* a, const p3v_qkv_spli
   if (a->M != sp->B * sp->L || a->N != (nh + 2 * nkv) * hd || a->K <= 0 || a->K % TKB || a->lda < a->K || a->ldw < a->K || a->lda % 16 || a->ldw % 16) return P3V_ERR_ARG;
   if (((uintptr_t)a->A | (uintptr_t)a->W | (uintptr_t)sp->q_out | (uintptr_t)sp->k_dst | (uintptr_t)sp->v_dst | (uintptr_t)sp->cos_t | (uintptr_t)sp->sin_t) & 15) return P3V_ERR_ARG;
   const int dpos0 = sp->dst_off_is_past ? sp->past : 0;
-  if (hd % 32 || (hd / 2) % 16 || (nh * hd) % 256 || (nkv * hd) % 256 || dpos0 % 8 || sp->dst_t % 8 || p3v_tuning().gemm_no_qkv_fuse) return P3V_ERR_UNSUPPORTED;
+  if (hd % 32 || (hd / 2) % 16 || (nh * hd) % 256 || (nkv * hd) % 256 || dpos0 % 8 || sp->dst_t % 8 || !qkv_rows_ok(sp->B, sp->L) ||
+      p3v_tuning().gemm_no_qkv_fuse) return P3V_ERR_UNSUPPORTED;
   if ((size_t)a->N * a->ldw >= ((size_t)1 << 32) || (size_t)a->M * a->lda >= ((size_t)1 << 32) || (size_t)256 * a->lda >= ((size_t)1 << 31) ||
       (size_t)256 * a->ldw >= ((size_t)1 << 31)) return P3V_ERR_UNSUPPORTED;                                  // 32-bit buffer offsets
   const GemmF8P p = {a->A, a->a_scale, a->W, a->w_scale, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0,

@@ -23,6 +23,10 @@ struct QkvP {
   float q_scale;
 };
 
+// The V^T epilogue stores runs of eight tokens, which may cross the end of ONE batch row: several rows of fewer than 7 tokens do not fit
+// (the run's last token would need two or more steps), and the launchers decline them.
+static inline bool qkv_rows_ok(int B, int L) { return B == 1 || L >= 7; }
+
 // W row fetched for tile column `rr` (0 .. tile width - 1) of a Q / K tile whose first pair is p0; row0 = first W row of the region
 __device__ __forceinline__ int qkv_pair_row(const QkvP& q, int row0, int p0, int rr) {
   const int half = q.hd >> 1;

@@ -164,6 +164,22 @@ for t, M in (({tile}, 64), (43, 64), (83, 64)):
     assert r.returncode == 0, (r.returncode, r.stderr[-1500:])
 
 
+def test_fused_qkv_projections_decline_several_rows_of_fewer_than_seven_tokens():
+    """The V^T epilogue's runs of eight tokens cross the end of one batch row at most.  Everything else about these calls is taken, so
+    the answer comes from that check (no kernel starts: declined on the host)."""
+    from phi_3_vision_mlx_amd import _lib as L, ops
+    l = L.lib()
+    buf = ctypes.create_string_buffer(4096)
+    p = (ctypes.addressof(buf) + 15) // 16 * 16
+    hd, nh, K = 64, 16, 128
+    N = 3 * nh * hd
+    for B, Lq in ((5, 3), (30, 6), (2, 1), (300, 4), (180, 6)):
+        M = B * Lq
+        sp = L.QkvSplit(0, 0, p, p, p, B, Lq, nh, nh, hd, 0, 128, 1, 0, 1, 1.0)
+        assert l.p3v_gemm_qkv(ctypes.byref(L.GemmArgs(p, p, 0, 0, 0, 0, M, N, K, K, K, N, ops.EPI_NONE, 0, 0, 0, 0)), ctypes.byref(sp), None) == L.ERR_UNSUPPORTED
+        assert l.p3v_gemm_qkv_fp8(ctypes.byref(L.GemmF8Args(p, p, p, p, 0, 0, M, N, K, K, K, N, ops.EPI_NONE)), ctypes.byref(sp), None) == L.ERR_UNSUPPORTED
+
+
 def test_product_never_imports_the_oracle():
     pkg = os.path.join(ROOT, "phi-3-vision-mlx_amd")
     for dirpath, _, files in os.walk(pkg):

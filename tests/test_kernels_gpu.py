@@ -855,6 +855,7 @@ def test_gemm_tiles_agree(ops, epi, M, N, K):
     # across row ends
     (17, 577, 16, 16, 64, 1024, 0, False, True, -1), (5, 577, 16, 16, 64, 128, 0, False, True, 0), (3, 1001, 8, 4, 96, 128, 0, True, False, -1),
     (4, 61, 16, 16, 64, 128, 0, False, False, -1), (3, 85, 8, 4, 96, 192, 0, True, False, -1),
+    (20, 7, 16, 16, 64, 128, 0, True, False, -1), (150, 7, 16, 16, 64, 128, 8, True, False, -1),      # the shortest rows of a batch
 ])
 def test_gemm_qkv_fused(ops, B, L, nh, nkv, hd, K, past, rot, bias, big):
     """p3v_gemm_qkv (qkv projection with head split + rotation + KV append in its epilogue) against the two calls it replaces --
@@ -888,7 +889,8 @@ def test_gemm_qkv_fused(ops, B, L, nh, nkv, hd, K, past, rot, bias, big):
 
 
 @pytest.mark.parametrize("B,L,nh,nkv,hd,K,past,rot", [(1, 2531, 32, 32, 96, 256, 0, True), (1, 17, 8, 8, 96, 384, 64, True), (2, 128, 16, 4, 64, 128, 0, True),
-                                                     (3, 333, 16, 8, 96, 640, 8, True), (1, 257, 16, 16, 64, 128, 0, False), (5, 577, 8, 8, 96, 128, 0, True)])
+                                                     (3, 333, 16, 8, 96, 640, 8, True), (1, 257, 16, 16, 64, 128, 0, False), (5, 577, 8, 8, 96, 128, 0, True),
+                                                     (37, 7, 16, 16, 64, 128, 8, True), (1, 3, 16, 16, 64, 128, 0, True)])
 def test_gemm_qkv_fp8_fused(ops, B, L, nh, nkv, hd, K, past, rot):
     """p3v_gemm_qkv_fp8 against p3v_gemm_fp8, then p3v_rope_kv_append: queries, K rows and V^T columns with the same bits, the rest of the
     caches untouched; row counts at and next to the 128-row Q / K tiles and the 256-token V tiles, regions of different widths."""
