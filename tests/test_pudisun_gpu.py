@@ -98,7 +98,7 @@ def test_rms_norm_and_projection_into_outputs_of_the_two_launches(M, N, K, form)
     assert torch.isnan(out[:, N:].float()).all()
 
 
-@pytest.mark.parametrize("hidden,off", [(8, 0), (3072, 0), (3072, 1), (2049, 0), (4104, 0)])
+@pytest.mark.parametrize("hidden,off", [(8, 0), (3072, 0), (3072, 1), (2049, 0), (4104, 0), (12, 0), (2052, 4), (3072, 2)])
 def test_embedding_rows_of_every_width_and_alignment(hidden, off):
     from phi_3_vision_mlx_amd import ops
     ids = torch.tensor([3, -1, 9, 99], dtype=torch.int32, device=DEV)
