@@ -275,6 +275,9 @@ int p3v_attention_decode(const p3v_attn_decode_args_t* args /* host */, void* st
  * residual in ONE launch (merge_in_launch = 1, the 128-key one-tile plan); 2 (round 6) = merge_in_launch = 0: the launch that merges
  * the split-KV partials also carries the o_proj + residual (long contexts, 64-key plans) -- same arguments, same bits. */
 int p3v_attention_decode_can_fuse_oproj(int B, int L, int n_heads, int hd, int n_split, int cache_t, int o_n, int merge_in_launch);
+/* 1: p3v_attention_decode (without o_proj_w) runs this shape as one workgroup per (row, head), without split partials (host query; the
+ * rule is about time: the results of the two forms differ by rounding) */
+int p3v_attention_decode_rows_fit(int B, int L, int n_heads, int n_kv, int cache_t);
 /* Which role workgroup `wg` of the fused launch's 1-D grid (n_heads * n_split workgroups) plays under placement `map` (the
  * attn_fo_map tuning knob: 2 = default, 1 = the round's first form): out[0] = key split, out[1] = head, out[2] / out[3] = its
  * projection units (rows [8 u, 8 u + 8) of o_proj; -1 = none).  Split n_split - 1 of a head is its merging workgroup.  Workgroups

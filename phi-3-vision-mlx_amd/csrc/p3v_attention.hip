@@ -2897,15 +2897,28 @@ extern "C" int p3v_attention_decode_fused_role(int wg, int n_heads, int n_split,
   return P3V_OK;
 }
 
-// (row, head) pairs that go one to a workgroup (k_attn_decode_rows), by pairs and cache capacity.  us against the split forms, 32 heads:
-//   short caches, from half a chip of pairs on: 4 rows x 128 5.4 : 6.0, 8 x 256 9.1 : 10.9, 16 x 256 14.9 : 17.9
-//   longer ones only where every CU gets the same number of pairs, a CU's share being what it waits for: 8 rows x 576 14.4 : 15.7,
-//   16 x 576 25.8 : 26.6, but 12 x 576 22.7 : 20.8; past ~640 keys the split forms' 64-key lines win (16 x 832 34.9 : 33.9)
-static bool attn_rows_fit(int pairs, int cache_t) {
+// (row, head) pairs that go one to a workgroup (k_attn_decode_rows), by pairs and cache capacity.  us against the split forms, 32 heads, full
+// caches of rows of the same length (the split forms' best case; with caches a third full they are 1.1-1.6x behind everywhere below 256):
+//   short caches, from half a chip of pairs on: 4 rows x 128 5.9 : 6.1, 8 x 256 9.1 : 11.3, 16 x 256 13.7 : 18.2
+//   longer ones only where every CU gets the same number of pairs, a CU's share being what it waits for: 8 rows x 576 13.1 : 15.8,
+//   16 x 576 21.2 : 26.3, but 12 x 576 22.7 : 20.8; past ~640 keys the split forms' 64-key lines win (16 x 832 34.9 : 33.9)
+// One new token a row, 129 .. 256 keys: a second round of pairs for less than half of the CUs costs more than it gives up to 192 (9 rows
+// 10.4 : 9.3, 10 10.6 : 9.7; 12 10.8 : 10.7, 9 x 256 11.8 : 12.3), and with shared kv heads, whose keys and values the split forms' neighbours
+// find in the L2, an uneven share does (8 kv heads: 4 x 256 7.9 : 7.1, 6 x 256 8.5 : 8.1, 9 x 192 11.0 : 9.7, 12 x 192 11.4 : 10.9; but 8 x 256
+// 9.3 : 9.4, 14 x 192 11.6 : 12.0).
+// Several new tokens a row: the split forms write and merge a partial for each (4 tokens, 9 x 192 10.7 : 15.4).
+static bool attn_rows_fit(int pairs, int grp, int L, int cache_t) {
   const int pin = p3v_tuning().attn_rows;
   if (pin >= 0) return pin != 0;
   const int idle = (pairs + 255) / 256 * 256 - pairs;           // CUs without a pair in the last round over the chip's 256
-  return pairs >= 128 && pairs <= 512 && (cache_t <= 256 || (cache_t <= 640 && idle <= 64));
+  if (pairs < 128 || pairs > 512) return false;
+  if (cache_t > 256) return cache_t <= 640 && idle <= 64;
+  if (cache_t <= 128 || L > 1) return true;
+  return grp > 1 ? 6 * idle <= pairs : cache_t > 192 || idle <= 128;
+}
+extern "C" int p3v_attention_decode_rows_fit(int B, int L, int n_heads, int n_kv, int cache_t) {
+  if (B <= 0 || L <= 0 || n_heads <= 0 || n_kv <= 0 || n_heads % n_kv || cache_t <= 0) return 0;
+  return attn_rows_fit(B * n_heads, n_heads / n_kv, L, cache_t);
 }
 
 extern "C" int p3v_attention_decode(const p3v_attn_decode_args_t* a, void* stream) {
@@ -2940,7 +2953,7 @@ extern "C" int p3v_attention_decode(const p3v_attn_decode_args_t* a, void* strea
     P3V_CHECK_LAUNCH();
     return P3V_OK;
   }
-  if (!a->o_proj_w && attn_rows_fit(a->B * a->n_heads, a->cache_t)) {
+  if (!a->o_proj_w && attn_rows_fit(a->B * a->n_heads, grp, a->L, a->cache_t)) {
     hipLaunchKernelGGL(k_attn_decode_rows, dim3(a->n_heads, a->B), dim3(256), 0, s, p);
     P3V_CHECK_LAUNCH();
     return P3V_OK;

@@ -164,6 +164,19 @@ for t, M in (({tile}, 64), (43, 64), (83, 64)):
     assert r.returncode == 0, (r.returncode, r.stderr[-1500:])
 
 
+def test_which_decode_batches_run_one_workgroup_per_row_and_head():
+    """(rows, new tokens, heads, kv heads, capacity) where the form was measured faster, and where it was not: an uneven second round
+    of pairs, shared kv heads, few pairs, long caches."""
+    from phi_3_vision_mlx_amd import _lib
+    fit = _lib.lib().p3v_attention_decode_rows_fit
+    for yes in ((4, 1, 32, 32, 128), (4, 1, 32, 32, 192), (8, 1, 32, 32, 192), (12, 1, 32, 32, 192), (16, 1, 32, 32, 256), (9, 1, 32, 32, 256), (9, 4, 32, 32, 192),
+                (15, 1, 32, 32, 640), (6, 1, 32, 32, 512), (8, 1, 32, 8, 256), (9, 1, 32, 8, 128), (14, 1, 32, 8, 192), (16, 16, 32, 32, 256), (32, 1, 16, 16, 192)):
+        assert fit(*yes) == 1, yes
+    for no in ((9, 1, 32, 32, 192), (10, 1, 32, 32, 192), (11, 1, 32, 32, 192), (4, 1, 32, 8, 256), (6, 1, 32, 8, 256), (9, 1, 32, 8, 192), (9, 1, 32, 8, 256), (12, 1, 32, 8, 192),
+               (12, 1, 32, 32, 576), (4, 1, 32, 32, 320), (3, 1, 32, 32, 128), (17, 1, 32, 32, 128), (8, 1, 32, 32, 704), (0, 1, 32, 32, 128), (4, 1, 32, 0, 128), (4, 1, 32, 5, 128)):
+        assert fit(*no) == 0, no
+
+
 def test_fused_qkv_projections_decline_several_rows_of_fewer_than_seven_tokens():
     """The V^T epilogue's runs of eight tokens cross the end of one batch row at most.  Everything else about these calls is taken, so
     the answer comes from that check (no kernel starts: declined on the host)."""
