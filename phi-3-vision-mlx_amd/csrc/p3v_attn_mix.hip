@@ -66,13 +66,14 @@ __host__ __device__ static inline int mix_q_first(int past, int T) { const int d
 __host__ __device__ static inline int mix_q_count(int past, int L, int T) {
   return T > ((past + L - 1) >> 5) + 1 ? 0 : ((L + 15) >> 4) - mix_q_first(past, T);
 }
-// Run number `wid` in the order of the runs' lengths: the full ones split by split, then the partial ones by decreasing length -- with a
-// workgroup per CU, long runs that start late are what the last CUs wait for (2048 rows: 18 tiles' time instead of 23 - 27).
+// Run number `wid`.  With more runs than CUs in the order of their lengths: the full ones split by split, then the partial ones by
+// decreasing length -- long runs that start late are what the last CUs wait for (2048 rows: 18 tiles' time instead of 23 - 27).  Else split by
+// split, which takes 2 us less to find out.
 struct MixRun { int qt, split, b; };
 __device__ __forceinline__ MixRun mix_run(int wid, const AttnMixP& p) {
   const int per = p.tiles_per_split, n_qt = (p.L + 15) >> 4;
   for (int s = 0; s < p.n_split; ++s) {
-    const int n = p.B * mix_q_count(p.past, p.L, (s + 1) * per);
+    const int n = p.B * mix_q_count(p.past, p.L, p.by_length ? (s + 1) * per : s * per + 1);
     if (wid < n) return {n_qt - 1 - wid / p.B, s, wid % p.B};
     wid -= n;
   }
@@ -110,7 +111,7 @@ __global__ void __launch_bounds__(512, 1) k_attn_mix_prefill(AttnMixP p) {
   float* MM = AL + C::HM * 256;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lc = lane & 15, lg = lane >> 4;
   MixRun run = {((p.L + 15) >> 4) - 1 - (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z};             // longest rows first
-  if (p.by_size) run = mix_run(blockIdx.x, p);
+  if (p.runs) run = mix_run(blockIdx.x, p);
   if (run.qt < 0) return;
   const int qt = run.qt, split = run.split, b = run.b;
   const int q0 = qt * 16, per = p.H / p.G, past = p.d_past ? *p.d_past : p.past, first = p.pad_len ? p.pad_len[b] : 0;
@@ -642,16 +643,55 @@ static bool mix_fast(int H, int G, int dim, int vdim, int f32) {
   return !f32 && H <= MIX_MAX_H && dim <= 128 && vdim <= 128;
 }
 
-// Prompts: key tiles of a run.  A CU's share of all of them: with the runs in order of length the launch then lasts about that long.
-// Not below 4 (what a run costs besides its tiles), at most MIX_MAX_ROW_SPLIT runs a query tile.
-// A prompt in 8 layers, us, against equal parts for about 320 workgroups in their plain order: 2048 tokens 5168 -> 5110, 2500 7340 -> 6685,
-// 3000 7999 -> 7770, 4096 11797 -> 11300, 512 and 1500 alike.  (At 2048 the attention itself 184 -> 170 us, where the longest CU's tiles
-// go from 22 to 17: with every CU busy a tile takes longer, its 393 KB of keys and values come out of the L2s at 10.7 TB/s.)
+// When the last run of a prompt's, cut into runs of up to `per` key tiles, is done, in the time of a key tile.  The runs start by decreasing
+// length; run i goes to shader engine i % MIX_ENGINES (XCD by XCD, then engine by engine in them) and waits for its first free CU.  The first
+// engine has the longest of every MIX_ENGINES runs, and a run too many before the others: its end is the launch's.  MIX_RUN_FIXED: what a run
+// costs besides its tiles.  (With one pool of CUs instead of engines the cut chosen by it was up to 1.2x behind the best, with these within 3 %.)
+#define MIX_CUS 256
+#define MIX_ENGINES 32
+#define MIX_RUN_FIXED 2
+#define MIX_PLAN_TILES 4096            // longest key range that is looked at in this detail
+static int mix_runs_end(int B, int L, int past, int per, int cus) {
+  int by_length[MIX_PLAN_TILES + 1], free_at[128] = {}, end = 0;
+  for (int i = 0; i <= per; ++i) by_length[i] = 0;
+  for (int q = 0; q < L; q += 16) {
+    const int t = ((past + min(q + 15, L - 1)) >> 5) + 1;
+    by_length[per] += t / per * B;
+    if (t % per) by_length[t % per] += B;
+  }
+  const int n = min(max(cus / MIX_ENGINES, 1), 128);
+  for (int len = per, i = 0, up_to = 0; len > 0; --len)
+    for (up_to += by_length[len]; i < up_to; i += MIX_ENGINES) {
+      int c = 0;
+      for (int k = 1; k < n; ++k) c = free_at[k] < free_at[c] ? k : c;
+      free_at[c] += len + MIX_RUN_FIXED;
+      end = max(end, free_at[c]);
+    }
+  return end;
+}
+// Prompts: key tiles of a run, of the cuts into equal parts and some lengths from a CU's share of all tiles on, not below 4: the one whose last
+// CU is done first, a tile's time for the merge and a fifth for each partial a row of it reads.  A launch of a few more runs than CUs is what costs:
+// 2 x 700 rows in runs of 4 tiles are 288 for 256 CUs, in runs of 5 240 (32 heads x 96, 8 kv heads: 74.4 : 60.6 us).  Prompts of two and more
+// query tiles a CU stay whole.  us of the attention of 32 heads x 96, against equal parts for about 320 workgroups in their plain order:
+// 700 rows 77 -> 73, 1500 146 -> 125, 2048 208 -> 184, 2500 362 -> 253, 4096 674 -> 593, 1000 behind 6000 593 -> 435; none of 176 shapes of 17 ..
+// 8192 rows, 1 .. 8 sequences, 0 .. 6000 keys before and four head layouts slower by more than the runs differ.
 static int mix_run_tiles(int B, int L, int past) {
+  const int tiles = ((past + L - 1) >> 5) + 1, want = p3v_tuning().mix_wgs, cus = want > 0 ? min(want, 4096) : MIX_CUS;
+  const long qt = (long)p3v_cdiv(L, 16) * B;
+  if (qt >= 2L * cus) return tiles;
+  if (tiles > MIX_PLAN_TILES) return p3v_cdiv(tiles, min(max(cus / qt, 1L), (long)MIX_MAX_ROW_SPLIT));
   long sum = 0;
   for (int q = 0; q < L; q += 16) sum += ((past + min(q + 15, L - 1)) >> 5) + 1;
-  const int want = p3v_tuning().mix_wgs;
-  return max(max(4, p3v_cdiv(sum * B, want > 0 ? want : 256)), p3v_cdiv(((past + L - 1) >> 5) + 1, MIX_MAX_ROW_SPLIT));
+  const int share = max(max(4, p3v_cdiv(sum * B, cus)), p3v_cdiv(tiles, MIX_MAX_ROW_SPLIT)), step = max(1, share / 20);
+  int best = tiles;
+  float best_end = (float)mix_runs_end(B, L, past, tiles, cus);
+  for (int i = 2; i < MIX_MAX_ROW_SPLIT + 9; ++i) {
+    const int per = i <= MIX_MAX_ROW_SPLIT ? p3v_cdiv(tiles, i) : share + (i - MIX_MAX_ROW_SPLIT - 1) * step;
+    if (per < 4 || 4 * per < 3 * share || per >= tiles) continue;
+    const float end = (float)mix_runs_end(B, L, past, per, cus) + 1.f + 0.2f * (float)p3v_cdiv(tiles, per);
+    if (end < best_end) best_end = end, best = per;
+  }
+  return best;
 }
 
 extern "C" int p3v_attn_mix_plan(int B, int L, int H, int G, int dim, int vdim, int n_keys, int f32) {
@@ -661,7 +701,7 @@ extern "C" int p3v_attn_mix_plan(int B, int L, int H, int G, int dim, int vdim, 
     const int tiles = p3v_cdiv(n_keys, 16), per = p3v_cdiv(tiles, max(1, (want > 0 ? want : 256) / B));
     return min(p3v_cdiv(tiles, per), MIX_MAX_SPLIT);
   }
-  return p3v_cdiv(p3v_cdiv(n_keys, 32), mix_run_tiles(B, L, n_keys - L));
+  return p3v_cdiv(p3v_cdiv(max(n_keys, L), 32), mix_run_tiles(B, L, max(n_keys - L, 0)));
 }
 
 extern "C" int64_t p3v_attn_mix_ws_bytes(int B, int L, int H, int vdim, int n_split) {
@@ -684,11 +724,7 @@ static int launch_prefill(const AttnMixP& p, hipStream_t s) {
     attr_set = true;
   }
   dim3 grid(p3v_cdiv(p.L, 16), p.n_split, p.B);
-  if (p.by_size) {
-    int runs = 0;
-    for (int sp = 0; sp < p.n_split; ++sp) runs += p.B * mix_q_count(p.past, p.L, sp * p.tiles_per_split + 1);
-    grid = dim3(runs);
-  }
+  if (p.runs) grid = dim3(p.runs);
   hipLaunchKernelGGL((k_attn_mix_prefill<HW, DC, VC, SHARED>), grid, dim3(512), MixCfg<HW>::LDS, s, p);
   P3V_CHECK_LAUNCH();
   return p.n_split > 1 ? mix_combine(p, s) : P3V_OK;
@@ -723,8 +759,14 @@ extern "C" int p3v_attn_mix(const p3v_mix_args_t* a, void* stream) {
   // (the position may be a device value: the splits then cover the capacity)
   const int tiles = p3v_cdiv(a->d_past ? a->Tp : a->past + a->L, 32);
   p.tiles_per_split = p3v_cdiv(tiles, a->n_split);
-  p.by_size = !a->d_past && a->n_split > 1;
-  if (const int per = mix_run_tiles(a->B, a->L, a->past); p.by_size && p3v_cdiv(tiles, per) == a->n_split) p.tiles_per_split = per;   // as planned
+  if (!a->d_past && a->n_split > 1)
+    if (const int per = mix_run_tiles(a->B, a->L, a->past); p3v_cdiv(tiles, per) == a->n_split) p.tiles_per_split = per;   // as planned
+  // (query tile, split) pairs for more than the CUs, some of them without keys to see: the runs alone (with empty pairs between them they
+  // crowd on some CUs: 900 rows in 8 parts 75 : 98 us)
+  if (!a->d_past && a->n_split > 1 && (long)p3v_cdiv(a->L, 16) * a->n_split * a->B > MIX_CUS) {
+    for (int sp = 0; sp < p.n_split; ++sp) p.runs += p.B * mix_q_count(p.past, p.L, sp * p.tiles_per_split + 1);
+    p.by_length = p.runs > MIX_CUS;
+  }
   if (p.n_split > 1 && p.L == 1) return P3V_ERR_ARG;                     // (k_attn_mix_combine's splits are 16-key tiles)
   const int per = p.H / p.G;                                             // query heads of a key / value head
   if (p.H <= 8) return prefill_dc<1, true>(p, s);

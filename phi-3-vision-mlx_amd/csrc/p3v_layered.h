@@ -75,11 +75,11 @@ struct AttnMixP {
   const void* q; const void* k; const void* v; const bf16_t* talk; const bf16_t* sink; const void* gate; void* out; float* ws;
   const int32_t* pad_len; const int32_t* d_past;
   float scale; int B, L, H, G, dim, vdim, dimp, vdimp, ld, past, Tp, n_split, tiles_per_split;
-  int by_size;                                                           // prompts: workgroups in the order of their runs' lengths (mix_run)
+  int runs, by_length;                                                   // prompts: 0, or a workgroup for each of so many runs (mix_run), longest first
 };
 static inline AttnMixP attn_mix_params(const p3v_mix_args_t* a) {
   return {a->q, a->k, a->v, a->talk, a->sink, a->gate, a->out, a->ws, a->pad_len, a->d_past, a->scale,
-          a->B, a->L, a->H, a->G, a->dim, a->vdim, a->dimp, a->vdimp, a->ld, a->past, a->Tp, a->n_split, 0, 0};
+          a->B, a->L, a->H, a->G, a->dim, a->vdim, a->dimp, a->vdimp, a->ld, a->past, a->Tp, a->n_split, 0, 0, 0};
 }
 
 int p3v_dyt_check(const p3v_dyt_args_t* a);

@@ -203,6 +203,11 @@ def test_launch_planning_and_struct_layouts():
     l = _lib.lib()
     assert l.p3v_attn_mix_plan(1, 1, 32, 8, 96, 96, 2176, 0) == 136 and l.p3v_attn_mix_plan(1, 1, 32, 8, 96, 96, 8320, 0) <= 260
     assert l.p3v_attn_mix_plan(8, 1, 32, 8, 96, 96, 2176, 0) <= 32 and l.p3v_attn_mix_plan(1, 4096, 32, 8, 96, 96, 4096, 0) in range(1, 17)
+    # prompts: parts whose runs do not spill a few over the chip's CUs (2 x 700 rows in 6 parts are 288 runs for 256), whole where two tiles follow four
+    for B, L, past, want in ((1, 130, 0, 1), (2, 700, 0, 5), (1, 1200, 0, 6), (1, 2048, 0, 4), (1, 2500, 0, 3), (1, 1000, 6000, 5), (1, 8192, 0, 1), (64, 500, 0, 1),
+                             (1, 17, 131000, 16), (1, 17, 10 ** 7, 16), (1, 4000, 10 ** 6, 1), (1, 1, 0, 1)):
+        got = l.p3v_attn_mix_plan(B, L, 32, 8, 96, 96, past + L, 0)
+        assert got == want, (B, L, past, got)
     for bad in ((1, 1, 33, 11, 96, 96, 100, 0), (1, 1, 8, 8, 160, 96, 100, 0), (1, 1, 8, 8, 96, 96, 100, 1), (0, 1, 8, 8, 96, 96, 100, 0)):
         assert l.p3v_attn_mix_plan(*bad) == 0                    # the any-size kernel
     assert l.p3v_attn_mix_ws_bytes(2, 3, 4, 10, 5) == 2 * 3 * 5 * 4 * 12 * 4

@@ -305,7 +305,8 @@ def test_mixed_attention_key_splits(H, G, dim, vdim, n_split):
         close(got[:, 0], np.stack(want), BF16)
 
 
-@pytest.mark.parametrize("B,L,past,pads", [(1, 16, 300, None), (1, 700, 0, None), (2, 333, 31, [0, 40]), (3, 1025, 0, [0, 64, 1000]), (1, 1500, 545, [7])])
+@pytest.mark.parametrize("B,L,past,pads", [(1, 16, 300, None), (1, 700, 0, None), (2, 333, 31, [0, 40]), (3, 1025, 0, [0, 64, 1000]), (1, 1500, 545, [7]),
+                                              (1, 2048, 0, None), (2, 1200, 3, [5, 700])])
 def test_mixed_attention_runs_by_length(B, L, past, pads):
     """The planned runs, in their order of length (whole and partial ones, several rows, a position inside a tile), give the rows of one
     run per query tile; the same runs in their plain order (the position on the device) too.  All three sum the same fp32 terms."""
