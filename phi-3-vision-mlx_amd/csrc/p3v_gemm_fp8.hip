@@ -15,7 +15,8 @@
 //             threads: 8 CONSUMER waves as 2(M) x 4(N), ONE MFMA per 16 x 16 block and K-tile, and 4 PRODUCER waves that only
 //             request K-tiles by LDS-DMA (as p3v_gemm_pc.hip): rows of 128 BYTES, 16-byte chunk c of row r stored at chunk
 //             c ^ (r & 7), swizzled on the source address; three buffers of a K-tile (four from 128 x 192 down: what 160 KiB
-//             hold), so a request has two or three K-tiles' time to land.
+//             hold), so a request has two or three K-tiles' time to land.  256 x 256 tiles on eight waves that do both, where only they fill a
+//             round (k_gemm_f8_tall).
 //             What bounds it: the producers' requests, ~60 ns per round of four 1-KiB pieces (a K-tile of 128 x 256 takes 0.69 us
 //             where its MFMAs take 0.43), and, with all CUs at it, the chip's power: the same launches on all-zero operands are
 //             20-25 % faster.  Against the form it replaced (256-row tiles, eight waves that request and multiply, two buffers and a
@@ -46,6 +47,73 @@ struct TileF8 { int a_off[8], b_off[8]; __amdgpu_buffer_rsrc_t rs_a, rs_b; };   
 
 #define F8_BUF(mb, nb) ((32 * (mb) + 64 * (nb)) * TKB)
 #define F8_STAGES(mb, nb) (160 * 1024 / F8_BUF(mb, nb) < 4 ? 160 * 1024 / F8_BUF(mb, nb) : 4)
+
+// A wave's 16 MB x 16 NB sums at rows mrow0 - fc .., outputs from column nw on, straight from the accumulators: lane (fc = lane & 15, fq = lane >> 4)
+// holds columns 4 fq .. 4 fq + 3 of block row fc; lanes q and q ^ 1 trade packed halves of two neighbouring column blocks: 16-byte stores.
+template <int EPI, int MB, int NB>
+__device__ __forceinline__ void f8_epilogue(const GemmF8P& p, const f32x4_t (&acc)[MB][NB], int mrow0, int nw, int fq) {
+  constexpr bool SILU = EPI == P3V_EPI_SILU_MUL;
+  constexpr int HB = SILU ? NB / 2 : NB;                           // column blocks of outputs of a wave
+  float sc[NB][4];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int n = SILU ? nw + j % HB * 16 + fq * 4 + j / HB * p.N : nw + j * 16 + fq * 4;
+    const f32x4_a4 c = *(const f32x4_a4*)(p.sw + n);
+    sc[j][0] = c[0], sc[j][1] = c[1], sc[j][2] = c[2], sc[j][3] = c[3];
+  }
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+    const int m = mrow0 + i * 16;
+    const float s = p.sa[min(m, p.M - 1)];
+    uint32_t pk[HB][2];
+#pragma unroll
+    for (int j = 0; j < HB; ++j) {
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v[r] = acc[i][j][r] * (s * sc[j][r]);
+        if (SILU) {
+          // gate / up are bf16 Linear outputs, every elementwise op after them rounds to bf16 (phi.py:469-471)
+          const float g = bf16_round(v[r]), u = bf16_round(acc[i][(HB + j) % NB][r] * (s * sc[(HB + j) % NB][r]));
+          v[r] = bf16_round(g * bf16_round(1.f / (1.f + __expf(-g)))) * u;
+        }
+      }
+      pk[j][0] = pack_bf16x2(v[0], v[1]), pk[j][1] = pack_bf16x2(v[2], v[3]);
+    }
+#pragma unroll
+    for (int jp = 0; jp < HB / 2; ++jp) {
+      u32x4_t w;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        auto sw = __builtin_amdgcn_permlane16_swap(pk[2 * jp][k], pk[2 * jp + 1][k], false, false);
+        w[k] = sw[0], w[2 + k] = sw[1];
+      }
+      const int n = nw + (2 * jp + (fq & 1)) * 16 + (fq >> 1) * 8;
+      if (m < p.M) {
+        const size_t o = (size_t)m * p.ldo + n;
+        if (EPI == P3V_EPI_RESID_BF16) {
+          const u32x4_t rw = *(const u32x4_t*)(p.resid + o);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) w[k] = pack_bf16x2(bf16lo(rw[k]) + bf16lo(w[k]), bf16hi(rw[k]) + bf16hi(w[k]));
+        }
+        *(u32x4_t*)(p.out + o) = w;
+      }
+    }
+    if (HB & 1) {                                     // the block without a partner: four columns, 8 bytes
+      const int n = nw + (HB - 1) * 16 + fq * 4;
+      if (m < p.M) {
+        const size_t o = (size_t)m * p.ldo + n;
+        u32x2_t w = {pk[HB - 1][0], pk[HB - 1][1]};
+        if (EPI == P3V_EPI_RESID_BF16) {
+          const u32x2_t rw = *(const u32x2_t*)(p.resid + o);
+#pragma unroll
+          for (int k = 0; k < 2; ++k) w[k] = pack_bf16x2(bf16lo(rw[k]) + bf16lo(w[k]), bf16hi(rw[k]) + bf16hi(w[k]));
+        }
+        *(u32x2_t*)(p.out + o) = w;
+      }
+    }
+  }
+}
 
 // MB, NB: 16-row / 16-column blocks of a consumer wave (2 x 4 waves: a tile of 32 MB rows x 64 NB columns)
 template <int EPI, int MB, int NB>
@@ -219,8 +287,6 @@ __global__ void __launch_bounds__(768, 1) k_gemm_f8(GemmF8P p) {
       slot = nslot;
     }
 
-    // ---- epilogue, straight from the accumulators: lane (fc = lane & 15, fq = lane >> 4) holds columns 4 fq .. 4 fq + 3 of block row fc;
-    // lanes q and q ^ 1 trade packed halves of two neighbouring column blocks: 16-byte stores (p3v_gemm256_epi.h)
     const int fc = lane & 15, fq = lane >> 4;
     if constexpr (QKV) {                                           // the same products of sum and scales, then p3v_gemm_qkv's epilogues
       if (at.swapped) {
@@ -262,70 +328,116 @@ __global__ void __launch_bounds__(768, 1) k_gemm_f8(GemmF8P p) {
       }
       continue;
     }
-    const int mrow0 = m0 + wr * MB * 16 + fc, nw = n0 + wc * (n_out_tile / 4);
-    float sc[NB][4];
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      const int n = SILU ? nw + j % HB * 16 + fq * 4 + j / HB * p.N : nw + j * 16 + fq * 4;
-      const f32x4_a4 c = *(const f32x4_a4*)(p.sw + n);
-      sc[j][0] = c[0], sc[j][1] = c[1], sc[j][2] = c[2], sc[j][3] = c[3];
-    }
-#pragma unroll
-    for (int i = 0; i < MB; ++i) {
-      const int m = mrow0 + i * 16;
-      const float s = p.sa[min(m, p.M - 1)];
-      uint32_t pk[HB][2];
-#pragma unroll
-      for (int j = 0; j < HB; ++j) {
-        float v[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          v[r] = acc[i][j][r] * (s * sc[j][r]);
-          if (SILU) {
-            // gate / up are bf16 Linear outputs, every elementwise op after them rounds to bf16 (phi.py:469-471)
-            const float g = bf16_round(v[r]), u = bf16_round(acc[i][(HB + j) % NB][r] * (s * sc[(HB + j) % NB][r]));
-            v[r] = bf16_round(g * bf16_round(1.f / (1.f + __expf(-g)))) * u;
-          }
-        }
-        pk[j][0] = pack_bf16x2(v[0], v[1]), pk[j][1] = pack_bf16x2(v[2], v[3]);
-      }
-#pragma unroll
-      for (int jp = 0; jp < HB / 2; ++jp) {
-        u32x4_t w;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          auto sw = __builtin_amdgcn_permlane16_swap(pk[2 * jp][k], pk[2 * jp + 1][k], false, false);
-          w[k] = sw[0], w[2 + k] = sw[1];
-        }
-        const int n = nw + (2 * jp + (fq & 1)) * 16 + (fq >> 1) * 8;
-        if (m < p.M) {
-          const size_t o = (size_t)m * p.ldo + n;
-          if (EPI == P3V_EPI_RESID_BF16) {
-            const u32x4_t rw = *(const u32x4_t*)(p.resid + o);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) w[k] = pack_bf16x2(bf16lo(rw[k]) + bf16lo(w[k]), bf16hi(rw[k]) + bf16hi(w[k]));
-          }
-          *(u32x4_t*)(p.out + o) = w;
-        }
-      }
-      if (HB & 1) {                                     // the block without a partner: four columns, 8 bytes
-        const int n = nw + (HB - 1) * 16 + fq * 4;
-        if (m < p.M) {
-          const size_t o = (size_t)m * p.ldo + n;
-          u32x2_t w = {pk[HB - 1][0], pk[HB - 1][1]};
-          if (EPI == P3V_EPI_RESID_BF16) {
-            const u32x2_t rw = *(const u32x2_t*)(p.resid + o);
-#pragma unroll
-            for (int k = 0; k < 2; ++k) w[k] = pack_bf16x2(bf16lo(rw[k]) + bf16lo(w[k]), bf16hi(rw[k]) + bf16hi(w[k]));
-          }
-          *(u32x2_t*)(p.out + o) = w;
-        }
-      }
-    }
+    f8_epilogue<EPI, MB, NB>(p, acc, m0 + wr * MB * 16 + fc, n0 + wc * (n_out_tile / 4), fq);
   }
 }
 
+// 256 x 256 tiles for the sizes whose rounds only they fill (16 column tiles x 16 row tiles and the like): eight waves as 2(M) x 4(N) that request and
+// multiply, two LDS buffers, a full wait and barrier per K-tile, one tile per workgroup.  Two thirds of the flat tiles' staged bytes per
+// product, but the requests stand in front of the MFMAs.  us, against 128 x 256: 4500 x 3072 x 3072 44.5 : 47.6, 4500 x 3072 x 8192 94 : 98,
+// 1700 x 9216 x 3072 41.8 : 44.1, gate | up of 900 rows 45.6 : 47.1.
+struct OffF8 { int a[2][2], b[2][2]; __amdgpu_buffer_rsrc_t rs_a, rs_w; };
+template <int EPI>
+__global__ void __launch_bounds__(512, 1) k_gemm_f8_tall(GemmF8P p) {
+  constexpr bool SILU = EPI == P3V_EPI_SILU_MUL;
+  constexpr int TM = 256, TN = 256, n_out_tile = SILU ? TN / 2 : TN, HALF_BYTES = 128 * TKB, BUF_BYTES = 4 * HALF_BYTES;    // A0 A1 B0 B1
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave >> 2, wc = wave & 3;
+  const int gx = p.N / n_out_tile, gy = (p.M + TM - 1) / TM, nwg = gx * gy;
+  int m0, n0;
+  {   // XCD-aware order, as above
+    const int wid = blockIdx.x, q = nwg >> 3, r = nwg & 7, xcd = wid & 7, loc = wid >> 3;
+    const int id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + loc;
+    constexpr int BAND = 4;
+    const int band = id / (BAND * gx), in_band = id % (BAND * gx), rows = min(BAND, gy - band * BAND);
+    m0 = (band * BAND + in_band % rows) * TM, n0 = in_band / rows * n_out_tile;
+  }
+  OffF8 t;      // (declared outside the template: see TileF8's use)
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int rr = h * 128 + q * 64 + (tid >> 3), sw = ((tid & 7) ^ (rr & 7)) * 16, in = rr & 63;
+      const int br = SILU ? n0 + (rr >> 6) * 32 + (in & 31) + (in >> 5) * p.N : n0 + rr;       // (SiLU: 32 gate rows + the 32 up rows of the same outputs)
+      t.a[h][q] = (min(m0 + rr, p.M - 1) - m0) * p.lda + sw;
+      t.b[h][q] = (int)((unsigned)br * (unsigned)p.ldw + (unsigned)sw);
+    }
+  t.rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + (size_t)m0 * p.lda), 0, 0xffffffff, 0x00020000);
+  t.rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, 0xffffffff, 0x00020000);
+  auto dma = [&](bool b_side, int kt, int buf) {                  // both halves of one operand's K-tile
+    unsigned char* base = smem + buf * BUF_BYTES + (b_side ? 2 : 0) * HALF_BYTES + wave * 1024;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        lptr_t dst = (lptr_t)(base + h * HALF_BYTES + q * 8192);
+        const int vo = b_side ? t.b[h][q] : t.a[h][q];
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(b_side ? t.rs_w : t.rs_a, dst, 16, vo, kt * TKB, 0, 0);
+      }
+  };
+  f32x4_t acc[8][4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  const int frow = lane & 15, fchunk = lane >> 4, nk = p.K / TKB;
+  const int fo0 = frow * 128 + ((fchunk ^ (frow & 7)) << 4), fo1 = frow * 128 + (((4 + fchunk) ^ (frow & 7)) << 4);      // (as above)
+  dma(false, 0, 0);
+  dma(true, 0, 0);
+  for (int kt = 0; kt < nk; ++kt) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    const unsigned char* ta = smem + (kt & 1) * BUF_BYTES + wr * HALF_BYTES;
+    const unsigned char* tb = smem + (kt & 1) * BUF_BYTES + 2 * HALF_BYTES + wc * 64 * 128;
+    const bool more = kt + 1 < nk;
+    i32x8_t fa[4], fa1[4], fb[2], fb1[2];
+    auto read = [&](const unsigned char* base, auto& f) {
+#pragma unroll
+      for (int i = 0; i < (int)(sizeof(f) / sizeof(f[0])); ++i) {
+        const u32x4_t lo = *(const u32x4_t*)(base + i * 2048 + fo0), hi = *(const u32x4_t*)(base + i * 2048 + fo1);
+        f[i] = (i32x8_t){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+      }
+    };
+    auto quad = [&](int i0, int j0, auto& a, auto& b) {            // (W fragment first: the block comes out TRANSPOSED)
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i0 + i][j0 + j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b[j], a[i], acc[i0 + i][j0 + j], 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
+      __builtin_amdgcn_s_setprio(0);
+    };
+    read(tb, fb);                                                  // fragments of a quadrant are requested ahead of the MFMAs in front of it
+    read(ta, fa);
+    if (more) dma(false, kt + 1, (kt + 1) & 1);
+    read(tb + 2 * 2048, fb1);
+    __builtin_amdgcn_sched_barrier(0);
+    quad(0, 0, fa, fb);
+    __builtin_amdgcn_sched_barrier(0);
+    read(ta + 4 * 2048, fa1);
+    if (more) dma(true, kt + 1, (kt + 1) & 1);
+    __builtin_amdgcn_sched_barrier(0);
+    quad(0, 2, fa, fb1);
+    __builtin_amdgcn_sched_barrier(0);
+    quad(4, 2, fa1, fb1);
+    quad(4, 0, fa1, fb);
+  }
+  f8_epilogue<EPI, 8, 4>(p, acc, m0 + wr * 128 + frow, n0 + wc * (n_out_tile / 4), fchunk);
+}
 int p3v_gemm256_cus();                                             // p3v_gemm256.hip
+
+template <int EPI>
+static int launch_f8_tall(const GemmF8P& p, hipStream_t s) {
+  constexpr int LDS = 2 * F8_BUF(8, 4);
+  static bool attr_set = false;
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)k_gemm_f8_tall<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return P3V_ERR_HIP;
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(k_gemm_f8_tall<EPI>, dim3(p.N / (EPI == P3V_EPI_SILU_MUL ? 128 : 256) * p3v_cdiv(p.M, 256)), dim3(512), LDS, s, p);
+  P3V_CHECK_LAUNCH();
+  return P3V_OK;
+}
 
 template <int EPI, int MB, int NB>
 static int launch_f8_v(const GemmF8P& p, hipStream_t s) {
@@ -344,12 +456,14 @@ static int launch_f8_v(const GemmF8P& p, hipStream_t s) {
   return P3V_OK;
 }
 
-// the tile whose rounds over the chip cost least.  A round's cost by tile, 128 x 256 = 100, measured over M 256 .. 8192 and the
-// decoder's four projections: 160 x 256 takes 1.02-1.18 of it (least where the chip's power is the limit), 128 x 192 0.87,
-// 128 x 128 0.69.  So 2531 rows x 3072 go in one round of 240 wide tiles (28.2 us; 480 narrow ones 30.4), 2048 in 256 of 192 columns
-// (23.8; wide 25.2), 1024 in 192 narrow ones (17.4; wide 23.5), 2531 x 16384 in 4 rounds of 160 rows (112; 5 of 128 rows 118).
+// the tile whose rounds over the chip cost least.  A round's cost by tile, 128 x 256 = 100, measured over M 17 .. 16000 and the decoder's
+// four projections: 160 x 256 takes 1.02-1.18 of it (least where the chip's power is the limit), 128 x 192 0.87, 128 x 128 0.69, 256 x 256
+// 1.65-1.95 (counted as 1.94, where its round replaces two).  So 2531 rows x 3072 go in one round of 240 wide tiles (27.0 us; 480 narrow ones
+// 29.8), 2048 in 256 of 192 columns (23.8; wide 25.7), 1024 in 192 narrow ones (18.0; wide 24.7), 2531 x 16384 in 4 rounds of 160 rows (108; 5 of
+// 128 rows 110), 1700 x 9216 in one of 252 tall tiles (41.8; 160 rows 46.6).  The choice is within 2 % of the best tile there but at 4500 and 6800 x
+// 9216 and 4500 x 16384 (3 - 5 %).
 static long f8_tile_plan(int M, int N, bool silu, int& mb, int& nb) {
-  static const struct { int mb, nb, cost; } tiles[] = {{4, 4, 100}, {5, 4, 110}, {4, 3, 87}, {4, 2, 69}};
+  static const struct { int mb, nb, cost; } tiles[] = {{4, 4, 100}, {5, 4, 110}, {4, 3, 87}, {4, 2, 69}, {8, 4, 194}};
   const int n_cu = p3v_gemm256_cus(), pin = p3v_tuning().gemm_f8_narrow;
   long best = -1;
   for (const auto& t : tiles) {
@@ -369,6 +483,7 @@ static int launch_f8(const GemmF8P& p, hipStream_t s) {
   if constexpr (EPI != P3V_EPI_SILU_MUL)
     if (nb == 3) return launch_f8_v<EPI, 4, 3>(p, s);
   if (nb == 2) return launch_f8_v<EPI, 4, 2>(p, s);
+  if (mb == 8) return launch_f8_tall<EPI>(p, s);
   return mb == 5 ? launch_f8_v<EPI, 5, 4>(p, s) : launch_f8_v<EPI, 4, 4>(p, s);
 }
 

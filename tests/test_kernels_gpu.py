@@ -1641,13 +1641,13 @@ def test_gemm_fp8_tiles_agree(ops, request, epi, M, N, K):
     old = ops.set_tuning("gemm_f8_narrow", -1)
     request.addfinalizer(lambda: ops.set_tuning("gemm_f8_narrow", old))
     outs = []
-    for tile in (-1, 44, 54, 43, 42):                            # (a tile that does not divide N falls back to the choice by shape)
+    for tile in (-1, 44, 54, 43, 42, 84):                        # (a tile that does not divide N falls back to the choice by shape)
         ops.set_tuning("gemm_f8_narrow", tile)
         out = torch.full((M + 1, N), float("nan"), dtype=BF16).cuda()                # (a guard row behind the last one)
         ops.gemm_fp8(*dev, EPI, resid=None if resid is None else resid.cuda(), out=out)
         assert torch.isnan(out[M].float()).all(), tile
         outs.append(out[:M].clone())
-    for tile, out in zip((44, 54, 43, 42), outs[1:]):
+    for tile, out in zip((44, 54, 43, 42, 84), outs[1:]):
         assert torch.equal(out.view(torch.int16), outs[0].view(torch.int16)), tile
     y = (a8.view(torch.float8_e4m3fn).double() * sa[:, None].double()) @ (w8.view(torch.float8_e4m3fn).double() * sw[:, None].double()).t()
     if epi == "silu":
