@@ -352,17 +352,19 @@ static int gemm_big_rows(const p3v_gemm_args_t* a) {
 // Which tile runs the whole problem in one launch (*mb, *nb: a tile of 32 mb x 64 nb), or false: the packing above (or 128 x 128 tiles).
 // A launch lasts whole rounds of the chip's workgroups, so what counts is how a tile height divides the rows: 2531 x 3072 is 120
 // tiles of 256 x 256 (half the chip idle) but 240 of 128 x 256.  Times of one round in us, K-tiles of 64 = t, fitted to M = 1100 .. 9809 x
-// the decoder's and the vision tower's projections (every choice within 4 % of the best tile there): the flat tiles of
-// p3v_gemm_pc.hip 6.6 + 0.69 t (128 x 256), 7.9 + 0.79 t (160 x 256), 5.5 + 0.61 t (128 x 192); the tall ones of p3v_gemm256.hip
-// 9.5 + 1.28 t (256 x 256), 8.2 + 1.20 t (224 x 256), 8.1 + 1.11 t (256 x 192), a twentieth more per K-tile from the second round on (power);
-// 512 tiles of 128 x 128 6.0 + 0.785 t, up to 256 of them 4.4 + 0.635 t.  A tile has to promise 5 %; short K loops (< 1024) stay.
+// the decoder's and the vision tower's projections: the flat tiles of p3v_gemm_pc.hip 6.6 + 0.69 t (128 x 256), 7.9 + 0.79 t (160 x 256),
+// 5.5 + 0.61 t (128 x 192); the tall ones of p3v_gemm256.hip 9.5 + 1.28 t (256 x 256), 8.2 + 1.27 t (224 x 256), 8.1 + 1.11 t (256 x 192), a
+// twentieth more per K-tile from the second round on (power); 512 tiles of 128 x 128 6.0 + 0.785 t, up to 256 of them 4.4 + 0.635 t.  A tile
+// has to promise 5 %; short K loops (< 1024) stay.  The fit is for full rounds: of the sizes measured (profiles/gemm_tile_plan_sweep.txt) no choice
+// is slower than the packing by more than the runs differ; some are not the fastest tile, most of all below 1300 rows, where rounds of less
+// than 160 workgroups are faster than the fit says (1154 x 3072 x 8192 95, 128 x 192 69).
 // Measured (us, before -> now): 2531 x 3072 x 8192 117 -> 105, 2048 x 9472 x 3072 114 -> 97, 9809 x 1024 x 4096 (+ fp32 residual) 95 -> 73,
 // 4096 x 3072 x 8192 174 -> 163, 640 x 16384 x 3072 (gate | up) 103 -> 58.
 static bool gemm_tile_plan(const p3v_gemm_args_t* a, int rows_big, int* mb, int* nb) {
   const bool gated = P3V_GATED(a->epilogue);
   if (a->M <= 256 || a->K < 1024 || a->epilogue == P3V_EPI_PATCH || p3v_tuning().gemm_128 || p3v_tuning().gemm_big_rows >= 0) return false;
   struct Tile { int mb, nb; float f, c, more; };
-  static const Tile tiles[] = {{8, 4, 9.5f, 1.285f, 0.07f}, {7, 4, 8.2f, 1.20f, 0.03f}, {8, 3, 8.1f, 1.106f, 0.f},
+  static const Tile tiles[] = {{8, 4, 9.5f, 1.285f, 0.07f}, {7, 4, 8.2f, 1.27f, 0.03f}, {8, 3, 8.1f, 1.106f, 0.f},
                                {5, 4, 7.9f, 0.79f, 0.05f},  {4, 4, 6.6f, 0.69f, 0.05f}, {4, 3, 5.5f, 0.61f, 0.f}};
   const float kt = (float)(a->K / BK);
   auto time = [&](const Tile& t, int M) {
@@ -382,6 +384,14 @@ static bool gemm_tile_plan(const p3v_gemm_args_t* a, int rows_big, int* mb, int*
     if (c < best) { best = c; *mb = t.mb; *nb = t.nb; found = true; }
   }
   return found;
+}
+
+extern "C" int p3v_gemm_plan(int M, int N, int K, int epilogue) {
+  if (M <= 0 || N <= 0 || K <= 0 || epilogue < 0 || epilogue > P3V_EPI_GELU_MUL) return 0;
+  p3v_gemm_args_t a = {};
+  a.M = M, a.N = N, a.K = K, a.epilogue = epilogue;
+  int mb, nb;
+  return gemm_tile_plan(&a, p3v_tuning().gemm_128 ? 0 : gemm_big_rows(&a), &mb, &nb) ? 10 * mb + nb : 0;
 }
 
 // ---- split-K for prompt-sized-but-small M (17 .. 256 rows: short chat prompts, the text group of a mixed batch).  One

@@ -164,6 +164,24 @@ for t, M in (({tile}, 64), (43, 64), (83, 64)):
     assert r.returncode == 0, (r.returncode, r.stderr[-1500:])
 
 
+def test_which_tile_runs_a_prompt_sized_projection():
+    """One size for every tile, and sizes that stay on the row packing: where no tile promises enough, 224-row tiles for one full round
+    (slower than 256 x 256 there), short K loops, few rows."""
+    from phi_3_vision_mlx_amd import _lib, ops
+    l, v = _lib.lib(), ctypes.c_int()
+    assert l.p3v_get_tuning(b"gemm_big_rows", ctypes.byref(v)) == 0 and l.p3v_set_tuning(b"gemm_big_rows", -1) == 0
+    try:
+        for M, N, K, epi, want in ((2531, 3072, 8192, ops.EPI_RESID_BF16, 44), (640, 8192, 3072, ops.EPI_SILU_MUL, 54), (1300, 3072, 3072, ops.EPI_NONE, 43),
+                                   (900, 8192, 3072, ops.EPI_SILU_MUL, 84), (700, 8192, 3072, ops.EPI_GELU_MUL, 74), (1237, 9216, 3072, ops.EPI_NONE, 83),
+                                   (2885, 4096, 1024, ops.EPI_BIAS_QGELU, 74), (9809, 1024, 4096, ops.EPI_BIAS_RESID_F32, 54),
+                                   (1500, 9216, 3072, ops.EPI_NONE, 0), (1024, 9472, 3072, ops.EPI_NONE, 0), (1300, 8192, 3072, ops.EPI_SILU_MUL, 0),
+                                   (2531, 3072, 512, ops.EPI_NONE, 0), (256, 8192, 3072, ops.EPI_NONE, 0), (2531, 3000, 3072, ops.EPI_NONE, 0),
+                                   (2531, 1024, 1024, ops.EPI_PATCH, 0), (0, 3072, 3072, ops.EPI_NONE, 0), (2531, 3072, 3072, 99, 0)):
+            assert l.p3v_gemm_plan(M, N, K, epi) == want, (M, N, K, epi, l.p3v_gemm_plan(M, N, K, epi))
+    finally:
+        l.p3v_set_tuning(b"gemm_big_rows", v.value)
+
+
 def test_which_decode_batches_run_one_workgroup_per_row_and_head():
     """(rows, new tokens, heads, kv heads, capacity) where the form was measured faster, and where it was not: an uneven second round
     of pairs, shared kv heads, few pairs, long caches."""
