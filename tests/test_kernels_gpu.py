@@ -818,7 +818,7 @@ def test_merge_launch_with_fused_oproj_under_grouped_queries(ops):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 768, 64), (129, 768, 128), (257, 3072, 1024), (1111, 768, 192), (4001, 3072, 128), (2300, 9216, 64)])
-@pytest.mark.parametrize("epi", ["none", "silu", "gelu", "resid_bf16", "resid_f32", "scale"])
+@pytest.mark.parametrize("epi", ["none", "silu", "gelu", "resid_bf16", "resid_f32", "scale", "bias", "bias_qgelu", "bias_gelu", "f32"])
 def test_gemm_tiles_agree(ops, epi, M, N, K):
     """Every tile of the large GEMM kernels (one and several rounds of the chip, fewer K-tiles than LDS buffers, ragged last rows) against
     the 128 x 128 tiles: the same products in the same order, bit for bit."""
@@ -826,7 +826,8 @@ def test_gemm_tiles_agree(ops, epi, M, N, K):
     a, w = g((M, K), 40).cuda(), g((2 * N if gated else N, K), 41, 1.0 / math.sqrt(K)).cuda()
     v, r = g((N,), 42, 0.5).cuda(), g((M, N), 43, 1.0, BF16 if epi == "resid_bf16" else F32).cuda()
     kw = {"none": {}, "silu": dict(epilogue=ops.EPI_SILU_MUL), "gelu": dict(epilogue=ops.EPI_GELU_MUL), "resid_bf16": dict(epilogue=ops.EPI_RESID_BF16, resid=r),
-          "resid_f32": dict(epilogue=ops.EPI_BIAS_RESID_F32, resid=r, bias=v), "scale": dict(epilogue=ops.EPI_SCALE_RESID_F32, resid=r, col_scale=v)}[epi]
+          "resid_f32": dict(epilogue=ops.EPI_BIAS_RESID_F32, resid=r, bias=v), "scale": dict(epilogue=ops.EPI_SCALE_RESID_F32, resid=r, col_scale=v), "bias": dict(epilogue=ops.EPI_BIAS, bias=v),
+          "bias_qgelu": dict(epilogue=ops.EPI_BIAS_QGELU, bias=v), "bias_gelu": dict(epilogue=ops.EPI_BIAS_GELU, bias=v), "f32": dict(epilogue=ops.EPI_F32)}[epi]
     names = ("gemm_tile", "gemm_128", "gemm_no_skinny", "gemm_no_splitk")
     saved = [ops.set_tuning(n, x) for n, x in zip(names, (-1, 1, 1, 1))]
     try:
@@ -839,6 +840,46 @@ def test_gemm_tiles_agree(ops, epi, M, N, K):
     finally:
         for n, x in zip(names, saved):
             ops.set_tuning(n, x)
+
+
+@pytest.mark.parametrize("M,N,K,gated,tile", [(385, 9216, 1024, False, 43), (641, 9216, 2048, False, 44), (257, 6144, 2048, True, 44), (1300, 6144, 1024, False, 54),
+                                              (385, 9216, 1024, True, 54), (1300, 9216, 1024, False, 74), (500, 9216, 1024, True, 74), (1793, 6144, 1024, False, 83),
+                                              (700, 9216, 1024, True, 84)])
+def test_gemm_runs_the_planned_tile(ops, M, N, K, gated, tile):
+    """The launcher's own choice (no pin) for one size of every tile and kind of epilogue, against the 128 x 128 tiles bit for bit."""
+    epi = ops.EPI_SILU_MUL if gated else ops.EPI_BIAS_QGELU
+    a, w, v = g((M, K), 44).cuda(), g((2 * N if gated else N, K), 45, 1.0 / math.sqrt(K)).cuda(), g((N,), 46, 0.5).cuda()
+    kw = {} if gated else dict(bias=v)
+    saved = ops.set_tuning("gemm_big_rows", -1), ops.set_tuning("gemm_128", 0)
+    try:
+        assert ops.L.lib().p3v_gemm_plan(M, N, K, epi) == tile
+        got = ops.gemm(a, w, epi, **kw)
+        ops.set_tuning("gemm_128", 1)
+        assert torch.equal(got, ops.gemm(a, w, epi, **kw))
+    finally:
+        ops.set_tuning("gemm_big_rows", saved[0]), ops.set_tuning("gemm_128", saved[1])
+
+
+@pytest.mark.parametrize("n", [700, 1300, 2531])
+def test_prompt_on_planned_tiles_gives_the_row_packings_bits(ops, n):
+    """A prompt of the decoder's own widths (two layers) with the tiles the launcher plans -- the tests' default pins the row packing -- and
+    with 128 x 128 tiles alone: logits and the layers' caches bit for bit."""
+    from phi_3_vision_mlx_amd.api import load_synthetic
+    from phi_3_vision_mlx_amd.config import phi3v_config_dict
+    model, _ = load_synthetic(blind_model=True, config={**phi3v_config_dict(vision=False), "num_hidden_layers": 2}, seed=3)
+    ids = np.random.default_rng(n).integers(3, 32000, (1, n))
+    cfg, l = model.cfg, ops.L.lib()
+    saved = ops.set_tuning("gemm_big_rows", -1), ops.set_tuning("gemm_128", 0)
+    try:
+        assert any(l.p3v_gemm_plan(n, N, K, e) for N, K, e in ((cfg.hidden_size, cfg.hidden_size, ops.EPI_RESID_BF16), (cfg.intermediate_size, cfg.hidden_size, ops.EPI_SILU_MUL),
+                                                                (cfg.hidden_size, cfg.intermediate_size, ops.EPI_RESID_BF16)))
+        got, cache = model(input_ids=ids, max_tokens=4)
+        got, k, v = got.clone(), cache[0].state.k[..., :n, :].clone(), cache[0].state.v[..., :n].clone()
+        ops.set_tuning("gemm_128", 1)
+        want, cache = model(input_ids=ids, max_tokens=4)
+        assert torch.equal(got, want) and torch.equal(k, cache[0].state.k[..., :n, :]) and torch.equal(v, cache[0].state.v[..., :n])
+    finally:
+        ops.set_tuning("gemm_big_rows", saved[0]), ops.set_tuning("gemm_128", saved[1])
 
 
 @pytest.mark.parametrize("B,L,nh,nkv,hd,K,past,rot,bias,big", [
@@ -991,8 +1032,9 @@ def test_kv_quantize_mlx4_keys_from_exact_fp32_rotation(ops):
 @pytest.mark.parametrize("dev_past", [False, True])
 def test_attention_decode_rows(ops, request, B, L, past, T, nh, nkv, pads, dev_past):
     """One workgroup per (row, head) against the split form: lengths at and next to a 32-key tile and a wave's turn (128 keys), new
-    rows on both sides of a tile and up to the capacity's last key, shared kv heads, padding that ends inside, at and one short of the
-    last key; the caches must come out with the same bits.  Both round P to bf16 (2^-9) against different maxima, then the output."""
+    rows on both sides of a tile and up to the capacity's last key, shared kv heads, padding; the caches must come out with the same bits.
+    Both round P to bf16 (2^-9) against different maxima, then the output: a bound on values, in which a single key of a long row is not
+    seen (the next test's business)."""
     hd = 96
     qkv, kc, vc = g((B * L, (nh + 2 * nkv) * hd), 70), g((B, nkv, T, hd), 71), g((B, nkv, hd, T), 72)
     torch.manual_seed(7)
@@ -1012,6 +1054,65 @@ def test_attention_decode_rows(ops, request, B, L, past, T, nh, nkv, pads, dev_p
         res.append((out, k, v))
     assert torch.equal(res[0][1], res[1][1]) and torch.equal(res[0][2], res[1][2])
     close(res[1][0], res[0][0], rtol=2 ** -8, atol=2 * 2 ** -9 * vc.float().abs().max().item())
+
+
+@pytest.mark.parametrize("B,L,past,T,nh,nkv,pads", [(1, 1, 0, 64, 2, 2, None), (3, 1, 33, 64, 4, 2, [0, 32, 33]), (1, 16, 120, 192, 2, 1, None), (2, 5, 251, 256, 4, 1, [0, 250]),
+                                                    (2, 3, 509, 512, 2, 2, [3, 255]), (2, 1, 575, 576, 2, 2, [0, 64]), (3, 4, 600, 640, 2, 2, [0, 31, 599]),
+                                                    (4, 1, 700, 832, 2, 2, [0, 64, 699, 700])])
+def test_attention_decode_rows_at_every_edge_key(ops, request, B, L, past, T, nh, nkv, pads):
+    """One key decides the output of its (row, kv head): the first and the last of every 32-key tile, those around the padding's end, the
+    newest cached one, every new one (for its own query and for the query before it), the first behind the last.  Its score is 16 above the
+    others' scale, so one dropped or wrongly visible key moves the output by the size of the values, at every length; checked in
+    float64, on keys and queries rounded to bf16 as they are stored.  The kernel rounds P and the output to bf16: 2^-8 of the largest value."""
+    hd, grp, alpha = 96, nh // nkv, 16.0
+    half, scale, pad_of = hd // 2, hd ** -0.5, pads or [0] * B
+    qkv0, kc0, vc = g((B * L, (nh + 2 * nkv) * hd), 80), g((B, nkv, T, hd), 81), g((B, nkv, hd, T), 82)
+    gen = torch.Generator().manual_seed(83)
+    cos, sin = torch.rand((B, L, half), generator=gen) + 0.2, torch.rand((B, L, half), generator=gen)
+    bf64 = lambda x: x.to(BF16).double()
+    rot = lambda x, c, s: torch.cat([x[..., :half] * c - x[..., half:] * s, x[..., half:] * c + x[..., :half] * s], -1)
+    unrot = lambda y, c, s: torch.cat([y[..., :half] * c + y[..., half:] * s, y[..., half:] * c - y[..., :half] * s], -1) / (c * c + s * s).repeat(2)
+    c64, s64 = cos.double(), sin.double()
+
+    def edges(pad):
+        at = {t + e for t in range(0, past, 32) for e in (0, 31)} | {pad - 1, pad, pad + 1, past - 1}
+        got = [(t, L - 1) for t in sorted(at) if 0 <= t < past] + [(past + r, i) for r in range(L) for i in (r, r - 1) if i >= 0]
+        return [e for e in got + [(t, L - 1) for t in {past + L, (past + L) | 31} if t < T] if past + e[1] >= pad]
+    todo = [[edges(pad_of[b])[h::nkv] for h in range(nkv)] for b in range(B)]
+    old = ops.set_tuning("attn_rows", 1)
+    request.addfinalizer(lambda: ops.set_tuning("attn_rows", old))
+    pad = None if pads is None else torch.tensor(pads, dtype=torch.int32).cuda()
+    ws = ops.attention_ws(B, L, nh, hd, 1, "cuda")
+    for n in range(max(len(e) for row in todo for e in row)):
+        x, kc, want, decisive = qkv0.view(B, L, nh + 2 * nkv, hd).clone(), kc0.clone(), torch.zeros((B, L, nh, hd), dtype=torch.float64), 0
+        for b in range(B):
+            q = bf64(rot(x[b, :, :nh].double(), c64[b][:, None], s64[b][:, None]))                   # [L, nh, hd]
+            for h in range(nkv):
+                t, i = todo[b][h][n] if n < len(todo[b][h]) else (None, None)
+                if t is not None:
+                    k = alpha * q[i, h * grp] / (q[i, h * grp].square().sum() * scale)
+                    if past <= t < past + L:
+                        x[b, t - past, nh + h] = unrot(k, c64[b, t - past], s64[b, t - past]).to(BF16)
+                    else:
+                        kc[b, h, t] = k.to(BF16)
+                keys = torch.cat([kc[b, h, :past].double(), bf64(rot(x[b, :, nh + h].double(), c64[b], s64[b]))])
+                vals = torch.cat([vc[b, h, :, :past].double().T, x[b, :, nh + nkv + h].double()])
+                s = torch.einsum("lgd,td->lgt", q[:, h * grp:(h + 1) * grp], keys) * scale
+                seen = (torch.arange(past + L)[None] <= past + torch.arange(L)[:, None]) & (torch.arange(past + L)[None] >= pad_of[b])
+                s = s.masked_fill(~seen[:, None], float("-inf"))
+                live = seen.any(1)
+                want[b, live, h * grp:(h + 1) * grp] = torch.softmax(s[live], -1) @ vals
+                if t is not None:                                # the key's weight, seen or not, against all that the query sees
+                    others = s[i, 0].clone()
+                    if t < past + L:
+                        others[t] = float("-inf")
+                    assert alpha - 1.0 - torch.logsumexp(others, 0).item() > 3.0, (b, h, t, i)
+                    decisive += 1
+        assert decisive
+        k, v, out = kc.cuda(), vc.cuda(), torch.full((B, L, nh * hd), float("nan"), dtype=BF16).cuda()
+        ops.attention_decode(x.view(B * L, -1).cuda(), cos.cuda(), sin.cuda(), L, k, v, out, B, L, nh, nkv, hd, scale, past, T, ws, 1, pad_len=pad, merge_in_launch=False)
+        err = (out.cpu().double().view(B, L, nh, hd) - want).abs().max().item()
+        assert err < 2 ** -7 * vc.float().abs().max().item(), (n, err, [[e[n] if n < len(e) else None for e in row] for row in todo])
 
 
 @pytest.mark.parametrize("seed", range(4))
