@@ -680,6 +680,8 @@ static int mix_run_tiles(int B, int L, int past) {
   const long qt = (long)p3v_cdiv(L, 16) * B;
   if (qt >= 2L * cus) return tiles;
   if (tiles > MIX_PLAN_TILES) return p3v_cdiv(tiles, min(max(cus / qt, 1L), (long)MIX_MAX_ROW_SPLIT));
+  static thread_local int last[5] = {};                                  // (10 us at 4000 rows, asked for twice by every layer of a prompt)
+  if (last[0] == B && last[1] == L && last[2] == past && last[3] == cus) return last[4];
   long sum = 0;
   for (int q = 0; q < L; q += 16) sum += ((past + min(q + 15, L - 1)) >> 5) + 1;
   const int share = max(max(4, p3v_cdiv(sum * B, cus)), p3v_cdiv(tiles, MIX_MAX_ROW_SPLIT)), step = max(1, share / 20);
@@ -691,6 +693,7 @@ static int mix_run_tiles(int B, int L, int past) {
     const float end = (float)mix_runs_end(B, L, past, per, cus) + 1.f + 0.2f * (float)p3v_cdiv(tiles, per);
     if (end < best_end) best_end = end, best = per;
   }
+  last[0] = B, last[1] = L, last[2] = past, last[3] = cus, last[4] = best;
   return best;
 }
 
