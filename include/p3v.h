@@ -104,7 +104,7 @@ int p3v_gemm(const p3v_gemm_args_t* args /* host */, void* stream);
  * between 256 x 256 and 128 x 128 tiles, or one of the kernels for few rows (they come first, up to 256 rows) */
 int p3v_gemm_plan(int M, int N, int K, int epilogue);
 int64_t p3v_gemm_ws_bytes(int M, int N, int K, int epilogue);
-/* Round 6: 9 .. 32 rows of A on bf16 weights with K = 3072 or 8192 (a 9 .. 32-sequence decode batch; the reference's batched benchmark
+/* 9 .. 32 rows of A on bf16 weights with K = 3072 or 8192 (a 9 .. 32-sequence decode batch; the reference's batched benchmark
  * runs 15, phi_3_vision_mlx.py:1226-1243) take a register-streaming kernel inside p3v_gemm / p3v_gemm_resid_norm (weights HBM ->
  * registers in whole lines, A resident as MFMA fragments): this query says how -- 0 = not that kernel's shape, 1 = one pass,
  * S > 1 = S K slices through the `ws` partials + the reduction launch.  Host-only. */
@@ -181,7 +181,7 @@ int p3v_rope_kv_append(const uint16_t* qkv, const float* cos_t, const float* sin
                        int past, const int32_t* d_past, int dst_t, int dst_off_is_past,
                        int tab_t, int tab_div, float q_scale, void* stream);
 
-/* ---- a residual projection whose consumer is an RMSNorm, as one launch sequence (round 5; phi.py:478-484: `r + o_proj(...)` followed
+/* ---- a residual projection whose consumer is an RMSNorm, as one launch sequence (phi.py:478-484: `r + o_proj(...)` followed
  *      by `post_attention_layernorm`, `r + down_proj(...)` followed by the next layer's `input_layernorm`):
  *      p3v_gemm_resid_norm(g, w, eps, normed) == p3v_gemm(g) with P3V_EPI_RESID_BF16 + p3v_rmsnorm(g->out, w, normed, M, N, eps), bit
  *      for bit, where the projection runs as K slices (9 .. 256 rows and N small enough that the split pays: the fp32 partials are
@@ -189,7 +189,7 @@ int p3v_rope_kv_append(const uint16_t* qkv, const float* cos_t, const float* sin
  *      two calls -- for every other shape, without a workspace of p3v_gemm_ws_bytes(), or N > 3072.  normed: bf16 [M, N] contiguous. */
 int p3v_gemm_resid_norm(const p3v_gemm_args_t* gemm /* host */, const uint16_t* norm_w, float eps, uint16_t* normed, void* stream);
 
-/* ---- the qkv projection with the split, the rotation and the KV append in its EPILOGUE (round 5):
+/* ---- the qkv projection with the split, the rotation and the KV append in its EPILOGUE:
  *      p3v_gemm_qkv(g, s) == p3v_gemm(g) into a scratch [M, N] + p3v_rope_kv_append(scratch, ...) with s's arguments, bit for bit, in the
  *      GEMM's launches alone (phi.py:437-452 / 140-147: `qkv_proj` + `split` + `_rotate_half` + KVCache append; CLIP: q/k/v projections
  *      + head split).  g: A [B*L, K], W [(nh + 2 nkv) * hd, K] (q rows, k rows, v rows), epilogue P3V_EPI_NONE or P3V_EPI_BIAS; out /
@@ -263,7 +263,7 @@ typedef struct {
   int merge_in_launch; /* nonzero: the split-KV partials are merged by the last split of each (b, head) INSIDE the attention
                           launch; 0 = a separate merge launch.  Either way `ws` must hold 0xFF in every byte before its first use
                           (hipMemset) and every launch leaves it so: a partial word is valid when it is not the all-ones pattern */
-  /* optional (round 4): the layer's o_proj + residual in the SAME launch (phi.py:460, 483), for shapes
+  /* optional: the layer's o_proj + residual in the SAME launch (phi.py:460, 483), for shapes
    * p3v_attention_decode_can_fuse_oproj() accepts.  o_proj_w [o_n, n_heads * hd] bf16; o_proj_x [o_n] bf16 is the residual row,
    * updated in place: x += bf16(W_o . attention output), bit-identical to p3v_gemv with P3V_EPI_RESID_BF16 on `out`.  `out` must
    * hold 0xFF in every byte when the launch starts (the projecting workgroups poll its words); `o_rearm` (n_heads * hd bf16) is
@@ -275,14 +275,14 @@ typedef struct {
 } p3v_attn_decode_args_t;
 int p3v_attention_decode(const p3v_attn_decode_args_t* args /* host */, void* stream);
 /* Does p3v_attention_decode take `o_proj_w` for this shape on this device (host query, no launch)?  0 = no; 1 = attention + o_proj +
- * residual in ONE launch (merge_in_launch = 1, the 128-key one-tile plan); 2 (round 6) = merge_in_launch = 0: the launch that merges
+ * residual in ONE launch (merge_in_launch = 1, the 128-key one-tile plan); 2 = merge_in_launch = 0: the launch that merges
  * the split-KV partials also carries the o_proj + residual (long contexts, 64-key plans) -- same arguments, same bits. */
 int p3v_attention_decode_can_fuse_oproj(int B, int L, int n_heads, int hd, int n_split, int cache_t, int o_n, int merge_in_launch);
 /* 1: p3v_attention_decode (without o_proj_w) runs this shape as one workgroup per (row, head), without split partials (host query; the
  * rule is about time: the results of the two forms differ by rounding) */
 int p3v_attention_decode_rows_fit(int B, int L, int n_heads, int n_kv, int cache_t);
 /* Which role workgroup `wg` of the fused launch's 1-D grid (n_heads * n_split workgroups) plays under placement `map` (the
- * attn_fo_map tuning knob: 2 = default, 1 = the round's first form): out[0] = key split, out[1] = head, out[2] / out[3] = its
+ * attn_fo_map tuning knob: 2 = default, 1 = its first form): out[0] = key split, out[1] = head, out[2] / out[3] = its
  * projection units (rows [8 u, 8 u + 8) of o_proj; -1 = none).  Split n_split - 1 of a head is its merging workgroup.  Workgroups
  * L and L +- 256 share a CU on this part (round-robin dispatch), which is what the placement is built on: mergers sit alone with
  * one tile-only workgroup, projection units ride on the last workgroup of every other CU.  Returns P3V_ERR_UNSUPPORTED for shapes
@@ -326,7 +326,7 @@ typedef struct {
   float scale;
   int merge_in_launch;    /* as p3v_attn_decode_args_t.merge_in_launch (honoured with one tile per split and n_split <= 16 on
                              the 64-key plan, always on the 128-key plan; otherwise the merge launch runs) */
-  /* optional (round 4), as p3v_attn_decode_args_t's o_proj_* fields but for e4m3 weights: o_proj_w8 [o_n, n_heads * hd] bytes with
+  /* optional, as p3v_attn_decode_args_t's o_proj_* fields but for e4m3 weights: o_proj_w8 [o_n, n_heads * hd] bytes with
    * one fp32 scale per row; x += bf16(scale * (W8 . attention output)), bit-identical to p3v_gemv_fp8 with P3V_EPI_RESID_BF16.
    * For shapes p3v_attention_decode_q8_can_fuse_oproj() accepts; `out` all 0xFF on entry, `o_rearm` set to 0xFF. */
   const uint8_t* o_proj_w8; const float* o_proj_scale; uint16_t* o_proj_x; uint16_t* o_rearm; int o_n;
@@ -357,7 +357,7 @@ int p3v_topk(const uint16_t* x, int32_t* idx_out, int rows, int n, int k, int64_
  * phi_3_vision_mlx.py:264,297-305; w = scale * q + bias per 64 input columns, mx.quantized_matmul).
  * W [N or 2N, K/8] u32 in the DEVICE nibble order (weights 8d..8d+7 at bits 0,16,4,20,8,24,12,28 of dword d;
  * weights.q4_repack converts MLX's sequential order), sb [N or 2N, K/64] u32 = scale bf16 | bias bf16 << 16.
- * p3v_gemv_q4: decode projection, K = 3072 or 8192.  M = 1: same norm / epilogue options as p3v_gemv.  2 <= M <= 16 (round 6: a
+ * p3v_gemv_q4: decode projection, K = 3072 or 8192.  M = 1: same norm / epilogue options as p3v_gemv.  2 <= M <= 16 (a
  *   decode batch, a constrained-decoding step; N % 16 == 0 (SiLU: % 8)): the packed weights are dequantised in registers (fp16
  *   scale * q + bias, two weights per instruction) in front of the fp16 MFMA -- 0.5 byte per weight from HBM at every batch size, as
  *   the reference's QuantizedLinear (phi_3_vision_mlx.py:296).  norm_w: up to 8 rows the input RMSNorm may ride along (the rows are
@@ -415,7 +415,7 @@ int p3v_step_begin(const int32_t* tok, const uint16_t* table, uint16_t* x_out, c
 int p3v_step_end(const uint16_t* logits, int32_t* next_tok, int32_t* tok, int32_t* history, int32_t* d_step,
                  int32_t* d_past, int32_t* ticket, int B, int n, int max_steps, void* stream);
 
-/* Round 6: the same two stages WITHOUT launches of their own -- folded into the step's first projection (layer 0's RMSNorm + qkv)
+/* The same two stages WITHOUT launches of their own -- folded into the step's first projection (layer 0's RMSNorm + qkv)
  * and its last (final norm + lm_head, phi.py:597-608, phi_3_vision_mlx.py:386-393): p3v_gemv with
  *   begin (tok != NULL):      x row b = embed_table[clamp(tok[b])] instead of args->x; the rows are also written to x_out (the residual
  *                             stream) and the rotation rows of position *d_past staged into cos_out / sin_out, as p3v_step_begin does;

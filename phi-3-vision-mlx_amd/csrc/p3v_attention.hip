@@ -416,7 +416,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(AttnP p) {
 // (64 rows x 2*HD bytes, contiguous) and the V^T tile (HD rows x 128 bytes) go HBM/L2 -> LDS by LDS-DMA, each wave
 // issuing a quarter of the tile's 1 KiB pieces -- no staging registers, no ds_write pass, no per-tile address
 // arithmetic (k_attn_prefill spends most of its issue slots there).  Bank-conflict swizzles on the source side:
-//   192-byte K rows (HD = 96): chunk c ^ (-(row >> 2) & 3) (round 3: the round-2 form (row >> 2) & 3 was 2-way conflicted on ds_read_b128);   128-byte rows (K at HD = 64, V^T): chunk c ^ ((row >> 1) & 7).
+//   192-byte K rows (HD = 96): chunk c ^ (-(row >> 2) & 3) ((row >> 2) & 3 is 2-way conflicted on ds_read_b128);   128-byte rows (K at HD = 64, V^T): chunk c ^ ((row >> 1) & 7).
 // Two LDS buffers, one barrier per tile; compute part and masks identical to k_attn_prefill.
 typedef const __attribute__((address_space(1))) void* pf_gptr_t;
 typedef __attribute__((address_space(3))) void* pf_lptr_t;
@@ -719,7 +719,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill_dma(AttnP p) {
 }
 
 // =====================================================================================
-// Ping-pong prefill attention (round 3).  Where k_attn_prefill_dma lost its time (in-kernel phase counters):
+// Ping-pong prefill attention.  Where k_attn_prefill_dma lost its time (in-kernel phase counters):
 // per 64-key tile a wave spent 830 cycles on the 24 S^T MFMAs (384 matrix-pipe cycles), 2430 on the softmax (~700 VALU
 // cycles) and 1450 on the 28 PV MFMAs (448) -- neither pipe of a SIMD was busier than ~35 %: the SIMD's two waves (one of
 // each of the CU's two workgroups) drift in and out of the same phase, share the pipe they both want and leave the other
@@ -848,7 +848,7 @@ __global__ void __launch_bounds__(512, 1) k_attn_prefill_pp(AttnP p) {
   // batch overwrites: K(jb - 1), read in M(jb - 1) (steps 2 jb - 2 / 2 jb - 1) -> three K slots; V^T(jb - 2), read in
   // softmax(jb - 2) (steps 2 jb - 3 / 2 jb - 2) -> FOUR V^T slots (with three, group A's batch jb would land on the tile
   // group B's softmax(jb - 1) is still reading in step 2 jb).  Prologue batches -2, -1 = tiles 0, 1 (clamped into [0, NT)).
-  // DV (round 3, late): the matrix phase is the longer one and a DMA issue costs its wave ~100 cycles of MFMA issue, so batch
+  // DV: the matrix phase is the longer one and a DMA issue costs its wave ~100 cycles of MFMA issue, so batch
   // jb >= 1 is issued one step EARLIER, at the top of the wave's VALU phase softmax(jb - 1) (A: step 2 jb - 1, B: 2 jb); the
   // slots it overwrites must then be one tile older: K(jb - 2) (last read in M(jb - 2), steps 2 jb - 4 / 2 jb - 3) -> FOUR
   // K slots, V^T(jb - 3) (second half read in M(jb - 2)) -> FIVE V^T slots (with four, A's batch would land in step 2 jb - 1 on
@@ -1218,7 +1218,7 @@ __global__ void __launch_bounds__(512, 1) k_attn_prefill_pp(AttnP p) {
 // Which prompt-sized kernel (measured, 32 heads x 96, causal, random data; profiles/r03_attn_prefill_kernels.txt; the table the
 // launcher's rules come from sits at the rules, in launch_attn_prefill):
 //   dma (128 queries, 4 waves, two workgroups per CU): every plain-Q call (the ViT, cached calls) below 3072 tokens, pre-scaled
-//       prompts of several rows up to ~3500 tokens -- since it got the deferred-reference softmax: 946 TF/s at 8k (round 2: 606-623);
+//       prompts of several rows up to ~3500 tokens -- since it got the deferred-reference softmax: 946 TF/s at 8k (606-623 without it);
 //   il  (interleaved; 128 or 256 queries): pre-scaled prompts -- ONE row from 768 tokens, several rows from 3584, everything from 6144;
 //   pp  (ping-pong, 256 queries): what is left for it -- plain Q or head dim 64 from 3072 tokens.
 #include "p3v_attn_il.h"
@@ -1394,7 +1394,7 @@ extern "C" int p3v_timing_read(long long* out, int n) {
 __device__ __forceinline__ void st_wt(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float ld_wt(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ bool is_sentinel(float v) { return __builtin_bit_cast(uint32_t, v) == WS_SENTINEL; }
-// Round 6: 16- and 8-byte write-through stores for the sentinels a merge puts back (24 x 16 bytes + 8 per record instead of 98 dword
+// 16- and 8-byte write-through stores for the sentinels a merge puts back (24 x 16 bytes + 8 per record instead of 98 dword
 // stores: a write-through `sc1` store leaves the CU as one fabric write per lane whatever its width, MI355X_MICROARCH.md).  The same
 // widening of the partial records and of the merged row was built and measured SLOWER (+25 us per decode step: the wide stores of a
 // record become visible to the polling merger ~0.5 us later; profiles/r06_attn_oproj_placement.txt), so those stay dword stores.
@@ -1839,7 +1839,7 @@ __device__ __forceinline__ void attn_decode_body(const AttnDecP& p, const int bx
   DBG_W(11, false);
 }
 
-// ---- 128-key tiles (round 2).  Same structure as attn_decode_body, twice the keys per workgroup: wave w owns keys
+// ---- 128-key tiles.  Same structure as attn_decode_body, twice the keys per workgroup: wave w owns keys
 // [32w, 32w + 32) -- two 16-key S^T blocks (6 MFMA 16x16x32), an 8-value-per-lane softmax, and O^T += V^T.P^T as 6 MFMA
 // 16x16x32 whose k index runs over both blocks (k = (j / 4) * 16 + 4g + j % 4, the same permutation on the V^T fragment:
 // two 8-byte reads) with P straight from the two accumulators.  Why: at the bench context the 64-key plan needs 1344-1408
@@ -1864,10 +1864,10 @@ __device__ __forceinline__ void attn_decode_body(const AttnDecP& p, const int bx
 // arithmetic (lane l holds chunks l, l + 64, ..; dot8 in chunk order; DPP wave sum; resid + bf16 round), so the step's results do
 // not depend on whether the projection was fused.  One launch (~5 us) and its boundary leave the layer.  The attention output
 // lives in two buffers used by alternate layers: a launch re-arms the one it does not use.
-// Round 6: WHERE the roles of the fused launch sit.  Measured (tools/scratch/wg_census_r6.hip): workgroup L of a launch whose
+// WHERE the roles of the fused launch sit.  Measured (tools/scratch/wg_census_r6.hip): workgroup L of a launch whose
 // workgroups are all resident runs on XCD L % 8 and shares its CU with workgroups L +- 256 -- the dispatcher deals them round
 // robin over the 256 CUs -- so "virtual CU" v = L % 256, slot = L / 256 says who is co-resident with whom (for speed only: nothing
-// below is needed for correctness).  With the (split, head) grid of rounds 4-5 the 32 merging workgroups shared their CUs with
+// below is needed for correctness).  With the (split, head) grid the 32 merging workgroups shared their CUs with
 // workgroups streaming 48 KB of W_o each, whose loads sit in the same per-CU memory queue as the merger's polls (a hand-over costs
 // 1.1 us into a quiet CU, 2.5-2.9 us into a streaming one: MI355X_MICROARCH.md, handoff-1to1), and W_o requests of a CU's first
 // workgroup got ahead of its last workgroup's tile DMA.  Now: G = heads x splits workgroups as a 1-D grid; CUs v < r = G % 256
@@ -1960,7 +1960,7 @@ __device__ __forceinline__ void fo_project(const FoP f, const int o_wl, unsigned
     if (wave == 0) {
       // bounded by WALL TIME (100 MHz counter), 5 ms: the launch itself lasts ~15 us, and a run whose workgroups are not all resident
       // (a profiler that masks CUs or serialises workgroups, a co-tenant process) must fail FAST and loudly -- NaN row, negative token,
-      // api.greedy_loop re-plans with separate launches -- not after 65536 polls per workgroup (rounds 4-5: ~65 ms each, 32 launches per
+      // api.greedy_loop re-plans with separate launches -- not after 65536 polls per workgroup (~65 ms each, 32 launches per
       // step: whole-graph rocprofv3 --pmc passes did not finish).  P3V_PROFILING=1 plans the separate launches from the start.
       bool to = false;
       const long long t_wait = wall_clock64();
@@ -2059,7 +2059,7 @@ __device__ __forceinline__ void fo_project(const FoP f, const int o_wl, unsigned
 
 template <int FO = 0>                                          // FO_NONE, FO_BF16 or FO_Q4: the o_proj weights' format
 __device__ __forceinline__ void attn_decode_body128(const AttnDecP& p, const int bx, const int by, const int bz, unsigned char* KV,
-                                                    const int o_unit = -2, const int o_unit2 = -1) {   // -2: projection units by (head, split) rank (rounds 4-5)
+                                                    const int o_unit = -2, const int o_unit2 = -1) {   // -2: projection units by (head, split) rank
   constexpr int TK = 128, WK = 32, HD = 96, KROW = HD * 2, VROWB = TK * 2, NKS = 3, NDT = 6, CPR = 12;
   constexpr int KS_BYTES = WK * KROW;                          // 6 KiB per wave = 16 x 96 fp32: the wave's O partial parks here
   static_assert(KS_BYTES >= 16 * HD * 4, "a wave's O partial reuses its K slice");
@@ -2083,10 +2083,10 @@ __device__ __forceinline__ void attn_decode_body128(const AttnDecP& p, const int
 #endif
   int past = p.past, pad = 0;
   // With d_past, p.past is a LOWER BOUND of the cache length (the prompt length when the graph was captured; negative = no
-  // bound known: every tile is requested at once, as in round 3): a
+  // bound known: every tile is requested at once): a
   // tile that starts below it is certainly live and is requested at once; one at or beyond it may lie wholly past the live
   // keys (the cache CAPACITY is prompt + max_tokens, rounded up to the tile) -- it waits for the length and fetches nothing
-  // when dead.  (Round 3 fetched every tile of the capacity: 1.06x the live bytes at the bench shape, 1.2x with max_tokens = 512.)
+  // when dead.  (Fetching every tile of the capacity: 1.06x the live bytes at the bench shape, 1.2x with max_tokens = 512.)
   const int past_lb = p.past;
   if (p.d_past) asm volatile("s_load_dword %0, %1, 0x0" : "=s"(past) : "s"(p.d_past) : "memory");
   if (p.pad_len) asm volatile("s_load_dword %0, %1, 0x0" : "=s"(pad) : "s"(p.pad_len + b) : "memory");
@@ -2790,7 +2790,7 @@ __global__ void __launch_bounds__(64 * CMB_G) k_attn_combine2(const float* __res
   combine_rows<false>(ws, out, L, nh, hd, n_split, (int)blockIdx.x);
 }
 
-// Round 6, long contexts (the split-KV plans whose partials are merged by a launch of their own: more than 48 tiles of 128 keys, i.e.
+// Long contexts (the split-KV plans whose partials are merged by a launch of their own: more than 48 tiles of 128 keys, i.e.
 // every context beyond ~6k tokens up to the model's 128k): the merge launch also carries the layer's o_proj + residual (B = L = 1),
 // as k_attn_decode128_o does for the one-tile plans.  Workgroups 0 .. nh - 1 merge one head each (k_attn_combine2's arithmetic, the row
 // published as 48 write-through words); the others are fo_project units (two row-pair quartets each): their W_o rows are requested at
@@ -3619,7 +3619,7 @@ __global__ void __launch_bounds__(256) k_attn_decode_q8s(AttnDecQ8P p) {
   }
 }
 
-// ---- int8 twin of k_attn_decode128 (round 2): 4 waves x one 128-key tile, wave w owns keys [32w, 32w + 32).
+// ---- int8 twin of k_attn_decode128: 4 waves x one 128-key tile, wave w owns keys [32w, 32w + 32).
 // The RAW BYTES go HBM -> LDS by LDS-DMA (K slice: 32 rows x 96 B, contiguous in the cache; V^T tile by rows: 96 x 128 B,
 // 16-byte chunk c of row d stored at c ^ (d & 7)) -- half the bytes of the bf16 kernel and no pass through registers --
 // and become fp16 operands (1024 + code, see u8x16_to_f16) only when a fragment is read: ds_read_b64 / 2 x ds_read_b32 +
@@ -3935,7 +3935,7 @@ extern "C" int p3v_attention_decode_q8(const p3v_attn_decode_q8_args_t* a, void*
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid(a->n_split, a->n_heads, a->B);
   const bool old_only = p3v_tuning().q8_old != 0;   // A/B knob
-  // the o_proj rides either in the one-tile attention launch (in-launch merge) or in the merge launch (k_attn_combine_o, round 6)
+  // the o_proj rides either in the one-tile attention launch (in-launch merge) or in the merge launch (k_attn_combine_o)
   const bool merge_o = a->o_proj_w8 && !a->merge_in_launch;
   if (merge_o) {
     if (!combine_o_ok(a->B, a->L, a->n_heads, a->hd, a->n_split, a->o_n)) return P3V_ERR_UNSUPPORTED;

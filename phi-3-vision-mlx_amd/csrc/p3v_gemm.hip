@@ -16,7 +16,7 @@
 //             MFMAs take the W fragment FIRST, so a lane holds 4 consecutive columns
 //             of one output row; bf16 outputs pair two column blocks with
 //             v_permlane16_swap -> 16-byte stores of 8 consecutive columns, no LDS
-//             staging (rounds 1-4 went through a wave-private LDS tile).
+//             staging.
 //
 // Roofline: MFMA-bound for M >= ~512 (2*M*N*K flops vs (M+N)*K*2 bytes).
 #include <stdlib.h>
@@ -189,7 +189,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm(GemmP p) {
     }
   }
 
-  // ---- epilogue straight from the accumulators (round 5; rounds 1-4 staged the tile through LDS between two barriers).  The
+  // ---- epilogue straight from the accumulators (not staged through LDS between two barriers).  The
   // MFMAs take the W fragment first, so a 16 x 16 block comes out transposed: lane (c = lane & 15, q = lane >> 4) holds the four
   // consecutive columns 4q .. 4q+3 of output row c.  fp32 outputs store them as they are (16 bytes); bf16 outputs first trade
   // packed halves of two neighbouring column blocks between lanes q and q ^ 1 (v_permlane16_swap): 8 consecutive columns per lane.
@@ -662,7 +662,7 @@ extern "C" int p3v_gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp,
   // what the fused epilogue needs (anything else: P3V_ERR_UNSUPPORTED, the caller runs p3v_gemm + p3v_rope_kv_append):
   // prompt-sized M; rotation pairs in blocks of 16 inside a head; whole 128-column tiles per region; an 8-aligned append offset
   const int dpos0 = sp->dst_off_is_past ? sp->past : 0;
-  // (round 6: batch rows of any length -- the V^T runs are then stored at whatever offset they fall on, qkv_epilogue_vt)
+  // (batch rows of any length -- the V^T runs are then stored at whatever offset they fall on, qkv_epilogue_vt)
   if (hd % 32 || half % 16 || dpos0 % 8 || sp->dst_t % 8 || !qkv_rows_ok(sp->B, sp->L) || p3v_tuning().gemm_no_qkv_fuse) return P3V_ERR_UNSUPPORTED;
   if ((size_t)a->M * a->lda * 2 >= (1ull << 32) || (size_t)a->N * a->ldw * 2 >= (1ull << 32)) return P3V_ERR_UNSUPPORTED;
   hipStream_t s = (hipStream_t)stream;

@@ -1,18 +1,17 @@
-// Large-tile variant of the dense projection for prefill-sized problems (N % 256 == 0, K % 64 == 0; p3v_gemm decides
-// how many rows of a problem it gets):
-//   256(M) x 256(N) x 64(K) tile (template: 224 rows, or 192 columns, for problems whose rounds they fill better), 512 threads = 8 waves as 2(M) x 4(N), each wave 128 x 64 =
-//   8 x 4 v_mfma_f32_16x16x32_bf16 accumulators (128 registers), 2.67 MFMAs per LDS fragment read
+// Large-tile variant of the dense projection for prefill-sized problems (K % 64 == 0, columns in whole tiles; p3v_gemm decides which rows of a
+// problem it gets and in which of its tiles):
+//   256(M) x 256(N) x 64(K) tile (template: 224 rows, or 192 columns, for problems whose rounds they fill better), 512 threads = 8 waves
+//   as 2(M) x 4(N), each wave 128 x 64 = 8 x 4 v_mfma_f32_16x16x32_bf16 accumulators (128 registers), 2.67 MFMAs per LDS fragment read
 //   (the 128x128 kernel: 2.0) and 25 % less global->LDS traffic per flop.
-//   K-tile t lives in LDS buffer t&1 (2 x 64 KiB); a tile is four PHASES (one 64x32 accumulator quadrant = 16
-//   MFMAs each).  The four 16-KiB half-tiles of tile t+1 are requested by LDS-DMA in the first two phases of
-//   tile t, each batch AFTER that phase's fragment reads are issued (SCHED 0x50): measured against one
-//   half-tile per phase (the last one then has only 16 MFMAs to land before the vmcnt(0)) +12 % at 4096^3
-//   (1170 -> 1310 TF/s), against all four up front +7 % (eight DMA issues ahead of the first fragment reads
-//   delay the first MFMA).  The fragment reads are software-pipelined (ORDER 2): the fragments of phase p+1 are requested
-//   before the MFMAs of phase p (second A-fragment buffer, 256 registers, no spill), +1.5-2 % at 4096^3 / 8192^3
-//   (1.28 -> 1.30, 1.32 -> 1.34 PFLOP/s).  One vmcnt(0) + barrier per K-tile.  No barrier inside a tile: the waves
+//   K-tile t lives in LDS buffer t&1 (2 x 64 KiB); a tile is four quadrants (64 x 32 accumulators = 16 MFMAs each).  K-tile t+1 is
+//   requested by LDS-DMA during the first two quadrants of K-tile t, A behind the first's fragment reads, B behind the second's: measured
+//   against a quarter per quadrant (the last one then has only 16 MFMAs to land before the vmcnt(0)) +12 % at 4096^3 (1170 -> 1310 TF/s),
+//   against all of it up front +7 % (eight DMA issues ahead of the first fragment reads delay the first MFMA).  The fragment reads are
+//   software-pipelined: the fragments of the next quadrant are requested before the MFMAs of this one (second A-fragment buffer: all 256
+//   registers, and one or two spilled in the gated and erf-GELU forms, reloaded once per output tile: no difference measured), +1.5-2 % at
+//   4096^3 / 8192^3 (1.28 -> 1.30, 1.32 -> 1.34 PFLOP/s).  One vmcnt(0) + barrier per K-tile.  No barrier inside a tile: the waves
 //   de-phase, one wave's fragment reads overlap another's MFMAs.
-//   Same XOR-swizzled LDS image and the same epilogues as p3v_gemm.hip; round 5: stored straight from the accumulators.
+//   Same XOR-swizzled LDS image and the same epilogues as p3v_gemm.hip; stored straight from the accumulators.
 #include <stdlib.h>
 
 #include "p3v_gemm256_epi.h"
@@ -48,7 +47,7 @@ __global__ void __launch_bounds__(512, 1) k_gemm256(Gemm256P p) {
   // (P3V_EPI_QKV: N = (nh + 2 nkv) * hd; column tiles 0 .. nq-1 are Q, then K, then V -- p3v_gemm_qkv.h)
   const int nq_t = QKV ? p.q.nh * p.q.hd / TN : 0, nk_t = QKV ? p.q.nkv * p.q.hd / TN : 0;
 
-  // ---- PERSISTENT over output tiles (round 3): workgroup b takes tiles b, b + G, b + 2G, ... (G = gridDim.x, a multiple of 8,
+  // ---- PERSISTENT over output tiles: workgroup b takes tiles b, b + G, b + 2G, ... (G = gridDim.x, a multiple of 8,
   // so a workgroup's tiles keep its XCD in the XCD-aware order below).  The K-tile stream runs ACROSS tile seams: during the
   // last K-tile of a tile the first K-tile of the workgroup's NEXT tile is requested into the other LDS buffer, and the
   // epilogue (staged through the buffer that was just consumed) runs under that DMA -- the 64-KiB cold fetch that opened every
@@ -198,7 +197,7 @@ __global__ void __launch_bounds__(512, 1) k_gemm256(Gemm256P p) {
         else dma_a(nt, 0, nb);
       }
     };
-    // (Measured and removed, round 3: the eight LDS-DMA pieces of a wave SPREAD over the first two quads, one piece every four
+    // (Measured and removed: the eight LDS-DMA pieces of a wave SPREAD over the first two quads, one piece every four
     //  MFMAs, instead of two bursts of four in front of them -- 18-30 % SLOWER on every shape.  tools/gemm256_timeline.py: a
     //  piece costs its wave ~80-150 cycles of instruction issue wherever it stands (580-750 cycles for 12 fragment reads + 4
     //  pieces, ~300 for 8 + 4, against 1024 for the K-tile's 64 MFMAs); inside a quad those cycles come out of the wave's own
@@ -262,7 +261,7 @@ static int launch_gemm256_v(const Gemm256P& p, hipStream_t s) {
   const int n_cu = p3v_gemm256_cus();
   if (!n_cu) return P3V_ERR_HIP;
   const int tiles = p3v_cdiv(p.N, P3V_GATED(EPI) ? TN / 2 : TN) * p3v_cdiv(p.M, TM);
-  const int persist = p3v_tuning().gemm_persistent;                // 0: one workgroup per tile (round 2), else the persistent loop
+  const int persist = p3v_tuning().gemm_persistent;                // 0: one workgroup per tile, else the persistent loop
   dim3 grid(persist ? min(tiles, n_cu) : tiles);
   hipLaunchKernelGGL((k_gemm256<EPI, MB, NB>), grid, dim3(512), LDS, s, p);
   P3V_CHECK_LAUNCH();

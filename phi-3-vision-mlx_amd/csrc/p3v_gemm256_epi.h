@@ -17,10 +17,10 @@ struct Gemm256P {
 
 __device__ __forceinline__ float gelu_erf2(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
 
-// ---- epilogue: 16 MB x 16 NB outputs per wave, STRAIGHT FROM THE ACCUMULATORS (round 5).  The MFMAs take the W fragment as their
+// ---- epilogue: 16 MB x 16 NB outputs per wave, STRAIGHT FROM THE ACCUMULATORS.  The MFMAs take the W fragment as their
 // first operand, so a 16 x 16 block comes out transposed: lane (c = lane & 15, q = lane >> 4) holds, for output row
 // m = block row c, the FOUR CONSECUTIVE columns 4q .. 4q+3 (the plain operand order gives four rows of one column, which is
-// why rounds 1-4 staged every tile through a wave-private LDS image: 64 ds_write_b32 + 32 ds_read_b128 per lane and tile,
+// what would make a tile go through a wave-private LDS image: 64 ds_write_b32 + 32 ds_read_b128 per lane and tile,
 // ~4 us per tile).  fp32 outputs: those four values are one 16-byte store.  bf16 outputs: the lane pairs (q, q ^ 1) trade the
 // packed halves of two neighbouring column blocks with v_permlane16_swap, after which every lane owns 8 consecutive columns
 // = one 16-byte store (even q: block 2jp, odd q: block 2jp + 1; columns 8 * (q >> 1) .. + 8 of it).  No LDS, no barrier:

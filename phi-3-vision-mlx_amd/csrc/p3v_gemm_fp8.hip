@@ -20,10 +20,11 @@
 //             What bounds it: the producers' requests, ~60 ns per round of four 1-KiB pieces (a K-tile of 128 x 256 takes 0.69 us
 //             where its MFMAs take 0.43), and, with all CUs at it, the chip's power: the same launches on all-zero operands are
 //             20-25 % faster.  Against the form it replaced (256-row tiles, eight waves that request and multiply, two buffers and a
-//             full wait per K-tile, one tile per workgroup, outputs staged through LDS), us at M = 2531 / 1024 / 256:
+//             full wait per K-tile, one tile per workgroup, outputs staged through LDS), us at M = 2531 / 1024 / 256, launches by themselves in a graph:
 //               gate_up 131 / 51 / 44 -> 112 / 50 / 18    qkv 79 / 52 / 26 -> 64 / 30 / 16 (K = 3072)
 //               o 29.2 / 27.7 / 25.5 -> 28.2 / 17.4 / 15.4   down 63 / 58 / 57 -> 56 / 32 / 30 (K = 8192)
-//             2.2-2.4 PFLOP/s from 2500 rows on.
+//             2.2-2.4 PFLOP/s from 2500 rows on in such a graph.  Inside a prompt, under the profiler, a launch follows others at the
+//             chip's power limit and takes 15 % longer: gate_up 129 at 2531 rows, and the four together 1.8 PFLOP/s.
 //   epilogue  scales, then none / residual add / SiLU(gate) * up, bf16 out, straight from the accumulators (p3v_gemm256_epi.h).
 #include <stdlib.h>
 

@@ -6,7 +6,7 @@
 //            0.85 with three, most of it DMA issue in front of the MFMAs; here 0.81 (0.65 with 192 workgroups).
 //   staging  S = 3 (128 x 192: 4) LDS buffers; one barrier per K-tile, in the middle of it: the fragments of one 32-wide half are
 //            multiplied while those of the other are read, so a K-tile's buffer is free, and refilled, half a K-tile before its last MFMA.
-//   bound    the LDS-DMA: 88 - 98 KB/us and CU in pieces of 8 rows x 128 B, i.e. 0.5 us for the 48 KB of a 128 x 256 K-tile against 0.45 of
+//   bound    the LDS-DMA: 88 - 98 KB/us and CU in pieces of 8 rows x 128 B (profiles/lds_dma_probe.txt), i.e. 0.5 us for the 48 KB of a 128 x 256 K-tile against 0.45 of
 //            MFMAs; larger tiles do not fit the 168 registers that twelve waves leave each other.
 // 2531 x 3072 x 8192 (+ residual) 117 -> 105 us (1.21 PFLOP/s), 9809 x 1024 x 4096 (+ fp32 residual) 95 -> 73, 2048 x 9472 x 3072 114 -> 97.
 // Same K order and epilogue as the other tiles: bit-identical results.

@@ -1,4 +1,4 @@
-// The qkv projection with the head split, the rotation and the KV append in its epilogue (round 5): p3v_gemm_qkv =
+// The qkv projection with the head split, the rotation and the KV append in its epilogue: p3v_gemm_qkv =
 // p3v_gemm(qkv_proj) + p3v_rope_kv_append in the launches of the GEMM alone.  Shared by the 256 x 256 and the 128 x 128 tile kernels.
 //
 // What makes it fit the accumulator layout (a lane holds 4 consecutive output columns of one row, p3v_gemm256_epi.h):
@@ -153,7 +153,7 @@ __device__ __forceinline__ void qkv_epilogue_vt(const QkvP& q, f32x4_t (&acc)[NI
         bf16_t* dst = q.v_dst + (((size_t)b * q.nkv + head) * q.hd + d) * (size_t)q.dst_t + q.dpos0 + l;
         if (t + 8 <= M && l + 8 <= q.L) {                      // the run lies in one batch row
           if (!(l & 1)) {
-            // even token offset: the run is dword-aligned (16-byte aligned for one batch row, or rows of L % 8 == 0 tokens; round 6:
+            // even token offset: the run is dword-aligned (16-byte aligned for one batch row, or rows of L % 8 == 0 tokens;
             // any row length -- CLIP's 577-token crops start one token later in every crop) -- one dwordx4 store either way
             typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
             *(u32x4_a4*)dst = w;

@@ -1,4 +1,4 @@
-// Projections  C[M, N] = x[M, K] * W[N, K]^T  for 9 .. 32 rows of x (round 6): a batched decode step of 9 .. 32 sequences -- the
+// Projections  C[M, N] = x[M, K] * W[N, K]^T  for 9 .. 32 rows of x: a batched decode step of 9 .. 32 sequences -- the
 // reference's own batched benchmark runs 15 (phi_3_vision_mlx.py:1226-1243) -- and any continuous-batching server.  At these M the
 // projection is a WEIGHT STREAM; the 64-row tiles of p3v_gemm_skinny.hip stage every weight byte through LDS next to a re-read x
 // panel (W x 3 bytes staged per launch, 2.1 - 4.4 TB/s of weights, B = 9 slower per token than B = 8).  This kernel is k_gemv_mfma8

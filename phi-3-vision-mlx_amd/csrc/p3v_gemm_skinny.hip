@@ -1,4 +1,4 @@
-// Prompt-sized-but-short projections  C[M, N] = A[M, K] * W[N, K]^T  for 9 .. 256 rows (round 5): a 128-token chat prompt, the text
+// Prompt-sized-but-short projections  C[M, N] = A[M, K] * W[N, K]^T  for 9 .. 256 rows: a 128-token chat prompt, the text
 // group of a mixed batch, a 9..128-row decode batch.  At these M the GEMM is a WEIGHT STREAM (2 * 128 * N * K flops against N * K * 2
 // bytes: ~13 GFLOP for the 100 MB of gate_up, both worth ~10-17 us), and what decides its speed is how many K-tiles a workgroup
 // has on the wire: the 128 x 128-tile kernel (p3v_gemm.hip) holds ONE ahead and pays a DMA round trip (~1.3 us at this load) per
@@ -6,7 +6,9 @@
 //   tile      128(M) x 64(N) x 64(K): twice the workgroups per weight matrix, so gate_up (256 tiles) and qkv (144) run in one pass
 //             and the others with a smaller split over K (o_proj 4, down 4 slices: one workgroup per CU, partials <= a quarter of
 //             the weight bytes).  The kernel's bound: every workgroup re-reads the A panel from L2 beside its weight stream from
-//             HBM, and in one CU the two add up -- the same requests without any compute take 27.7 of gate_up's 30 us at 128 rows.
+//             HBM, and in one CU the two add up -- the same requests without any compute take as long as gate_up, 30 us at 128
+//             rows (rows 6144 bytes apart; weights alone 18.5, both packed 25.9: profiles/lds_dma_probe.txt).  Rows of A and W 128 bytes further apart: gate_up 30.2 ->
+//             27.7, qkv 26 -> 24.3, but down 22.6 -> 25.4; the weights lie unpadded, as the other kernels and the loader have them.
 //             128 x 128 tiles (W x 2 staged, half the workgroups) were not faster on any shape (the template keeps the variant).
 //   staging   LDS-DMA into a ring of 6 stages (A 16 KiB + W 8 KiB each), 5 in flight behind a counted vmcnt; one workgroup per CU
 //             (<= 64 rows: 64-row tiles, A 8 KiB per stage -- a third less staged per K-tile, the same sums bit for bit: 60 -> 53 us

@@ -335,7 +335,7 @@ extern "C" int p3v_gemv_timing_read(long long* out, int n) {
 #else
 #define GMARK(k)
 #endif
-// Round 2: PERSISTENT over row sets.  The per-workgroup timeline (-DP3V_ATTN_TIMING, tools/gemv8_timeline.py) of the
+// PERSISTENT over row sets.  The per-workgroup timeline (-DP3V_ATTN_TIMING, tools/gemv8_timeline.py) of the
 // one-set-per-workgroup form (qkv: 576 workgroups, 3 per CU) showed the activations arriving 2-11 us after entry (27.6 MB
 // of x reads of the same 48 KB by 2304 waves) and the RMSNorm pass over 8 x 768 values per wave costing another 3 us with
 // 12 waves per CU doing it at once: the weights had landed long before anybody could use them (16.2 us for 56.6 MB).  Now
@@ -706,7 +706,7 @@ extern "C" int p3v_gemv(const p3v_gemv_args_t* a, void* stream) {
   const int rows_variant = p3v_tuning().gemv_rows;
   // smallest M the 8-row MFMA kernel takes: 2 since it became persistent with the RMSNorm scale in the epilogue (decode step
   // at ctx 2531, B = 2 / 3 / 4: 2.08 / 2.43 / 2.66 ms with the MT-row streaming kernel, 1.99 / 2.16 / 2.35 with this one);
-  // P3V_GEMV8_MIN=5 restores the round-1 split
+  // P3V_GEMV8_MIN=5 gives 2 .. 4 rows to the MT-row streaming kernel
   const int rows8_min = p3v_tuning().gemv8_min;
   if (rows_variant && variant == 3 && a->M >= 2 && a->M <= 4 && a->M < rows8_min && a->N % 2 == 0 && a->epilogue != P3V_EPI_F32 && a->epilogue != P3V_EPI_GELU_MUL && !scaled &&
       (a->K == 3072 || a->K == 8192)) {

@@ -1,6 +1,6 @@
 // Body of the streaming M = 1 GEMV (k_gemv3, p3v_gemv.hip), shared with the o_proj stage of the fused attention launch
 // (fo_project, p3v_attention.hip).  (Two more fused launches once shared it -- a GEMV chain and a qkv-projection + attention launch,
-// both bit-exact, both slower than separate launches; removed in round 4, described in DESIGN.md section 3.1.)
+// both bit-exact, both slower than separate launches; removed.)
 #pragma once
 #include <type_traits>
 
@@ -38,7 +38,7 @@ __device__ __forceinline__ float dot8(u32x4_t w, u32x4_t x, float acc) {
 typedef std::integral_constant<int, 0> IC0;
 typedef std::integral_constant<int, 1> IC1;
 
-// Round 6: the two ends of a replayed greedy decode step ride in the step's first and last projection (p3v_gemv_step):
+// The two ends of a replayed greedy decode step ride in the step's first and last projection (p3v_gemv_step):
 //  STEP_BEGIN  x row m = embed_table[clamp(tok[m])] (what p3v_step_begin gathered into x_out); workgroup 0 also writes the rows to
 //              x_out -- the residual stream the later launches update in place -- and stages the rotation rows of position *d_past.
 //  STEP_END    arg-max of the output rows (first maximum of the bf16 values; a NaN row reports -1) + p3v_step_end's bookkeeping:

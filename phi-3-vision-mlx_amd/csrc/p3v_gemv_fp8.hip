@@ -22,7 +22,7 @@ struct GemvF8P {
 
 // ---------------------------------------------------------------- M = 1 streaming (see k_gemv3)
 // STEP (p3v_gemv3_body.h): STEP_BEGIN / STEP_END carry the replayed greedy step's embedding gather + rotation rows / arg-max + bookkeeping,
-// exactly as gemv3_body does for bf16 weights (round 6: config 5's step is 129 launches too)
+// exactly as gemv3_body does for bf16 weights (config 5's step is 129 launches too)
 template <int NST, int CH, int STEP>
 __device__ __forceinline__ void gemv3_f8_body(const GemvF8P& p, int units_per_wave, int wpw, unsigned char* smem, float* red, const GemvStepP* sp) {
   constexpr int CHUNKS = NST * CH * 64;                 // 16-byte weight chunks per row (K = 16 * CHUNKS)

@@ -263,9 +263,9 @@ extern "C" int p3v_gemv_q4_step(const p3v_gemv_q4_args_t* a, const p3v_gemv_step
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
-// 2 .. 16 rows of x on the 4-bit weights (round 6): the reference runs QuantizedLinear at every batch size
-// (phi_3_vision_mlx.py:296; README batched 4-bit benchmark), rounds 3-5 dequantised the WHOLE matrix into a bf16 scratch per call
-// (2 launches, 5 x the 4-bit bytes moved).  This is k_gemm_rows (p3v_gemm_rows.hip) on the packed weights: the lane that held a
+// 2 .. 16 rows of x on the 4-bit weights: the reference runs QuantizedLinear at every batch size
+// (phi_3_vision_mlx.py:296; README batched 4-bit benchmark).  Dequantising the WHOLE matrix into a bf16 scratch per call
+// is 2 launches and 5 x the 4-bit bytes moved.  This is k_gemm_rows (p3v_gemm_rows.hip) on the packed weights: the lane that held a
 // 16-byte bf16 chunk of a weight line now loads 16 bytes = 32 WEIGHTS of the row (eight lanes cover the 128-byte line that holds a
 // row's 256-weight block: whole lines per instruction, 0.5 byte per weight from HBM), all of one 64-weight group (dword j of the
 // lane = weights 64 g + 32 h + 8 j ..+7 of the block: group g), so ONE scale | bias word per (lane, block, row set) dequantises them in

@@ -165,7 +165,7 @@ def _decode_result(kind, words):
 
 def pack_results(local_idx, local_results):
     """This rank's results as ONE int32 tensor: [n | request ids | kinds | lengths | payload] (kinds: `_encode_result`).
-    (Round 5: the result gather used to pickle Python objects through all_gather_object; round 6: typed per result, so float
+    (Typed per result and not pickled through all_gather_object, so float
     scores and scalar results survive a world > 1 gather unchanged instead of being truncated / raising.)"""
     enc = [_encode_result(r) for r in local_results]
     flat = [len(enc)] + [int(i) for i in local_idx] + [k for k, _ in enc] + [len(q) for _, q in enc] + [v for _, q in enc for v in q]

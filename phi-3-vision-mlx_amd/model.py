@@ -150,7 +150,7 @@ class Phi3VModel(DecoderModel):
             return ops.gemv_q4(x, q4[0], q4[1], epilogue, resid=resid, norm_w=norm_w, norm_eps=eps, out=out)
         if (q4 is not None and 2 <= M <= 16 and K in (3072, 8192) and os.environ.get("P3V_Q4_ROWS", "1") != "0"
                 and (q4[0].shape[0] // (2 if epilogue == EPI_SILU_MUL else 1)) % 16 == 0):
-            # 2 .. 16 rows straight on the 4-bit weights (round 6: k_gemv8_q4 / k_gemm_rows_q4; the reference runs QuantizedLinear at
+            # 2 .. 16 rows straight on the 4-bit weights (k_gemv8_q4 / k_gemm_rows_q4; the reference runs QuantizedLinear at
             # every batch size, phi_3_vision_mlx.py:296) instead of dequantising the whole matrix into the bf16 scratch per call
             if norm_w is not None and (M > 8 or os.environ.get("P3V_Q4_ROWS8_NORM", "1") == "0"):
                 x, norm_w = ops.rmsnorm(x, norm_w, eps, out=h), None       # 9 .. 16 rows: one p3v_rmsnorm launch in front
@@ -220,7 +220,7 @@ class Phi3VModel(DecoderModel):
     def clip_forward(self, pix):
         """ClipModel.__call__ (phi.py:216-221) on live crops; pix f32 [n,3,336,336] -> f32 [n,577,D]
         (row 0 = CLS, which the caller skips).
-        Round 6: the tower's ~280 launches cost the host as long to enqueue (25 - 30 us each in Python + ctypes) as the GPU to run, so a
+        The tower's ~280 launches cost the host as long to enqueue (25 - 30 us each in Python + ctypes) as the GPU to run, so a
         crop count seen for the SECOND time is captured as one hipGraph over buffers the entry owns (as the short-prompt prefill,
         _prefill_captured) and later images of that geometry cost one copy + one graph launch; the returned features are the
         entry's buffer -- the caller consumes them on the same stream before the next image can overwrite them.  Same kernels in
@@ -283,7 +283,7 @@ class Phi3VModel(DecoderModel):
             ops.layernorm(x2, w[lp + "layer_norm1.weight"], w[lp + "layer_norm1.bias"], eps, out=h)
             wq, bq = self.clip_qkv[j]
             # head split; the queries leave it multiplied by scale * log2(e) like the decoder's (the attention's softmax is then the
-            # bare exp2: k_attn_prefill_dma<64, PRE> 59 -> 49 us per layer at 17 crops, tools/clip_attn_probe.py).  Round 6: the split
+            # bare exp2: k_attn_prefill_dma<64, PRE> 59 -> 49 us per layer at 17 crops, tools/clip_attn_probe.py).  The split
             # rides in the projection's epilogue here too (ops.gemm_qkv: Q, K rows and V^T columns straight from the accumulators) --
             # a crop is 577 tokens, so the 8-token V^T runs start one token later in every crop; the epilogue now stores them at
             # whatever offset they fall on (one dwordx4 at even offsets, three stores at odd ones, element-wise across a crop end).
@@ -387,7 +387,7 @@ class Phi3VModel(DecoderModel):
     def _plan_fused_oproj(self, bufs, B, L, T, quantized=False):
         """B = L = 1 decode: attention + o_proj + residual as ONE launch per layer where the library takes the shape -- on bf16 or
         MLX 4-bit weights and a bf16 cache (k_attn_decode128_o / _o4), or on e4m3 weights and the int8 cache (config 5:
-        k_attn_decode128_q8<true>); p3v_attention.hip.  Long contexts (round 6), whose partials are merged by a launch of their own:
+        k_attn_decode128_q8<true>); p3v_attention.hip.  Long contexts, whose partials are merged by a launch of their own:
         that launch carries the o_proj (k_attn_combine_o).  The attention output then lives in two buffers that alternate layers use, both all-ones (= "not written
         yet") between launches; P3V_ATTN_FUSE_OPROJ=0 switches it off."""
         cfg = self.cfg
@@ -402,7 +402,7 @@ class Phi3VModel(DecoderModel):
               and B == 1 and L == 1
               and cfg.num_hidden_layers % 2 == 0 and not self.serving
               and not self.adapters and (o_key in self.w8) == bool(quantized) and not (quantized and o_key in self.w4)
-              # (without the in-launch merge -- long contexts: the MERGE launch carries the o_proj, k_attn_combine_o, round 6)
+              # (without the in-launch merge -- long contexts: the MERGE launch carries the o_proj, k_attn_combine_o)
               and can(B, L, cfg.num_attention_heads, self.hd, bufs["n_split"], T, cfg.hidden_size, bool(bufs.get("attn_merge", False))))
         if not ok and bufs.get("attn_merge", False) and B == 1 and L == 1 and not quantized:
             # Short contexts (64-key one-tile plans: the in-launch form above is for 128-key tiles): attention that only writes its partials

@@ -249,7 +249,7 @@ def synth_weights(cfg, seed=0, device="cpu", std_scale=1.0, lm_head_spread=0.0, 
     std_scale > 1 sharpens the logits of tiny test models (wider top-2 margins);
     lm_head_spread > 0 makes the greedy argmax decisive (`peaked_lm_head`);
     outliers: None | True (= OUTLIERS) | dict of `add_outliers` arguments -> heavy-tailed activations;
-    residual_scale: the WELL-CONDITIONED checkpoint of the parity tests (round 5) -- the decoder's residual-branch output
+    residual_scale: the WELL-CONDITIONED checkpoint of the parity tests -- the decoder's residual-branch output
     projections (o_proj, down_proj) times this factor (True = 1 / sqrt(2 * n_layers), the usual depth-scaled initialisation).
     With plain N(0, 0.02) everywhere each of the 32 layers adds a branch as large as the stream itself and a single bf16
     rounding grows to ~6 % of the logits; depth-scaled, the stream is dominated by the embedding and the
