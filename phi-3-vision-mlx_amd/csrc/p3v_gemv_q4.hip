@@ -10,8 +10,11 @@
 //   SB [N, K/64] u32: scale (bf16) | bias (bf16) << 16.
 // Per 16-weight piece p of a row, with D = sum_k x_k (128 + q_k) and X = sum_k x_k (16 activations, shared by all rows,
 // precomputed in LDS):   contribution = scale * (D - 128 X) + bias * X.
-// Same streaming skeleton as k_gemv3: x (+RMSNorm) staged in LDS, (row pair, stage) pipeline with two register buffers,
-// unconditional loads, branch-free body.  HBM-bound: N*K/2 + N*K/16 bytes per launch.
+// One row (k_gemv3_q4): x (+RMSNorm) staged in LDS while the weights of the wave's first U row pairs are on their way, their sums and their
+// epilogue together at the end.  The bytes (N*K/2 + N*K/16) are a quarter of the bf16 kernel's for as many products, so its instructions count as much as
+// its bytes: 11 per 8 weights, 6 per piece, and one reduction and epilogue per U pairs instead of one each (gate_up: 880 vector instructions a
+// wave, 3 of its 8 us; 1180 before).  16 waves per CU: 4.08 ms per four steps of the 32-layer decoder at 128 columns (8 waves 4.11, 12 4.14, 20 4.12; before 4.52):
+// per launch gate_up 9.0 -> 8.1 us, qkv 7.2 -> 6.6, down 7.1 -> 5.9.
 #include <stdlib.h>
 
 #include <type_traits>
@@ -27,18 +30,37 @@ struct GemvQ4P {
 };
 typedef std::integral_constant<int, 0> QC0;
 typedef std::integral_constant<int, 1> QC1;
+template <int I, int N, class F>
+__device__ __forceinline__ void q4_each(F&& f) {          // f(integral_constant I .. N - 1), unrolled
+  if constexpr (I < N) { f(std::integral_constant<int, I>{}); q4_each<I + 1, N>(f); }
+}
+// one addition of a wave reduction for two values at once: a's in the lower half (even rows of 16 lanes), b's in the upper (odd rows)
+__device__ __forceinline__ float swap32_add(float a, float b) {
+  auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  unsigned x = r[0], y = r[1];
+  asm("" : "+v"(x), "+v"(y));                           // (see rows_swap32)
+  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+}
+__device__ __forceinline__ float swap16_add(float a, float b) {
+  auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  unsigned x = r[0], y = r[1];
+  asm("" : "+v"(x), "+v"(y));
+  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+}
 // NST stages x NP 16-weight pieces per lane per row: K = NST * NP * 64 * 16
 // STEP (p3v_gemv3_body.h): STEP_BEGIN / STEP_END carry the replayed greedy step's two ends, as gemv3_body does for bf16 weights
-template <int NST, int NP, int STEP>
+template <int NST, int NP, int DEPTH, bool ONE, int STEP>
 __device__ __forceinline__ void gemv3_q4_body(const GemvQ4P& p, int units_per_wave, int wpw, unsigned char* smem, float* red, const GemvStepP* sp) {
   constexpr int PIECES = NST * NP * 64;                 // 16-weight pieces per row
   constexpr int K = PIECES * 16, XCH = K / 8;           // 16-byte x chunks
   constexpr int XC = (XCH + 255) / 256;
+  static_assert(DEPTH % NST == 0 && DEPTH / NST <= 4, "whole row pairs, at most four");
+  constexpr int U = DEPTH / NST, LU = U == 3 ? 4 : U;   // row pairs requested together; lanes are dealt to LU of them
   u32x4_t* xs = (u32x4_t*)smem;                         // [K] bf16 x (normalised)
   float* xsum = (float*)(smem + K * 2);                 // [PIECES] sum of the 16 activations of a piece
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool silu = p.epi == P3V_EPI_SILU_MUL, has_res = p.epi == P3V_EPI_RESID_BF16;
-  const int u_begin = wave < wpw ? min(p.units, (blockIdx.x * wpw + wave) * units_per_wave) : p.units;   // (wpw: see p3v_gemv_wpw)
+  const int u_begin = wave < wpw ? min(p.units, ((int)blockIdx.x * wpw + wave) * units_per_wave) : p.units;   // (wpw: see p3v_gemv_wpw)
   const int u_end = min(p.units, u_begin + units_per_wave);
   const int n_st = (u_end - u_begin) * NST;
 
@@ -53,14 +75,14 @@ __device__ __forceinline__ void gemv3_q4_body(const GemvQ4P& p, int units_per_wa
   for (int k = 0; k < XC; ++k) {
     const int c = min(tid + k * 256, XCH - 1);
     xv[k] = ((const u32x4_t*)xrow[0])[c];
-    gv[k] = p.norm_w ? ((const u32x4_t*)p.norm_w)[c] : (u32x4_t){0, 0, 0, 0};
+    gv[k] = ((const u32x4_t*)(p.norm_w ? p.norm_w : xrow[0]))[c];
   }
-  u32x2_t wbuf[2][2][NP];
-  uint32_t sbuf[2][2][NP];
-  uint32_t rbuf[2];
+  u32x2_t wbuf[DEPTH][2][NP];
+  uint32_t sbuf[DEPTH][2][NP];
+  uint32_t rbuf = 0;                                     // residual pair of this lane's unit of the group at hand
   auto issue = [&](int gs, auto bufc) {
     constexpr int buf = decltype(bufc)::value;
-    const int u = min(u_begin + gs / NST, p.units - 1), s = gs % NST;
+    const int u = min(u_begin + gs / NST, u_end - 1), s = gs % NST;         // (beyond the wave's rows: its last pair again)
     const int r0 = silu ? u : 2 * u, r1 = silu ? u + p.N : min(2 * u + 1, p.N - 1);
     const u32x2_t* w0 = (const u32x2_t*)(p.W + (size_t)r0 * (K / 8)) + s * NP * 64 + lane;
     const u32x2_t* w1 = (const u32x2_t*)(p.W + (size_t)r1 * (K / 8)) + s * NP * 64 + lane;
@@ -73,55 +95,70 @@ __device__ __forceinline__ void gemv3_q4_body(const GemvQ4P& p, int units_per_wa
       sbuf[buf][0][j] = s0[j * 16];
       sbuf[buf][1][j] = s1[j * 16];
     }
-    rbuf[buf] = has_res ? *(const uint32_t*)(p.resid + 2 * u) : 0u;
+    __builtin_amdgcn_sched_barrier(0);                   // stage by stage: they are waited for in this order
   };
-  if (n_st > 0) issue(0, QC0{});
-
-  float r = 1.f;
-  if (p.norm_w) {
-    float ss = 0.f;
+  auto stage_x = [&]() {                                 // x (normalised) and its piece sums into LDS: all waves of the workgroup
+    float r = 1.f;
+    if (p.norm_w) {
+      float ss = 0.f;
 #pragma unroll
-    for (int k = 0; k < XC; ++k)
-      if (tid + k * 256 < XCH) {
+      for (int k = 0; k < XC; ++k)
+        if (tid + k * 256 < XCH) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) { const float a = bf16lo(xv[k][j]), b = bf16hi(xv[k][j]); ss += a * a + b * b; }
+          for (int j = 0; j < 4; ++j) { const float a = bf16lo(xv[k][j]), b = bf16hi(xv[k][j]); ss += a * a + b * b; }
+        }
+      ss = wave_sum(ss);
+      if (lane == 0) red[wave] = ss;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      r = rsqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)K + p.eps);
+    }
+#pragma unroll
+    for (int k = 0; k < XC; ++k) {
+      const int c = tid + k * 256;
+      if (c < XCH) {                                       // (wave-uniform: XCH is a multiple of 64)
+        u32x4_t o = xv[k];
+        if (p.norm_w) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            o[j] = rms_pair(xv[k][j], r, gv[k][j]);
+        }
+        xs[c] = o;
+        float t = 0.f;                                     // X of the piece whose halves lie in lanes 2 i and 2 i + 1, from the (rounded) activations the dots see
+#pragma unroll
+        for (int j = 0; j < 4; ++j) { const float h = bf16lo(o[j]) + bf16hi(o[j]); t += h + P3V_DPP_F32(h, 0xB1); }
+        if (!(tid & 1)) xsum[c >> 1] = t;
       }
-    ss = wave_sum(ss);
-    if (lane == 0) red[wave] = ss;
+    }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
-    r = rsqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)K + p.eps);
-  }
-#pragma unroll
-  for (int k = 0; k < XC; ++k) {
-    const int c = tid + k * 256;
-    if (c < XCH) {
-      u32x4_t o = xv[k];
-      if (p.norm_w) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          o[j] = rms_pair(xv[k][j], r, gv[k][j]);
-      }
-      xs[c] = o;
-    }
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  for (int pc = tid; pc < PIECES; pc += 256) {           // X of every piece, from the (rounded) activations the dots see
-    const u32x4_t a = xs[2 * pc], b = xs[2 * pc + 1];
-    float t = 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) t += (bf16lo(a[j]) + bf16hi(a[j])) + (bf16lo(b[j]) + bf16hi(b[j]));
-    xsum[pc] = t;
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-
-  float a0 = 0.f, a1 = 0.f;
+  };
   ArgMaxVI best[1] = {ArgMaxVI{-INFINITY, 0x7fffffff}};      // STEP_END: this wave's arg-max candidate (lane 0's copy counts)
-  auto compute = [&](int gs, auto bufc) {
-    constexpr int buf = decltype(bufc)::value;
-    const int s = gs % NST;
+  auto step_tail = [&]() {
+    if (STEP == STEP_BEGIN && blockIdx.x == 0) gemv_step_begin_tail<1>(sp, xrow, 1, XCH, tid);
+    if (STEP == STEP_END) gemv_step_end_tail<1>(sp, best, 1, (int)blockIdx.x, tid);
+  };
+  // A wave without rows has a path of its own: where its path met the others', hipcc would count only the loads that both issued, and
+  // the wait for x would be one for all weights (it was: the norm began when the first rows had landed).
+  if (n_st <= 0) {
+    stage_x();
+    step_tail();
+    return;
+  }
+  const int unit_of = LU == 1 ? 0 : lane / (64 / LU);            // pair of a group whose sums end in this lane
+  auto resid_of = [&](int gs) {                                  // (an unconditional load: x where there is no residual)
+    return *(const uint32_t*)(has_res ? p.resid + 2 * min(u_begin + gs / NST + unit_of, u_end - 1) : xrow[0]);
+  };
+  q4_each<0, DEPTH>([&](auto d) { issue(d, d); });
+  rbuf = resid_of(0);
+  stage_x();
+
+  // A group of U row pairs: their sums stay in the lanes until all are there, the last two steps of the reduction serve two pairs
+  // each (the additions of wave_sum, in its order), and the epilogue runs once, lane unit_of * 64 / LU holding pair unit_of.
+  float acc[U][2];
+  auto compute = [&](auto dc) {
+    constexpr int d = decltype(dc)::value, un = d / NST, s = d % NST;
+    if constexpr (s == 0) acc[un][0] = acc[un][1] = 0.f;
 #pragma unroll
     for (int j = 0; j < NP; ++j) {
       const int pc = (s * NP + j) * 64 + lane;
@@ -129,64 +166,81 @@ __device__ __forceinline__ void gemv3_q4_body(const GemvQ4P& p, int units_per_wa
       const float X = xsum[pc], X128 = 128.f * X;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const u32x2_t w = wbuf[buf][h][j];
+        const u32x2_t w = wbuf[d][h][j];
         const float D = dot8_q4(w[1], xb, dot8_q4(w[0], xa, 0.f));
-        const uint32_t sb = sbuf[buf][h][j];
-        const float c = bf16lo(sb) * (D - X128) + bf16hi(sb) * X;
-        if (h == 0) a0 += c; else a1 += c;
+        const uint32_t sb = sbuf[d][h][j];
+        acc[un][h] += bf16lo(sb) * (D - X128) + bf16hi(sb) * X;
       }
     }
-    if (s == NST - 1) {
-      const int u = u_begin + gs / NST;
-      a0 = wave_sum(a0);
-      a1 = wave_sum(a1);
-      if (lane == 0) {
-        if (silu) {
-          const float g = bf16_round(a0), up = bf16_round(a1);
-          ((bf16_t*)p.out)[u] = f32_to_bf16(bf16_round(g * bf16_round(1.f / (1.f + __expf(-g)))) * up);
-        } else if (p.epi == P3V_EPI_F32) {
-          ((float*)p.out)[2 * u] = a0;
-          ((float*)p.out)[2 * u + 1] = a1;
-        } else {
-          float v0 = a0, v1 = a1;
-          if (has_res) { v0 = bf16lo(rbuf[buf]) + bf16_round(v0); v1 = bf16hi(rbuf[buf]) + bf16_round(v1); }
-          *(uint32_t*)((bf16_t*)p.out + 2 * u) = pack_bf16x2(v0, v1);
-          if (STEP == STEP_END) {                              // on the values just stored (bf16)
-            amax_take(best[0], bf16_round(v0), 2 * u);
-            if (2 * u + 1 < p.N) amax_take(best[0], bf16_round(v1), 2 * u + 1);
-          }
-        }
+  };
+  auto finish = [&](int u0) {
+    float v[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float t[4];
+#pragma unroll
+      for (int k = 0; k < LU; ++k) {
+        t[k] = acc[k < U ? k : U - 1][h];
+        if (k >= U) continue;
+        t[k] += P3V_DPP_F32(t[k], 0xB1);
+        t[k] += P3V_DPP_F32(t[k], 0x4E);
+        t[k] += P3V_DPP_F32(t[k], 0x124);
+        t[k] += P3V_DPP_F32(t[k], 0x128);
       }
-      a0 = a1 = 0.f;
+      if constexpr (LU == 1) v[h] = rows_sum(t[0]);
+      if constexpr (LU == 2) v[h] = swap16_add(swap32_add(t[0], t[1]), swap32_add(t[0], t[1]));
+      if constexpr (LU == 4) v[h] = swap16_add(swap32_add(t[0], t[2]), swap32_add(t[1], t[3]));
+    }
+    const int u = u0 + unit_of;
+    if ((lane & (64 / LU - 1)) || u >= u_end || unit_of >= U) return;
+    if (silu) {
+      const float g = bf16_round(v[0]), up = bf16_round(v[1]);
+      ((bf16_t*)p.out)[u] = f32_to_bf16(bf16_round(g * bf16_round(1.f / (1.f + __expf(-g)))) * up);
+    } else if (p.epi == P3V_EPI_F32) {
+      ((float*)p.out)[2 * u] = v[0];
+      ((float*)p.out)[2 * u + 1] = v[1];
+    } else {
+      if (has_res) { v[0] = bf16lo(rbuf) + bf16_round(v[0]); v[1] = bf16hi(rbuf) + bf16_round(v[1]); }
+      *(uint32_t*)((bf16_t*)p.out + 2 * u) = pack_bf16x2(v[0], v[1]);
+      if (STEP == STEP_END) {                                    // on the values just stored (bf16)
+        amax_take(best[0], bf16_round(v[0]), 2 * u);
+        if (2 * u + 1 < p.N) amax_take(best[0], bf16_round(v[1]), 2 * u + 1);
+      }
     }
   };
   int gs = 0;
-  while (gs + 2 < n_st) {
-    issue(gs + 1, QC1{}); compute(gs, QC0{});
-    issue(gs + 2, QC0{}); compute(gs + 1, QC1{});
-    gs += 2;
+  for (; !ONE && gs + DEPTH < n_st; gs += DEPTH) {
+    const uint32_t next = resid_of(gs + DEPTH);
+    q4_each<0, DEPTH>([&](auto d) { compute(d); issue(gs + DEPTH + d, d); });
+    finish(u_begin + gs / NST);
+    rbuf = next;
   }
-  if (gs + 1 < n_st) {
-    issue(gs + 1, QC1{}); compute(gs, QC0{}); compute(gs + 1, QC1{});
-  } else if (gs < n_st) {
-    compute(gs, QC0{});
+  q4_each<0, DEPTH>([&](auto d) { compute(d); });
+  finish(u_begin + gs / NST);
+  if (STEP == STEP_END && LU > 1) {                              // the lanes that finished a pair: their candidates meet in lane 0
+#pragma unroll
+    for (int off = 64 / LU; off < 64; off <<= 1) {
+      ArgMaxVI o;
+      o.v = __shfl_xor(best[0].v, off, 64);
+      o.i = __shfl_xor(best[0].i, off, 64);
+      best[0] = amax_better(best[0], o);
+    }
   }
-  if (STEP == STEP_BEGIN && blockIdx.x == 0) gemv_step_begin_tail<1>(sp, xrow, 1, XCH, tid);
-  if (STEP == STEP_END) gemv_step_end_tail<1>(sp, best, 1, (int)blockIdx.x, tid);
+  step_tail();
 }
 
-template <int NST, int NP>
+template <int NST, int NP, int DEPTH, bool ONE>
 __global__ void __launch_bounds__(256) k_gemv3_q4(GemvQ4P p, int units_per_wave, int wpw) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ float red[4];
-  gemv3_q4_body<NST, NP, STEP_NONE>(p, units_per_wave, wpw, smem, red, nullptr);
+  gemv3_q4_body<NST, NP, DEPTH, ONE, STEP_NONE>(p, units_per_wave, wpw, smem, red, nullptr);
 }
 
-template <int NST, int NP, int STEP>
+template <int NST, int NP, int DEPTH, bool ONE, int STEP>
 __global__ void __launch_bounds__(256) k_gemv3_q4_step(GemvQ4P p, int units_per_wave, int wpw, GemvStepP sp) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ float red[4];
-  gemv3_q4_body<NST, NP, STEP>(p, units_per_wave, wpw, smem, red, &sp);
+  gemv3_q4_body<NST, NP, DEPTH, ONE, STEP>(p, units_per_wave, wpw, smem, red, &sp);
 }
 
 // W4 / SB -> bf16 [rows, K] (prefill and batched decode run the bf16 kernels on a dequantised scratch copy)
@@ -228,12 +282,26 @@ static int launch_gemv3_q4(const GemvQ4P& p, hipStream_t s, const GemvStepP* sp 
   int upw = p3v_cdiv(p.units, n_cu * wpc);
   if (upw < 1) upw = 1;
   const int waves = p3v_cdiv(p.units, upw);
-  const int wpw = p3v_gemv_wpw(waves, n_cu, p3v_tuning().gemv_wpw);
-  if constexpr (STEP != STEP_NONE) {
-    if (p3v_cdiv(waves, wpw) > P3V_GEMV_STEP_MAX_WG) return P3V_ERR_UNSUPPORTED;        // (amax_ws holds one candidate per workgroup)
-    hipLaunchKernelGGL((k_gemv3_q4_step<NST, NP, STEP>), dim3(p3v_cdiv(waves, wpw)), dim3(256), (size_t)p.K * 2 + (size_t)p.K / 4, s, p, upw, wpw, *sp);
-  } else {
-    hipLaunchKernelGGL((k_gemv3_q4<NST, NP>), dim3(p3v_cdiv(waves, wpw)), dim3(256), (size_t)p.K * 2 + (size_t)p.K / 4, s, p, upw, wpw);
+  int wpw = p3v_gemv_wpw(waves, n_cu, p3v_tuning().gemv_wpw);
+  if (STEP != STEP_NONE && p3v_cdiv(waves, wpw) > P3V_GEMV_STEP_MAX_WG) wpw = 4;
+  const dim3 grid(p3v_cdiv(waves, wpw));
+  const size_t lds = (size_t)p.K * 2 + (size_t)p.K / 4;
+  if (STEP != STEP_NONE && (int)grid.x > P3V_GEMV_STEP_MAX_WG) return P3V_ERR_UNSUPPORTED;   // (amax_ws holds one candidate per workgroup)
+  const int pairs = upw <= 4 / NST ? upw : NST == 1 && upw % 4 && upw % 3 == 0 ? 3 : 4 / NST;
+  auto launch = [&](auto d) {
+    if constexpr (STEP != STEP_NONE) {
+      if (upw == pairs) hipLaunchKernelGGL((k_gemv3_q4_step<NST, NP, d(), true, STEP>), grid, dim3(256), lds, s, p, upw, wpw, *sp);
+      else hipLaunchKernelGGL((k_gemv3_q4_step<NST, NP, d(), false, STEP>), grid, dim3(256), lds, s, p, upw, wpw, *sp);
+    } else {
+      if (upw == pairs) hipLaunchKernelGGL((k_gemv3_q4<NST, NP, d(), true>), grid, dim3(256), lds, s, p, upw, wpw);
+      else hipLaunchKernelGGL((k_gemv3_q4<NST, NP, d(), false>), grid, dim3(256), lds, s, p, upw, wpw);
+    }
+  };
+  if (pairs == 1) launch(std::integral_constant<int, NST>{});
+  else if (pairs == 2) launch(std::integral_constant<int, 2 * NST>{});
+  else if constexpr (NST == 1) {
+    if (pairs == 3) launch(std::integral_constant<int, 3>{});
+    else launch(std::integral_constant<int, 4>{});
   }
   P3V_CHECK_LAUNCH();
   return P3V_OK;

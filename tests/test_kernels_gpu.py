@@ -1601,6 +1601,43 @@ def test_gemv_q4_and_dequant(ops, N, K, epi, norm):
     close(got, ref, rtol=2 ** -6, atol=3e-2)
 
 
+@pytest.mark.parametrize("K,pairs", [(3072, (1, 2, 257, 511, 513, 700, 768, 1025, 1281, 1500, 2049)), (8192, (1, 257, 513, 770))])
+@pytest.mark.parametrize("epi", ["none", "silu", "f32", "resid"])
+def test_gemv_q4_row_groups(ops, K, pairs, epi):
+    """One row, every number of row pairs a wave may hold (1 .. 4 at once, then several groups, the last of them short; waves without rows):
+    one wave per CU is asked for, so that few rows are many per wave.  Against the product in 64 bits: a piece of 16 sums x (128 + q) in
+    fp32, an error of up to 16 * 143 * 2^-24 scale per |x|, and its 192 .. 512 pieces are added in 12 .. 16 steps; with max |w| = 8 scale
+    both are below 2^-15 max |w| sum |x|.  Beside it the rounding of the bf16 result."""
+    from phi_3_vision_mlx_amd.ops import EPI_F32, EPI_NONE, EPI_RESID_BF16, EPI_SILU_MUL
+    from phi_3_vision_mlx_amd.weights import mlx_dequantize, mlx_quantize, q4_repack
+    e = {"none": EPI_NONE, "resid": EPI_RESID_BF16, "silu": EPI_SILU_MUL, "f32": EPI_F32}[epi]
+    w = g((2 * max(pairs) * (2 if epi == "silu" else 1), K), 410, 0.03)
+    packed, sc, bi = mlx_quantize(w)
+    wd = mlx_dequantize(packed, sc, bi).cuda()
+    x = g((1, K), 411).cuda()
+    old = ops.set_tuning("gemv_q4_wpc", 1)
+    try:
+        for n in pairs:
+            N = 2 * n
+            rows = 2 * N if epi == "silu" else N
+            w4, sb = (t.cuda() for t in q4_repack(packed[:rows], sc[:rows], bi[:rows]))
+            res = g((1, N), 412).cuda()
+            buf = torch.full((1, N + 64), 7.0, dtype=F32 if epi == "f32" else BF16).cuda()      # behind the row: untouched
+            got = ops.gemv_q4(x, w4, sb, e, resid=res if epi == "resid" else None, out=buf[:, :N])
+            assert torch.all(buf[:, N:] == 7.0)
+            y = x.double() @ wd[:rows].double().t()
+            tol = 2.0 ** -15 * wd.abs().max() * x.double().abs().sum()
+            if epi == "silu":
+                gt, up = y[:, :N], y[:, N:]
+                ref, tol = torch.nn.functional.silu(gt) * up, tol * (1 + gt.abs() + up.abs())
+            else:
+                ref = y + res.double() if epi == "resid" else y
+            slack = {"none": 2.0 ** -8, "resid": 2.0 ** -7, "silu": 2.0 ** -5, "f32": 0.0}[epi] * (ref.abs() + (y[:, :N].abs() if epi == "resid" else 0))
+            assert torch.all((got.double() - ref).abs() <= slack + tol), (n, (got.double() - ref).abs().max())
+    finally:
+        ops.set_tuning("gemv_q4_wpc", old)
+
+
 @pytest.mark.parametrize("M", [2, 5, 8, 15, 16])
 @pytest.mark.parametrize("N,K,epi", [(9216, 3072, "none"), (3072, 3072, "resid"), (8192, 3072, "silu"), (3072, 8192, "resid"), (32064, 3072, "none")])
 def test_gemv_q4_rows_2_to_16(ops, N, K, epi, M):
