@@ -132,8 +132,9 @@ static int launch_gemv(const GemvP& p, hipStream_t s) {
 // written so that hipcc can keep COUNTED s_waitcnt vmcnt(N) everywhere -- every load is
 // unconditional and the pipeline body is branch-free (a predicated load or a branch between
 // issue and use makes the compiler fall back to vmcnt(0), which drains the prefetch):
-//   * x (+ norm weight) chunks are requested first, then the wave's first weight stage, so
-//     the RMSNorm prologue waits only for the older x loads while the weights stream in;
+//   * x (+ norm weight) chunks are requested first, then the wave's first two weight stages, so
+//     the RMSNorm prologue waits only for the older x loads while the weights stream in (before, it
+//     waited for the first stage with no second one requested: 6744 -> 6681 us per four steps at 2531 columns);
 //   * (row pair, K stage) software pipeline with two register buffers: stage s+1 is in
 //     flight (2*CH 16-byte loads per lane) while stage s is reduced; the residual needed by
 //     the epilogue travels with the stage (no dependent load at the end of a row);
@@ -148,27 +149,27 @@ extern "C" int p3v_gemv_timing_read(long long* out, int n) {
 #else
 #define GMARK(k)
 #endif
-template <int MT, int NST, int CH>
+template <int MT, int NST, int CH, int NS>
 __global__ void __launch_bounds__(256) k_gemv3(GemvP p, int units_per_wave, int wpw) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ float red[8];
   GMARK(0);
-  gemv3_body<MT, NST, CH>(p, units_per_wave, blockIdx.x, smem, red, wpw);
+  gemv3_body<MT, NST, CH, STEP_NONE, 0, NS>(p, units_per_wave, blockIdx.x, smem, red, wpw);
   GMARK(1);
 }
 
-template <int NST, int CH, int VAR>
+template <int NST, int CH, int VAR, int NS>
 __global__ void __launch_bounds__(256) k_gemv3_layered(GemvP p, int units_per_wave, int wpw) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ float red[8];
-  gemv3_body<1, NST, CH, STEP_NONE, VAR>(p, units_per_wave, blockIdx.x, smem, red, wpw);
+  gemv3_body<1, NST, CH, STEP_NONE, VAR, NS>(p, units_per_wave, blockIdx.x, smem, red, wpw);
 }
 
-template <int MT, int NST, int CH, int STEP>
+template <int MT, int NST, int CH, int STEP, int NS>
 __global__ void __launch_bounds__(256) k_gemv3_step(GemvP p, int units_per_wave, int wpw, GemvStepP sp) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ float red[8];
-  gemv3_body<MT, NST, CH, STEP>(p, units_per_wave, blockIdx.x, smem, red, wpw, &sp);
+  gemv3_body<MT, NST, CH, STEP, 0, NS>(p, units_per_wave, blockIdx.x, smem, red, wpw, &sp);
 }
 
 template <int MT, int NST, int CH, int STEP = STEP_NONE, int VAR = 0>
@@ -186,20 +187,37 @@ static int launch_gemv3(const GemvP& p, hipStream_t s, const GemvStepP* sp = nul
   const int waves = p3v_cdiv(p.units, upw);
   const int wpw_ = p3v_gemv_wpw(waves, n_cu, p3v_tuning().gemv_wpw);   // 4 or 3 row-streaming waves per workgroup
   const size_t lds = (size_t)MT * p.K * 2;
-  static bool attr_set = false;
-  if (!attr_set && lds > 48 * 1024) {
-    if (hipFuncSetAttribute((const void*)k_gemv3<MT, NST, CH>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256) != hipSuccess)
-      return P3V_ERR_HIP;
-    attr_set = true;
+  const dim3 grid(p3v_cdiv(waves, wpw_));
+  if (STEP != STEP_NONE && (int)grid.x > P3V_GEMV_STEP_MAX_WG) return P3V_ERR_UNSUPPORTED;      // (amax_ws holds one candidate per workgroup and row)
+  int rc = P3V_OK;
+  auto launch = [&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    if constexpr (MT > 1) {
+      static bool attr_set = false;
+      if (!attr_set && lds > 48 * 1024) {
+        if (hipFuncSetAttribute((const void*)k_gemv3<MT, NST, CH, NS>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256) != hipSuccess) {
+          rc = P3V_ERR_HIP;
+          return;
+        }
+        attr_set = true;
+      }
+    }
+    if constexpr (VAR != 0) hipLaunchKernelGGL((k_gemv3_layered<NST, CH, VAR, NS>), grid, dim3(256), lds, s, p, upw, wpw_);
+    else if constexpr (STEP != STEP_NONE) hipLaunchKernelGGL((k_gemv3_step<MT, NST, CH, STEP, NS>), grid, dim3(256), lds, s, p, upw, wpw_, *sp);
+    else hipLaunchKernelGGL((k_gemv3<MT, NST, CH, NS>), grid, dim3(256), lds, s, p, upw, wpw_);
+  };
+  const int n_st = MT == 1 && upw * NST <= 4 ? upw * NST : 0;
+  auto exact = [&](auto ns) {                             // (a number of steps that whole row pairs can make)
+    if constexpr (MT == 1 && decltype(ns)::value % NST == 0) launch(ns);
+  };
+  switch (n_st) {
+    case 1: exact(std::integral_constant<int, 1>{}); break;
+    case 2: exact(std::integral_constant<int, 2>{}); break;
+    case 3: exact(std::integral_constant<int, 3>{}); break;
+    case 4: exact(std::integral_constant<int, 4>{}); break;
+    default: launch(IC0{});
   }
-  if constexpr (VAR != 0) {
-    hipLaunchKernelGGL((k_gemv3_layered<NST, CH, VAR>), dim3(p3v_cdiv(waves, wpw_)), dim3(256), lds, s, p, upw, wpw_);
-  } else if constexpr (STEP != STEP_NONE) {
-    if (p3v_cdiv(waves, wpw_) > P3V_GEMV_STEP_MAX_WG) return P3V_ERR_UNSUPPORTED;      // (amax_ws holds one candidate per workgroup and row)
-    hipLaunchKernelGGL((k_gemv3_step<MT, NST, CH, STEP>), dim3(p3v_cdiv(waves, wpw_)), dim3(256), lds, s, p, upw, wpw_, *sp);
-  } else {
-    hipLaunchKernelGGL((k_gemv3<MT, NST, CH>), dim3(p3v_cdiv(waves, wpw_)), dim3(256), lds, s, p, upw, wpw_);
-  }
+  if (rc != P3V_OK) return rc;
   P3V_CHECK_LAUNCH();
   return P3V_OK;
 }

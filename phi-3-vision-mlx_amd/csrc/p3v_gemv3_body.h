@@ -154,13 +154,22 @@ __device__ __forceinline__ void gemv_step_end_tail(const GemvStepP* sp, const Ar
 // wpw: waves of the 4-wave workgroup that take rows (4, or 3: wave 3 then only helps with the prologue).  1536 streaming waves
 // (qkv, o_proj, down) as 384 four-wave workgroups put two workgroups on half of the CUs and one on the others, and the launch
 // lasts as long as the doubly loaded CUs; 512 workgroups x 3 waves load every CU alike (tools/gemv_timeline.py).
-template <int MT, int NST, int CH, int STEP = STEP_NONE, int VAR = 0>
+//
+// NS: (row pair, K stage) steps of a full wave where the launcher knows them (1 .. 4): straight-line code; 0: any number, in a loop.
+// Two steps' weights are requested ahead of the norm, and no branch stands between a request and its use: where a path without a
+// request joins one with it, hipcc counts only what both issued, and the wait for x becomes a wait for the weights (it was: the norm
+// then ran with nothing on its way, half a microsecond of every launch).
+template <int I, int N, class F>
+__device__ __forceinline__ void gemv_each(F&& f) {        // f(integral_constant I .. N - 1), unrolled
+  if constexpr (I < N) { f(std::integral_constant<int, I>{}); gemv_each<I + 1, N>(f); }
+}
+template <int MT, int NST, int CH, int STEP = STEP_NONE, int VAR = 0, int NS = 0>
 __device__ __forceinline__ void gemv3_body(const GemvP& p, int units_per_wave, int bx, unsigned char* smem, float* red, int wpw = 4,
                                            const GemvStepP* sp = nullptr) {
   constexpr int CHUNKS = NST * CH * 64;                 // 16-byte chunks per row (K = 8 * CHUNKS)
   constexpr int XC = (CHUNKS + 255) / 256;              // x chunks per thread
   u32x4_t* xs = (u32x4_t*)smem;                         // [MT][CHUNKS] bf16 x (normalised)
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool silu = VAR ? P3V_GATED(p.epi) : p.epi == P3V_EPI_SILU_MUL;
   const bool has_res = p.epi == P3V_EPI_RESID_BF16;
   const int u_begin = wave < wpw ? min(p.units, (bx * wpw + wave) * units_per_wave) : p.units;
@@ -215,7 +224,7 @@ __device__ __forceinline__ void gemv3_body(const GemvP& p, int units_per_wave, i
     for (int m = 0; m < MT; ++m)
       if constexpr (!DYT && !RMS) xv[m][k] = ((const u32x4_t*)xrow[m])[c];
     if constexpr (DYT || RMS) gv[k] = ((const u32x4_t*)p.dyt.w)[c];
-    else gv[k] = p.norm_w ? ((const u32x4_t*)p.norm_w)[c] : (u32x4_t){0, 0, 0, 0};
+    else gv[k] = ((const u32x4_t*)(p.norm_w ? p.norm_w : xrow[0]))[c];      // (unused without a norm, and requested all the same)
   }
 
   // ---- 2. weight pipeline state
@@ -224,7 +233,7 @@ __device__ __forceinline__ void gemv3_body(const GemvP& p, int units_per_wave, i
   float2 fbuf[2];                                        // GEMV_SCALED: the fp32 residual pair, rbuf its column scales
   auto issue = [&](int gs, auto bufc) {
     constexpr int buf = decltype(bufc)::value;
-    const int u = min(u_begin + gs / NST, p.units - 1), s = gs % NST;
+    const int u = min(u_begin + gs / NST, u_end - 1), s = gs % NST;       // (beyond the wave's rows: its last pair again)
     const int r0 = silu ? u : 2 * u;
     const int r1 = silu ? u + p.N : min(2 * u + 1, p.N - 1);
     const u32x4_t* w0 = (const u32x4_t*)(p.W + (size_t)r0 * (CHUNKS * 8)) + s * CH * 64 + lane;
@@ -240,103 +249,117 @@ __device__ __forceinline__ void gemv3_body(const GemvP& p, int units_per_wave, i
     }
 #pragma unroll
     for (int m = 0; m < (SCALED ? 0 : MT); ++m) {        // 4-byte aligned: r0 = 2u is even, N is even on this path
-      const bf16_t* rp = p.resid + (size_t)min(m, p.M - 1) * p.N + 2 * u;
-      rbuf[buf][m] = !has_res ? 0u : *(const uint32_t*)rp;
+      rbuf[buf][m] = *(const uint32_t*)(has_res ? p.resid + (size_t)min(m, p.M - 1) * p.N + 2 * u : (const bf16_t*)p.W);
     }
+    __builtin_amdgcn_sched_barrier(0);                   // step by step: they are waited for in this order
   };
-  if (n_st > 0) issue(0, IC0{});
 
   // ---- 3. RMSNorm prologue (waits for the x loads only) -> LDS
-  if constexpr (DYT) {
-    const float al = p.dyt.alpha;
-#pragma unroll
-    for (int k = 0; k < XC; ++k) {
-      const int c = tid + k * 256;
-      if (c < CHUNKS) {
-        const float xe[8] = {dx[k][0].x, dx[k][0].y, dx[k][0].z, dx[k][0].w, dx[k][1].x, dx[k][1].y, dx[k][1].z, dx[k][1].w};
-        const float pe[8] = {dh[k][0].x, dh[k][0].y, dh[k][0].z, dh[k][0].w, dh[k][1].x, dh[k][1].y, dh[k][1].z, dh[k][1].w};
-        float h[8], s[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float g = j & 1 ? bf16hi(gv[k][j >> 1]) : bf16lo(gv[k][j >> 1]), b = j & 1 ? bf16hi(db[k][j >> 1]) : bf16lo(db[k][j >> 1]);
-          h[j] = tanhf(xe[j] * al) * g + b;
-          const float mu = j & 1 ? bf16hi(dm[k][j >> 1]) : bf16lo(dm[k][j >> 1]);
-          s[j] = p.dyt.mu ? h[j] + ((d_prev ? pe[j] : 0.f) - h[j]) * mu : h[j];
-        }
-        xs[c] = (u32x4_t){pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]), pack_bf16x2(s[4], s[5]), pack_bf16x2(s[6], s[7])};
-        if (p.dyt.mu && bx == 0) {                        // (another slot than the one every workgroup reads: R >= 2)
-          float4* hw = (float4*)(p.dyt.hist + (size_t)(d_pos % p.dyt.R) * (CHUNKS * 8)) + 2 * c;
-          hw[0] = make_float4(h[0], h[1], h[2], h[3]), hw[1] = make_float4(h[4], h[5], h[6], h[7]);
-        }
-      }
-    }
-  }
-  if constexpr (RMS) {
-    float ss = 0.f;
-#pragma unroll
-    for (int k = 0; k < XC; ++k)
-      if (tid + k * 256 < CHUNKS) {
-        ss += dx[k][0].x * dx[k][0].x + dx[k][0].y * dx[k][0].y + dx[k][0].z * dx[k][0].z + dx[k][0].w * dx[k][0].w;
-        ss += dx[k][1].x * dx[k][1].x + dx[k][1].y * dx[k][1].y + dx[k][1].z * dx[k][1].z + dx[k][1].w * dx[k][1].w;
-      }
-    ss = wave_sum(ss);
-    if (lane == 0) red[wave] = ss;
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    const float r = p.dyt.alpha / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)(CHUNKS * 8) + p.eps);
-#pragma unroll
-    for (int k = 0; k < XC; ++k) {
-      const int c = tid + k * 256;
-      if (c < CHUNKS)
-        xs[c] = (u32x4_t){pack_bf16x2(dx[k][0].x * (r * bf16lo(gv[k][0])), dx[k][0].y * (r * bf16hi(gv[k][0]))),
-                          pack_bf16x2(dx[k][0].z * (r * bf16lo(gv[k][1])), dx[k][0].w * (r * bf16hi(gv[k][1]))),
-                          pack_bf16x2(dx[k][1].x * (r * bf16lo(gv[k][2])), dx[k][1].y * (r * bf16hi(gv[k][2]))),
-                          pack_bf16x2(dx[k][1].z * (r * bf16lo(gv[k][3])), dx[k][1].w * (r * bf16hi(gv[k][3])))};
-    }
-  }
-#pragma unroll
-  for (int m = 0; m < (DYT || RMS ? 0 : MT); ++m) {
-    float r = 1.f;
-    if (p.norm_w) {
-      float ss = 0.f;
+  auto stage_x = [&]() {
+    if constexpr (DYT) {
+      const float al = p.dyt.alpha;
 #pragma unroll
       for (int k = 0; k < XC; ++k) {
-        if (tid + k * 256 < CHUNKS) {
+        const int c = tid + k * 256;
+        if (c < CHUNKS) {
+          const float xe[8] = {dx[k][0].x, dx[k][0].y, dx[k][0].z, dx[k][0].w, dx[k][1].x, dx[k][1].y, dx[k][1].z, dx[k][1].w};
+          const float pe[8] = {dh[k][0].x, dh[k][0].y, dh[k][0].z, dh[k][0].w, dh[k][1].x, dh[k][1].y, dh[k][1].z, dh[k][1].w};
+          float h[8], s[8];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) { const float a = bf16lo(xv[m][k][j]), b = bf16hi(xv[m][k][j]); ss += a * a + b * b; }
+          for (int j = 0; j < 8; ++j) {
+            const float g = j & 1 ? bf16hi(gv[k][j >> 1]) : bf16lo(gv[k][j >> 1]), b = j & 1 ? bf16hi(db[k][j >> 1]) : bf16lo(db[k][j >> 1]);
+            h[j] = tanhf(xe[j] * al) * g + b;
+            const float mu = j & 1 ? bf16hi(dm[k][j >> 1]) : bf16lo(dm[k][j >> 1]);
+            s[j] = p.dyt.mu ? h[j] + ((d_prev ? pe[j] : 0.f) - h[j]) * mu : h[j];
+          }
+          xs[c] = (u32x4_t){pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]), pack_bf16x2(s[4], s[5]), pack_bf16x2(s[6], s[7])};
+          if (p.dyt.mu && bx == 0) {                        // (another slot than the one every workgroup reads: R >= 2)
+            float4* hw = (float4*)(p.dyt.hist + (size_t)(d_pos % p.dyt.R) * (CHUNKS * 8)) + 2 * c;
+            hw[0] = make_float4(h[0], h[1], h[2], h[3]), hw[1] = make_float4(h[4], h[5], h[6], h[7]);
+          }
         }
       }
+    }
+    if constexpr (RMS) {
+      float ss = 0.f;
+#pragma unroll
+      for (int k = 0; k < XC; ++k)
+        if (tid + k * 256 < CHUNKS) {
+          ss += dx[k][0].x * dx[k][0].x + dx[k][0].y * dx[k][0].y + dx[k][0].z * dx[k][0].z + dx[k][0].w * dx[k][0].w;
+          ss += dx[k][1].x * dx[k][1].x + dx[k][1].y * dx[k][1].y + dx[k][1].z * dx[k][1].z + dx[k][1].w * dx[k][1].w;
+        }
       ss = wave_sum(ss);
-      if (lane == 0) red[wave + 4 * (m & 1)] = ss;
+      if (lane == 0) red[wave] = ss;
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
-      const float* rr = red + 4 * (m & 1);
-      r = rsqrtf(((rr[0] + rr[1]) + (rr[2] + rr[3])) / (float)(CHUNKS * 8) + p.eps);
-    }
+      const float r = p.dyt.alpha / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)(CHUNKS * 8) + p.eps);
 #pragma unroll
-    for (int k = 0; k < XC; ++k) {
-      const int c = tid + k * 256;
-      if (c < CHUNKS) {
-        u32x4_t o = xv[m][k];
-        if (p.norm_w) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            o[j] = rms_pair(xv[m][k][j], r, gv[k][j]);
-        }
-        xs[m * CHUNKS + c] = m < p.M ? o : (u32x4_t){0, 0, 0, 0};
+      for (int k = 0; k < XC; ++k) {
+        const int c = tid + k * 256;
+        if (c < CHUNKS)
+          xs[c] = (u32x4_t){pack_bf16x2(dx[k][0].x * (r * bf16lo(gv[k][0])), dx[k][0].y * (r * bf16hi(gv[k][0]))),
+                            pack_bf16x2(dx[k][0].z * (r * bf16lo(gv[k][1])), dx[k][0].w * (r * bf16hi(gv[k][1]))),
+                            pack_bf16x2(dx[k][1].x * (r * bf16lo(gv[k][2])), dx[k][1].y * (r * bf16hi(gv[k][2]))),
+                            pack_bf16x2(dx[k][1].z * (r * bf16lo(gv[k][3])), dx[k][1].w * (r * bf16hi(gv[k][3])))};
       }
     }
+#pragma unroll
+    for (int m = 0; m < (DYT || RMS ? 0 : MT); ++m) {
+      float r = 1.f;
+      if (p.norm_w) {
+        float ss = 0.f;
+#pragma unroll
+        for (int k = 0; k < XC; ++k) {
+          if (tid + k * 256 < CHUNKS) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { const float a = bf16lo(xv[m][k][j]), b = bf16hi(xv[m][k][j]); ss += a * a + b * b; }
+          }
+        }
+        ss = wave_sum(ss);
+        if (lane == 0) red[wave + 4 * (m & 1)] = ss;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        const float* rr = red + 4 * (m & 1);
+        r = rsqrtf(((rr[0] + rr[1]) + (rr[2] + rr[3])) / (float)(CHUNKS * 8) + p.eps);
+      }
+#pragma unroll
+      for (int k = 0; k < XC; ++k) {
+        const int c = tid + k * 256;
+        if (c < CHUNKS) {
+          u32x4_t o = xv[m][k];
+          if (p.norm_w) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              o[j] = rms_pair(xv[m][k][j], r, gv[k][j]);
+          }
+          xs[m * CHUNKS + c] = m < p.M ? o : (u32x4_t){0, 0, 0, 0};
+        }
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+  };
+
+  ArgMaxVI best[MT];                                         // STEP_END: this wave's arg-max candidates (lane 0's copy counts)
+#pragma unroll
+  for (int m = 0; m < MT; ++m) best[m] = ArgMaxVI{-INFINITY, 0x7fffffff};
+  auto step_tail = [&]() {
+    if (STEP == STEP_BEGIN && bx == 0) gemv_step_begin_tail<MT>(sp, xrow, p.M, CHUNKS, tid);
+    if (STEP == STEP_END) gemv_step_end_tail<MT>(sp, best, p.M, bx, tid);
+  };
+  if (n_st <= 0) {                                       // a wave without rows: its own path
+    stage_x();
+    step_tail();
+    return;
   }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
+  issue(0, IC0{});
+  if constexpr (NS != 1) issue(1, IC1{});
+  stage_x();
 
   // ---- 4. pipeline
   float a0[MT], a1[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) a0[m] = a1[m] = 0.f;
-  ArgMaxVI best[MT];                                         // STEP_END: this wave's arg-max candidates (lane 0's copy counts)
-#pragma unroll
-  for (int m = 0; m < MT; ++m) best[m] = ArgMaxVI{-INFINITY, 0x7fffffff};
   auto compute = [&](int gs, auto bufc) {
     constexpr int buf = decltype(bufc)::value;
     const int s = gs % NST;
@@ -353,7 +376,7 @@ __device__ __forceinline__ void gemv3_body(const GemvP& p, int units_per_wave, i
       const int u = u_begin + gs / NST;
 #pragma unroll
       for (int m = 0; m < MT; ++m) { a0[m] = wave_sum(a0[m]); a1[m] = wave_sum(a1[m]); }
-      if (lane == 0) {
+      if (lane == 0 && u < u_end) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
           if (m < p.M) {
@@ -381,21 +404,27 @@ __device__ __forceinline__ void gemv3_body(const GemvP& p, int units_per_wave, i
       for (int m = 0; m < MT; ++m) a0[m] = a1[m] = 0.f;
     }
   };
-  int gs = 0;
-  while (gs + 2 < n_st) {                                 // branch-free body: counted vmcnt survives
-    issue(gs + 1, IC1{});
-    compute(gs, IC0{});
-    issue(gs + 2, IC0{});
-    compute(gs + 1, IC1{});
-    gs += 2;
+  if constexpr (NS > 0) {
+    gemv_each<0, NS>([&](auto st) {
+      constexpr int v = decltype(st)::value;
+      const std::integral_constant<int, v & 1> buf;
+      compute(v, buf);
+      if constexpr (v + 2 < NS) issue(v + 2, buf);
+    });
+  } else {
+    int gs = 0;
+    for (; gs + 3 < n_st; gs += 2) {
+      compute(gs, IC0{}); issue(gs + 2, IC0{});
+      compute(gs + 1, IC1{}); issue(gs + 3, IC1{});
+    }
+    if (gs + 2 < n_st) {                                  // three left
+      compute(gs, IC0{}); issue(gs + 2, IC0{});
+      compute(gs + 1, IC1{});
+      compute(gs + 2, IC0{});
+    } else {
+      compute(gs, IC0{});
+      if (gs + 1 < n_st) compute(gs + 1, IC1{});
+    }
   }
-  if (gs + 1 < n_st) {
-    issue(gs + 1, IC1{});
-    compute(gs, IC0{});
-    compute(gs + 1, IC1{});
-  } else if (gs < n_st) {
-    compute(gs, IC0{});
-  }
-  if (STEP == STEP_BEGIN && bx == 0) gemv_step_begin_tail<MT>(sp, xrow, p.M, CHUNKS, tid);
-  if (STEP == STEP_END) gemv_step_end_tail<MT>(sp, best, p.M, bx, tid);
+  step_tail();
 }

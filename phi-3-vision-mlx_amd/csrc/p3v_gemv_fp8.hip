@@ -23,15 +23,16 @@ struct GemvF8P {
 // ---------------------------------------------------------------- M = 1 streaming (see k_gemv3)
 // STEP (p3v_gemv3_body.h): STEP_BEGIN / STEP_END carry the replayed greedy step's embedding gather + rotation rows / arg-max + bookkeeping,
 // exactly as gemv3_body does for bf16 weights (config 5's step is 129 launches too)
-template <int NST, int CH, int STEP>
+// NS: (row pair, K stage) steps of a full wave, 0 = any number in a loop; requests and the norm as in gemv3_body
+template <int NST, int CH, int NS, int STEP>
 __device__ __forceinline__ void gemv3_f8_body(const GemvF8P& p, int units_per_wave, int wpw, unsigned char* smem, float* red, const GemvStepP* sp) {
   constexpr int CHUNKS = NST * CH * 64;                 // 16-byte weight chunks per row (K = 16 * CHUNKS)
   constexpr int XCH = CHUNKS * 2;                       // 16-byte x chunks
   constexpr int XC = (XCH + 255) / 256;
   u32x4_t* xs = (u32x4_t*)smem;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool silu = p.epi == P3V_EPI_SILU_MUL, has_res = p.epi == P3V_EPI_RESID_BF16;
-  const int u_begin = wave < wpw ? min(p.units, (blockIdx.x * wpw + wave) * units_per_wave) : p.units;   // (wpw: see p3v_gemv_wpw)
+  const int u_begin = wave < wpw ? min(p.units, ((int)blockIdx.x * wpw + wave) * units_per_wave) : p.units;   // (wpw: see p3v_gemv_wpw)
   const int u_end = min(p.units, u_begin + units_per_wave);
   const int n_st = (u_end - u_begin) * NST;
 
@@ -46,14 +47,14 @@ __device__ __forceinline__ void gemv3_f8_body(const GemvF8P& p, int units_per_wa
   for (int k = 0; k < XC; ++k) {
     const int c = min(tid + k * 256, XCH - 1);
     xv[k] = ((const u32x4_t*)xrow[0])[c];
-    gv[k] = p.norm_w ? ((const u32x4_t*)p.norm_w)[c] : (u32x4_t){0, 0, 0, 0};
+    gv[k] = ((const u32x4_t*)(p.norm_w ? p.norm_w : xrow[0]))[c];
   }
   u32x4_t wbuf[2][2][CH];
   uint32_t rbuf[2];
   float sbuf[2][2];
   auto issue = [&](int gs, auto bufc) {
     constexpr int buf = decltype(bufc)::value;
-    const int u = min(u_begin + gs / NST, p.units - 1), s = gs % NST;
+    const int u = min(u_begin + gs / NST, u_end - 1), s = gs % NST;
     const int r0 = silu ? u : 2 * u, r1 = silu ? u + p.N : min(2 * u + 1, p.N - 1);
     const u32x4_t* w0 = (const u32x4_t*)(p.W + (size_t)r0 * (CHUNKS * 16)) + s * CH * 64 + lane;
     const u32x4_t* w1 = (const u32x4_t*)(p.W + (size_t)r1 * (CHUNKS * 16)) + s * CH * 64 + lane;
@@ -62,45 +63,59 @@ __device__ __forceinline__ void gemv3_f8_body(const GemvF8P& p, int units_per_wa
       wbuf[buf][0][j] = __builtin_nontemporal_load(w0 + j * 64);
       wbuf[buf][1][j] = __builtin_nontemporal_load(w1 + j * 64);
     }
-    rbuf[buf] = has_res ? *(const uint32_t*)(p.resid + 2 * u) : 0u;
+    rbuf[buf] = *(const uint32_t*)(has_res ? p.resid + 2 * u : xrow[0]);
     sbuf[buf][0] = p.wscale[r0];
     sbuf[buf][1] = p.wscale[r1];
+    __builtin_amdgcn_sched_barrier(0);
   };
-  if (n_st > 0) issue(0, IC0{});
 
-  float r = 1.f;
-  if (p.norm_w) {
-    float ss = 0.f;
+  auto stage_x = [&]() {
+    float r = 1.f;
+    if (p.norm_w) {
+      float ss = 0.f;
 #pragma unroll
-    for (int k = 0; k < XC; ++k)
-      if (tid + k * 256 < XCH) {
+      for (int k = 0; k < XC; ++k)
+        if (tid + k * 256 < XCH) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) { const float a = bf16lo(xv[k][j]), b = bf16hi(xv[k][j]); ss += a * a + b * b; }
+          for (int j = 0; j < 4; ++j) { const float a = bf16lo(xv[k][j]), b = bf16hi(xv[k][j]); ss += a * a + b * b; }
+        }
+      ss = wave_sum(ss);
+      if (lane == 0) red[wave] = ss;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      r = rsqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)(CHUNKS * 16) + p.eps);
+    }
+#pragma unroll
+    for (int k = 0; k < XC; ++k) {
+      const int c = tid + k * 256;
+      if (c < XCH) {
+        u32x4_t o = xv[k];
+        if (p.norm_w) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            o[j] = rms_pair(xv[k][j], r, gv[k][j]);
+        }
+        xs[c] = o;
       }
-    ss = wave_sum(ss);
-    if (lane == 0) red[wave] = ss;
+    }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
-    r = rsqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)(CHUNKS * 16) + p.eps);
+  };
+  ArgMaxVI best[1] = {ArgMaxVI{-INFINITY, 0x7fffffff}};      // STEP_END: this wave's arg-max candidate (lane 0's copy counts)
+  auto step_tail = [&]() {
+    if (STEP == STEP_BEGIN && blockIdx.x == 0) gemv_step_begin_tail<1>(sp, xrow, 1, XCH, tid);
+    if (STEP == STEP_END) gemv_step_end_tail<1>(sp, best, 1, (int)blockIdx.x, tid);
+  };
+  if (n_st <= 0) {                                            // a wave without rows: its own path
+    stage_x();
+    step_tail();
+    return;
   }
-#pragma unroll
-  for (int k = 0; k < XC; ++k) {
-    const int c = tid + k * 256;
-    if (c < XCH) {
-      u32x4_t o = xv[k];
-      if (p.norm_w) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          o[j] = rms_pair(xv[k][j], r, gv[k][j]);
-      }
-      xs[c] = o;
-    }
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
+  issue(0, IC0{});
+  if constexpr (NS != 1) issue(1, IC1{});
+  stage_x();
 
   float a0 = 0.f, a1 = 0.f;
-  ArgMaxVI best[1] = {ArgMaxVI{-INFINITY, 0x7fffffff}};      // STEP_END: this wave's arg-max candidate (lane 0's copy counts)
   auto compute = [&](int gs, auto bufc) {
     constexpr int buf = decltype(bufc)::value;
     const int s = gs % NST;
@@ -115,7 +130,7 @@ __device__ __forceinline__ void gemv3_f8_body(const GemvF8P& p, int units_per_wa
       const int u = u_begin + gs / NST;
       a0 = wave_sum(a0) * sbuf[buf][0];
       a1 = wave_sum(a1) * sbuf[buf][1];
-      if (lane == 0) {
+      if (lane == 0 && u < u_end) {
         if (silu) {
           const float g = bf16_round(a0), up = bf16_round(a1);
           ((bf16_t*)p.out)[u] = f32_to_bf16(bf16_round(g * bf16_round(1.f / (1.f + __expf(-g)))) * up);
@@ -135,30 +150,43 @@ __device__ __forceinline__ void gemv3_f8_body(const GemvF8P& p, int units_per_wa
       a0 = a1 = 0.f;
     }
   };
-  int gs = 0;
-  while (gs + 2 < n_st) {
-    issue(gs + 1, IC1{}); compute(gs, IC0{});
-    issue(gs + 2, IC0{}); compute(gs + 1, IC1{});
-    gs += 2;
+  if constexpr (NS > 0) {
+    gemv_each<0, NS>([&](auto st) {
+      constexpr int v = decltype(st)::value;
+      const std::integral_constant<int, v & 1> buf;
+      compute(v, buf);
+      if constexpr (v + 2 < NS) issue(v + 2, buf);
+    });
+  } else {
+    int gs = 0;
+    for (; gs + 3 < n_st; gs += 2) {
+      compute(gs, IC0{}); issue(gs + 2, IC0{});
+      compute(gs + 1, IC1{}); issue(gs + 3, IC1{});
+    }
+    if (gs + 2 < n_st) {                                       // three left
+      compute(gs, IC0{}); issue(gs + 2, IC0{});
+      compute(gs + 1, IC1{});
+      compute(gs + 2, IC0{});
+    } else {
+      compute(gs, IC0{});
+      if (gs + 1 < n_st) compute(gs + 1, IC1{});
+    }
   }
-  if (gs + 1 < n_st) { issue(gs + 1, IC1{}); compute(gs, IC0{}); compute(gs + 1, IC1{}); }
-  else if (gs < n_st) compute(gs, IC0{});
-  if (STEP == STEP_BEGIN && blockIdx.x == 0) gemv_step_begin_tail<1>(sp, xrow, 1, XCH, tid);
-  if (STEP == STEP_END) gemv_step_end_tail<1>(sp, best, 1, (int)blockIdx.x, tid);
+  step_tail();
 }
 
-template <int NST, int CH>
+template <int NST, int CH, int NS>
 __global__ void __launch_bounds__(256) k_gemv3_f8(GemvF8P p, int units_per_wave, int wpw) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ float red[4];
-  gemv3_f8_body<NST, CH, STEP_NONE>(p, units_per_wave, wpw, smem, red, nullptr);
+  gemv3_f8_body<NST, CH, NS, STEP_NONE>(p, units_per_wave, wpw, smem, red, nullptr);
 }
 
-template <int NST, int CH, int STEP>
+template <int NST, int CH, int NS, int STEP>
 __global__ void __launch_bounds__(256) k_gemv3_f8_step(GemvF8P p, int units_per_wave, int wpw, GemvStepP sp) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ float red[4];
-  gemv3_f8_body<NST, CH, STEP>(p, units_per_wave, wpw, smem, red, &sp);
+  gemv3_f8_body<NST, CH, NS, STEP>(p, units_per_wave, wpw, smem, red, &sp);
 }
 
 // ---------------------------------------------------------------- 2 <= M <= 16 through the matrix cores (see k_gemv_mfma)
@@ -461,11 +489,21 @@ static int launch_gemv3_f8(const GemvF8P& p, hipStream_t s, const GemvStepP* sp 
   if (upw < 1) upw = 1;
   const int waves = p3v_cdiv(p.units, upw);
   const int wpw = p3v_gemv_wpw(waves, n_cu, p3v_tuning().gemv_wpw);
-  if constexpr (STEP != STEP_NONE) {
-    if (p3v_cdiv(waves, wpw) > P3V_GEMV_STEP_MAX_WG) return P3V_ERR_UNSUPPORTED;        // (amax_ws holds one candidate per workgroup)
-    hipLaunchKernelGGL((k_gemv3_f8_step<NST, CH, STEP>), dim3(p3v_cdiv(waves, wpw)), dim3(256), (size_t)p.K * 2, s, p, upw, wpw, *sp);
-  } else {
-    hipLaunchKernelGGL((k_gemv3_f8<NST, CH>), dim3(p3v_cdiv(waves, wpw)), dim3(256), (size_t)p.K * 2, s, p, upw, wpw);
+  const dim3 grid(p3v_cdiv(waves, wpw));
+  const size_t lds = (size_t)p.K * 2;
+  if (STEP != STEP_NONE && (int)grid.x > P3V_GEMV_STEP_MAX_WG) return P3V_ERR_UNSUPPORTED;        // (amax_ws holds one candidate per workgroup)
+  auto launch = [&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    if constexpr (NS % NST) return;                              // (not a number of whole row pairs)
+    else if constexpr (STEP != STEP_NONE) hipLaunchKernelGGL((k_gemv3_f8_step<NST, CH, NS, STEP>), grid, dim3(256), lds, s, p, upw, wpw, *sp);
+    else hipLaunchKernelGGL((k_gemv3_f8<NST, CH, NS>), grid, dim3(256), lds, s, p, upw, wpw);
+  };
+  switch (upw * NST) {
+    case 1: launch(IC1{}); break;
+    case 2: launch(std::integral_constant<int, 2>{}); break;
+    case 3: launch(std::integral_constant<int, 3>{}); break;
+    case 4: launch(std::integral_constant<int, 4>{}); break;
+    default: launch(IC0{});
   }
   P3V_CHECK_LAUNCH();
   return P3V_OK;

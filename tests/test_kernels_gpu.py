@@ -1638,6 +1638,41 @@ def test_gemv_q4_row_groups(ops, K, pairs, epi):
         ops.set_tuning("gemv_q4_wpc", old)
 
 
+@pytest.mark.parametrize("K,pairs", [(3072, (1, 257, 513, 1023, 1281, 1537)), (8192, (1, 258, 515))])
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+@pytest.mark.parametrize("epi", ["none", "silu", "f32", "resid"])
+def test_gemv_row_steps(ops, K, pairs, kind, epi):
+    """One row, every number of (row pair, K stage) steps a wave may have (1 .. 4 as straight-line code, more in the loop, the last wave
+    shorter than the others; waves without rows), with one wave per CU.  Against the product in 64 bits: a lane adds 48 .. 128 times and
+    the lanes 6 times in fp32, an error below 2^-17 sum |x w|; beside it the rounding of the bf16 result."""
+    from phi_3_vision_mlx_amd.ops import EPI_F32, EPI_NONE, EPI_RESID_BF16, EPI_SILU_MUL
+    e = {"none": EPI_NONE, "resid": EPI_RESID_BF16, "silu": EPI_SILU_MUL, "f32": EPI_F32}[epi]
+    w = g((2 * max(pairs) * (2 if epi == "silu" else 1), K), 420, 0.03).cuda()
+    x, knob = g((1, K), 421).cuda(), "gemv_wpc" if kind == "bf16" else "gemv_f8_wpc"
+    w8, sc = ops.quantize_fp8_rows(w)
+    wd = w.double() if kind == "bf16" else w8.view(torch.float8_e4m3fn).double() * sc.double()[:, None]
+    old = ops.set_tuning(knob, 1)
+    try:
+        for n in pairs:
+            N = 2 * n
+            rows = 2 * N if epi == "silu" else N
+            res = g((1, N), 422).cuda()
+            buf = torch.full((1, N + 64), 7.0, dtype=F32 if epi == "f32" else BF16).cuda()      # behind the row: untouched
+            kw = dict(resid=res if epi == "resid" else None, out=buf[:, :N])
+            got = ops.gemv(x, w[:rows], e, **kw) if kind == "bf16" else ops.gemv_fp8(x, w8[:rows], sc[:rows], e, **kw)
+            assert torch.all(buf[:, N:] == 7.0)
+            y, tol = x.double() @ wd[:rows].t(), 2.0 ** -17 * (x.double().abs() @ wd[:rows].abs().t())
+            if epi == "silu":
+                gt, up = y[:, :N], y[:, N:]
+                ref, tol = torch.nn.functional.silu(gt) * up, tol[:, :N] * (1 + up.abs()) + tol[:, N:] * (1 + gt.abs())
+            else:
+                ref = y + res.double() if epi == "resid" else y
+            slack = {"none": 2.0 ** -8, "resid": 2.0 ** -7, "silu": 2.0 ** -5, "f32": 0.0}[epi] * (ref.abs() + (y[:, :N].abs() if epi == "resid" else 0))
+            assert torch.all((got.double() - ref).abs() <= slack + tol), (n, (got.double() - ref).abs().max())
+    finally:
+        ops.set_tuning(knob, old)
+
+
 @pytest.mark.parametrize("M", [2, 5, 8, 15, 16])
 @pytest.mark.parametrize("N,K,epi", [(9216, 3072, "none"), (3072, 3072, "resid"), (8192, 3072, "silu"), (3072, 8192, "resid"), (32064, 3072, "none")])
 def test_gemv_q4_rows_2_to_16(ops, N, K, epi, M):
