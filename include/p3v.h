@@ -189,6 +189,18 @@ int p3v_rope_kv_append(const uint16_t* qkv, const float* cos_t, const float* sin
  *      two calls -- for every other shape, without a workspace of p3v_gemm_ws_bytes(), or N > 3072.  normed: bf16 [M, N] contiguous. */
 int p3v_gemm_resid_norm(const p3v_gemm_args_t* gemm /* host */, const uint16_t* norm_w, float eps, uint16_t* normed, void* stream);
 
+/* ---- the same pair for 9 .. 16 rows (a decode batch), the norm split between the projection in front of it and the one behind, no
+ *      launch between them:
+ *      p3v_gemm_rows_resid:  out = resid + bf16(A W^T), scaled = bf16(out * norm_w) [M, N] contiguous, and sumsq[p][m] (fp32, [parts][16],
+ *        rows of A beyond M undefined) = sum of out[m][n]^2 over the columns of piece p.  parts = p3v_gemm_rows_resid_parts(M, N, K), at most
+ *        256; 0: not a shape of this call (9 <= M <= 16, N % 16 == 0, K = 3072).  epilogue: P3V_EPI_RESID_BF16; resid may be out.
+ *      p3v_gemm_rows_scaled: out = (A W^T) * rsqrt(sum_p sumsq[p][m] / K + eps), A = scaled; epilogue none or P3V_EPI_SILU_MUL, K = 3072.
+ *      Together RMSNorm(out) W^T with one rounding of the normalised input where p3v_rmsnorm makes two.  P3V_ERR_UNSUPPORTED: nothing
+ *      launched.  Graph-capturable; scaled and sumsq are live between the two calls. */
+int p3v_gemm_rows_resid_parts(int M, int N, int K);
+int p3v_gemm_rows_resid(const p3v_gemm_args_t* gemm /* host */, const uint16_t* norm_w, uint16_t* scaled, float* sumsq, void* stream);
+int p3v_gemm_rows_scaled(const p3v_gemm_args_t* gemm /* host */, const float* sumsq, int parts, float eps, void* stream);
+
 /* ---- the qkv projection with the split, the rotation and the KV append in its EPILOGUE:
  *      p3v_gemm_qkv(g, s) == p3v_gemm(g) into a scratch [M, N] + p3v_rope_kv_append(scratch, ...) with s's arguments, bit for bit, in the
  *      GEMM's launches alone (phi.py:437-452 / 140-147: `qkv_proj` + `split` + `_rotate_half` + KVCache append; CLIP: q/k/v projections

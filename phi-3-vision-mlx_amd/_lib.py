@@ -152,6 +152,9 @@ SIGNATURES = {
     "p3v_gemm_qkv_fp8": (i32, [C.POINTER(GemmF8Args), C.POINTER(QkvSplit), vp]),
     "p3v_gemm_qkv_fp8_pays": (i32, [i32, i32, i32, i32]),
     "p3v_gemm_resid_norm": (i32, [C.POINTER(GemmArgs), vp, f32, vp, vp]),
+    "p3v_gemm_rows_resid_parts": (i32, [i32, i32, i32]),
+    "p3v_gemm_rows_resid": (i32, [C.POINTER(GemmArgs), vp, vp, vp, vp]),
+    "p3v_gemm_rows_scaled": (i32, [C.POINTER(GemmArgs), vp, i32, f32, vp]),
     "p3v_kv_quantize_mlx4": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, vp, vp, vp, i32, i32, i32, i32, i32, vp]),
     "p3v_attention_decode_q8": (i32, [C.POINTER(AttnDecQ8Args), vp]),
     "p3v_attention_decode_q8_can_fuse_oproj": (i32, [i32, i32, i32, i32, i32, i32, i32, i32]),

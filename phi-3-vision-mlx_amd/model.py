@@ -182,6 +182,16 @@ class Phi3VModel(DecoderModel):
             return False
         return ops.gemm_resid_norm(o, self.w[key], x, norm_w, self.cfg.rms_norm_eps, h[:M], out=x)
 
+    def _proj_resid_scaled(self, o, key, x, norm_w, h, sq, next_key):
+        """x += bf16(o @ W^T), h = bf16(x * norm_w) and the rows' sums of squares (ops.gemm_rows_resid), for the projection `next_key` that
+        finishes the RMSNorm (ops.gemm_rows_scaled); 0 -- nothing done -- where either of them does not take it."""
+        M, K = o.shape
+        wn = self.w.get(next_key)
+        if (sq is None or not 9 <= M <= 16 or key not in self.w or wn is None or key in self.adapters or next_key in self.adapters
+                or wn.shape[1] != 3072 or wn.shape[0] % 16 or os.environ.get("P3V_RESID_NORM_FUSE", "1") == "0"):
+            return 0
+        return ops.gemm_rows_resid(o, self.w[key], x, norm_w, h[:M], sq, out=x)
+
     # ------------------------------------------------------------------ vision tower
     def _prep_vision(self):
         c = self.cfg.clip
@@ -382,6 +392,8 @@ class Phi3VModel(DecoderModel):
             q=torch.empty((B, nh, L, hd), dtype=BF16, device=dev), o=torch.empty((M, nh * hd), dtype=BF16, device=dev),
             qkv=torch.empty((M, (nh + 2 * nkv) * hd), dtype=BF16, device=dev), a=torch.empty((M, I), dtype=BF16, device=dev),
             h=torch.empty((M, H), dtype=BF16, device=dev), n_split=0, ws=None)
+        if 9 <= M <= 16:
+            bufs["sq"] = torch.empty((256, 16), dtype=F32, device=dev)       # sums of squares of the rows behind `h` (ops.gemm_rows_resid)
         return bufs
 
     def _plan_fused_oproj(self, bufs, B, L, T, quantized=False):
@@ -593,15 +605,19 @@ class Phi3VModel(DecoderModel):
             # Short prompts and decode batches (9 .. 256 rows): o_proj and down_proj run as K slices, and the launch that adds the slices also writes the
             # RMSNorm of the new residual stream into `h` -- the next projection's input (ops.gemm_resid_norm; bit-identical to the
             # two launches it replaces).
-            normed = False
+            # 9 .. 16 rows, o_proj and gate_up: no launch at all between them (ops.gemm_rows_resid / gemm_rows_scaled).
+            normed, parts, gu = False, 0, p + "mlp.gate_up_proj.weight"
             if not (bufs.get("fuse_o", False) and L <= ops.L.DECODE_MAX_L and n_beam == 1):
-                normed = self._proj_resid_norm(o, p + "self_attn.o_proj.weight", x, w[p + "post_attention_layernorm.weight"], h)
+                parts = self._proj_resid_scaled(o, p + "self_attn.o_proj.weight", x, w[p + "post_attention_layernorm.weight"], h, bufs.get("sq"), gu)
+                normed = parts or self._proj_resid_norm(o, p + "self_attn.o_proj.weight", x, w[p + "post_attention_layernorm.weight"], h)
                 if not normed:
                     self._proj(o, p + "self_attn.o_proj.weight", EPI_RESID_BF16, resid=x, out=x)
-            if normed:
-                self._proj(h, p + "mlp.gate_up_proj.weight", EPI_SILU_MUL, out=a)
+            if parts:
+                ops.gemm_rows_scaled(h, w[gu], bufs["sq"], parts, eps, EPI_SILU_MUL, out=a)
+            elif normed:
+                self._proj(h, gu, EPI_SILU_MUL, out=a)
             else:
-                self._proj(x, p + "mlp.gate_up_proj.weight", EPI_SILU_MUL, norm_w=w[p + "post_attention_layernorm.weight"], out=a, h=h)
+                self._proj(x, gu, EPI_SILU_MUL, norm_w=w[p + "post_attention_layernorm.weight"], out=a, h=h)
             normed_in = False
             if i + 1 < cfg.num_hidden_layers:
                 normed_in = self._proj_resid_norm(a, p + "mlp.down_proj.weight", x, w[f"model.layers.{i + 1}.input_layernorm.weight"], h)

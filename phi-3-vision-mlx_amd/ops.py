@@ -159,6 +159,41 @@ def gemm_resid_norm(a, w, resid, norm_w, eps, normed, out=None):
     return True
 
 
+def gemm_rows_resid(a, w, resid, norm_w, scaled, sumsq, out=None):
+    """out = resid + bf16(a @ w^T), scaled = bf16(out * norm_w) and sumsq [parts, 16] = the squares of out's rows piece by piece, in one
+    launch: the first half of the RMSNorm in front of the next projection (gemm_rows_scaled is the other).  Returns the number of pieces;
+    0, nothing launched, for a shape the library does not take (it takes 9 .. 16 rows and K = 3072)."""
+    _chk(a, BF16, "a"), _chk(w, BF16, "w"), _chk(resid, BF16, "resid"), _chk(norm_w, BF16, "norm_w"), _chk(scaled, BF16, "scaled"), _chk(sumsq, F32, "sumsq")
+    M, K = a.shape
+    N = w.shape[0]
+    if w.shape[1] != K or resid.shape != (M, N) or scaled.shape != (M, N) or norm_w.numel() != N or not scaled.is_contiguous():
+        raise ValueError(f"gemm_rows_resid: shapes {a.shape} x {w.shape}, resid {resid.shape}, scaled {scaled.shape}")
+    parts = L.lib().p3v_gemm_rows_resid_parts(M, N, K)
+    if not parts:
+        return 0
+    if sumsq.numel() < parts * 16:
+        raise ValueError(f"gemm_rows_resid: sumsq holds {sumsq.numel()} of {parts * 16} values")
+    if out is None:
+        out = torch.empty((M, N), dtype=BF16, device=a.device)
+    if out.stride(0) != resid.stride(0):
+        raise ValueError("gemm_rows_resid: resid and out are laid out alike")
+    args = L.GemmArgs(_p(a), _p(w), _p(out), None, _p(resid), None, M, N, K, a.stride(0), w.stride(0), out.stride(0), EPI_RESID_BF16, 0, None, 0)
+    L.check(L.lib().p3v_gemm_rows_resid(C.byref(args), _p(norm_w), _p(scaled), _p(sumsq), _stream()), "gemm_rows_resid")
+    return parts
+
+
+def gemm_rows_scaled(scaled, w, sumsq, parts, eps, epilogue=EPI_NONE, out=None):
+    """RMSNorm(x) @ w^T from gemm_rows_resid's scaled rows and sums of squares."""
+    _chk(scaled, BF16, "scaled"), _chk(w, BF16, "w"), _chk(sumsq, F32, "sumsq")
+    M, K = scaled.shape
+    N = w.shape[0] // 2 if epilogue in GATED else w.shape[0]
+    if out is None:
+        out = torch.empty((M, N), dtype=BF16, device=scaled.device)
+    args = L.GemmArgs(_p(scaled), _p(w), _p(out), None, None, None, M, N, K, scaled.stride(0), w.stride(0), out.stride(0), epilogue, 0, None, 0)
+    L.check(L.lib().p3v_gemm_rows_scaled(C.byref(args), _p(sumsq), parts, float(eps), _stream()), "gemm_rows_scaled")
+    return out
+
+
 GEMV_MAX_M = 16
 
 

@@ -1673,6 +1673,47 @@ def test_gemv_row_steps(ops, K, pairs, kind, epi):
         ops.set_tuning(knob, old)
 
 
+@pytest.mark.parametrize("M", [9, 13, 16])
+@pytest.mark.parametrize("N", [3072, 1040, 16, 4096])
+def test_gemm_rows_resid_scaled(ops, M, N, K=3072):
+    """p3v_gemm_rows_resid: the residual row is bf16(A W^T) added once (the fp32 sums differ in order from 64 bits: below 2^-17 sum |a w|),
+    scaled and sumsq are functions of the row just written; resid may be out.  p3v_gemm_rows_scaled behind it: the RMSNorm'ed projection in
+    64 bits within the rounding of the scaled rows (2^-9 relative per product, summed in quadrature over K: 6 standard deviations)."""
+    a, w, r, nw = g((M, K), 430).cuda(), g((N, K), 431, 0.02).cuda(), g((M, N), 432).cuda(), (g((N,), 433) * 0.1 + 1).cuda()
+    scaled = torch.full((M + 1, N), 7.0, dtype=BF16).cuda()
+    sq = torch.full((256, 16), float("nan")).cuda()
+    out = r.clone()
+    parts = ops.gemm_rows_resid(a, w, out, nw, scaled[:M], sq, out=out)
+    assert parts == N // 16 and torch.all(scaled[M] == 7.0) and torch.all(torch.isnan(sq[parts:]))
+    y = a.double() @ w.double().t()
+    tol = 2.0 ** -17 * (a.double().abs() @ w.double().abs().t()) + 2.0 ** -8 * (y.abs() + (r.double() + y).abs())
+    assert torch.all((out.double() - (r.double() + y)).abs() <= tol)
+    assert torch.equal(scaled[:M], (out.float() * nw.float()).to(BF16))
+    assert torch.allclose(sq[:parts, :M].double(), out.double().pow(2).view(M, parts, 16).sum(-1).t(), rtol=2.0 ** -20, atol=0)
+    if N != 3072:
+        return
+    for epi, rows in ((ops.EPI_NONE, 9216), (ops.EPI_NONE, 16), (ops.EPI_SILU_MUL, 2 * 8192), (ops.EPI_SILU_MUL, 2 * 24)):
+        wn = g((rows, N), 434, 0.02).cuda()
+        got = ops.gemm_rows_scaled(scaled[:M], wn, sq, parts, 1e-5, epi).double()
+        xn = out.double() * torch.rsqrt(out.double().pow(2).mean(-1, keepdim=True) + 1e-5) * nw.double()
+        y = xn @ wn.double().t()
+        tol = 6 * 2.0 ** -9 * (xn.pow(2) @ wn.double().pow(2).t()).sqrt() + 2.0 ** -8 * y.abs()
+        if epi == ops.EPI_SILU_MUL:
+            n = rows // 2
+            gt, up = y[:, :n], y[:, n:]
+            y, tol = torch.nn.functional.silu(gt) * up, tol[:, :n] * (1 + up.abs()) + tol[:, n:] * (1 + gt.abs()) + 2.0 ** -6 * (gt * up).abs()
+        assert torch.all((got - y).abs() <= tol), (epi, rows, ((got - y).abs() / tol).max())
+
+
+def test_gemm_rows_resid_refuses(ops):
+    """Shapes of other kernels: 0, nothing launched (outputs untouched)."""
+    for M, K, N in ((8, 3072, 3072), (17, 3072, 3072), (12, 8192, 3072), (12, 3072, 3080), (12, 3072, 8192)):
+        a, w, r, nw = g((M, K), 435).cuda(), g((N, K), 436).cuda(), g((M, N), 437).cuda(), g((N,), 438).cuda()
+        s, sq, o = torch.full((M, N), 7.0, dtype=BF16).cuda(), torch.full((512, 16), 7.0).cuda(), torch.full((M, N), 7.0, dtype=BF16).cuda()
+        assert ops.gemm_rows_resid(a, w, r, nw, s, sq, out=o) == 0
+        assert torch.all(s == 7.0) and torch.all(sq == 7.0) and torch.all(o == 7.0)
+
+
 @pytest.mark.parametrize("M", [2, 5, 8, 15, 16])
 @pytest.mark.parametrize("N,K,epi", [(9216, 3072, "none"), (3072, 3072, "resid"), (8192, 3072, "silu"), (3072, 8192, "resid"), (32064, 3072, "none")])
 def test_gemv_q4_rows_2_to_16(ops, N, K, epi, M):
