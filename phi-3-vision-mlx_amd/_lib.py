@@ -148,6 +148,9 @@ SIGNATURES = {
     "p3v_kv_quantize": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]),
     "p3v_kv_dequantize": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]),
     "p3v_gemm_qkv": (i32, [vp, vp, vp]),
+    "p3v_gemm_qkv_merge": (i32, [vp, vp, vp, i64, vp]),
+    "p3v_gemm_merge": (i32, [C.POINTER(GemmArgs), vp, i64, vp]),
+    "p3v_gemm_merge_ws_bytes": (i64, [i32, i32, i32, i32, i32]),
     "p3v_gemm_plan": (i32, [i32, i32, i32, i32]),
     "p3v_gemm_qkv_fp8": (i32, [C.POINTER(GemmF8Args), C.POINTER(QkvSplit), vp]),
     "p3v_gemm_qkv_fp8_pays": (i32, [i32, i32, i32, i32]),

@@ -649,7 +649,8 @@ static int gemm128(const p3v_gemm_args_t* a, hipStream_t s) {
 int p3v_gemm256_qkv(const p3v_gemm_args_t* a, const QkvP& q, hipStream_t s);   // p3v_gemm256.hip
 int p3v_gemm_skinny_qkv(const p3v_gemm_args_t* a, const QkvP& q, hipStream_t s);   // p3v_gemm_skinny.hip
 
-extern "C" int p3v_gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* stream) {
+int p3v_gemm_skinny_qkv_merge(const p3v_gemm_args_t* a, const QkvP& q, void* ws, int64_t ws_bytes, hipStream_t s);   // p3v_gemm_skinny.hip
+static int gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* merge_ws, int64_t merge_bytes, void* stream) {
   if (!a || !sp || !a->A || !a->W || !sp->q_out || !sp->k_dst || !sp->v_dst || (!sp->cos_t) != (!sp->sin_t)) return P3V_ERR_ARG;
   if (a->epilogue != P3V_EPI_NONE && a->epilogue != P3V_EPI_BIAS) return P3V_ERR_ARG;
   if (a->epilogue == P3V_EPI_BIAS && !a->bias) return P3V_ERR_ARG;
@@ -668,6 +669,7 @@ extern "C" int p3v_gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp,
   hipStream_t s = (hipStream_t)stream;
   QkvP q = {sp->cos_t, sp->sin_t, sp->q_out, sp->k_dst, sp->v_dst, sp->L, nh, nkv, hd, sp->past, dpos0, sp->dst_t, sp->tab_t, sp->tab_div, 0,
             sp->q_scale};
+  if (merge_ws) return p3v_gemm_skinny_qkv_merge(a, q, merge_ws, merge_bytes, s);
   if (a->M < 1024) return p3v_gemm_skinny_qkv(a, q, s);       // 17 .. 256 rows: the weight-streaming kernel (or "unsupported")
   if ((nh * hd) % BN || (nkv * hd) % BN || p3v_tuning().gemm_128) return P3V_ERR_UNSUPPORTED;
   p3v_gemm_args_t plain = *a;
@@ -686,4 +688,8 @@ extern "C" int p3v_gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp,
     return launch_gemm<P3V_EPI_QKV>(p, s);
   }
   return P3V_OK;
+}
+extern "C" int p3v_gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* stream) { return gemm_qkv(a, sp, nullptr, 0, stream); }
+extern "C" int p3v_gemm_qkv_merge(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* ws, int64_t ws_bytes, void* stream) {
+  return ws ? gemm_qkv(a, sp, ws, ws_bytes, stream) : P3V_ERR_ARG;
 }

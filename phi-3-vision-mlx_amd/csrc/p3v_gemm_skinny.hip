@@ -25,7 +25,7 @@
 
 #define SK_BM 128
 #define SK_BK 64
-#define SK_TN 64                    // tile width the launcher uses (TN = 128: measured, not faster -- see the header)
+#define SK_TN 64                    // tile width of the one-pass and partial-sum forms (TN = 128: measured, not faster -- see the header; MERGE takes it)
 #ifndef SK_ABL
 #define SK_ABL 0                    // timing experiments: 1 = A always K-tile 0 (one L2/L1-hot tile), 2 = W likewise, 3 = no MFMAs after K-tile 0
 #endif
@@ -71,46 +71,52 @@ struct SkinnyP {
   const bf16_t* col_scale;         // P3V_EPI_SCALE_RESID_F32
   int kslice;                      // 0: one pass with the epilogue; else K columns per slice, fp32 partials
   QkvP q;                          // P3V_EPI_QKV only (p3v_gemm_qkv.h): head split + rotation + KV append in the epilogue
+  float* xpart; unsigned* xflag;   // MERGE: partial tiles [tile][slice][consumer wave][block][lane] x 4, counters [tile][consumer wave] (0 between launches)
+  int nk_part;                     // MERGE: K-tiles of a slice other than the last
 };
+#define SK_MERGE_POLLS (1u << 22)  // (seconds: the partials' workgroups are ahead of the waiting one in dispatch order)
 
 #define P3V_EPI_QKV 100            // internal, as in the other GEMM kernels
 
-template <int EPI, bool PART, int TN, int TM = SK_BM>
+// MERGE: gridDim.z slices of K, summed inside the launch (see p3v_gemm_merge below)
+template <int EPI, bool PART, int TN, int TM = SK_BM, bool MERGE = false>
 __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
   typedef SkCfg<TN, TM> C;
   static_assert(TM == SK_BM || EPI != P3V_EPI_QKV, "the qkv epilogue's V tiles are 128 dimensions tall");
+  static_assert(!MERGE || (!PART && TN == 128), "merged slices: 128-column tiles");
   constexpr bool SILU = P3V_GATED(EPI);
   constexpr int NS = C::NS, NI = C::NI;
   static_assert(NS - 2 <= 4 && (NS - 2) * C::PER < 64, "sk_wait_stages covers 4 stages in flight");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr bool QKV = EPI == P3V_EPI_QKV;
-  static_assert(!QKV || (TN == 64 && !PART), "the qkv epilogue: 64-column tiles, one pass");
+  static_assert(!QKV || !PART, "the qkv epilogue needs whole sums");
   constexpr int n_out_tile = SILU ? TN / 2 : TN;
   int n0 = blockIdx.x * n_out_tile, m0 = blockIdx.y * TM;
   const int kz = blockIdx.z;
-  const int nk = (PART ? p.kslice : p.K) / SK_BK, kt0 = kz * nk;
+  const bool last = !MERGE || kz == (int)gridDim.z - 1;          // the slice that adds the others' sums to its own
+  const int nk = MERGE ? (last ? p.K / SK_BK - kz * p.nk_part : p.nk_part) : (PART ? p.kslice : p.K) / SK_BK, kt0 = kz * (MERGE ? p.nk_part : nk);
   // P3V_EPI_QKV (p3v_gemm_qkv.h), a one-dimensional grid: first the Q and K tiles (128 tokens x 32 rotation pairs, W rows fetched in
   // pair order), M-tile-major; then the V tiles with the operand roles swapped (128 V dimensions on the tile's A side, 64 tokens on
   // its B side), so that a lane ends up with consecutive TOKENS of one dimension for the transposed cache.
   bool swapped = false, is_k = false;
   int row0 = 0;
   if (QKV) {
-    const int nq_t = p.q.nh * p.q.hd / 64, nk_t = p.q.nkv * p.q.hd / 64, nqk = nq_t + nk_t, mt = (p.M + SK_BM - 1) / SK_BM;
+    const int nq_t = p.q.nh * p.q.hd / TN, nk_t = p.q.nkv * p.q.hd / TN, nqk = nq_t + nk_t, mt = (p.M + SK_BM - 1) / SK_BM;
     int t = blockIdx.x;
     if (t < nqk * mt) {
       const int n_t = t % nqk;
       m0 = (t / nqk) * SK_BM;
       is_k = n_t >= nq_t;
       row0 = is_k ? p.q.nh * p.q.hd : 0;
-      n0 = (n_t - (is_k ? nq_t : 0)) * 64;                     // first column INSIDE the region
+      n0 = (n_t - (is_k ? nq_t : 0)) * TN;                     // first column INSIDE the region
     } else {
       t -= nqk * mt;
       const int nv_t = p.q.nkv * p.q.hd / SK_BM;
       swapped = true;
       row0 = (p.q.nh + p.q.nkv) * p.q.hd;
       n0 = (t % nv_t) * SK_BM;                                 // first V dimension of the tile (its A side)
-      m0 = (t / nv_t) * 64;                                    // first token (its B side)
+      m0 = (t / nv_t) * TN;                                    // first token (its B side)
     }
   }
 
@@ -222,11 +228,64 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
     }
   }
 
+  if constexpr (MERGE) {
+    // A wave of another slice writes its blocks past the caches, waits until they are there and counts itself in; the last slice's wave of
+    // the same place waits for all of them and adds them in slice order.  Its workgroups come last in dispatch order, so whatever they
+    // wait for runs or has run; it has more K-tiles than the others, whose sums are on their way meanwhile.
+    const int tile = (int)blockIdx.x, others = (int)gridDim.z - 1;
+    // (rows and, in a V tile, tokens beyond M: nothing is stored for them)
+    const bool live = (QKV && swapped ? m0 + wc * 64 : m0 + wr * NI * 16) < p.M;
+    unsigned* flag = p.xflag + tile * 4 + wave;
+    constexpr int WAVE_BYTES = NI * 4 * 1024;
+    const __amdgpu_buffer_rsrc_t rs_p = __builtin_amdgcn_make_buffer_rsrc((void*)(p.xpart + (size_t)(tile * others) * (WAVE_BYTES)), 0, others * 4 * WAVE_BYTES, 0x00020000);
+    const int my = lane * 16;
+    if (!last) {
+      if (!live) return;
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][j]), rs_p, my + (i * 4 + j) * 1024, (kz * 4 + wave) * WAVE_BYTES, 16);   // (16: sc1)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (lane == 0) __hip_atomic_fetch_add(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+    if (live) {
+      bool late = true;
+      for (unsigned n = 0; n < SK_MERGE_POLLS; ++n) {
+        if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == (unsigned)others) { late = false; break; }
+        __builtin_amdgcn_s_sleep(1);
+      }
+      asm volatile("" ::: "memory");
+      auto load = [&](u32x4_t (&v)[NI][4], int z) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[i][j] = __builtin_amdgcn_raw_buffer_load_b128(rs_p, my + (i * 4 + j) * 1024, (z * 4 + wave) * WAVE_BYTES, 16);
+      };
+      auto add = [&](const u32x4_t (&v)[NI][4]) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[i][j] += __builtin_bit_cast(f32x4_t, v[i][j]);
+      };
+      u32x4_t v[NI][4];
+      for (int z = 0; z < others; ++z) { load(v, z); add(v); }   // (two slices' loads at once: no faster)
+      if (late) {                                                // loud, not wrong
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4_t){__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
+      }
+      if (lane == 0) __hip_atomic_store(flag, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+
   // ---- epilogue, straight from the accumulators: lane (fc = lane & 15, fq = lane >> 4) holds columns 4 fq .. 4 fq + 3 of block
   //      row fc (see p3v_gemm256_epi.h)
   if constexpr (QKV) {
-    if (!swapped) qkv_epilogue_rot<NI>(p.q, acc, nullptr, is_k, row0, n0 >> 1, m0 + wr * NI * 16, p.M, lane);
-    else qkv_epilogue_vt<NI>(p.q, acc, nullptr, n0 + wr * NI * 16, m0, p.M, lane);
+    if (!swapped) qkv_epilogue_rot<NI>(p.q, acc, nullptr, is_k, row0, (n0 >> 1) + wc * 32, m0 + wr * NI * 16, p.M, lane);
+    else qkv_epilogue_vt<NI>(p.q, acc, nullptr, n0 + wr * NI * 16, m0 + wc * 64, p.M, lane);
     return;
   }
   const int fc = lane & 15, fq = lane >> 4;
@@ -382,7 +441,7 @@ int p3v_gemm_skinny_partials(const p3v_gemm_args_t* a, int* S_out, hipStream_t s
   if (S <= 1 || !a->ws || a->ws_bytes < (int64_t)S * a->M * w_rows * 4) return P3V_ERR_UNSUPPORTED;
   if ((uintptr_t)a->ws & 15) return P3V_ERR_ARG;
   *S_out = S;
-  const SkinnyP p = {a->A, a->W, a->ws, a->resid, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, a->col_scale, a->K / S, {}};
+  const SkinnyP p = {a->A, a->W, a->ws, a->resid, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, a->col_scale, a->K / S, {}, nullptr, nullptr, 0};
   if (silu) return launch_skinny<P3V_EPI_SILU_MUL>(p, S, s);                       // (partials: the activation is the reduction's)
   if (a->epilogue == P3V_EPI_RESID_BF16) return launch_skinny<P3V_EPI_RESID_BF16>(p, S, s);
   return launch_skinny<P3V_EPI_NONE>(p, S, s);
@@ -401,7 +460,7 @@ int p3v_gemm_skinny_try(const p3v_gemm_args_t* a, hipStream_t s) {
   if (rc == P3V_OK) return p3v_splitk_reduce((const float*)a->ws, a, S, s);
   if (rc != P3V_ERR_UNSUPPORTED) return rc;
   if (sk_slices(a->M, a->N, a->K, a->epilogue) == 0) return P3V_ERR_UNSUPPORTED;   // (a rows shape whose slices found no workspace and that the tile kernel does not take)
-  const SkinnyP p = {a->A, a->W, a->out, a->resid, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, a->col_scale, 0, {}};
+  const SkinnyP p = {a->A, a->W, a->out, a->resid, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, a->col_scale, 0, {}, nullptr, nullptr, 0};
   if (a->epilogue == P3V_EPI_SCALE_RESID_F32) return launch_skinny<P3V_EPI_SCALE_RESID_F32>(p, 1, s);
   if (a->epilogue == P3V_EPI_SILU_MUL) return launch_skinny<P3V_EPI_SILU_MUL>(p, 1, s);
   if (a->epilogue == P3V_EPI_GELU_MUL) return launch_skinny<P3V_EPI_GELU_MUL>(p, 1, s);
@@ -422,9 +481,75 @@ int p3v_gemm_skinny_qkv(const p3v_gemm_args_t* a, const QkvP& q, hipStream_t s) 
       return P3V_ERR_HIP;
     attr_set = true;
   }
-  const SkinnyP p = {a->A, a->W, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0, nullptr, 0, q};
+  const SkinnyP p = {a->A, a->W, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0, nullptr, 0, q, nullptr, nullptr, 0};
   const int mt = p3v_cdiv(a->M, SK_BM), tiles = ((q.nh + q.nkv) * q.hd / 64) * mt + (q.nkv * q.hd / SK_BM) * p3v_cdiv(a->M, 64);
   hipLaunchKernelGGL((k_gemm_skinny<P3V_EPI_QKV, false, SK_TN>), dim3(tiles), dim3(512), SkCfg<SK_TN>::LDS, s, p);
   P3V_CHECK_LAUNCH();
   return P3V_OK;
+}
+
+// ---- K slices that meet inside the launch: qkv of 17 .. 128 rows, gated projections of 105 .. 128.
+// What these launches wait for is the bytes a CU requests, the A panel from L2 among them (the header), and qkv keeps only 144 CUs busy
+// besides: on 128-column tiles a CU asks for half the A bytes per weight byte, and slices of K bring the workgroups back to one for
+// (nearly) every CU.  Their fp32 sums through a launch of their own would cost what that gains; here the last slice's workgroup of a tile
+// takes them over (k_gemm_skinny, MERGE).  It has a few K-tiles more than the others, while whose sums are under way (qkv 18 : 15 : 15 of
+// 48; 16 each: 24.8 us, 20 : 14 : 14 23.5).  qkv 27.7 -> 22.4 us at 128 rows, 27.6 -> 19.0 at 64, 22.7 -> 18 at 17; gate_up 29.5 -> 26.9 at
+// 128, 27.2 -> 26.3 at 112, 26.1 -> 26.1 at 104 (64 rows, on 64-row tiles of the one-pass form: 22.0 : 23.1).  Every slice finishing a
+// share of the blocks instead: 26.8 and 30.9, the hand-over through memory then being behind everybody's products.
+#define SK_MERGE_FLAGS 4096        // bytes of counters in front of the partials (zero before the first launch; every launch leaves them zero)
+struct MergePlan { int S, nk_part, tiles; };
+static MergePlan merge_plan(int M, int N, int K, int epilogue, bool qkv) {
+  const MergePlan none = {0, 0, 0};
+  const P3vTuning& t = p3v_tuning();
+  const int rows = P3V_GATED(epilogue) ? 2 * N : N, nk = K / SK_BK, tiles = rows / 128;
+  if (t.gemm_no_skinny || t.gemm_no_merge || M <= (qkv ? 16 : 104) || M > SK_BM || K % SK_BK || rows % 128 || N % 32) return none;
+  if (!qkv && !P3V_GATED(epilogue)) return none;
+  const int S = tiles ? 256 / tiles : 0;                         // one workgroup per CU
+  if (S < 2 || S > 4 || nk < 8 * S || tiles * 4 * 4 > SK_MERGE_FLAGS) return none;
+  return {S, (nk - (nk + 15) / 16) / S, tiles};
+}
+extern "C" int64_t p3v_gemm_merge_ws_bytes(int M, int N, int K, int epilogue, int qkv) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const MergePlan pl = merge_plan(M, N, K, epilogue, qkv != 0);
+  return pl.S ? SK_MERGE_FLAGS + (int64_t)pl.tiles * (pl.S - 1) * (SK_BM * 128 * 4) : 0;
+}
+template <int EPI>
+static int launch_merge(SkinnyP p, const MergePlan& pl, void* ws, hipStream_t s) {
+  typedef SkCfg<128> C;
+  static bool attr_set = false;
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)k_gemm_skinny<EPI, false, 128, SK_BM, true>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS) != hipSuccess) return P3V_ERR_HIP;
+    attr_set = true;
+  }
+  p.xflag = (unsigned*)ws, p.xpart = (float*)((unsigned char*)ws + SK_MERGE_FLAGS), p.nk_part = pl.nk_part;
+  hipLaunchKernelGGL((k_gemm_skinny<EPI, false, 128, SK_BM, true>), dim3(pl.tiles, 1, pl.S), dim3(512), C::LDS, s, p);
+  P3V_CHECK_LAUNCH();
+  return P3V_OK;
+}
+static int merge_args(const p3v_gemm_args_t* a, const void* ws, int64_t ws_bytes, const MergePlan& pl) {
+  if (!pl.S || !ws || ws_bytes < SK_MERGE_FLAGS + (int64_t)pl.tiles * (pl.S - 1) * (SK_BM * 128 * 4)) return P3V_ERR_UNSUPPORTED;
+  if ((uintptr_t)ws & 15) return P3V_ERR_ARG;
+  const size_t rows = (size_t)a->N * (P3V_GATED(a->epilogue) ? 2 : 1);
+  return (size_t)a->M * a->lda * 2 >= (1ull << 32) || rows * a->ldw * 2 >= (1ull << 32) ? P3V_ERR_UNSUPPORTED : P3V_OK;
+}
+extern "C" int p3v_gemm_merge(const p3v_gemm_args_t* a, void* ws, int64_t ws_bytes, void* stream) {
+  if (!a || !a->A || !a->W || !a->out || a->M <= 0 || a->N <= 0 || a->K <= 0 || a->K % SK_BK) return P3V_ERR_ARG;
+  if (a->lda < a->K || a->ldw < a->K || a->lda % 8 || a->ldw % 8 || a->ldo % 8 || a->ldo < a->N) return P3V_ERR_ARG;
+  if (((uintptr_t)a->A | (uintptr_t)a->W | (uintptr_t)a->out) & 15) return P3V_ERR_ARG;
+  if (a->bias) return P3V_ERR_UNSUPPORTED;
+  const MergePlan pl = merge_plan(a->M, a->N, a->K, a->epilogue, false);
+  const int rc = merge_args(a, ws, ws_bytes, pl);
+  if (rc != P3V_OK) return rc;
+  const SkinnyP p = {a->A, a->W, a->out, nullptr, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, nullptr, 0, {}, nullptr, nullptr, 0};
+  hipStream_t s = (hipStream_t)stream;
+  return a->epilogue == P3V_EPI_GELU_MUL ? launch_merge<P3V_EPI_GELU_MUL>(p, pl, ws, s) : launch_merge<P3V_EPI_SILU_MUL>(p, pl, ws, s);
+}
+// p3v_gemm_qkv's case (p3v_gemm.hip has checked the call)
+int p3v_gemm_skinny_qkv_merge(const p3v_gemm_args_t* a, const QkvP& q, void* ws, int64_t ws_bytes, hipStream_t s) {
+  if (a->bias || (q.nh * q.hd) % 128 || (q.nkv * q.hd) % 128) return P3V_ERR_UNSUPPORTED;
+  const MergePlan pl = merge_plan(a->M, a->N, a->K, P3V_EPI_NONE, true);
+  const int rc = merge_args(a, ws, ws_bytes, pl);
+  if (rc != P3V_OK) return rc;
+  const SkinnyP p = {a->A, a->W, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0, nullptr, 0, q, nullptr, nullptr, 0};
+  return launch_merge<P3V_EPI_QKV>(p, pl, ws, s);
 }

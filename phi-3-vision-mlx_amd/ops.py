@@ -6,6 +6,7 @@ Each op names the MLX call site of the reference it replaces.
 """
 import contextlib
 import ctypes as C
+import os
 
 import torch
 
@@ -114,6 +115,51 @@ def _gemm_workspace(device, nbytes):
         buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _gemm_ws[key] = buf
     return buf
+
+
+_merge_ws = {}
+
+
+def _merge_workspace(device, nbytes):
+    """Workspace of the launches that sum their K slices themselves (p3v_gemm_merge, p3v_gemm_qkv_merge): its counters are zero between
+    launches, so it is theirs alone -- one per (device, stream), or the graph's own."""
+    if _ws_owner is not None:
+        holder, frozen = _ws_owner
+        if holder.get("merge") is None or holder["merge"].numel() < nbytes:
+            if frozen:
+                raise RuntimeError(f"merge workspace of {nbytes} bytes requested under graph capture")
+            holder["merge"] = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+        return holder["merge"]
+    key = (device.index, _stream())
+    buf = _merge_ws.get(key)
+    if buf is None or buf.numel() < nbytes:
+        buf = _merge_ws[key] = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+    return buf
+
+
+def _merge_allowed():
+    # P3V_PROFILING=1: no launch may wait for another workgroup of its own grid (a profiler that serialises or masks them)
+    return os.environ.get("P3V_GEMM_MERGE", "1") != "0" and os.environ.get("P3V_PROFILING") != "1"
+
+
+def gemm_merge(a, w, epilogue, out):
+    """gemm with a gated epilogue as K slices summed inside the launch (include/p3v.h); False, nothing launched, where the library does not
+    take the shape that way."""
+    _chk(a, BF16, "a"), _chk(w, BF16, "w")
+    M, K = a.shape
+    N = w.shape[0] // 2
+    if w.shape[1] != K:
+        raise ValueError(f"gemm_merge: K mismatch {a.shape} x {w.shape}")
+    n = L.lib().p3v_gemm_merge_ws_bytes(M, N, K, epilogue, 0) if epilogue in GATED and _merge_allowed() else 0
+    if not n:
+        return False
+    ws = _merge_workspace(a.device, n)
+    args = L.GemmArgs(_p(a), _p(w), _p(out), None, None, None, M, N, K, a.stride(0), w.stride(0), out.stride(0), epilogue, 0, None, 0, None)
+    rc = L.lib().p3v_gemm_merge(C.byref(args), _p(ws), ws.numel(), _stream())
+    if rc == L.ERR_UNSUPPORTED:
+        return False
+    L.check(rc, "gemm_merge")
+    return True
 
 
 def gemm(a, w, epilogue=EPI_NONE, bias=None, resid=None, out=None, n_out=None, pos=None, patches_per_img=0, ldo=None,
@@ -380,6 +426,24 @@ def gemm_qkv(a, w, cos_t, sin_t, q_out, k_dst, v_dst, B, Lq, nh, nkv, hd, past, 
     if rc == L.ERR_UNSUPPORTED:
         return False
     L.check(rc, "gemm_qkv")
+    return True
+
+
+def gemm_qkv_merge(a, w, cos_t, sin_t, q_out, k_dst, v_dst, B, Lq, nh, nkv, hd, past, dst_t, dst_off_is_past, tab_t=0, tab_div=1, q_scale=1.0):
+    """gemm_qkv as K slices summed inside the launch; False -- nothing launched -- when the library does not take the shape that way."""
+    _chk(a, BF16, "a"), _chk(w, BF16, "w")
+    M, K = a.shape
+    n = L.lib().p3v_gemm_merge_ws_bytes(M, w.shape[0], K, EPI_NONE, 1) if _merge_allowed() else 0
+    if not n:
+        return False
+    ws = _merge_workspace(a.device, n)
+    g = L.GemmArgs(_p(a), _p(w), 0, 0, 0, 0, M, w.shape[0], K, a.stride(0), w.stride(0), w.shape[0], EPI_NONE, 0, 0, 0)
+    sp = L.QkvSplit(_p(cos_t), _p(sin_t), _p(q_out), _p(k_dst), _p(v_dst), B, Lq, nh, nkv, hd, int(past), dst_t, int(dst_off_is_past),
+                    tab_t, tab_div, float(q_scale))
+    rc = L.lib().p3v_gemm_qkv_merge(C.byref(g), C.byref(sp), _p(ws), ws.numel(), _stream())
+    if rc == L.ERR_UNSUPPORTED:
+        return False
+    L.check(rc, "gemm_qkv_merge")
     return True
 
 
@@ -764,6 +828,8 @@ def project(x, w, epilogue=EPI_NONE, resid=None, col_scale=None, out=None):
         if M <= 8 and (1 << (M - 1).bit_length()) * K * 2 <= 160 * 1024 - 256:     # (the rows of x in a workgroup's LDS)
             return gemv(x, w, epilogue, resid=resid, out=out, col_scale=col_scale)
         if K % 64 == 0 and N % 8 == 0:
+            if epilogue in GATED and 104 < M <= 128 and gemm_merge(x, w, epilogue, out):
+                return out
             return gemm(x, w, epilogue, resid=resid, out=out, col_scale=col_scale)
     args = L.GemmArgs(_p(x), _p(w), _p(out), 0, _p(resid), 0, M, N, K, x.stride(0), w.stride(0), out.stride(0), epilogue, 0, 0, 0, _p(col_scale))
     L.check(L.lib().p3v_gemm_any(C.byref(args), int(f32), _stream()), "gemm_any")

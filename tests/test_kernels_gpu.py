@@ -929,6 +929,92 @@ def test_gemm_qkv_fused(ops, B, L, nh, nkv, hd, K, past, rot, bias, big):
     assert not torch.equal(k1, k0) and not torch.equal(v1, v0)
 
 
+def _merge_counters(ops):
+    return [b[:4096].view(torch.int32) for b in ops._merge_ws.values()]
+
+
+@pytest.mark.parametrize("B,L,nh,nkv,hd,K,past,rot", [(1, 17, 32, 32, 96, 3072, 64, True), (1, 63, 32, 32, 96, 3072, 0, True), (1, 65, 32, 32, 96, 1536, 0, True),
+                                                     (1, 100, 32, 32, 96, 3072, 8, True), (1, 128, 32, 32, 96, 3072, 0, True), (2, 61, 32, 32, 96, 1536, 0, True),
+                                                     (1, 113, 32, 32, 128, 1088, 0, True), (3, 40, 32, 24, 96, 2112, 0, False)])
+def test_gemm_qkv_merge(ops, B, L, nh, nkv, hd, K, past, rot):
+    """p3v_gemm_qkv_merge against p3v_gemm_qkv: the same products, their fp32 sums in slices of K.  |w| = K^-1/2: a sum of K terms of
+    size 1 / sqrt(K), rounded K / 32 times in other places, moves by less than 2^-16; where that crosses a rounding to bf16 an element of
+    a rotation pair (a, b) is one step (2^-7) off, a rotated one that of |a| + |b| and, its own rounding behind it, another step.  Three launches and a graph's replays: the same
+    bits, the counters back at zero."""
+    M, N, T = B * L, (nh + 2 * nkv) * hd, past + L + 5
+    Tp = (T + 127) // 128 * 128
+    a, w = g((M, K), 400).cuda(), g((N, K), 401, 1.0 / math.sqrt(K)).cuda()
+    torch.manual_seed(3)
+    cos, sin = (torch.rand((B, T, hd // 2), device="cuda"), torch.rand((B, T, hd // 2), device="cuda")) if rot else (None, None)
+    k0, v0 = g((B, nkv, Tp, hd), 403).cuda(), g((B, nkv, hd, Tp), 404).cuda()
+    fresh = lambda: (torch.full((B, nh, L, hd), 7.0, dtype=BF16, device="cuda"), k0.clone(), v0.clone())
+    ref = fresh()
+    assert ops.gemm_qkv(a, w, cos, sin, *ref, B, L, nh, nkv, hd, past, Tp, True, T, 1, q_scale=1.3)
+    outs = []
+    for _ in range(3):
+        outs.append(fresh())
+        assert ops.gemm_qkv_merge(a, w, cos, sin, *outs[-1], B, L, nh, nkv, hd, past, Tp, True, T, 1, q_scale=1.3), "shape not taken"
+        assert all(not c.any() for c in _merge_counters(ops))
+    raw = (a.float() @ w.float().t()).abs().view(B, L, nh + 2 * nkv, hd)
+    raw[:, :, :nh + nkv] += raw[:, :, :nh + nkv].roll(hd // 2, -1)
+    size = [torch.zeros_like(t, dtype=F32) for t in ref]
+    size[0][:] = 1.3 * raw[:, :, :nh].transpose(1, 2)
+    size[1][:, :, past:past + L], size[2][..., past:past + L] = raw[:, :, nh:nh + nkv].transpose(1, 2), raw[:, :, nh + nkv:].permute(0, 2, 3, 1)
+    for x, r, m in zip(outs[0], ref, size):
+        assert torch.all((x.float() - r.float()).abs() <= 2 * 2.0 ** -7 * m + 2.0 ** -14)
+        assert (x != r).float().mean() < 0.02
+    assert torch.equal(outs[0][1][:, :, :past], k0[:, :, :past]) and torch.equal(outs[0][1][:, :, past + L:], k0[:, :, past + L:])
+    assert torch.equal(outs[0][2][..., :past], v0[..., :past]) and torch.equal(outs[0][2][..., past + L:], v0[..., past + L:])
+    for o in outs[1:]:
+        assert all(torch.equal(x, y) for x, y in zip(o, outs[0]))
+    buf, holder = fresh(), {}
+    with ops.owned_gemm_workspace(holder, frozen=False):
+        ops.gemm_qkv_merge(a, w, cos, sin, *buf, B, L, nh, nkv, hd, past, Tp, True, T, 1, q_scale=1.3)
+    torch.cuda.synchronize()
+    graph, side = ops.Graph(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side), ops.owned_gemm_workspace(holder, frozen=True):
+        graph.begin()
+        for _ in range(2):
+            ops.gemm_qkv_merge(a, w, cos, sin, *buf, B, L, nh, nkv, hd, past, Tp, True, T, 1, q_scale=1.3)
+        graph.end()
+    torch.cuda.current_stream().wait_stream(side)
+    for _ in range(3):
+        for t, r in zip(buf, fresh()):
+            t.copy_(r)
+        graph.launch()
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(buf, outs[0])) and not holder["merge"][:4096].any()
+
+
+@pytest.mark.parametrize("M,N,K", [(105, 8192, 3072), (128, 8192, 3072), (120, 5504, 1024), (113, 4096, 2112)])
+@pytest.mark.parametrize("epi", ["silu", "gelu"])
+def test_gemm_merge(ops, M, N, K, epi):
+    """p3v_gemm_merge against the product in 64 bits, as p3v_gemm's gated epilogues are (tolerances of the bf16 output and of the SiLU's
+    roundings), at tiles dealt to 2 .. 4 slices; rows behind the output untouched; repeatable."""
+    e = ops.EPI_SILU_MUL if epi == "silu" else ops.EPI_GELU_MUL
+    a, w = g((M, K), 440).cuda(), g((2 * N, K), 441, 1.0 / math.sqrt(K)).cuda()
+    out = torch.full((M + 3, N), 7.0, dtype=BF16).cuda()
+    assert ops.gemm_merge(a, w, e, out[:M]), "shape not taken"
+    assert torch.all(out[M:] == 7.0) and all(not c.any() for c in _merge_counters(ops))
+    y = a.double() @ w.double().t()
+    gt, up = y[:, :N], y[:, N:]
+    act = torch.nn.functional.silu(gt) if epi == "silu" else torch.nn.functional.gelu(gt, approximate="tanh")
+    ref = act * up
+    tol = 2.0 ** -14 * (2 + gt.abs() + up.abs()) + (2.0 ** -6 if epi == "silu" else 2.0 ** -8) * (ref.abs() + 2.0 ** -2 * up.abs() * gt.abs())
+    assert torch.all((out[:M].double() - ref).abs() <= tol), ((out[:M].double() - ref).abs() - tol).max()
+    again = torch.empty((M, N), dtype=BF16).cuda()
+    assert ops.gemm_merge(a, w, e, again) and torch.equal(again, out[:M])
+
+
+def test_gemm_merge_refuses(ops):
+    """Shapes of the other kernels: False, nothing launched."""
+    for M, N, K in ((104, 8192, 3072), (129, 8192, 3072), (128, 8192, 512), (128, 1024, 3072), (128, 16384, 3072)):
+        out = torch.full((M, N), 7.0, dtype=BF16).cuda()
+        assert not ops.gemm_merge(torch.zeros((M, K), dtype=BF16).cuda(), torch.zeros((2 * N, K), dtype=BF16).cuda(), ops.EPI_SILU_MUL, out)
+        assert torch.all(out == 7.0)
+
+
 @pytest.mark.parametrize("B,L,nh,nkv,hd,K,past,rot", [(1, 2531, 32, 32, 96, 256, 0, True), (1, 17, 8, 8, 96, 384, 64, True), (2, 128, 16, 4, 64, 128, 0, True),
                                                      (3, 333, 16, 8, 96, 640, 8, True), (1, 257, 16, 16, 64, 128, 0, False), (5, 577, 8, 8, 96, 128, 0, True),
                                                      (37, 7, 16, 16, 64, 128, 8, True), (1, 3, 16, 16, 64, 128, 0, True)])
