@@ -188,6 +188,13 @@ int p3v_rope_kv_append(const uint16_t* qkv, const float* cos_t, const float* sin
  *      summed, the residual added, the row normalised by the SAME launch).  P3V_ERR_UNSUPPORTED -- nothing launched, the caller runs the
  *      two calls -- for every other shape, without a workspace of p3v_gemm_ws_bytes(), or N > 3072.  normed: bf16 [M, N] contiguous. */
 int p3v_gemm_resid_norm(const p3v_gemm_args_t* gemm /* host */, const uint16_t* norm_w, float eps, uint16_t* normed, void* stream);
+/* ---- a residual projection of some hundred rows (P3V_EPI_RESID_BF16, _BIAS_RESID_F32, _SCALE_RESID_F32) as slices of K on the tiles of the
+ *      large problems: p3v_gemm's products, the slices' fp32 sums added in slice order by a second launch, which applies the epilogue and,
+ *      with norm_w and normed [M, N] (P3V_EPI_RESID_BF16, N <= 3072; both or neither), writes RMSNorm(out) beside it, bit for bit
+ *      p3v_rmsnorm's.  gemm->ws: p3v_gemm_slices_ws_bytes bytes (0: not a shape of this call), live between the two launches only.
+ *      P3V_ERR_UNSUPPORTED: nothing launched, the caller runs p3v_gemm (+ p3v_rmsnorm).  out may be resid.  Graph-capturable. */
+int64_t p3v_gemm_slices_ws_bytes(int M, int N, int K, int epilogue);
+int p3v_gemm_slices(const p3v_gemm_args_t* gemm /* host */, const uint16_t* norm_w, float eps, uint16_t* normed, void* stream);
 
 /* ---- the same pair for 9 .. 16 rows (a decode batch), the norm split between the projection in front of it and the one behind, no
  *      launch between them:

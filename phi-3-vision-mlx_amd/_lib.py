@@ -154,6 +154,8 @@ SIGNATURES = {
     "p3v_gemm_plan": (i32, [i32, i32, i32, i32]),
     "p3v_gemm_qkv_fp8": (i32, [C.POINTER(GemmF8Args), C.POINTER(QkvSplit), vp]),
     "p3v_gemm_qkv_fp8_pays": (i32, [i32, i32, i32, i32]),
+    "p3v_gemm_slices": (i32, [C.POINTER(GemmArgs), vp, f32, vp, vp]),
+    "p3v_gemm_slices_ws_bytes": (i64, [i32, i32, i32, i32]),
     "p3v_gemm_resid_norm": (i32, [C.POINTER(GemmArgs), vp, f32, vp, vp]),
     "p3v_gemm_rows_resid_parts": (i32, [i32, i32, i32]),
     "p3v_gemm_rows_resid": (i32, [C.POINTER(GemmArgs), vp, vp, vp, vp]),

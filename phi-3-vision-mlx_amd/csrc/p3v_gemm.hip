@@ -409,6 +409,7 @@ __global__ void __launch_bounds__(256) k_splitk_reduce(const float* __restrict__
   if (i >= (long)M * per_row) return;
   const int m = (int)(i / per_row), n = (int)(i - (long)m * per_row) * 8;
   float v[8] = {0, 0, 0, 0, 0, 0, 0, 0}, u[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 4
   for (int z = 0; z < S; ++z) {
     const float* pr = part + ((size_t)z * M + m) * ldp + n;
     const float4 a0 = *(const float4*)pr, a1 = *(const float4*)(pr + 4);
@@ -428,11 +429,16 @@ __global__ void __launch_bounds__(256) k_splitk_reduce(const float* __restrict__
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = r[e] + bf16_round(v[e]);
   }
-  if (EPI == P3V_EPI_SCALE_RESID_F32) {
-    float c[8];
-    load8_bf16(col_scale + n, c);
+  if (EPI == P3V_EPI_SCALE_RESID_F32 || EPI == P3V_EPI_BIAS_RESID_F32) {
+    float c[8] = {0, 0, 0, 0, 0, 0, 0, 0};          // (col_scale carries the bias of the latter; may be null)
+    if (EPI == P3V_EPI_SCALE_RESID_F32 || col_scale) load8_bf16(col_scale + n, c);
     const float* r = (const float*)resid + o;
     const float4 r0 = *(const float4*)r, r1 = *(const float4*)(r + 4);
+    if (EPI == P3V_EPI_BIAS_RESID_F32) {
+      *(float4*)((float*)out + o) = make_float4(r0.x + (v[0] + c[0]), r0.y + (v[1] + c[1]), r0.z + (v[2] + c[2]), r0.w + (v[3] + c[3]));
+      *(float4*)((float*)out + o + 4) = make_float4(r1.x + (v[4] + c[4]), r1.y + (v[5] + c[5]), r1.z + (v[6] + c[6]), r1.w + (v[7] + c[7]));
+      return;
+    }
     *(float4*)((float*)out + o) = make_float4(r0.x + c[0] * v[0], r0.y + c[1] * v[1], r0.z + c[2] * v[2], r0.w + c[3] * v[3]);
     *(float4*)((float*)out + o + 4) = make_float4(r1.x + c[4] * v[4], r1.y + c[5] * v[5], r1.z + c[6] * v[6], r1.w + c[7] * v[7]);
     return;
@@ -455,6 +461,7 @@ __global__ void __launch_bounds__(384) k_splitk_reduce_norm(const float* __restr
   u32x4_t v = {0u, 0u, 0u, 0u}, g = {0u, 0u, 0u, 0u};
   if (c < chunks) {
     float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 4
     for (int z = 0; z < S; ++z) {
       const float* pr = part + ((size_t)z * M + row) * N + c * 8;
       const float4 a0 = *(const float4*)pr, a1 = *(const float4*)(pr + 4);
@@ -554,6 +561,8 @@ int p3v_splitk_reduce(const float* part, const p3v_gemm_args_t* a, int S, hipStr
   else if (silu) hipLaunchKernelGGL(k_splitk_reduce<P3V_EPI_SILU_MUL>, grid, dim3(256), 0, s, part, a->out, a->resid, a->col_scale, a->M, a->N, w_rows, a->ldo, S);
   else if (a->epilogue == P3V_EPI_SCALE_RESID_F32)
     hipLaunchKernelGGL(k_splitk_reduce<P3V_EPI_SCALE_RESID_F32>, grid, dim3(256), 0, s, part, a->out, a->resid, a->col_scale, a->M, a->N, w_rows, a->ldo, S);
+  else if (a->epilogue == P3V_EPI_BIAS_RESID_F32)
+    hipLaunchKernelGGL(k_splitk_reduce<P3V_EPI_BIAS_RESID_F32>, grid, dim3(256), 0, s, part, a->out, a->resid, a->bias, a->M, a->N, w_rows, a->ldo, S);
   else if (a->epilogue == P3V_EPI_RESID_BF16)
     hipLaunchKernelGGL(k_splitk_reduce<P3V_EPI_RESID_BF16>, grid, dim3(256), 0, s, part, a->out, a->resid, a->col_scale, a->M, a->N, w_rows, a->ldo, S);
   else hipLaunchKernelGGL(k_splitk_reduce<P3V_EPI_NONE>, grid, dim3(256), 0, s, part, a->out, a->resid, a->col_scale, a->M, a->N, w_rows, a->ldo, S);
@@ -574,6 +583,72 @@ static int gemm_splitk(const p3v_gemm_args_t* a, hipStream_t s) {
   const int rc = launch_gemm<P3V_EPI_F32>(p, s);
   if (rc != P3V_OK) return rc;
   return p3v_splitk_reduce(part, a, S, s);
+}
+
+// ---- K slices on the flat tiles (p3v_gemm_pc.hip): residual projections of some hundred rows, whose tiles leave most of the chip idle.
+// 300 x 3072 has 48 tiles of 128 x 192 and 1154 x 1024 (two image crops) 40 of 128 x 256: as many slices of K as one round of the chip takes,
+// whole K-tiles each, fp32 partials in the caller's workspace, and a second launch that adds them in slice order.  Measured in us, with the
+// RMSNorm behind it where there is one, against the paths of p3v_gemm (+ p3v_rmsnorm): 300 x 3072 x 8192 44.6 -> 31.7, 512 56.2 -> 39.3,
+// 1000 90.5 -> 59.5, 1536 91.8 -> 78.6; 512 x 3072 x 3072 31.8 -> 25.8, 1100 51.5 -> 37.5; 577 x 1024 x 4096 (bias, fp32 residual) 60.6 -> 22.8,
+// 2308 58.8 -> 33.8, 4039 60.9 -> 45.5.
+// The rule: one round's time by tile, fitted to those and 40 more (within 2 us): a constant for both launches, the K-tiles of the longest slice,
+// and 0.2 us per MB of partials written and read.  It has to promise 5 % over one pass on one of the flat tiles (gemm_tile_plan's times) and
+// the 6 us of the norm's own launch (up to 256 rows over the kernel for few rows, from where that needs two passes over a long K: 256 x 3072 x
+// 8192 35.2 -> 30.8, 160 29.2 -> 27.8, 128 24.7 -> 25.4); the sizes it turns down measured slower (1300 x 3072 x 3072: 42.1 against 40.5; 1154 x 1024 x 1024: 21.1, 15.7).
+struct SlicePlan { int S, mb, nb; };
+static SlicePlan gemm_slices_plan(int M, int N, int K, int epilogue) {
+  const P3vTuning& t = p3v_tuning();
+  const SlicePlan none = {0, 0, 0};
+  if (!t.gemm_slices || (t.gemm_slices < 0 && M <= (K < 8192 ? 256 : 192)) || K % BK) return none;
+  if (epilogue != P3V_EPI_RESID_BF16 && epilogue != P3V_EPI_BIAS_RESID_F32 && epilogue != P3V_EPI_SCALE_RESID_F32) return none;
+  if (t.gemm_slices > 0) {
+    const SlicePlan p = {t.gemm_slices / 100, t.gemm_slices / 10 % 10, t.gemm_slices % 10};
+    return p.S < 1 || p.S > K / BK || !p.nb || N % (64 * p.nb) ? none : p;
+  }
+  struct Tile { int mb, nb; float f, c, one_f, one_c; };
+  static const Tile tiles[] = {{4, 3, 13.3f, 0.64f, 5.5f, 0.61f}, {4, 4, 14.f, 0.72f, 6.6f, 0.69f}, {5, 4, 15.f, 0.87f, 7.9f, 0.79f}};
+  const int nk = K / BK;
+  float one = 1e30f, best = 1e30f;
+  SlicePlan plan = none;
+  for (const Tile& t : tiles) {
+    if (N % (64 * t.nb)) continue;
+    const long n = (long)p3v_cdiv(M, 32 * t.mb) * (N / (64 * t.nb));
+    one = fminf(one, (float)p3v_cdiv(n, 256) * (t.one_f + t.one_c * nk));
+    for (int S = 2; S <= 16 && n * S <= 256 && nk >= 3 * S; ++S) {
+      const float c = t.f + t.c * p3v_cdiv(nk, S) + 0.2f * S * M * N * 4e-6f;
+      if (c < best) best = c, plan = {S, t.mb, t.nb};
+    }
+  }
+  return best < 0.95f * (one + (epilogue == P3V_EPI_RESID_BF16 ? 6.f : 0.f)) ? plan : none;
+}
+
+extern "C" int64_t p3v_gemm_slices_ws_bytes(int M, int N, int K, int epilogue) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return (int64_t)gemm_slices_plan(M, N, K, epilogue).S * M * N * 4;
+}
+
+int p3v_gemm256_slices(const p3v_gemm_args_t* a, float* part, int S, int mb, int nb, hipStream_t s);   // p3v_gemm256.hip
+
+extern "C" int p3v_gemm_slices(const p3v_gemm_args_t* a, const uint16_t* norm_w, float eps, uint16_t* normed, void* stream) {
+  if (!a || !a->A || !a->W || !a->out || !a->resid || !norm_w != !normed) return P3V_ERR_ARG;
+  if (a->M <= 0 || a->N <= 0 || a->K <= 0 || a->K % BK || a->N % 8 || a->ldo % 8 || a->ldo < a->N) return P3V_ERR_ARG;
+  if (a->lda < a->K || a->ldw < a->K || a->lda % 8 || a->ldw % 8) return P3V_ERR_ARG;
+  if (((uintptr_t)a->A | (uintptr_t)a->W | (uintptr_t)a->out | (uintptr_t)a->resid | (uintptr_t)a->bias | (uintptr_t)a->col_scale | (uintptr_t)norm_w | (uintptr_t)normed | (uintptr_t)a->ws) & 15)
+    return P3V_ERR_ARG;
+  const bool scale = a->epilogue == P3V_EPI_SCALE_RESID_F32;
+  if (scale != (a->col_scale != nullptr)) return P3V_ERR_ARG;
+  if (a->bias && a->epilogue != P3V_EPI_BIAS_RESID_F32) return P3V_ERR_ARG;
+  if (norm_w && (a->epilogue != P3V_EPI_RESID_BF16 || a->N > 6 * 64 * 8)) return P3V_ERR_UNSUPPORTED;
+  const SlicePlan p = gemm_slices_plan(a->M, a->N, a->K, a->epilogue);
+  if (!p.S || !a->ws || a->ws_bytes < (int64_t)p.S * a->M * a->N * 4) return P3V_ERR_UNSUPPORTED;
+  hipStream_t s = (hipStream_t)stream;
+  float* part = (float*)a->ws;
+  if (const int rc = p3v_gemm256_slices(a, part, p.S, p.mb, p.nb, s); rc != P3V_OK) return rc;
+  if (!norm_w) return p3v_splitk_reduce(part, a, p.S, s);
+  hipLaunchKernelGGL(k_splitk_reduce_norm, dim3(a->M), dim3(384), 0, s, part, (bf16_t*)a->out, (const bf16_t*)a->resid,
+                     (const u32x4_t*)norm_w, (u32x4_t*)normed, a->M, a->N, a->ldo, p.S, 1.0f / (float)a->N, eps);
+  P3V_CHECK_LAUNCH();
+  return P3V_OK;
 }
 
 extern "C" int p3v_gemm(const p3v_gemm_args_t* a, void* stream) {

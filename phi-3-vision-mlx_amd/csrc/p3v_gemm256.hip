@@ -323,3 +323,12 @@ int p3v_gemm256_try(const p3v_gemm_args_t* a, int mb, int nb, hipStream_t s) {
     default: return P3V_ERR_UNSUPPORTED;
   }
 }
+
+// the K slices of p3v_gemm_slices (p3v_gemm.hip): fp32 partials [S, M, N] of a whole problem on a flat tile
+int p3v_gemm256_slices(const p3v_gemm_args_t* a, float* part, int S, int mb, int nb, hipStream_t s) {
+  const int tile = 10 * mb + nb;
+  if ((tile != 54 && tile != 44 && tile != 43) || a->N % (64 * nb) || a->K % TK || S < 1 || S > a->K / TK) return P3V_ERR_UNSUPPORTED;
+  if ((size_t)a->N * a->ldw * 2 >= ((size_t)1 << 32) || (size_t)a->M * a->lda * 2 >= ((size_t)1 << 32)) return P3V_ERR_UNSUPPORTED;  // 32-bit buffer offsets
+  const Gemm256P p = {a->A, a->W, part, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, a->N, {}, S};
+  return p3v_gemm_pc(p, P3V_EPI_PART, mb, nb, s);
+}

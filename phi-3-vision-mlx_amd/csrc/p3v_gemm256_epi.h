@@ -4,6 +4,8 @@
 
 #define P3V_EPI_QKV 100                // internal: the qkv projection with split + RoPE + KV append in the epilogue (p3v_gemm_qkv.h)
 
+#define P3V_EPI_PART 101               // internal: the fp32 partial sums of one slice of K, out [slices, M, N] (p3v_gemm_slices, p3v_gemm.hip)
+
 #define TK 64
 
 typedef const __attribute__((address_space(1))) void* gptr_t;
@@ -13,6 +15,7 @@ struct Gemm256P {
   const bf16_t* A; const bf16_t* W; void* out; const bf16_t* bias; const void* resid;
   int M, N, K, lda, ldw, ldo;
   QkvP q;                                // P3V_EPI_QKV only
+  int slices;                            // P3V_EPI_PART only: slice z takes the K-tiles z nk / slices .. (z + 1) nk / slices
 };
 
 __device__ __forceinline__ float gelu_erf2(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }

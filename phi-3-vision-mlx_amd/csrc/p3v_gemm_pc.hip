@@ -10,6 +10,7 @@
 //            MFMAs; larger tiles do not fit the 168 registers that twelve waves leave each other.
 // 2531 x 3072 x 8192 (+ residual) 117 -> 105 us (1.21 PFLOP/s), 9809 x 1024 x 4096 (+ fp32 residual) 95 -> 73, 2048 x 9472 x 3072 114 -> 97.
 // Same K order and epilogue as the other tiles: bit-identical results.
+// P3V_EPI_PART: the tiles of one slice of K after the other, fp32 partials (p3v_gemm_slices, p3v_gemm.hip, which has the rule and the times).
 // (Tried and left out: touching the lines of later K-tiles ahead of the DMA, one dword per line -- 64 lines cost the address path as
 //  much as four pieces: 105 -> 137 us; 4 consumers of twice the size without producers: 121 us.)
 #include "p3v_gemm256_epi.h"
@@ -32,32 +33,45 @@ __global__ void __launch_bounds__(768, 1) k_gemm_pc(Gemm256P p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform: LDS-DMA bases stay in SGPRs
   constexpr int n_out_tile = SILU ? TN / 2 : TN;
-  const int gx = (p.N + n_out_tile - 1) / n_out_tile, gy = (p.M + TM - 1) / TM, nwg = gx * gy;
+  constexpr bool PART = EPI == P3V_EPI_PART;
+  const int gx = (p.N + n_out_tile - 1) / n_out_tile, gy = (p.M + TM - 1) / TM, nwg = PART ? gx * gy * p.slices : gx * gy;
   const int nk = p.K / TK;
 
   // ---- PERSISTENT over output tiles: workgroup b takes tiles b, b + G, b + 2G, ... (G = gridDim.x, a multiple of 8, so a
   // workgroup's tiles keep its XCD in the XCD-aware order below), one stream of K-tiles across all of them.
-  auto place = [&](int wid, int& m0, int& n0) {
+  // PART: the slices one after the other, so an XCD keeps to one slice of K or two: A and W pass each L2 once, whatever the tile order.
+  auto place = [&](int wid, int& m0, int& n0, int& z) {
     const int q = nwg >> 3, r = nwg & 7, xcd = wid & 7, loc = wid >> 3;
-    const int id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + loc;
+    int id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + loc;
+    z = 0;
+    if (PART) z = id / (gx * gy), id -= z * (gx * gy);
     constexpr int BAND = 4;
     const int band = id / (BAND * gx), in_band = id % (BAND * gx);
     const int rows = min(BAND, gy - band * BAND);
     m0 = (band * BAND + in_band % rows) * TM, n0 = in_band / rows * n_out_tile;
   };
+  auto k_begin = [&](int z) { return PART ? z * nk / p.slices : 0; };
+  auto k_end = [&](int z) { return PART ? (z + 1) * nk / p.slices : nk; };
   if ((int)blockIdx.x >= nwg) return;
-  const int n_mine = (nwg - 1 - (int)blockIdx.x) / (int)gridDim.x + 1, total = n_mine * nk;      // output tiles, K-tiles of this workgroup
+  int total = 0;                                                  // K-tiles of this workgroup
+  if (PART) {
+    for (int wid = blockIdx.x, m0, n0, z; wid < nwg; wid += gridDim.x) place(wid, m0, n0, z), total += k_end(z) - k_begin(z);
+  } else {
+    total = ((nwg - 1 - (int)blockIdx.x) / (int)gridDim.x + 1) * nk;
+  }
 
   if (wave >= 8) {
     // ---- PRODUCERS.  A request = 8 tile rows x 128 B (1 KiB) by LDS-DMA; the 16-byte chunks of a row are swizzled on the source side.
     // Buffer addressing (SGPR descriptor + 32-bit per-lane byte offset + SGPR K offset): no vector ALU work at all.
     const int pw = wave - 8, srow = pw * 8 + (lane >> 3), sw = ((lane & 7) ^ (lane >> 3)) * 8;
     const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, 0xffffffff, 0x00020000);
+    int dk = 0, dk_end = nk;                                      // the K-tiles still to be requested for the tile in hand
     TilePc dt;   // (declared outside the template: a builtin called with a member of a DEPENDENT type is only checked at
                   //  instantiation, fails there in the HOST pass -- no such builtin -- and hipcc silently drops the host stub)
     auto aim = [&](int wid) {
-      int m0, n0;
-      place(wid, m0, n0);
+      int m0, n0, z;
+      place(wid, m0, n0, z);
+      dk = k_begin(z), dk_end = k_end(z);
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const int rr = q * 32 + srow;
@@ -71,7 +85,7 @@ __global__ void __launch_bounds__(768, 1) k_gemm_pc(Gemm256P p) {
       }
       dt.rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + (size_t)m0 * p.lda), 0, 0xffffffff, 0x00020000);
     };
-    int dwid = blockIdx.x, dk = 0, slot = 0;                      // the next K-tile to request, and its buffer
+    int dwid = blockIdx.x, slot = 0;                              // the tile in hand, and the next K-tile's buffer
     aim(dwid);
     auto request = [&]() {
       unsigned char* base = smem + slot * (int)BUF_BYTES + pw * 1024;
@@ -93,8 +107,7 @@ __global__ void __launch_bounds__(768, 1) k_gemm_pc(Gemm256P p) {
         }
       }
       slot = slot == S - 1 ? 0 : slot + 1;
-      if (++dk == nk) {
-        dk = 0;
+      if (++dk == dk_end) {
         dwid += gridDim.x;
         if (dwid < nwg) aim(dwid);
       }
@@ -143,8 +156,9 @@ __global__ void __launch_bounds__(768, 1) k_gemm_pc(Gemm256P p) {
   int slot = 0;                                                   // LDS buffer of the K-tile in hand
   __builtin_amdgcn_s_barrier();
   for (int wid = blockIdx.x; wid < nwg; wid += gridDim.x) {
-    int m0, n0;
-    place(wid, m0, n0);
+    int m0, n0, z;
+    place(wid, m0, n0, z);
+    const int nkt = k_end(z) - k_begin(z);
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -153,16 +167,22 @@ __global__ void __launch_bounds__(768, 1) k_gemm_pc(Gemm256P p) {
     for (int n = 0; n < MB + NB; ++n) fetch(n, 0, slot);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll 1
-    for (int kt = 0; kt < nk; ++kt) {
+    for (int kt = 0; kt < nkt; ++kt) {
       const int nslot = slot == S - 1 ? 0 : slot + 1;
-      const bool last = kt + 1 == nk;                              // (nothing is fetched behind a tile's last K-tile: the epilogue needs the registers)
+      const bool last = kt + 1 == nkt;                             // (nothing is fetched behind a tile's last K-tile: the epilogue needs the registers)
       half(0, true, slot);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");           // the K-tile in hand is in registers: its buffer is given back
       if (!last || wid + (int)gridDim.x < nwg) __builtin_amdgcn_s_barrier();
       half(1, !last, nslot);
       slot = nslot;
     }
-    gemm256_epilogue<EPI, MB, NB>(p, acc, m0 + wr * MB * 16, n0 + wc * (n_out_tile / 4), lane);   // straight from the accumulators: p3v_gemm256_epi.h
+    if constexpr (PART) {
+      Gemm256P part = p;
+      part.out = (float*)p.out + (size_t)z * p.M * p.ldo;
+      gemm256_epilogue<P3V_EPI_F32, MB, NB>(part, acc, m0 + wr * MB * 16, n0 + wc * (n_out_tile / 4), lane);
+    } else {
+      gemm256_epilogue<EPI, MB, NB>(p, acc, m0 + wr * MB * 16, n0 + wc * (n_out_tile / 4), lane);  // straight from the accumulators: p3v_gemm256_epi.h
+    }
   }
 }
 
@@ -178,7 +198,7 @@ static int launch_pc_v(const Gemm256P& p, hipStream_t s) {
   }
   const int n_cu = p3v_gemm256_cus();
   if (!n_cu) return P3V_ERR_HIP;
-  const int tiles = p3v_cdiv(p.N, P3V_GATED(EPI) ? 32 * NB : 64 * NB) * p3v_cdiv(p.M, 32 * MB);
+  const int tiles = p3v_cdiv(p.N, P3V_GATED(EPI) ? 32 * NB : 64 * NB) * p3v_cdiv(p.M, 32 * MB) * (EPI == P3V_EPI_PART ? p.slices : 1);
   hipLaunchKernelGGL((k_gemm_pc<EPI, MB, NB>), dim3(min(tiles, n_cu)), dim3(768), LDS, s, p);
   P3V_CHECK_LAUNCH();
   return P3V_OK;
@@ -203,6 +223,7 @@ int p3v_gemm_pc(const Gemm256P& p, int epi, int mb, int nb, hipStream_t s) {
     case P3V_EPI_GELU_MUL: return launch_pc<P3V_EPI_GELU_MUL>(p, mb, nb, s);
     case P3V_EPI_F32: return launch_pc<P3V_EPI_F32>(p, mb, nb, s);
     case P3V_EPI_SCALE_RESID_F32: return launch_pc<P3V_EPI_SCALE_RESID_F32>(p, mb, nb, s);
+    case P3V_EPI_PART: return launch_pc<P3V_EPI_PART>(p, mb, nb, s);
     default: return P3V_ERR_UNSUPPORTED;
   }
 }

@@ -173,16 +173,19 @@ class Phi3VModel(DecoderModel):
             x = ops.rmsnorm(x, norm_w, eps, out=h)
         if epilogue == EPI_SILU_MUL and 104 < M <= 128 and out is not None and ops.gemm_merge(x, w, epilogue, out):
             return out
+        if epilogue == EPI_RESID_BF16 and out is not None and ops.gemm_slices(x, w, epilogue, resid, out):
+            return out
         return ops.gemm(x, w, epilogue, resid=resid, out=out)
 
     def _proj_resid_norm(self, o, key, x, norm_w, h):
-        """x += bf16(o @ W^T) and h = RMSNorm(x) * norm_w from the projection's own launches (ops.gemm_resid_norm); False -- nothing
+        """x += bf16(o @ W^T) and h = RMSNorm(x) * norm_w from the projection's own launches (ops.gemm_slices, ops.gemm_resid_norm); False -- nothing
         done -- where that does not apply (adapters, quantised weights, shapes the library does not run as K slices)."""
         M = o.shape[0]
         if (key in self.adapters or key not in self.w or M <= 8 or h.shape[0] < M
                 or os.environ.get("P3V_RESID_NORM_FUSE", "1") == "0"):
             return False
-        return ops.gemm_resid_norm(o, self.w[key], x, norm_w, self.cfg.rms_norm_eps, h[:M], out=x)
+        w, eps = self.w[key], self.cfg.rms_norm_eps
+        return ops.gemm_slices(o, w, EPI_RESID_BF16, x, x, norm=(norm_w, eps, h[:M])) or ops.gemm_resid_norm(o, w, x, norm_w, eps, h[:M], out=x)
 
     def _proj_resid_scaled(self, o, key, x, norm_w, h, sq, next_key):
         """x += bf16(o @ W^T), h = bf16(x * norm_w) and the rows' sums of squares (ops.gemm_rows_resid), for the projection `next_key` that
@@ -306,12 +309,16 @@ class Phi3VModel(DecoderModel):
                 ops.gemm(h, wq, EPI_BIAS, bias=bq, out=qkv)
                 ops.rope_kv_append(qkv, None, None, q, k, v, n, T, nh, nh, 64, 0, Tp, False, q_scale=qs)
             ops.attention(q, o, n, T, nh, nh, 64, 64 ** -0.5, False, k_past=k, v_past=v, past_t=Tp, new_is_cache=True, q_prescaled=pre)
-            ops.gemm(o, w[lp + "self_attn.out_proj.weight"], EPI_BIAS_RESID_F32, bias=w[lp + "self_attn.out_proj.bias"],
-                     resid=x2, out=x2)
+            self._clip_resid(o, lp + "self_attn.out_proj", x2)
             ops.layernorm(x2, w[lp + "layer_norm2.weight"], w[lp + "layer_norm2.bias"], eps, out=h)
             ops.gemm(h, w[lp + "mlp.fc1.weight"], EPI_BIAS_QGELU, bias=w[lp + "mlp.fc1.bias"], out=f)
-            ops.gemm(f, w[lp + "mlp.fc2.weight"], EPI_BIAS_RESID_F32, bias=w[lp + "mlp.fc2.bias"], resid=x2, out=x2)
+            self._clip_resid(f, lp + "mlp.fc2", x2)
         return x
+
+    def _clip_resid(self, a, key, x):
+        w, bias = self.w[key + ".weight"], self.w[key + ".bias"]
+        if not ops.gemm_slices(a, w, EPI_BIAS_RESID_F32, x, x, bias=bias):
+            ops.gemm(a, w, EPI_BIAS_RESID_F32, bias=bias, resid=x, out=x)
 
     def vision_embed(self, x, pixel_values, image_sizes, positions, L):
         """Phi3ImageEmbedding.__call__ (phi.py:393-416): ViT on the live crops

@@ -205,6 +205,34 @@ def gemm_resid_norm(a, w, resid, norm_w, eps, normed, out=None):
     return True
 
 
+def gemm_slices(a, w, epilogue, resid, out, bias=None, col_scale=None, norm=None):
+    """gemm with a residual epilogue as slices of K (include/p3v.h: p3v_gemm_slices); norm = (weight, eps, normed): and normed = RMSNorm(out)
+    from the launch that adds the slices (EPI_RESID_BF16).  False -- nothing launched -- where the library does not take the shape that way."""
+    M, K = a.shape
+    N = w.shape[0]
+    n = L.lib().p3v_gemm_slices_ws_bytes(M, N, K, epilogue)
+    if not n:
+        return False
+    stream = F32 if epilogue in (EPI_BIAS_RESID_F32, EPI_SCALE_RESID_F32) else BF16
+    _chk(a, BF16, "a"), _chk(w, BF16, "w"), _chk(resid, stream, "resid"), _chk(out, stream, "out")
+    if w.shape[1] != K or resid.shape != (M, N) or out.shape != (M, N):
+        raise ValueError(f"gemm_slices: shapes {a.shape} x {w.shape}, resid {resid.shape}, out {out.shape}")
+    for v, name in ((bias, "bias"), (col_scale, "col_scale"), (norm[0] if norm else None, "norm weight")):
+        if v is not None and _chk(v, BF16, name).numel() != N:
+            raise ValueError(f"gemm_slices: {name} of {v.numel()} for {N} columns")
+    norm_w, eps, normed = norm or (None, 0.0, None)
+    if normed is not None and _chk(normed, BF16, "normed").shape != (M, N):
+        raise ValueError(f"gemm_slices: normed {normed.shape}")
+    ws = _gemm_workspace(a.device, n)
+    args = L.GemmArgs(_p(a), _p(w), _p(out), _p(bias), _p(resid), None, M, N, K, a.stride(0), w.stride(0), out.stride(0), epilogue, 0,
+                      _p(ws), ws.numel(), _p(col_scale))
+    rc = L.lib().p3v_gemm_slices(C.byref(args), _p(norm_w), float(eps), _p(normed), _stream())
+    if rc == L.ERR_UNSUPPORTED:
+        return False
+    L.check(rc, "gemm_slices")
+    return True
+
+
 def gemm_rows_resid(a, w, resid, norm_w, scaled, sumsq, out=None):
     """out = resid + bf16(a @ w^T), scaled = bf16(out * norm_w) and sumsq [parts, 16] = the squares of out's rows piece by piece, in one
     launch: the first half of the RMSNorm in front of the next projection (gemm_rows_scaled is the other).  Returns the number of pieces;
@@ -829,6 +857,8 @@ def project(x, w, epilogue=EPI_NONE, resid=None, col_scale=None, out=None):
             return gemv(x, w, epilogue, resid=resid, out=out, col_scale=col_scale)
         if K % 64 == 0 and N % 8 == 0:
             if epilogue in GATED and 104 < M <= 128 and gemm_merge(x, w, epilogue, out):
+                return out
+            if scaled and gemm_slices(x, w, epilogue, resid, out, col_scale=col_scale):
                 return out
             return gemm(x, w, epilogue, resid=resid, out=out, col_scale=col_scale)
     args = L.GemmArgs(_p(x), _p(w), _p(out), 0, _p(resid), 0, M, N, K, x.stride(0), w.stride(0), out.stride(0), epilogue, 0, 0, 0, _p(col_scale))

@@ -286,6 +286,54 @@ def test_gemm_resid_norm_is_the_two_calls(ops, M, N, K):
     assert bool((sentinel == 7.0).all())
 
 
+@pytest.mark.parametrize("M,N,K,pin,kind", [(300, 3072, 8192, -1, "norm"), (200, 3072, 8192, -1, "norm"), (1023, 3072, 3072, -1, "norm"), (257, 384, 192, 343, "norm"),
+                                            (129, 768, 448, 344, "norm"), (161, 256, 1024, 1654, "norm"), (1, 512, 704, 554, "norm"), (641, 1536, 320, 244, "norm"),
+                                            (577, 1024, 4096, -1, "bias"), (2308, 1024, 4096, -1, "bias"), (33, 192, 256, 443, "bias"),
+                                            (768, 3072, 8192, -1, "scale"), (5, 256, 576, 944, "scale"), (4000, 3072, 192, 354, "norm")])
+def test_gemm_slices(ops, M, N, K, pin, kind):
+    """p3v_gemm_slices: the planned slices of the models' sizes, and pinned ones (100 S + tile) with slices of one K-tile, of unequal lengths,
+    over several rounds of the chip, ragged last rows.  The stream: within one bf16 step of its value and of the product's from fp64 (the
+    product is rounded, then the sum), fp32 streams within K fp32 roundings; the norm: p3v_rmsnorm of the stream, bit for bit; in place."""
+    f32 = kind != "norm"
+    a, w, r = g((M, K), 76).cuda(), g((N, K), 77, 1.0 / math.sqrt(K)).cuda(), g((M, N), 78, 1.0, F32 if f32 else BF16).cuda()
+    v = (g((N,), 79, 0.3) + 1).cuda()
+    epi = {"norm": ops.EPI_RESID_BF16, "bias": ops.EPI_BIAS_RESID_F32, "scale": ops.EPI_SCALE_RESID_F32}[kind]
+    kw = {"norm": {}, "bias": dict(bias=v), "scale": dict(col_scale=v)}[kind]
+    prod = a.double() @ w.double().t()
+    want = r.double() + (prod if kind == "norm" else prod + v.double() if kind == "bias" else prod * v.double())
+    out, normed = torch.full_like(r, 7.0), torch.full((M, N), 7.0, dtype=BF16, device="cuda")
+    saved = ops.set_tuning("gemm_slices", pin)
+    try:
+        assert ops.gemm_slices(a, w, epi, r, out, norm=None if f32 else (v, 1e-5, normed), **kw)
+        tol = (a.double().abs() @ w.double().abs().t()) * (1 + v.double().abs()) * K * 2 ** -24 + 1e-6 if f32 else 2 ** -8 * (want.abs() + prod.abs()) * 1.01 + 1e-5
+        assert bool(((out.double() - want).abs() <= tol).all())
+        if not f32:
+            assert torch.equal(normed, ops.rmsnorm(out, v, 1e-5))
+        x = r.clone()
+        assert ops.gemm_slices(a, w, epi, x, x, **kw) and torch.equal(x, out)
+    finally:
+        ops.set_tuning("gemm_slices", saved)
+
+
+@pytest.mark.parametrize("M,N,K,epi", [(300, 3072, 3072, "NONE"), (300, 3072, 3072, "SILU_MUL"), (192, 3072, 8192, "RESID_BF16"), (256, 3072, 3072, "RESID_BF16"),
+                                       (2531, 3072, 8192, "RESID_BF16"), (9809, 1024, 4096, "BIAS_RESID_F32"), (577, 1024, 1024, "BIAS_RESID_F32"), (300, 3080, 3072, "RESID_BF16")])
+def test_gemm_slices_refuses(ops, M, N, K, epi):
+    """Epilogues and sizes that run in one pass (or on the kernels for few rows), and widths without a whole tile: no workspace, no launch."""
+    import ctypes as C
+    l, L = ops.L.lib(), ops.L
+    epi = getattr(ops, "EPI_" + epi)
+    assert l.p3v_gemm_slices_ws_bytes(M, N, K, epi) == 0 and l.p3v_gemm_slices_ws_bytes(0, N, K, epi) == 0
+    a, w = torch.zeros((M, K), dtype=BF16, device="cuda"), torch.zeros((2 * N, K), dtype=BF16, device="cuda")
+    r = torch.full((M, N), 3.0, dtype=F32, device="cuda")
+    ws = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+    args = L.GemmArgs(a.data_ptr(), w.data_ptr(), r.data_ptr(), None, r.data_ptr(), None, M, N, K, K, K, N, epi, 0, ws.data_ptr(), ws.numel(), None)
+    assert l.p3v_gemm_slices(C.byref(args), None, 0.0, None, ops._stream()) == L.ERR_UNSUPPORTED
+    args.ws_bytes, args.M, args.N, args.K, args.lda, args.ldw, args.ldo, args.epilogue = 16, 300, 3072, 3072, 3072, 3072, 3072, ops.EPI_RESID_BF16
+    assert l.p3v_gemm_slices(C.byref(args), None, 0.0, None, ops._stream()) == L.ERR_UNSUPPORTED      # a workspace too small
+    torch.cuda.synchronize()
+    assert bool((r == 3.0).all())
+
+
 @pytest.mark.parametrize("epi,M,N,K", [("resid_bf16", 129, 3072, 8192), ("silu", 40, 1024, 3072), ("none", 300, 9216, 3072)])
 def test_gemm_splitk_workspace_is_the_callers(ops, epi, M, N, K):
     """p3v_gemm never allocates: the split-K partials live in a workspace the caller sizes with p3v_gemm_ws_bytes.  With the
