@@ -214,8 +214,8 @@ int p3v_gemm_rows_scaled(const p3v_gemm_args_t* gemm /* host */, const float* su
  *      + head split).  g: A [B*L, K], W [(nh + 2 nkv) * hd, K] (q rows, k rows, v rows), epilogue P3V_EPI_NONE or P3V_EPI_BIAS; out /
  *      resid / ws unused.  P3V_ERR_UNSUPPORTED (nothing launched) unless hd % 32 == 0, (hd / 2) % 16 == 0, an 8-aligned append
  *      offset and dst_t (batch rows of any length L from 7 on -- CLIP's 577-token crops), and either M >= 1024 with whole 128-column tiles per region (the 256 x 256 /
- *      128 x 128-tile kernels) or 9 <= M <= 256 without bias, whole 64-column Q / K tiles and 128-row V tiles (the 128 x 64-tile
- *      weight-streaming kernel) -- callers then run the two calls. */
+ *      128 x 128-tile kernels), 257 <= M < 1024 with whole 256-column Q / K tiles where p3v_gemm would take a flat tile in one round, or 9 <= M <= 256 without bias, whole
+ *      64-column Q / K tiles and 128-row V tiles (the 128 x 64-tile weight-streaming kernel) -- callers then run the two calls. */
 typedef struct {
   const float* cos_t; const float* sin_t;          /* as p3v_rope_kv_append; both null: plain head split */
   uint16_t* q_out; uint16_t* k_dst; uint16_t* v_dst;

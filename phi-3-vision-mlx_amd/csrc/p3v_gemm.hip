@@ -326,7 +326,8 @@ static int gemm128(const p3v_gemm_args_t* a, hipStream_t s);
 // per round; a round of big tiles costs 1, a round of small ones 0.675 (half the output area at 0.97 vs 1.31
 // PFLOP/s), a last round that leaves every CU at most one small workgroup 0.42 -- pick the cheapest whole-round
 // packing, e.g. 2531 x 16384 (gate_up): 8 x 64 = 512 big tiles = 2 rounds + 4 x 128 small = 1 round.
-static int gemm_big_rows(const p3v_gemm_args_t* a) {
+static int gemm_big_rows(const p3v_gemm_args_t* a, float* cost = nullptr) {
+  if (cost) *cost = 1e30f;
   const int n_big = P3V_GATED(a->epilogue) ? 128 : 256, n_small = n_big / 2;
   if (a->M < 1024 || a->N % n_big || a->epilogue == P3V_EPI_PATCH) return 0;
   if (const int force = p3v_tuning().gemm_big_rows; force >= 0) return min(force / 256 * 256, a->M);   // tests: pin the split
@@ -346,6 +347,7 @@ static int gemm_big_rows(const p3v_gemm_args_t* a) {
     if (big && small) c += 0.04f;                       // the second launch
     if (c < best - 1e-4f) { best = c; best_rows = rows_big; }
   }
+  if (cost) *cost = best;
   return best_rows;
 }
 
@@ -725,6 +727,43 @@ int p3v_gemm256_qkv(const p3v_gemm_args_t* a, const QkvP& q, hipStream_t s);   /
 int p3v_gemm_skinny_qkv(const p3v_gemm_args_t* a, const QkvP& q, hipStream_t s);   // p3v_gemm_skinny.hip
 
 int p3v_gemm_skinny_qkv_merge(const p3v_gemm_args_t* a, const QkvP& q, void* ws, int64_t ws_bytes, hipStream_t s);   // p3v_gemm_skinny.hip
+int p3v_qkv_flat_tiles(const QkvP& q, int M, int mb);                                        // p3v_gemm_pc.hip
+int p3v_gemm256_flat_qkv(const p3v_gemm_args_t* a, const QkvP& q, int mb, hipStream_t s);      // p3v_gemm256.hip
+
+// The qkv projection on the flat tiles of p3v_gemm_pc.hip: 32 mb rows a tile, or 0.
+// Below 1024 rows the alternative is p3v_gemm and the split as a launch of its own: the same tile saves that launch for 4 us of epilogue (900 x
+// 9216 x 3072 59.0 -> 55.2 us, 768 55.9 -> 52.7), as long as one round of the chip takes the tiles, of which there are more (a V tile's rows are
+// dimensions, its columns 256 tokens).  From 1024 rows on it is the packing of 256 x 256 and 128 x 128 tiles below, of which the first leave a
+// round half empty here and there: 1024 rows 83.0 -> 57.7, 2048 124 -> 103, 1800 118 -> 101; 2885 x 3072 x 1024 (five image crops) 36.1 -> 30.0,
+// 7501 70.5 -> 65.7; it stays the faster for 1100 .. 1500 (82 - 85) and 2531 rows (135, here 136) and for 17 crops (80, here 81).
+// Times fitted to 25 sizes of either: a tile's constant and time per K-tile, 0.6 of the constant for every further round; the packing in its own
+// units of 8.5 + 1.57 K-tiles.  3 % have to be promised.
+static int qkv_flat_plan(const p3v_gemm_args_t* a, const QkvP& q) {
+  const int pin = p3v_tuning().gemm_qkv_flat;
+  if (!pin || a->M <= 256 || (q.nh * q.hd) % 256 || (q.nkv * q.hd) % 256) return 0;
+  if (pin > 0) return pin;
+  if (p3v_tuning().gemm_128 || p3v_tuning().gemm_big_rows >= 0) return 0;
+  p3v_gemm_args_t plain = *a;
+  if (a->M < 1024) {
+    int mb = 0, nb = 0;
+    if (splitk_slices(a->M, a->N, a->K, a->epilogue) > 1 || !gemm_tile_plan(&plain, 0, &mb, &nb) || nb != 4 || (mb != 4 && mb != 5)) return 0;
+    return p3v_qkv_flat_tiles(q, a->M, mb) <= 256 ? mb : 0;
+  }
+  plain.epilogue = P3V_EPI_NONE;
+  const float kt = (float)(a->K / BK);
+  static const struct { int mb; float f, c; } tiles[] = {{2, 2.2f, 0.89f}, {3, 8.2f, 0.78f}, {4, 11.2f, 0.866f}, {5, 16.f, 0.87f}};
+  float best;
+  gemm_big_rows(&plain, &best);
+  best = 0.97f * (3.f + best * (8.5f + 1.57f * kt));
+  int mb = 0;
+  for (const auto& t : tiles) {
+    const int rounds = p3v_cdiv(p3v_qkv_flat_tiles(q, a->M, t.mb), 256);
+    const float c = t.f * (1.f + 0.6f * (rounds - 1)) + rounds * t.c * kt;
+    if (c < best) best = c, mb = t.mb;
+  }
+  return mb;
+}
+
 static int gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* merge_ws, int64_t merge_bytes, void* stream) {
   if (!a || !sp || !a->A || !a->W || !sp->q_out || !sp->k_dst || !sp->v_dst || (!sp->cos_t) != (!sp->sin_t)) return P3V_ERR_ARG;
   if (a->epilogue != P3V_EPI_NONE && a->epilogue != P3V_EPI_BIAS) return P3V_ERR_ARG;
@@ -745,6 +784,10 @@ static int gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* m
   QkvP q = {sp->cos_t, sp->sin_t, sp->q_out, sp->k_dst, sp->v_dst, sp->L, nh, nkv, hd, sp->past, dpos0, sp->dst_t, sp->tab_t, sp->tab_div, 0,
             sp->q_scale};
   if (merge_ws) return p3v_gemm_skinny_qkv_merge(a, q, merge_ws, merge_bytes, s);
+  if (const int mb = qkv_flat_plan(a, q)) {
+    const int rc = p3v_gemm256_flat_qkv(a, q, mb, s);
+    if (rc != P3V_ERR_UNSUPPORTED) return rc;
+  }
   if (a->M < 1024) return p3v_gemm_skinny_qkv(a, q, s);       // 17 .. 256 rows: the weight-streaming kernel (or "unsupported")
   if ((nh * hd) % BN || (nkv * hd) % BN || p3v_tuning().gemm_128) return P3V_ERR_UNSUPPORTED;
   p3v_gemm_args_t plain = *a;

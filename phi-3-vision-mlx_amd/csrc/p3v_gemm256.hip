@@ -332,3 +332,11 @@ int p3v_gemm256_slices(const p3v_gemm_args_t* a, float* part, int S, int mb, int
   const Gemm256P p = {a->A, a->W, part, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, a->N, {}, S};
   return p3v_gemm_pc(p, P3V_EPI_PART, mb, nb, s);
 }
+
+// the qkv projection on flat tiles of 32 mb rows (qkv_flat_plan, p3v_gemm.hip)
+int p3v_gemm256_flat_qkv(const p3v_gemm_args_t* a, const QkvP& q, int mb, hipStream_t s) {
+  if (mb < 2 || mb > 5 || a->K % TK || (q.nh * q.hd) % 256 || (q.nkv * q.hd) % 256) return P3V_ERR_UNSUPPORTED;
+  if ((size_t)a->N * a->ldw * 2 >= ((size_t)1 << 32) || (size_t)a->M * a->lda * 2 >= ((size_t)1 << 32) || (size_t)256 * a->ldw * 2 >= ((size_t)1 << 31)) return P3V_ERR_UNSUPPORTED;
+  const Gemm256P p = {a->A, a->W, nullptr, a->bias, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0, q, 0};
+  return p3v_gemm_pc(p, P3V_EPI_QKV, mb, 4, s);
+}

@@ -10,14 +10,17 @@
 //            MFMAs; larger tiles do not fit the 168 registers that twelve waves leave each other.
 // 2531 x 3072 x 8192 (+ residual) 117 -> 105 us (1.21 PFLOP/s), 9809 x 1024 x 4096 (+ fp32 residual) 95 -> 73, 2048 x 9472 x 3072 114 -> 97.
 // Same K order and epilogue as the other tiles: bit-identical results.
+// P3V_EPI_QKV: split, rotation and KV append in the epilogue, tiles of 64 and 96 rows too (qkv_flat_plan, p3v_gemm.hip, has the rule and the
+// times; a K-tile of 64 x 256 takes as long as one of 128 x 256, waiting for its weights, but a short K gets through the chip sooner).
 // P3V_EPI_PART: the tiles of one slice of K after the other, fp32 partials (p3v_gemm_slices, p3v_gemm.hip, which has the rule and the times).
 // (Tried and left out: touching the lines of later K-tiles ahead of the DMA, one dword per line -- 64 lines cost the address path as
 //  much as four pieces: 105 -> 137 us; 4 consumers of twice the size without producers: 121 us.)
 #include "p3v_gemm256_epi.h"
 
 struct TilePc {                        // where the requests of an output tile's K-tiles come from
-  int a_off[8], b_off[8]; __amdgpu_buffer_rsrc_t rs_a;
+  int a_off[8], b_off[8]; __amdgpu_buffer_rsrc_t rs_a, rs_b;
 };
+struct PlacePc { int m0, n0, z, swapped, is_k, row0; };           // z: slice of K; the others P3V_EPI_QKV: V tile (operand roles swapped) / K region / first W row of the region
 
 #define GPC_BUF(mb, nb) ((32 * (mb) + 64 * (nb)) * TK * 2)
 #define GPC_STAGES(mb, nb) (160 * 1024 / GPC_BUF(mb, nb) < 4 ? 160 * 1024 / GPC_BUF(mb, nb) : 4)
@@ -33,29 +36,45 @@ __global__ void __launch_bounds__(768, 1) k_gemm_pc(Gemm256P p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform: LDS-DMA bases stay in SGPRs
   constexpr int n_out_tile = SILU ? TN / 2 : TN;
-  constexpr bool PART = EPI == P3V_EPI_PART;
-  const int gx = (p.N + n_out_tile - 1) / n_out_tile, gy = (p.M + TM - 1) / TM, nwg = PART ? gx * gy * p.slices : gx * gy;
+  constexpr bool PART = EPI == P3V_EPI_PART, QKV = EPI == P3V_EPI_QKV;
+  static_assert(!QKV || NB == 4, "both halves of 32 rotation pairs in a wave");
+  // (QKV: column tiles 0 .. nq - 1 are Q, the others K; behind them the V tiles, TM rows of W_v by TN tokens -- p3v_gemm_qkv.h)
+  const int nq = QKV ? p.q.nh * p.q.hd / TN : 0, v_rows = QKV ? p.q.nkv * p.q.hd : 0, vx = QKV ? (p.M + TN - 1) / TN : 0;
+  const int gx = QKV ? nq + v_rows / TN : (p.N + n_out_tile - 1) / n_out_tile, gy = (p.M + TM - 1) / TM;
+  const int nwg = QKV ? gx * gy + vx * ((v_rows + TM - 1) / TM) : PART ? gx * gy * p.slices : gx * gy;
   const int nk = p.K / TK;
 
   // ---- PERSISTENT over output tiles: workgroup b takes tiles b, b + G, b + 2G, ... (G = gridDim.x, a multiple of 8, so a
   // workgroup's tiles keep its XCD in the XCD-aware order below), one stream of K-tiles across all of them.
   // PART: the slices one after the other, so an XCD keeps to one slice of K or two: A and W pass each L2 once, whatever the tile order.
-  auto place = [&](int wid, int& m0, int& n0, int& z) {
+  auto place = [&](int wid) {
     const int q = nwg >> 3, r = nwg & 7, xcd = wid & 7, loc = wid >> 3;
     int id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + loc;
-    z = 0;
-    if (PART) z = id / (gx * gy), id -= z * (gx * gy);
+    PlacePc t = {0, 0, 0, 0, 0, 0};
+    if (PART) t.z = id / (gx * gy), id -= t.z * (gx * gy);
+    if (QKV && id >= gx * gy) {
+      id -= gx * gy;
+      t.swapped = 1, t.row0 = (p.q.nh + p.q.nkv) * p.q.hd, t.m0 = id % vx * TN, t.n0 = id / vx * TM;
+      return t;
+    }
     constexpr int BAND = 4;
     const int band = id / (BAND * gx), in_band = id % (BAND * gx);
     const int rows = min(BAND, gy - band * BAND);
-    m0 = (band * BAND + in_band % rows) * TM, n0 = in_band / rows * n_out_tile;
+    int x = in_band / rows;
+    t.m0 = (band * BAND + in_band % rows) * TM;
+    if (QKV && x >= nq) t.is_k = 1, t.row0 = p.q.nh * p.q.hd, x -= nq;
+    t.n0 = x * n_out_tile;                                        // (QKV: first column INSIDE the region)
+    return t;
   };
   auto k_begin = [&](int z) { return PART ? z * nk / p.slices : 0; };
   auto k_end = [&](int z) { return PART ? (z + 1) * nk / p.slices : nk; };
   if ((int)blockIdx.x >= nwg) return;
   int total = 0;                                                  // K-tiles of this workgroup
   if (PART) {
-    for (int wid = blockIdx.x, m0, n0, z; wid < nwg; wid += gridDim.x) place(wid, m0, n0, z), total += k_end(z) - k_begin(z);
+    for (int wid = blockIdx.x; wid < nwg; wid += gridDim.x) {
+      const int z = place(wid).z;
+      total += k_end(z) - k_begin(z);
+    }
   } else {
     total = ((nwg - 1 - (int)blockIdx.x) / (int)gridDim.x + 1) * nk;
   }
@@ -64,26 +83,32 @@ __global__ void __launch_bounds__(768, 1) k_gemm_pc(Gemm256P p) {
     // ---- PRODUCERS.  A request = 8 tile rows x 128 B (1 KiB) by LDS-DMA; the 16-byte chunks of a row are swizzled on the source side.
     // Buffer addressing (SGPR descriptor + 32-bit per-lane byte offset + SGPR K offset): no vector ALU work at all.
     const int pw = wave - 8, srow = pw * 8 + (lane >> 3), sw = ((lane & 7) ^ (lane >> 3)) * 8;
-    const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, 0xffffffff, 0x00020000);
     int dk = 0, dk_end = nk;                                      // the K-tiles still to be requested for the tile in hand
     TilePc dt;   // (declared outside the template: a builtin called with a member of a DEPENDENT type is only checked at
-                  //  instantiation, fails there in the HOST pass -- no such builtin -- and hipcc silently drops the host stub)
+                 //  instantiation, fails there in the HOST pass -- no such builtin -- and hipcc silently drops the host stub)
     auto aim = [&](int wid) {
-      int m0, n0, z;
-      place(wid, m0, n0, z);
-      dk = k_begin(z), dk_end = k_end(z);
+      const PlacePc t = place(wid);
+      const int m0 = t.m0, n0 = t.n0;
+      dk = k_begin(t.z), dk_end = k_end(t.z);
+      const bool v = QKV && t.swapped;                            // V tile: W rows fill the A side, tokens the B side
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const int rr = q * 32 + srow;
         int br = n0 + rr;
         if (SILU)                                     // a group of 64 tile columns = 32 gate rows + the 32 up rows of the same outputs
           br = min(n0 + (rr >> 6) * 32 + ((rr >> 4) & 1) * 16 + (rr & 15), p.N - 1) + ((rr & 63) >> 5) * p.N;
+        else if (QKV)                                 // pair order (both halves of a rotation pair in one lane)
+          br = v ? min(m0 + rr, p.M - 1) : qkv_pair_row(p.q, t.row0, n0 >> 1, rr);
         else
           br = min(br, p.N - 1);
-        dt.a_off[q] = ((min(m0 + rr, p.M - 1) - m0) * p.lda + sw) * 2;
-        dt.b_off[q] = (int)(((unsigned)br * (unsigned)p.ldw + (unsigned)sw) * 2u);   // < 2^32: checked by the launcher
+        const int ar = v ? min(n0 + rr, v_rows - 1) - n0 : min(m0 + rr, p.M - 1) - m0;
+        dt.a_off[q] = (ar * (v ? p.ldw : p.lda) + sw) * 2;
+        dt.b_off[q] = (int)(((unsigned)br * (unsigned)(v ? p.lda : p.ldw) + (unsigned)sw) * 2u);   // < 2^32: checked by the launcher
       }
-      dt.rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + (size_t)m0 * p.lda), 0, 0xffffffff, 0x00020000);
+      const bf16_t* pa = v ? p.W + (size_t)(t.row0 + n0) * p.ldw : p.A + (size_t)m0 * p.lda;
+      const bf16_t* pb = v ? p.A : p.W;
+      dt.rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)pa, 0, 0xffffffff, 0x00020000);
+      dt.rs_b = __builtin_amdgcn_make_buffer_rsrc((void*)pb, 0, 0xffffffff, 0x00020000);
     };
     int dwid = blockIdx.x, slot = 0;                              // the tile in hand, and the next K-tile's buffer
     aim(dwid);
@@ -103,7 +128,7 @@ __global__ void __launch_bounds__(768, 1) k_gemm_pc(Gemm256P p) {
         if (q < nb) {
           lptr_t dst = (lptr_t)(base + a_bytes + q * 4096);
           const int vo = dt.b_off[q];
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, dst, 16, vo, dk * (TK * 2), 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(dt.rs_b, dst, 16, vo, dk * (TK * 2), 0, 0);
         }
       }
       slot = slot == S - 1 ? 0 : slot + 1;
@@ -156,9 +181,8 @@ __global__ void __launch_bounds__(768, 1) k_gemm_pc(Gemm256P p) {
   int slot = 0;                                                   // LDS buffer of the K-tile in hand
   __builtin_amdgcn_s_barrier();
   for (int wid = blockIdx.x; wid < nwg; wid += gridDim.x) {
-    int m0, n0, z;
-    place(wid, m0, n0, z);
-    const int nkt = k_end(z) - k_begin(z);
+    const PlacePc t = place(wid);
+    const int m0 = t.m0, n0 = t.n0, nkt = k_end(t.z) - k_begin(t.z);
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -178,8 +202,11 @@ __global__ void __launch_bounds__(768, 1) k_gemm_pc(Gemm256P p) {
     }
     if constexpr (PART) {
       Gemm256P part = p;
-      part.out = (float*)p.out + (size_t)z * p.M * p.ldo;
+      part.out = (float*)p.out + (size_t)t.z * p.M * p.ldo;
       gemm256_epilogue<P3V_EPI_F32, MB, NB>(part, acc, m0 + wr * MB * 16, n0 + wc * (n_out_tile / 4), lane);
+    } else if constexpr (QKV) {
+      if (!t.swapped) qkv_epilogue_rot<MB, 2>(p.q, acc, p.bias, t.is_k, t.row0, (n0 >> 1) + wc * 32, m0 + wr * MB * 16, p.M, lane);
+      else qkv_epilogue_vt<MB>(p.q, acc, p.bias ? p.bias + t.row0 : nullptr, n0 + wr * MB * 16, m0 + wc * 64, p.M, lane, v_rows);
     } else {
       gemm256_epilogue<EPI, MB, NB>(p, acc, m0 + wr * MB * 16, n0 + wc * (n_out_tile / 4), lane);  // straight from the accumulators: p3v_gemm256_epi.h
     }
@@ -187,6 +214,8 @@ __global__ void __launch_bounds__(768, 1) k_gemm_pc(Gemm256P p) {
 }
 
 int p3v_gemm256_cus();                                             // p3v_gemm256.hip
+
+int p3v_qkv_flat_tiles(const QkvP& q, int M, int mb);
 
 template <int EPI, int MB, int NB>
 static int launch_pc_v(const Gemm256P& p, hipStream_t s) {
@@ -198,16 +227,26 @@ static int launch_pc_v(const Gemm256P& p, hipStream_t s) {
   }
   const int n_cu = p3v_gemm256_cus();
   if (!n_cu) return P3V_ERR_HIP;
-  const int tiles = p3v_cdiv(p.N, P3V_GATED(EPI) ? 32 * NB : 64 * NB) * p3v_cdiv(p.M, 32 * MB) * (EPI == P3V_EPI_PART ? p.slices : 1);
+  int tiles = p3v_cdiv(p.N, P3V_GATED(EPI) ? 32 * NB : 64 * NB) * p3v_cdiv(p.M, 32 * MB) * (EPI == P3V_EPI_PART ? p.slices : 1);
+  if (EPI == P3V_EPI_QKV) tiles = p3v_qkv_flat_tiles(p.q, p.M, MB);
   hipLaunchKernelGGL((k_gemm_pc<EPI, MB, NB>), dim3(min(tiles, n_cu)), dim3(768), LDS, s, p);
   P3V_CHECK_LAUNCH();
   return P3V_OK;
 }
 
+// output tiles of the qkv projection on tiles of 32 mb rows x 256 columns
+int p3v_qkv_flat_tiles(const QkvP& q, int M, int mb) {
+  return (q.nh + q.nkv) * q.hd / 256 * p3v_cdiv(M, 32 * mb) + p3v_cdiv(q.nkv * q.hd, 32 * mb) * p3v_cdiv(M, 256);
+}
+
 template <int EPI>
 static int launch_pc(const Gemm256P& p, int mb, int nb, hipStream_t s) {
-  if constexpr (!P3V_GATED(EPI))
+  if constexpr (!P3V_GATED(EPI) && EPI != P3V_EPI_QKV)
     if (nb == 3) return launch_pc_v<EPI, 4, 3>(p, s);
+  if constexpr (EPI == P3V_EPI_QKV) {
+    if (mb == 2) return launch_pc_v<EPI, 2, 4>(p, s);
+    if (mb == 3) return launch_pc_v<EPI, 3, 4>(p, s);
+  }
   return mb == 4 ? launch_pc_v<EPI, 4, 4>(p, s) : launch_pc_v<EPI, 5, 4>(p, s);
 }
 
@@ -223,6 +262,7 @@ int p3v_gemm_pc(const Gemm256P& p, int epi, int mb, int nb, hipStream_t s) {
     case P3V_EPI_GELU_MUL: return launch_pc<P3V_EPI_GELU_MUL>(p, mb, nb, s);
     case P3V_EPI_F32: return launch_pc<P3V_EPI_F32>(p, mb, nb, s);
     case P3V_EPI_SCALE_RESID_F32: return launch_pc<P3V_EPI_SCALE_RESID_F32>(p, mb, nb, s);
+    case P3V_EPI_QKV: return launch_pc<P3V_EPI_QKV>(p, mb, nb, s);
     case P3V_EPI_PART: return launch_pc<P3V_EPI_PART>(p, mb, nb, s);
     default: return P3V_ERR_UNSUPPORTED;
   }

@@ -36,7 +36,8 @@ __device__ __forceinline__ int qkv_pair_row(const QkvP& q, int row0, int p0, int
 }
 
 // Q / K tile: acc[i][j] = block row i (16 tokens from m_first), blocks 0, 1 = first halves of pairs pw .. pw + 31, blocks 2, 3 = second
-template <int NI>
+// (G block rows' rotation tables at a time)
+template <int NI, int G = (NI < 4 ? NI : 4)>
 __device__ __forceinline__ void qkv_epilogue_rot(const QkvP& q, f32x4_t (&acc)[NI][4], const bf16_t* bias, bool is_k, int row0, int pw,
                                                  int m_first, int M, int lane) {
   const int fc = lane & 15, fq = lane >> 4, half = q.hd >> 1;
@@ -64,8 +65,8 @@ __device__ __forceinline__ void qkv_epilogue_rot(const QkvP& q, f32x4_t (&acc)[N
   int b0 = 0, l0 = q.m_base + (m00 < M ? m00 : M - 1);
   if (l0 >= q.L) { b0 = l0 / q.L; l0 -= b0 * q.L; }
   // The rotation tables cost 4 sixteen-byte loads per block row: requested FOUR BLOCK ROWS AT A TIME (64 registers; the fragment
-  // registers of the K loop are free here), so a tile pays two round trips to the L2 instead of eight dependent ones.
-  constexpr int G = NI < 4 ? NI : 4;
+  // registers of the K loop are free here), so a tile pays two round trips to the L2 instead of eight dependent ones.  (Two at a time
+  // in the kernel of twelve waves, which has 168 registers.)
 #pragma unroll
   for (int ig = 0; ig < NI; ig += G) {
     float4 cs4[G][2], sn4[G][2];
@@ -73,6 +74,7 @@ __device__ __forceinline__ void qkv_epilogue_rot(const QkvP& q, f32x4_t (&acc)[N
 #pragma unroll
     for (int ii = 0; ii < G; ++ii) {
       const int i = ig + ii;
+      if (i >= NI) continue;
       int l = l0 + i * 16, b = b0;
       const int m = m00 + i * 16;
       if (m >= M) l = l0 + (M - 1 - (m00 < M ? m00 : M - 1));   // clamped rows: any valid table row (nothing is stored for them)
@@ -86,7 +88,9 @@ __device__ __forceinline__ void qkv_epilogue_rot(const QkvP& q, f32x4_t (&acc)[N
     }
 #pragma unroll
     for (int ii = 0; ii < G; ++ii) {
-      const int i = ig + ii, m = m00 + i * 16, b = bb[ii], l = ll[ii];
+      const int i = ig + ii;
+      if (i >= NI) continue;
+      const int m = m00 + i * 16, b = bb[ii], l = ll[ii];
       uint32_t pk1[2][2], pk2[2][2];
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
@@ -124,15 +128,15 @@ __device__ __forceinline__ void qkv_epilogue_rot(const QkvP& q, f32x4_t (&acc)[N
 }
 
 // V tile (operand roles swapped): acc[i][j] = block row i of 16 V dimensions from fv_first (index into [nkv * hd]), block column j of
-// 16 tokens from t_first.  bias_v = bias + first W row of the V region, or null.
+// 16 tokens from t_first.  bias_v = bias + first W row of the V region, or null.  fv_end: dimensions from there on are not stored.
 template <int NI>
 __device__ __forceinline__ void qkv_epilogue_vt(const QkvP& q, f32x4_t (&acc)[NI][4], const bf16_t* bias_v, int fv_first, int t_first,
-                                                int M, int lane) {
+                                                int M, int lane, int fv_end = 0x7fffffff) {
   const int fc = lane & 15, fq = lane >> 4;
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int fv = fv_first + i * 16 + fc, head = fv / q.hd, d = fv - head * q.hd;
-    const float bv = bias_v ? bf16_to_f32(bias_v[fv]) : 0.f;
+    const float bv = bias_v && fv < fv_end ? bf16_to_f32(bias_v[fv]) : 0.f;
 #pragma unroll
     for (int jp = 0; jp < 2; ++jp) {
       uint32_t pk[2][2];
@@ -148,7 +152,7 @@ __device__ __forceinline__ void qkv_epilogue_vt(const QkvP& q, f32x4_t (&acc)[NI
         w[k] = sw[0], w[2 + k] = sw[1];
       }
       const int t = t_first + (2 * jp + (fq & 1)) * 16 + (fq >> 1) * 8;      // 8 consecutive tokens t .. t + 7
-      if (t < M) {
+      if (t < M && fv < fv_end) {
         const int mg = q.m_base + t, b = mg < q.L ? 0 : mg / q.L, l = mg - b * q.L;
         bf16_t* dst = q.v_dst + (((size_t)b * q.nkv + head) * q.hd + d) * (size_t)q.dst_t + q.dpos0 + l;
         if (t + 8 <= M && l + 8 <= q.L) {                      // the run lies in one batch row

@@ -517,7 +517,7 @@ class Phi3VModel(DecoderModel):
             fused_qkv = False
             k_w = p + "self_attn.qkv_proj.weight"
             if (L > ops.L.DECODE_MAX_L and n_beam == 1 and k_w in w and k_w not in self.adapters and not mlx4_first
-                    and (M >= 1024 or M <= 256) and os.environ.get("P3V_QKV_FUSE", "1") != "0"):
+                    and os.environ.get("P3V_QKV_FUSE", "1") != "0"):
                 kd, vd = (st.k_tmp, st.v_tmp) if st.quantized else (st.k[i], st.v[i])
                 if not (st.quantized and past > 0 and not getattr(st, "fresh_rows", False)):
                     hn = h if normed_in else ops.rmsnorm(x, w[p + "input_layernorm.weight"], eps, out=h)

@@ -1086,6 +1086,49 @@ def test_gemm_qkv_fp8_fused(ops, B, L, nh, nkv, hd, K, past, rot):
     assert torch.equal(k2, k1) and torch.equal(v2, v1)
 
 
+@pytest.mark.parametrize("mb", [2, 3, 4, 5])
+@pytest.mark.parametrize("B,L,nh,nkv,hd,K,past,rot,bias", [(1, 257, 8, 8, 96, 192, 0, True, False), (1, 641, 16, 8, 96, 64, 64, True, False), (3, 100, 16, 4, 64, 320, 0, True, False),
+                                                           (2, 577, 16, 16, 64, 256, 0, False, True), (1, 1100, 32, 32, 96, 128, 8, True, False), (40, 7, 8, 8, 96, 448, 8, True, False)])
+def test_gemm_qkv_flat_tiles(ops, B, L, nh, nkv, hd, K, past, rot, bias, mb):
+    """p3v_gemm_qkv on every flat tile (ragged last rows, V regions that end inside a tile, several rounds of the chip, batch rows that start
+    anywhere in a tile) against p3v_gemm, then p3v_rope_kv_append: the same bits, the rest of the caches untouched."""
+    M, N = B * L, (nh + 2 * nkv) * hd
+    a, w, bq = g((M, K), 420).cuda(), g((N, K), 421, 1.0 / math.sqrt(K)).cuda(), g((N,), 422, 0.5).cuda() if bias else None
+    T = past + L + 5
+    Tp = (T + 127) // 128 * 128
+    cos, sin = (torch.rand((B, T, hd // 2), device="cuda") for _ in range(2)) if rot else (None, None)
+    k0, v0 = g((B, nkv, Tp, hd), 423).cuda(), g((B, nkv, hd, Tp), 424).cuda()
+    outs = [(torch.full((B, nh, L, hd), 7.0, dtype=BF16, device="cuda"), k0.clone(), v0.clone()) for _ in range(2)]
+    saved = ops.set_tuning("gemm_qkv_flat", mb), ops.set_tuning("gemm_no_splitk", 1)
+    try:
+        qkv = ops.gemm(a, w, ops.EPI_BIAS, bias=bq) if bias else ops.gemm(a, w)
+        ops.rope_kv_append(qkv, cos, sin, *outs[0], B, L, nh, nkv, hd, past, Tp, True, T, 1, q_scale=1.3)
+        assert ops.gemm_qkv(a, w, cos, sin, *outs[1], B, L, nh, nkv, hd, past, Tp, True, T, 1, q_scale=1.3, bias=bq)
+    finally:
+        ops.set_tuning("gemm_qkv_flat", saved[0]), ops.set_tuning("gemm_no_splitk", saved[1])
+    for x, y, name in zip(*outs, ("Q", "K cache", "V cache")):
+        assert torch.equal(x, y), f"{name}: {(x != y).sum().item()} elements differ"
+
+
+@pytest.mark.parametrize("M,taken", [(768, True), (900, True), (1023, True), (2048, True), (300, False), (512, False)])
+def test_gemm_qkv_flat_tiles_where_planned(ops, M, taken):
+    """The launcher's own choice at the decoder's widths: below 1024 rows only where one round of the chip takes the tiles."""
+    nh, hd, K = 32, 96, 3072
+    a, w = g((M, K), 425).cuda(), g((3 * nh * hd, K), 426, 1.0 / math.sqrt(K)).cuda()
+    T, Tp = M + 5, (M + 5 + 127) // 128 * 128
+    cos, sin = torch.rand((1, T, hd // 2), device="cuda"), torch.rand((1, T, hd // 2), device="cuda")
+    outs = [tuple(torch.zeros(s, dtype=BF16, device="cuda") for s in ((1, nh, M, hd), (1, nh, Tp, hd), (1, nh, hd, Tp))) for _ in range(2)]
+    saved = ops.set_tuning("gemm_big_rows", -1), ops.set_tuning("gemm_128", 0)
+    try:
+        assert ops.gemm_qkv(a, w, cos, sin, *outs[0], 1, M, nh, nh, hd, 0, Tp, True, T, 1) == taken
+        if taken:
+            ops.rope_kv_append(ops.gemm(a, w), cos, sin, *outs[1], 1, M, nh, nh, hd, 0, Tp, True, T, 1)
+    finally:
+        ops.set_tuning("gemm_big_rows", saved[0]), ops.set_tuning("gemm_128", saved[1])
+    for x, y, name in zip(*outs, ("Q", "K cache", "V cache")):
+        assert torch.equal(x, y), f"{name}: {(x != y).sum().item()} elements differ"
+
+
 def test_gemm_qkv_declines_what_it_cannot_fuse(ops):
     """Decode-sized inputs (<= 8 rows) and unaligned append offsets: P3V_ERR_UNSUPPORTED, nothing written."""
     nh, hd, K = 16, 64, 128
