@@ -162,7 +162,9 @@ __device__ __forceinline__ void gla_span(const GlaP& p, int b, int l0, int& lo, 
 __host__ __device__ __forceinline__ int gla_dim16(int n) { return (n + 15) / 16 * 16; }
 __host__ __device__ __forceinline__ int gla_stride(int n) { return gla_dim16(n) + 4; }
 #define GLA_TS (GLA_C + 4)
-__host__ __device__ __forceinline__ int gla_key_rows(int dim) { return max(gla_dim16(dim), 32); }     // (also the scratch of gla_decays)
+#define GLA_A1 (GLA_C * 20 * 4)      // bytes of gla_decays' scratch
+// k_gla_chunk's first LDS block: the running sums, then, in their place, the keys
+__host__ __device__ __forceinline__ int gla_chunk_rows(int dim) { return max(GLA_C * gla_stride(dim), gla_dim16(dim) * GLA_TS); }
 // workspace: states [chunk, B, H, dim, vdim], decays of whole chunks [chunk, B, H, dim], running sums [B L, H, dim]
 __host__ __device__ __forceinline__ size_t gla_decay_at(const GlaP& p, int nc) { return (size_t)nc * p.B * p.H * p.dim * p.vdim; }
 __host__ __device__ __forceinline__ size_t gla_sums_at(const GlaP& p, int nc) { return gla_decay_at(p, nc) + (size_t)nc * p.B * p.H * p.dim; }
@@ -264,14 +266,17 @@ template <typename T, int NC> struct GlaRows {
 // The fp32 MFMA takes one k per lane group; four of them in a row are given k = 4 group + 0 .. 3 of a run of 16, so that an operand's four
 // values are one LDS read.
 // NK, NV: 64-channel groups of a key, of a value
+// A workgroup is a chain of latencies (rows in, running sums, products, states out), so what counts is how many share a CU: the keys take
+// the place of the running sums in LDS (48 -> 30 KB at 64 x 96 channels), and the 1024 workgroups of 2048 tokens x 32 heads are resident at
+// once instead of in two rounds: 40 -> 34 us.
 template <typename T, int NK, int NV>
 __global__ void __launch_bounds__(256) k_gla_chunk(GlaP p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int ch = blockIdx.x, h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, lane = tid & 63, lc = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int dim = p.dim, vdim = p.vdim, DS = gla_stride(dim), l0 = ch * GLA_C;
-  float *cum = (float*)smem, *kd = cum + GLA_C * DS;                     // [64][DS], [dim16][TS]
-  T* vt = (T*)(kd + gla_key_rows(dim) * GLA_TS);                           // [vdim16][TS]
+  float *cum = (float*)smem, *kd = cum;                                  // [64][DS], then [dim16][TS]
+  T* vt = (T*)(cum + gla_chunk_rows(dim));                                 // [vdim16][TS]; gla_decays' scratch before
   int lo, hi;
   gla_span(p, b, l0, lo, hi);
   const T* base = (const T*)p.y + ((size_t)b * p.L + l0) * p.ld;
@@ -279,32 +284,42 @@ __global__ void __launch_bounds__(256) k_gla_chunk(GlaP p) {
   GlaRows<T, NV> vx;
   vx.load(base + 2 * p.H * dim + h * vdim, p.ld, vdim, lo, hi, tid);
   kx.load(base + (p.H + h) * dim, p.ld, dim, lo, hi, tid);
-  gla_decays<T>(p, b, h, l0, lo, hi, cum, DS, kd);
+  gla_decays<T>(p, b, h, l0, lo, hi, cum, DS, (float*)vt);
   vx.put_transposed(vt, vdim, tid);
   const size_t row = (size_t)ch * p.B * p.H + (size_t)b * p.H + h;
   float* decay = p.ws + gla_decay_at(p, gridDim.x) + row * dim;
   float* sums = p.ws + gla_sums_at(p, gridDim.x) + ((size_t)b * p.L + l0) * p.H * dim + h * dim;
   const int t8 = tid & 31, c8 = (tid >> 5) * 8;
+  float end[NK][8], c[NK][2][8];
 #pragma unroll
   for (int n = 0; n < NK; ++n) {
     const int c0 = n * 64 + c8;
-    if (c0 >= gla_dim16(dim)) continue;
-    float end[8] = {};
-    if (c0 < dim) load_acts<8>(cum + (GLA_C - 1) * DS + c0, end);
-    if (t8 == 0 && c0 < dim)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) decay[c0 + j] = __builtin_amdgcn_exp2f(end[j]);
+    for (int j = 0; j < 8; ++j) end[n][j] = c[n][0][j] = c[n][1][j] = 0.f;
+    if (c0 >= dim) continue;
+    load_acts<8>(cum + (GLA_C - 1) * DS + c0, end[n]);
+    if (t8 == 0)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) decay[c0 + j] = __builtin_amdgcn_exp2f(end[n][j]);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int t = t8 + 32 * i;
-      float c[8] = {};
-      if (c0 < dim) load_acts<8>(cum + t * DS + c0, c);
-      if (l0 + t < p.L && c0 < dim) store_acts<8>(sums + (size_t)t * p.H * dim + c0, c);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) kd[(c0 + j) * GLA_TS + t] = kx.get(n, i, j) * __builtin_amdgcn_exp2f(fminf(end[j] - c[j], 0.f));
+      load_acts<8>(cum + t * DS + c0, c[n][i]);
+      if (l0 + t < p.L) store_acts<8>(sums + (size_t)t * p.H * dim + c0, c[n][i]);
     }
   }
-  __syncthreads();
+  lds_barrier();                                                         // the sums are in registers: the keys take their place
+#pragma unroll
+  for (int n = 0; n < NK; ++n) {
+    const int c0 = n * 64 + c8;
+    if (c0 < gla_dim16(dim))
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          kd[(c0 + j) * GLA_TS + t8 + 32 * i] = kx.get(n, i, j) * __builtin_amdgcn_exp2f(fminf(end[n][j] - c[n][i][j], 0.f));
+  }
+  lds_barrier();
   // A operand: row = key channel; B operand: column = value channel; a wave takes consecutive tiles, the keys of a row of them stay
   const int VT = (vdim + 15) / 16, tiles = (dim + 15) / 16 * VT, per = (tiles + 3) / 4;
   float* dst = p.ws + row * dim * vdim;
@@ -500,7 +515,7 @@ __global__ void __launch_bounds__(256, VT <= 8 ? 3 : 2) k_gla_out(GlaP p) {
 #define GLA_MAX_LDS (160 * 1024)
 static int gla_lds_out(int dim, int vdim, int e) { return GLA_C * gla_stride(dim) * (4 + e) + gla_dim16(vdim) * GLA_TS * e; }
 static int gla_lds_chunk(int dim, int vdim, int e) {
-  return GLA_C * gla_stride(dim) * 4 + gla_key_rows(dim) * GLA_TS * 4 + gla_dim16(vdim) * GLA_TS * e;
+  return gla_chunk_rows(dim) * 4 + max(gla_dim16(vdim) * GLA_TS * e, GLA_A1);
 }
 
 // chunks of a call (0: token by token)
