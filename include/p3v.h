@@ -304,10 +304,11 @@ typedef struct {
 int p3v_attention_decode(const p3v_attn_decode_args_t* args /* host */, void* stream);
 /* Does p3v_attention_decode take `o_proj_w` for this shape on this device (host query, no launch)?  0 = no; 1 = attention + o_proj +
  * residual in ONE launch (merge_in_launch = 1, the 128-key one-tile plan); 2 = merge_in_launch = 0: the launch that merges
- * the split-KV partials also carries the o_proj + residual (long contexts, 64-key plans) -- same arguments, same bits. */
+ * the split-KV partials also carries the o_proj + residual (long contexts, 64-key plans) -- same arguments, same bits.  Short caches need
+ * no partials and then no merge: one launch there too (the form follows from the shape alone, with o_proj_w or without). */
 int p3v_attention_decode_can_fuse_oproj(int B, int L, int n_heads, int hd, int n_split, int cache_t, int o_n, int merge_in_launch);
-/* 1: p3v_attention_decode (without o_proj_w) runs this shape as one workgroup per (row, head), without split partials (host query; the
- * rule is about time: the results of the two forms differ by rounding) */
+/* 1: p3v_attention_decode (without o_proj_w) runs this batch as one workgroup per (row, head), without split partials (host query; the
+ * rule is about time: the results of the two forms differ by rounding; B = L = 1 with merge_in_launch = 0 has a rule of its own) */
 int p3v_attention_decode_rows_fit(int B, int L, int n_heads, int n_kv, int cache_t);
 /* Which role workgroup `wg` of the fused launch's 1-D grid (n_heads * n_split workgroups) plays under placement `map` (the
  * attn_fo_map tuning knob: 2 = default, 1 = its first form): out[0] = key split, out[1] = head, out[2] / out[3] = its

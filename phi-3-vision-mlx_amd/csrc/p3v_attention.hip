@@ -2554,15 +2554,23 @@ __global__ void __launch_bounds__(64) k_attn_decode_stream(AttnDecP p) {
 // What bounds it: ~6 us that do not depend on the length (launch, the new rows, the first tiles' latency, the merge), then one CU's
 // share of the keys at 28-30 KB/us, 5.7 TB/s when all CUs have one.  Fragments loaded straight from the caches, 16 pieces of 64
 // bytes per instruction and no LDS at all, ran at the same rate; eight waves a pair 0.5-4 us slower.
-__global__ void __launch_bounds__(256, 2) k_attn_decode_rows(AttnDecP p) {
-  constexpr int NW = 4, HD = 96, TK = 32, NKS = 3, NDT = 6, CPR = 12, ROWB = HD * 2 + 16, LQ = P3V_DECODE_MAX_L;
-  __shared__ __attribute__((aligned(16))) unsigned char Qs[16 * ROWB], Kn[LQ * ROWB];      // rotated queries, rotated new keys
-  __shared__ __attribute__((aligned(16))) bf16_t Vn[LQ * HD];                              // new values
-  constexpr int KSTR = HD * 2 + 16, VSTR = TK * 2 + 16, TILE = TK * KSTR + HD * VSTR, PSTR = HD + 4;
-  __shared__ __attribute__((aligned(16))) unsigned char tiles[NW][TILE];                   // per wave: K rows, V^T rows; at the end O, m, l of its queries
+struct __attribute__((aligned(16))) RowsLds {
+  static constexpr int NW = 4, HD = 96, TK = 32, ROWB = HD * 2 + 16, LQ = P3V_DECODE_MAX_L;
+  static constexpr int KSTR = HD * 2 + 16, VSTR = TK * 2 + 16, TILE = TK * KSTR + HD * VSTR, PSTR = HD + 4;
+  unsigned char Qs[16 * ROWB], Kn[LQ * ROWB];                  // rotated queries, rotated new keys
+  bf16_t Vn[LQ * HD];                                          // new values
+  unsigned char tiles[NW][TILE];                               // per wave: K rows, V^T rows; at the end O, m, l of its queries
   static_assert(16 * PSTR * 4 <= TILE, "");
+};
+template <bool WT>                                             // WT: the output row goes out write-through, for consumers polling it in the same launch
+__device__ __forceinline__ void attn_rows_body(const AttnDecP& p, const int b, const int head, RowsLds& lds) {
+  constexpr int NW = RowsLds::NW, HD = RowsLds::HD, TK = RowsLds::TK, NKS = 3, NDT = 6, CPR = 12, ROWB = RowsLds::ROWB;
+  constexpr int KSTR = RowsLds::KSTR, VSTR = RowsLds::VSTR, PSTR = RowsLds::PSTR;
+  unsigned char *Qs = lds.Qs, *Kn = lds.Kn;
+  bf16_t* Vn = lds.Vn;
+  auto& tiles = lds.tiles;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, qi = lane & 15, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int b = blockIdx.y, head = blockIdx.x, kvh = (head * p.grp_magic) >> 16;
+  const int kvh = (head * p.grp_magic) >> 16;
   const bool kv_writer = head == kvh * p.grp;
   const float sc2 = p.scale * 1.4426950408889634f;            // softmax on exp2
   const int row_w = (p.nh + 2 * p.nkv) * HD;
@@ -2718,9 +2726,40 @@ __global__ void __launch_bounds__(256, 2) k_attn_decode_rows(AttnDecP p) {
       const float c = __builtin_amdgcn_exp2f(part(k)[HD] - Mu);
       a0 += c * part(k)[d], a1 += c * part(k)[d + 1], l += c * part(k)[HD + 1];
     }
-    *(uint32_t*)(p.out + ((size_t)b * p.L + q) * (p.nh * HD) + head * HD + d) = pack_bf16x2(l > 0.f ? a0 / l : 0.f, l > 0.f ? a1 / l : 0.f);
+    uint32_t* to = (uint32_t*)(p.out + ((size_t)b * p.L + q) * (p.nh * HD) + head * HD + d);
+    const uint32_t v = pack_bf16x2(l > 0.f ? a0 / l : 0.f, l > 0.f ? a1 / l : 0.f);
+    if (WT) __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *to = v;
   }
 }
+
+__global__ void __launch_bounds__(256, 2) k_attn_decode_rows(AttnDecP p) {
+  __shared__ RowsLds lds;
+  attn_rows_body<false>(p, blockIdx.y, blockIdx.x, lds);
+}
+
+// One row, one new token, a short cache (attn_row1_fit): workgroups 0 .. nh - 1 are k_attn_decode_rows, the others project the layer's
+// o_proj + residual as k_attn_combine_o's do: their rows of W_o are requested at once and wait in registers for the heads' words.  No split
+// partials, so one hand-over through memory where attention, merge launch and merge had two and a launch boundary.  224 workgroups,
+// all resident at once.  What bounds it: launch, new rows, hand-over and dot 6.5 us, then one CU's share of the keys at 28-30 KB/us (eight
+// waves a head instead of four: no faster).  4-bit / bf16 weights, 60 keys 9.84 / 9.78 -> 7.91 / 7.54 us, 130 keys 9.98 / 10.0 -> 9.24 / 9.39.
+template <int KIND>
+__global__ void __launch_bounds__(256) k_attn_rows_o(AttnDecP p, int n_units) {
+  __shared__ RowsLds lds;
+  static_assert(sizeof(lds.tiles) >= 7 * 1024 + 768, "the projection's share");
+  const int u = (int)blockIdx.x - p.nh;
+  if (u < 0) {
+    if (blockIdx.x == 0) {                                     // re-arm the other layer parity's buffer (nobody reads it in this launch)
+      uint32_t* ra = (uint32_t*)p.o_rearm;
+      for (int i = threadIdx.x; i < p.nh * 96 / 2; i += 256) ra[i] = 0xffffffffu;
+    }
+    attn_rows_body<true>(p, 0, blockIdx.x, lds);
+    return;
+  }
+  const int n_uw = (int)gridDim.x - p.nh;
+  fo_project<KIND, 2>(FoP{p.o_w, p.o_sb, p.o_x, p.out, p.nh}, u, lds.tiles[0], u + n_uw < n_units ? u + n_uw : -1);
+}
+
 
 // merge split-KV partials: one block of G = 4 or 8 64-lane groups per (b, head, query): thread (grp, d) loads
 // (m, l, o[d]) of its share of the splits (batches of 4 independent loads), reduces them against its own
@@ -2916,6 +2955,16 @@ static bool attn_rows_fit(int pairs, int grp, int L, int cache_t) {
   if (cache_t <= 128 || L > 1) return true;
   return grp > 1 ? 6 * idle <= pairs : cache_t > 192 || idle <= 128;
 }
+// One row with one new token on a short cache, where the merge is not pinned into the launch: one workgroup per head, no partials (with the
+// layer's o_proj beside them in k_attn_rows_o).  us with o_proj against splits + merge launch, 4-bit weights (bf16: +-0.2 of these), keys in a
+// cache of: 60 in 128 7.9 : 9.8, 130 in 192 9.4 : 10.1, 250 in 256 9.8 : 10.3, 300 in 320 10.8 : 10.6, 370 in 384 10.9 : 10.8, 500 in 512
+// 11.7 : 10.8; a capacity is half full on average, so up to 384 (250 in 384 9.9 : 10.8).  8 kv heads, whose keys the splits' neighbours find in the L2: 130 in 192 9.6 : 10.3, 130 in 256 9.5 : 9.7, 250 in 256 10.1 : 10.0
+// (bf16 10.5 : 10.0).
+static bool attn_row1_fit(int B, int L, int n_heads, int grp, int cache_t, int merge_in_launch) {
+  if (B != 1 || L != 1 || n_heads * 96 != 3072 || merge_in_launch) return false;
+  const int pin = p3v_tuning().attn_rows;
+  return pin >= 0 ? pin != 0 : cache_t <= (grp > 1 ? 192 : 384);
+}
 extern "C" int p3v_attention_decode_rows_fit(int B, int L, int n_heads, int n_kv, int cache_t) {
   if (B <= 0 || L <= 0 || n_heads <= 0 || n_kv <= 0 || n_heads % n_kv || cache_t <= 0) return 0;
   return attn_rows_fit(B * n_heads, n_heads / n_kv, L, cache_t);
@@ -2953,7 +3002,16 @@ extern "C" int p3v_attention_decode(const p3v_attn_decode_args_t* a, void* strea
     P3V_CHECK_LAUNCH();
     return P3V_OK;
   }
-  if (!a->o_proj_w && attn_rows_fit(a->B * a->n_heads, grp, a->L, a->cache_t)) {
+  const bool row1 = attn_row1_fit(a->B, a->L, a->n_heads, grp, a->cache_t, a->merge_in_launch);
+  if (fuse_form == 2 && row1) {                                // attention + o_proj + residual in one launch, without split partials
+    const int n_units = a->o_n / 8;
+    const dim3 grid_o(a->n_heads + (n_units + 1) / 2);
+    if (a->o_proj_sb) hipLaunchKernelGGL(k_attn_rows_o<FO_Q4>, grid_o, dim3(256), 0, s, p, n_units);
+    else hipLaunchKernelGGL(k_attn_rows_o<FO_BF16>, grid_o, dim3(256), 0, s, p, n_units);
+    P3V_CHECK_LAUNCH();
+    return P3V_OK;
+  }
+  if (!a->o_proj_w && (row1 || attn_rows_fit(a->B * a->n_heads, grp, a->L, a->cache_t))) {
     hipLaunchKernelGGL(k_attn_decode_rows, dim3(a->n_heads, a->B), dim3(256), 0, s, p);
     P3V_CHECK_LAUNCH();
     return P3V_OK;

@@ -865,6 +865,29 @@ def test_merge_launch_with_fused_oproj_under_grouped_queries(ops):
     test_merge_launch_with_fused_oproj_is_bit_identical_to_three_launches(ops, 300, 384, 3, False, True, nkv=8)
 
 
+@pytest.mark.parametrize("q4", [False, True], ids=["bf16", "q4"])
+@pytest.mark.parametrize("past,cap,nkv", [(0, 64, 32), (127, 128, 32), (128, 192, 8), (191, 256, 32), (383, 384, 32)])
+def test_short_cache_with_fused_oproj(ops, request, past, cap, nkv, q4):
+    """k_attn_rows_o: one workgroup per head and the o_proj beside them, at the edges of a round of its waves (128 keys) and of the cache.  The
+    same bits as k_attn_decode_rows and a GEMV; against the split form, whose maxima P is rounded against are others (2^-9) before the
+    output is (2^-9): a bound on values."""
+    test_merge_launch_with_fused_oproj_is_bit_identical_to_three_launches(ops, past, cap, cap // 64, False, q4, nkv=nkv)
+    nh, hd = 32, 96
+    qkv, kc, vc = g((1, (nh + 2 * nkv) * hd), 90).cuda(), g((1, nkv, cap, hd), 91), g((1, nkv, hd, cap), 92)
+    cos, sin = torch.rand((1, 1, hd // 2)).cuda(), torch.rand((1, 1, hd // 2)).cuda()
+    ws = ops.attention_ws(1, 1, nh, hd, cap // 64, "cuda")
+    old = ops.set_tuning("attn_rows", -1)
+    request.addfinalizer(lambda: ops.set_tuning("attn_rows", old))
+    res = []
+    for rows in (0, -1):
+        ops.set_tuning("attn_rows", rows)
+        k, v, out = kc.cuda(), vc.cuda(), torch.full((1, 1, nh * hd), float("nan"), dtype=BF16).cuda()
+        ops.attention_decode(qkv, cos, sin, 1, k, v, out, 1, 1, nh, nkv, hd, hd ** -0.5, past, cap, ws, cap // 64, merge_in_launch=False)
+        res.append((out, k, v))
+    assert torch.equal(res[0][1], res[1][1]) and torch.equal(res[0][2], res[1][2])
+    close(res[1][0], res[0][0], rtol=2 ** -8, atol=2 * 2 ** -9 * vc.float().abs().max().item())
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 768, 64), (129, 768, 128), (257, 3072, 1024), (1111, 768, 192), (4001, 3072, 128), (2300, 9216, 64)])
 @pytest.mark.parametrize("epi", ["none", "silu", "gelu", "resid_bf16", "resid_f32", "scale", "bias", "bias_qgelu", "bias_gelu", "f32"])
 def test_gemm_tiles_agree(ops, epi, M, N, K):
