@@ -118,6 +118,56 @@ __global__ void __launch_bounds__(256) k_dyt(DytP p, T* __restrict__ out, bool s
     prev = h;
   }
 }
+// The same, four channels a lane and the run's rows requested together (k_dyt: one element a lane and load, each row's behind the one before it):
+// 2048 x 3072 16.7 -> 9.3 us (38 MB, which a large copy moves in 8); with the shift 11.8 -> 10.9.
+template <typename T, bool SHIFT>
+__global__ void __launch_bounds__(256) k_dyt4(DytP p, T* __restrict__ out, bool store_hist) {
+  const int c = (blockIdx.x * 256 + threadIdx.x) * 4, b = SHIFT ? blockIdx.z : 0, l0 = blockIdx.y * DYT_ROWS;
+  if (c >= p.H) return;
+  const int rows = SHIFT ? p.L : p.B * p.L, l1 = min(rows, l0 + DYT_ROWS);      // (without a shift every row is for itself)
+  const float* x = p.x + (size_t)b * p.L * p.H + c;
+  T* o = out + (size_t)b * p.L * p.H + c;
+  float4 xv[DYT_ROWS];
+#pragma unroll
+  for (int j = 0; j < DYT_ROWS; ++j) xv[j] = *(const float4*)(x + (size_t)min(l0 + j, l1 - 1) * p.H);
+  const float4 before = SHIFT ? *(const float4*)(x + (size_t)max(l0 - 1, 0) * p.H) : make_float4(0.f, 0.f, 0.f, 0.f);
+  float w[4], bb[4], mu[4], prev[4] = {0.f, 0.f, 0.f, 0.f};
+  load4(p.w + c, w);
+  load4(p.b + c, bb);
+  auto act = [&](const float4& v, float (&h)[4]) {
+    h[0] = tanhf(v.x * p.alpha) * w[0] + bb[0], h[1] = tanhf(v.y * p.alpha) * w[1] + bb[1];
+    h[2] = tanhf(v.z * p.alpha) * w[2] + bb[2], h[3] = tanhf(v.w * p.alpha) * w[3] + bb[3];
+  };
+  int past = 0, first = 0;
+  if (SHIFT) {
+    load4(p.mu + c, mu);
+    past = p.d_past ? *p.d_past : p.past, first = p.pad_len ? p.pad_len[b] : 0;
+    if (past + l0 > first) {
+      if (l0 > 0) act(before, prev);
+      else load4(p.hist + ((size_t)b * p.R + (past - 1) % p.R) * p.H + c, prev);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < DYT_ROWS; ++j) {
+    const int l = l0 + j;
+    if (l >= l1) return;
+    float h[4];
+    act(xv[j], h);
+    if (SHIFT) {
+      float y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (past + l == first) prev[e] = 0.f;
+        y[e] = h[e] + (prev[e] - h[e]) * mu[e];
+        prev[e] = h[e];
+      }
+      store4(o + (size_t)l * p.H, y);
+      if (store_hist && l >= p.L - p.R) store4(p.hist + ((size_t)b * p.R + (past + l) % p.R) * p.H + c, h);
+    } else {
+      store4(o + (size_t)l * p.H, h);
+    }
+  }
+}
 // the history of a call so long that it wraps onto the slot its own first token reads: a launch of its own, behind k_dyt
 __global__ void __launch_bounds__(256) k_dyt_hist(DytP p) {
   const int c = blockIdx.x * 256 + threadIdx.x, b = blockIdx.z, l = p.L - 1 - blockIdx.y;
@@ -139,7 +189,14 @@ extern "C" int p3v_dyt(const p3v_dyt_args_t* a, void* out, int out_f32, void* st
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid(p3v_cdiv(p.H, 256), p3v_cdiv(p.L, DYT_ROWS), p.B);
   const bool late = p.mu && p.L >= p.R;
-  if (out_f32) hipLaunchKernelGGL(k_dyt<float>, grid, dim3(256), 0, s, p, (float*)out, !late);
+  const bool wide = p.H % 4 == 0 && !(((uintptr_t)p.x | (uintptr_t)p.hist | (uintptr_t)out) & 15) && !(((uintptr_t)p.w | (uintptr_t)p.b | (uintptr_t)p.mu) & 7);
+  const dim3 grid4(p3v_cdiv(p.H, 1024), p3v_cdiv(p.mu ? p.L : p.B * p.L, DYT_ROWS), p.mu ? p.B : 1);
+  if (wide && grid4.y <= 65535 && (long)p.B * p.L < 0x7fffffff) {
+    if (p.mu && out_f32) hipLaunchKernelGGL((k_dyt4<float, true>), grid4, dim3(256), 0, s, p, (float*)out, !late);
+    else if (p.mu) hipLaunchKernelGGL((k_dyt4<bf16_t, true>), grid4, dim3(256), 0, s, p, (bf16_t*)out, !late);
+    else if (out_f32) hipLaunchKernelGGL((k_dyt4<float, false>), grid4, dim3(256), 0, s, p, (float*)out, false);
+    else hipLaunchKernelGGL((k_dyt4<bf16_t, false>), grid4, dim3(256), 0, s, p, (bf16_t*)out, false);
+  } else if (out_f32) hipLaunchKernelGGL(k_dyt<float>, grid, dim3(256), 0, s, p, (float*)out, !late);
   else hipLaunchKernelGGL(k_dyt<bf16_t>, grid, dim3(256), 0, s, p, (bf16_t*)out, !late);
   if (late) hipLaunchKernelGGL(k_dyt_hist, dim3(p3v_cdiv(p.H, 256), p.R, p.B), dim3(256), 0, s, p);
   P3V_CHECK_LAUNCH();
@@ -239,7 +296,9 @@ extern "C" int p3v_gemm_any(const p3v_gemm_args_t* a, int a_f32, void* stream) {
 // ---------------------------------------------------------------- head split: whole-projection q / k norms, value mixing, cache append
 // gridDim.x walks the 16-token blocks of the value cache that a call touches; gridDim.z shares a block's work: 4 workgroups for the
 // query / key norms (a wave per token), 4 for a quarter of the value columns each.
-template <typename T, int V>
+// CH > 0: a token's query and key rows are requested together and stay in registers, CH 8-element pieces a lane each (one piece after the other,
+// read again behind the norm, the wave waits for two dozen round trips: 2048 tokens x 32 heads x 96 32.3 -> 23.2 us, 88 MB).
+template <typename T, int V, int CH>
 __global__ void __launch_bounds__(256) k_qkv_heads(QkvHeadsP p) {
   const int b = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int past = p.d_past ? *p.d_past : p.past;
@@ -251,6 +310,41 @@ __global__ void __launch_bounds__(256) k_qkv_heads(QkvHeadsP p) {
   if (part < 4 && pos >= pos_lo && pos < pos_hi) {
     const int l = pos - past;
     const T* row = base + ((size_t)b * p.L + l) * p.ld;
+    if constexpr (CH > 0) {
+      float v[2][CH][8];
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int i = 0; i < CH; ++i) load_acts<8>(row + r * nq + min((i * 64 + lane) * 8, (r ? nk : nq) - 8), v[r][i]);
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        const int n = r ? nk : nq;
+        const bf16_t* norm = r ? p.k_norm : p.q_norm;
+        u32x4_t g[CH];
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+          const int e = (i * 64 + lane) * 8;
+          g[i] = *(const u32x4_t*)(norm + min(e, n - 8));
+          if (e < n) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) ss += v[r][i][j] * v[r][i][j];
+          }
+        }
+        const float rn = 1.f / sqrtf(wave_sum(ss) / (float)n + p.eps);
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+          const int e = (i * 64 + lane) * 8;
+          if (e >= n) continue;
+          const int h = e / p.dim, d = e - h * p.dim;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[r][i][j] = v[r][i][j] * rn * (j & 1 ? bf16hi(g[i][j >> 1]) : bf16lo(g[i][j >> 1]));
+          T* dst = r ? (T*)p.k + (((size_t)b * p.G + h) * p.Tp + pos) * p.dimp : (T*)p.q + (((size_t)b * p.H + h) * p.L + l) * p.dimp;
+          store_acts<8>(dst + d, v[r][i]);
+        }
+      }
+      return;
+    }
     float sq = 0.f, sk = 0.f;
     for (int e = lane * V; e < nq; e += 64 * V) { float v[V]; load_acts<V>(row + e, v);
 #pragma unroll
@@ -280,31 +374,31 @@ __global__ void __launch_bounds__(256) k_qkv_heads(QkvHeadsP p) {
   if constexpr (V == 8) {
     // a whole block of 16 tokens: 8 columns per thread, 16-byte loads, the 16 x 8 values turned around in registers
     if (p.vdim % 8 == 0 && (!p.v_first || p.ld_first % 8 == 0) && pos_hi - pos_lo == 16) {
-      for (int e = ((part - 4) * 256 + threadIdx.x) * 8; e < nv; e += 8192) {
+      // (8 columns of 8 tokens a thread, dealt evenly to the four workgroups; the two halves of a 32-byte run to the same one)
+      const int pieces = nv / 8, per = (pieces + 3) / 4, c0 = (part - 4) * per, n = min(per, pieces - c0);
+      for (int u = threadIdx.x; u < 2 * n; u += 256) {
+        const int half = u >= n ? 1 : 0, e = (c0 + u - half * n) * 8;
         const int g = e / p.vdim, d = e - g * p.vdim;
         T* dst = (T*)p.v + ((((size_t)b * p.G + g) * (p.Tp >> 4) + blk) * p.vdimp + d) * 16;
         const T* src = base + ((size_t)b * p.L + pos_lo - past) * p.ld + nq + nk + e;
         const T* first = p.v_first ? (const T*)p.v_first + ((size_t)b * p.L + pos_lo - past) * p.ld_first + e : nullptr;
+        float x[8][8];
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          float x[8][8];
+        for (int j = 0; j < 8; ++j) {
+          load_acts<8>(src + (size_t)(half * 8 + j) * p.ld, x[j]);
+          if (first) {
+            float f[8];
+            load_acts<8>(first + (size_t)(half * 8 + j) * p.ld_first, f);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            load_acts<8>(src + (size_t)(half * 8 + j) * p.ld, x[j]);
-            if (first) {
-              float f[8];
-              load_acts<8>(first + (size_t)(half * 8 + j) * p.ld_first, f);
-#pragma unroll
-              for (int k = 0; k < 8; ++k) x[j][k] = (1.f - p.vmix) * x[j][k] + p.vmix * f[k];
-            }
+            for (int k = 0; k < 8; ++k) x[j][k] = (1.f - p.vmix) * x[j][k] + p.vmix * f[k];
           }
+        }
 #pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            float y[8];
+        for (int k = 0; k < 8; ++k) {
+          float y[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) y[j] = x[j][k];
-            store_acts<8>(dst + k * 16 + half * 8, y);
-          }
+          for (int j = 0; j < 8; ++j) y[j] = x[j][k];
+          store_acts<8>(dst + k * 16 + half * 8, y);
         }
       }
       return;
@@ -339,13 +433,16 @@ extern "C" int p3v_qkv_heads(const p3v_mix_args_t* a, void* stream) {
                        a->B, a->L, a->H, a->G, a->dim, a->vdim, a->dimp, a->vdimp, a->ld, a->ld_first, a->past, a->Tp};
   const dim3 grid(a->L == 1 ? 1 : p3v_cdiv(a->L + 15, 16) + (a->d_past ? 1 : 0), a->B, 8);
   const bool vec = a->dim % 8 == 0 && a->ld % 8 == 0;
+  const bool held = vec && a->H * a->dim <= 3072 && !(((uintptr_t)a->q_norm | (uintptr_t)a->k_norm) & 15);
   hipStream_t s = (hipStream_t)stream;
   if (a->f32) {
-    if (vec) hipLaunchKernelGGL((k_qkv_heads<float, 8>), grid, dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((k_qkv_heads<float, 1>), grid, dim3(256), 0, s, p);
+    if (held) hipLaunchKernelGGL((k_qkv_heads<float, 8, 6>), grid, dim3(256), 0, s, p);
+    else if (vec) hipLaunchKernelGGL((k_qkv_heads<float, 8, 0>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((k_qkv_heads<float, 1, 0>), grid, dim3(256), 0, s, p);
   } else {
-    if (vec) hipLaunchKernelGGL((k_qkv_heads<bf16_t, 8>), grid, dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((k_qkv_heads<bf16_t, 1>), grid, dim3(256), 0, s, p);
+    if (held) hipLaunchKernelGGL((k_qkv_heads<bf16_t, 8, 6>), grid, dim3(256), 0, s, p);
+    else if (vec) hipLaunchKernelGGL((k_qkv_heads<bf16_t, 8, 0>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((k_qkv_heads<bf16_t, 1, 0>), grid, dim3(256), 0, s, p);
   }
   P3V_CHECK_LAUNCH();
   return P3V_OK;

@@ -151,6 +151,53 @@ def test_dynamic_tanh_and_token_shift(R, parts):
     assert np.abs(host(plain).reshape(B, T, H) - orc.dyt(host(xd), 0.75, w, b)).max() < 0.02
 
 
+def shifted(t):
+    """The same values one element further on, where no wide load may start."""
+    s = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+    return s.copy_(t)
+
+
+@pytest.mark.parametrize("dt", [F32, BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("B,L,H,R", [(1, 1, 4, 2), (2, 7, 300, 5), (1, 8, 1028, 64), (2, 9, 3072, 3), (3, 40, 1024, 8)])
+def test_wide_and_narrow_dynamic_tanh_agree(B, L, H, R, dt):
+    """Four channels a lane and eight rows a run against one of each, which rows at odd addresses take: the same bits, the history too."""
+    from phi_3_vision_mlx_amd import ops
+    r = np.random.default_rng(H)
+    x, w, b, mu = dev(r.normal(0, 2, (B * L, H)), F32), dev(bf(r.normal(1, 0.3, H))), dev(bf(r.normal(0, 0.3, H))), dev(bf(r.uniform(0, 1, H)))
+    hist0, pad = dev(r.normal(0, 1, (B, R, H)), F32), torch.tensor([0, 4, 2][:B], dtype=I32, device=DEV)
+    got = []
+    for xi in (x, shifted(x)):
+        hist, out, plain = hist0.clone(), torch.empty((B * L, H), dtype=dt, device=DEV), torch.empty((B * L, H), dtype=dt, device=DEV)
+        ops.dyt(xi, (0.75, w, b), out, B, L, shift=mu, hist=hist, past=3, pad_len=pad)
+        ops.dyt(xi, (0.75, w, b), plain, B, L)
+        got.append((out, hist, plain))
+    for a, c in zip(*got):
+        assert torch.equal(a, c)
+
+
+@pytest.mark.parametrize("dt", [F32, BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("L,past,H,G,dim,vdim", [(1, 0, 2, 2, 8, 32), (17, 15, 4, 2, 72, 40), (40, 3, 32, 32, 96, 96), (33, 16, 32, 8, 96, 64)])
+def test_head_split_with_its_rows_held_and_read_twice(L, past, H, G, dim, vdim, dt):
+    """Rows of up to 3072 stay in registers where the norms' weights allow wide loads; elsewhere they are read twice.  The values have the same
+    bits; a lane's sum of at most 48 squares may be contracted to FMAs at other places, 48 x 2^-24 of the norm, then one rounding to T."""
+    from phi_3_vision_mlx_amd import ops
+    r = np.random.default_rng(dim)
+    from phi_3_vision_mlx_amd.cache import round_up
+    dp, vp, Tp, width = round_up(dim, 32), round_up(vdim, 32), 96, (H + G) * dim + G * vdim + H
+    qkv = dev(r.normal(0, 1, (L, (width + 7) // 8 * 8)), dt)
+    first, qn, kn = dev(r.normal(0, 1, (L, G * vdim)), dt), dev(bf(r.normal(1, 0.2, H * dim))), dev(bf(r.normal(1, 0.2, G * dim)))
+    talk, sink = dev(bf(np.eye(H))), dev(bf(np.zeros(H)))
+    got = []
+    for norms in ((qn, kn), (shifted(qn), shifted(kn))):
+        q, k, v = (torch.zeros(s, dtype=dt, device=DEV) for s in ((H * L * dp,), (1, G, Tp, dp), (1, G, Tp // 16, vp, 16)))
+        out = torch.empty((L, H * vdim), dtype=dt, device=DEV)
+        ops.attention_mixed(qkv, q, k, v, out, norms, talk, sink, 1, L, H, G, dim, vdim, 1e-5, dim ** -0.5, past, v_first=first, vmix=0.25, n_split=0)
+        got.append((q, k, v))
+    for name, a, c in zip("qkv", *got):
+        diff = (a.double() - c.double()).abs()
+        assert (diff <= c.double().abs() * (0 if name == "v" else 2.0 ** -18 if dt == F32 else 2.0 ** -7)).all(), (name, diff.max().item())
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 64, 128), (1, 320, 1024), (1, 128, 3072), (1, 64, 8192), (2, 50, 136), (5, 96, 2048), (8, 64, 3072), (8, 40, 12288), (12, 128, 3072), (16, 192, 512),
                                    (16, 64, 8192), (60, 128, 1024), (300, 3072, 512), (1100, 512, 256), (1100, 256, 192)])
 def test_scaled_residual_epilogue(M, N, K):
