@@ -10,12 +10,12 @@ struct LatP {
   const float* cos_t; const float* sin_t; void* c; void* q; const void* kx; const void* vx; void* out; float* ws;
   const int32_t* pad_len; const int32_t* d_past;
   float eps, scale;
-  int B, L, H, dim, rot, vdim, rank, rankp, rotp, dimp, ld, past, Tp, tab_n, n_keys, n_split, tiles_per_split;
+  int B, L, H, dim, rot, vdim, rank, rankp, rotp, dimp, ld, past, Tp, tab_n, n_keys, n_split, tiles_per_split, out_rows;
 };
 static inline LatP lat_params(const p3v_latent_args_t* a) {
   return {a->y, a->c_norm, a->uk, a->ukt, a->uv, a->sink, a->cos_t, a->sin_t, a->c, a->q, a->kx, a->vx, a->out, a->ws, a->pad_len, a->d_past,
           a->eps, a->scale, a->B, a->L, a->H, a->dim, a->rot, a->vdim, a->rank, a->rankp, a->rotp, a->dimp, a->ld, a->past, a->Tp, a->tab_n,
-          a->n_keys, a->n_split, 0};
+          a->n_keys, a->n_split, 0, 0};
 }
 // first columns of a packed row
 __host__ __device__ __forceinline__ int lat_dkv_col(const LatP& p) { return p.H * (p.dim + p.rot); }

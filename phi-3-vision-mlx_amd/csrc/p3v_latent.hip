@@ -228,8 +228,11 @@ __global__ void __launch_bounds__(256) k_latent_attn(LatP p) {
 }
 
 // ---------------------------------------------------------------- merge, value up-projection, gate
-// A workgroup per (head, 32 value dimensions, 16 rows): two 16-dimension tiles x four quarters of the rank; weights and, for few rows, the
+// A workgroup per (head, 32 value dimensions, out_rows rows): two 16-dimension tiles x four quarters of the rank; weights and, for few rows, the
 // partials are requested before anything else.
+// What bounds it is the partials a CU pulls (5 rows x 18 splits of 512 ranks are 184 KB, for each 32 dimensions again): with all rows of a call
+// in one workgroup the 96 of them for 32 heads x 96 leave most CUs idle, so as many rows go to one as brings about 300
+// (5 rows at 1024 keys 8.8 -> 8.15 us; requesting all splits at once costs the second workgroup of a CU: 10.6).
 #define LAT_MAX_SPLIT 128
 template <int RC>
 __global__ void __launch_bounds__(512) k_latent_out(LatP p) {
@@ -238,7 +241,7 @@ __global__ void __launch_bounds__(512) k_latent_out(LatP p) {
   __shared__ __attribute__((aligned(16))) bf16_t ol[16 * OS];
   __shared__ float4 part[512];
   const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lc = lane & 15, lg = lane >> 4;
-  const int row0 = blockIdx.z * 16, M = p.B * p.L, n_row = min(16, M - row0), kq = wave >> 1, v0 = blockIdx.y * 32 + (wave & 1) * 16;
+  const int row0 = blockIdx.z * p.out_rows, M = p.B * p.L, n_row = min(p.out_rows, M - row0), kq = wave >> 1, v0 = blockIdx.y * 32 + (wave & 1) * 16;
   constexpr int R4 = RC * 16, U = 8;                                     // float4 columns of a latent; splits requested at once
   const int items = n_row * R4, G = items >= 512 ? 1 : 512 / items, g = G > 1 ? tid / items : 0;
   const size_t step = (size_t)p.H * p.rankp;
@@ -447,7 +450,10 @@ template <int RC, int RT> static int launch_attn(const LatP& p, hipStream_t s) {
     set = true;
   }
   hipLaunchKernelGGL((k_latent_attn<RC, RT>), dim3(p.n_split, p3v_cdiv(p.H, 16), p.B * p.L), dim3(256), (LatCfg<RC, RT>::LDS), s, p);
-  hipLaunchKernelGGL(k_latent_out<RC>, dim3(p.H, p3v_cdiv(p.vdim, 32), p3v_cdiv(p.B * p.L, 16)), dim3(512), 0, s, p);
+  LatP po = p;
+  const int M = p.B * p.L, cols = p3v_cdiv(p.vdim, 32);
+  po.out_rows = min(16, p3v_cdiv((long)M * p.H * cols, 300));
+  hipLaunchKernelGGL(k_latent_out<RC>, dim3(p.H, cols, p3v_cdiv(M, po.out_rows)), dim3(512), 0, s, po);
   P3V_CHECK_LAUNCH();
   return P3V_OK;
 }

@@ -218,6 +218,18 @@ def test_latent_attention_forms_agree(H, dim, rot, vdim, rank):
         close(m.run(one, past + L, pads, plan=plan, d_past=plan == 2)[:, 0], want, BF16, plan)
 
 
+@pytest.mark.parametrize("B,L,H", [(1, 1, 32), (4, 1, 32), (7, 1, 32), (13, 1, 24), (5, 13, 20), (3, 16, 32)])
+def test_latent_attention_rows_of_a_merging_workgroup(B, L, H):
+    """As many rows to a workgroup of the merge as bring 300 of them: 1 .. 16, the last one's share smaller."""
+    past, pads = 130, [(37 * b) % 130 for b in range(B)]
+    m = Latent(H, 64, 32, 96, 512, B, 192, BF16, seed=B, scaling=YARN)
+    y = m.y(past + L)
+    m.run(y[:, :past].contiguous(), 0, pads)
+    got = m.run(y[:, past:].contiguous(), past, pads)
+    for b in range(B):
+        close(got[b], m.oracle(host(y)[b], pads[b])[past:], BF16, b)
+
+
 @pytest.mark.parametrize("dt", [F32, BF16])
 @pytest.mark.parametrize("far", [0, 1, 15, 63, 64, 127, 128, 255, 256, 399])
 def test_one_far_key_decides(far, dt):
