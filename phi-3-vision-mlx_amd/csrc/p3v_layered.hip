@@ -118,18 +118,20 @@ __global__ void __launch_bounds__(256) k_dyt(DytP p, T* __restrict__ out, bool s
     prev = h;
   }
 }
-// The same, four channels a lane and the run's rows requested together (k_dyt: one element a lane and load, each row's behind the one before it):
-// 2048 x 3072 16.7 -> 9.3 us (38 MB, which a large copy moves in 8); with the shift 11.8 -> 10.9.
-template <typename T, bool SHIFT>
+// The same, four channels a lane and RUN rows, requested together.  A wave's tanhs are a serial chain (four rows of four: 1 us), so the runs are
+// short: one row, two where there are waves enough (and, with the shift, where the row before costs its tanhs once more).  us, k_dyt and here,
+// 3072 channels: 8 rows 2.25 : 2.2, 256 3.4 : 2.7, 1024 7.3 : 4.7, 2048 16.4 : 7.7 (38 MB), 8192 57 : 23; with the shift 17 6.0 : 4.6, 256 6.1 : 5.4,
+// 512 6.5 : 6.4, 2048 14.2 : 13.0, but single tokens 2.5 : 2.65, which k_dyt keeps, and rows that wide loads cannot take.
+template <typename T, bool SHIFT, int RUN>
 __global__ void __launch_bounds__(256) k_dyt4(DytP p, T* __restrict__ out, bool store_hist) {
-  const int c = (blockIdx.x * 256 + threadIdx.x) * 4, b = SHIFT ? blockIdx.z : 0, l0 = blockIdx.y * DYT_ROWS;
+  const int c = (blockIdx.x * 256 + threadIdx.x) * 4, b = SHIFT ? blockIdx.z : 0, l0 = blockIdx.y * RUN;
   if (c >= p.H) return;
-  const int rows = SHIFT ? p.L : p.B * p.L, l1 = min(rows, l0 + DYT_ROWS);      // (without a shift every row is for itself)
+  const int rows = SHIFT ? p.L : p.B * p.L, l1 = min(rows, l0 + RUN);      // (without a shift every row is for itself)
   const float* x = p.x + (size_t)b * p.L * p.H + c;
   T* o = out + (size_t)b * p.L * p.H + c;
-  float4 xv[DYT_ROWS];
+  float4 xv[RUN];
 #pragma unroll
-  for (int j = 0; j < DYT_ROWS; ++j) xv[j] = *(const float4*)(x + (size_t)min(l0 + j, l1 - 1) * p.H);
+  for (int j = 0; j < RUN; ++j) xv[j] = *(const float4*)(x + (size_t)min(l0 + j, l1 - 1) * p.H);
   const float4 before = SHIFT ? *(const float4*)(x + (size_t)max(l0 - 1, 0) * p.H) : make_float4(0.f, 0.f, 0.f, 0.f);
   float w[4], bb[4], mu[4], prev[4] = {0.f, 0.f, 0.f, 0.f};
   load4(p.w + c, w);
@@ -148,7 +150,7 @@ __global__ void __launch_bounds__(256) k_dyt4(DytP p, T* __restrict__ out, bool 
     }
   }
 #pragma unroll
-  for (int j = 0; j < DYT_ROWS; ++j) {
+  for (int j = 0; j < RUN; ++j) {
     const int l = l0 + j;
     if (l >= l1) return;
     float h[4];
@@ -190,12 +192,18 @@ extern "C" int p3v_dyt(const p3v_dyt_args_t* a, void* out, int out_f32, void* st
   const dim3 grid(p3v_cdiv(p.H, 256), p3v_cdiv(p.L, DYT_ROWS), p.B);
   const bool late = p.mu && p.L >= p.R;
   const bool wide = p.H % 4 == 0 && !(((uintptr_t)p.x | (uintptr_t)p.hist | (uintptr_t)out) & 15) && !(((uintptr_t)p.w | (uintptr_t)p.b | (uintptr_t)p.mu) & 7);
-  const dim3 grid4(p3v_cdiv(p.H, 1024), p3v_cdiv(p.mu ? p.L : p.B * p.L, DYT_ROWS), p.mu ? p.B : 1);
-  if (wide && grid4.y <= 65535 && (long)p.B * p.L < 0x7fffffff) {
-    if (p.mu && out_f32) hipLaunchKernelGGL((k_dyt4<float, true>), grid4, dim3(256), 0, s, p, (float*)out, !late);
-    else if (p.mu) hipLaunchKernelGGL((k_dyt4<bf16_t, true>), grid4, dim3(256), 0, s, p, (bf16_t*)out, !late);
-    else if (out_f32) hipLaunchKernelGGL((k_dyt4<float, false>), grid4, dim3(256), 0, s, p, (float*)out, false);
-    else hipLaunchKernelGGL((k_dyt4<bf16_t, false>), grid4, dim3(256), 0, s, p, (bf16_t*)out, false);
+  const long rows = p.mu ? p.L : (long)p.B * p.L;               // those a run may come from
+  const bool two = rows > (p.mu ? 400 : 1500);
+  const dim3 grid4(p3v_cdiv(p.H, 1024), p3v_cdiv(rows, two ? 2 : 1), p.mu ? p.B : 1);
+  if (wide && !(p.mu && p.L == 1) && p3v_cdiv(rows, two ? 2 : 1) <= 65535) {
+#define P3V_DYT4(T, SHIFT)                                                                                                  \
+  if (two) hipLaunchKernelGGL((k_dyt4<T, SHIFT, 2>), grid4, dim3(256), 0, s, p, (T*)out, SHIFT && !late);                    \
+  else hipLaunchKernelGGL((k_dyt4<T, SHIFT, 1>), grid4, dim3(256), 0, s, p, (T*)out, SHIFT && !late);
+    if (p.mu && out_f32) { P3V_DYT4(float, true) }
+    else if (p.mu) { P3V_DYT4(bf16_t, true) }
+    else if (out_f32) { P3V_DYT4(float, false) }
+    else { P3V_DYT4(bf16_t, false) }
+#undef P3V_DYT4
   } else if (out_f32) hipLaunchKernelGGL(k_dyt<float>, grid, dim3(256), 0, s, p, (float*)out, !late);
   else hipLaunchKernelGGL(k_dyt<bf16_t>, grid, dim3(256), 0, s, p, (bf16_t*)out, !late);
   if (late) hipLaunchKernelGGL(k_dyt_hist, dim3(p3v_cdiv(p.H, 256), p.R, p.B), dim3(256), 0, s, p);

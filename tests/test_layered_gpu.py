@@ -158,9 +158,9 @@ def shifted(t):
 
 
 @pytest.mark.parametrize("dt", [F32, BF16], ids=["f32", "bf16"])
-@pytest.mark.parametrize("B,L,H,R", [(1, 1, 4, 2), (2, 7, 300, 5), (1, 8, 1028, 64), (2, 9, 3072, 3), (3, 40, 1024, 8)])
+@pytest.mark.parametrize("B,L,H,R", [(1, 1, 4, 2), (2, 7, 300, 5), (1, 400, 1028, 64), (2, 401, 3072, 3), (3, 502, 1024, 8), (1, 1503, 36, 5)])
 def test_wide_and_narrow_dynamic_tanh_agree(B, L, H, R, dt):
-    """Four channels a lane and eight rows a run against one of each, which rows at odd addresses take: the same bits, the history too."""
+    """Four channels a lane, in runs of one row and of two, against k_dyt, which rows at odd addresses take: the same bits, the history too."""
     from phi_3_vision_mlx_amd import ops
     r = np.random.default_rng(H)
     x, w, b, mu = dev(r.normal(0, 2, (B * L, H)), F32), dev(bf(r.normal(1, 0.3, H))), dev(bf(r.normal(0, 0.3, H))), dev(bf(r.uniform(0, 1, H)))
