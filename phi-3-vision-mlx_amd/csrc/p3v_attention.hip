@@ -420,7 +420,8 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(AttnP p) {
 // Two LDS buffers, one barrier per tile; compute part and masks identical to k_attn_prefill.
 typedef const __attribute__((address_space(1))) void* pf_gptr_t;
 typedef __attribute__((address_space(3))) void* pf_lptr_t;
-template <int HD, bool PRE>                                    // PRE: Q arrives multiplied by scale * log2(e) (p3v_rope_kv_append's q_scale)
+// PRE: Q arrives multiplied by scale * log2(e) (p3v_rope_kv_append's q_scale).  U: 16-query blocks of a wave, 64 U queries of a workgroup
+template <int HD, bool PRE, int U>
 __global__ void __launch_bounds__(256, 2) k_attn_prefill_dma(AttnP p) {
   constexpr int KROW = HD * 2, VROW = 128, NKS = HD / 32, NDT = HD / 16, CPR = HD / 8;
   constexpr int KTILE = 64 * KROW, VTILE = HD * VROW, BUF = KTILE + VTILE;
@@ -432,24 +433,25 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill_dma(AttnP p) {
   // block i costs i+1 tiles, so the dispatcher sees the longest jobs first and the tail of the launch is made of short
   // ones -- interleaving `head_group` heads at a time, so that the K/V of the heads in flight stay cache-resident
   // (all heads for short prompts; 8 or 4 when one head's K/V is megabytes).
-  const int nqb = (p.L + 127) >> 7, per_group = p.head_group * nqb;
+  constexpr int QB = 64 * U;
+  const int nqb = (p.L + QB - 1) / QB, per_group = p.head_group * nqb;
   const int grp = blockIdx.x / per_group, within = blockIdx.x - grp * per_group;
   const int qblk = nqb - 1 - within / p.head_group;
   const int b = blockIdx.z, head = grp * p.head_group + within % p.head_group, kvh = head / (p.nh / p.nkv);
   const int past = p.d_past ? *p.d_past : p.past;
   const int total = past + p.L;
   const int pad = p.pad_len ? p.pad_len[b / p.pad_div] : 0;
-  const int qb0 = qblk * 128, q0 = qb0 + wave * 32;
-  const int kv_end = p.causal ? min(total, past + qb0 + 128) : total;
+  const int qb0 = qblk * QB, q0 = qb0 + wave * 16 * U;
+  const int kv_end = p.causal ? min(total, past + qb0 + QB) : total;
   const int kv_begin = pad & ~63;
-  const int wave_last = p.causal ? past + q0 + 31 : total;  // last key position this wave can see
+  const int wave_last = p.causal ? past + q0 + 16 * U - 1 : total;  // last key position this wave can see
   const float sc2 = p.sc2;                                            // scale * log2(e)
 
-  bf16x8_t qf[2][NKS];
-  int qpos[2];
-  bool qvalid[2];
+  bf16x8_t qf[U][NKS];
+  int qpos[U];
+  bool qvalid[U];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int qrow = q0 + u * 16 + qi;
     qvalid[u] = qrow < p.L;
     qpos[u] = past + qrow;
@@ -519,15 +521,18 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill_dma(AttnP p) {
   // 4 MFMAs per tile instead of 32 v_add + two cross-lane reductions: the kernel is VALU-bound, the matrix pipe is 70 % idle.
   const u32x4_t ones_w = qi == 0 ? (u32x4_t){0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u} : (u32x4_t){0u, 0u, 0u, 0u};
   const bf16x8_t ones_f = __builtin_bit_cast(bf16x8_t, ones_w);
-  float m_run[2] = {PRE ? 0.f : -INFINITY, PRE ? 0.f : -INFINITY};   // PRE: reference of the exponent (finite always), log2 units; else: running maximum
-  unsigned long long unset[2] = {~0ull, ~0ull};              // lanes whose query has not seen a visible key yet: the next one sets the reference
-  f32x4_t negm[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};   // (PRE) -reference, the C operand of the S^T products
-  f32x4_t ol[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-  f32x4_t o[2][NDT];
+  float m_run[U];                                             // PRE: reference of the exponent (finite always), log2 units; else: running maximum
+  unsigned long long unset[U];                               // lanes whose query has not seen a visible key yet: the next one sets the reference
+  f32x4_t negm[U];                                           // (PRE) -reference, the C operand of the S^T products
+  f32x4_t ol[U];
+  f32x4_t o[U][NDT];
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+  for (int u = 0; u < U; ++u) {
+    m_run[u] = PRE ? 0.f : -INFINITY, unset[u] = ~0ull;
+    negm[u] = ol[u] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int d = 0; d < NDT; ++d) o[u][d] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  }
 
   if (kv_begin < kv_end) stage(kv_begin, 0);
   int buf = 0;
@@ -537,25 +542,25 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill_dma(AttnP p) {
     if (kv0 + 64 < kv_end) stage(kv0 + 64, buf ^ 1);          // next tile streams in under the MFMAs below
     if (kv0 <= wave_last) {                                   // wave-uniform: tiles above this wave's diagonal are skipped
       const unsigned char* Ks = smem + buf * BUF;
-      f32x4_t s[2][4];
+      f32x4_t s[U][4];
       // the two MFMA blocks of a tile run at raised wave priority: the SIMD's other wave is usually in its softmax, and a
       // wave that has to wait for VALU slots between its MFMAs also loses the matrix pipe (8k: 650 -> 630 us)
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
-        s[0][st] = PRE ? negm[0] : (f32x4_t){0.f, 0.f, 0.f, 0.f};   // PRE: the accumulators START at -reference: the product IS the exponent
-        s[1][st] = PRE ? negm[1] : (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < U; ++u) s[u][st] = PRE ? negm[u] : (f32x4_t){0.f, 0.f, 0.f, 0.f};   // PRE: the accumulators START at -reference: the product IS the exponent
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
           const bf16x8_t kf = *(const bf16x8_t*)(Ks + k_rd[ks] + st * 16 * KROW);
-          s[0][st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[0][ks], s[0][st], 0, 0, 0);
-          s[1][st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[1][ks], s[1][st], 0, 0, 0);
+#pragma unroll
+          for (int u = 0; u < U; ++u) s[u][st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[u][ks], s[u][st], 0, 0, 0);
         }
       }
       __builtin_amdgcn_s_setprio(0);
       // every key of the tile visible to every query of the wave -> no per-element mask work (wave-uniform)
       const bool interior = kv0 + 64 <= kv_end && kv0 >= pad && past + q0 >= pad && (!p.causal || kv0 + 63 <= past + q0);
-      bf16x8_t pf[2][2];
+      bf16x8_t pf[U][2];
       // PRE (pre-scaled Q: the decoder's prompts): softmax with a DEFERRED reference, as k_attn_prefill_pp / _il -- the S^T
       // accumulators started at -reference, so the product IS the exponent; the reference moves only on the query's first
       // visible tile and when a score exceeds it by more than 2^8 (wave-uniform slow path: O, l and the tile's scores are
@@ -575,7 +580,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill_dma(AttnP p) {
       asm volatile("s_nop 7\n\ts_nop 4");
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < U; ++u) {
         if (!interior) {
           const float ninf = -INFINITY;
 #pragma unroll
@@ -637,7 +642,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill_dma(AttnP p) {
       }
       } else {
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < U; ++u) {
         float m_t = -INFINITY;
         if (interior) {
 #pragma unroll
@@ -690,21 +695,22 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill_dma(AttnP p) {
           const u32x2_t a1 = *(const u32x2_t*)(Ks + v_rd[2 * st + 1] + d * 16 * VROW);
           const u32x4_t aw = {a0[0], a0[1], a1[0], a1[1]};
           const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, aw);
-          o[0][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[0][st], o[0][d], 0, 0, 0);
-          o[1][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[1][st], o[1][d], 0, 0, 0);
+#pragma unroll
+          for (int u = 0; u < U; ++u) o[u][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[u][st], o[u][d], 0, 0, 0);
         }
 #pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        ol[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_f, pf[0][st], ol[0], 0, 0, 0);
-        ol[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_f, pf[1][st], ol[1], 0, 0, 0);
-      }
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int u = 0; u < U; ++u) ol[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones_f, pf[u][st], ol[u], 0, 0, 0);
       __builtin_amdgcn_s_setprio(0);
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  const float l_fin[2] = {rows_sum(ol[0][0]), rows_sum(ol[1][0])};   // the sum sits in the g = 0 lane of the query's column (all lanes take part)
+  float l_fin[U];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
+  for (int u = 0; u < U; ++u) l_fin[u] = rows_sum(ol[u][0]);   // the sum sits in the g = 0 lane of the query's column (all lanes take part)
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
     if (!qvalid[u]) continue;
     const float inv = l_fin[u] > 0.f ? 1.f / l_fin[u] : 0.f;
     bf16_t* op = p.out + ((size_t)b * p.L + (q0 + u * 16 + qi)) * (size_t)(p.nh * HD) + head * HD + 4 * g;
@@ -1223,6 +1229,13 @@ __global__ void __launch_bounds__(512, 1) k_attn_prefill_pp(AttnP p) {
 //   pp  (ping-pong, 256 queries): what is left for it -- plain Q or head dim 64 from 3072 tokens.
 #include "p3v_attn_il.h"
 constexpr int P3V_ATTN_PP_MIN_L = 3072;                          // tools/attn_short_probe.py: dma / pp 65.2 / 67.5 us at 2531, 82.3 / 79.0 at 3072
+// 64 queries a workgroup of k_attn_prefill_dma, one 16-query block a wave: a wave's softmax runs at one instruction per 8 - 10 cycles whatever the
+// others do, so half the blocks are half of that chain, for twice the requests of keys and values -- while the chip is not full of them.
+// us with two blocks a wave and one, 32 heads x 96, causal: 17 tokens 5.6 : 4.9, 128 8.3 : 6.5, 256 11.7 : 9.2, 512 17.6 : 13.7, 767 23.2 : 19.0;
+// 8 rows x 128 10.6 : 9.5, 4 x 384 18.9 : 16.0; 16 heads x 64, 577 tokens, no mask: 1 crop 16.5 : 12.2, 6 (480 workgroups of two blocks)
+// 22.2 : 21.0, 8 (640) 28.2 : 30.3.
+static bool dma_half_blocks(int pairs, int L) { return (long)pairs * p3v_cdiv(L, 128) <= 512; }
+
 template <int HD>
 static int launch_attn_prefill(const AttnP& p, hipStream_t s) {
   constexpr int LDS = 2 * (64 * (HD * 2 + 16) + HD * (64 * 2 + 16));
@@ -1237,9 +1250,9 @@ static int launch_attn_prefill(const AttnP& p, hipStream_t s) {
     constexpr int LDS2 = 2 * (64 * HD * 2 + HD * 128);
     static bool attr2_set = false;
     if (!attr2_set) {
-      if (hipFuncSetAttribute((const void*)k_attn_prefill_dma<HD, true>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS2) != hipSuccess ||
-          hipFuncSetAttribute((const void*)k_attn_prefill_dma<HD, false>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS2) != hipSuccess)
-        return P3V_ERR_HIP;
+      for (const void* fn : {(const void*)k_attn_prefill_dma<HD, true, 2>, (const void*)k_attn_prefill_dma<HD, false, 2>,
+                             (const void*)k_attn_prefill_dma<HD, true, 1>, (const void*)k_attn_prefill_dma<HD, false, 1>})
+        if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, LDS2) != hipSuccess) return P3V_ERR_HIP;
       attr2_set = true;
     }
     AttnP q = p;
@@ -1249,13 +1262,14 @@ static int launch_attn_prefill(const AttnP& p, hipStream_t s) {
     const int il = p3v_tuning().attn_il;                         // the interleaved kernel (pre-scaled Q only)
     // Which kernel for a pre-scaled prompt (tools/attn_il4_probe.py, 32 heads x 96, causal, us; dma / il 4 waves / il 8 waves):
     //   B = 1:  512: 15.9 / 16.4 / 22.2   768: 21.1 / 20.1 / 26.6   1280: 32.3 / 27.1 / 34.8   2531: 64.6 / 52.6 / 58.8
+    //           (with 64 queries a workgroup, dma / il 4 waves: 768: 19.1 / 21.7   1024: 23.8 / 25.8   1152: 27.1 / 28.1   1280: 29.7 / 30.0   1536: 35.4 / 33.9)
     //           3072: 81.4 / 74.6 / 69.5   4096: 119 / 114 / 108    8192: 436 / 403 / 377
     //   B = 2:  1280: 40.0 / 36.5 / 40.3   2531: 91.8 / 99.8 / 106   4096: 221 / 219 / 228   5120: 343 / 320 / 328
     //   B = 4:  2531: 168 / 183 / 190      3072: 252 / 254 / 271   4096: 426 / 410 / 418   6144: 939 / 886 / 893   8192: 1614 / 1504 / 1477
     //   B = 8:  1280: 112 / 127 / 142      2531: 385 / 396 / 414
     // -> long prompts: 256-query workgroups (half the L2 -> LDS bytes per flop); ONE row of a few thousand tokens: 128-query
     //    workgroups of the interleaved kernel (best balance, two workgroups per CU); several rows: the 128-query kernel up to ~3500 tokens.
-    const bool il_auto = p.L >= 6144 || (p.B == 1 ? p.L >= 768 : p.L >= 3584);
+    const bool il_auto = p.L >= 6144 || (p.B == 1 ? p.L >= 1280 : p.L >= 3584);
     if (p.q_prescaled && (il > 0 || (il < 0 && pp != 0 && il_auto))) {   // (pp = 0 pins the dma kernel)
       constexpr int LDS4 = 3 * 64 * HD * 2 + 3 * HD * 128;
       static bool attr4_set = false;
@@ -1288,8 +1302,11 @@ static int launch_attn_prefill(const AttnP& p, hipStream_t s) {
       P3V_CHECK_LAUNCH();
       return P3V_OK;
     }
-    if (p.q_prescaled) hipLaunchKernelGGL((k_attn_prefill_dma<HD, true>), dim3(p.nh * p3v_cdiv(p.L, 128), 1, p.B), dim3(256), LDS2, s, q);
-    else hipLaunchKernelGGL((k_attn_prefill_dma<HD, false>), dim3(p.nh * p3v_cdiv(p.L, 128), 1, p.B), dim3(256), LDS2, s, q);
+    const int wu = p3v_tuning().attn_dma_u;                      // 16-query blocks a wave; -1: by shape
+    const bool half = wu > 0 ? wu == 1 : dma_half_blocks(p.nh * p.B, p.L);
+    const dim3 grid_d(p.nh * p3v_cdiv(p.L, half ? 64 : 128), 1, p.B);
+    if (p.q_prescaled) hipLaunchKernelGGL((half ? k_attn_prefill_dma<HD, true, 1> : k_attn_prefill_dma<HD, true, 2>), grid_d, dim3(256), LDS2, s, q);
+    else hipLaunchKernelGGL((half ? k_attn_prefill_dma<HD, false, 1> : k_attn_prefill_dma<HD, false, 2>), grid_d, dim3(256), LDS2, s, q);
   } else {
     hipLaunchKernelGGL(k_attn_prefill<HD>, grid, dim3(256), LDS, s, p);
   }

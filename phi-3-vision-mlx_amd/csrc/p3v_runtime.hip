@@ -49,7 +49,7 @@ const Knob kKnobs[] = {
     {"gemm_qkv_flat", &P3vTuning::gemm_qkv_flat, -1},
     {"gemm_rows", &P3vTuning::gemm_rows, 1},              {"gemm_tile", &P3vTuning::gemm_tile, -1},
     {"mix_wgs", &P3vTuning::mix_wgs, 0},
-    {"attn_rows", &P3vTuning::attn_rows, -1},
+    {"attn_rows", &P3vTuning::attn_rows, -1},               {"attn_dma_u", &P3vTuning::attn_dma_u, -1},
     {"attn_fo_map", &P3vTuning::attn_fo_map, 2},              {"attn_fo_map_q8", &P3vTuning::attn_fo_map_q8, 0},
 };
 P3vTuning g_tuning;

@@ -614,6 +614,22 @@ def test_attention_prefill_kernels(ops, orc, B, L, past, hd, nh, causal, pads, p
         _prefill_case(ops, orc, B, L, past, hd, nh, causal, pads, prescaled, pp, il_waves=4)      # 128-query workgroups
 
 
+@pytest.mark.parametrize("prescaled", [True, False], ids=["prescaled", "plain"])
+@pytest.mark.parametrize("B,L,past,hd,nh,causal,pads", [
+    (1, 128, 0, 96, 2, True, None), (1, 65, 0, 96, 2, True, None), (1, 17, 0, 96, 1, True, None), (2, 200, 0, 96, 2, True, [0, 131]),
+    (2, 33, 100, 96, 1, True, [3, 100]), (1, 577, 0, 64, 2, False, None), (1, 700, 0, 96, 1, True, None),
+])
+def test_attention_prefill_one_block_a_wave(ops, orc, request, B, L, past, hd, nh, causal, pads, prescaled):
+    """k_attn_prefill_dma with 64 queries a workgroup: a 16-query block is worked on alike whether its wave has another one or not, so the same bits."""
+    old = ops.set_tuning("attn_dma_u", -1)
+    request.addfinalizer(lambda: ops.set_tuning("attn_dma_u", old))
+    got = []
+    for u in (1, 2):
+        ops.set_tuning("attn_dma_u", u)
+        got.append(_prefill_case(ops, orc, B, L, past, hd, nh, causal, pads, prescaled, 0, spike=(0, L - 1, L // 2)))
+    assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("pp", [2, 1, 0], ids=["interleaved", "pingpong", "dma"])
 def test_attention_prefill_long_context_spot_rows(ops, orc, pp):
     """12288 queries x 12288 keys x 8 heads (K / V^T far larger than the L2: the LDS-DMA tiles arrive LATE, which is what
