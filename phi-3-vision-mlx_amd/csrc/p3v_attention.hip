@@ -30,6 +30,7 @@ struct AttnP {
   int B, L, nh, nkv, past, past_t, past_div, new_t, pad_div, causal, split_mode, n_split, new_is_cache;
   float scale;
   int head_group;              // k_attn_prefill_dma / _pp: heads whose query blocks are interleaved in launch order
+  int cu_blocks;               // k_attn_prefill_dma: query blocks of all heads that give each CU one workgroup, or 0 (query_block)
   float sc2;                   // what S = Q.K^T is multiplied by before exp2: scale * log2(e), or 1 when Q arrives pre-scaled
   int q_prescaled;
 };
@@ -420,6 +421,16 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(AttnP p) {
 // Two LDS buffers, one barrier per tile; compute part and masks identical to k_attn_prefill.
 typedef const __attribute__((address_space(1))) void* pf_gptr_t;
 typedef __attribute__((address_space(3))) void* pf_lptr_t;
+// The query block in place `at` of the launch order: longest first, but the second workgroup a CU gets -- dispatch goes round-robin over the CUs, so
+// it comes cu_blocks places behind the first -- in the opposite order, longest beside shortest (all of one row's heads in one group).  us, one row
+// of 32 heads x 96, 64 queries a workgroup: 768 tokens 19.1 -> 18.5, 1024 23.8 -> 22.7, 1280 29.7 -> 28.6.  (k_attn_prefill_il waits for its longest
+// workgroup whoever shares the CU: 54.3 us at 2531 tokens either way.)
+__device__ __forceinline__ int query_block(const AttnP& p, int at, int nqb) {
+  const int n = p.cu_blocks;
+  if (n && at >= n && at < 2 * n) at = n + min(2 * n, nqb) - 1 - at;
+  return nqb - 1 - at;
+}
+
 // PRE: Q arrives multiplied by scale * log2(e) (p3v_rope_kv_append's q_scale).  U: 16-query blocks of a wave, 64 U queries of a workgroup
 template <int HD, bool PRE, int U>
 __global__ void __launch_bounds__(256, 2) k_attn_prefill_dma(AttnP p) {
@@ -436,7 +447,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill_dma(AttnP p) {
   constexpr int QB = 64 * U;
   const int nqb = (p.L + QB - 1) / QB, per_group = p.head_group * nqb;
   const int grp = blockIdx.x / per_group, within = blockIdx.x - grp * per_group;
-  const int qblk = nqb - 1 - within / p.head_group;
+  const int qblk = query_block(p, within / p.head_group, nqb);
   const int b = blockIdx.z, head = grp * p.head_group + within % p.head_group, kvh = head / (p.nh / p.nkv);
   const int past = p.d_past ? *p.d_past : p.past;
   const int total = past + p.L;
@@ -1258,18 +1269,19 @@ static int launch_attn_prefill(const AttnP& p, hipStream_t s) {
     AttnP q = p;
     const size_t kv_bytes = (size_t)(p.past + p.L) * HD * 4;     // one head's K + V^T
     q.head_group = kv_bytes * p.nh <= (64u << 20) ? p.nh : (p.nh % 8 == 0 && kv_bytes * 8 <= (128u << 20) ? 8 : (p.nh % 4 == 0 ? 4 : p.nh));
+    q.cu_blocks = p.B == 1 && q.head_group == p.nh && 256 % p.nh == 0 && p.causal ? 256 / p.nh : 0;   // (one row: a second row's workgroups come behind all of the first's)
     const int pp = p3v_tuning().attn_pp;                         // -1: by shape; 0 / 1: pin (kernel tests run both)
     const int il = p3v_tuning().attn_il;                         // the interleaved kernel (pre-scaled Q only)
     // Which kernel for a pre-scaled prompt (tools/attn_il4_probe.py, 32 heads x 96, causal, us; dma / il 4 waves / il 8 waves):
     //   B = 1:  512: 15.9 / 16.4 / 22.2   768: 21.1 / 20.1 / 26.6   1280: 32.3 / 27.1 / 34.8   2531: 64.6 / 52.6 / 58.8
-    //           (with 64 queries a workgroup, dma / il 4 waves: 768: 19.1 / 21.7   1024: 23.8 / 25.8   1152: 27.1 / 28.1   1280: 29.7 / 30.0   1536: 35.4 / 33.9)
+    //           (with 64 queries a workgroup, dma / il 4 waves: 768: 18.5 / 21.7   1024: 22.7 / 25.8   1280: 28.6 / 30.1   1408: 31.2 / 31.9   1472: 32.6 / 32.0   1536: 34.0 / 33.8)
     //           3072: 81.4 / 74.6 / 69.5   4096: 119 / 114 / 108    8192: 436 / 403 / 377
     //   B = 2:  1280: 40.0 / 36.5 / 40.3   2531: 91.8 / 99.8 / 106   4096: 221 / 219 / 228   5120: 343 / 320 / 328
     //   B = 4:  2531: 168 / 183 / 190      3072: 252 / 254 / 271   4096: 426 / 410 / 418   6144: 939 / 886 / 893   8192: 1614 / 1504 / 1477
     //   B = 8:  1280: 112 / 127 / 142      2531: 385 / 396 / 414
     // -> long prompts: 256-query workgroups (half the L2 -> LDS bytes per flop); ONE row of a few thousand tokens: 128-query
     //    workgroups of the interleaved kernel (best balance, two workgroups per CU); several rows: the 128-query kernel up to ~3500 tokens.
-    const bool il_auto = p.L >= 6144 || (p.B == 1 ? p.L >= 1280 : p.L >= 3584);
+    const bool il_auto = p.L >= 6144 || (p.B == 1 ? p.L > 1408 : p.L >= 3584);
     if (p.q_prescaled && (il > 0 || (il < 0 && pp != 0 && il_auto))) {   // (pp = 0 pins the dma kernel)
       constexpr int LDS4 = 3 * 64 * HD * 2 + 3 * HD * 128;
       static bool attr4_set = false;

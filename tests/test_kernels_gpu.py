@@ -618,6 +618,7 @@ def test_attention_prefill_kernels(ops, orc, B, L, past, hd, nh, causal, pads, p
 @pytest.mark.parametrize("B,L,past,hd,nh,causal,pads", [
     (1, 128, 0, 96, 2, True, None), (1, 65, 0, 96, 2, True, None), (1, 17, 0, 96, 1, True, None), (2, 200, 0, 96, 2, True, [0, 131]),
     (2, 33, 100, 96, 1, True, [3, 100]), (1, 577, 0, 64, 2, False, None), (1, 700, 0, 96, 1, True, None),
+    (1, 513, 0, 96, 64, True, None), (1, 300, 20, 96, 128, True, [30]),      # 4 and 2 blocks to a round of the chip: 9 and 5 of them in the paired order
 ])
 def test_attention_prefill_one_block_a_wave(ops, orc, request, B, L, past, hd, nh, causal, pads, prescaled):
     """k_attn_prefill_dma with 64 queries a workgroup: a 16-query block is worked on alike whether its wave has another one or not, so the same bits."""
