@@ -423,7 +423,7 @@ typedef const __attribute__((address_space(1))) void* pf_gptr_t;
 typedef __attribute__((address_space(3))) void* pf_lptr_t;
 // The query block in place `at` of the launch order: longest first, but the second workgroup a CU gets -- dispatch goes round-robin over the CUs, so
 // it comes cu_blocks places behind the first -- in the opposite order, longest beside shortest (all of one row's heads in one group).  us, one row
-// of 32 heads x 96, 64 queries a workgroup: 768 tokens 19.1 -> 18.5, 1024 23.8 -> 22.7, 1280 29.7 -> 28.6.  (k_attn_prefill_il waits for its longest
+// of 32 heads x 96, 64 queries a workgroup: 576 and 640 tokens unchanged, 768 19.1 -> 18.5, 1024 23.8 -> 22.7.  (k_attn_prefill_il waits for its longest
 // workgroup whoever shares the CU: 54.3 us at 2531 tokens either way.)
 __device__ __forceinline__ int query_block(const AttnP& p, int at, int nqb) {
   const int n = p.cu_blocks;
@@ -1274,14 +1274,15 @@ static int launch_attn_prefill(const AttnP& p, hipStream_t s) {
     const int il = p3v_tuning().attn_il;                         // the interleaved kernel (pre-scaled Q only)
     // Which kernel for a pre-scaled prompt (tools/attn_il4_probe.py, 32 heads x 96, causal, us; dma / il 4 waves / il 8 waves):
     //   B = 1:  512: 15.9 / 16.4 / 22.2   768: 21.1 / 20.1 / 26.6   1280: 32.3 / 27.1 / 34.8   2531: 64.6 / 52.6 / 58.8
-    //           (with 64 queries a workgroup, dma / il 4 waves: 768: 18.5 / 21.7   1024: 22.7 / 25.8   1280: 28.6 / 30.1   1408: 31.2 / 31.9   1472: 32.6 / 32.0   1536: 34.0 / 33.8)
+    //           (with 64 queries a workgroup, dma / il 4 waves: 768: 18.5 / 21.7   1024: 22.7 / 25.8   1280: 28.6 / 30.1   1408: 31.2 / 31.9   1472: 32.6 / 32.0.
+    //            Not taken up: the two round differently, which 32 layers of 8-bit activations carry to 6 % of a logit, either 5 % from 64 bits)
     //           3072: 81.4 / 74.6 / 69.5   4096: 119 / 114 / 108    8192: 436 / 403 / 377
     //   B = 2:  1280: 40.0 / 36.5 / 40.3   2531: 91.8 / 99.8 / 106   4096: 221 / 219 / 228   5120: 343 / 320 / 328
     //   B = 4:  2531: 168 / 183 / 190      3072: 252 / 254 / 271   4096: 426 / 410 / 418   6144: 939 / 886 / 893   8192: 1614 / 1504 / 1477
     //   B = 8:  1280: 112 / 127 / 142      2531: 385 / 396 / 414
     // -> long prompts: 256-query workgroups (half the L2 -> LDS bytes per flop); ONE row of a few thousand tokens: 128-query
     //    workgroups of the interleaved kernel (best balance, two workgroups per CU); several rows: the 128-query kernel up to ~3500 tokens.
-    const bool il_auto = p.L >= 6144 || (p.B == 1 ? p.L > 1408 : p.L >= 3584);
+    const bool il_auto = p.L >= 6144 || (p.B == 1 ? p.L >= 768 : p.L >= 3584);
     if (p.q_prescaled && (il > 0 || (il < 0 && pp != 0 && il_auto))) {   // (pp = 0 pins the dma kernel)
       constexpr int LDS4 = 3 * 64 * HD * 2 + 3 * HD * 128;
       static bool attr4_set = false;

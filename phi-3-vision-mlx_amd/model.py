@@ -428,7 +428,8 @@ class Phi3VModel(DecoderModel):
         if not ok and bufs.get("attn_merge", False) and B == 1 and L == 1 and not quantized:
             # Short contexts (64-key one-tile plans: the in-launch form above is for 128-key tiles): attention that only writes its partials
             # + the merge launch carrying the o_proj beats attention with the in-launch merge + an o_proj launch (1.587 -> 1.570 ms per
-            # step at 128 keys, 1.662 -> 1.652 at 1000; with the int8 cache it loses: 1.165 -> 1.179 at 128 keys, so not there)
+            # step at 128 keys, 1.662 -> 1.652 at 1000; with the int8 cache it loses: 1.165 -> 1.179 at 128 keys, so not there; caches of up to 384
+            # columns then need no partials at all: one launch, k_attn_rows_o)
             bufs["attn_merge"] = False
             self._plan_fused_oproj(bufs, B, L, T, quantized)
             if not bufs["fuse_o"]:
