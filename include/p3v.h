@@ -227,9 +227,10 @@ int p3v_gemm_qkv(const p3v_gemm_args_t* gemm /* host */, const p3v_qkv_split_t* 
 /* ---- p3v_gemm_qkv of 17 .. 128 rows, and p3v_gemm with a gated epilogue (SiLU, GELU) of 105 .. 128, as slices of K that are summed inside
  *      the launch: the same products, the slices' fp32 sums added in slice order.  ws: p3v_gemm_merge_ws_bytes(M, N, K, epilogue, qkv) bytes
  *      (0: not a shape of these calls; N = output columns, qkv = 1 for the former), 16-byte aligned and ZERO in its first 4096 before the
- *      first call, which every call leaves zero again -- so one for each stream, for these calls alone.  A workgroup waits only for ones
- *      ahead of it in dispatch order, and never without end: when the bound is reached its outputs are NaN.  P3V_ERR_UNSUPPORTED: nothing
- *      launched.  Graph-capturable. */
+ *      first call, which every call leaves as the next one needs it -- so one for each stream, for these calls alone.  A workgroup waits
+ *      only for ones ahead of it in dispatch order, and never without end: when the bound is reached its outputs of that call are NaN (the
+ *      next call's are not: its counters hold multiples of four then, and count on from there).  P3V_ERR_UNSUPPORTED: nothing launched.
+ *      Graph-capturable. */
 int64_t p3v_gemm_merge_ws_bytes(int M, int N, int K, int epilogue, int qkv);
 int p3v_gemm_merge(const p3v_gemm_args_t* gemm /* host */, void* ws, int64_t ws_bytes, void* stream);
 int p3v_gemm_qkv_merge(const p3v_gemm_args_t* gemm /* host */, const p3v_qkv_split_t* split /* host */, void* ws, int64_t ws_bytes, void* stream);

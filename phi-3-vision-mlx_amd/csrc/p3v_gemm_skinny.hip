@@ -71,10 +71,10 @@ struct SkinnyP {
   const bf16_t* col_scale;         // P3V_EPI_SCALE_RESID_F32
   int kslice;                      // 0: one pass with the epilogue; else K columns per slice, fp32 partials
   QkvP q;                          // P3V_EPI_QKV only (p3v_gemm_qkv.h): head split + rotation + KV append in the epilogue
-  float* xpart; unsigned* xflag;   // MERGE: partial tiles [tile][slice][consumer wave][block][lane] x 4, counters [tile][consumer wave] (0 between launches)
+  float* xpart; unsigned* xflag;   // MERGE: partial tiles [tile][slice][consumer wave][block][lane] x 4, counters [tile][consumer wave] (multiples of 4 between launches)
   int nk_part;                     // MERGE: K-tiles of a slice other than the last
+  unsigned polls;                  // MERGE: how often the last slice looks at a counter before it gives up
 };
-#define SK_MERGE_POLLS (1u << 22)  // (seconds: the partials' workgroups are ahead of the waiting one in dispatch order)
 
 #define P3V_EPI_QKV 100            // internal, as in the other GEMM kernels
 
@@ -232,6 +232,9 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
     // A wave of another slice writes its blocks past the caches, waits until they are there and counts itself in; the last slice's wave of
     // the same place waits for all of them and adds them in slice order.  Its workgroups come last in dispatch order, so whatever they
     // wait for runs or has run; it has more K-tiles than the others, whose sums are on their way meanwhile.
+    // A counter is a multiple of 4 between launches and counts modulo 4 (at most three others: merge_plan).  The waiting wave puts it back
+    // to 0; one that gave up cannot, the late ones are still to count themselves in: it adds what they leave to the next multiple, so that
+    // the next launch on this workspace, which starts behind them, waits for its own partials again.
     const int tile = (int)blockIdx.x, others = (int)gridDim.z - 1;
     // (rows and, in a V tile, tokens beyond M: nothing is stored for them)
     const bool live = (QKV && swapped ? m0 + wc * 64 : m0 + wr * NI * 16) < p.M;
@@ -252,8 +255,8 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
     }
     if (live) {
       bool late = true;
-      for (unsigned n = 0; n < SK_MERGE_POLLS; ++n) {
-        if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == (unsigned)others) { late = false; break; }
+      for (unsigned n = 0; n < p.polls; ++n) {
+        if ((__builtin_amdgcn_readfirstlane(__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) & 3u) == (unsigned)others) { late = false; break; }
         __builtin_amdgcn_s_sleep(1);
       }
       asm volatile("" ::: "memory");
@@ -277,7 +280,10 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4_t){__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
       }
-      if (lane == 0) __hip_atomic_store(flag, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (lane == 0) {
+        if (late) __hip_atomic_fetch_add(flag, 4u - (unsigned)others, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else __hip_atomic_store(flag, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
     }
   }
 
@@ -441,7 +447,7 @@ int p3v_gemm_skinny_partials(const p3v_gemm_args_t* a, int* S_out, hipStream_t s
   if (S <= 1 || !a->ws || a->ws_bytes < (int64_t)S * a->M * w_rows * 4) return P3V_ERR_UNSUPPORTED;
   if ((uintptr_t)a->ws & 15) return P3V_ERR_ARG;
   *S_out = S;
-  const SkinnyP p = {a->A, a->W, a->ws, a->resid, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, a->col_scale, a->K / S, {}, nullptr, nullptr, 0};
+  const SkinnyP p = {a->A, a->W, a->ws, a->resid, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, a->col_scale, a->K / S, {}, nullptr, nullptr, 0, 0};
   if (silu) return launch_skinny<P3V_EPI_SILU_MUL>(p, S, s);                       // (partials: the activation is the reduction's)
   if (a->epilogue == P3V_EPI_RESID_BF16) return launch_skinny<P3V_EPI_RESID_BF16>(p, S, s);
   return launch_skinny<P3V_EPI_NONE>(p, S, s);
@@ -460,7 +466,7 @@ int p3v_gemm_skinny_try(const p3v_gemm_args_t* a, hipStream_t s) {
   if (rc == P3V_OK) return p3v_splitk_reduce((const float*)a->ws, a, S, s);
   if (rc != P3V_ERR_UNSUPPORTED) return rc;
   if (sk_slices(a->M, a->N, a->K, a->epilogue) == 0) return P3V_ERR_UNSUPPORTED;   // (a rows shape whose slices found no workspace and that the tile kernel does not take)
-  const SkinnyP p = {a->A, a->W, a->out, a->resid, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, a->col_scale, 0, {}, nullptr, nullptr, 0};
+  const SkinnyP p = {a->A, a->W, a->out, a->resid, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, a->col_scale, 0, {}, nullptr, nullptr, 0, 0};
   if (a->epilogue == P3V_EPI_SCALE_RESID_F32) return launch_skinny<P3V_EPI_SCALE_RESID_F32>(p, 1, s);
   if (a->epilogue == P3V_EPI_SILU_MUL) return launch_skinny<P3V_EPI_SILU_MUL>(p, 1, s);
   if (a->epilogue == P3V_EPI_GELU_MUL) return launch_skinny<P3V_EPI_GELU_MUL>(p, 1, s);
@@ -481,7 +487,7 @@ int p3v_gemm_skinny_qkv(const p3v_gemm_args_t* a, const QkvP& q, hipStream_t s) 
       return P3V_ERR_HIP;
     attr_set = true;
   }
-  const SkinnyP p = {a->A, a->W, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0, nullptr, 0, q, nullptr, nullptr, 0};
+  const SkinnyP p = {a->A, a->W, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0, nullptr, 0, q, nullptr, nullptr, 0, 0};
   const int mt = p3v_cdiv(a->M, SK_BM), tiles = ((q.nh + q.nkv) * q.hd / 64) * mt + (q.nkv * q.hd / SK_BM) * p3v_cdiv(a->M, 64);
   hipLaunchKernelGGL((k_gemm_skinny<P3V_EPI_QKV, false, SK_TN>), dim3(tiles), dim3(512), SkCfg<SK_TN>::LDS, s, p);
   P3V_CHECK_LAUNCH();
@@ -496,7 +502,7 @@ int p3v_gemm_skinny_qkv(const p3v_gemm_args_t* a, const QkvP& q, hipStream_t s) 
 // 48; 16 each: 24.8 us, 20 : 14 : 14 23.5).  qkv 27.7 -> 22.4 us at 128 rows, 27.6 -> 19.0 at 64, 22.7 -> 18 at 17; gate_up 29.5 -> 26.9 at
 // 128, 27.2 -> 26.3 at 112, 26.1 -> 26.1 at 104 (64 rows, on 64-row tiles of the one-pass form: 22.0 : 23.1).  Every slice finishing a
 // share of the blocks instead: 26.8 and 30.9, the hand-over through memory then being behind everybody's products.
-#define SK_MERGE_FLAGS 4096        // bytes of counters in front of the partials (zero before the first launch; every launch leaves them zero)
+#define SK_MERGE_FLAGS 4096        // bytes of counters in front of the partials (zero before the first launch; every launch leaves them multiples of 4)
 struct MergePlan { int S, nk_part, tiles; };
 static MergePlan merge_plan(int M, int N, int K, int epilogue, bool qkv) {
   const MergePlan none = {0, 0, 0};
@@ -521,7 +527,7 @@ static int launch_merge(SkinnyP p, const MergePlan& pl, void* ws, hipStream_t s)
     if (hipFuncSetAttribute((const void*)k_gemm_skinny<EPI, false, 128, SK_BM, true>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS) != hipSuccess) return P3V_ERR_HIP;
     attr_set = true;
   }
-  p.xflag = (unsigned*)ws, p.xpart = (float*)((unsigned char*)ws + SK_MERGE_FLAGS), p.nk_part = pl.nk_part;
+  p.xflag = (unsigned*)ws, p.xpart = (float*)((unsigned char*)ws + SK_MERGE_FLAGS), p.nk_part = pl.nk_part, p.polls = (unsigned)max(p3v_tuning().gemm_merge_polls, 0);
   hipLaunchKernelGGL((k_gemm_skinny<EPI, false, 128, SK_BM, true>), dim3(pl.tiles, 1, pl.S), dim3(512), C::LDS, s, p);
   P3V_CHECK_LAUNCH();
   return P3V_OK;
@@ -540,7 +546,7 @@ extern "C" int p3v_gemm_merge(const p3v_gemm_args_t* a, void* ws, int64_t ws_byt
   const MergePlan pl = merge_plan(a->M, a->N, a->K, a->epilogue, false);
   const int rc = merge_args(a, ws, ws_bytes, pl);
   if (rc != P3V_OK) return rc;
-  const SkinnyP p = {a->A, a->W, a->out, nullptr, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, nullptr, 0, {}, nullptr, nullptr, 0};
+  const SkinnyP p = {a->A, a->W, a->out, nullptr, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, nullptr, 0, {}, nullptr, nullptr, 0, 0};
   hipStream_t s = (hipStream_t)stream;
   return a->epilogue == P3V_EPI_GELU_MUL ? launch_merge<P3V_EPI_GELU_MUL>(p, pl, ws, s) : launch_merge<P3V_EPI_SILU_MUL>(p, pl, ws, s);
 }
@@ -550,6 +556,6 @@ int p3v_gemm_skinny_qkv_merge(const p3v_gemm_args_t* a, const QkvP& q, void* ws,
   const MergePlan pl = merge_plan(a->M, a->N, a->K, P3V_EPI_NONE, true);
   const int rc = merge_args(a, ws, ws_bytes, pl);
   if (rc != P3V_OK) return rc;
-  const SkinnyP p = {a->A, a->W, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0, nullptr, 0, q, nullptr, nullptr, 0};
+  const SkinnyP p = {a->A, a->W, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0, nullptr, 0, q, nullptr, nullptr, 0, 0};
   return launch_merge<P3V_EPI_QKV>(p, pl, ws, s);
 }

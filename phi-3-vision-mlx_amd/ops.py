@@ -121,8 +121,8 @@ _merge_ws = {}
 
 
 def _merge_workspace(device, nbytes):
-    """Workspace of the launches that sum their K slices themselves (p3v_gemm_merge, p3v_gemm_qkv_merge): its counters are zero between
-    launches, so it is theirs alone -- one per (device, stream), or the graph's own."""
+    """Workspace of the launches that sum their K slices themselves (p3v_gemm_merge, p3v_gemm_qkv_merge): its counters carry over from
+    launch to launch, so it is theirs alone -- one per (device, stream), or the graph's own."""
     if _ws_owner is not None:
         holder, frozen = _ws_owner
         if holder.get("merge") is None or holder["merge"].numel() < nbytes:

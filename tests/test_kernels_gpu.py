@@ -1095,6 +1095,36 @@ def test_gemm_merge(ops, M, N, K, epi):
     assert ops.gemm_merge(a, w, e, again) and torch.equal(again, out[:M])
 
 
+def test_gemm_merge_after_a_wait_that_gave_up(ops, request):
+    """A launch whose waits give up at once (no look at the counters allowed: every kernel exits as ever) is NaN throughout, and the launches
+    behind it on the same workspace, of the same number of slices or another, are right: late partials are never counted for theirs."""
+    polls = ops.set_tuning("gemm_merge_polls", 1 << 22)
+    request.addfinalizer(lambda: ops.set_tuning("gemm_merge_polls", polls))
+    calls = []
+    for M, N, K in ((113, 4096, 2112), (128, 8192, 3072)):       # 4 and 2 slices
+        a, w = g((M, K), 450).cuda(), g((2 * N, K), 451, 1.0 / math.sqrt(K)).cuda()
+        calls.append((lambda out, a=a, w=w: ops.gemm_merge(a, w, ops.EPI_SILU_MUL, out[0]), lambda M=M, N=N: [torch.zeros((M, N), dtype=BF16).cuda()]))
+    a, w = g((67, 3072), 452).cuda(), g((9216, 3072), 453, 1.0 / math.sqrt(3072)).cuda()                   # 3 slices, waves without rows
+
+    def qkv_out():
+        return [torch.zeros(s, dtype=BF16).cuda() for s in ((1, 32, 67, 96), (1, 32, 72, 96), (1, 32, 96, 72))]
+    calls.append((lambda o: ops.gemm_qkv_merge(a, w, None, None, *o, 1, 67, 32, 32, 96, 0, 72, True), qkv_out))
+
+    def run(i, looks):
+        ops.set_tuning("gemm_merge_polls", looks)
+        out = calls[i][1]()
+        assert calls[i][0](out), "shape not taken"
+        return [t[:, :, :67] if i == 2 and t.shape[2] == 72 else t[..., :67] if i == 2 and t.shape[3] == 72 else t for t in out]
+    want = [run(i, 1 << 22) for i in range(3)]
+    assert all(torch.isfinite(t.float()).all() for o in want for t in o)
+    for late, then in ((0, 0), (1, 1), (2, 2), (0, 2), (2, 1), (1, 0)):
+        for _ in range(2):
+            assert all(torch.isnan(t.float()).all() for t in run(late, 0))
+        for i in (then, late):
+            for _ in range(2):
+                assert all(torch.equal(x, y) for x, y in zip(run(i, 1 << 22), want[i])), (late, then, i)
+
+
 def test_gemm_merge_refuses(ops):
     """Shapes of the other kernels: False, nothing launched."""
     for M, N, K in ((104, 8192, 3072), (129, 8192, 3072), (128, 8192, 512), (128, 1024, 3072), (128, 16384, 3072)):
