@@ -45,7 +45,8 @@ class DecoderModel:
         self.cfg, self.device = cfg, torch.device(device)
         self.hidden_hook = None                      # fn(layer, x [B*L, H], B, L) after every decoder layer (diagnostics)
         # A long-lived owner that may share the GPU with other streams / processes (server.py) sets this: the decode step then
-        # uses no launch that needs all of its workgroups resident at once.  One-shot generate() on an exclusive GPU keeps them.
+        # uses no launch that needs all of its workgroups resident at once, and a prompt none that waits for workgroups of its own grid
+        # (ops.gemm_merge, ops.gemm_qkv_merge).  One-shot generate() on an exclusive GPU keeps them.
         self.serving = os.environ.get("P3V_SHARED_GPU", "0") == "1"
         self.epoch = 0                               # bumped whenever captured decode graphs become stale
         self._prefill_graphs = {}                    # (S, max_tokens, ..) -> captured short-prompt prefill (see _prefill_captured)
@@ -263,6 +264,7 @@ class DecoderModel:
             key = self._prefill_key(S, max_tokens)
         if key is None:
             return None
+        key += (self.serving,)                                    # (which launches the capture holds)
         e = self._prefill_graphs.get(key)
         if e is None:
             if self._prefill_seen.get(key, 0) < 1:                # first sighting: eager (one-off lengths never pay for a capture)

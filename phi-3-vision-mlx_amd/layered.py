@@ -35,8 +35,8 @@ class DynamicTanh:
             raise ValueError("a dynamic tanh has no scale to take a multiplier into")
         self.args = (float(w[name + ".alpha"]), w[name].to(dev, BF16).contiguous(), w[name + ".b"].to(dev, BF16).contiguous())
 
-    def project(self, x, w, h, epilogue=EPI_NONE, out=None, B=1, Lq=1, **shift):
-        return ops.project_dyt(x, self.args, w, h, epilogue, out=out, B=B, Lq=Lq, **shift)
+    def project(self, x, w, h, epilogue=EPI_NONE, out=None, B=1, Lq=1, alone=True, **shift):
+        return ops.project_dyt(x, self.args, w, h, epilogue, out=out, B=B, Lq=Lq, alone=alone, **shift)
 
 
 class RmsNorm:
@@ -46,8 +46,8 @@ class RmsNorm:
         m = cfg.residual_mult
         self.args = (w[name].to(dev, BF16).contiguous(), cfg.norm_eps / (m * m), gain if m > 0 else -gain)
 
-    def project(self, x, w, h, epilogue=EPI_NONE, out=None, B=1, Lq=1):
-        return ops.project_rms(x, self.args, w, h, epilogue, out=out)
+    def project(self, x, w, h, epilogue=EPI_NONE, out=None, B=1, Lq=1, alone=True):
+        return ops.project_rms(x, self.args, w, h, epilogue, out=out, alone=alone)
 
 
 NORMS = {"dyt": DynamicTanh, "rms": RmsNorm}
@@ -167,7 +167,7 @@ class LayeredModel(DecoderModel):
             if ly.mlp:
                 ff = ly.spec.mlp.ff
                 h, a = h[:rows], bufs["a"][:rows * ff].view(rows, ff)
-                ly.norm2.project(x, ly.gate_up, h, ly.act, out=a, B=rows)
+                ly.norm2.project(x, ly.gate_up, h, ly.act, out=a, B=rows, alone=not self.serving)
                 ops.project(a, ly.down, EPI_SCALE_RESID_F32, resid=x, col_scale=ly.ls2, out=x)
             if self.hidden_hook is not None:
                 self.hidden_hook(i, x * self.cfg.residual_mult, B, rows // B)

@@ -171,7 +171,7 @@ class Phi3VModel(DecoderModel):
             return ops.gemv(x, w, epilogue, resid=resid, norm_w=norm_w, norm_eps=eps, out=out)
         if norm_w is not None:
             x = ops.rmsnorm(x, norm_w, eps, out=h)
-        if epilogue == EPI_SILU_MUL and 104 < M <= 128 and out is not None and ops.gemm_merge(x, w, epilogue, out):
+        if epilogue == EPI_SILU_MUL and 104 < M <= 128 and out is not None and not self.serving and ops.gemm_merge(x, w, epilogue, out):
             return out
         if epilogue == EPI_RESID_BF16 and out is not None and ops.gemm_slices(x, w, epilogue, resid, out):
             return out
@@ -524,7 +524,7 @@ class Phi3VModel(DecoderModel):
                     hn = h if normed_in else ops.rmsnorm(x, w[p + "input_layernorm.weight"], eps, out=h)
                     normed_in = True                            # (`h` holds the normalised input now, whatever the fused call answers)
                     qkv_args = (hn, w[k_w], st.cos, st.sin, q, kd, vd, B, L, nh, nkv, hd, past, st.Tp, True, st.T, 1)
-                    fused_qkv = (M <= 128 and ops.gemm_qkv_merge(*qkv_args, q_scale=scale * ops.Q_PRESCALE)
+                    fused_qkv = (M <= 128 and not self.serving and ops.gemm_qkv_merge(*qkv_args, q_scale=scale * ops.Q_PRESCALE)
                                  or ops.gemm_qkv(*qkv_args, q_scale=scale * ops.Q_PRESCALE))
             f8_w = self.w8.get(k_w)                             # the same on e4m3 weights and quantised rows
             if (f8_w is not None and L > ops.L.DECODE_MAX_L and n_beam == 1 and k_w not in self.adapters and not mlx4_first and self.fp8_act

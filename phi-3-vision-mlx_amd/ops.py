@@ -789,7 +789,7 @@ def _dyt_args(x, norm, B, Lq, shift, hist, past, d_past, pad_len):
                      int(past), hist.shape[1] if shift is not None else 0, B, Lq, H)
 
 
-def project_dyt(x, norm, w, h, epilogue=EPI_NONE, out=None, B=1, Lq=1, **shift):
+def project_dyt(x, norm, w, h, epilogue=EPI_NONE, out=None, B=1, Lq=1, alone=True, **shift):
     """project(dyt(x)): one launch for a single bf16 row of a width the streaming kernel takes, else the two (h: their scratch rows)."""
     M, H = B * Lq, x.shape[-1]
     if M == 1 and h.dtype == BF16 and out is not None:
@@ -804,7 +804,7 @@ def project_dyt(x, norm, w, h, epilogue=EPI_NONE, out=None, B=1, Lq=1, **shift):
             L.check(rc, "gemv_dyt")
             return out
     dyt(x, norm, h, B, Lq, **shift)
-    return project(h[:M], w, epilogue, out=out)
+    return project(h[:M], w, epilogue, out=out, alone=alone)
 
 
 def rms_rows(x, norm, out):
@@ -818,7 +818,7 @@ def rms_rows(x, norm, out):
     return out
 
 
-def project_rms(x, norm, w, h, epilogue=EPI_NONE, out=None):
+def project_rms(x, norm, w, h, epilogue=EPI_NONE, out=None, alone=True):
     """project(rms_rows(x)): one launch for up to 8 bf16 rows of a width the streaming kernels take, else the two (h: their scratch rows).
     2 .. 8 rows: outputs that the one launch does not write (fp32, rows of a wider matrix) go through the two."""
     M, H = x.shape
@@ -833,12 +833,13 @@ def project_rms(x, norm, w, h, epilogue=EPI_NONE, out=None):
             L.check(rc, "gemv_rms")
             return out
     rms_rows(x, norm, h)
-    return project(h[:M], w, epilogue, out=out)
+    return project(h[:M], w, epilogue, out=out, alone=alone)
 
 
-def project(x, w, epilogue=EPI_NONE, resid=None, col_scale=None, out=None):
+def project(x, w, epilogue=EPI_NONE, resid=None, col_scale=None, out=None, alone=True):
     """One projection of a layered decoder, x [M, K] bf16 or fp32: the weight-streaming GEMV, the MFMA GEMM, or -- fp32 rows, and sizes
-    those do not take -- the fp32-arithmetic kernel of every size."""
+    those do not take -- the fp32-arithmetic kernel of every size.  alone: is the GPU the caller's alone (a launch may wait for workgroups of
+    its own grid)?"""
     f32 = x.dtype == F32
     _chk(x, F32 if f32 else BF16, "x"), _chk(w, BF16, "w")
     M, K = x.shape
@@ -856,7 +857,7 @@ def project(x, w, epilogue=EPI_NONE, resid=None, col_scale=None, out=None):
         if M <= 8 and (1 << (M - 1).bit_length()) * K * 2 <= 160 * 1024 - 256:     # (the rows of x in a workgroup's LDS)
             return gemv(x, w, epilogue, resid=resid, out=out, col_scale=col_scale)
         if K % 64 == 0 and N % 8 == 0:
-            if epilogue in GATED and 104 < M <= 128 and gemm_merge(x, w, epilogue, out):
+            if alone and epilogue in GATED and 104 < M <= 128 and gemm_merge(x, w, epilogue, out):
                 return out
             if scaled and gemm_slices(x, w, epilogue, resid, out, col_scale=col_scale):
                 return out

@@ -519,6 +519,21 @@ def test_rewind_and_read_only_beams():
         m(input_ids=t[None, :2], cache=cache)
 
 
+def test_prompts_of_a_server_wait_for_no_other_workgroup(monkeypatch):
+    """A model that does not own the GPU never asks for the gated projections whose K slices are summed inside the launch."""
+    from phi_3_vision_mlx_amd import ops
+    m, w, d = build("streamed", "bfloat16")
+    asked = []
+    monkeypatch.setattr(ops, "gemm_merge", lambda *a: (asked.append(1), False)[1])
+    t, got = tokens(d, 110, 9), []
+    for serving in (False, True):
+        monkeypatch.setattr(m, "serving", serving)
+        got.append(m(input_ids=t[None], max_tokens=1, full_logits=True)[0])
+        assert bool(asked) != serving
+        asked.clear()
+    assert torch.equal(got[0], got[1])
+
+
 def test_captured_prefill_is_the_eager_one():
     """A prompt length seen twice is captured; later prompts of that length replay, with eager work in between, and each keeps its own
     cache while it is alive."""

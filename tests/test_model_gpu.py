@@ -1332,6 +1332,36 @@ def test_full_width_4bit_batched_decode_rows_equal_their_solo_runs(B):
     torch.cuda.empty_cache()
 
 
+def test_prompts_of_a_server_run_no_launch_that_waits_for_its_own_grid(monkeypatch):
+    """A model that does not own the GPU (model.serving) sums no K slices inside a launch, in an eager prompt or a captured one, also
+    where the capture of that length was made before the model was told: the logits are those with the merged launches switched off."""
+    from phi_3_vision_mlx_amd import ops
+    from phi_3_vision_mlx_amd.api import load_synthetic
+    model, _ = load_synthetic(blind_model=True, seed=3, num_hidden_layers=2, device="cuda:0")
+    calls = []
+    for name in ("gemm_merge", "gemm_qkv_merge"):
+        monkeypatch.setattr(ops, name, lambda *a, _f=getattr(ops, name), _n=name, **kw: (calls.append(_n), _f(*a, **kw))[1])
+    ids = rand_ids(120, 22)
+
+    def prompt():                                                # eager, captured, replayed
+        return [model(input_ids=ids, max_tokens=4)[0].clone() for _ in range(3)]
+    model.serving = False
+    own = prompt()
+    assert set(calls) == {"gemm_merge", "gemm_qkv_merge"} and len(model._prefill_graphs) == 1
+    calls.clear()
+    model.serving = True
+    shared = prompt()
+    assert not calls
+    model.serving = False
+    assert all(torch.equal(x, own[0]) for x in prompt())         # (the first capture again)
+    monkeypatch.setenv("P3V_GEMM_MERGE", "0")
+    monkeypatch.setenv("P3V_PREFILL_GRAPH", "0")
+    want = model(input_ids=ids, max_tokens=4)[0]
+    assert all(torch.equal(x, want) for x in shared) and not torch.equal(own[0], want)
+    del model
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("layers,serving", [(3, False), (2, False), (2, True)], ids=["odd-stack", "even-stack", "even-stack-server"])
 def test_fused_oproj_decode_needs_an_even_stack_and_an_exclusive_gpu(layers, serving, monkeypatch):
     """the fused attention + o_proj launch of layer i re-arms the OTHER parity's output buffer, so an odd number of
