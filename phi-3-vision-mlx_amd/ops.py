@@ -35,6 +35,13 @@ def _chk(t, dtype, name):
     return t
 
 
+def _chk_out(t, dtype, shape, like, name):
+    """A caller's output rows: they may lie in a wider matrix, nothing else."""
+    if t.device != like.device or t.dtype != dtype or tuple(t.shape) != shape or t.stride(1) != 1:
+        raise ValueError(f"{name}: {t.dtype} {tuple(t.shape)} (strides {tuple(t.stride())}) on {t.device} for {dtype} {shape} on {like.device}")
+    return t
+
+
 GATED = (EPI_SILU_MUL, EPI_GELU_MUL)                             # W = [gate; up]: out has half of its rows as columns
 
 
@@ -153,6 +160,7 @@ def gemm_merge(a, w, epilogue, out):
     n = L.lib().p3v_gemm_merge_ws_bytes(M, N, K, epilogue, 0) if epilogue in GATED and _merge_allowed() else 0
     if not n:
         return False
+    _chk_out(out, BF16, (M, N), a, "gemm_merge: out")
     ws = _merge_workspace(a.device, n)
     args = L.GemmArgs(_p(a), _p(w), _p(out), None, None, None, M, N, K, a.stride(0), w.stride(0), out.stride(0), epilogue, 0, None, 0, None)
     rc = L.lib().p3v_gemm_merge(C.byref(args), _p(ws), ws.numel(), _stream())
@@ -249,7 +257,7 @@ def gemm_rows_resid(a, w, resid, norm_w, scaled, sumsq, out=None):
         raise ValueError(f"gemm_rows_resid: sumsq holds {sumsq.numel()} of {parts * 16} values")
     if out is None:
         out = torch.empty((M, N), dtype=BF16, device=a.device)
-    if out.stride(0) != resid.stride(0):
+    if _chk_out(out, BF16, (M, N), a, "gemm_rows_resid: out").stride(0) != resid.stride(0):
         raise ValueError("gemm_rows_resid: resid and out are laid out alike")
     args = L.GemmArgs(_p(a), _p(w), _p(out), None, _p(resid), None, M, N, K, a.stride(0), w.stride(0), out.stride(0), EPI_RESID_BF16, 0, None, 0)
     L.check(L.lib().p3v_gemm_rows_resid(C.byref(args), _p(norm_w), _p(scaled), _p(sumsq), _stream()), "gemm_rows_resid")
@@ -261,8 +269,11 @@ def gemm_rows_scaled(scaled, w, sumsq, parts, eps, epilogue=EPI_NONE, out=None):
     _chk(scaled, BF16, "scaled"), _chk(w, BF16, "w"), _chk(sumsq, F32, "sumsq")
     M, K = scaled.shape
     N = w.shape[0] // 2 if epilogue in GATED else w.shape[0]
+    if w.shape[1] != K or sumsq.numel() < parts * 16:
+        raise ValueError(f"gemm_rows_scaled: shapes {tuple(scaled.shape)} x {tuple(w.shape)}, sumsq holds {sumsq.numel()} of {parts * 16} values")
     if out is None:
         out = torch.empty((M, N), dtype=BF16, device=scaled.device)
+    _chk_out(out, BF16, (M, N), scaled, "gemm_rows_scaled: out")
     args = L.GemmArgs(_p(scaled), _p(w), _p(out), None, None, None, M, N, K, scaled.stride(0), w.stride(0), out.stride(0), epilogue, 0, None, 0)
     L.check(L.lib().p3v_gemm_rows_scaled(C.byref(args), _p(sumsq), parts, float(eps), _stream()), "gemm_rows_scaled")
     return out

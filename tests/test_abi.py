@@ -63,6 +63,53 @@ def test_ops_fail_loudly_without_gpu_or_library(monkeypatch):
         _lib.lib()
 
 
+def test_row_projections_check_what_they_are_given(monkeypatch):
+    """gemm_merge, gemm_rows_resid, gemm_rows_scaled: a given output of another type or size, a weight of another width, too few sums of
+    squares -- an error before anything is launched; what fits is launched, rows of a wider matrix among it (launches are recorded here,
+    tensors are on the CPU)."""
+    import types
+
+    import torch
+    from phi_3_vision_mlx_amd import _lib, ops
+    real, launched, bf = _lib.lib(), [], torch.bfloat16
+    stub = types.SimpleNamespace(p3v_gemm_merge_ws_bytes=real.p3v_gemm_merge_ws_bytes, p3v_gemm_rows_resid_parts=real.p3v_gemm_rows_resid_parts,
+                                 **{n: lambda *a, n=n: launched.append(n) or 0 for n in ("p3v_gemm_merge", "p3v_gemm_rows_resid", "p3v_gemm_rows_scaled")})
+    monkeypatch.setattr(ops.L, "lib", lambda: stub)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_chk", lambda t, dtype, name: t)
+    monkeypatch.setattr(ops, "_merge_ws", {})
+
+    def rows(m, n, dtype=bf):
+        return torch.empty((m, n), dtype=dtype)
+    a, w, K = rows(112, 3072), rows(2 * 4096, 3072), 3072
+
+    def merge(out):
+        return ops.gemm_merge(a, w, ops.EPI_SILU_MUL, out)
+    x, wo, nw, scaled, sq = rows(12, K), rows(3072, K), rows(1, 3072)[0], rows(12, 3072), rows(192, 16, torch.float32)
+
+    def resid(out):
+        return ops.gemm_rows_resid(x, wo, rows(12, 3072), nw, scaled, sq, out=out)
+    wg = rows(2 * 64, K)
+
+    def behind(out, w=wg, sq=sq, parts=192):
+        return ops.gemm_rows_scaled(scaled, w, sq, parts, 1e-5, ops.EPI_SILU_MUL, out=out)
+    for call, m, n in ((merge, 112, 4096), (resid, 12, 3072), (behind, 12, 64)):
+        for bad in (rows(m, n, torch.float32), rows(m - 1, n), rows(m, n - 8), rows(m, n + 8), rows(m, 2 * n)[:, ::2], rows(n, m).t()):
+            with pytest.raises(ValueError):
+                call(bad)
+        assert not launched, call
+        call(rows(m, n))
+        if call is not resid:                                    # (whose output lies as its residual does)
+            call(rows(m, n + 8)[:, :n])
+        assert launched
+        launched.clear()
+    for kw in (dict(w=rows(128, K + 64)), dict(w=rows(128, K - 64)), dict(sq=rows(191, 16, torch.float32)), dict(parts=193)):
+        with pytest.raises(ValueError):
+            behind(None, **kw)
+    assert not launched
+    assert behind(None).shape == (12, 64) and launched
+
+
 def test_library_never_allocates_or_reads_the_environment_per_launch():
     """include/p3v.h: launches never allocate or synchronise (callers pass workspaces, e.g. p3v_gemm_ws_bytes); knobs come
     from ONE table filled once (p3v_runtime.hip).  Checked on the sources and on the library's undefined symbols."""
