@@ -129,7 +129,8 @@ _merge_ws = {}
 
 def _merge_workspace(device, nbytes):
     """Workspace of the launches that sum their K slices themselves (p3v_gemm_merge, p3v_gemm_qkv_merge): its counters carry over from
-    launch to launch, so it is theirs alone -- one per (device, stream), or the graph's own."""
+    launch to launch, so it is theirs alone -- one per (device, stream), or the graph's own.  None under a capture that owns none: zeros
+    that are only recorded are none for the launches before the first replay, and a replay may run beside the stream's own launches."""
     if _ws_owner is not None:
         holder, frozen = _ws_owner
         if holder.get("merge") is None or holder["merge"].numel() < nbytes:
@@ -137,6 +138,8 @@ def _merge_workspace(device, nbytes):
                 raise RuntimeError(f"merge workspace of {nbytes} bytes requested under graph capture")
             holder["merge"] = torch.zeros(nbytes, dtype=torch.uint8, device=device)
         return holder["merge"]
+    if torch.cuda.is_current_stream_capturing():
+        return None
     key = (device.index, _stream())
     buf = _merge_ws.get(key)
     if buf is None or buf.numel() < nbytes:
@@ -162,6 +165,8 @@ def gemm_merge(a, w, epilogue, out):
         return False
     _chk_out(out, BF16, (M, N), a, "gemm_merge: out")
     ws = _merge_workspace(a.device, n)
+    if ws is None:
+        return False
     args = L.GemmArgs(_p(a), _p(w), _p(out), None, None, None, M, N, K, a.stride(0), w.stride(0), out.stride(0), epilogue, 0, None, 0, None)
     rc = L.lib().p3v_gemm_merge(C.byref(args), _p(ws), ws.numel(), _stream())
     if rc == L.ERR_UNSUPPORTED:
@@ -476,6 +481,8 @@ def gemm_qkv_merge(a, w, cos_t, sin_t, q_out, k_dst, v_dst, B, Lq, nh, nkv, hd, 
     if not n:
         return False
     ws = _merge_workspace(a.device, n)
+    if ws is None:
+        return False
     g = L.GemmArgs(_p(a), _p(w), 0, 0, 0, 0, M, w.shape[0], K, a.stride(0), w.stride(0), w.shape[0], EPI_NONE, 0, 0, 0)
     sp = L.QkvSplit(_p(cos_t), _p(sin_t), _p(q_out), _p(k_dst), _p(v_dst), B, Lq, nh, nkv, hd, int(past), dst_t, int(dst_off_is_past),
                     tab_t, tab_div, float(q_scale))

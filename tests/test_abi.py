@@ -78,6 +78,7 @@ def test_row_projections_check_what_they_are_given(monkeypatch):
     monkeypatch.setattr(ops, "_stream", lambda: 0)
     monkeypatch.setattr(ops, "_chk", lambda t, dtype, name: t)
     monkeypatch.setattr(ops, "_merge_ws", {})
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
 
     def rows(m, n, dtype=bf):
         return torch.empty((m, n), dtype=dtype)
