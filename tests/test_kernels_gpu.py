@@ -1125,6 +1125,32 @@ def test_gemm_merge_after_a_wait_that_gave_up(ops, request):
                 assert all(torch.equal(x, y) for x, y in zip(run(i, 1 << 22), want[i])), (late, then, i)
 
 
+def test_gemm_merge_under_a_capture_without_a_workspace_of_its_own(ops, monkeypatch):
+    """Declined, nothing launched and no workspace made: counters that a capture only records as zeroed would be those of the stream's later
+    launches.  Eager launches on that stream before and behind the capture are right."""
+    monkeypatch.setattr(ops, "_merge_ws", {})
+    a, w = g((113, 2112), 454).cuda(), g((8192, 2112), 455, 1.0 / math.sqrt(2112)).cuda()
+    qa, qw = g((67, 3072), 456).cuda(), g((9216, 3072), 457, 1.0 / math.sqrt(3072)).cuda()
+    out = [torch.zeros((113, 4096), dtype=BF16).cuda() for _ in range(3)]
+    cap = [torch.full(s, 7.0, dtype=BF16).cuda() for s in ((113, 4096), (1, 32, 67, 96), (1, 32, 72, 96), (1, 32, 96, 72))]
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for known in (False, True):
+            graph = ops.Graph()
+            graph.begin()
+            taken = ops.gemm_merge(a, w, ops.EPI_SILU_MUL, cap[0]), ops.gemm_qkv_merge(qa, qw, None, None, *cap[1:], 1, 67, 32, 32, 96, 0, 72, True)
+            cap[0][:1, :1].copy_(cap[0][1:2, :1])                # (a graph of one launch)
+            graph.end()
+            assert taken == (False, False) and bool(ops._merge_ws) == known
+            graph.launch()
+            assert ops.gemm_merge(a, w, ops.EPI_SILU_MUL, out[known])
+        assert ops.gemm_merge(a, w, ops.EPI_SILU_MUL, out[2])
+    torch.cuda.synchronize()
+    assert all(torch.all(c == 7.0) for c in cap)
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2]) and torch.isfinite(out[0].float()).all() and out[0].any()
+
+
 def test_gemm_merge_refuses(ops):
     """Shapes of the other kernels: False, nothing launched."""
     for M, N, K in ((104, 8192, 3072), (129, 8192, 3072), (128, 8192, 512), (128, 1024, 3072), (128, 16384, 3072)):
