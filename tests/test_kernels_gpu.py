@@ -832,12 +832,20 @@ def test_attention_decode_with_fused_oproj_is_bit_identical_to_two_launches(ops,
 
 
 @pytest.mark.parametrize("q4", [False, True], ids=["bf16", "q4"])
-@pytest.mark.parametrize("past,cap,n_split,dev_past", [(7000, 7168, 112, False), (9000, 9216, 24, True), (300, 384, 3, False), (33000, 33280, 24, True)])
-def test_merge_launch_with_fused_oproj_is_bit_identical_to_three_launches(ops, past, cap, n_split, dev_past, q4, nkv=32):
+@pytest.mark.parametrize("past,cap,n_split,dev_past", [(7000, 7168, 112, False), (9000, 9216, 24, True), (300, 384, 3, False), (500, 512, 8, False), (1000, 1024, 16, True), (33000, 33280, 24, True)])
+def test_merge_launch_with_fused_oproj_is_bit_identical_to_three_launches(ops, past, cap, n_split, dev_past, q4, nkv=32, rows=0):
     """k_attn_combine_o (round 6): plans whose split-KV partials are merged by a launch of their own (long contexts; 64-key tiles or
     the multi-tile streaming kernel) -- the merge launch also carries o_proj + residual (B = L = 1).  Against attention + merge + GEMV:
     attention output, residual row and caches BIT-IDENTICAL, ten launches alike, the other output buffer re-armed, the workspace
-    left all-ones."""
+    left all-ones.  rows: the attn_rows knob -- 0 keeps short caches on partials and a merge, -1 is the launcher's choice."""
+    old = ops.set_tuning("attn_rows", rows)
+    try:
+        _merge_launch_with_fused_oproj(ops, past, cap, n_split, dev_past, q4, nkv)
+    finally:
+        ops.set_tuning("attn_rows", old)
+
+
+def _merge_launch_with_fused_oproj(ops, past, cap, n_split, dev_past, q4, nkv):
     from phi_3_vision_mlx_amd.weights import mlx_quantize, q4_repack
     B, L, nh, hd, H = 1, 1, 32, 96, 3072
     T = cap
@@ -888,7 +896,7 @@ def test_short_cache_with_fused_oproj(ops, request, past, cap, nkv, q4):
     """k_attn_rows_o: one workgroup per head and the o_proj beside them, at the edges of a round of its waves (128 keys) and of the cache.  The
     same bits as k_attn_decode_rows and a GEMV; against the split form, whose maxima P is rounded against are others (2^-9) before the
     output is (2^-9): a bound on values."""
-    test_merge_launch_with_fused_oproj_is_bit_identical_to_three_launches(ops, past, cap, cap // 64, False, q4, nkv=nkv)
+    test_merge_launch_with_fused_oproj_is_bit_identical_to_three_launches(ops, past, cap, cap // 64, False, q4, nkv=nkv, rows=-1)
     nh, hd = 32, 96
     qkv, kc, vc = g((1, (nh + 2 * nkv) * hd), 90).cuda(), g((1, nkv, cap, hd), 91), g((1, nkv, hd, cap), 92)
     cos, sin = torch.rand((1, 1, hd // 2)).cuda(), torch.rand((1, 1, hd // 2)).cuda()
