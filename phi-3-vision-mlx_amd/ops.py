@@ -7,6 +7,7 @@ Each op names the MLX call site of the reference it replaces.
 import contextlib
 import ctypes as C
 import os
+import threading
 
 import torch
 
@@ -84,7 +85,13 @@ def set_tuning(name, value):
 _gemm_ws = {}     # (device index, stream handle) -> grow-only byte buffer for p3v_gemm's split-K partials
 
 
-_ws_owner = None     # (holder dict, frozen?) while a hipGraph is being built: the GRAPH owns its split-K workspace
+class _WsOwner(threading.local):
+    """(holder dict, frozen?) while this thread builds a hipGraph: the GRAPH owns its split-K workspace.  Another thread's launches run
+    beside the capture, on their own stream and in their own workspace."""
+    now = None
+
+
+_ws_owner = _WsOwner()
 
 
 @contextlib.contextmanager
@@ -94,19 +101,18 @@ def owned_gemm_workspace(holder, frozen):
     may happen under hipStreamBeginCapture, and the pointer is baked into the graph -- a request the warm-up did not size
     raises instead.  (the per-(device, stream) buffer below was first allocated on the capture's side stream,
     i.e. under capture, and a later regrow would have freed what the graph still writes to.)"""
-    global _ws_owner
-    prev, _ws_owner = _ws_owner, (holder, frozen)
+    prev, _ws_owner.now = _ws_owner.now, (holder, frozen)
     try:
         yield holder
     finally:
-        _ws_owner = prev
+        _ws_owner.now = prev
 
 
 def _gemm_workspace(device, nbytes):
     """The library never allocates (include/p3v.h): the caller owns the split-K workspace.  One grow-only torch buffer per
     (device, stream): it is live only between the two launches of one p3v_gemm call, so launches on one stream share it."""
-    if _ws_owner is not None:
-        holder, frozen = _ws_owner
+    if _ws_owner.now is not None:
+        holder, frozen = _ws_owner.now
         buf = holder.get("buf")
         if buf is None or buf.numel() < nbytes:
             if frozen:
@@ -131,8 +137,8 @@ def _merge_workspace(device, nbytes):
     """Workspace of the launches that sum their K slices themselves (p3v_gemm_merge, p3v_gemm_qkv_merge): its counters carry over from
     launch to launch, so it is theirs alone -- one per (device, stream), or the graph's own.  None under a capture that owns none: zeros
     that are only recorded are none for the launches before the first replay, and a replay may run beside the stream's own launches."""
-    if _ws_owner is not None:
-        holder, frozen = _ws_owner
+    if _ws_owner.now is not None:
+        holder, frozen = _ws_owner.now
         if holder.get("merge") is None or holder["merge"].numel() < nbytes:
             if frozen:
                 raise RuntimeError(f"merge workspace of {nbytes} bytes requested under graph capture")

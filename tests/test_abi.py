@@ -111,6 +111,32 @@ def test_row_projections_check_what_they_are_given(monkeypatch):
     assert behind(None).shape == (12, 64) and launched
 
 
+def test_a_graphs_workspace_is_its_threads_alone(monkeypatch):
+    """While one thread builds a graph in a workspace the graph owns, another thread's launches get their stream's (buffers on the CPU here)."""
+    import threading
+
+    import torch
+    from phi_3_vision_mlx_amd import ops
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_gemm_ws", {})
+    monkeypatch.setattr(ops, "_merge_ws", {})
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    dev, holder, other = torch.device("cpu"), {}, []
+
+    def ask():
+        return [f(dev, 8192).data_ptr() for f in (ops._gemm_workspace, ops._merge_workspace)]
+
+    def beside():
+        t = threading.Thread(target=lambda: other.append(ask()))
+        t.start(), t.join()
+    for frozen in (False, True):
+        with ops.owned_gemm_workspace(holder, frozen=frozen):
+            mine = ask()
+            beside()
+            assert ask() == mine == [holder["buf"].data_ptr(), holder["merge"].data_ptr()]
+    assert other[0] == other[1] == ask() and not set(other[0]) & set(mine)
+
+
 def test_library_never_allocates_or_reads_the_environment_per_launch():
     """include/p3v.h: launches never allocate or synchronise (callers pass workspaces, e.g. p3v_gemm_ws_bytes); knobs come
     from ONE table filled once (p3v_runtime.hip).  Checked on the sources and on the library's undefined symbols."""
