@@ -192,7 +192,8 @@ int p3v_gemm_resid_norm(const p3v_gemm_args_t* gemm /* host */, const uint16_t* 
  *      large problems: p3v_gemm's products, the slices' fp32 sums added in slice order by a second launch, which applies the epilogue and,
  *      with norm_w and normed [M, N] (P3V_EPI_RESID_BF16, N <= 3072; both or neither), writes RMSNorm(out) beside it, bit for bit
  *      p3v_rmsnorm's.  gemm->ws: p3v_gemm_slices_ws_bytes bytes (0: not a shape of this call), live between the two launches only.
- *      P3V_ERR_UNSUPPORTED: nothing launched, the caller runs p3v_gemm (+ p3v_rmsnorm).  out may be resid.  Graph-capturable. */
+ *      P3V_ERR_UNSUPPORTED: nothing launched, the caller runs p3v_gemm (+ p3v_rmsnorm).  out may be resid, whose rows lie ldo apart as out's
+ *      do.  Graph-capturable. */
 int64_t p3v_gemm_slices_ws_bytes(int M, int N, int K, int epilogue);
 int p3v_gemm_slices(const p3v_gemm_args_t* gemm /* host */, const uint16_t* norm_w, float eps, uint16_t* normed, void* stream);
 

@@ -422,9 +422,10 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(AttnP p) {
 typedef const __attribute__((address_space(1))) void* pf_gptr_t;
 typedef __attribute__((address_space(3))) void* pf_lptr_t;
 // The query block in place `at` of the launch order: longest first, but the second workgroup a CU gets -- dispatch goes round-robin over the CUs, so
-// it comes cu_blocks places behind the first -- in the opposite order, longest beside shortest (all of one row's heads in one group).  us, one row
-// of 32 heads x 96, 64 queries a workgroup: 576 and 640 tokens unchanged, 768 19.1 -> 18.5, 1024 23.8 -> 22.7.  (k_attn_prefill_il waits for its longest
-// workgroup whoever shares the CU: 54.3 us at 2531 tokens either way.)
+// it comes cu_blocks places behind the first -- in the opposite order, longest beside shortest (all of one row's heads in one group).  us without and
+// with it, one row of 32 heads x 96: pre-scaled prompts, which come here up to 767 tokens, 576 16.1 : 16.1, 640 17.5 : 17.2, 704 18.5 : 18.1,
+// 767 19.6 : 19.1; plain queries up to 3071, 1024 23.9 : 23.0, 1500 35.2 : 33.8, 2531 71.3 : 70.3, 2900 81.2 : 81.2.  (k_attn_prefill_il waits for its
+// longest workgroup whoever shares the CU: 54.3 us at 2531 tokens either way.)
 __device__ __forceinline__ int query_block(const AttnP& p, int at, int nqb) {
   const int n = p.cu_blocks;
   if (n && at >= n && at < 2 * n) at = n + min(2 * n, nqb) - 1 - at;
@@ -1275,7 +1276,8 @@ static int launch_attn_prefill(const AttnP& p, hipStream_t s) {
     // Which kernel for a pre-scaled prompt (tools/attn_il4_probe.py, 32 heads x 96, causal, us; dma / il 4 waves / il 8 waves):
     //   B = 1:  512: 15.9 / 16.4 / 22.2   768: 21.1 / 20.1 / 26.6   1280: 32.3 / 27.1 / 34.8   2531: 64.6 / 52.6 / 58.8
     //           (with 64 queries a workgroup, dma / il 4 waves: 768: 18.5 / 21.7   1024: 22.7 / 25.8   1280: 28.6 / 30.1   1408: 31.2 / 31.9   1472: 32.6 / 32.0.
-    //            Not taken up: the two round differently, which 32 layers of 8-bit activations carry to 6 % of a logit, either 5 % from 64 bits)
+    //            Not taken up: the two round differently, which in a prompt of 8-bit activations 32 layers carry to 6 % of a logit, either 5 % from
+    //            64 bits, and nothing here tells such a prompt from one of 16-bit activations, to which that does not apply)
     //           3072: 81.4 / 74.6 / 69.5   4096: 119 / 114 / 108    8192: 436 / 403 / 377
     //   B = 2:  1280: 40.0 / 36.5 / 40.3   2531: 91.8 / 99.8 / 106   4096: 221 / 219 / 228   5120: 343 / 320 / 328
     //   B = 4:  2531: 168 / 183 / 190      3072: 252 / 254 / 271   4096: 426 / 410 / 418   6144: 939 / 886 / 893   8192: 1614 / 1504 / 1477

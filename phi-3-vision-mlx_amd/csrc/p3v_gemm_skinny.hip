@@ -9,7 +9,8 @@
 //             HBM, and in one CU the two add up -- the same requests without any compute take as long as gate_up, 30 us at 128
 //             rows (rows 6144 bytes apart; weights alone 18.5, both packed 25.9: profiles/lds_dma_probe.txt).  Rows of A and W 128 bytes further apart: gate_up 30.2 ->
 //             27.7, qkv 26 -> 24.3, but down 22.6 -> 25.4; the weights lie unpadded, as the other kernels and the loader have them.
-//             128 x 128 tiles (W x 2 staged, half the workgroups) were not faster on any shape (the template keeps the variant).
+//             128 x 128 tiles (W x 2 staged, half the workgroups) in one pass or with partials in memory were not faster on any shape; where
+//             the K slices that fill the chip again are summed inside the launch they are (p3v_gemm_merge, at the end).
 //   staging   LDS-DMA into a ring of 6 stages (A 16 KiB + W 8 KiB each), 5 in flight behind a counted vmcnt; one workgroup per CU
 //             (<= 64 rows: 64-row tiles, A 8 KiB per stage -- a third less staged per K-tile, the same sums bit for bit: 60 -> 53 us
 //             per decoder layer at 17 rows)
@@ -25,7 +26,7 @@
 
 #define SK_BM 128
 #define SK_BK 64
-#define SK_TN 64                    // tile width of the one-pass and partial-sum forms (TN = 128: measured, not faster -- see the header; MERGE takes it)
+#define SK_TN 64                    // tile width of the one-pass and partial-sum forms (MERGE: 128)
 #ifndef SK_ABL
 #define SK_ABL 0                    // timing experiments: 1 = A always K-tile 0 (one L2/L1-hot tile), 2 = W likewise, 3 = no MFMAs after K-tile 0
 #endif

@@ -13,7 +13,8 @@
 // One row (k_gemv3_q4): x (+RMSNorm) staged in LDS while the weights of the wave's first U row pairs are on their way, their sums and their
 // epilogue together at the end.  The bytes (N*K/2 + N*K/16) are a quarter of the bf16 kernel's for as many products, so its instructions count as much as
 // its bytes: 11 per 8 weights, 6 per piece, and one reduction and epilogue per U pairs instead of one each (gate_up: 880 vector instructions a
-// wave, 3 of its 8 us; 1180 before).  16 waves per CU: 4.08 ms per four steps of the 32-layer decoder at 128 columns (8 waves 4.11, 12 4.14, 20 4.12; before 4.52):
+// wave, 3 of its 8 us; 1180 before).  16 waves per CU: with attention and o_proj as two launches 4.08 ms per four steps of the 32-layer decoder at 128
+// columns (8 waves 4.11, 12 4.14, 20 4.12; before 4.52; 3.9 with the two as one, k_attn_rows_o):
 // per launch gate_up 9.0 -> 8.1 us, qkv 7.2 -> 6.6, down 7.1 -> 5.9.
 #include <stdlib.h>
 
