@@ -4,7 +4,7 @@
  * tensor op on its hot path is a call into the third-party `mlx` wheel.  Each
  * entry point below therefore replaces one MLX call site (or a fused group of
  * them) in the reference's `phi.py` / `phi_3_vision_mlx.py`; the call site is
- * cited as file:line next to each declaration (see SURVEY.md section 2.3).
+ * cited as file:line next to each declaration.
  *
  * Conventions
  *   - plain pointers and sizes only; all pointers are DEVICE pointers unless
@@ -141,7 +141,7 @@ typedef struct {
 int p3v_gemv_fp8(const p3v_gemv_fp8_args_t* args /* host */, void* stream);
 int p3v_dequant_fp8(const uint8_t* w8, const float* w_scale, uint16_t* out_bf16, int rows, int K, void* stream);
 
-/* ---- W8A8 projection on the fp8 matrix cores (BASELINE config 5, prompt-sized inputs; the same call sites:
+/* ---- W8A8 projection on the fp8 matrix cores (prompt-sized inputs; the same call sites:
  * QuantizedLinear, phi_3_vision_mlx.py:264,291-305, under `quantize_model=True`).
  *   out[M, N] = epilogue((a_scale[m] * w_scale[n]) * sum_k A8[m,k] * W8[n,k])     A8 [M, lda], W8 [N or 2N, ldw]: e4m3 bytes
  * on v_mfma_scale_f32_16x16x128_f8f6f4 (block scales 1.0).  epilogue: P3V_EPI_NONE, P3V_EPI_RESID_BF16 (resid bf16 [M, ldo]),
@@ -249,7 +249,7 @@ int p3v_gemm_qkv_fp8_pays(int M, int n_q, int n_kv, int K);      /* 1: faster th
  * appended to the cache).  V^T columns beyond the valid keys must hold finite values.
  * out [B, L, nh*hd] bf16.
  * Query i sees key t iff (!causal || t <= past+i) && t >= pad_len[b]; a query
- * that is itself padding outputs 0 (SURVEY.md App. A Q7).  hd in {64, 96}. */
+ * that is itself padding outputs 0.  hd in {64, 96}. */
 typedef struct {
   const uint16_t* q;
   const uint16_t* k_past; const uint16_t* v_past;

@@ -10,10 +10,10 @@ Host code stays Python; everything that touches the device goes through
 
 `quantize_cache=True` selects the int8 KV cache and `quantize_model=True` fp8 (e4m3) decoder weights (or the reference's
 own 4-bit group-64 format: an MLX `*_Q` checkpoint directory if present, or `quantize_format="int4"`) -- the build's
-analogues of the reference's 4-bit prompt cache / int4 weights (BASELINE config 5).
+analogues of the reference's 4-bit prompt cache / int4 weights.
 `use_adapter=True` attaches the LoRA adapter of `adapters/<model dir name>` (or `adapter_path=...`) at inference
 (reference phi_3_vision_mlx.py:266-271); training adapters is not part of this build.
-Not carried over (out of scope, SURVEY.md section 2): the `<|api_input|>` tool hook,
+Not carried over (out of scope): the `<|api_input|>` tool hook,
 HF-hub download (`_setup`): a model directory must exist locally, or pass
 `synthetic=...` to `load()` for seeded random weights of the real architecture.
 """

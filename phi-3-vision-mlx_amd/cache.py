@@ -33,7 +33,7 @@ class CacheState:
         # cache_format="mlx4" (opt-in): the reference's OWN quantised cache -- MLX 4-bit group-32 codes of the PROMPT's K / V, later
         # tokens unquantised (phi.py:528-540).  The codes are kept in the reference's format (k4 / v4 + scale | bias), and the
         # bf16 cache rows hold their dequantised values, which is what every later call of the reference attends on: the decode
-        # path is then the plain bf16 one.  (Default for quantize_cache=True: int8 for all tokens, BASELINE config 5.)
+        # path is then the plain bf16 one.  (Default for quantize_cache=True: int8 for all tokens.)
         self.mlx4 = self.quantized and getattr(cfg, "cache_format", "int8") == "mlx4"
         if self.quantized and getattr(cfg, "cache_format", "int8") not in ("int8", "mlx4"):
             raise ValueError(f"cache_format must be 'int8' or 'mlx4', got {cfg.cache_format!r}")

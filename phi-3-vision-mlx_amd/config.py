@@ -1,7 +1,7 @@
 """Model configuration for the Phi-3-Vision / Phi-3-mini-128K hot path.
 
 Mirrors what the reference reads from ``config.json`` into a SimpleNamespace
-(reference phi_3_vision_mlx.py:359-363, keys listed in SURVEY.md App. B).
+(reference phi_3_vision_mlx.py:359-363).
 The rope factor arrays are the Phi-3-vision-128k-instruct values printed in the
 reference's own notebook (assets/su_rope_explained.ipynb, cell 9); a real
 ``config.json`` always overrides them.

@@ -1881,7 +1881,7 @@ __device__ __forceinline__ void attn_decode_body(const AttnDecP& p, const int bx
 // many partials.  LDS image: [K slice of wave 0..3: 32 keys x 192 B, chunk c of row r at c ^ ((r >> 2) & 3)]
 // [V^T tile: 96 rows x 256 B, chunk c (of 16) of row d at c ^ (d & 15): the 16 rows x 2 key groups of a ds_read_b64 lane
 // group hit 32 different 8-byte slots].  The merge scratch aliases the (dead) tile region.
-// Schedule (the "V2" of profiles/ and DESIGN.md; V1, the same kernel without it, is in the history): the per-workgroup timeline (-DP3V_ATTN_TIMING,
+// Schedule (the "V2" of profiles/; V1, the same kernel without it, is in the history): the per-workgroup timeline (-DP3V_ATTN_TIMING,
 // tools/attn_timeline.py) showed that everything after the DMA issue ran AFTER the whole tile had landed: memory
 // returns in order, and the compiler answers a pending `global_load_lds` with vmcnt(0) at every later wait.  V2 issues the
 // tile as `buffer_load ... lds` (counted waits stay possible), AFTER the small loads of the new rows, and hides from the
@@ -2941,7 +2941,7 @@ extern "C" int p3v_attention_decode_can_fuse_oproj(int B, int L, int n_heads, in
   if ((long)(n_split - 1) * n_heads * 8 < o_n) return 0;
   // every workgroup of the launch must be resident at once (the projecting ones wait for the merging ones): ask the runtime how
   // many of THIS kernel fit a CU rather than assume the 3 that its 52 KB of LDS and ~100 VGPRs give today
-  // (cached PER DEVICE: ADVICE r04 -- a process-wide value was whatever the first device that asked had)
+  // (cached PER DEVICE: a process-wide value would be whatever the first device that asked had)
   static long capacity_of[P3V_MAX_DEVICES] = {0};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= P3V_MAX_DEVICES) return 0;
@@ -3063,8 +3063,8 @@ extern "C" int p3v_attention_decode(const p3v_attn_decode_args_t* a, void* strea
 }
 
 // =====================================================================================
-// int8 KV cache (quantize_cache=True; BASELINE config 5; replaces the reference's 4-bit group-32 prompt
-// cache, phi.py:528-540, SURVEY.md App. A Q12): K rows and V^T columns are stored as offset-binary bytes
+// int8 KV cache (quantize_cache=True; replaces the reference's 4-bit group-32 prompt
+// cache, phi.py:528-540): K rows and V^T columns are stored as offset-binary bytes
 // u = round(x / s) + 128 with one fp32 scale s per (batch row, kv head, token); halves the bytes a decode
 // step streams.  As in the reference, the PREFILL attends over the exact keys/values and only the
 // stored copy is quantised (phi.py:531-533); a decode step attends over the dequantised cache plus its

@@ -1,5 +1,5 @@
-// fp8 (OCP e4m3fn) weight-only projections for the decode path (quantize_model=True; BASELINE config 5;
-// replaces the reference's int4 group-64 `nn.quantize`, phi_3_vision_mlx.py:264,296 -- SURVEY.md K23).
+// fp8 (OCP e4m3fn) weight-only projections for the decode path (quantize_model=True;
+// replaces the reference's int4 group-64 `nn.quantize`, phi_3_vision_mlx.py:264,296).
 // Weights: u8 [N, K] e4m3 bit patterns, one fp32 scale per output row (w = fp8 * scale[n]); activations stay
 // bf16 and all accumulation is fp32, so the only new error is the weight rounding.  A decode step then
 // streams half the bytes: the kernels below are the fp8 twins of k_gemv3 / k_gemv_mfma in p3v_gemv.hip.

@@ -64,7 +64,7 @@ class DecoderModel:
         are mid-generation.  All rows start empty (pad_len = window: every key masked).  The window fixes the RoPE regime
         of every row (phi.py:492: one choice per call from prompt + max_tokens): window <= 4096 -> short factors, beyond
         -> long factors; the engine admits only requests that would pick the same factors alone.  With
-        `quantize_cache=True` the rows keep the int8 KV cache (BASELINE config 5)."""
+        `quantize_cache=True` the rows keep the int8 KV cache."""
         st = self._new_state(slots, 0, window, None, None, shared_tables=False)
         st.pad_len = torch.full((slots,), window, dtype=I32, device=self.device)
         st.slots = True
@@ -196,7 +196,7 @@ class DecoderModel:
         Returns (logits [B, L', V] in the model's activation type, cache).  On a prefill call (cache is None)
         only the last position is projected through lm_head (L' = 1) unless
         `full_logits=True`: every caller in the reference reads `logits[:, -1]`
-        of a prefill only (SURVEY.md App. A Q8); cached calls return all L rows."""
+        of a prefill only; cached calls return all L rows."""
         cfg = self.cfg
         if torch.is_tensor(input_ids):
             ids = input_ids.to(self.device, I32)
@@ -248,7 +248,7 @@ class DecoderModel:
 
     def _prefill_captured(self, ids, S, max_tokens):
         """Short text prompts (B = 1, 17 .. 512 tokens) are launch-bound: ~390 launches of a few microseconds each, every one paid
-        for in Python + ctypes time (4.5 ms of wall time for 3.6 ms of kernels).  A (length, max_tokens) pair seen
+        for in Python + ctypes time (128 tokens: 4.5 ms of wall time for 3.6 ms of kernels).  A (length, max_tokens) pair seen
         for the SECOND time is captured as ONE hipGraph over buffers the entry owns -- ids, activations, rotation tables, the KV
         cache itself -- and later prompts of that geometry cost one 0.5 KB copy + one graph launch.  The entry's cache is LEASED to
         the caller: every call gets its own CacheState object (a shallow copy of the entry's: same tensors, same decode graphs, its

@@ -1,4 +1,4 @@
-"""Batch sharding over the GPUs of one node (SURVEY.md section 8e).
+"""Batch sharding over the GPUs of one node.
 
 The reference has no distributed code; sequences never interact (per-row mask and
 position ids, reference phi.py:238-239, 553-559), so the path shards by REQUEST:
@@ -235,7 +235,7 @@ def _all_max(value, group=None):
 
 def generate_sharded(prompts, images=None, preload=None, max_tokens=512, group=None, max_batch=8, apply_chat_template=True,
                      return_tokens=False):
-    """Batched `generate()` over all ranks -- BASELINE config 4 (mixed image + text requests).
+    """Batched `generate()` over all ranks (mixed image + text requests).
 
     `prompts`: list of str.  `images`: None, or a list with one entry (an image / path / URL as `generate` takes it, or
     None) per prompt.  Rank 0's request table is broadcast (`broadcast_requests`: text + decoded RGB pixels as one uint8 tensor, ~340 KB per 336x336 image);

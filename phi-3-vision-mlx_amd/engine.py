@@ -1,4 +1,4 @@
-"""Continuous batching at decode-step granularity (SURVEY.md 8f item 1; the reference has none: its server runs one
+"""Continuous batching at decode-step granularity (the reference has none: its server runs one
 `generate` per HTTP request, server.py:17).
 
 One GPU, one captured decode graph over a fixed number of SLOTS (batch rows).  Every row has its own left padding and
@@ -17,7 +17,7 @@ RoPE regime (phi.py:492: ONE short/long factor choice per call, from prompt + ma
 serves ONE regime: `window <= 4096` -> short factors and only requests with S + max_tokens <= 4096 (what each of them
 alone would pick); `window > 4096` -> long factors and only requests with S + max_tokens > 4096.  `RegimeRouter` puts
 one engine of each kind behind a single `submit` and steps both from one thread.  With `quantize_cache=True` models the
-slot state keeps the int8 KV cache of BASELINE config 5 (`model.new_slot_state`).
+slot state keeps the int8 KV cache (`model.new_slot_state`).
 
 Admission is FIFO with bounded overtaking: a request that does not fit the current column is skipped by newer ones for
 at most `patience` decode steps; after that nothing newer is admitted, the engine drains, and the column moves to the

@@ -1,7 +1,7 @@
-"""Continuous-batching engines composed with the batch-sharded deployment: one process per GPU, weights replicated
-(BASELINE.json north_star), every rank stepping its OWN engine.ContinuousEngine (or RegimeRouter); rank 0 owns the request
+"""Continuous-batching engines composed with the batch-sharded deployment: one process per GPU, weights replicated,
+every rank stepping its OWN engine.ContinuousEngine (or RegimeRouter); rank 0 owns the request
 surface (the HTTP handler's `submit`) and hands each request to the rank with the fewest requests outstanding.  This is
-SURVEY.md 8 row f1's "request queue feeding the batch-sharded engine" for the continuous engine (the one-shot path is
+the request queue feeding the batch-sharded engine for the continuous engine (the one-shot path is
 dist.generate_sharded); the reference has no counterpart (its server.py serves one process).
 
 No data-path collective: a request is independent of every other one, so the only traffic between ranks is the request itself

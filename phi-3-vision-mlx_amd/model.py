@@ -17,9 +17,8 @@ HBM layout
                k-contiguous MFMA operands for QK^T and PV with plain 16-byte loads
   RoPE tables  fp32 cos/sin [B, T, hd/2] built once per prompt (one short/long choice, Q2)
   residual     decoder: bf16 [B*L, H]; ViT: fp32 [crops, 577, 1024]
-Dtype flow differs from the reference only where stated in DESIGN.md
-(bf16 K cache / bf16 MFMA operands instead of fp32 attention), within the
-tolerance the parity tests state.
+Dtype flow differs from the reference only in attention (bf16 K cache and
+bf16 MFMA operands instead of fp32), within the tolerance the parity tests state.
 """
 import math
 import os

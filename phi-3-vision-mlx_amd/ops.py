@@ -99,8 +99,8 @@ def owned_gemm_workspace(holder, frozen):
     """Route every split-K workspace request inside the block to `holder["buf"]` (a dict the caller keeps alive as long as the
     graph).  frozen=False (the warm-up run): the buffer is allocated / grown as needed.  frozen=True (the capture): no allocation
     may happen under hipStreamBeginCapture, and the pointer is baked into the graph -- a request the warm-up did not size
-    raises instead.  (the per-(device, stream) buffer below was first allocated on the capture's side stream,
-    i.e. under capture, and a later regrow would have freed what the graph still writes to.)"""
+    raises instead.  (The per-(device, stream) buffer below would be allocated on the capture's side stream, i.e. under
+    capture, and a later regrow would free what the graph still writes to.)"""
     prev, _ws_owner.now = _ws_owner.now, (holder, frozen)
     try:
         yield holder

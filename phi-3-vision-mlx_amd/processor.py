@@ -7,7 +7,7 @@ Outputs are NumPy arrays (the model object moves them to the GPU); with
 ``return_mx`` kept only for signature compatibility.
 
 `Phi3VImageProcessor` reproduces the reference bit for bit, including the
-degenerate two-tap "bicubic" global crop -- but the
+degenerate two-tap "bicubic" global crop (phi.py:365-371) -- but the
 reference's 4-deep Python loop over 336x336x3 pixels (phi.py:365-371, ~5.6 s
 per image) is evaluated as four vectorised gathers with the identical
 floating-point association, see `interpolate_336`.
@@ -196,7 +196,7 @@ def collate_requests(requests, width=None):
     """B = 1 model inputs (`processor(text)` / `processor(text, images)` results) -> ONE left-padded batch.
 
     The reference batches text prompts only (`_tokenize`, phi.py:233-245) and runs image prompts at B = 1
-    (phi_3_vision_mlx.py:377-378, `_merge` phi.py:276); BASELINE config 4 batches mixed image + text requests, so the
+    (phi_3_vision_mlx.py:377-378, `_merge` phi.py:276); a served batch mixes image + text requests, so the
     batch is built with `_tokenize`'s own conventions -- left pad with id 0, position id 1 and mask 0 on the pad,
     positions 0..n-1 on the tokens -- and every image's slot positions move to (batch row, column + pad).  A row of the
     batch then sees exactly what its B = 1 run sees (pad keys get zero weight, Q7), which is what the parity tests check."""

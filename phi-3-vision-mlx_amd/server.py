@@ -9,7 +9,7 @@
      a byte cap and a pixel cap -- never on the engine thread -- and errors never echo the path.)
 
 with one difference in the plumbing: requests do not call the model from the HTTP thread.  They go into a queue that a
-single engine thread drains (the model object holds one in-flight sequence group, SURVEY.md 8b).  By default every
+single engine thread drains (the model object holds one in-flight sequence group).  By default every
 request is its own `generate` call, as in the reference's server -- a client's output never depends on who else is in
 flight.  `merge=True` (opt-in, `--merge`) folds requests that wait at the same time and ask for the same `max_tokens`
 into ONE batched call: throughput for left-pad geometry that now depends on the longest co-batched prompt (results of

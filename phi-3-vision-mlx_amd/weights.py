@@ -1,5 +1,5 @@
 """Weight tables for the hot path: names/shapes in the HF layout the reference
-loads (reference phi_3_vision_mlx.py:371-374; SURVEY.md App. B), a seeded
+loads (reference phi_3_vision_mlx.py:371-374), a seeded
 synthetic generator that is bit-identical on CPU and GPU, and a safetensors
 directory loader.
 
@@ -252,7 +252,7 @@ def synth_weights(cfg, seed=0, device="cpu", std_scale=1.0, lm_head_spread=0.0, 
     residual_scale: the WELL-CONDITIONED checkpoint of the parity tests -- the decoder's residual-branch output
     projections (o_proj, down_proj) times this factor (True = 1 / sqrt(2 * n_layers), the usual depth-scaled initialisation).
     With plain N(0, 0.02) everywhere each of the 32 layers adds a branch as large as the stream itself and a single bf16
-    rounding grows to ~6 % of the logits (DESIGN.md section 4); depth-scaled, the stream is dominated by the embedding and the
+    rounding grows to ~6 % of the logits; depth-scaled, the stream is dominated by the embedding and the
     error of two correct implementations stays near 1 %."""
     w = {n: synth_tensor(n, s, k, seed, device, std_scale) for n, s, k in weight_specs(cfg)}
     if residual_scale:
