@@ -528,7 +528,7 @@ static int launch_merge(SkinnyP p, const MergePlan& pl, void* ws, hipStream_t s)
     if (hipFuncSetAttribute((const void*)k_gemm_skinny<EPI, false, 128, SK_BM, true>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS) != hipSuccess) return P3V_ERR_HIP;
     attr_set = true;
   }
-  p.xflag = (unsigned*)ws, p.xpart = (float*)((unsigned char*)ws + SK_MERGE_FLAGS), p.nk_part = pl.nk_part, p.polls = (unsigned)max(p3v_tuning().gemm_merge_polls, 0);
+  p.xflag = (unsigned*)ws, p.xpart = (float*)((unsigned char*)ws + SK_MERGE_FLAGS), p.nk_part = pl.nk_part, p.polls = p3v_tuning().gemm_merge_polls < 0 ? 1u << 22 : (unsigned)p3v_tuning().gemm_merge_polls;
   hipLaunchKernelGGL((k_gemm_skinny<EPI, false, 128, SK_BM, true>), dim3(pl.tiles, 1, pl.S), dim3(512), C::LDS, s, p);
   P3V_CHECK_LAUNCH();
   return P3V_OK;

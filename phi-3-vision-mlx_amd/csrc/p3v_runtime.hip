@@ -46,7 +46,7 @@ const Knob kKnobs[] = {
     {"gemm_no_skinny", &P3vTuning::gemm_no_skinny, 0},      {"gemm_skinny_max_m", &P3vTuning::gemm_skinny_max_m, 256},
     {"gemm_skinny_s", &P3vTuning::gemm_skinny_s, 0},            {"gemm_skinny_tm128", &P3vTuning::gemm_skinny_tm128, 0},
     {"gemm_no_merge", &P3vTuning::gemm_no_merge, 0},        {"gemm_slices", &P3vTuning::gemm_slices, -1},
-    {"gemm_merge_polls", &P3vTuning::gemm_merge_polls, 1 << 22}, {"gemm_qkv_flat", &P3vTuning::gemm_qkv_flat, -1},
+    {"gemm_merge_polls", &P3vTuning::gemm_merge_polls, -1}, {"gemm_qkv_flat", &P3vTuning::gemm_qkv_flat, -1},
     {"gemm_rows", &P3vTuning::gemm_rows, 1},              {"gemm_tile", &P3vTuning::gemm_tile, -1},
     {"mix_wgs", &P3vTuning::mix_wgs, 0},
     {"attn_rows", &P3vTuning::attn_rows, -1},               {"attn_dma_u", &P3vTuning::attn_dma_u, -1},

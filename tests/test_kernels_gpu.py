@@ -1106,7 +1106,7 @@ def test_gemm_merge(ops, M, N, K, epi):
 def test_gemm_merge_after_a_wait_that_gave_up(ops, request):
     """A launch whose waits give up at once (no look at the counters allowed: every kernel exits as ever) is NaN throughout, and the launches
     behind it on the same workspace, of the same number of slices or another, are right: late partials are never counted for theirs."""
-    polls = ops.set_tuning("gemm_merge_polls", 1 << 22)
+    polls = ops.set_tuning("gemm_merge_polls", -1)
     request.addfinalizer(lambda: ops.set_tuning("gemm_merge_polls", polls))
     calls = []
     for M, N, K in ((113, 4096, 2112), (128, 8192, 3072)):       # 4 and 2 slices
@@ -1123,14 +1123,14 @@ def test_gemm_merge_after_a_wait_that_gave_up(ops, request):
         out = calls[i][1]()
         assert calls[i][0](out), "shape not taken"
         return [t[:, :, :67] if i == 2 and t.shape[2] == 72 else t[..., :67] if i == 2 and t.shape[3] == 72 else t for t in out]
-    want = [run(i, 1 << 22) for i in range(3)]
+    want = [run(i, -1) for i in range(3)]
     assert all(torch.isfinite(t.float()).all() for o in want for t in o)
     for late, then in ((0, 0), (1, 1), (2, 2), (0, 2), (2, 1), (1, 0)):
         for _ in range(2):
             assert all(torch.isnan(t.float()).all() for t in run(late, 0))
         for i in (then, late):
             for _ in range(2):
-                assert all(torch.equal(x, y) for x, y in zip(run(i, 1 << 22), want[i])), (late, then, i)
+                assert all(torch.equal(x, y) for x, y in zip(run(i, -1), want[i])), (late, then, i)
 
 
 def test_gemm_merge_under_a_capture_without_a_workspace_of_its_own(ops, monkeypatch):
