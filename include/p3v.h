@@ -100,9 +100,11 @@ typedef struct {
  * is only live between the two launches of one call, so calls on ONE stream may share it; concurrent streams need their
  * own.  Graph-capturable. */
 int p3v_gemm(const p3v_gemm_args_t* args /* host */, void* stream);
-/* The tile p3v_gemm runs a prompt-sized problem on in one launch (host query): 10 mb + nb for 32 mb rows x 64 nb columns of W, 0: rows split
- * between 256 x 256 and 128 x 128 tiles, or one of the kernels for few rows (they come first, up to 256 rows) */
+/* The tile of a prompt-sized problem in one launch (host queries): 10 mb + nb for 32 mb rows x 64 nb columns of W, 0: rows split between 256 x 256
+ * and 128 x 128 tiles, or one of the kernels for few rows (they come first, up to 256 rows).  p3v_gemm_plan: by whole rounds of the chip, without
+ * the tiles of 192 rows; p3v_gemm_tile: what p3v_gemm runs, by how full the rounds are as well */
 int p3v_gemm_plan(int M, int N, int K, int epilogue);
+int p3v_gemm_tile(int M, int N, int K, int epilogue);
 int64_t p3v_gemm_ws_bytes(int M, int N, int K, int epilogue);
 /* 9 .. 32 rows of A on bf16 weights with K = 3072 or 8192 (a 9 .. 32-sequence decode batch; the reference's batched benchmark
  * runs 15, phi_3_vision_mlx.py:1226-1243) take a register-streaming kernel inside p3v_gemm / p3v_gemm_resid_norm (weights HBM ->

@@ -63,14 +63,45 @@ __device__ __forceinline__ float p3v_sigmoid(float x) { return __builtin_amdgcn_
 //  SiLU: every intermediate rounded to bf16, as the reference's array expression rounds it (phi.py:469-471)
 //  GELU (tanh form): 0.5 g (1 + tanh(sqrt(2/pi) (g + 0.044715 g^3))) in fp32 = g sigmoid(2 u): no cancellation for any g
 #define P3V_GATED(epi) ((epi) == P3V_EPI_SILU_MUL || (epi) == P3V_EPI_GELU_MUL)
+// n / (1 + e) for e = an exponential, 0 .. inf, as a quarter of n / (1/4 + e/4), whose reciprocal the hardware does not flush: a Newton step on
+// that reciprocal is within an ulp and gives a SiLU the same 16 bits as the IEEE quotient for each of the 65536 values that its gate, rounded to
+// 16 bits, can have; with n, a second step on the quotient.  (The compiler's own division takes 11 instructions, two of them transcendental; the
+// gated epilogue of 256 x 256 tiles, 128 outputs a lane on one wave per SIMD, goes from 28 to 20 an output.)
+__device__ __forceinline__ float p3v_rcp_1p(float e) {
+  const float d = fmaf(e, 0.25f, 0.25f);
+  float y = __builtin_amdgcn_rcpf(d);
+  y = fmaf(fmaf(-d, y, 1.f), y, y);
+  return 0.25f * __builtin_amdgcn_div_fixupf(y, d, 1.f);
+}
+__device__ __forceinline__ float p3v_div_1p(float n, float e) {
+  const float d = fmaf(e, 0.25f, 0.25f);
+  float y = __builtin_amdgcn_rcpf(d);
+  y = fmaf(fmaf(-d, y, 1.f), y, y);
+  float q = n * y;
+  q = fmaf(fmaf(-d, q, n), y, q);
+  return 0.25f * __builtin_amdgcn_div_fixupf(q, d, n);
+}
 __device__ __forceinline__ float p3v_gelu_tanh(float g) {
   const float u = 0.7978845608028654f * (g + 0.044715f * g * g * g);
-  return g / (1.f + __expf(-2.f * u));
+  return p3v_div_1p(g, __expf(-2.f * u));
 }
 __device__ __forceinline__ float p3v_gated(int epi, float gate, float up) {
   if (epi == P3V_EPI_GELU_MUL) return p3v_gelu_tanh(gate) * up;
   const float g = bf16_round(gate), u = bf16_round(up);
-  return bf16_round(g * bf16_round(1.f / (1.f + __expf(-g)))) * u;
+  return bf16_round(g * bf16_round(p3v_rcp_1p(__expf(-g)))) * u;
+}
+// two outputs, rounded and packed: the same bits, the roundings in pairs (the empty asm keeps the compiler from taking the pairs apart again)
+__device__ __forceinline__ uint32_t p3v_round2(float lo, float hi) {
+  uint32_t w = pack_bf16x2(lo, hi);
+  asm("" : "+v"(w));
+  return w;
+}
+__device__ __forceinline__ uint32_t p3v_gated2(int epi, float gate0, float gate1, float up0, float up1) {
+  if (epi == P3V_EPI_GELU_MUL) return pack_bf16x2(p3v_gelu_tanh(gate0) * up0, p3v_gelu_tanh(gate1) * up1);
+  const uint32_t g = p3v_round2(gate0, gate1), u = p3v_round2(up0, up1);
+  const uint32_t s = p3v_round2(p3v_rcp_1p(__expf(-bf16lo(g))), p3v_rcp_1p(__expf(-bf16hi(g))));
+  const uint32_t a = p3v_round2(bf16lo(g) * bf16lo(s), bf16hi(g) * bf16hi(s));
+  return pack_bf16x2(bf16lo(a) * bf16lo(u), bf16hi(a) * bf16hi(u));
 }
 
 // nn.RMSNorm = mx.fast.rms_norm (phi.py:478-479, 571): w * astype(x * rsqrt(mean x^2 + eps), bf16) -- the normalised value is
@@ -167,13 +198,13 @@ static inline int p3v_gemv_wpw(int waves, int n_cu, int forced) {
 // it): no launch reads the environment.  -1 = "let the launcher decide".
 struct P3vTuning {
   int gemm_big_rows;        // rows given to the 256x256-tile GEMM (-1: cost model)
-  int gemm_tile;            // 10 mb + nb: pin the tile of the large GEMM (32 mb x 64 nb); -1: cost model
+  int gemm_tile;            // 10 mb + nb: pin the tile of the large GEMM (32 mb x 64 nb; of 192 rows: 164, 163); -1: cost model
   int gemm_no_splitk, gemm_splitk_max_m, gemm_splitk_max_s, gemm_splitk_wgs, gemm_128, gemm_persistent;
   int gemm_rows;            // 1: 9 .. 32 rows on the register-streaming kernel (p3v_gemm_rows.hip), 0: on the 64-row tiles of p3v_gemm_skinny.hip
   int gemm_no_skinny, gemm_skinny_max_m, gemm_skinny_s, gemm_skinny_tm128, gemm_no_merge;   // the 128 x 64-tile weight-streaming kernel for 17 .. max_m rows (p3v_gemm_skinny.hip)
   int gemm_merge_polls;     // p3v_gemm_merge, p3v_gemm_qkv_merge: looks at a counter before a wait is given up; -1: 2^22 (seconds); tests: 0
   int gemm_slices;          // p3v_gemm_slices: -1: by shape, 0: never, 100 S + 10 mb + nb: S slices of K on tiles of 32 mb x 64 nb
-  int gemm_qkv_flat;        // p3v_gemm_qkv on tiles of 32 x gemm_qkv_flat rows (2 .. 5): -1: by shape, 0: never
+  int gemm_qkv_flat;        // p3v_gemm_qkv on tiles of 32 x gemm_qkv_flat rows (2 .. 8): -1: by shape, 0: never
   int gemm_no_qkv_fuse;     // 1: p3v_gemm_qkv reports P3V_ERR_UNSUPPORTED (callers then run p3v_gemm + p3v_rope_kv_append)
   int gemm_f8_narrow;       // tile of the fp8 GEMM: -1: by shape, 0 / 1: 256 / 128 columns, 10 mb + nb: 32 mb x 64 nb
   int attn_no_dma, attn_old, attn_pp, attn_il, attn_il_waves, combine_g, kvq_old, q8_old;

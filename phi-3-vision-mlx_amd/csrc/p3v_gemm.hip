@@ -208,10 +208,8 @@ __global__ void __launch_bounds__(256, 2) k_gemm(GemmP p) {
       uint32_t pk[2][2];
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        float o4[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o4[r] = p3v_gated(EPI, acc[i][j][r], acc[i][2 + j][r]);
-        pk[j][0] = pack_bf16x2(o4[0], o4[1]), pk[j][1] = pack_bf16x2(o4[2], o4[3]);
+        for (int h = 0; h < 2; ++h) pk[j][h] = p3v_gated2(EPI, acc[i][j][2 * h], acc[i][j][2 * h + 1], acc[i][2 + j][2 * h], acc[i][2 + j][2 * h + 1]);
       }
       u32x4_t w;
 #pragma unroll
@@ -326,8 +324,7 @@ static int gemm128(const p3v_gemm_args_t* a, hipStream_t s);
 // per round; a round of big tiles costs 1, a round of small ones 0.675 (half the output area at 0.97 vs 1.31
 // PFLOP/s), a last round that leaves every CU at most one small workgroup 0.42 -- pick the cheapest whole-round
 // packing, e.g. 2531 x 16384 (gate_up): 8 x 64 = 512 big tiles = 2 rounds + 4 x 128 small = 1 round.
-static int gemm_big_rows(const p3v_gemm_args_t* a, float* cost = nullptr) {
-  if (cost) *cost = 1e30f;
+static int gemm_big_rows(const p3v_gemm_args_t* a) {
   const int n_big = P3V_GATED(a->epilogue) ? 128 : 256, n_small = n_big / 2;
   if (a->M < 1024 || a->N % n_big || a->epilogue == P3V_EPI_PATCH) return 0;
   if (const int force = p3v_tuning().gemm_big_rows; force >= 0) return min(force / 256 * 256, a->M);   // tests: pin the split
@@ -347,7 +344,6 @@ static int gemm_big_rows(const p3v_gemm_args_t* a, float* cost = nullptr) {
     if (big && small) c += 0.04f;                       // the second launch
     if (c < best - 1e-4f) { best = c; best_rows = rows_big; }
   }
-  if (cost) *cost = best;
   return best_rows;
 }
 
@@ -388,12 +384,64 @@ static bool gemm_tile_plan(const p3v_gemm_args_t* a, int rows_big, int* mb, int*
   return found;
 }
 
+// The tile that p3v_gemm runs, 10 mb + nb, or 0: the packing.  The plan above knows rounds; how long one lasts also depends on how full it is
+// (power: 24 workgroups of 256 x 256 over 128 K-tiles 137 us, 240 of them 155), and the tiles of 192 rows are priced here alone.  t K-tiles, r
+// rounds of which u are filled: once + r (f + c t) + u fill t, and per round what a gated, a 32-bit residual or a GELU epilogue takes more; fitted to
+// 20 heights, 257 .. 9809 rows, of eight projections of the decoder and the vision tower with their weights from memory (3 - 5 % of a time at
+// most sizes).  Another tile than the plan's has to promise 2 %; what it then runs is within 0.6 % of the fastest measured tile on average, 5 % at
+// most beyond 1000 rows.  Measured (us, the plan on these kernels -> this): 2300 x 16384 x 3072 (gate | up) 192 -> 169, 2531 193 -> 187, 768 67 ->
+// 60; 2531 x 9216 x 3072 115 -> 107, 4096 175 -> 163; 3072 x 8192: 6000 rows 238 -> 219, 8192 313 -> 286; 2048 x 10496 x 3072 117 -> 107.
+static int gemm_tile_choice(const p3v_gemm_args_t* a, int rows_big) {
+  int mb = 0, nb = 0;
+  const int plan = gemm_tile_plan(a, rows_big, &mb, &nb) ? 10 * mb + nb : 0;
+  if (a->M <= 256 || a->K < 1024 || a->epilogue == P3V_EPI_PATCH || p3v_tuning().gemm_128 || p3v_tuning().gemm_big_rows >= 0) return plan;
+  struct Tile { int mb, nb; float once, f, c, fill, gated, f32, act; };
+  static const Tile tiles[] = {{8, 4, 2.9f, 8.3f, 0.94f, 0.258f, 1.4f, 7.1f, 0.f}, {7, 4, 3.1f, 7.f, 0.857f, 0.214f, 1.4f, 6.3f, 0.f},
+                               {6, 4, 3.9f, 5.5f, 0.765f, 0.193f, 1.8f, 5.2f, 0.f}, {8, 3, 3.f, 6.3f, 0.754f, 0.207f, 0.f, 5.3f, 0.f},
+                               {6, 3, 5.9f, 3.9f, 0.6f, 0.166f, 0.f, 3.9f, 0.f}, {5, 4, 5.2f, 2.5f, 0.698f, 0.199f, 1.8f, 4.1f, 1.8f},
+                               {4, 4, 5.4f, 1.6f, 0.64f, 0.167f, 1.4f, 3.4f, 1.5f}, {4, 3, 6.5f, 3.6f, 0.467f, 0.144f, 0.f, 2.5f, 1.1f}};
+  const bool gated = P3V_GATED(a->epilogue), f32 = a->epilogue == P3V_EPI_BIAS_RESID_F32 || a->epilogue == P3V_EPI_SCALE_RESID_F32 || a->epilogue == P3V_EPI_F32;
+  const bool act = a->epilogue == P3V_EPI_BIAS_QGELU || a->epilogue == P3V_EPI_BIAS_GELU;
+  const float kt = (float)(a->K / BK);
+  auto time = [&](const Tile& t, int M) {
+    const long n = (long)p3v_cdiv(M, 32 * t.mb) * (a->N / (gated ? 32 * t.nb : 64 * t.nb));
+    const float used = n / 256.f, rounds = (float)((n + 255) / 256);
+    return t.once + rounds * (t.f + (gated ? t.gated : f32 ? t.f32 : act ? t.act : 0.f) + t.c * kt) + used * t.fill * kt;
+  };
+  float best = 0.f;
+  if (plan) {
+    for (const Tile& t : tiles)
+      if (plan == 10 * t.mb + t.nb) best = time(t, a->M);
+  } else {
+    if (rows_big) best = time(tiles[0], rows_big);
+    if (rows_big < a->M) {
+      const long small = (long)p3v_cdiv(a->M - rows_big, BM) * p3v_cdiv(a->N, gated ? BN / 2 : BN), rest = small % 512;
+      best += (small / 512 + (rest > 256)) * (6.0f + 0.95f * kt) + (rest > 0 && rest <= 256 ? 4.4f + 0.85f * kt : 0.f) + (rows_big ? 3.8f : 0.f);
+    }
+  }
+  best *= 0.98f;
+  int choice = plan;
+  for (const Tile& t : tiles) {
+    if (a->N % (gated ? 32 * t.nb : 64 * t.nb) || (gated && t.nb != 4)) continue;
+    const float c = time(t, a->M);
+    if (c < best) best = c, choice = 10 * t.mb + t.nb;
+  }
+  return choice;
+}
+
 extern "C" int p3v_gemm_plan(int M, int N, int K, int epilogue) {
   if (M <= 0 || N <= 0 || K <= 0 || epilogue < 0 || epilogue > P3V_EPI_GELU_MUL) return 0;
   p3v_gemm_args_t a = {};
   a.M = M, a.N = N, a.K = K, a.epilogue = epilogue;
   int mb, nb;
   return gemm_tile_plan(&a, p3v_tuning().gemm_128 ? 0 : gemm_big_rows(&a), &mb, &nb) ? 10 * mb + nb : 0;
+}
+
+extern "C" int p3v_gemm_tile(int M, int N, int K, int epilogue) {
+  if (M <= 0 || N <= 0 || K <= 0 || epilogue < 0 || epilogue > P3V_EPI_GELU_MUL) return 0;
+  p3v_gemm_args_t a = {};
+  a.M = M, a.N = N, a.K = K, a.epilogue = epilogue;
+  return gemm_tile_choice(&a, p3v_tuning().gemm_128 ? 0 : gemm_big_rows(&a));
 }
 
 // ---- split-K for prompt-sized-but-small M (17 .. 256 rows: short chat prompts, the text group of a mixed batch).  One
@@ -669,7 +717,11 @@ extern "C" int p3v_gemm(const p3v_gemm_args_t* a, void* stream) {
     if ((size_t)a->M * a->lda * 2 >= (1ull << 32) || w_rows * a->ldw * 2 >= (1ull << 32)) return P3V_ERR_UNSUPPORTED;
   }
   hipStream_t s = (hipStream_t)stream;
-  if (const int t = p3v_tuning().gemm_tile; t > 0) return p3v_gemm256_try(a, t / 10, t % 10, s);
+  if (int t = p3v_tuning().gemm_tile; t > 0) {                   // (the tiles of 192 rows: 164 and 163)
+    if (t / 10 == 6) return P3V_ERR_UNSUPPORTED;
+    if (t / 10 == 16) t -= 100;
+    return p3v_gemm256_try(a, t / 10, t % 10, s);
+  }
   if (!a->bias) {                                              // 17 .. 256 rows: the weight-streaming kernel (p3v_gemm_skinny.hip)
     const int rc = p3v_gemm_skinny_try(a, s);
     if (rc != P3V_ERR_UNSUPPORTED) return rc;
@@ -680,8 +732,8 @@ extern "C" int p3v_gemm(const p3v_gemm_args_t* a, void* stream) {
   }
   const bool big_tiles = !p3v_tuning().gemm_128;
   const int rows_big = big_tiles ? gemm_big_rows(a) : 0;
-  if (int mb, nb; gemm_tile_plan(a, rows_big, &mb, &nb)) {
-    const int rc = p3v_gemm256_try(a, mb, nb, s);
+  if (const int t = gemm_tile_choice(a, rows_big)) {
+    const int rc = p3v_gemm256_try(a, t / 10, t % 10, s);
     if (rc != P3V_ERR_UNSUPPORTED) return rc;
   }
   if (rows_big > 0) {
@@ -730,35 +782,33 @@ int p3v_gemm_skinny_qkv_merge(const p3v_gemm_args_t* a, const QkvP& q, void* ws,
 int p3v_qkv_flat_tiles(const QkvP& q, int M, int mb);                                        // p3v_gemm_pc.hip
 int p3v_gemm256_flat_qkv(const p3v_gemm_args_t* a, const QkvP& q, int mb, hipStream_t s);      // p3v_gemm256.hip
 
-// The qkv projection on the flat tiles of p3v_gemm_pc.hip: 32 mb rows a tile, or 0.
+// The qkv projection in one launch on tiles of 32 mb rows x 256 columns (p3v_gemm_pc.hip up to 160 rows, p3v_gemm256.hip from 192): mb, or 0.
 // Below 1024 rows the alternative is p3v_gemm and the split as a launch of its own: the same tile saves that launch for 4 us of epilogue (900 x
 // 9216 x 3072 59.0 -> 55.2 us, 768 55.9 -> 52.7), as long as one round of the chip takes the tiles, of which there are more (a V tile's rows are
-// dimensions, its columns 256 tokens).  From 1024 rows on it is the packing of 256 x 256 and 128 x 128 tiles below, of which the first leave a
-// round half empty here and there: 1024 rows 83.0 -> 57.7, 2048 124 -> 103, 1800 118 -> 101; 2885 x 3072 x 1024 (five image crops) 36.1 -> 30.0,
-// 7501 70.5 -> 65.7; it stays the faster for 1100 .. 1500 (82 - 85) and 2531 rows (135, here 136) and for 17 crops (80, here 81).
-// Times fitted to 25 sizes of either: a tile's constant and time per K-tile, 0.6 of the constant for every further round; the packing in its own
-// units of 8.5 + 1.57 K-tiles.  3 % have to be promised.
-static int qkv_flat_plan(const p3v_gemm_args_t* a, const QkvP& q) {
+// dimensions, its columns 256 tokens).  From 1024 rows on every height is priced as in gemm_tile_choice, fitted to 19 prompts of 300 .. 16384
+// tokens and 2 .. 17 image crops: the height it names was the fastest measured at all of them but one (1 %).  Against rows split between
+// 256 x 256 and 128 x 128 tiles or tiles of at most 160 rows: 1536 tokens 81 -> 75 us, 2531 140 -> 127, 4096 217 -> 209, 16384 789 -> 749; 17 crops
+// 80 -> 75, 9 crops 47 -> 42.
+static int qkv_tile_plan(const p3v_gemm_args_t* a, const QkvP& q) {
   const int pin = p3v_tuning().gemm_qkv_flat;
   if (!pin || a->M <= 256 || (q.nh * q.hd) % 256 || (q.nkv * q.hd) % 256) return 0;
   if (pin > 0) return pin;
   if (p3v_tuning().gemm_128 || p3v_tuning().gemm_big_rows >= 0) return 0;
-  p3v_gemm_args_t plain = *a;
   if (a->M < 1024) {
+    p3v_gemm_args_t plain = *a;
     int mb = 0, nb = 0;
     if (splitk_slices(a->M, a->N, a->K, a->epilogue) > 1 || !gemm_tile_plan(&plain, 0, &mb, &nb) || nb != 4 || (mb != 4 && mb != 5)) return 0;
     return p3v_qkv_flat_tiles(q, a->M, mb) <= 256 ? mb : 0;
   }
-  plain.epilogue = P3V_EPI_NONE;
+  static const struct { int mb; float once, f, c, fill; } tiles[] = {{2, 4.2f, 5.8f, 0.25f, 0.237f}, {3, 4.5f, 7.9f, 0.29f, 0.316f}, {4, 5.1f, 8.05f, 0.273f, 0.531f},
+                                                                     {5, 7.1f, 9.3f, 0.363f, 0.542f}, {6, 2.8f, 12.7f, 0.62f, 0.402f}, {7, 4.2f, 14.1f, 0.633f, 0.523f},
+                                                                     {8, 4.5f, 16.f, 0.739f, 0.554f}};
   const float kt = (float)(a->K / BK);
-  static const struct { int mb; float f, c; } tiles[] = {{2, 2.2f, 0.89f}, {3, 8.2f, 0.78f}, {4, 11.2f, 0.866f}, {5, 16.f, 0.87f}};
-  float best;
-  gemm_big_rows(&plain, &best);
-  best = 0.97f * (3.f + best * (8.5f + 1.57f * kt));
+  float best = 1e30f;
   int mb = 0;
   for (const auto& t : tiles) {
-    const int rounds = p3v_cdiv(p3v_qkv_flat_tiles(q, a->M, t.mb), 256);
-    const float c = t.f * (1.f + 0.6f * (rounds - 1)) + rounds * t.c * kt;
+    const int n = p3v_qkv_flat_tiles(q, a->M, t.mb);
+    const float c = t.once + p3v_cdiv(n, 256) * (t.f + t.c * kt) + n / 256.f * t.fill * kt;
     if (c < best) best = c, mb = t.mb;
   }
   return mb;
@@ -784,7 +834,7 @@ static int gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* m
   QkvP q = {sp->cos_t, sp->sin_t, sp->q_out, sp->k_dst, sp->v_dst, sp->L, nh, nkv, hd, sp->past, dpos0, sp->dst_t, sp->tab_t, sp->tab_div, 0,
             sp->q_scale};
   if (merge_ws) return p3v_gemm_skinny_qkv_merge(a, q, merge_ws, merge_bytes, s);
-  if (const int mb = qkv_flat_plan(a, q)) {
+  if (const int mb = qkv_tile_plan(a, q)) {
     const int rc = p3v_gemm256_flat_qkv(a, q, mb, s);
     if (rc != P3V_ERR_UNSUPPORTED) return rc;
   }

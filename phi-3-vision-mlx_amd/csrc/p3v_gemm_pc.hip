@@ -200,15 +200,17 @@ __global__ void __launch_bounds__(768, 1) k_gemm_pc(Gemm256P p) {
       half(1, !last, nslot);
       slot = nslot;
     }
+    int lane_e = lane;                                            // (opaque: what the epilogue derives from it is not to be held through the K loop)
+    asm volatile("" : "+v"(lane_e));
     if constexpr (PART) {
       Gemm256P part = p;
       part.out = (float*)p.out + (size_t)t.z * p.M * p.ldo;
-      gemm256_epilogue<P3V_EPI_F32, MB, NB>(part, acc, m0 + wr * MB * 16, n0 + wc * (n_out_tile / 4), lane);
+      gemm256_epilogue<P3V_EPI_F32, MB, NB>(part, acc, m0 + wr * MB * 16, n0 + wc * (n_out_tile / 4), lane_e);
     } else if constexpr (QKV) {
-      if (!t.swapped) qkv_epilogue_rot<MB, 2>(p.q, acc, p.bias, t.is_k, t.row0, (n0 >> 1) + wc * 32, m0 + wr * MB * 16, p.M, lane);
-      else qkv_epilogue_vt<MB>(p.q, acc, p.bias ? p.bias + t.row0 : nullptr, n0 + wr * MB * 16, m0 + wc * 64, p.M, lane, v_rows);
+      if (!t.swapped) qkv_epilogue_rot<MB, 2>(p.q, acc, p.bias, t.is_k, t.row0, (n0 >> 1) + wc * 32, m0 + wr * MB * 16, p.M, lane_e);
+      else qkv_epilogue_vt<MB>(p.q, acc, p.bias ? p.bias + t.row0 : nullptr, n0 + wr * MB * 16, m0 + wc * 64, p.M, lane_e, v_rows);
     } else {
-      gemm256_epilogue<EPI, MB, NB>(p, acc, m0 + wr * MB * 16, n0 + wc * (n_out_tile / 4), lane);  // straight from the accumulators: p3v_gemm256_epi.h
+      gemm256_epilogue<EPI, MB, NB>(p, acc, m0 + wr * MB * 16, n0 + wc * (n_out_tile / 4), lane_e);  // straight from the accumulators: p3v_gemm256_epi.h
     }
   }
 }

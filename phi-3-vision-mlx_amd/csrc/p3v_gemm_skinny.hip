@@ -320,10 +320,8 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
       uint32_t pk[2][2];
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        float o4[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o4[r] = p3v_gated(EPI, acc[i][j][r], acc[i][2 + j][r]);
-        pk[j][0] = pack_bf16x2(o4[0], o4[1]), pk[j][1] = pack_bf16x2(o4[2], o4[3]);
+        for (int h = 0; h < 2; ++h) pk[j][h] = p3v_gated2(EPI, acc[i][j][2 * h], acc[i][j][2 * h + 1], acc[i][2 + j][2 * h], acc[i][2 + j][2 * h + 1]);
       }
       u32x4_t w;
 #pragma unroll

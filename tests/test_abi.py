@@ -256,6 +256,22 @@ def test_which_tile_runs_a_prompt_sized_projection():
         l.p3v_set_tuning(b"gemm_big_rows", v.value)
 
 
+def test_which_tile_p3v_gemm_runs():
+    """The tile by how full the chip's rounds are: those of 192 rows and the other heights where they were measured the fastest, the plan's own
+    answer elsewhere, and for what is never priced (few rows, short K, a tile height that does not divide the columns)."""
+    from phi_3_vision_mlx_amd import _lib, ops
+    l, v = _lib.lib(), ctypes.c_int()
+    assert l.p3v_get_tuning(b"gemm_big_rows", ctypes.byref(v)) == 0 and l.p3v_set_tuning(b"gemm_big_rows", -1) == 0
+    try:
+        for M, N, K, epi, want in ((768, 8192, 3072, ops.EPI_SILU_MUL, 64), (2300, 8192, 3072, ops.EPI_SILU_MUL, 64), (2531, 8192, 3072, ops.EPI_SILU_MUL, 74),
+                                   (2531, 9216, 3072, ops.EPI_NONE, 64), (900, 9216, 3072, ops.EPI_NONE, 63), (6000, 3072, 8192, ops.EPI_RESID_BF16, 63),
+                                   (8192, 3072, 8192, ops.EPI_RESID_BF16, 83), (9809, 4096, 1024, ops.EPI_BIAS_QGELU, 74), (640, 8192, 3072, ops.EPI_SILU_MUL, 54),
+                                   (2531, 3072, 512, ops.EPI_NONE, 0), (256, 8192, 3072, ops.EPI_NONE, 0), (2531, 3000, 3072, ops.EPI_NONE, 0), (0, 3072, 3072, ops.EPI_NONE, 0)):
+            assert l.p3v_gemm_tile(M, N, K, epi) == want, (M, N, K, epi, l.p3v_gemm_tile(M, N, K, epi))
+    finally:
+        l.p3v_set_tuning(b"gemm_big_rows", v.value)
+
+
 def test_which_decode_batches_run_one_workgroup_per_row_and_head():
     """(rows, new tokens, heads, kv heads, capacity) where the form was measured faster, and where it was not: an uneven second round
     of pairs, shared kv heads, few pairs, long caches."""

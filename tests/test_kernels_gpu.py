@@ -938,6 +938,27 @@ def test_gemm_tiles_agree(ops, epi, M, N, K):
             ops.set_tuning(n, x)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 768, 64), (193, 768, 128), (1111, 768, 192), (4001, 3072, 128), (2300, 9216, 64)])
+@pytest.mark.parametrize("epi", ["none", "silu", "resid_bf16", "resid_f32", "scale", "bias_qgelu", "f32"])
+def test_gemm_192_row_tiles_agree(ops, epi, M, N, K):
+    """The tiles of 192 rows (pinned as 164 and 163) as test_gemm_tiles_agree: one and several rounds, fewer K-tiles than LDS buffers, ragged rows."""
+    gated = epi == "silu"
+    a, w = g((M, K), 40).cuda(), g((2 * N if gated else N, K), 41, 1.0 / math.sqrt(K)).cuda()
+    v, r = g((N,), 42, 0.5).cuda(), g((M, N), 43, 1.0, BF16 if epi == "resid_bf16" else F32).cuda()
+    kw = {"none": {}, "silu": dict(epilogue=ops.EPI_SILU_MUL), "resid_bf16": dict(epilogue=ops.EPI_RESID_BF16, resid=r), "bias_qgelu": dict(epilogue=ops.EPI_BIAS_QGELU, bias=v),
+          "resid_f32": dict(epilogue=ops.EPI_BIAS_RESID_F32, resid=r, bias=v), "scale": dict(epilogue=ops.EPI_SCALE_RESID_F32, resid=r, col_scale=v), "f32": dict(epilogue=ops.EPI_F32)}[epi]
+    names = ("gemm_tile", "gemm_128", "gemm_no_skinny", "gemm_no_splitk")
+    saved = [ops.set_tuning(n, x) for n, x in zip(names, (-1, 1, 1, 1))]
+    try:
+        want = ops.gemm(a, w, **kw)
+        for tile in (164,) if gated else (164, 163):
+            ops.set_tuning("gemm_tile", tile)
+            assert torch.equal(ops.gemm(a, w, **kw), want), f"tile {tile}"
+    finally:
+        for n, x in zip(names, saved):
+            ops.set_tuning(n, x)
+
+
 @pytest.mark.parametrize("M,N,K,gated,tile", [(385, 9216, 1024, False, 43), (641, 9216, 2048, False, 44), (257, 6144, 2048, True, 44), (1300, 6144, 1024, False, 54),
                                               (385, 9216, 1024, True, 54), (1300, 9216, 1024, False, 74), (500, 9216, 1024, True, 74), (1793, 6144, 1024, False, 83),
                                               (700, 9216, 1024, True, 84)])
@@ -1212,6 +1233,14 @@ def test_gemm_qkv_flat_tiles(ops, B, L, nh, nkv, hd, K, past, rot, bias, mb):
         ops.set_tuning("gemm_qkv_flat", saved[0]), ops.set_tuning("gemm_no_splitk", saved[1])
     for x, y, name in zip(*outs, ("Q", "K cache", "V cache")):
         assert torch.equal(x, y), f"{name}: {(x != y).sum().item()} elements differ"
+
+
+@pytest.mark.parametrize("mb", [6, 7, 8])
+@pytest.mark.parametrize("B,L,nh,nkv,hd,K,past,rot,bias", [(1, 257, 8, 8, 96, 192, 0, True, False), (1, 641, 16, 8, 96, 64, 64, True, False), (3, 100, 16, 4, 64, 320, 0, True, True),
+                                                           (17, 577, 16, 16, 64, 256, 0, False, True), (1, 4500, 32, 32, 96, 128, 8, True, False), (40, 7, 8, 8, 96, 448, 8, True, False)])
+def test_gemm_qkv_tall_tiles(ops, B, L, nh, nkv, hd, K, past, rot, bias, mb):
+    """As test_gemm_qkv_flat_tiles, on tiles of 192, 224 and 256 rows: one wave per SIMD, tables requested ahead, rows beyond M stored as row M - 1."""
+    test_gemm_qkv_flat_tiles(ops, B, L, nh, nkv, hd, K, past, rot, bias, mb)
 
 
 @pytest.mark.parametrize("M,taken", [(768, True), (900, True), (1023, True), (2048, True), (300, False), (512, False)])
