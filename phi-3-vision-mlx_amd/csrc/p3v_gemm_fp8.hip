@@ -11,22 +11,22 @@
 //             twice the bf16 rate on this chip (the unscaled 16x16x32 fp8 MFMA runs at the bf16 rate).  A lane holds 32
 //             k bytes of its row (lane & 15) for k-block lane >> 4 -- the SAME bytes for A and B, so which k they are
 //             does not matter (the kernel takes 16-byte chunks fchunk and fchunk + 4: bank-conflict-free reads).
-//   tile      128 or 160(M) x 256 / 192 / 128(N) x 128(K), chosen by how the tiles fill the chip's rounds (f8_tile_plan).  768
+//   tile      chosen by time (f8_tile_plan).  Flat ones, 128 or 160(M) x 256 / 192 / 128(N) x 128(K): 768
 //             threads: 8 CONSUMER waves as 2(M) x 4(N), ONE MFMA per 16 x 16 block and K-tile, and 4 PRODUCER waves that only
 //             request K-tiles by LDS-DMA (as p3v_gemm_pc.hip): rows of 128 BYTES, 16-byte chunk c of row r stored at chunk
 //             c ^ (r & 7), swizzled on the source address; three buffers of a K-tile (four from 128 x 192 down: what 160 KiB
-//             hold), so a request has two or three K-tiles' time to land.  256 x 256 tiles on eight waves that do both, where only they fill a
-//             round (k_gemm_f8_tall).
-//             What bounds it: the producers' requests, ~60 ns per round of four 1-KiB pieces (a K-tile of 128 x 256 takes 0.69 us
-//             where its MFMAs take 0.43), and, with all CUs at it, the chip's power: the same launches on all-zero operands are
-//             20-25 % faster.  Against the form it replaced (256-row tiles, eight waves that request and multiply, two buffers and a
-//             full wait per K-tile, one tile per workgroup, outputs staged through LDS), us at M = 2531 / 1024 / 256, launches by themselves in a graph:
-//               gate_up 131 / 51 / 44 -> 112 / 50 / 18    qkv 79 / 52 / 26 -> 64 / 30 / 16 (K = 3072)
-//               o 29.2 / 27.7 / 25.5 -> 28.2 / 17.4 / 15.4   down 63 / 58 / 57 -> 56 / 32 / 30 (K = 8192)
-//             2.2-2.4 PFLOP/s from 2500 rows on in such a graph.  Inside a prompt, under the profiler, a launch follows others at the
-//             chip's power limit and takes 15 % longer: gate_up 129 at 2531 rows, and the four together 1.8 PFLOP/s.
+//             hold), so a request has two or three K-tiles' time to land.  Tall ones, 192, 224 or 256 x 256, on FOUR waves that request and
+//             multiply (k_gemm_f8_w4).
+//             What bounds it: the requests, ~60 ns per four 1-KiB pieces of a CU (a K-tile of 192 x 256 takes 0.9 us in one round of 64 of
+//             them, where its MFMAs take 0.64), and, with all CUs at it, the chip's power: the same launches on all-zero operands are
+//             20-25 % faster.  The tall tiles against the flat ones, us, weights from memory, launch behind launch: gate | up (16384 x 3072) 2300 rows
+//             122 -> 93, 2531 124 -> 106, 4096 198 -> 164, 8192 367 -> 327 (2.5 PFLOP/s); 9216 x 3072 2531 rows 71 -> 61, 4096 106 -> 97; 3072 x 8192
+//             3500 92 -> 69, 4096 99 -> 79; 3072 x 3072 4096 50 -> 37.  One round of flat tiles that fills the chip stays ahead of one of tall ones
+//             that does not: 3072 x 8192 at 2531 rows 59 (128 rows), 62 (192).
 //   epilogue  scales, then none / residual add / SiLU(gate) * up, bf16 out, straight from the accumulators (p3v_gemm256_epi.h).
 #include <stdlib.h>
+
+#include <type_traits>
 
 #include "p3v_gemm_qkv.h"
 
@@ -333,109 +333,256 @@ __global__ void __launch_bounds__(768, 1) k_gemm_f8(GemmF8P p) {
   }
 }
 
-// 256 x 256 tiles for the sizes whose rounds only they fill (16 column tiles x 16 row tiles and the like): eight waves as 2(M) x 4(N) that request and
-// multiply, two LDS buffers, a full wait and barrier per K-tile, one tile per workgroup.  Two thirds of the flat tiles' staged bytes per
-// product, but the requests stand in front of the MFMAs.  us, against 128 x 256: 4500 x 3072 x 3072 44.5 : 47.6, 4500 x 3072 x 8192 94 : 98,
-// 1700 x 9216 x 3072 41.8 : 44.1, gate | up of 900 rows 45.6 : 47.1.
-struct OffF8 { int a[2][2], b[2][2]; __amdgpu_buffer_rsrc_t rs_a, rs_w; };
-template <int EPI>
-__global__ void __launch_bounds__(512, 1) k_gemm_f8_tall(GemmF8P p) {
+// A wave's sums of 64 columns of W (column group g of NG; SiLU: 32 gate, then the 32 up rows of the same outputs) at rows m0 .., outputs from n0 on:
+// as f8_epilogue, in one straight line (p3v_gemm256_epi.h: buffer stores whose bounds check drops the rows beyond M; the sums stay in
+// accumulation registers until their row's turn; scales and residual rows are requested ahead, one wave per SIMD has nobody to cover for it).
+template <int EPI, int MB, int NG>
+__device__ __forceinline__ void f8_epilogue_w4(const GemmF8P& p, f32x4_t (&acc)[NG][MB][4], int m0, int n0, int lane) {
+  constexpr bool SILU = EPI == P3V_EPI_SILU_MUL, RESID = EPI == P3V_EPI_RESID_BF16;
+  constexpr int NOUT = SILU ? 32 : 64;                             // outputs of a group
+  const int fc = lane & 15, fq = lane >> 4;
+  float s[MB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) s[i] = p.sa[min(m0 + fc + i * 16, p.M - 1)];
+  f32x4_t sc[NG][4];
+#pragma unroll
+  for (int g = 0; g < NG; ++g)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sc[g][j] = *(const f32x4_a4*)(p.sw + n0 + g * NOUT + (SILU ? j % 2 * 16 + j / 2 * p.N : j * 16) + fq * 4);
+  const size_t first = ((size_t)m0 * p.ldo + n0) * 2;
+  const __amdgpu_buffer_rsrc_t rs_o = __builtin_amdgcn_make_buffer_rsrc((unsigned char*)p.out + first, 0, 0x7fffffff, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs_r = __builtin_amdgcn_make_buffer_rsrc((unsigned char*)p.resid + (RESID ? first : 0), 0, 0x7fffffff, 0x00020000);
+  auto at = [&](int i) { return m0 + fc + i * 16 < p.M ? (fc + i * 16) * p.ldo * 2 + ((fq & 1) * 16 + (fq >> 1) * 8) * 2 : (int)0x80000000; };
+  constexpr int TURNS = NG * MB, RN = 6;
+  u32x4_t rw[RESID ? RN : 1][2];
+  auto ask = [&](int t) {
+    if constexpr (RESID)
+#pragma unroll
+      for (int jp = 0; jp < 2; ++jp) rw[t % RN][jp] = __builtin_amdgcn_raw_buffer_load_b128(rs_r, at(t % MB) + t / MB * NOUT * 2 + jp * 64, 0, 0);
+  };
+#pragma unroll
+  for (int t = 0; t < RN; ++t) ask(t);
+#pragma unroll
+  for (int t = 0; t < TURNS; ++t) {
+    const int g = t / MB, i = t % MB;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) asm volatile("" : "+a"(acc[g][i][j]));
+    float v[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[j][r] = acc[g][i][j][r] * (s[i] * sc[g][j][r]);
+    uint32_t pk[4][2];
+    constexpr int NJ = SILU ? 2 : 4;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        pk[j][h] = SILU ? p3v_gated2(EPI, v[j][2 * h], v[j][2 * h + 1], v[(2 + j) % 4][2 * h], v[(2 + j) % 4][2 * h + 1]) : pack_bf16x2(v[j][2 * h], v[j][2 * h + 1]);
+#pragma unroll
+    for (int jp = 0; jp < NJ / 2; ++jp) {
+      u32x4_t w;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        auto sw = __builtin_amdgcn_permlane16_swap(pk[2 * jp][k], pk[2 * jp + 1][k], false, false);
+        w[k] = sw[0], w[2 + k] = sw[1];
+      }
+      if constexpr (RESID)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = pack_bf16x2(bf16lo(rw[t % RN][jp][k]) + bf16lo(w[k]), bf16hi(rw[t % RN][jp][k]) + bf16hi(w[k]));
+      __builtin_amdgcn_raw_buffer_store_b128(w, rs_o, at(i) + g * NOUT * 2 + jp * 64, 0, 0);
+    }
+    if (t + RN < TURNS) ask(t + RN);
+  }
+}
+
+// Tall tiles: 256, 224 or 192 rows x 256 columns on FOUR waves of 16 MB x 128 outputs, one per SIMD, that request and multiply (p3v_gemm256.hip's form).
+// The eight consumers of the flat tiles keep the LDS busy for more cycles than their MFMAs take (160 x 256: 1531 against 1288 a K-tile, reads and
+// DMA); these read 4 MFMAs' worth a fragment: 1536 of 2061.  One MFMA takes a whole K-tile of a block, and both operands' fragments of one K-tile
+// fill 128 registers, so a K-tile is multiplied column block by column block: its W fragments arrive as they are needed (the first two a K-tile
+// early), A's, all of the next K-tile, in the second register set meanwhile.  The sets change places with every K-tile: the loop takes two
+// (K % 256 == 0).  One barrier per K-tile, behind its last W fragment; from there on until the next one a request every few MFMAs, A two
+// K-tiles ahead, W three.
+struct AimF8 { int a_off[8], b_off[8]; __amdgpu_buffer_rsrc_t rs_a, rs_b; };     // (declared outside the template: see TileF8's use)
+template <int EPI, int MB>
+__global__ void __launch_bounds__(256, 1) k_gemm_f8_w4(GemmF8P p) {
   constexpr bool SILU = EPI == P3V_EPI_SILU_MUL;
-  constexpr int TM = 256, TN = 256, n_out_tile = SILU ? TN / 2 : TN, HALF_BYTES = 128 * TKB, BUF_BYTES = 4 * HALF_BYTES;    // A0 A1 B0 B1
+  constexpr int NB = 8, NG = 2, TM = 32 * MB, TN = 256, A_BYTES = TM * TKB, B_BYTES = TN * TKB, B0 = 2 * A_BYTES;    // LDS: two buffers of A, three of W
+  constexpr int NM = MB * NB, NF = MB + NB;                        // MFMAs and requests of a K-tile
+  constexpr int TURN = 2 * (NB - 2) + 4, STEP = (NM - TURN - 2) / NF;                              // where buffers change hands; MFMAs per request behind it
+  constexpr bool ZERO = MB == 8;                                   // (the allocator spills the sums if they start in the first MFMAs)
+  static_assert(STEP >= 2 && 2 * MB <= TURN && NM - TURN - 1 >= 4 + 2 * MB, "");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave >> 2, wc = wave & 3;
-  const int gx = p.N / n_out_tile, gy = (p.M + TM - 1) / TM, nwg = gx * gy;
-  int m0, n0;
-  {   // XCD-aware order, as above
-    const int wid = blockIdx.x, q = nwg >> 3, r = nwg & 7, xcd = wid & 7, loc = wid >> 3;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave >> 1, wc = wave & 1;
+  constexpr int n_out_tile = SILU ? TN / 2 : TN;
+  const int gx = p.N / n_out_tile, gy = (p.M + TM - 1) / TM, nwg = gx * gy, nk = p.K / TKB;
+  auto place = [&](int wid) {                                      // persistent, XCD-aware order, as above
+    const int q = nwg >> 3, r = nwg & 7, xcd = wid & 7, loc = wid >> 3;
     const int id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + loc;
     constexpr int BAND = 4;
     const int band = id / (BAND * gx), in_band = id % (BAND * gx), rows = min(BAND, gy - band * BAND);
-    m0 = (band * BAND + in_band % rows) * TM, n0 = in_band / rows * n_out_tile;
-  }
-  OffF8 t;      // (declared outside the template: see TileF8's use)
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int rr = h * 128 + q * 64 + (tid >> 3), sw = ((tid & 7) ^ (rr & 7)) * 16, in = rr & 63;
-      const int br = SILU ? n0 + (rr >> 6) * 32 + (in & 31) + (in >> 5) * p.N : n0 + rr;       // (SiLU: 32 gate rows + the 32 up rows of the same outputs)
-      t.a[h][q] = (min(m0 + rr, p.M - 1) - m0) * p.lda + sw;
-      t.b[h][q] = (int)((unsigned)br * (unsigned)p.ldw + (unsigned)sw);
-    }
-  t.rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + (size_t)m0 * p.lda), 0, 0xffffffff, 0x00020000);
-  t.rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, 0xffffffff, 0x00020000);
-  auto dma = [&](bool b_side, int kt, int buf) {                  // both halves of one operand's K-tile
-    unsigned char* base = smem + buf * BUF_BYTES + (b_side ? 2 : 0) * HALF_BYTES + wave * 1024;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        lptr_t dst = (lptr_t)(base + h * HALF_BYTES + q * 8192);
-        const int vo = b_side ? t.b[h][q] : t.a[h][q];
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(b_side ? t.rs_w : t.rs_a, dst, 16, vo, kt * TKB, 0, 0);
-      }
+    const PlaceF8 t = {(band * BAND + in_band % rows) * TM, in_band / rows * n_out_tile, 0, 0, 0};
+    return t;
   };
-  f32x4_t acc[8][4];
+  const int sw = ((tid & 7) ^ ((tid >> 3) & 7)) * 16;
+  AimF8 aim;
+  int wa = blockIdx.x, ka = 0, wb = blockIdx.x, kb = 0;            // the K-tiles to be requested next: output tile, K
+  auto aim_a = [&]() {
+    const PlaceF8 t = place(wa);
+    int srow = tid >> 3;                                           // (opaque: what follows from it is not to be held through the K loop)
+    asm volatile("" : "+v"(srow));
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+    for (int q = 0; q < MB; ++q) aim.a_off[q] = (min(t.m0 + q * 32 + srow, p.M - 1) - t.m0) * p.lda + sw;
+    aim.rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)(p.A + (size_t)t.m0 * p.lda), 0, 0xffffffff, 0x00020000);
+  };
+  auto aim_b = [&]() {
+    const PlaceF8 t = place(wb);
+    int srow = tid >> 3;
+    asm volatile("" : "+v"(srow));
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  const int frow = lane & 15, fchunk = lane >> 4, nk = p.K / TKB;
-  const int fo0 = frow * 128 + ((fchunk ^ (frow & 7)) << 4), fo1 = frow * 128 + (((4 + fchunk) ^ (frow & 7)) << 4);      // (as above)
-  dma(false, 0, 0);
-  dma(true, 0, 0);
-  for (int kt = 0; kt < nk; ++kt) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    const unsigned char* ta = smem + (kt & 1) * BUF_BYTES + wr * HALF_BYTES;
-    const unsigned char* tb = smem + (kt & 1) * BUF_BYTES + 2 * HALF_BYTES + wc * 64 * 128;
-    const bool more = kt + 1 < nk;
-    i32x8_t fa[4], fa1[4], fb[2], fb1[2];
-    auto read = [&](const unsigned char* base, auto& f) {
+    for (int q = 0; q < NB; ++q) {
+      const int rr = q * 32 + srow, in = rr & 63;
+      const int br = SILU ? t.n0 + (rr >> 6) * 32 + (in & 31) + (in >> 5) * p.N : t.n0 + rr;   // (SiLU: 32 gate rows + the 32 up rows of the same outputs)
+      aim.b_off[q] = (int)((unsigned)br * (unsigned)p.ldw + (unsigned)sw);
+    }
+    aim.rs_b = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, 0xffffffff, 0x00020000);
+  };
+  // (behind the last K-tile the requests repeat it: every K-tile has the same number of them, and the counted waits hold to the end)
+  auto next_a = [&]() {
+    if (++ka < nk) return;
+    if (wa + (int)gridDim.x < nwg) wa += gridDim.x, ka = 0, aim_a();
+    else ka = nk - 1;
+  };
+  auto next_b = [&]() {
+    if (++kb < nk) return;
+    if (wb + (int)gridDim.x < nwg) wb += gridDim.x, kb = 0, aim_b();
+    else kb = nk - 1;
+  };
+  auto request = [&](int n, int as, int bs) {
+    if (n < MB) {
+      lptr_t dst = (lptr_t)(smem + as + n * 4096 + wave * 1024);
+      const int vo = aim.a_off[n & 7];
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(aim.rs_a, dst, 16, vo, ka * TKB, 0, 0);
+    } else {
+      lptr_t dst = (lptr_t)(smem + (int)B0 + bs + (n - (int)MB) * 4096 + wave * 1024);
+      const int vo = aim.b_off[(n - (int)MB) & 7];
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(aim.rs_b, dst, 16, vo, kb * TKB, 0, 0);
+    }
+  };
+  int wid = blockIdx.x;
+  if (wid >= nwg) return;
+  aim_a(), aim_b();
 #pragma unroll
-      for (int i = 0; i < (int)(sizeof(f) / sizeof(f[0])); ++i) {
-        const u32x4_t lo = *(const u32x4_t*)(base + i * 2048 + fo0), hi = *(const u32x4_t*)(base + i * 2048 + fo1);
-        f[i] = (i32x8_t){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-      }
-    };
-    auto quad = [&](int i0, int j0, auto& a, auto& b) {            // (W fragment first: the block comes out TRANSPOSED)
-      __builtin_amdgcn_s_setprio(1);
+  for (int t = 0; t < 2; ++t) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i0 + i][j0 + j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b[j], a[i], acc[i0 + i][j0 + j], 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
-      __builtin_amdgcn_s_setprio(0);
-    };
-    read(tb, fb);                                                  // fragments of a quadrant are requested ahead of the MFMAs in front of it
-    read(ta, fa);
-    if (more) dma(false, kt + 1, (kt + 1) & 1);
-    read(tb + 2 * 2048, fb1);
-    __builtin_amdgcn_sched_barrier(0);
-    quad(0, 0, fa, fb);
-    __builtin_amdgcn_sched_barrier(0);
-    read(ta + 4 * 2048, fa1);
-    if (more) dma(true, kt + 1, (kt + 1) & 1);
-    __builtin_amdgcn_sched_barrier(0);
-    quad(0, 2, fa, fb1);
-    __builtin_amdgcn_sched_barrier(0);
-    quad(4, 2, fa1, fb1);
-    quad(4, 0, fa1, fb);
+    for (int n = 0; n < NF; ++n) request(n, t * A_BYTES, t * B_BYTES);
+    next_a(), next_b();
   }
-  f8_epilogue<EPI, 8, 4>(p, acc, m0 + wr * 128 + frow, n0 + wc * (n_out_tile / 4), fchunk);
+#pragma unroll
+  for (int n = MB; n < NF; ++n) request(n, 0, 2 * B_BYTES);
+  next_b();
+
+  const int frow = lane & 15, fchunk = lane >> 4;
+  const int fo0 = frow * 128 + ((fchunk ^ (frow & 7)) << 4);       // (chunks fchunk and fchunk + 4 of the row, as above)
+  int as = 0, bs = 0;                                              // the buffers of the K-tile in hand
+  f32x4_t acc[NG][MB][4];
+  i32x8_t fa[2][MB], fb[NB];
+  auto half = [&](i32x8_t& f, int h, const unsigned char* t) {     // a half of a fragment
+    const u32x4_t v = *(const u32x4_t*)(t + (fo0 ^ (h * 64)));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) f[4 * h + k] = (int)v[k];
+  };
+  auto read_b = [&](int n, int bs) { half(fb[n >> 1], n & 1, smem + B0 + bs + wc * (NB * 2048) + (n >> 1) * 2048); };
+  auto read_a = [&](i32x8_t (&f)[MB], int n, int as) { half(f[n >> 1], n & 1, smem + as + wr * (MB * 2048) + (n >> 1) * 2048); };
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NF + NB) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int n = 0; n < 4; ++n) read_b(n, 0);
+#pragma unroll
+  for (int n = 0; n < 2 * MB; ++n) read_a(fa[0], n, 0);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NB) : "memory");
+  for (;;) {
+    const PlaceF8 t = place(wid);
+    bool first_pair = true;
+    auto k_tile = [&](auto first, auto odd) {                      // (first of an output tile: the sums start here, and the next K-tile has been waited for)
+      constexpr bool FIRST = decltype(first)::value;
+      constexpr int P = decltype(odd)::value;
+      const int an = as ^ A_BYTES, bn = bs == 2 * B_BYTES ? 0 : bs + B_BYTES;
+      auto mma = [&](int m) {                                      // (W fragment first: the block comes out TRANSPOSED)
+        const int j = m / MB, i = m % MB;
+        f32x4_t& c = acc[j / 4][i][j % 4];
+        c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[j], fa[P][i], FIRST ? (f32x4_t){0.f, 0.f, 0.f, 0.f} : c, 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int m = 0; m < TURN; ++m) {
+        if (m < 2 * (NB - 2)) read_b(4 + m, bs);
+        mma(m);
+      }
+      // the next K-tile is in LDS, this one in registers: its buffers are given back
+      if (!(ZERO && P == 0 ? first_pair : FIRST)) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NB) : "memory");
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int m = TURN; m < NM; ++m) {
+        if (m > TURN) {                                            // the next K-tile's first two fragments of W, and all of A's
+          const int n = m - TURN - 1;
+          if (n < 4) read_b(n, bn);
+          else if (n < 4 + 2 * MB) read_a(fa[1 - P], n - 4, an);
+        }
+        if (m >= TURN + 2 && (m - TURN - 2) % STEP == 0 && (m - TURN - 2) / STEP < NF) request((m - TURN - 2) / STEP, as, bs);
+        mma(m);
+      }
+      // (an MFMA has no side effects: without this the first K-tile's are moved down, behind the branches, to where the second one's need them)
+#pragma unroll
+      for (int m = 0; m < NM; ++m) asm volatile("" : "+a"(acc[m / MB / 4][m % MB][m / MB % 4]));
+      next_a(), next_b();
+      as = an, bs = bn;
+    };
+    if constexpr (ZERO)
+#pragma unroll
+      for (int m = 0; m < NM; ++m) {
+        acc[m / MB / 4][m % MB][m / MB % 4] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        asm volatile("" : "+a"(acc[m / MB / 4][m % MB][m / MB % 4]));
+      }
+    if constexpr (!ZERO) {
+      k_tile(std::true_type{}, std::integral_constant<int, 0>{});
+      k_tile(std::false_type{}, std::integral_constant<int, 1>{});
+    }
+#pragma unroll 1
+    for (int kt = ZERO ? 0 : 2; kt < nk; kt += 2) {
+      k_tile(std::false_type{}, std::integral_constant<int, 0>{});
+      k_tile(std::false_type{}, std::integral_constant<int, 1>{});
+      first_pair = false;
+    }
+    // (what the next K-tile's turn waits for, waited for ahead of the epilogue's stores, which the same counter counts)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NB) : "memory");
+    int lane_e = lane;                                             // (opaque, as in aim_a)
+    asm volatile("" : "+v"(lane_e));
+    f8_epilogue_w4<EPI, MB, NG>(p, acc, t.m0 + wr * MB * 16, t.n0 + wc * (n_out_tile / 2), lane_e);
+    if (wid + (int)gridDim.x >= nwg) break;
+    wid += gridDim.x;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // (the requests that repeat the last K-tile: LDS is given back behind them)
 }
 int p3v_gemm256_cus();                                             // p3v_gemm256.hip
 
-template <int EPI>
-static int launch_f8_tall(const GemmF8P& p, hipStream_t s) {
-  constexpr int LDS = 2 * F8_BUF(8, 4);
+template <int EPI, int MB>
+static int launch_f8_w4(const GemmF8P& p, hipStream_t s) {
+  constexpr int LDS = (2 * 32 * MB + 3 * 256) * TKB;
   static bool attr_set = false;
   if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)k_gemm_f8_tall<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return P3V_ERR_HIP;
+    if (hipFuncSetAttribute((const void*)k_gemm_f8_w4<EPI, MB>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return P3V_ERR_HIP;
     attr_set = true;
   }
-  hipLaunchKernelGGL(k_gemm_f8_tall<EPI>, dim3(p.N / (EPI == P3V_EPI_SILU_MUL ? 128 : 256) * p3v_cdiv(p.M, 256)), dim3(512), LDS, s, p);
+  const int n_cu = p3v_gemm256_cus();
+  if (!n_cu) return P3V_ERR_HIP;
+  const int tiles = p.N / (EPI == P3V_EPI_SILU_MUL ? 128 : 256) * p3v_cdiv(p.M, 32 * MB);
+  hipLaunchKernelGGL((k_gemm_f8_w4<EPI, MB>), dim3(min(tiles, n_cu)), dim3(256), LDS, s, p);
   P3V_CHECK_LAUNCH();
   return P3V_OK;
 }
@@ -457,22 +604,25 @@ static int launch_f8_v(const GemmF8P& p, hipStream_t s) {
   return P3V_OK;
 }
 
-// the tile whose rounds over the chip cost least.  A round's cost by tile, 128 x 256 = 100, measured over M 17 .. 16000 and the decoder's
-// four projections: 160 x 256 takes 1.02-1.18 of it (least where the chip's power is the limit), 128 x 192 0.87, 128 x 128 0.69, 256 x 256
-// 1.65-1.95 (counted as 1.94, where its round replaces two).  So 2531 rows x 3072 go in one round of 240 wide tiles (27.0 us; 480 narrow ones
-// 29.8), 2048 in 256 of 192 columns (23.8; wide 25.7), 1024 in 192 narrow ones (18.0; wide 24.7), 2531 x 16384 in 4 rounds of 160 rows (108; 5 of
-// 128 rows 110), 1700 x 9216 in one of 252 tall tiles (41.8; 160 rows 46.6).  The choice is within 2 % of the best tile there but at 4500 and 6800 x
-// 9216 and 4500 x 16384 (3 - 5 %).
-static long f8_tile_plan(int M, int N, bool silu, int& mb, int& nb) {
-  static const struct { int mb, nb, cost; } tiles[] = {{4, 4, 100}, {5, 4, 110}, {4, 3, 87}, {4, 2, 69}, {8, 4, 194}};
-  const int n_cu = p3v_gemm256_cus(), pin = p3v_tuning().gemm_f8_narrow;
-  long best = -1;
+// The tile that takes least time, which is returned (us).  t K-tiles, r rounds of which u are filled (a fuller chip runs slower: power): once +
+// r (f + c t) + u fill t, a gated epilogue's more per round; fitted to 20 heights, 128 .. 8192 rows, of the decoder's four projections with their
+// weights from memory (3 - 8 % of a time).  What it names was the fastest of the seven at 76 of those 80 sizes, 3 % off at one (6000 x 3072 x
+// 8192), less at the others; the rounds alone, as it was before the tall tiles ran on four waves, cost 7.7 % on average.
+struct F8Tile { int mb, nb; float once, f, c, fill, gated; };
+static float f8_tile_plan(int M, int N, int K, int ldo, bool silu, int& mb, int& nb) {
+  static const F8Tile tiles[] = {{4, 4, 7.5f, 4.5f, 0.63f, 0.097f, 3.f},    {5, 4, 7.f, 4.3f, 0.691f, 0.192f, 2.7f}, {4, 3, 7.1f, 3.1f, 0.522f, 0.11f, 0.f},
+                                 {4, 2, 6.6f, 2.7f, 0.384f, 0.094f, 1.f},  {8, 4, 3.4f, 8.4f, 0.942f, 0.267f, 2.f}, {7, 4, 4.1f, 7.2f, 0.834f, 0.206f, 1.8f},
+                                 {6, 4, 4.8f, 6.8f, 0.724f, 0.16f, 2.f}};
+  const int n_cu = max(p3v_gemm256_cus(), 1), pin = p3v_tuning().gemm_f8_narrow;
+  const float kt = (float)(K / TKB);
+  float best = -1.f;
   for (const auto& t : tiles) {
     const int n_tile = silu ? 32 * t.nb : 64 * t.nb;
-    if (N % n_tile || (silu && t.nb % 2)) continue;
-    long c = (p3v_cdiv((long)(N / n_tile) * p3v_cdiv(M, 32 * t.mb), (long)max(n_cu, 1))) * t.cost;
-    if (pin == 10 * t.mb + t.nb || (pin == 0 && t.mb == 4 && t.nb == 4) || (pin == 1 && t.nb == 2)) c = 0;
-    if (best < 0 || c < best) best = c, mb = t.mb, nb = t.nb;
+    if (N % n_tile || (silu && t.nb % 2) || (t.mb > 5 && (K % (2 * TKB) || ldo >= 1 << 22))) continue;      // (four waves: K-tiles in pairs, 32-bit store offsets)
+    const long n = (long)(N / n_tile) * p3v_cdiv(M, 32 * t.mb);
+    float c = t.once + (float)p3v_cdiv(n, (long)n_cu) * (t.f + (silu ? t.gated : 0.f) + t.c * kt) + (float)n / (float)n_cu * t.fill * kt;
+    if (pin == 10 * t.mb + t.nb || (pin == 0 && t.mb == 4 && t.nb == 4) || (pin == 1 && t.nb == 2)) c = 0.f;
+    if (best < 0.f || c < best) best = c, mb = t.mb, nb = t.nb;
   }
   return best;
 }
@@ -480,11 +630,13 @@ static long f8_tile_plan(int M, int N, bool silu, int& mb, int& nb) {
 template <int EPI>
 static int launch_f8(const GemmF8P& p, hipStream_t s) {
   int mb = 0, nb = 0;
-  f8_tile_plan(p.M, p.N, EPI == P3V_EPI_SILU_MUL, mb, nb);
+  f8_tile_plan(p.M, p.N, p.K, p.ldo, EPI == P3V_EPI_SILU_MUL, mb, nb);
   if constexpr (EPI != P3V_EPI_SILU_MUL)
     if (nb == 3) return launch_f8_v<EPI, 4, 3>(p, s);
   if (nb == 2) return launch_f8_v<EPI, 4, 2>(p, s);
-  if (mb == 8) return launch_f8_tall<EPI>(p, s);
+  if (mb == 8) return launch_f8_w4<EPI, 8>(p, s);
+  if (mb == 7) return launch_f8_w4<EPI, 7>(p, s);
+  if (mb == 6) return launch_f8_w4<EPI, 6>(p, s);
   return mb == 5 ? launch_f8_v<EPI, 5, 4>(p, s) : launch_f8_v<EPI, 4, 4>(p, s);
 }
 
@@ -508,17 +660,18 @@ extern "C" int p3v_gemm_fp8(const p3v_gemm_fp8_args_t* a, void* stream) {
   }
 }
 
-// Whether one launch beats the two.  It writes and reads 47 MB less (2531 rows), but runs on 128 x 256 tiles alone and each of their rounds
-// is 4.1 us longer; rounds of 128 x 256 from f8_tile_plan's measurements, the split + rotation 2.5 us + 7.8 ns a row of 9216.  us, two :
-// one at K = 3072: 640 rows 29.2 : 27.0, 1300 53.3 : 48.4, 2531 85.6 : 77.2, 4096 130.7 : 123.0, 8192 273 : 226, but 256 20.4 : 23.7,
-// 1024 38.8 : 46.2 and 2048 68.6 : 72.3, where tiles of 160 rows fill their rounds.
+// Whether one launch beats the two.  It writes and reads 47 MB less (2531 rows), but runs on 128 x 256 tiles alone; the split + rotation take
+// 2.5 us + 7.8 ns a row of 9216.  Both sides as in f8_tile_plan.  us, two : one at K = 3072: 640 rows 33.8 : 32.0, 768 36.5 : 31.5, 5193 156 : 153,
+// 8192 258 : 229, 16384 487 : 452, but 256 25.7 : 30.6, 1024 40.5 : 49.8, 2048 71.4 : 75.8, where tiles of other heights fill their rounds.
+// (Tiles of 192 and 224 rows on four waves under this epilogue, with one wave per SIMD to run it: no faster than the faster of the two at any size.)
 extern "C" int p3v_gemm_qkv_fp8_pays(int M, int n_q, int n_kv, int K) {
   if (M <= 0 || K <= 0 || n_q <= 0 || n_kv <= 0 || n_q % 256 || n_kv % 256) return 0;
   int mb, nb;
   const int N = n_q + 2 * n_kv, n_cu = max(p3v_gemm256_cus(), 1);
-  const float round = 7.6f + 0.575f * (float)(K / TKB), rows = (float)M * (float)N;
+  const float kt = (float)(K / TKB), rows = (float)M * (float)N;
   const long tiles = (long)(n_q + n_kv) / 256 * p3v_cdiv(M, 128) + (long)n_kv / 128 * p3v_cdiv(M, 256);
-  return p3v_cdiv(tiles, (long)n_cu) * (round + 4.1f) < 0.01f * (float)f8_tile_plan(M, N, false, mb, nb) * round + 2.5f + 8.5e-7f * rows;
+  const float one = 7.9f + p3v_cdiv(tiles, (long)n_cu) * (5.7f + 0.63f * kt) + (float)tiles / (float)n_cu * 0.16f * kt;
+  return one < f8_tile_plan(M, N, K, N, false, mb, nb) + 2.5f + 8.5e-7f * rows;
 }
 
 // p3v_gemm_fp8 (epilogue NONE) + p3v_rope_kv_append in one launch, bit for bit, on 128 x 256 tiles: the projection's 47 MB (2531 rows) are

@@ -2183,6 +2183,33 @@ def test_gemm_fp8_tiles_agree(ops, request, epi, M, N, K):
     close(outs[0], ref.float(), rtol=5 * 2 ** -9, atol=5 * 2 ** -9 * y.abs().max().item())
 
 
+@pytest.mark.parametrize("epi", ["none", "resid", "silu"])
+@pytest.mark.parametrize("M,cols,K", [(1, 1, 256), (192, 1, 512), (193, 3, 256), (225, 2, 1024), (257, 1, 3072), (4301, 12, 256), (2531, 24, 512)])
+def test_gemm_fp8_tall_tiles(ops, request, epi, M, cols, K):
+    """The fp8 GEMM's tiles of 192, 224 and 256 rows against the flat 128-row tile: the same sums in the same order, the same bits.  Two K-tiles (the
+    least: the products' loop takes two) and more, row counts at and past a tile's, outputs of several rounds of the chip (4301 and 2531 rows:
+    the requests run from one output tile into the next), the row behind the last untouched."""
+    N = cols * (128 if epi == "silu" else 256)
+    EPI = {"none": ops.EPI_NONE, "resid": ops.EPI_RESID_BF16, "silu": ops.EPI_SILU_MUL}[epi]
+    rows = 2 * N if epi == "silu" else N
+    gen = torch.Generator().manual_seed(61)
+    a8, w8 = _e4m3(g((M, K), 62, 1.0, F32)).view(torch.uint8).cuda(), _e4m3(g((rows, K), 63, 1.0, F32)).view(torch.uint8).cuda()
+    sa, sw = (torch.rand((M,), generator=gen) + 0.5).cuda(), ((torch.rand((rows,), generator=gen) + 0.5) / K).cuda()
+    x = g((M + 1, N), 64, 1.0).cuda()
+    old = ops.set_tuning("gemm_f8_narrow", -1)
+    request.addfinalizer(lambda: ops.set_tuning("gemm_f8_narrow", old))
+    outs = {}
+    for tile in (44, 64, 74, 84, -1):
+        ops.set_tuning("gemm_f8_narrow", tile)
+        out = x.clone()
+        ops.gemm_fp8(a8, sa, w8, sw, EPI, resid=out[:M] if epi == "resid" else None, out=out[:M])      # (the residual is added in place)
+        assert torch.equal(out[M], x[M]), tile
+        outs[tile] = out[:M]
+    for tile in (64, 74, 84, -1):
+        assert torch.equal(outs[tile], outs[44]), tile
+    assert torch.isfinite(outs[44].float()).all() and not torch.equal(outs[44], x[:M])
+
+
 def test_gemm_fp8_asymmetric_identity(ops):
     """A = I (scaled), asymmetric W: catches a transposed / permuted C write and a wrong lane -> k mapping."""
     K = N = 256
