@@ -51,8 +51,9 @@ __global__ void __launch_bounds__(256) k_rmsnorm(const u32x4_t* __restrict__ x, 
   }
 }
 
-// the same with the row held in registers (CH 16-byte chunks per lane): x is read once instead of twice
-template <int CH>
+// the same with the row held in registers (CH 16-byte chunks per lane): x is read once instead of twice.  FULL: the row fills the chunks, nothing is
+// masked (128 x 3072 3.4 -> 3.1 us, 640 4.1 -> 3.8, 2531 8.3 -> 8.1)
+template <int CH, bool FULL>
 __global__ void __launch_bounds__(256) k_rmsnorm_r(const u32x4_t* __restrict__ x, const u32x4_t* __restrict__ w,
                                                    u32x4_t* __restrict__ y, int rows, int chunks, float inv_h, float eps) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -63,8 +64,8 @@ __global__ void __launch_bounds__(256) k_rmsnorm_r(const u32x4_t* __restrict__ x
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = i * 64 + lane;
-    v[i] = c < chunks ? xr[c] : (u32x4_t){0u, 0u, 0u, 0u};
-    g[i] = c < chunks ? w[c] : (u32x4_t){0u, 0u, 0u, 0u};
+    v[i] = FULL || c < chunks ? xr[c] : (u32x4_t){0u, 0u, 0u, 0u};
+    g[i] = FULL || c < chunks ? w[c] : (u32x4_t){0u, 0u, 0u, 0u};
   }
   float ss = 0.f;
 #pragma unroll
@@ -79,7 +80,7 @@ __global__ void __launch_bounds__(256) k_rmsnorm_r(const u32x4_t* __restrict__ x
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = i * 64 + lane;
-    if (c < chunks) {
+    if (FULL || c < chunks) {
       u32x4_t o;
 #pragma unroll
       for (int j = 0; j < 4; ++j) o[j] = rms_pair(v[i][j], r, g[i][j]);
@@ -93,7 +94,7 @@ extern "C" int p3v_rmsnorm(const uint16_t* x, const uint16_t* w, uint16_t* y, in
   if (rows == 0) return P3V_OK;
   const int chunks = hidden / 8;
   if (chunks <= 6 * 64) {   // hidden <= 3072: same per-lane summation order as k_rmsnorm, so the results are bit-identical
-    hipLaunchKernelGGL(k_rmsnorm_r<6>, dim3(p3v_cdiv(rows, 4)), dim3(256), 0, (hipStream_t)stream, (const u32x4_t*)x,
+    hipLaunchKernelGGL((chunks == 6 * 64 ? k_rmsnorm_r<6, true> : k_rmsnorm_r<6, false>), dim3(p3v_cdiv(rows, 4)), dim3(256), 0, (hipStream_t)stream, (const u32x4_t*)x,
                        (const u32x4_t*)w, (u32x4_t*)y, rows, chunks, 1.0f / hidden, eps);
     P3V_CHECK_LAUNCH();
     return P3V_OK;

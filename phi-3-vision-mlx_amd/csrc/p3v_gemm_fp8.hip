@@ -698,9 +698,11 @@ extern "C" int p3v_gemm_qkv_fp8(const p3v_gemm_fp8_args_t* a, const p3v_qkv_spli
 // h = bf16(x * rsqrt(mean x^2 + eps) * g): exactly the row p3v_rmsnorm would have written (phi.py:478-479, 482, 484).
 // The row is read ONCE and stays in registers (CH 16-byte chunks per lane: 6 for K = 3072, 16 for K = 8192) through the
 // sum of squares, the maximum and the conversion: 3 bytes of traffic per element.
-// The gain is requested with the row (a second trip behind the sum of squares otherwise): 640 x 3072 4.90 -> 4.67 us, 2531 9.48 -> 9.17, 8192
-// 21.3 -> 18.3.  Without the norm 2531 rows take 6.8: the rest is its arithmetic, 13 vector instructions an element.
-template <bool NORM, int CH>
+// The gain is requested with the row (a second trip behind the sum of squares otherwise), and where the row fills the lanes' chunks (FULL: K = 3072,
+// 8192) nothing is masked: the branches around every chunk kept its arithmetic behind the last load.  us: 128 x 3072 with the norm 4.4 -> 3.8, 640
+// 5.0 -> 4.2, 2531 9.6 -> 8.5, 8192 21.5 -> 17.6; 2531 x 8192 without 14.8 -> 14.0 (62 MB: 4.4 TB/s).  Not for 3072 without the norm: 128 rows
+// 3.0 -> 3.2, 2531 6.9 either way.
+template <bool NORM, int CH, bool FULL>
 __global__ void __launch_bounds__(256) k_quant_fp8_rows(const u32x4_t* __restrict__ x, const u32x4_t* __restrict__ g,
                                                         u32x2_t* __restrict__ q, float* __restrict__ scale, int rows,
                                                         int chunks, float inv_h, float eps) {
@@ -713,8 +715,8 @@ __global__ void __launch_bounds__(256) k_quant_fp8_rows(const u32x4_t* __restric
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = i * 64 + lane;
-    v[i] = c < chunks ? xr[c] : (u32x4_t){0u, 0u, 0u, 0u};
-    if constexpr (G_AHEAD) gv[i] = c < chunks ? g[c] : (u32x4_t){0u, 0u, 0u, 0u};
+    v[i] = FULL || c < chunks ? xr[c] : (u32x4_t){0u, 0u, 0u, 0u};
+    if constexpr (G_AHEAD) gv[i] = FULL || c < chunks ? g[c] : (u32x4_t){0u, 0u, 0u, 0u};
   }
   float r = 1.f;
   if (NORM) {
@@ -732,7 +734,7 @@ __global__ void __launch_bounds__(256) k_quant_fp8_rows(const u32x4_t* __restric
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = i * 64 + lane;
-    if (NORM && c < chunks) {
+    if (NORM && (FULL || c < chunks)) {
       const u32x4_t w = G_AHEAD ? gv[i % (G_AHEAD ? CH : 1)] : g[c];
 #pragma unroll
       for (int j = 0; j < 4; ++j) v[i][j] = rms_pair(v[i][j], r, w[j]);
@@ -748,7 +750,7 @@ __global__ void __launch_bounds__(256) k_quant_fp8_rows(const u32x4_t* __restric
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = i * 64 + lane;
-    if (c < chunks) {
+    if (FULL || c < chunks) {
       u32x2_t o;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
@@ -764,8 +766,8 @@ __global__ void __launch_bounds__(256) k_quant_fp8_rows(const u32x4_t* __restric
 
 template <bool NORM, int CH>
 static void launch_quant(const uint16_t* x, const uint16_t* norm_w, float eps, uint8_t* q, float* scale, int rows, int K, hipStream_t s) {
-  hipLaunchKernelGGL((k_quant_fp8_rows<NORM, CH>), dim3(p3v_cdiv(rows, 4)), dim3(256), 0, s, (const u32x4_t*)x, (const u32x4_t*)norm_w,
-                     (u32x2_t*)q, scale, rows, K / 8, 1.0f / K, eps);
+  const auto fn = (NORM || CH > 6) && K == CH * 512 ? k_quant_fp8_rows<NORM, CH, NORM || (CH > 6)> : k_quant_fp8_rows<NORM, CH, false>;
+  hipLaunchKernelGGL(fn, dim3(p3v_cdiv(rows, 4)), dim3(256), 0, s, (const u32x4_t*)x, (const u32x4_t*)norm_w, (u32x2_t*)q, scale, rows, K / 8, 1.0f / K, eps);
 }
 
 extern "C" int p3v_quant_fp8_rows(const uint16_t* x, const uint16_t* norm_w, float eps, uint8_t* q, float* scale, int rows,

@@ -2116,6 +2116,19 @@ def test_quant_fp8_rows(ops, rows, K, norm):
         assert (dq - h).abs().max().item() <= 2 ** -3 * h.abs().amax().item()
 
 
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("rows,K", [(3, 8), (5, 512), (7, 3064), (6, 3072), (9, 3080), (5, 8184), (4, 8192)])
+def test_quant_fp8_rows_widths(ops, rows, K, norm):
+    """Rows that fill the lanes' chunks (3072, 8192: the unmasked form) and those next to them, one chunk short of it, one past it, and tiny."""
+    test_quant_fp8_rows(ops, rows, K, norm)
+
+
+@pytest.mark.parametrize("rows,H", [(3, 8), (6, 3064), (7, 3072), (5, 3080)])
+def test_rmsnorm_widths(ops, orc, rows, H):
+    """The same for the plain norm (3072: unmasked)."""
+    test_rmsnorm(ops, orc, rows, H)
+
+
 @pytest.mark.parametrize("narrow", [None, "0", "1"])
 @pytest.mark.parametrize("epi,M,N,K", [("none", 300, 512, 384), ("none", 2531, 9216, 3072), ("resid", 2531, 3072, 8192),
                                        ("silu", 700, 1024, 3072), ("resid", 17, 256, 128), ("none", 513, 384, 256)])
