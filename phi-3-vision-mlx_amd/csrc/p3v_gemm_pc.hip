@@ -10,7 +10,7 @@
 //            MFMAs; larger tiles do not fit the 168 registers that twelve waves leave each other.
 // 2531 x 3072 x 8192 (+ residual) 117 -> 105 us (1.21 PFLOP/s), 9809 x 1024 x 4096 (+ fp32 residual) 95 -> 73, 2048 x 9472 x 3072 114 -> 97.
 // Same K order and epilogue as the other tiles: bit-identical results.
-// P3V_EPI_QKV: split, rotation and KV append in the epilogue, tiles of 64 and 96 rows too (qkv_flat_plan, p3v_gemm.hip, has the rule and the
+// P3V_EPI_QKV: split, rotation and KV append in the epilogue, tiles of 64 and 96 rows too (qkv_tile_plan, p3v_gemm.hip, has the rule and the
 // times; a K-tile of 64 x 256 takes as long as one of 128 x 256, waiting for its weights, but a short K gets through the chip sooner).
 // P3V_EPI_PART: the tiles of one slice of K after the other, fp32 partials (p3v_gemm_slices, p3v_gemm.hip, which has the rule and the times).
 // (Tried and left out: touching the lines of later K-tiles ahead of the DMA, one dword per line -- 64 lines cost the address path as
