@@ -17,9 +17,9 @@
 //             c ^ (r & 7), swizzled on the source address; three buffers of a K-tile (four from 128 x 192 down: what 160 KiB
 //             hold), so a request has two or three K-tiles' time to land.  Tall ones, 192, 224 or 256 x 256, on FOUR waves that request and
 //             multiply (k_gemm_f8_w4).
-//             What bounds it: the requests, ~60 ns per four 1-KiB pieces of a CU (a K-tile of 192 x 256 takes 0.9 us in one round of 64 of
-//             them, where its MFMAs take 0.64), and, with all CUs at it, the chip's power: the same launches on all-zero operands are
-//             20-25 % faster.  The tall tiles against the flat ones, us, weights from memory, launch behind launch: gate | up (16384 x 3072) 2300 rows
+//             What bounds it: the requests, 60 ns per four 1-KiB pieces of a CU with the weights from memory, 40 with all of it in the L2s
+//             (a K-tile of 192 x 256, 0.64 us of MFMAs, takes 0.81 - 0.85 and 0.73 where 12 - 60 CUs are at it), and, with all CUs at it, the
+//             chip's power (0.97 - 1.03): the same launches on all-zero operands are 20-25 % faster.  The tall tiles against the flat ones, us, weights from memory, launch behind launch: gate | up (16384 x 3072) 2300 rows
 //             122 -> 93, 2531 124 -> 106, 4096 198 -> 164, 8192 367 -> 327 (2.5 PFLOP/s); 9216 x 3072 2531 rows 71 -> 61, 4096 106 -> 97; 3072 x 8192
 //             3500 92 -> 69, 4096 99 -> 79; 3072 x 3072 4096 50 -> 37.  One round of flat tiles that fills the chip stays ahead of one of tall ones
 //             that does not: 3072 x 8192 at 2531 rows 59 (128 rows), 62 (192).
@@ -606,8 +606,8 @@ static int launch_f8_v(const GemmF8P& p, hipStream_t s) {
 
 // The tile that takes least time, which is returned (us).  t K-tiles, r rounds of which u are filled (a fuller chip runs slower: power): once +
 // r (f + c t) + u fill t, a gated epilogue's more per round; fitted to 20 heights, 128 .. 8192 rows, of the decoder's four projections with their
-// weights from memory (3 - 8 % of a time).  What it names was the fastest of the seven at 76 of those 80 sizes, 3 % off at one (6000 x 3072 x
-// 8192), less at the others; the rounds alone, as it was before the tall tiles ran on four waves, cost 7.7 % on average.
+// weights from memory (3 - 8 % of a time).  What it names was the fastest of the seven at 77 of those 80 sizes, 3 % off at one (6000 x 3072 x
+// 8192), 1.5 % or less at two; the rounds alone, as it was before the tall tiles ran on four waves, cost 7.7 % on average.
 struct F8Tile { int mb, nb; float once, f, c, fill, gated; };
 static float f8_tile_plan(int M, int N, int K, int ldo, bool silu, int& mb, int& nb) {
   static const F8Tile tiles[] = {{4, 4, 7.5f, 4.5f, 0.63f, 0.097f, 3.f},    {5, 4, 7.f, 4.3f, 0.691f, 0.192f, 2.7f}, {4, 3, 7.1f, 3.1f, 0.522f, 0.11f, 0.f},
