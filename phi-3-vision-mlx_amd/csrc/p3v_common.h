@@ -63,10 +63,11 @@ __device__ __forceinline__ float p3v_sigmoid(float x) { return __builtin_amdgcn_
 //  SiLU: every intermediate rounded to bf16, as the reference's array expression rounds it (phi.py:469-471)
 //  GELU (tanh form): 0.5 g (1 + tanh(sqrt(2/pi) (g + 0.044715 g^3))) in fp32 = g sigmoid(2 u): no cancellation for any g
 #define P3V_GATED(epi) ((epi) == P3V_EPI_SILU_MUL || (epi) == P3V_EPI_GELU_MUL)
-// n / (1 + e) for e = an exponential, 0 .. inf, as a quarter of n / (1/4 + e/4), whose reciprocal the hardware does not flush: a Newton step on
-// that reciprocal is within an ulp and gives a SiLU the same 16 bits as the IEEE quotient for each of the 65536 values that its gate, rounded to
-// 16 bits, can have; with n, a second step on the quotient.  (The compiler's own division takes 11 instructions, two of them transcendental; the
-// gated epilogue of 256 x 256 tiles, 128 outputs a lane on one wave per SIMD, goes from 28 to 20 an output.)
+// n / (1 + e) for e = an exponential, 0 .. inf: by the reciprocal of 1/4 + e/4, which the hardware does not flush, and a Newton step on it; with n, a
+// second step on the quotient, which is formed with 1 / (1 + e) <= 1, so that no n overflows on the way.  The quotient has the bits of the IEEE division
+// for each of the 2^32 gates of a GELU, the reciprocal gives a SiLU the same 16 bits for each of the 65536 values that its gate, rounded to 16 bits, can
+// have.  (The compiler's own division takes 11 instructions, two of them transcendental; the gated epilogue of 256 x 256 tiles, 128 outputs a lane on
+// one wave per SIMD, goes from 28 to 20 an output with a SiLU.)
 __device__ __forceinline__ float p3v_rcp_1p(float e) {
   const float d = fmaf(e, 0.25f, 0.25f);
   float y = __builtin_amdgcn_rcpf(d);
@@ -74,12 +75,12 @@ __device__ __forceinline__ float p3v_rcp_1p(float e) {
   return 0.25f * __builtin_amdgcn_div_fixupf(y, d, 1.f);
 }
 __device__ __forceinline__ float p3v_div_1p(float n, float e) {
-  const float d = fmaf(e, 0.25f, 0.25f);
-  float y = __builtin_amdgcn_rcpf(d);
-  y = fmaf(fmaf(-d, y, 1.f), y, y);
+  const float d = 1.f + e, c = fmaf(e, 0.25f, 0.25f);
+  float y = __builtin_amdgcn_rcpf(c);
+  y = 0.25f * fmaf(fmaf(-c, y, 1.f), y, y);
   float q = n * y;
   q = fmaf(fmaf(-d, q, n), y, q);
-  return 0.25f * __builtin_amdgcn_div_fixupf(q, d, n);
+  return __builtin_amdgcn_div_fixupf(q, d, n);
 }
 __device__ __forceinline__ float p3v_gelu_tanh(float g) {
   const float u = 0.7978845608028654f * (g + 0.044715f * g * g * g);

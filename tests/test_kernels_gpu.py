@@ -959,6 +959,30 @@ def test_gemm_192_row_tiles_agree(ops, epi, M, N, K):
             ops.set_tuning(n, x)
 
 
+@pytest.mark.parametrize("tile", [-1, 84, 54])
+@pytest.mark.parametrize("epi", ["silu", "gelu"])
+def test_gated_epilogues_on_every_finite_gate(ops, epi, tile):
+    """Every finite 16-bit value as a gate, up = 1, against 64 bits.  The gate column picks one of eight values a row, so the sum is that value exactly.
+    GELU: one rounding to bf16 (2^-9) and an exponential whose argument, at most 89, is rounded a few times (89 x 4 x 2^-24): below 2^-8.  SiLU:
+    sigmoid and product are rounded to bf16, either a step (2^-8) off where it lies next to a tie: below 2^-7.  Where the exponential is beyond 2^128 the
+    quotient is 0, less than 89 x 2^-128 off."""
+    vals = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(BF16)
+    vals = torch.where(torch.isfinite(vals), vals, torch.zeros((), dtype=BF16))
+    a, w = torch.zeros((8192, 64), dtype=BF16), torch.zeros((256, 64), dtype=BF16)
+    a[:, :8], a[:, 8] = vals.view(8192, 8), 1.0
+    w[torch.arange(128), torch.arange(128) % 8], w[128:, 8] = 1.0, 1.0
+    saved = ops.set_tuning("gemm_tile", tile)
+    try:
+        got = ops.gemm(a.cuda(), w.cuda(), ops.EPI_SILU_MUL if epi == "silu" else ops.EPI_GELU_MUL).cpu().double()
+    finally:
+        ops.set_tuning("gemm_tile", saved)
+    assert torch.equal(got[:, :8].repeat(1, 16), got)
+    g64 = vals.view(8192, 8).double()
+    want = torch.nn.functional.silu(g64) if epi == "silu" else g64 * torch.sigmoid(2 * math.sqrt(2 / math.pi) * (g64 + 0.044715 * g64 ** 3))
+    err = (got[:, :8] - want).abs() - (2 ** -7 if epi == "silu" else 2 ** -8) * want.abs() - 89 * 2.0 ** -128
+    assert not (err > 0).any() and torch.isfinite(got).all(), [(x.item(), y.item()) for x, y in zip(g64[~(err <= 0)][:4], got[:, :8][~(err <= 0)][:4])]
+
+
 @pytest.mark.parametrize("M,N,K,gated,tile", [(385, 9216, 1024, False, 43), (641, 9216, 2048, False, 44), (257, 6144, 2048, True, 44), (1300, 6144, 1024, False, 54),
                                               (385, 9216, 1024, True, 54), (1300, 9216, 1024, False, 74), (500, 9216, 1024, True, 74), (1793, 6144, 1024, False, 83),
                                               (700, 9216, 1024, True, 84)])
