@@ -325,6 +325,7 @@ int p3v_gemm256_try(const p3v_gemm_args_t* a, int mb, int nb, hipStream_t s) {
 int p3v_gemm256_slices(const p3v_gemm_args_t* a, float* part, int S, int mb, int nb, hipStream_t s) {
   const int tile = 10 * mb + nb;
   if ((tile != 54 && tile != 44 && tile != 43) || a->N % (64 * nb) || a->K % TK || S < 1 || S > a->K / TK) return P3V_ERR_UNSUPPORTED;
+  if ((size_t)80 * a->N * 4 >= ((size_t)1 << 31)) return P3V_ERR_UNSUPPORTED;   // the partials' 32-bit store offsets, 80 rows of a wave at most
   if ((size_t)a->N * a->ldw * 2 >= ((size_t)1 << 32) || (size_t)a->M * a->lda * 2 >= ((size_t)1 << 32)) return P3V_ERR_UNSUPPORTED;  // 32-bit buffer offsets
   const Gemm256P p = {a->A, a->W, part, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, a->N, {}, S};
   return p3v_gemm_pc(p, P3V_EPI_PART, mb, nb, s);

@@ -238,6 +238,21 @@ for t, M in (({tile}, 64), (43, 64), (83, 64)):
     assert r.returncode == 0, (r.returncode, r.stderr[-1500:])
 
 
+def test_k_slices_decline_partials_beyond_32_bit_offsets():
+    """The partials are stored at 32-bit byte offsets from a wave's first output: 80 rows of N floats have to stay below 2^31.  (Nothing is launched.)"""
+    from phi_3_vision_mlx_amd import _lib as L, ops
+    l, buf, v = L.lib(), ctypes.create_string_buffer(4096), ctypes.c_int()
+    p, N = (ctypes.addressof(buf) + 15) // 16 * 16, (2 ** 31 // 320 // 256 + 1) * 256
+    assert l.p3v_get_tuning(b"gemm_slices", ctypes.byref(v)) == 0
+    try:
+        for tile in (154, 144):                                   # one slice on tiles of 160 / 128 x 256
+            assert l.p3v_set_tuning(b"gemm_slices", tile) == 0
+            a = L.GemmArgs(p, p, p, 0, p, 0, 1, N, 64, 64, 64, N, ops.EPI_RESID_BF16, 0, p, N * 4, 0)
+            assert l.p3v_gemm_slices(ctypes.byref(a), None, 0.0, None, None) == L.ERR_UNSUPPORTED
+    finally:
+        l.p3v_set_tuning(b"gemm_slices", v.value)
+
+
 def test_which_tile_runs_a_prompt_sized_projection():
     """One size for every tile, and sizes that stay on the row packing: where no tile promises enough, 224-row tiles for one full round
     (slower than 256 x 256 there), short K loops, few rows."""
