@@ -158,6 +158,9 @@ typedef struct {
   int M, N, K, lda, ldw, ldo, epilogue;
 } p3v_gemm_fp8_args_t;
 int p3v_gemm_fp8(const p3v_gemm_fp8_args_t* args /* host */, void* stream);
+/* The tile p3v_gemm_fp8 runs (host query): 10 mb + nb for 32 mb rows x 64 nb rows of W, the value that the knob "gemm_f8_narrow" pins it with.  A pin that the
+ * problem cannot run on (columns that are no whole tiles) leaves the choice by shape.  0: not a problem of that call */
+int p3v_gemm_fp8_tile(int M, int N, int K, int epilogue);
 int p3v_quant_fp8_rows(const uint16_t* x, const uint16_t* norm_w /* optional */, float eps, uint8_t* q, float* scale,
                        int rows, int K, void* stream);
 

@@ -401,9 +401,10 @@ __device__ __forceinline__ void f8_epilogue_w4(const GemmF8P& p, f32x4_t (&acc)[
 // The eight consumers of the flat tiles keep the LDS busy for more cycles than their MFMAs take (160 x 256: 1531 against 1288 a K-tile, reads and
 // DMA); these read 4 MFMAs' worth a fragment: 1536 of 2061.  One MFMA takes a whole K-tile of a block, and both operands' fragments of one K-tile
 // fill 128 registers, so a K-tile is multiplied column block by column block: its W fragments arrive as they are needed (the first two a K-tile
-// early), A's, all of the next K-tile, in the second register set meanwhile.  The sets change places with every K-tile: the loop takes two
-// (K % 256 == 0).  One barrier per K-tile, behind its last W fragment; from there on until the next one a request every few MFMAs, A two
-// K-tiles ahead, W three.
+// early), A's, all of the next K-tile, in the second register set meanwhile.  The sets change places with every K-tile: the loop takes two; an odd
+// last one moves the second set into the first, 64 moves an output tile (1300 x 9216 x 3200 48 us on the flat tiles, 34 here; gate | up of 2048
+// rows, K = 2944: 102, 80).  One barrier per K-tile, behind its last W fragment; from there on until the next one a request every few MFMAs, A two K-tiles
+// ahead, W three.
 struct AimF8 { int a_off[8], b_off[8]; __amdgpu_buffer_rsrc_t rs_a, rs_b; };     // (declared outside the template: see TileF8's use)
 template <int EPI, int MB>
 __global__ void __launch_bounds__(256, 1) k_gemm_f8_w4(GemmF8P p) {
@@ -554,10 +555,15 @@ __global__ void __launch_bounds__(256, 1) k_gemm_f8_w4(GemmF8P p) {
       k_tile(std::false_type{}, std::integral_constant<int, 1>{});
     }
 #pragma unroll 1
-    for (int kt = ZERO ? 0 : 2; kt < nk; kt += 2) {
+    for (int kt = ZERO ? 0 : 2; kt + 1 < nk; kt += 2) {
       k_tile(std::false_type{}, std::integral_constant<int, 0>{});
       k_tile(std::false_type{}, std::integral_constant<int, 1>{});
       first_pair = false;
+    }
+    if (nk & 1) {                                                  // the next output tile starts in the first register set again
+      k_tile(std::false_type{}, std::integral_constant<int, 0>{});
+#pragma unroll
+      for (int i = 0; i < MB; ++i) fa[0][i] = fa[1][i];
     }
     // (what the next K-tile's turn waits for, waited for ahead of the epilogue's stores, which the same counter counts)
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NB) : "memory");
@@ -608,17 +614,18 @@ static int launch_f8_v(const GemmF8P& p, hipStream_t s) {
 // r (f + c t) + u fill t, a gated epilogue's more per round; fitted to 20 heights, 128 .. 8192 rows, of the decoder's four projections with their
 // weights from memory (3 - 8 % of a time).  What it names was the fastest of the seven at 77 of those 80 sizes, 3 % off at one (6000 x 3072 x
 // 8192), 1.5 % or less at two; the rounds alone, as it was before the tall tiles ran on four waves, cost 7.7 % on average.
+static int f8_cus() { const int n = p3v_gemm256_cus(); return n ? n : 256; }     // (no device: host queries)
 struct F8Tile { int mb, nb; float once, f, c, fill, gated; };
 static float f8_tile_plan(int M, int N, int K, int ldo, bool silu, int& mb, int& nb) {
   static const F8Tile tiles[] = {{4, 4, 7.5f, 4.5f, 0.63f, 0.097f, 3.f},    {5, 4, 7.f, 4.3f, 0.691f, 0.192f, 2.7f}, {4, 3, 7.1f, 3.1f, 0.522f, 0.11f, 0.f},
                                  {4, 2, 6.6f, 2.7f, 0.384f, 0.094f, 1.f},  {8, 4, 3.4f, 8.4f, 0.942f, 0.267f, 2.f}, {7, 4, 4.1f, 7.2f, 0.834f, 0.206f, 1.8f},
                                  {6, 4, 4.8f, 6.8f, 0.724f, 0.16f, 2.f}};
-  const int n_cu = max(p3v_gemm256_cus(), 1), pin = p3v_tuning().gemm_f8_narrow;
+  const int n_cu = f8_cus(), pin = p3v_tuning().gemm_f8_narrow;
   const float kt = (float)(K / TKB);
   float best = -1.f;
   for (const auto& t : tiles) {
     const int n_tile = silu ? 32 * t.nb : 64 * t.nb;
-    if (N % n_tile || (silu && t.nb % 2) || (t.mb > 5 && (K % (2 * TKB) || ldo >= 1 << 22))) continue;      // (four waves: K-tiles in pairs, 32-bit store offsets)
+    if (N % n_tile || (silu && t.nb % 2) || (t.mb > 5 && ((t.mb < 8 && K < 2 * TKB) || ldo >= 1 << 22))) continue;      // (four waves: the first two K-tiles apart from the others below 256 rows; 32-bit store offsets)
     const long n = (long)(N / n_tile) * p3v_cdiv(M, 32 * t.mb);
     float c = t.once + (float)p3v_cdiv(n, (long)n_cu) * (t.f + (silu ? t.gated : 0.f) + t.c * kt) + (float)n / (float)n_cu * t.fill * kt;
     if (pin == 10 * t.mb + t.nb || (pin == 0 && t.mb == 4 && t.nb == 4) || (pin == 1 && t.nb == 2)) c = 0.f;
@@ -638,6 +645,13 @@ static int launch_f8(const GemmF8P& p, hipStream_t s) {
   if (mb == 7) return launch_f8_w4<EPI, 7>(p, s);
   if (mb == 6) return launch_f8_w4<EPI, 6>(p, s);
   return mb == 5 ? launch_f8_v<EPI, 5, 4>(p, s) : launch_f8_v<EPI, 4, 4>(p, s);
+}
+
+extern "C" int p3v_gemm_fp8_tile(int M, int N, int K, int epilogue) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % TKB || N % 128 || (epilogue != P3V_EPI_NONE && epilogue != P3V_EPI_RESID_BF16 && epilogue != P3V_EPI_SILU_MUL)) return 0;
+  int mb = 0, nb = 0;
+  f8_tile_plan(M, N, K, N, epilogue == P3V_EPI_SILU_MUL, mb, nb);
+  return 10 * mb + nb;
 }
 
 extern "C" int p3v_gemm_fp8(const p3v_gemm_fp8_args_t* a, void* stream) {
@@ -667,7 +681,7 @@ extern "C" int p3v_gemm_fp8(const p3v_gemm_fp8_args_t* a, void* stream) {
 extern "C" int p3v_gemm_qkv_fp8_pays(int M, int n_q, int n_kv, int K) {
   if (M <= 0 || K <= 0 || n_q <= 0 || n_kv <= 0 || n_q % 256 || n_kv % 256) return 0;
   int mb, nb;
-  const int N = n_q + 2 * n_kv, n_cu = max(p3v_gemm256_cus(), 1);
+  const int N = n_q + 2 * n_kv, n_cu = f8_cus();
   const float kt = (float)(K / TKB), rows = (float)M * (float)N;
   const long tiles = (long)(n_q + n_kv) / 256 * p3v_cdiv(M, 128) + (long)n_kv / 128 * p3v_cdiv(M, 256);
   const float one = 7.9f + p3v_cdiv(tiles, (long)n_cu) * (5.7f + 0.63f * kt) + (float)tiles / (float)n_cu * 0.16f * kt;

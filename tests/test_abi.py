@@ -287,6 +287,27 @@ def test_which_tile_p3v_gemm_runs():
         l.p3v_set_tuning(b"gemm_big_rows", v.value)
 
 
+def test_which_tile_runs_an_fp8_projection():
+    """A pin names the tile that runs, for odd numbers of K-tiles too; one that the problem does not divide into leaves the choice by shape."""
+    from phi_3_vision_mlx_amd import _lib, ops
+    l, v = _lib.lib(), ctypes.c_int()
+    assert l.p3v_get_tuning(b"gemm_f8_narrow", ctypes.byref(v)) == 0
+    try:
+        for K in (256, 384, 640, 3200):
+            for tile in (44, 54, 42, 43, 64, 74, 84):
+                assert l.p3v_set_tuning(b"gemm_f8_narrow", tile) == 0
+                assert l.p3v_gemm_fp8_tile(1300, 9216, K, ops.EPI_NONE) == tile, (K, tile)
+                if tile != 43:
+                    assert l.p3v_gemm_fp8_tile(1300, 8192, K, ops.EPI_SILU_MUL) == tile, (K, tile)
+        assert l.p3v_set_tuning(b"gemm_f8_narrow", 43) == 0
+        free = l.p3v_gemm_fp8_tile(1300, 4096, 384, ops.EPI_NONE)
+        assert free != 43 and l.p3v_set_tuning(b"gemm_f8_narrow", -1) == 0 and l.p3v_gemm_fp8_tile(1300, 4096, 384, ops.EPI_NONE) == free
+        for M, N, K, epi in ((0, 256, 256, ops.EPI_NONE), (1, 100, 256, ops.EPI_NONE), (1, 256, 64, ops.EPI_NONE), (1, 256, 256, ops.EPI_GELU_MUL)):
+            assert l.p3v_gemm_fp8_tile(M, N, K, epi) == 0
+    finally:
+        l.p3v_set_tuning(b"gemm_f8_narrow", v.value)
+
+
 def test_which_decode_batches_run_one_workgroup_per_row_and_head():
     """(rows, new tokens, heads, kv heads, capacity) where the form was measured faster, and where it was not: an uneven second round
     of pairs, shared kv heads, few pairs, long caches."""

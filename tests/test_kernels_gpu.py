@@ -2221,11 +2221,13 @@ def test_gemm_fp8_tiles_agree(ops, request, epi, M, N, K):
 
 
 @pytest.mark.parametrize("epi", ["none", "resid", "silu"])
-@pytest.mark.parametrize("M,cols,K", [(1, 1, 256), (192, 1, 512), (193, 3, 256), (225, 2, 1024), (257, 1, 3072), (4301, 12, 256), (2531, 24, 512)])
+@pytest.mark.parametrize("M,cols,K", [(1, 1, 256), (192, 1, 512), (193, 3, 256), (225, 2, 1024), (257, 1, 3072), (4301, 12, 256), (2531, 24, 512),
+                                      (257, 2, 384), (193, 1, 640), (4301, 24, 256), (4301, 24, 384), (4301, 24, 768), (8449, 24, 640), (8449, 24, 256), (300, 3, 128)])
 def test_gemm_fp8_tall_tiles(ops, request, epi, M, cols, K):
-    """The fp8 GEMM's tiles of 192, 224 and 256 rows against the flat 128-row tile: the same sums in the same order, the same bits.  Two K-tiles (the
-    least: the products' loop takes two) and more, row counts at and past a tile's, outputs of several rounds of the chip (4301 and 2531 rows:
-    the requests run from one output tile into the next), the row behind the last untouched."""
+    """The fp8 GEMM's tiles of 192, 224 and 256 rows against the flat 128-row tile: the same sums in the same order, the same bits.  One K-tile (256 rows
+    alone), two and more, even and odd numbers of them (the products' loop takes two), row counts at and past a tile's, outputs of several rounds of the
+    chip (256 workgroups: 4301 rows of 24 column tiles are 408 of 256 rows, 8449 are 816, the third and fourth output tile of a workgroup; the requests run
+    from one output tile into the next), the row behind the last untouched."""
     N = cols * (128 if epi == "silu" else 256)
     EPI = {"none": ops.EPI_NONE, "resid": ops.EPI_RESID_BF16, "silu": ops.EPI_SILU_MUL}[epi]
     rows = 2 * N if epi == "silu" else N
@@ -2238,6 +2240,7 @@ def test_gemm_fp8_tall_tiles(ops, request, epi, M, cols, K):
     outs = {}
     for tile in (44, 64, 74, 84, -1):
         ops.set_tuning("gemm_f8_narrow", tile)
+        assert tile < 0 or (K < 256 and tile in (64, 74)) or ops.L.lib().p3v_gemm_fp8_tile(M, N, K, EPI) == tile
         out = x.clone()
         ops.gemm_fp8(a8, sa, w8, sw, EPI, resid=out[:M] if epi == "resid" else None, out=out[:M])      # (the residual is added in place)
         assert torch.equal(out[M], x[M]), tile
