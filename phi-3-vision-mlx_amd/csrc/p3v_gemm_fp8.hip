@@ -610,24 +610,30 @@ static int launch_f8_v(const GemmF8P& p, hipStream_t s) {
   return P3V_OK;
 }
 
-// The tile that takes least time, which is returned (us).  t K-tiles, r rounds of which u are filled (a fuller chip runs slower: power): once +
-// r (f + c t) + u fill t, a gated epilogue's more per round; fitted to 20 heights, 128 .. 8192 rows, of the decoder's four projections with their
-// weights from memory (3 - 8 % of a time).  What it names was the fastest of the seven at 77 of those 80 sizes, 3 % off at one (6000 x 3072 x
-// 8192), 1.5 % or less at two; the rounds alone, as it was before the tall tiles ran on four waves, cost 7.7 % on average.
+// The tile that takes least time, which is returned (us).  t K-tiles, r rounds of which u are filled (a fuller chip runs slower: power, and the outputs'
+// way to memory): once + r (f + c t) + u (fill t + out), a gated or residual epilogue's more per round; fitted to 24 heights, 128 .. 9809 rows, of 15
+// projections of K = 256 .. 8192 (even and odd numbers of K-tiles) with their weights from memory (4 - 8 % of a time; profiles/gemm_fp8_tile_sweep.txt).  What it
+// names is 0.2 % slower than the fastest of the seven on average over those 360 sizes, 6.8 % at most (with each projection's own times left out of the
+// fit: the same).  The fit to K = 3072 and 8192 alone that this one replaces: 1.4 %, 20 % at most, at short K (4096 x 384, 1300 rows 9.8 -> 8.9 us; 9216 x 3072,
+// 1024 rows 31.3 -> 29.9); rounds alone: 7.7 % at K = 3072 and 8192.
 static int f8_cus() { const int n = p3v_gemm256_cus(); return n ? n : 256; }     // (no device: host queries)
-struct F8Tile { int mb, nb; float once, f, c, fill, gated; };
-static float f8_tile_plan(int M, int N, int K, int ldo, bool silu, int& mb, int& nb) {
-  static const F8Tile tiles[] = {{4, 4, 7.5f, 4.5f, 0.63f, 0.097f, 3.f},    {5, 4, 7.f, 4.3f, 0.691f, 0.192f, 2.7f}, {4, 3, 7.1f, 3.1f, 0.522f, 0.11f, 0.f},
-                                 {4, 2, 6.6f, 2.7f, 0.384f, 0.094f, 1.f},  {8, 4, 3.4f, 8.4f, 0.942f, 0.267f, 2.f}, {7, 4, 4.1f, 7.2f, 0.834f, 0.206f, 1.8f},
-                                 {6, 4, 4.8f, 6.8f, 0.724f, 0.16f, 2.f}};
+struct F8Tile { int mb, nb; float once, f, gated, resid, c, fill, out; };
+static float f8_tile_plan(int M, int N, int K, int ldo, int epilogue, int& mb, int& nb) {
+  static const F8Tile tiles[] = {{4, 4, 4.82f, 0.1f, 1.75f, 1.45f, 0.779f, 0.023f, 2.48f},  {5, 4, 5.01f, 0.71f, 2.18f, 1.85f, 0.804f, 0.103f, 2.57f},
+                                 {4, 3, 5.72f, 0.42f, 0.f, 1.64f, 0.569f, 0.054f, 1.86f},   {4, 2, 3.87f, 0.21f, 0.76f, 0.72f, 0.492f, 0.017f, 1.44f},
+                                 {8, 4, 5.02f, 3.29f, 1.82f, 2.34f, 0.98f, 0.269f, 2.46f},  {7, 4, 5.18f, 2.09f, 1.69f, 1.88f, 0.897f, 0.2f, 2.45f},
+                                 {6, 4, 4.97f, 1.57f, 1.4f, 1.25f, 0.847f, 0.141f, 2.36f}};
   const int n_cu = f8_cus(), pin = p3v_tuning().gemm_f8_narrow;
+  const bool silu = epilogue == P3V_EPI_SILU_MUL, resid = epilogue == P3V_EPI_RESID_BF16;
   const float kt = (float)(K / TKB);
   float best = -1.f;
   for (const auto& t : tiles) {
     const int n_tile = silu ? 32 * t.nb : 64 * t.nb;
-    if (N % n_tile || (silu && t.nb % 2) || (t.mb > 5 && ((t.mb < 8 && K < 2 * TKB) || ldo >= 1 << 22))) continue;      // (four waves: the first two K-tiles apart from the others below 256 rows; 32-bit store offsets)
+    if (N % n_tile || (silu && t.nb % 2)) continue;
+    if (t.mb > 5 && ((t.mb < 8 && K < 2 * TKB) || ldo >= 1 << 22)) continue;      // (four waves: two K-tiles come first below 256 rows; 32-bit store offsets)
     const long n = (long)(N / n_tile) * p3v_cdiv(M, 32 * t.mb);
-    float c = t.once + (float)p3v_cdiv(n, (long)n_cu) * (t.f + (silu ? t.gated : 0.f) + t.c * kt) + (float)n / (float)n_cu * t.fill * kt;
+    const float rounds = (float)p3v_cdiv(n, (long)n_cu), used = (float)n / (float)n_cu;
+    float c = t.once + rounds * (t.f + (silu ? t.gated : resid ? t.resid : 0.f) + t.c * kt) + used * (t.fill * kt + t.out);
     if (pin == 10 * t.mb + t.nb || (pin == 0 && t.mb == 4 && t.nb == 4) || (pin == 1 && t.nb == 2)) c = 0.f;
     if (best < 0.f || c < best) best = c, mb = t.mb, nb = t.nb;
   }
@@ -637,7 +643,7 @@ static float f8_tile_plan(int M, int N, int K, int ldo, bool silu, int& mb, int&
 template <int EPI>
 static int launch_f8(const GemmF8P& p, hipStream_t s) {
   int mb = 0, nb = 0;
-  f8_tile_plan(p.M, p.N, p.K, p.ldo, EPI == P3V_EPI_SILU_MUL, mb, nb);
+  f8_tile_plan(p.M, p.N, p.K, p.ldo, EPI, mb, nb);
   if constexpr (EPI != P3V_EPI_SILU_MUL)
     if (nb == 3) return launch_f8_v<EPI, 4, 3>(p, s);
   if (nb == 2) return launch_f8_v<EPI, 4, 2>(p, s);
@@ -650,7 +656,7 @@ static int launch_f8(const GemmF8P& p, hipStream_t s) {
 extern "C" int p3v_gemm_fp8_tile(int M, int N, int K, int epilogue) {
   if (M <= 0 || N <= 0 || K <= 0 || K % TKB || N % 128 || (epilogue != P3V_EPI_NONE && epilogue != P3V_EPI_RESID_BF16 && epilogue != P3V_EPI_SILU_MUL)) return 0;
   int mb = 0, nb = 0;
-  f8_tile_plan(M, N, K, N, epilogue == P3V_EPI_SILU_MUL, mb, nb);
+  f8_tile_plan(M, N, K, N, epilogue, mb, nb);
   return 10 * mb + nb;
 }
 
@@ -674,18 +680,21 @@ extern "C" int p3v_gemm_fp8(const p3v_gemm_fp8_args_t* a, void* stream) {
   }
 }
 
-// Whether one launch beats the two.  It writes and reads 47 MB less (2531 rows), but runs on 128 x 256 tiles alone; the split + rotation take
-// 2.5 us + 7.8 ns a row of 9216.  Both sides as in f8_tile_plan.  us, two : one at K = 3072: 640 rows 33.8 : 32.0, 768 36.5 : 31.5, 5193 156 : 153,
-// 8192 258 : 229, 16384 487 : 452, but 256 25.7 : 30.6, 1024 40.5 : 49.8, 2048 71.4 : 75.8, where tiles of other heights fill their rounds.
+// Whether one launch beats the two.  It writes and reads 47 MB less (2531 rows), but runs on 128 x 256 tiles alone; the split + rotation take 3.7 us +
+// 7.9 ns a row of 9216, half as much again for rows beyond 120 MB.  Both sides as in f8_tile_plan, fitted to 48 sizes (24 of K = 3072, 32 + 32 + 32 heads; shared
+// kv heads, K = 384 .. 1024); one has to promise 3 %.  It names the slower way at one of them, by 1 %.  us, two : one at K = 3072: 577 rows 33.0 : 31.0, 768
+// 37.0 : 32.1, 2531 86 : 85, 8192 267 : 238, 16384 493 : 459, but 256 25.3 : 30.4, 1024 41.7 : 49.7, 2300 79 : 83, where tiles of other heights fill their rounds;
+// 2531 rows of 3072 x 1024 25 : 18.
 // (Tiles of 192 and 224 rows on four waves under this epilogue, with one wave per SIMD to run it: no faster than the faster of the two at any size.)
 extern "C" int p3v_gemm_qkv_fp8_pays(int M, int n_q, int n_kv, int K) {
   if (M <= 0 || K <= 0 || n_q <= 0 || n_kv <= 0 || n_q % 256 || n_kv % 256) return 0;
   int mb, nb;
   const int N = n_q + 2 * n_kv, n_cu = f8_cus();
-  const float kt = (float)(K / TKB), rows = (float)M * (float)N;
+  const float kt = (float)(K / TKB), out = (float)M * (float)N;
   const long tiles = (long)(n_q + n_kv) / 256 * p3v_cdiv(M, 128) + (long)n_kv / 128 * p3v_cdiv(M, 256);
-  const float one = 7.9f + p3v_cdiv(tiles, (long)n_cu) * (5.7f + 0.63f * kt) + (float)tiles / (float)n_cu * 0.16f * kt;
-  return one < f8_tile_plan(M, N, K, N, false, mb, nb) + 2.5f + 8.5e-7f * rows;
+  const float one = 6.66f + p3v_cdiv(tiles, (long)n_cu) * (1.73f + 0.62f * kt) + (float)tiles / (float)n_cu * (0.2f * kt + 4.23f);
+  const float two = f8_tile_plan(M, N, K, N, P3V_EPI_NONE, mb, nb) + 3.7f + 8.6e-7f * out + 5e-7f * fmaxf(out - 6e7f, 0.f);
+  return 1.03f * one < two;
 }
 
 // p3v_gemm_fp8 (epilogue NONE) + p3v_rope_kv_append in one launch, bit for bit, on 128 x 256 tiles: the projection's 47 MB (2531 rows) are

@@ -302,6 +302,15 @@ def test_which_tile_runs_an_fp8_projection():
         assert l.p3v_set_tuning(b"gemm_f8_narrow", 43) == 0
         free = l.p3v_gemm_fp8_tile(1300, 4096, 384, ops.EPI_NONE)
         assert free != 43 and l.p3v_set_tuning(b"gemm_f8_narrow", -1) == 0 and l.p3v_gemm_fp8_tile(1300, 4096, 384, ops.EPI_NONE) == free
+        # (by shape: the fastest measured tile, by 5 % or more, of short K, of K = 3072 and 8192, of odd numbers of K-tiles)
+        for M, N, K, epi, want in ((1300, 4096, 384, ops.EPI_NONE, 44), (768, 9216, 640, ops.EPI_NONE, 44), (1300, 9216, 640, ops.EPI_NONE, 64), (1300, 9216, 3200, ops.EPI_NONE, 64),
+                                   (1024, 9216, 3072, ops.EPI_NONE, 54), (320, 9216, 3072, ops.EPI_NONE, 42), (2531, 9216, 3072, ops.EPI_NONE, 64),
+                                   (2531, 8192, 3072, ops.EPI_SILU_MUL, 74), (2048, 8192, 2944, ops.EPI_SILU_MUL, 84), (2531, 3072, 8192, ops.EPI_RESID_BF16, 44),
+                                   (4096, 3072, 3072, ops.EPI_RESID_BF16, 74)):
+            assert l.p3v_gemm_fp8_tile(M, N, K, epi) == want, (M, N, K, epi, l.p3v_gemm_fp8_tile(M, N, K, epi))
+        for M, n_q, n_kv, K, want in ((256, 3072, 3072, 3072, 0), (577, 3072, 3072, 3072, 1), (768, 3072, 3072, 3072, 1), (1024, 3072, 3072, 3072, 0), (2048, 3072, 3072, 3072, 0),
+                                      (2300, 3072, 3072, 3072, 0), (8192, 3072, 3072, 3072, 1), (16384, 3072, 3072, 3072, 1), (2531, 1024, 1024, 1024, 1), (1536, 768, 768, 384, 1)):
+            assert l.p3v_gemm_qkv_fp8_pays(M, n_q, n_kv, K) == want, (M, n_q, n_kv, K)
         for M, N, K, epi in ((0, 256, 256, ops.EPI_NONE), (1, 100, 256, ops.EPI_NONE), (1, 256, 64, ops.EPI_NONE), (1, 256, 256, ops.EPI_GELU_MUL)):
             assert l.p3v_gemm_fp8_tile(M, N, K, epi) == 0
     finally:
