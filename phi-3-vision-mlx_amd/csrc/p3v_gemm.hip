@@ -43,7 +43,6 @@ struct GemmP {
   QkvP q;       // P3V_EPI_QKV only
 };
 
-__device__ __forceinline__ float gelu_erf(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
 
 __device__ __forceinline__ void load8_bf16(const bf16_t* p, float* v) {
   const u32x4_t w = *(const u32x4_t*)p;
@@ -274,7 +273,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm(GemmP p) {
         for (int r = 0; r < 4; ++r) {
           v[r] = acc[i][j][r] + bias[j][r];
           if (EPI == P3V_EPI_BIAS_QGELU) v[r] = v[r] * p3v_sigmoid(1.702f * v[r]);
-          else if (EPI == P3V_EPI_BIAS_GELU) v[r] = gelu_erf(v[r]);
+          else if (EPI == P3V_EPI_BIAS_GELU) v[r] = p3v_gelu_erf(v[r]);
         }
         pk[jj][0] = pack_bf16x2(v[0], v[1]), pk[jj][1] = pack_bf16x2(v[2], v[3]);
       }

@@ -18,8 +18,6 @@ struct Gemm256P {
   int slices;                            // P3V_EPI_PART only: slice z takes the K-tiles z nk / slices .. (z + 1) nk / slices
 };
 
-__device__ __forceinline__ float gelu_erf2(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
-
 // ---- epilogue: 16 MB x 16 NB outputs per wave, STRAIGHT FROM THE ACCUMULATORS.  The MFMAs take the W fragment as their
 // first operand, so a 16 x 16 block comes out transposed: lane (c = lane & 15, q = lane >> 4) holds, for output row
 // m = block row c, the FOUR CONSECUTIVE columns 4q .. 4q+3 (the plain operand order gives four rows of one column, which is
@@ -141,7 +139,7 @@ __device__ __forceinline__ void gemm256_epilogue(const Gemm256P& p, f32x4_t (&ac
             v[r] = acc[i][j][r];
             if constexpr (BIAS) v[r] += bias[j][r];
             if (EPI == P3V_EPI_BIAS_QGELU) v[r] = v[r] * p3v_sigmoid(1.702f * v[r]);
-            else if (EPI == P3V_EPI_BIAS_GELU) v[r] = gelu_erf2(v[r]);
+            else if (EPI == P3V_EPI_BIAS_GELU) v[r] = p3v_gelu_erf(v[r]);
           }
           pk[j][0] = pack_bf16x2(v[0], v[1]), pk[j][1] = pack_bf16x2(v[2], v[3]);
         }

@@ -983,6 +983,29 @@ def test_gated_epilogues_on_every_finite_gate(ops, epi, tile):
     assert not (err > 0).any() and torch.isfinite(got).all(), [(x.item(), y.item()) for x, y in zip(g64[~(err <= 0)][:4], got[:, :8][~(err <= 0)][:4])]
 
 
+@pytest.mark.parametrize("tile", [-1, 84, 44])
+def test_erf_gelu_on_every_finite_input(ops, tile):
+    """x P(x) for every finite 16-bit x against 64 bits: 8e-6 and one rounding to bf16 (2^-9) are below 2^-8; where exp(-x^2 / 2) is below 2^-126, beyond |x| = 13.3, it
+    may be 0.  Infinities and NaN as the plain formula has them."""
+    vals = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(BF16)
+    vals = torch.where(torch.isfinite(vals), vals, torch.zeros((), dtype=BF16))
+    a, w = torch.zeros((8192, 64), dtype=BF16), torch.zeros((768, 64), dtype=BF16)
+    a[:, :8] = vals.view(8192, 8)
+    w[torch.arange(768), torch.arange(768) % 8] = 1.0
+    bias = torch.zeros(768, dtype=BF16)
+    bias[8], bias[9], bias[10] = float("inf"), float("-inf"), float("nan")
+    saved = ops.set_tuning("gemm_tile", tile)
+    try:
+        got = ops.gemm(a.cuda(), w.cuda(), ops.EPI_BIAS_GELU, bias=bias.cuda()).cpu().double()
+    finally:
+        ops.set_tuning("gemm_tile", saved)
+    x = vals.view(8192, 8).double()
+    want = 0.5 * x * torch.special.erfc(-x * math.sqrt(0.5))
+    err = (got[:, :8] - want).abs() - 2 ** -8 * want.abs() - 14 * 2.0 ** -126
+    assert not (err > 0).any() and torch.isfinite(got[:, :8]).all(), [(p.item(), q.item()) for p, q in zip(x[~(err <= 0)][:4], got[:, :8][~(err <= 0)][:4])]
+    assert torch.equal(got[:, 16:24], got[:, :8]) and (got[:, 8] == math.inf).all() and torch.isnan(got[:, 9:11]).all()
+
+
 @pytest.mark.parametrize("M,N,K,gated,tile", [(385, 9216, 1024, False, 43), (641, 9216, 2048, False, 44), (257, 6144, 2048, True, 44), (1300, 6144, 1024, False, 54),
                                               (385, 9216, 1024, True, 54), (1300, 9216, 1024, False, 74), (500, 9216, 1024, True, 74), (1793, 6144, 1024, False, 83),
                                               (700, 9216, 1024, True, 84)])
