@@ -230,6 +230,9 @@ typedef struct {
   float q_scale;
 } p3v_qkv_split_t;
 int p3v_gemm_qkv(const p3v_gemm_args_t* gemm /* host */, const p3v_qkv_split_t* split /* host */, void* stream);
+/* The tile p3v_gemm_qkv runs on more than 256 rows (host query; n_q, n_kv: rows of W per region): mb for 32 mb rows x 256 columns, 1: 128 x 128, the value that the knob
+ * "gemm_qkv_flat" pins it with; 0: one of the kernels for few rows, 128 x 128 tiles of regions that are no whole 256 columns, or P3V_ERR_UNSUPPORTED */
+int p3v_gemm_qkv_tile(int M, int n_q, int n_kv, int K);
 /* ---- p3v_gemm_qkv of 17 .. 128 rows, and p3v_gemm with a gated epilogue (SiLU, GELU) of 105 .. 128, as slices of K that are summed inside
  *      the launch: the same products, the slices' fp32 sums added in slice order.  ws: p3v_gemm_merge_ws_bytes(M, N, K, epilogue, qkv) bytes
  *      (0: not a shape of these calls; N = output columns, qkv = 1 for the former), 16-byte aligned and ZERO in its first 4096 before the

@@ -154,6 +154,7 @@ SIGNATURES = {
     "p3v_gemm_plan": (i32, [i32, i32, i32, i32]),
     "p3v_gemm_tile": (i32, [i32, i32, i32, i32]),
     "p3v_gemm_fp8_tile": (i32, [i32, i32, i32, i32]),
+    "p3v_gemm_qkv_tile": (i32, [i32, i32, i32, i32]),
     "p3v_gemm_qkv_fp8": (i32, [C.POINTER(GemmF8Args), C.POINTER(QkvSplit), vp]),
     "p3v_gemm_qkv_fp8_pays": (i32, [i32, i32, i32, i32]),
     "p3v_gemm_slices": (i32, [C.POINTER(GemmArgs), vp, f32, vp, vp]),

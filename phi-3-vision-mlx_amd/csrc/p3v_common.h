@@ -218,7 +218,7 @@ struct P3vTuning {
   int gemm_no_skinny, gemm_skinny_max_m, gemm_skinny_s, gemm_skinny_tm128, gemm_no_merge;   // the 128 x 64-tile weight-streaming kernel for 17 .. max_m rows (p3v_gemm_skinny.hip)
   int gemm_merge_polls;     // p3v_gemm_merge, p3v_gemm_qkv_merge: looks at a counter before a wait is given up; -1: 2^22 (seconds); tests: 0
   int gemm_slices;          // p3v_gemm_slices: -1: by shape, 0: never, 100 S + 10 mb + nb: S slices of K on tiles of 32 mb x 64 nb
-  int gemm_qkv_flat;        // p3v_gemm_qkv on tiles of 32 x gemm_qkv_flat rows (2 .. 8): -1: by shape, 0: never
+  int gemm_qkv_flat;        // p3v_gemm_qkv on tiles of 32 x gemm_qkv_flat rows (2 .. 8; 1: 128 x 128): -1: by shape, 0: by the kernels for few rows or 128 x 128 tiles
   int gemm_no_qkv_fuse;     // 1: p3v_gemm_qkv reports P3V_ERR_UNSUPPORTED (callers then run p3v_gemm + p3v_rope_kv_append)
   int gemm_f8_narrow;       // tile of the fp8 GEMM: -1: by shape, 0 / 1: 256 / 128 columns, 10 mb + nb: 32 mb x 64 nb
   int attn_no_dma, attn_old, attn_pp, attn_il, attn_il_waves, combine_g, kvq_old, q8_old;

@@ -776,43 +776,60 @@ static int gemm128(const p3v_gemm_args_t* a, hipStream_t s) {
 }
 
 // ---- the qkv projection with the head split, the rotation and the KV append in its epilogue (p3v_gemm_qkv.h)
-int p3v_gemm256_qkv(const p3v_gemm_args_t* a, const QkvP& q, hipStream_t s);   // p3v_gemm256.hip
 int p3v_gemm_skinny_qkv(const p3v_gemm_args_t* a, const QkvP& q, hipStream_t s);   // p3v_gemm_skinny.hip
 
 int p3v_gemm_skinny_qkv_merge(const p3v_gemm_args_t* a, const QkvP& q, void* ws, int64_t ws_bytes, hipStream_t s);   // p3v_gemm_skinny.hip
 int p3v_qkv_flat_tiles(const QkvP& q, int M, int mb);                                        // p3v_gemm_pc.hip
 int p3v_gemm256_flat_qkv(const p3v_gemm_args_t* a, const QkvP& q, int mb, hipStream_t s);      // p3v_gemm256.hip
 
-// The qkv projection in one launch on tiles of 32 mb rows x 256 columns (p3v_gemm_pc.hip up to 160 rows, p3v_gemm256.hip from 192): mb, or 0.
+// The qkv projection in one launch on tiles of 32 mb rows x 256 columns (p3v_gemm_pc.hip up to 160 rows, p3v_gemm256.hip from 192) or, mb = 1, of 128 x 128
+// (k_gemm): mb, or 0.
 // Below 1024 rows the alternative is p3v_gemm and the split as a launch of its own: the same tile saves that launch for 4 us of epilogue (900 x
 // 9216 x 3072 59.0 -> 55.2 us, 768 55.9 -> 52.7), as long as one round of the chip takes the tiles, of which there are more (a V tile's rows are
-// dimensions, its columns 256 tokens).  From 1024 rows on every height is priced as in gemm_tile_choice, fitted to 19 prompts of 300 .. 16384
-// tokens and 2 .. 17 image crops: the height it names was the fastest measured at all of them but one (1 %).  Against rows split between
-// 256 x 256 and 128 x 128 tiles or tiles of at most 160 rows: 1536 tokens 81 -> 75 us, 2531 140 -> 127, 4096 217 -> 209, 16384 789 -> 749; 17 crops
-// 80 -> 75, 9 crops 47 -> 42.
+// dimensions, its columns 256 tokens).  From 1024 rows on every tile is priced as in gemm_tile_choice, 128 x 128 ones (two a CU: whole rounds of 512, and
+// the last one by whether it holds more than 256) for K <= 1024 alone, where their short prologue counts; fitted to 219 sizes: 21 heights, 1024 .. 16384 rows,
+// of nine projections with K = 256 .. 3072, and 2 .. 17 image crops (profiles/gemm_qkv_tile_sweep.txt).  The tile it names is 0.7 % slower than the fastest on
+// average, 15 % at most (K = 256); each projection left out of the fit: 1.0 %, 15 %.  At the decoder's own widths, 9216 x 3072, it is the fastest at each
+// of the 42 sizes of one and four prompts.  Measured, us, a fit without short K -> this: 1536 x 4608 x 512 16.7 -> 14.8, 8192 60 -> 56; 2048 x 9216 x 3072 104 ->
+// 103, 4096 205 -> 198; 11 crops 58.9 -> 56.6.
 static int qkv_tile_plan(const p3v_gemm_args_t* a, const QkvP& q) {
   const int pin = p3v_tuning().gemm_qkv_flat;
   if (!pin || a->M <= 256 || (q.nh * q.hd) % 256 || (q.nkv * q.hd) % 256) return 0;
   if (pin > 0) return pin;
-  if (p3v_tuning().gemm_128 || p3v_tuning().gemm_big_rows >= 0) return 0;
+  if (p3v_tuning().gemm_128) return 0;
   if (a->M < 1024) {
     p3v_gemm_args_t plain = *a;
     int mb = 0, nb = 0;
     if (splitk_slices(a->M, a->N, a->K, a->epilogue) > 1 || !gemm_tile_plan(&plain, 0, &mb, &nb) || nb != 4 || (mb != 4 && mb != 5)) return 0;
     return p3v_qkv_flat_tiles(q, a->M, mb) <= 256 ? mb : 0;
   }
-  static const struct { int mb; float once, f, c, fill; } tiles[] = {{2, 4.2f, 5.8f, 0.25f, 0.237f}, {3, 4.5f, 7.9f, 0.29f, 0.316f}, {4, 5.1f, 8.05f, 0.273f, 0.531f},
-                                                                     {5, 7.1f, 9.3f, 0.363f, 0.542f}, {6, 2.8f, 12.7f, 0.62f, 0.402f}, {7, 4.2f, 14.1f, 0.633f, 0.523f},
-                                                                     {8, 4.5f, 16.f, 0.739f, 0.554f}};
+  static const struct { int mb; float once, f, c, fill, out; } tiles[] = {{2, 4.32f, 3.74f, 0.182f, 0.389f, 0.f},    {3, 4.68f, 4.67f, 0.318f, 0.398f, 0.f},
+                                                                          {4, 5.11f, 4.64f, 0.507f, 0.312f, 1.77f},  {5, 5.38f, 6.17f, 0.584f, 0.358f, 1.52f},
+                                                                          {6, 4.1f, 9.78f, 0.685f, 0.372f, 1.88f},   {7, 4.67f, 10.44f, 0.802f, 0.38f, 2.24f},
+                                                                          {8, 4.96f, 11.85f, 0.879f, 0.446f, 2.45f}};
   const float kt = (float)(a->K / BK);
   float best = 1e30f;
   int mb = 0;
+  if (a->K <= 1024) {
+    const long n = (long)(a->N / BN) * p3v_cdiv(a->M, BM), rest = n % 512;
+    best = 4.63f + n / 512 * (2.09f + 0.516f * kt) + (rest > 0) * (1.58f + 0.423f * kt) + (rest > 256) * (1.03f + 0.036f * kt) + n / 512.f * (3.72f + 0.272f * kt);
+    mb = 1;
+  }
   for (const auto& t : tiles) {
     const int n = p3v_qkv_flat_tiles(q, a->M, t.mb);
-    const float c = t.once + p3v_cdiv(n, 256) * (t.f + t.c * kt) + n / 256.f * t.fill * kt;
+    const float c = t.once + p3v_cdiv(n, 256) * (t.f + t.c * kt) + n / 256.f * (t.fill * kt + t.out);
     if (c < best) best = c, mb = t.mb;
   }
   return mb;
+}
+
+extern "C" int p3v_gemm_qkv_tile(int M, int n_q, int n_kv, int K) {
+  if (M <= 0 || n_q <= 0 || n_kv <= 0 || K <= 0 || n_q % 32 || n_kv % 32 || K % BK) return 0;
+  p3v_gemm_args_t a = {};
+  QkvP q = {};
+  a.M = M, a.N = n_q + 2 * n_kv, a.K = K, a.epilogue = P3V_EPI_NONE;
+  q.nh = n_q / 32, q.nkv = n_kv / 32, q.hd = 32;
+  return qkv_tile_plan(&a, q);
 }
 
 static int gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* merge_ws, int64_t merge_bytes, void* stream) {
@@ -832,31 +849,15 @@ static int gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* m
   if (hd % 32 || half % 16 || dpos0 % 8 || sp->dst_t % 8 || !qkv_rows_ok(sp->B, sp->L) || p3v_tuning().gemm_no_qkv_fuse) return P3V_ERR_UNSUPPORTED;
   if ((size_t)a->M * a->lda * 2 >= (1ull << 32) || (size_t)a->N * a->ldw * 2 >= (1ull << 32)) return P3V_ERR_UNSUPPORTED;
   hipStream_t s = (hipStream_t)stream;
-  QkvP q = {sp->cos_t, sp->sin_t, sp->q_out, sp->k_dst, sp->v_dst, sp->L, nh, nkv, hd, sp->past, dpos0, sp->dst_t, sp->tab_t, sp->tab_div, 0,
+  QkvP q = {sp->cos_t, sp->sin_t, sp->q_out, sp->k_dst, sp->v_dst, sp->L, nh, nkv, hd, sp->past, dpos0, sp->dst_t, sp->tab_t, sp->tab_div,
             sp->q_scale};
   if (merge_ws) return p3v_gemm_skinny_qkv_merge(a, q, merge_ws, merge_bytes, s);
-  if (const int mb = qkv_tile_plan(a, q)) {
-    const int rc = p3v_gemm256_flat_qkv(a, q, mb, s);
-    if (rc != P3V_ERR_UNSUPPORTED) return rc;
-  }
-  if (a->M < 1024) return p3v_gemm_skinny_qkv(a, q, s);       // 17 .. 256 rows: the weight-streaming kernel (or "unsupported")
+  const int mb = qkv_tile_plan(a, q);
+  if (mb > 1) return p3v_gemm256_flat_qkv(a, q, mb, s);
+  if (!mb && a->M < 1024) return p3v_gemm_skinny_qkv(a, q, s);  // 17 .. 256 rows: the weight-streaming kernel (or "unsupported")
   if ((nh * hd) % BN || (nkv * hd) % BN || p3v_tuning().gemm_128) return P3V_ERR_UNSUPPORTED;
-  p3v_gemm_args_t plain = *a;
-  plain.epilogue = P3V_EPI_NONE;                                // (the row packing below prices the plain bf16 epilogue)
-  int rows_big = (nh * hd) % 256 || (nkv * hd) % 256 ? 0 : gemm_big_rows(&plain);
-  if (rows_big > 0) {
-    p3v_gemm_args_t top = *a;
-    top.M = rows_big;
-    const int rc = p3v_gemm256_qkv(&top, q, s);
-    if (rc == P3V_ERR_UNSUPPORTED) rows_big = 0;
-    else if (rc != P3V_OK) return rc;
-  }
-  if (rows_big < a->M) {
-    q.m_base = rows_big;
-    const GemmP p = {a->A + (size_t)rows_big * a->lda, a->W, nullptr, a->bias, nullptr, nullptr, a->M - rows_big, a->N, a->K, a->lda, a->ldw, 0, 0, 0, q};
-    return launch_gemm<P3V_EPI_QKV>(p, s);
-  }
-  return P3V_OK;
+  const GemmP p = {a->A, a->W, nullptr, a->bias, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0, 0, 0, q};
+  return launch_gemm<P3V_EPI_QKV>(p, s);
 }
 extern "C" int p3v_gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* stream) { return gemm_qkv(a, sp, nullptr, 0, stream); }
 extern "C" int p3v_gemm_qkv_merge(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* ws, int64_t ws_bytes, void* stream) {

@@ -287,14 +287,6 @@ static int launch_gemm256(const Gemm256P& p, int mb, int nb, hipStream_t s) {
 }
 int p3v_gemm_pc(const Gemm256P& p, int epi, int mb, int nb, hipStream_t s);       // p3v_gemm_pc.hip: the flat tiles
 
-// the qkv projection with split + RoPE + KV append in the epilogue (p3v_gemm_qkv, p3v_gemm.hip): rows of `a` on big tiles
-int p3v_gemm256_qkv(const p3v_gemm_args_t* a, const QkvP& q, hipStream_t s) {
-  if (a->N % 256 || a->K % TK || (q.nh * q.hd) % 256 || (q.nkv * q.hd) % 256) return P3V_ERR_UNSUPPORTED;
-  if ((size_t)a->N * a->ldw * 2 >= ((size_t)1 << 32) || (size_t)a->M * a->lda * 2 >= ((size_t)1 << 32)) return P3V_ERR_UNSUPPORTED;
-  const Gemm256P p = {a->A, a->W, nullptr, a->bias, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0, q};
-  return launch_gemm256<P3V_EPI_QKV>(p, 8, 4, s);
-}
-
 // called by p3v_gemm (which decides how many rows get the big tile); returns P3V_ERR_UNSUPPORTED to fall back
 int p3v_gemm256_try(const p3v_gemm_args_t* a, int mb, int nb, hipStream_t s) {
   // the tiles there are (the knob "gemm_tile" may ask for any); a gated epilogue needs whole gate / up pairs of a group of four column blocks

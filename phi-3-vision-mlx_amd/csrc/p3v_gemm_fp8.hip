@@ -711,7 +711,7 @@ extern "C" int p3v_gemm_qkv_fp8(const p3v_gemm_fp8_args_t* a, const p3v_qkv_spli
   if ((size_t)a->N * a->ldw >= ((size_t)1 << 32) || (size_t)a->M * a->lda >= ((size_t)1 << 32) || (size_t)256 * a->lda >= ((size_t)1 << 31) ||
       (size_t)256 * a->ldw >= ((size_t)1 << 31)) return P3V_ERR_UNSUPPORTED;                                  // 32-bit buffer offsets
   const GemmF8P p = {a->A, a->a_scale, a->W, a->w_scale, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0,
-                     {sp->cos_t, sp->sin_t, sp->q_out, sp->k_dst, sp->v_dst, sp->L, nh, nkv, hd, sp->past, dpos0, sp->dst_t, sp->tab_t, sp->tab_div, 0, sp->q_scale}};
+                     {sp->cos_t, sp->sin_t, sp->q_out, sp->k_dst, sp->v_dst, sp->L, nh, nkv, hd, sp->past, dpos0, sp->dst_t, sp->tab_t, sp->tab_div, sp->q_scale}};
   return launch_f8_v<P3V_EPI_QKV, 4, 4>(p, (hipStream_t)stream);
 }
 

@@ -1,5 +1,5 @@
 // The qkv projection with the head split, the rotation and the KV append in its epilogue: p3v_gemm_qkv =
-// p3v_gemm(qkv_proj) + p3v_rope_kv_append in the launches of the GEMM alone.  Shared by the 256 x 256 and the 128 x 128 tile kernels.
+// p3v_gemm(qkv_proj) + p3v_rope_kv_append in the launch of the GEMM alone.  Shared by the kernels of every tile.
 //
 // What makes it fit the accumulator layout (a lane holds 4 consecutive output columns of one row, p3v_gemm256_epi.h):
 //   * Q and K tiles: _rotate_half pairs dimension d with d + hd/2 (phi.py:419-423).  The tile's W rows are fetched in PAIR order --
@@ -7,7 +7,7 @@
 //     any W row for any tile row: the same trick as the SiLU epilogue's gate / up rows) -- so both halves of a pair sit in ONE lane
 //     (acc[i][j][r] and acc[i][j + 2][r]) and the rotation is lane-local.  16 pairs never straddle a head (hd/2 = 48 or 32).
 //   * V tiles: the cache keeps V TRANSPOSED ([.., hd, t]).  These tiles are computed with the operand roles swapped -- W rows fill the
-//     tile's A side, the tokens its B side (the tile is square and the K loop does not care) -- so a lane holds 4 consecutive TOKENS of
+//     tile's A side, the tokens its B side (a tile of R x 256 then holds R dimensions of 256 tokens; the K loop does not care) -- so a lane holds 4 consecutive TOKENS of
 //     one V dimension, and 8 after the v_permlane16_swap: one 16-byte store into a V^T row (rows whose length is not a multiple of 8
 //     -- CLIP's 577-token crops -- shift the run inside the row: still one dwordx4 store at even offsets, three stores at odd ones).
 // Arithmetic: exactly p3v_gemm's + p3v_rope_kv_append's (the Linear output rounded to bf16, rotation in fp32 on those values,
@@ -19,7 +19,6 @@ struct QkvP {
   const float* cos_t; const float* sin_t;        // [B / tab_div, tab_t, hd / 2] or both null: plain head split (CLIP)
   bf16_t* q_out; bf16_t* k_dst; bf16_t* v_dst;   // [B, nh, L, hd], [B, nkv, dst_t, hd], [B, nkv, hd, dst_t]
   int L, nh, nkv, hd, past, dpos0, dst_t, tab_t, tab_div;
-  int m_base;                                    // global token index of this launch's row 0 (rows after a big / small split)
   float q_scale;
 };
 
@@ -63,7 +62,7 @@ __device__ __forceinline__ void qkv_epilogue_rot_groups(const QkvP& q, f32x4_t (
     }
   // (b, l) of the lane's row in block 0; later blocks are 16 tokens further on (one division per tile, not per block)
   const int m00 = m_first + fc;
-  int b0 = 0, l0 = q.m_base + (m00 < M ? m00 : M - 1);
+  int b0 = 0, l0 = m00 < M ? m00 : M - 1;
   if (l0 >= q.L) { b0 = l0 / q.L; l0 -= b0 * q.L; }
   struct Turn { float4 cs[G][2], sn[G][2]; int bb[G], ll[G]; } ring[RING];
   auto ask = [&](int turn) {
@@ -170,7 +169,7 @@ __device__ __forceinline__ void qkv_epilogue_vt_groups(const QkvP& q, f32x4_t (&
 #pragma unroll
     for (int jp = 0; jp < 2; ++jp) {
       const int t = t_first + g * 64 + (2 * jp + (fq & 1)) * 16 + (fq >> 1) * 8;      // 8 consecutive tokens t .. t + 7
-      const int mg = q.m_base + t, b = mg < q.L ? 0 : mg / q.L, l = mg - b * q.L;
+      const int b = t < q.L ? 0 : t / q.L, l = t - b * q.L;
       tt[jp] = t, ll[jp] = l;
       run[jp] = q.v_dst + ((size_t)b * q.nkv * q.hd + fv_first + fc) * (size_t)q.dst_t + q.dpos0 + l;
       plain &= t + 8 <= M && l + 8 <= q.L && !(l & 1);

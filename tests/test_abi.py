@@ -317,6 +317,25 @@ def test_which_tile_runs_an_fp8_projection():
         l.p3v_set_tuning(b"gemm_f8_narrow", v.value)
 
 
+def test_which_tile_runs_a_qkv_projection():
+    """From 1024 rows on the fastest measured tile of (rows, rows of W for Q, for K and V, K): 128 x 128 ones at short K, every height at the decoder's
+    widths and the vision tower's; the knob names the same numbers; other regions, few rows and odd K are not priced."""
+    from phi_3_vision_mlx_amd import _lib
+    l, v, r = _lib.lib(), ctypes.c_int(), ctypes.c_int()
+    assert l.p3v_get_tuning(b"gemm_qkv_flat", ctypes.byref(v)) == 0 and l.p3v_get_tuning(b"gemm_big_rows", ctypes.byref(r)) == 0 and l.p3v_set_tuning(b"gemm_big_rows", -1) == 0
+    try:
+        for args, want in (((1536, 1536, 1536, 512), 1), ((8192, 1536, 1536, 512), 1), ((6000, 3072, 3072, 768), 1), ((1024, 1024, 1024, 256), 1), ((1154, 1024, 1024, 1024), 2),
+                           ((1536, 3072, 3072, 3072), 7), ((2048, 3072, 3072, 3072), 5), ((4096, 3072, 3072, 3072), 7), ((2531, 3072, 3072, 3072), 6), ((16384, 3072, 3072, 3072), 8),
+                           ((2885, 1024, 1024, 1024), 5), ((900, 3072, 3072, 3072), 5), ((2531, 3072, 3072, 100), 0), ((2531, 3072, 384, 3072), 0), ((256, 3072, 3072, 3072), 0), ((0, 3072, 3072, 3072), 0)):
+            assert l.p3v_set_tuning(b"gemm_qkv_flat", -1) == 0
+            assert l.p3v_gemm_qkv_tile(*args) == want, (args, l.p3v_gemm_qkv_tile(*args))
+            if want and args[0] >= 1024:
+                for pin in (1, 4, 8):
+                    assert l.p3v_set_tuning(b"gemm_qkv_flat", pin) == 0 and l.p3v_gemm_qkv_tile(*args) == pin
+    finally:
+        l.p3v_set_tuning(b"gemm_qkv_flat", v.value), l.p3v_set_tuning(b"gemm_big_rows", r.value)
+
+
 def test_which_decode_batches_run_one_workgroup_per_row_and_head():
     """(rows, new tokens, heads, kv heads, capacity) where the form was measured faster, and where it was not: an uneven second round
     of pairs, shared kv heads, few pairs, long caches."""

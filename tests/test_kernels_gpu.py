@@ -1046,23 +1046,23 @@ def test_prompt_on_planned_tiles_gives_the_row_packings_bits(ops, n):
         ops.set_tuning("gemm_big_rows", saved[0]), ops.set_tuning("gemm_128", saved[1])
 
 
-@pytest.mark.parametrize("B,L,nh,nkv,hd,K,past,rot,bias,big", [
-    (1, 2531, 32, 32, 96, 256, 0, True, False, -1),      # the bench prompt's shape (short K): big tiles + remainder rows, ragged end
-    (1, 2531, 32, 32, 96, 256, 0, True, False, 1000000),  # all rows on the 256 x 256 kernel
-    (1, 1300, 32, 32, 96, 128, 0, True, False, 0),        # all rows on the 128 x 128 kernel
-    (1, 1100, 8, 4, 96, 192, 64, True, False, 512),       # GQA regions of different widths, appended behind 64 cached keys
+@pytest.mark.parametrize("B,L,nh,nkv,hd,K,past,rot,bias,mb", [
+    (1, 2531, 32, 32, 96, 256, 0, True, False, -1),      # an image prompt's rows (short K), ragged end: the launcher's own tile
+    (1, 2531, 32, 32, 96, 256, 0, True, False, 8),        # 256 x 256 tiles
+    (1, 1300, 32, 32, 96, 128, 0, True, False, 1),        # 128 x 128 tiles
+    (1, 1100, 8, 4, 96, 192, 64, True, False, -1),        # GQA regions of different widths, no whole 256 columns (128 x 128 tiles), behind 64 cached keys
     (2, 1024, 16, 16, 64, 128, 0, False, True, -1),       # plain head split with bias (CLIP-like), two batch rows, L % 8 == 0
-    (3, 680, 16, 16, 64, 128, 8, True, True, 512),
+    (3, 680, 16, 16, 64, 128, 8, True, True, 1),
     # short prompts (17 .. 256 rows): the 128 x 64-tile weight-streaming kernel, Q / K tiles in pair order + V tiles with swapped roles
     (1, 128, 32, 32, 96, 256, 0, True, False, -1), (1, 100, 32, 32, 96, 192, 0, True, False, -1), (1, 17, 32, 32, 96, 128, 64, True, False, -1),
     (1, 250, 8, 4, 96, 192, 8, True, False, -1), (2, 64, 16, 16, 64, 128, 0, False, False, -1),
-    # round 6: batch rows whose length is not a multiple of 8 (CLIP: 577-token crops) -- the V^T runs fall on even and odd offsets and
+    # batch rows whose length is not a multiple of 8 (CLIP: 577-token crops) -- the V^T runs fall on even and odd offsets and
     # across row ends
-    (17, 577, 16, 16, 64, 1024, 0, False, True, -1), (5, 577, 16, 16, 64, 128, 0, False, True, 0), (3, 1001, 8, 4, 96, 128, 0, True, False, -1),
+    (17, 577, 16, 16, 64, 1024, 0, False, True, -1), (5, 577, 16, 16, 64, 128, 0, False, True, 1), (3, 1001, 8, 4, 96, 128, 0, True, False, -1),
     (4, 61, 16, 16, 64, 128, 0, False, False, -1), (3, 85, 8, 4, 96, 192, 0, True, False, -1),
     (20, 7, 16, 16, 64, 128, 0, True, False, -1), (150, 7, 16, 16, 64, 128, 8, True, False, -1),      # the shortest rows of a batch
 ])
-def test_gemm_qkv_fused(ops, B, L, nh, nkv, hd, K, past, rot, bias, big):
+def test_gemm_qkv_fused(ops, B, L, nh, nkv, hd, K, past, rot, bias, mb):
     """p3v_gemm_qkv (qkv projection with head split + rotation + KV append in its epilogue) against the two calls it replaces --
     p3v_gemm then p3v_rope_kv_append -- on the same inputs: rotated / scaled Q, the appended K rows and the appended V^T columns
     BIT-IDENTICAL, everything else in the caches untouched."""
@@ -1077,7 +1077,7 @@ def test_gemm_qkv_fused(ops, B, L, nh, nkv, hd, K, past, rot, bias, big):
     sin = torch.rand((B, T, half), device="cuda") if rot else None
     qs = 1.3
     k0, v0 = g((B, nkv, Tp, hd), 403).cuda(), g((B, nkv, hd, Tp), 404).cuda()
-    pinned = ops.set_tuning("gemm_big_rows", big)
+    pinned = ops.set_tuning("gemm_qkv_flat", mb)
     try:
         qkv = ops.gemm(a, w, ops.EPI_BIAS, bias=bq) if bias else ops.gemm(a, w)
         q1, k1, v1 = torch.empty((B, nh, L, hd), dtype=BF16, device="cuda"), k0.clone(), v0.clone()
@@ -1086,7 +1086,7 @@ def test_gemm_qkv_fused(ops, B, L, nh, nkv, hd, K, past, rot, bias, big):
         assert ops.gemm_qkv(a, w, cos, sin, q2, k2, v2, B, L, nh, nkv, hd, past, Tp, True, T, 1, q_scale=qs, bias=bq), "shape not taken"
         torch.cuda.synchronize()
     finally:
-        ops.set_tuning("gemm_big_rows", pinned)
+        ops.set_tuning("gemm_qkv_flat", pinned)
     assert torch.equal(q2, q1), f"Q differs ({(q2 != q1).sum().item()} elements)"
     assert torch.equal(k2, k1), f"K cache differs ({(k2 != k1).sum().item()} elements)"
     assert torch.equal(v2, v1), f"V^T cache differs ({(v2 != v1).sum().item()} elements)"
@@ -1258,11 +1258,11 @@ def test_gemm_qkv_fp8_fused(ops, B, L, nh, nkv, hd, K, past, rot):
     assert torch.equal(k2, k1) and torch.equal(v2, v1)
 
 
-@pytest.mark.parametrize("mb", [2, 3, 4, 5])
+@pytest.mark.parametrize("mb", [1, 2, 3, 4, 5])
 @pytest.mark.parametrize("B,L,nh,nkv,hd,K,past,rot,bias", [(1, 257, 8, 8, 96, 192, 0, True, False), (1, 641, 16, 8, 96, 64, 64, True, False), (3, 100, 16, 4, 64, 320, 0, True, False),
                                                            (2, 577, 16, 16, 64, 256, 0, False, True), (1, 1100, 32, 32, 96, 128, 8, True, False), (40, 7, 8, 8, 96, 448, 8, True, False)])
 def test_gemm_qkv_flat_tiles(ops, B, L, nh, nkv, hd, K, past, rot, bias, mb):
-    """p3v_gemm_qkv on every flat tile (ragged last rows, V regions that end inside a tile, several rounds of the chip, batch rows that start
+    """p3v_gemm_qkv on every flat tile and on 128 x 128 ones (1; ragged last rows, V regions that end inside a tile, several rounds of the chip, batch rows that start
     anywhere in a tile) against p3v_gemm, then p3v_rope_kv_append: the same bits, the rest of the caches untouched."""
     M, N = B * L, (nh + 2 * nkv) * hd
     a, w, bq = g((M, K), 420).cuda(), g((N, K), 421, 1.0 / math.sqrt(K)).cuda(), g((N,), 422, 0.5).cuda() if bias else None

@@ -111,8 +111,8 @@ def sweep_fp8(rows):
 
 
 def sweep_qkv(rows):
-    tiles = [2, 3, 4, 5, 6, 7, 8]
-    print("B x L, heads / kv x dim, K       M     own" + "".join(f"{t:>8}" for t in tiles) + "    (32 t rows a tile)")
+    tiles = [1, 2, 3, 4, 5, 6, 7, 8]
+    print("B x L, heads / kv x dim, K       M     own" + "".join(f"{t:>8}" for t in tiles) + "    (32 t rows a tile; 1: 128 x 128)")
     for B, L0, nh, nkv, hd, K in QKV:
         for L in [L0] if L0 else [r // B for r in rows]:
             M, N, Tp = B * L, (nh + 2 * nkv) * hd, (L + 127) // 128 * 128
