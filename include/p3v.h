@@ -100,9 +100,10 @@ typedef struct {
  * is only live between the two launches of one call, so calls on ONE stream may share it; concurrent streams need their
  * own.  Graph-capturable. */
 int p3v_gemm(const p3v_gemm_args_t* args /* host */, void* stream);
-/* The tile of a prompt-sized problem in one launch (host queries): 10 mb + nb for 32 mb rows x 64 nb columns of W, 0: rows split between 256 x 256
- * and 128 x 128 tiles, or one of the kernels for few rows (they come first, up to 256 rows).  p3v_gemm_plan: by whole rounds of the chip, without
- * the tiles of 192 rows; p3v_gemm_tile: what p3v_gemm runs, by how full the rounds are as well */
+/* The tile of a prompt-sized problem in one launch (host queries): 10 mb + nb for 32 mb rows x 64 nb columns of W, the value that the knob "gemm_tile" pins
+ * it with.  p3v_gemm_tile: what p3v_gemm runs with the workspace of p3v_gemm_ws_bytes, by a fitted time; 0: rows split between 256 x 256 and 128 x 128 tiles,
+ * 128 x 128 tiles alone, K slices (up to 1024 rows), or one of the kernels for few rows (up to 256).  p3v_gemm_plan: the older plan by whole rounds of the chip,
+ * without the tiles of 192 rows, the K slices and the kernels for few rows, which p3v_gemm_tile departs from where another tile promises 2 % */
 int p3v_gemm_plan(int M, int N, int K, int epilogue);
 int p3v_gemm_tile(int M, int N, int K, int epilogue);
 int64_t p3v_gemm_ws_bytes(int M, int N, int K, int epilogue);

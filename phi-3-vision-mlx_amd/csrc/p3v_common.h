@@ -212,7 +212,7 @@ static inline int p3v_gemv_wpw(int waves, int n_cu, int forced) {
 // it): no launch reads the environment.  -1 = "let the launcher decide".
 struct P3vTuning {
   int gemm_big_rows;        // rows given to the 256x256-tile GEMM (-1: cost model)
-  int gemm_tile;            // 10 mb + nb: pin the tile of the large GEMM (32 mb x 64 nb; of 192 rows: 164, 163); -1: cost model
+  int gemm_tile;            // 10 mb + nb: pin the tile of the large GEMM (32 mb x 64 nb); -1: cost model
   int gemm_no_splitk, gemm_splitk_max_m, gemm_splitk_max_s, gemm_splitk_wgs, gemm_128, gemm_persistent;
   int gemm_rows;            // 1: 9 .. 32 rows on the register-streaming kernel (p3v_gemm_rows.hip), 0: on the 64-row tiles of p3v_gemm_skinny.hip
   int gemm_no_skinny, gemm_skinny_max_m, gemm_skinny_s, gemm_skinny_tm128, gemm_no_merge;   // the 128 x 64-tile weight-streaming kernel for 17 .. max_m rows (p3v_gemm_skinny.hip)

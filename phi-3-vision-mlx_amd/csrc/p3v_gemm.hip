@@ -436,10 +436,13 @@ extern "C" int p3v_gemm_plan(int M, int N, int K, int epilogue) {
   return gemm_tile_plan(&a, p3v_tuning().gemm_128 ? 0 : gemm_big_rows(&a), &mb, &nb) ? 10 * mb + nb : 0;
 }
 
+int p3v_gemm_skinny_slices(int M, int N, int K, int epilogue);   // p3v_gemm_skinny.hip: 0 = not one of its shapes
+static int splitk_slices(int M, int N, int K, int epilogue);
 extern "C" int p3v_gemm_tile(int M, int N, int K, int epilogue) {
   if (M <= 0 || N <= 0 || K <= 0 || epilogue < 0 || epilogue > P3V_EPI_GELU_MUL) return 0;
   p3v_gemm_args_t a = {};
   a.M = M, a.N = N, a.K = K, a.epilogue = epilogue;
+  if (K % BK || p3v_gemm_skinny_slices(M, N, K, epilogue) || splitk_slices(M, N, K, epilogue) > 1) return 0;      // (p3v_gemm tries these first)
   return gemm_tile_choice(&a, p3v_tuning().gemm_128 ? 0 : gemm_big_rows(&a));
 }
 
@@ -571,7 +574,6 @@ static int splitk_slices(int M, int N, int K, int epilogue) {
   return S;
 }
 
-int p3v_gemm_skinny_slices(int M, int N, int K, int epilogue);   // p3v_gemm_skinny.hip: 0 = not one of its shapes
 int p3v_gemm_skinny_try(const p3v_gemm_args_t* a, hipStream_t s);
 
 extern "C" int64_t p3v_gemm_ws_bytes(int M, int N, int K, int epilogue) {
@@ -718,11 +720,7 @@ extern "C" int p3v_gemm(const p3v_gemm_args_t* a, void* stream) {
     if ((size_t)a->M * a->lda * 2 >= (1ull << 32) || w_rows * a->ldw * 2 >= (1ull << 32)) return P3V_ERR_UNSUPPORTED;
   }
   hipStream_t s = (hipStream_t)stream;
-  if (int t = p3v_tuning().gemm_tile; t > 0) {                   // (the tiles of 192 rows: 164 and 163)
-    if (t / 10 == 6) return P3V_ERR_UNSUPPORTED;
-    if (t / 10 == 16) t -= 100;
-    return p3v_gemm256_try(a, t / 10, t % 10, s);
-  }
+  if (const int t = p3v_tuning().gemm_tile; t > 0) return p3v_gemm256_try(a, t / 10, t % 10, s);
   if (!a->bias) {                                              // 17 .. 256 rows: the weight-streaming kernel (p3v_gemm_skinny.hip)
     const int rc = p3v_gemm_skinny_try(a, s);
     if (rc != P3V_ERR_UNSUPPORTED) return rc;

@@ -212,7 +212,7 @@ def test_fused_decode_attention_role_placement_is_a_bijection(n_split, mode):
     assert l.p3v_attention_decode_fused_role(G, nh, n_split, o_n, mode, out) == -22
 
 
-@pytest.mark.parametrize("tile", [1, 4, 40, 53, 64, 73, 80, 82, 94, 99, 844, -84])
+@pytest.mark.parametrize("tile", [1, 4, 40, 53, 62, 73, 80, 82, 94, 99, 164, 163, 844, -84])
 def test_a_pinned_gemm_tile_that_does_not_exist_is_refused(tile):
     """The knob "gemm_tile" takes any number: one that names no tile of the large GEMM kernels (or, gated, the 192-column ones) is an
     error code, not a division by zero and not another tile.  Negative: no pin.  A process of its own, since the fault would end it."""
@@ -225,11 +225,11 @@ l, buf = L.lib(), C.create_string_buffer(4096)
 p = (C.addressof(buf) + 15) // 16 * 16
 def gemm(M, epilogue):
     return l.p3v_gemm(C.byref(L.GemmArgs(p, p, p, 0, 0, 0, M, 768, 64, 64, 64, 768, epilogue, 0, 0, 0, 0)), None)
-for t, M in (({tile}, 64), (43, 64), (83, 64)):
+for t, M in (({tile}, 64), (43, 64), (63, 64), (83, 64)):
     assert l.p3v_set_tuning(b"gemm_tile", t) == 0
     if t < 0:
         assert gemm(0, ops.EPI_NONE) == 0
-    elif t not in (43, 83):
+    elif t not in (43, 63, 83):
         assert gemm(M, ops.EPI_NONE) == L.ERR_UNSUPPORTED, (t, gemm(M, ops.EPI_NONE))
     if t > 0:
         assert gemm(M, ops.EPI_SILU_MUL) == L.ERR_UNSUPPORTED and gemm(M, ops.EPI_GELU_MUL) == L.ERR_UNSUPPORTED, t
@@ -253,8 +253,8 @@ def test_k_slices_decline_partials_beyond_32_bit_offsets():
         l.p3v_set_tuning(b"gemm_slices", v.value)
 
 
-def test_which_tile_runs_a_prompt_sized_projection():
-    """One size for every tile, and sizes that stay on the row packing: where no tile promises enough, 224-row tiles for one full round
+def test_which_tile_the_plan_by_rounds_names():
+    """p3v_gemm_plan (what p3v_gemm departs from only for 2 %): one size for every tile, and sizes that stay on the row packing: where no tile promises enough, 224-row tiles for one full round
     (slower than 256 x 256 there), short K loops, few rows."""
     from phi_3_vision_mlx_amd import _lib, ops
     l, v = _lib.lib(), ctypes.c_int()
@@ -273,7 +273,7 @@ def test_which_tile_runs_a_prompt_sized_projection():
 
 def test_which_tile_p3v_gemm_runs():
     """The tile by how full the chip's rounds are: those of 192 rows and the other heights where they were measured the fastest, the plan's own
-    answer elsewhere, and for what is never priced (few rows, short K, a tile height that does not divide the columns)."""
+    answer elsewhere, and 0 for what other kernels take (few rows, K slices up to 1024 rows, short K, columns that no tile divides, a K that p3v_gemm refuses)."""
     from phi_3_vision_mlx_amd import _lib, ops
     l, v = _lib.lib(), ctypes.c_int()
     assert l.p3v_get_tuning(b"gemm_big_rows", ctypes.byref(v)) == 0 and l.p3v_set_tuning(b"gemm_big_rows", -1) == 0
@@ -281,7 +281,10 @@ def test_which_tile_p3v_gemm_runs():
         for M, N, K, epi, want in ((768, 8192, 3072, ops.EPI_SILU_MUL, 64), (2300, 8192, 3072, ops.EPI_SILU_MUL, 64), (2531, 8192, 3072, ops.EPI_SILU_MUL, 74),
                                    (2531, 9216, 3072, ops.EPI_NONE, 64), (900, 9216, 3072, ops.EPI_NONE, 63), (6000, 3072, 8192, ops.EPI_RESID_BF16, 63),
                                    (8192, 3072, 8192, ops.EPI_RESID_BF16, 83), (9809, 4096, 1024, ops.EPI_BIAS_QGELU, 74), (640, 8192, 3072, ops.EPI_SILU_MUL, 54),
+                                   (300, 3072, 3072, ops.EPI_NONE, 0), (500, 3072, 8192, ops.EPI_RESID_BF16, 0), (300, 3072, 3072, ops.EPI_BIAS, 43), (128, 8192, 3072, ops.EPI_SILU_MUL, 0),
+                                   (2531, 3072, 3080, ops.EPI_NONE, 0),
                                    (2531, 3072, 512, ops.EPI_NONE, 0), (256, 8192, 3072, ops.EPI_NONE, 0), (2531, 3000, 3072, ops.EPI_NONE, 0), (0, 3072, 3072, ops.EPI_NONE, 0)):
+            assert (l.p3v_gemm_ws_bytes(M, N, K, epi) > 0) <= (want == 0)
             assert l.p3v_gemm_tile(M, N, K, epi) == want, (M, N, K, epi, l.p3v_gemm_tile(M, N, K, epi))
     finally:
         l.p3v_set_tuning(b"gemm_big_rows", v.value)

@@ -928,7 +928,7 @@ def test_gemm_tiles_agree(ops, epi, M, N, K):
     saved = [ops.set_tuning(n, x) for n, x in zip(names, (-1, 1, 1, 1))]
     try:
         want = ops.gemm(a, w, **kw)
-        for tile in (84, 74, 83, 54, 44, 43):
+        for tile in (84, 74, 64, 83, 63, 54, 44, 43):
             if tile % 10 == 3 and gated:
                 continue
             ops.set_tuning("gemm_tile", tile)
@@ -939,19 +939,20 @@ def test_gemm_tiles_agree(ops, epi, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 768, 64), (193, 768, 128), (1111, 768, 192), (4001, 3072, 128), (2300, 9216, 64)])
-@pytest.mark.parametrize("epi", ["none", "silu", "resid_bf16", "resid_f32", "scale", "bias_qgelu", "f32"])
+@pytest.mark.parametrize("epi", ["none", "silu", "gelu", "resid_bf16", "resid_f32", "scale", "bias", "bias_qgelu", "bias_gelu", "f32"])
 def test_gemm_192_row_tiles_agree(ops, epi, M, N, K):
-    """The tiles of 192 rows (pinned as 164 and 163) as test_gemm_tiles_agree: one and several rounds, fewer K-tiles than LDS buffers, ragged rows."""
-    gated = epi == "silu"
+    """The tiles of 192 rows as test_gemm_tiles_agree: one and several rounds, fewer K-tiles than LDS buffers, ragged rows."""
+    gated = epi in ("silu", "gelu")
     a, w = g((M, K), 40).cuda(), g((2 * N if gated else N, K), 41, 1.0 / math.sqrt(K)).cuda()
     v, r = g((N,), 42, 0.5).cuda(), g((M, N), 43, 1.0, BF16 if epi == "resid_bf16" else F32).cuda()
     kw = {"none": {}, "silu": dict(epilogue=ops.EPI_SILU_MUL), "resid_bf16": dict(epilogue=ops.EPI_RESID_BF16, resid=r), "bias_qgelu": dict(epilogue=ops.EPI_BIAS_QGELU, bias=v),
+          "gelu": dict(epilogue=ops.EPI_GELU_MUL), "bias": dict(epilogue=ops.EPI_BIAS, bias=v), "bias_gelu": dict(epilogue=ops.EPI_BIAS_GELU, bias=v),
           "resid_f32": dict(epilogue=ops.EPI_BIAS_RESID_F32, resid=r, bias=v), "scale": dict(epilogue=ops.EPI_SCALE_RESID_F32, resid=r, col_scale=v), "f32": dict(epilogue=ops.EPI_F32)}[epi]
     names = ("gemm_tile", "gemm_128", "gemm_no_skinny", "gemm_no_splitk")
     saved = [ops.set_tuning(n, x) for n, x in zip(names, (-1, 1, 1, 1))]
     try:
         want = ops.gemm(a, w, **kw)
-        for tile in (164,) if gated else (164, 163):
+        for tile in (64,) if gated else (64, 63):
             ops.set_tuning("gemm_tile", tile)
             assert torch.equal(ops.gemm(a, w, **kw), want), f"tile {tile}"
     finally:
@@ -983,7 +984,7 @@ def test_gated_epilogues_on_every_finite_gate(ops, epi, tile):
     assert not (err > 0).any() and torch.isfinite(got).all(), [(x.item(), y.item()) for x, y in zip(g64[~(err <= 0)][:4], got[:, :8][~(err <= 0)][:4])]
 
 
-@pytest.mark.parametrize("tile", [-1, 84, 44])
+@pytest.mark.parametrize("tile", [-1, 84, 63, 44])
 def test_erf_gelu_on_every_finite_input(ops, tile):
     """x P(x) for every finite 16-bit x against 64 bits: 8e-6 and one rounding to bf16 (2^-9) are below 2^-8; where exp(-x^2 / 2) is below 2^-126, beyond |x| = 13.3, it
     may be 0.  Infinities and NaN as the plain formula has them."""
@@ -1006,9 +1007,10 @@ def test_erf_gelu_on_every_finite_input(ops, tile):
     assert torch.equal(got[:, 16:24], got[:, :8]) and (got[:, 8] == math.inf).all() and torch.isnan(got[:, 9:11]).all()
 
 
-@pytest.mark.parametrize("M,N,K,gated,tile", [(385, 9216, 1024, False, 43), (641, 9216, 2048, False, 44), (257, 6144, 2048, True, 44), (1300, 6144, 1024, False, 54),
-                                              (385, 9216, 1024, True, 54), (1300, 9216, 1024, False, 74), (500, 9216, 1024, True, 74), (1793, 6144, 1024, False, 83),
-                                              (700, 9216, 1024, True, 84)])
+@pytest.mark.parametrize("M,N,K,gated,tile", [(257, 1536, 2048, False, 43), (257, 2048, 2048, False, 44), (2087, 4096, 1024, False, 54), (1294, 6144, 1024, False, 63),
+                                              (2575, 4096, 1024, False, 64), (1355, 9216, 1024, False, 74), (1660, 6144, 1024, False, 83), (920, 16384, 1024, False, 84),
+                                              (257, 6144, 1024, True, 44), (1294, 3072, 1024, True, 54), (501, 9216, 1024, True, 64), (623, 9216, 1024, True, 74),
+                                              (684, 9216, 1024, True, 84)])
 def test_gemm_runs_the_planned_tile(ops, M, N, K, gated, tile):
     """The launcher's own choice (no pin) for one size of every tile and kind of epilogue, against the 128 x 128 tiles bit for bit."""
     epi = ops.EPI_SILU_MUL if gated else ops.EPI_BIAS_QGELU
@@ -1016,7 +1018,7 @@ def test_gemm_runs_the_planned_tile(ops, M, N, K, gated, tile):
     kw = {} if gated else dict(bias=v)
     saved = ops.set_tuning("gemm_big_rows", -1), ops.set_tuning("gemm_128", 0)
     try:
-        assert ops.L.lib().p3v_gemm_plan(M, N, K, epi) == tile
+        assert ops.L.lib().p3v_gemm_tile(M, N, K, epi) == tile
         got = ops.gemm(a, w, epi, **kw)
         ops.set_tuning("gemm_128", 1)
         assert torch.equal(got, ops.gemm(a, w, epi, **kw))
@@ -1026,7 +1028,7 @@ def test_gemm_runs_the_planned_tile(ops, M, N, K, gated, tile):
 
 @pytest.mark.parametrize("n", [700, 1300, 2531])
 def test_prompt_on_planned_tiles_gives_the_row_packings_bits(ops, n):
-    """A prompt of the decoder's own widths (two layers) with the tiles the launcher plans -- the tests' default pins the row packing -- and
+    """A prompt of the decoder's own widths (two layers) with the tiles the launcher chooses -- the tests' default pins the row packing -- and
     with 128 x 128 tiles alone: logits and the layers' caches bit for bit."""
     from phi_3_vision_mlx_amd.api import load_synthetic
     from phi_3_vision_mlx_amd.config import phi3v_config_dict
@@ -1035,7 +1037,7 @@ def test_prompt_on_planned_tiles_gives_the_row_packings_bits(ops, n):
     cfg, l = model.cfg, ops.L.lib()
     saved = ops.set_tuning("gemm_big_rows", -1), ops.set_tuning("gemm_128", 0)
     try:
-        assert any(l.p3v_gemm_plan(n, N, K, e) for N, K, e in ((cfg.hidden_size, cfg.hidden_size, ops.EPI_RESID_BF16), (cfg.intermediate_size, cfg.hidden_size, ops.EPI_SILU_MUL),
+        assert any(l.p3v_gemm_tile(n, N, K, e) for N, K, e in ((cfg.hidden_size, cfg.hidden_size, ops.EPI_RESID_BF16), (cfg.intermediate_size, cfg.hidden_size, ops.EPI_SILU_MUL),
                                                                 (cfg.hidden_size, cfg.intermediate_size, ops.EPI_RESID_BF16)))
         got, cache = model(input_ids=ids, max_tokens=4)
         got, k, v = got.clone(), cache[0].state.k[..., :n, :].clone(), cache[0].state.v[..., :n].clone()
