@@ -254,8 +254,8 @@ def test_k_slices_decline_partials_beyond_32_bit_offsets():
 
 
 def test_which_tile_the_plan_by_rounds_names():
-    """p3v_gemm_plan (what p3v_gemm departs from only for 2 %): one size for every tile, and sizes that stay on the row packing: where no tile promises enough, 224-row tiles for one full round
-    (slower than 256 x 256 there), short K loops, few rows."""
+    """p3v_gemm_plan (what p3v_gemm departs from only for 2 %): one size for every tile, and sizes that stay on the row packing: where no tile
+    promises enough, 224-row tiles for one full round (by the plan slower than 256 x 256 there), short K loops, few rows."""
     from phi_3_vision_mlx_amd import _lib, ops
     l, v = _lib.lib(), ctypes.c_int()
     assert l.p3v_get_tuning(b"gemm_big_rows", ctypes.byref(v)) == 0 and l.p3v_set_tuning(b"gemm_big_rows", -1) == 0

@@ -94,9 +94,11 @@ EPI_CASES = [
 
 
 @pytest.mark.parametrize("epi,M,N,K", EPI_CASES)
-def test_gemm(ops, epi, M, N, K):
-    # (conftest pins P3V_GEMM_BIG_ROWS=512, so every M >= 1024 case runs rows [0,512) on the big-tile kernel and the
-    #  rest on the small one: both kernels and the row offsets of A / out / resid are exercised on small shapes)
+def test_gemm(ops, request, epi, M, N, K):
+    # (pinned so that every M >= 1024 case runs rows [0,512) on the big-tile kernel and the rest on the small one: both
+    #  kernels and the row offsets of A / out / resid are exercised on small shapes)
+    pinned = ops.set_tuning("gemm_big_rows", 512)
+    request.addfinalizer(lambda: ops.set_tuning("gemm_big_rows", pinned))
     a = g((M, K), 10)
     nw = 2 * N if epi == "silu" else N
     w = g((nw, K), 11, 1.0 / math.sqrt(K))
@@ -138,8 +140,8 @@ def test_gemm(ops, epi, M, N, K):
 @pytest.mark.parametrize("epi,M,N,K", [("none", 2531, 9216, 3072), ("silu", 2531, 8192, 3072), ("resid_bf16", 2531, 3072, 3072),
                                        ("resid_f32", 9809, 1024, 1024), ("bias", 9809, 3072, 1024), ("none", 4096, 4096, 512)])
 def test_gemm_round_packing(ops, epi, M, N, K):
-    """The bench request's prefill shapes with the row split p3v_gemm's round-packing model picks (no pin), then all-big
-    and all-small tiles: the three must agree bit for bit (same K order, same epilogue arithmetic per element)."""
+    """The bench request's prefill shapes on the tile p3v_gemm chooses (no pin), then on all-big and all-small tiles: the three must agree
+    bit for bit (same K order, same epilogue arithmetic per element)."""
     a = g((M, K), 30).cuda()
     w = g(((2 * N if epi == "silu" else N), K), 31, 1.0 / math.sqrt(K)).cuda()
     bias = g((N,), 32, 0.5).cuda()
@@ -1028,7 +1030,7 @@ def test_gemm_runs_the_planned_tile(ops, M, N, K, gated, tile):
 
 @pytest.mark.parametrize("n", [700, 1300, 2531])
 def test_prompt_on_planned_tiles_gives_the_row_packings_bits(ops, n):
-    """A prompt of the decoder's own widths (two layers) with the tiles the launcher chooses -- the tests' default pins the row packing -- and
+    """A prompt of the decoder's own widths (two layers) with the tiles the launcher chooses and
     with 128 x 128 tiles alone: logits and the layers' caches bit for bit."""
     from phi_3_vision_mlx_amd.api import load_synthetic
     from phi_3_vision_mlx_amd.config import phi3v_config_dict
