@@ -318,17 +318,18 @@ static int launch_gemm(const GemmP& p, hipStream_t s) { return launch_gemm_v<EPI
 int p3v_gemm256_try(const p3v_gemm_args_t* a, int mb, int nb, hipStream_t s);   // p3v_gemm256.hip: tiles of 32 mb x 64 nb, P3V_ERR_UNSUPPORTED if the shape does not fit
 static int gemm128(const p3v_gemm_args_t* a, hipStream_t s);
 
-// How many leading rows go to the 256x256 kernel (a multiple of 256, or M for all of them); the rest runs on the
-// 128x128 kernel in a second launch on the same stream.  The machine holds 256 big workgroups or 512 small ones
-// per round; a round of big tiles costs 1, a round of small ones 0.675 (half the output area at 0.97 vs 1.31
-// PFLOP/s), a last round that leaves every CU at most one small workgroup 0.42 -- pick the cheapest whole-round
-// packing, e.g. 2531 x 16384 (gate_up): 8 x 64 = 512 big tiles = 2 rounds + 4 x 128 small = 1 round.
+// How many leading rows go to the 256 x 256 kernel (a multiple of 256, or M for all of them); the rest runs on the 128 x 128 kernel in a second
+// launch on the same stream.  The machine holds 256 big workgroups or 512 small ones per round; a round of big tiles costs 1, a round of small ones
+// 0.675, a last round that leaves every CU at most one small workgroup 0.42 -- the cheapest whole-round packing, e.g. 2531 x 16384 (gate_up): 8 x 64 =
+// 512 big tiles = 2 rounds + 4 x 128 small = 1 round.  It runs where gemm_tile_choice names no tile: short K (< 1024), columns that no tile divides, and
+// sizes where no tile promises 2 %.  The prices were measured on the eight-wave form of the big tile (1.31 PFLOP/s; 1.40 - 1.55 on four waves), a shorter
+// K's on its 128-KiB prologue and staged epilogue; they have not been taken again.
 static int gemm_big_rows(const p3v_gemm_args_t* a) {
   const int n_big = P3V_GATED(a->epilogue) ? 128 : 256, n_small = n_big / 2;
   if (a->M < 1024 || a->N % n_big || a->epilogue == P3V_EPI_PATCH) return 0;
   if (const int force = p3v_tuning().gemm_big_rows; force >= 0) return min(force / 256 * 256, a->M);   // tests: pin the split
   const int mt = p3v_cdiv(a->M, 256), nt_big = a->N / n_big, nt_small = p3v_cdiv(a->N, n_small);
-  // a short K loop leaves the big tile's 128-KiB prologue and four-pass epilogue exposed (one workgroup per CU)
+  // a short K loop leaves the big tile's prologue and epilogue exposed (one workgroup per CU)
   const float big_round = a->K >= 2048 ? 1.0f : 1.0f + 0.25f * (2048 - a->K) / 1024.f;
   float best = 1e30f;
   int best_rows = 0;
@@ -346,17 +347,13 @@ static int gemm_big_rows(const p3v_gemm_args_t* a) {
   return best_rows;
 }
 
-// Which tile runs the whole problem in one launch (*mb, *nb: a tile of 32 mb x 64 nb), or false: the packing above (or 128 x 128 tiles).
-// A launch lasts whole rounds of the chip's workgroups, so what counts is how a tile height divides the rows: 2531 x 3072 is 120
-// tiles of 256 x 256 (half the chip idle) but 240 of 128 x 256.  Times of one round in us, K-tiles of 64 = t, fitted to M = 1100 .. 9809 x
-// the decoder's and the vision tower's projections: the flat tiles of p3v_gemm_pc.hip 6.6 + 0.69 t (128 x 256), 7.9 + 0.79 t (160 x 256),
-// 5.5 + 0.61 t (128 x 192); the tall ones of p3v_gemm256.hip 9.5 + 1.28 t (256 x 256), 8.2 + 1.27 t (224 x 256), 8.1 + 1.11 t (256 x 192), a
-// twentieth more per K-tile from the second round on (power); 512 tiles of 128 x 128 6.0 + 0.785 t, up to 256 of them 4.4 + 0.635 t.  A tile
-// has to promise 5 %; short K loops (< 1024) stay.  The fit is for full rounds: of the sizes measured (profiles/gemm_tile_plan_sweep.txt) no choice
-// is slower than the packing by more than the runs differ; some are not the fastest tile, most of all below 1300 rows, where rounds of less
-// than 160 workgroups are faster than the fit says (1154 x 3072 x 8192 95, 128 x 192 69).
-// Measured (us, before -> now): 2531 x 3072 x 8192 117 -> 105, 2048 x 9472 x 3072 114 -> 97, 9809 x 1024 x 4096 (+ fp32 residual) 95 -> 73,
-// 4096 x 3072 x 8192 174 -> 163, 640 x 16384 x 3072 (gate | up) 103 -> 58.
+// The plan by whole rounds (*mb, *nb: a tile of 32 mb x 64 nb), or false: the packing above (or 128 x 128 tiles).  A launch lasts whole rounds of the
+// chip's workgroups, so what counts is how a tile height divides the rows: 2531 x 3072 is 120 tiles of 256 x 256 (half the chip idle) but 240 of
+// 128 x 256.  Times of one round in us, K-tiles of 64 = t, fitted to M = 1100 .. 9809 x the decoder's and the vision tower's projections: the flat tiles of
+// p3v_gemm_pc.hip 6.6 + 0.69 t (128 x 256), 7.9 + 0.79 t (160 x 256), 5.5 + 0.61 t (128 x 192); the tall ones 9.5 + 1.28 t (256 x 256), 8.2 + 1.27 t (224 x
+// 256), 8.1 + 1.11 t (256 x 192), a twentieth more per K-tile from the second round on (power); 512 tiles of 128 x 128 6.0 + 0.785 t, up to 256 of them 4.4 +
+// 0.635 t.  A tile has to promise 5 %; short K loops (< 1024) stay.  The tall tiles' times are those of their eight-wave form (the four-wave one: 8.3 + 1.2 t
+// at a full chip, gemm_tile_choice), so this is not what p3v_gemm runs: it is the choice's starting point, and the qkv projection's rule below 1024 rows.
 static bool gemm_tile_plan(const p3v_gemm_args_t* a, int rows_big, int* mb, int* nb) {
   const bool gated = P3V_GATED(a->epilogue);
   if (a->M <= 256 || a->K < 1024 || a->epilogue == P3V_EPI_PATCH || p3v_tuning().gemm_128 || p3v_tuning().gemm_big_rows >= 0) return false;
@@ -387,9 +384,10 @@ static bool gemm_tile_plan(const p3v_gemm_args_t* a, int rows_big, int* mb, int*
 // (power: 24 workgroups of 256 x 256 over 128 K-tiles 137 us, 240 of them 155), and the tiles of 192 rows are priced here alone.  t K-tiles, r
 // rounds of which u are filled: once + r (f + c t) + u fill t, and per round what a gated, a 32-bit residual or a GELU epilogue takes more; fitted to
 // 20 heights, 257 .. 9809 rows, of eight projections of the decoder and the vision tower with their weights from memory (3 - 5 % of a time at
-// most sizes).  Another tile than the plan's has to promise 2 %; what it then runs is within 0.6 % of the fastest measured tile on average, 5 % at
-// most beyond 1000 rows.  Measured (us, the plan on these kernels -> this): 2300 x 16384 x 3072 (gate | up) 192 -> 169, 2531 193 -> 187, 768 67 ->
-// 60; 2531 x 9216 x 3072 115 -> 107, 4096 175 -> 163; 3072 x 8192: 6000 rows 238 -> 219, 8192 313 -> 286; 2048 x 10496 x 3072 117 -> 107.
+// most sizes).  Another tile than the plan's has to promise 2 %.  Where it names a tile, that is within 0.3 % of the fastest measured one on average, 8.7 %
+// at most below 1000 rows and 6.4 % beyond (profiles/gemm_bf16_tile_sweep.txt, 130 sizes).  Measured (us, the plan on these kernels -> this): 2300 x 16384 x 3072
+// (gate | up) 192 -> 169, 2531 193 -> 187, 768 67 -> 60; 2531 x 9216 x 3072 115 -> 107, 4096 175 -> 163; 3072 x 8192: 6000 rows 238 -> 219, 8192 313 -> 286;
+// 2048 x 10496 x 3072 117 -> 107.
 static int gemm_tile_choice(const p3v_gemm_args_t* a, int rows_big) {
   int mb = 0, nb = 0;
   const int plan = gemm_tile_plan(a, rows_big, &mb, &nb) ? 10 * mb + nb : 0;

@@ -3,8 +3,9 @@
 //   256(M) x 256(N) x 64(K) tile (template: 224 or 192 rows, or 192 columns, for problems whose rounds they fill better), 256 threads = 4 waves as
 //   2(M) x 2(N), one per SIMD, each 128 x 128 = 8 x 8 v_mfma_f32_16x16x32_bf16 blocks: 256 accumulation registers, 4 MFMAs per LDS fragment read.
 //   Why     what bounds it is power and the LDS: with 8 waves of 128 x 64 (2.67 MFMAs a fragment) a K-tile's fragment reads and its LDS-DMA
-//           together take all 2048 cycles of its MFMAs at 128 B a cycle; with 128 x 128 a wave reads a third less.  Matrix pipe busy 0.62 -> 0.76 of
-//           the cycles, at a lower clock (1.87 GHz) for the same power.
+//           together take all 2048 cycles of its MFMAs at 128 B a cycle; with 128 x 128 a wave reads a third less.  Matrix pipe busy of the CUs' cycles,
+//           8 waves -> 4: 4096 x 4096 x 8192 0.73 -> 0.84, gate | up of 2531 rows 0.64 -> 0.76, at a lower clock for the same power (1.98 -> 1.84 GHz,
+//           2.21 -> 2.06; profiles/gemm256_four_waves_pmc.txt).
 //   Loop    half a K-tile (64 MFMAs) is multiplied while the other half's 16 fragments are read, one every two MFMAs; ONE barrier per K-tile, in
 //           the first half, where this K-tile is in registers and the next one in LDS: the buffers change hands there, and the requests of K-tiles
 //           to come go out one every six MFMAs from then on (LDS-DMA, 1 KiB each; W three K-tiles ahead, A two, or three where 160 KiB hold
@@ -84,8 +85,8 @@ __global__ void __launch_bounds__(256, 1) k_gemm256(Gemm256P p) {
 
   // ---- REQUESTS.  One = 8 tile rows x 128 B (1 KiB) of LDS-DMA by a wave, 32 rows by all four; the 16-byte chunks of a row are swizzled on
   // the source side.  Buffer addressing (SGPR descriptor + 32-bit per-lane byte offset + SGPR K offset): no vector ALU work at all.
-  // W, which comes from memory, runs three K-tiles ahead of the products, A, which the launch before wrote, SA; behind the last K-tile both repeat it (into buffers that nobody reads any more), so
-  // that every K-tile has the same requests and the counted waits hold to the end.
+  // W, which comes from memory, runs three K-tiles ahead of the products, A, which the launch before wrote, SA; behind the last K-tile both repeat it
+  // (into buffers that nobody reads any more), so that every K-tile has the same requests and the counted waits hold to the end.
   const int sw = ((tid & 7) ^ ((tid >> 3) & 7)) * 8;
   Aim256 aim;
   int wa = blockIdx.x, ka = 0, wb = blockIdx.x, kb = 0;           // the K-tiles to be requested next: output tile, K

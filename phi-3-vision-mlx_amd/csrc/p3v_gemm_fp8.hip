@@ -19,7 +19,8 @@
 //             multiply (k_gemm_f8_w4).
 //             What bounds it: the requests, 60 ns per four 1-KiB pieces of a CU with the weights from memory, 40 with all of it in the L2s
 //             (a K-tile of 192 x 256, 0.64 us of MFMAs, takes 0.81 - 0.85 and 0.73 where 12 - 60 CUs are at it), and, with all CUs at it, the
-//             chip's power (0.97 - 1.03): the same launches on all-zero operands are 20-25 % faster.  The tall tiles against the flat ones, us, weights from memory, launch behind launch: gate | up (16384 x 3072) 2300 rows
+//             chip's power (0.97 - 1.03): the same launches on all-zero operands are 20-25 % faster.  The tall tiles against the flat ones, us, weights
+//             from memory, launch behind launch: gate | up (16384 x 3072) 2300 rows
 //             122 -> 93, 2531 124 -> 106, 4096 198 -> 164, 8192 367 -> 327 (2.5 PFLOP/s); 9216 x 3072 2531 rows 71 -> 61, 4096 106 -> 97; 3072 x 8192
 //             3500 92 -> 69, 4096 99 -> 79; 3072 x 3072 4096 50 -> 37.  One round of flat tiles that fills the chip stays ahead of one of tall ones
 //             that does not: 3072 x 8192 at 2531 rows 59 (128 rows), 62 (192).

@@ -37,8 +37,8 @@ __device__ __forceinline__ int qkv_pair_row(const QkvP& q, int row0, int p0, int
 // Q / K tile: acc[g][i][j] = block row i (16 tokens from m_first) of column group g, blocks 0, 1 = first halves of pairs pw + 32 g .. + 31,
 // blocks 2, 3 = second.  The rotation tables cost 4 sixteen-byte loads per block row and group: requested G block rows at a time, a turn.
 // W4 (p3v_gemm256.hip, one wave per SIMD: nothing else covers a trip to memory): three turns' tables are on their way while a fourth's row is
-// rotated (256 rows x 9216 x 3072 in one round 77 -> 67 us), the sums stay in accumulation registers until their row's turn (p3v_gemm256_epi.h), and rows beyond M, which that kernel's
-// requests clamp to row M - 1, are stored as that row, bit for bit, instead of being branched around.
+// rotated (256 rows x 9216 x 3072 in one round 77 -> 67 us), the sums stay in accumulation registers until their row's turn (p3v_gemm256_epi.h), and
+// rows beyond M, which that kernel's requests clamp to row M - 1, are stored as that row, bit for bit, instead of being branched around.
 template <int NI, int G, bool W4, int NG>
 __device__ __forceinline__ void qkv_epilogue_rot_groups(const QkvP& q, f32x4_t (&acc)[NG][NI][4], const bf16_t* bias, bool is_k, int row0, int pw,
                                                         int m_first, int M, int lane) {
