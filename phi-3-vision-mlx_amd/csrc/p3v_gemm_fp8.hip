@@ -681,11 +681,12 @@ extern "C" int p3v_gemm_fp8(const p3v_gemm_fp8_args_t* a, void* stream) {
   }
 }
 
-// Whether one launch beats the two.  It writes and reads 47 MB less (2531 rows), but runs on 128 x 256 tiles alone; the split + rotation take 3.7 us +
-// 7.9 ns a row of 9216, half as much again for rows beyond 120 MB.  Both sides as in f8_tile_plan, fitted to 48 sizes (24 of K = 3072, 32 + 32 + 32 heads; shared
-// kv heads, K = 384 .. 1024); one has to promise 3 %.  It names the slower way at one of them, by 1 %.  us, two : one at K = 3072: 577 rows 33.0 : 31.0, 768
-// 37.0 : 32.1, 2531 86 : 85, 8192 267 : 238, 16384 493 : 459, but 256 25.3 : 30.4, 1024 41.7 : 49.7, 2300 79 : 83, where tiles of other heights fill their rounds;
-// 2531 rows of 3072 x 1024 25 : 18.
+// Whether one launch beats the two.  It writes and reads 47 MB less (2531 rows), but runs on 128 x 256 tiles alone.  Both sides as in f8_tile_plan; the split +
+// rotation, 3.5 us + 8.8 ns a row of 9216 and two fifths more beyond 40 MB of outputs, are what makes the rule agree best with 30 whole prompts of 256 .. 7000
+// tokens at the decoder's widths run either way (it names the slower one for five, by 2.4 us a layer at most) and with 24 sizes of other widths launch
+// behind launch.  (Launch behind launch, with the projection's outputs in the caches, they would be 3.7 us + 7.9 ns, and 2531 tokens would go the slower
+// way by 13 us.)  us a layer, two - one, in a prompt: 768 tokens 5, 2531 13, 4096 37, 6000 16, but 256 -5, 1024 -7, 1800 -10, 2700 -11, where tiles of
+// other heights fill their rounds; 8192 -15, where the rule says one (launch behind launch: +30).
 // (Tiles of 192 and 224 rows on four waves under this epilogue, with one wave per SIMD to run it: no faster than the faster of the two at any size.)
 extern "C" int p3v_gemm_qkv_fp8_pays(int M, int n_q, int n_kv, int K) {
   if (M <= 0 || K <= 0 || n_q <= 0 || n_kv <= 0 || n_q % 256 || n_kv % 256) return 0;
@@ -694,8 +695,7 @@ extern "C" int p3v_gemm_qkv_fp8_pays(int M, int n_q, int n_kv, int K) {
   const float kt = (float)(K / TKB), out = (float)M * (float)N;
   const long tiles = (long)(n_q + n_kv) / 256 * p3v_cdiv(M, 128) + (long)n_kv / 128 * p3v_cdiv(M, 256);
   const float one = 6.66f + p3v_cdiv(tiles, (long)n_cu) * (1.73f + 0.62f * kt) + (float)tiles / (float)n_cu * (0.2f * kt + 4.23f);
-  const float two = f8_tile_plan(M, N, K, N, P3V_EPI_NONE, mb, nb) + 3.7f + 8.6e-7f * out + 5e-7f * fmaxf(out - 6e7f, 0.f);
-  return 1.03f * one < two;
+  return one < f8_tile_plan(M, N, K, N, P3V_EPI_NONE, mb, nb) + 3.5f + 9.5e-7f * out + 4e-7f * fmaxf(out - 2e7f, 0.f);
 }
 
 // p3v_gemm_fp8 (epilogue NONE) + p3v_rope_kv_append in one launch, bit for bit, on 128 x 256 tiles: the projection's 47 MB (2531 rows) are

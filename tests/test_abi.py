@@ -311,8 +311,8 @@ def test_which_tile_runs_an_fp8_projection():
                                    (2531, 8192, 3072, ops.EPI_SILU_MUL, 74), (2048, 8192, 2944, ops.EPI_SILU_MUL, 84), (2531, 3072, 8192, ops.EPI_RESID_BF16, 44),
                                    (4096, 3072, 3072, ops.EPI_RESID_BF16, 74)):
             assert l.p3v_gemm_fp8_tile(M, N, K, epi) == want, (M, N, K, epi, l.p3v_gemm_fp8_tile(M, N, K, epi))
-        for M, n_q, n_kv, K, want in ((256, 3072, 3072, 3072, 0), (577, 3072, 3072, 3072, 1), (768, 3072, 3072, 3072, 1), (1024, 3072, 3072, 3072, 0), (2048, 3072, 3072, 3072, 0),
-                                      (2300, 3072, 3072, 3072, 0), (8192, 3072, 3072, 3072, 1), (16384, 3072, 3072, 3072, 1), (2531, 1024, 1024, 1024, 1), (1536, 768, 768, 384, 1)):
+        for M, n_q, n_kv, K, want in ((256, 3072, 3072, 3072, 0), (577, 3072, 3072, 3072, 1), (768, 3072, 3072, 3072, 1), (1024, 3072, 3072, 3072, 0), (1800, 3072, 3072, 3072, 0), (2048, 3072, 3072, 3072, 0),
+                                      (2531, 3072, 3072, 3072, 1), (2700, 3072, 3072, 3072, 0), (4096, 3072, 3072, 3072, 1), (6000, 3072, 3072, 3072, 1), (8192, 3072, 3072, 3072, 1), (16384, 3072, 3072, 3072, 1), (2531, 1024, 1024, 1024, 1), (1536, 768, 768, 384, 1)):
             assert l.p3v_gemm_qkv_fp8_pays(M, n_q, n_kv, K) == want, (M, n_q, n_kv, K)
         for M, N, K, epi in ((0, 256, 256, ops.EPI_NONE), (1, 100, 256, ops.EPI_NONE), (1, 256, 64, ops.EPI_NONE), (1, 256, 256, ops.EPI_GELU_MUL)):
             assert l.p3v_gemm_fp8_tile(M, N, K, epi) == 0
