@@ -56,7 +56,7 @@ def in_turn(knob, pins, run, flops, rate):
     return [x[len(x) // 2] if x else None for x in t]
 
 
-def row(label, M, choice, times, per):
+def row(label, M, choice, times, per):                           # choice: the tile of the library's own choice
     print(f"{label:<28}{M:>6}{choice:>8}" + "".join(f"{t / per:>8.1f}" if t else f"{'-':>8}" for t in times), flush=True)
 
 
@@ -66,7 +66,7 @@ def weights(n, k, bytes_each, make):
 
 def sweep_bf16(rows):
     tiles = [84, 74, 64, 83, 63, 54, 44, 43]
-    print("N x K (epilogue)                 M  choice" + "".join(f"{t:>8}" for t in tiles))
+    print("N x K (epilogue)                 M  choice     own" + "".join(f"{t:>8}" for t in tiles) + "    (own: the choice itself, no pin)")
     for N, K, epi in BF16:
         wn = 2 * N if epi == "silu" else N
         w = weights(wn, K, 2, lambda n, k: (torch.randn((n, k), device="cuda") * k ** -0.5).bfloat16())
@@ -84,7 +84,7 @@ def sweep_bf16(rows):
                     ops.gemm(a[i % 2], x, out=out, **kw)
                 return True
             times = in_turn("gemm_tile", [-1] + tiles, run, len(w) * 2.0 * M * wn * K, 1.1e15)
-            row(f"{N}{'(x2)' if epi == 'silu' else ''} x {K} {epi}", M, f"{times[0] / len(w):.1f}/{_lib.lib().p3v_gemm_tile(M, N, K, kw['epilogue'])}", times[1:], len(w))
+            row(f"{N}{'(x2)' if epi == 'silu' else ''} x {K} {epi}", M, _lib.lib().p3v_gemm_tile(M, N, K, kw["epilogue"]), times, len(w))
 
 
 def sweep_fp8(rows):
@@ -112,7 +112,7 @@ def sweep_fp8(rows):
 
 def sweep_qkv(rows):
     tiles = [1, 2, 3, 4, 5, 6, 7, 8]
-    print("B x L, heads / kv x dim, K       M     own" + "".join(f"{t:>8}" for t in tiles) + "    (32 t rows a tile; 1: 128 x 128)")
+    print("B x L, heads / kv x dim, K       M  choice     own" + "".join(f"{t:>8}" for t in tiles) + "    (32 t rows a tile; 1: 128 x 128)")
     for B, L0, nh, nkv, hd, K in QKV:
         for L in [L0] if L0 else [r // B for r in rows]:
             M, N, Tp = B * L, (nh + 2 * nkv) * hd, (L + 127) // 128 * 128
@@ -123,7 +123,7 @@ def sweep_qkv(rows):
             def run():
                 return all([ops.gemm_qkv(a, x, cos, cos, q, k, v, B, L, nh, nkv, hd, 0, Tp, True, Tp, 1, q_scale=0.5) for x in w])
             times = in_turn("gemm_qkv_flat", [-1] + tiles, run, len(w) * 2.0 * M * N * K, 1.1e15)
-            row(f"{B} x {L}, {nh} / {nkv} x {hd}, {K}", M, f"{times[0] / 12:.1f}" if times[0] else "-", times[1:], len(w))
+            row(f"{B} x {L}, {nh} / {nkv} x {hd}, {K}", M, _lib.lib().p3v_gemm_qkv_tile(M, nh * hd, nkv * hd, K), times, len(w))
 
 
 if __name__ == "__main__":
