@@ -117,11 +117,13 @@ def sweep_qkv(rows):
         for L in [L0] if L0 else [r // B for r in rows]:
             M, N, Tp = B * L, (nh + 2 * nkv) * hd, (L + 127) // 128 * 128
             w = [(torch.randn((N, K), device="cuda") * K ** -0.5).bfloat16() for _ in range(12)]
-            a, cos = torch.randn((M, K), device="cuda").bfloat16(), torch.rand((B, Tp, hd // 2), device="cuda")
+            # (image crops, L0: a bias and no rotation)
+            a, cos = torch.randn((M, K), device="cuda").bfloat16(), None if L0 else torch.rand((B, Tp, hd // 2), device="cuda")
+            bias = torch.randn((N,), device="cuda").bfloat16() if L0 else None
             q, k, v = (torch.zeros(s, device="cuda", dtype=torch.bfloat16) for s in ((B, nh, L, hd), (B, nkv, Tp, hd), (B, nkv, hd, Tp)))
 
             def run():
-                return all([ops.gemm_qkv(a, x, cos, cos, q, k, v, B, L, nh, nkv, hd, 0, Tp, True, Tp, 1, q_scale=0.5) for x in w])
+                return all([ops.gemm_qkv(a, x, cos, cos, q, k, v, B, L, nh, nkv, hd, 0, Tp, True, Tp, 1, q_scale=0.5, bias=bias) for x in w])
             times = in_turn("gemm_qkv_flat", [-1] + tiles, run, len(w) * 2.0 * M * N * K, 1.1e15)
             row(f"{B} x {L}, {nh} / {nkv} x {hd}, {K}", M, _lib.lib().p3v_gemm_qkv_tile(M, nh * hd, nkv * hd, K), times, len(w))
 
