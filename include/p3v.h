@@ -530,6 +530,11 @@ int p3v_attn_mix(const p3v_mix_args_t* args /* host */, void* stream);
 int p3v_attn_mix_decode(const p3v_mix_args_t* args /* host */, void* stream);
 int p3v_attn_mix_plan(int B, int L, int H, int G, int dim, int vdim, int n_keys, int f32);
 int64_t p3v_attn_mix_ws_bytes(int B, int L, int H, int vdim, int n_split);
+/* p3v_attn_mix of a prompt (the position on the host) with a workspace: the keys as matrix fragments and, unless the prompt is long, the mixed
+ * and exponentiated scores between two launches.  ws: 16-byte aligned, ws_bytes >= p3v_attn_mix_prompt_ws_bytes; 0 from it, or d_past, or wider
+ * caches than dim and vdim rounded up to 32: P3V_ERR_UNSUPPORTED. */
+int p3v_attn_mix_prompt(const p3v_mix_args_t* args /* host */, void* ws, int64_t ws_bytes, void* stream);
+int64_t p3v_attn_mix_prompt_ws_bytes(int B, int L, int H, int G, int dim, int vdim, int n_keys, int f32);
 
 /* RMS norm of fp32 rows: out = x / sqrt(mean x^2 + eps) * w * gain, one rounding (out bf16, or fp32 with out_f32) */
 int p3v_rms_rows(const float* x, const uint16_t* w, void* out, int out_f32, int rows, int H, float eps, float gain, void* stream);

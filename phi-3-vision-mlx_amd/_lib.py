@@ -193,6 +193,8 @@ SIGNATURES = {
     "p3v_attn_mix_decode": (i32, [C.POINTER(MixArgs), vp]),
     "p3v_attn_mix_plan": (i32, [i32, i32, i32, i32, i32, i32, i32, i32]),
     "p3v_attn_mix_ws_bytes": (i64, [i32, i32, i32, i32, i32]),
+    "p3v_attn_mix_prompt": (i32, [C.POINTER(MixArgs), vp, i64, vp]),
+    "p3v_attn_mix_prompt_ws_bytes": (i64, [i32, i32, i32, i32, i32, i32, i32, i32]),
     "p3v_rms_rows": (i32, [vp, vp, vp, i32, i32, i32, f32, f32, vp]),
     "p3v_gemv_rms": (i32, [C.POINTER(GemvArgs), vp, f32, vp]),
     "p3v_gla": (i32, [C.POINTER(GlaArgs), vp]),

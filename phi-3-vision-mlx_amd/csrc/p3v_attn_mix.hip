@@ -10,11 +10,7 @@
 // Scores, their mixing and the softmax are fp32.  The mixing runs on the bf16 matrix cores WITHOUT losing fp32: talk is bf16 data, and
 // a score is split into three bf16 terms whose sum is the fp32 value, so that every product is exact and only the fp32 accumulation
 // rounds -- an eighth of the cost of the fp32 matrix instruction.
-#include "p3v_layered.h"
-
-#define MIX_NEG (-1e30f)             // "no key yet": finite, so that differences of two of them stay 0
-#define MIX_MAX_H 32
-#define LOG2E 1.4426950408889634f
+#include "p3v_attn_mix.h"
 
 typedef __attribute__((ext_vector_type(2))) float f32x2_t;
 
@@ -60,42 +56,6 @@ template <int HW> struct MixCfg {
   static constexpr int S_BYTES = 16 * QS * 4, P_BYTES = HP * PH * 2, A_BYTES = HM * 16 * 16 * 4;
   static constexpr int LDS = S_BYTES + P_BYTES + 2 * A_BYTES + HM * 1024 + (HW == 4 ? 8 * 4096 : 0);
 };
-
-// A run = the key tiles [split * per, ..) of one query tile.  first query tile that sees 32-key tile T - 1, and how many do
-__host__ __device__ static inline int mix_q_first(int past, int T) { const int d = 32 * (T - 1) - 15 - past; return d <= 0 ? 0 : (d + 15) >> 4; }
-__host__ __device__ static inline int mix_q_count(int past, int L, int T) {
-  return T > ((past + L - 1) >> 5) + 1 ? 0 : ((L + 15) >> 4) - mix_q_first(past, T);
-}
-// Run number `wid`.  With more runs than CUs in the order of their lengths: the full ones split by split, then the partial ones by
-// decreasing length -- long runs that start late are what the last CUs wait for (2048 rows: 18 tiles' time instead of 23 - 27).  Else split by
-// split, which takes 2 us less to find out.
-struct MixRun { int qt, split, b; };
-__device__ __forceinline__ MixRun mix_run(int wid, const AttnMixP& p) {
-  const int per = p.tiles_per_split, n_qt = (p.L + 15) >> 4;
-  for (int s = 0; s < p.n_split; ++s) {
-    const int n = p.B * mix_q_count(p.past, p.L, p.by_length ? (s + 1) * per : s * per + 1);
-    if (wid < n) return {n_qt - 1 - wid / p.B, s, wid % p.B};
-    wid -= n;
-  }
-  const int lane = threadIdx.x & 63;
-  for (int o0 = 0; o0 < (per - 1) * p.n_split; o0 += 64) {               // (length, split) pairs, a lane each
-    const int o = o0 + lane, len = per - 1 - o / p.n_split, T = o % p.n_split * per + len;
-    const int n = len > 0 ? p.B * (mix_q_count(p.past, p.L, T) - mix_q_count(p.past, p.L, T + 1)) : 0;
-    int sum = n;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int v = __shfl_up(sum, d);
-      sum += lane >= d ? v : 0;
-    }
-    const unsigned long long hit = __ballot(wid < sum);
-    if (hit) {
-      const int l = __builtin_ctzll(hit), r = wid - __shfl(sum - n, l), q = __shfl(mix_q_first(p.past, T), l), sp = __shfl(o % p.n_split, l);
-      return {__builtin_amdgcn_readfirstlane(q + r / p.B), __builtin_amdgcn_readfirstlane(sp), __builtin_amdgcn_readfirstlane(r % p.B)};
-    }
-    wid -= __shfl(sum, 63);
-  }
-  return {-1, 0, 0};
-}
 
 template <int HW, int DC, int VC, bool SHARED>
 __global__ void __launch_bounds__(512, 1) k_attn_mix_prefill(AttnMixP p) {
@@ -164,25 +124,27 @@ __global__ void __launch_bounds__(512, 1) k_attn_mix_prefill(AttnMixP p) {
     for (int i = tid; i < C::S_BYTES / 4; i += 512) S[i] = 0.f;
   lds_barrier();
 
-  const bf16_t* kb = (const bf16_t*)p.k + (size_t)b * p.G * p.Tp * p.dimp;
+  const bf16_t* kb = (p.kx ? p.kx : (const bf16_t*)p.k) + (size_t)b * p.G * (p.kx ? p.kx_rows : p.Tp) * p.dimp;
   const bf16_t* vb = (const bf16_t*)p.v + (size_t)b * p.G * p.Tp * p.vdimp;
-  const uint32_t k_lane = (uint32_t)(lc * p.dimp + lg * 8), v_lane = (uint32_t)(((lg >> 1) * p.vdimp + lc) * 16 + (lg & 1) * 8);
+  // (rows of the cache, or their fragments: k_mix_keys)
+  const uint32_t k_lane = p.kx ? lane * 16 : (uint32_t)(lc * p.dimp + lg * 8) * 2, kc = p.kx ? 1024 : 64, k_rows = p.kx ? p.kx_rows : p.Tp;
+  const uint32_t v_lane = (uint32_t)(((lg >> 1) * p.vdimp + lc) * 16 + (lg & 1) * 8) * 2;
   const bool active = wave * HW < p.H;
   bf16x8_t kf[NB][2][DC], vf[NB][NV];
   auto load_k = [&](int t, int i) {
     const int g = min(wave * HW + i, p.H - 1) / per, bf = SHARED ? 0 : i & 1;
-    const bf16_t *k0 = kb + ((size_t)g * p.Tp + t * 32) * p.dimp, *k1 = k0 + (size_t)16 * p.dimp;
+    gptr_t k0 = (gptr_t)(kb + ((size_t)g * k_rows + t * 32) * p.dimp), k1 = k0 + (size_t)32 * p.dimp;
     asm volatile("" : "+s"(k0), "+s"(k1));                               // (scalar bases + one 32-bit lane offset: no 64-bit lane addresses)
 #pragma unroll
-    for (int c = 0; c < DC; ++c) kf[bf][0][c] = *(const bf16x8_t*)(k0 + k_lane + c * 32), kf[bf][1][c] = *(const bf16x8_t*)(k1 + k_lane + c * 32);
+    for (int c = 0; c < DC; ++c) kf[bf][0][c] = gload<bf16x8_t>(k0 + c * kc, k_lane), kf[bf][1][c] = gload<bf16x8_t>(k1 + c * kc, k_lane);
   };
   auto load_v = [&](int t, int i) {
     const int g = min(wave * HW + i, p.H - 1) / per, bf = SHARED ? 0 : i & 1;
-    const bf16_t* vr = vb + ((size_t)g * (p.Tp >> 4) + t * 2) * p.vdimp * 16;
+    gptr_t vr = (gptr_t)(vb + ((size_t)g * (p.Tp >> 4) + t * 2) * p.vdimp * 16);
     asm volatile("" : "+s"(vr));
 #pragma unroll
     for (int d = 0; d < NV; ++d)
-      vf[bf][d] = *(const bf16x8_t*)(vr + v_lane + d * 256);
+      vf[bf][d] = gload<bf16x8_t>(vr + d * 512, v_lane);
   };
   if (active && t0 < t1) load_k(t0, 0);
 
@@ -643,32 +605,6 @@ static bool mix_fast(int H, int G, int dim, int vdim, int f32) {
   return !f32 && H <= MIX_MAX_H && dim <= 128 && vdim <= 128;
 }
 
-// When the last run of a prompt's, cut into runs of up to `per` key tiles, is done, in the time of a key tile.  The runs start by decreasing
-// length; run i goes to shader engine i % MIX_ENGINES (XCD by XCD, then engine by engine in them) and waits for its first free CU.  The first
-// engine has the longest of every MIX_ENGINES runs, and a run too many before the others: its end is the launch's.  MIX_RUN_FIXED: what a run
-// costs besides its tiles.  (With one pool of CUs instead of engines the cut chosen by it was up to 1.2x behind the best, with these within 3 %.)
-#define MIX_CUS 256
-#define MIX_ENGINES 32
-#define MIX_RUN_FIXED 2
-#define MIX_PLAN_TILES 4096            // longest key range that is looked at in this detail
-static int mix_runs_end(int B, int L, int past, int per, int cus) {
-  int by_length[MIX_PLAN_TILES + 1], free_at[128] = {}, end = 0;
-  for (int i = 0; i <= per; ++i) by_length[i] = 0;
-  for (int q = 0; q < L; q += 16) {
-    const int t = ((past + min(q + 15, L - 1)) >> 5) + 1;
-    by_length[per] += t / per * B;
-    if (t % per) by_length[t % per] += B;
-  }
-  const int n = min(max(cus / MIX_ENGINES, 1), 128);
-  for (int len = per, i = 0, up_to = 0; len > 0; --len)
-    for (up_to += by_length[len]; i < up_to; i += MIX_ENGINES) {
-      int c = 0;
-      for (int k = 1; k < n; ++k) c = free_at[k] < free_at[c] ? k : c;
-      free_at[c] += len + MIX_RUN_FIXED;
-      end = max(end, free_at[c]);
-    }
-  return end;
-}
 // Prompts: key tiles of a run, of the cuts into equal parts and some lengths from a CU's share of all tiles on, not below 4: the one whose last
 // CU is done first, a tile's time for the merge and a fifth for each partial a row of it reads.  A launch of a few more runs than CUs is what costs:
 // 2 x 700 rows in runs of 4 tiles are 288 for 256 CUs, in runs of 5 240 (32 heads x 96, 8 kv heads: 74.4 : 60.6 us).  Prompts of two and more
@@ -751,22 +687,15 @@ static int prefill_dc(const AttnMixP& p, hipStream_t s) {
   }
 }
 
-extern "C" int p3v_attn_mix(const p3v_mix_args_t* a, void* stream) {
-  const int rc = p3v_mix_check(a);
-  if (rc != P3V_OK) return rc;
-  if (!a->q || !a->talk || !a->sink || !a->gate || !a->out || a->n_split < 0) return P3V_ERR_ARG;
-  hipStream_t s = (hipStream_t)stream;
-  if (a->n_split == 0 || a->vdimp > 128 || a->dimp > 128 || !mix_fast(a->H, a->G, a->dim, a->vdim, a->f32)) return p3v_attn_mix_any(a, s);
-  if (a->n_split > 1 && (!a->ws || a->n_split > MIX_MAX_ROW_SPLIT)) return P3V_ERR_ARG;
-  AttnMixP p = attn_mix_params(a);
+int mix_prefill(AttnMixP p, int n_keys, hipStream_t s) {
   // (the position may be a device value: the splits then cover the capacity)
-  const int tiles = p3v_cdiv(a->d_past ? a->Tp : a->past + a->L, 32);
-  p.tiles_per_split = p3v_cdiv(tiles, a->n_split);
-  if (!a->d_past && a->n_split > 1)
-    if (const int per = mix_run_tiles(a->B, a->L, a->past); p3v_cdiv(tiles, per) == a->n_split) p.tiles_per_split = per;   // as planned
+  const int tiles = p3v_cdiv(n_keys, 32);
+  p.tiles_per_split = p3v_cdiv(tiles, p.n_split);
+  if (!p.d_past && p.n_split > 1)
+    if (const int per = mix_run_tiles(p.B, p.L, p.past); p3v_cdiv(tiles, per) == p.n_split) p.tiles_per_split = per;   // as planned
   // (query tile, split) pairs for more than the CUs, some of them without keys to see: the runs alone (with empty pairs between them they
   // crowd on some CUs: 900 rows in 8 parts 75 : 98 us)
-  if (!a->d_past && a->n_split > 1 && (long)p3v_cdiv(a->L, 16) * a->n_split * a->B > MIX_CUS) {
+  if (!p.d_past && p.n_split > 1 && (long)p3v_cdiv(p.L, 16) * p.n_split * p.B > MIX_CUS) {
     for (int sp = 0; sp < p.n_split; ++sp) p.runs += p.B * mix_q_count(p.past, p.L, sp * p.tiles_per_split + 1);
     p.by_length = p.runs > MIX_CUS;
   }
@@ -775,6 +704,16 @@ extern "C" int p3v_attn_mix(const p3v_mix_args_t* a, void* stream) {
   if (p.H <= 8) return prefill_dc<1, true>(p, s);
   if (p.H <= 16) return per % 2 ? prefill_dc<2, false>(p, s) : prefill_dc<2, true>(p, s);
   return per % 4 ? prefill_dc<4, false>(p, s) : prefill_dc<4, true>(p, s);
+}
+
+extern "C" int p3v_attn_mix(const p3v_mix_args_t* a, void* stream) {
+  const int rc = p3v_mix_check(a);
+  if (rc != P3V_OK) return rc;
+  if (!a->q || !a->talk || !a->sink || !a->gate || !a->out || a->n_split < 0) return P3V_ERR_ARG;
+  hipStream_t s = (hipStream_t)stream;
+  if (a->n_split == 0 || a->vdimp > 128 || a->dimp > 128 || !mix_fast(a->H, a->G, a->dim, a->vdim, a->f32)) return p3v_attn_mix_any(a, s);
+  if (a->n_split > 1 && (!a->ws || a->n_split > MIX_MAX_ROW_SPLIT)) return P3V_ERR_ARG;
+  return mix_prefill(attn_mix_params(a), a->d_past ? a->Tp : a->past + a->L, s);
 }
 
 template <int GW, int DC, int NP>

@@ -59,6 +59,12 @@ __device__ __forceinline__ void load4(const float* p, float (&v)[4]) {
 __device__ __forceinline__ void store4(bf16_t* p, const float (&v)[4]) { *(u32x2_t*)p = (u32x2_t){pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])}; }
 __device__ __forceinline__ void store4(float* p, const float (&v)[4]) { *(float4*)p = make_float4(v[0], v[1], v[2], v[3]); }
 
+// Device memory by a pointer that says so: behind an empty asm, which keeps a base in scalar registers, the compiler no longer sees where a
+// generic one points, and a flat load waits for LDS as well.  A load takes a uniform base and a lane's 32-bit offset in BYTES (as elements it
+// could exceed 32 bits when scaled, and the address would be formed in two vector registers).
+typedef const __attribute__((address_space(1))) char* gptr_t;
+template <typename T> __device__ __forceinline__ T gload(gptr_t base, uint32_t bytes) { return *(const __attribute__((address_space(1))) T*)(base + bytes); }
+
 // ---- kernel parameters
 struct DytP {
   const float* x; const bf16_t* w; const bf16_t* b; const bf16_t* mu; float* hist; const int32_t* pad_len; const int32_t* d_past;
@@ -76,12 +82,14 @@ struct AttnMixP {
   const int32_t* pad_len; const int32_t* d_past;
   float scale; int B, L, H, G, dim, vdim, dimp, vdimp, ld, past, Tp, n_split, tiles_per_split;
   int runs, by_length;                                                   // prompts: 0, or a workgroup for each of so many runs (mix_run), longest first
+  const bf16_t* kx; int kx_rows;                                         // prompts: the keys as fragments (k_mix_keys), kx_rows a head; or null
 };
 static inline AttnMixP attn_mix_params(const p3v_mix_args_t* a) {
   return {a->q, a->k, a->v, a->talk, a->sink, a->gate, a->out, a->ws, a->pad_len, a->d_past, a->scale,
-          a->B, a->L, a->H, a->G, a->dim, a->vdim, a->dimp, a->vdimp, a->ld, a->past, a->Tp, a->n_split, 0, 0, 0};
+          a->B, a->L, a->H, a->G, a->dim, a->vdim, a->dimp, a->vdimp, a->ld, a->past, a->Tp, a->n_split, 0, 0, 0, nullptr, 0};
 }
 
 int p3v_dyt_check(const p3v_dyt_args_t* a);
 int p3v_mix_check(const p3v_mix_args_t* a);
 int p3v_attn_mix_any(const p3v_mix_args_t* a, hipStream_t s);
+int mix_prefill(AttnMixP p, int n_keys, hipStream_t s);                  // the one-launch kernel of prompts (p3v_attn_mix.hip)

@@ -55,12 +55,14 @@ class MixedHeads:
 
     def plan(self, B, L, n_keys):
         m = self.m
+        if ops.mix_prompt_ws_bytes(B, L, m.heads, m.kv_heads, m.dim, m.vdim, n_keys, self.T):
+            return -1
         return ops.mix_plan(B, L, m.heads, m.kv_heads, m.dim, m.vdim, n_keys, self.T)
 
     def buffers(self, B, L, n_keys):
-        m = self.m
-        return {"q": (B * L * m.heads * round_up(m.dim, 32), self.T),
-                "attn_ws": (ops.mix_ws_bytes(B, L, m.heads, m.vdim, self.plan(B, L, n_keys)) // 4, F32)}
+        m, plan = self.m, self.plan(B, L, n_keys)
+        ws = ops.mix_prompt_ws_bytes(B, L, m.heads, m.kv_heads, m.dim, m.vdim, n_keys, self.T) if plan < 0 else ops.mix_ws_bytes(B, L, m.heads, m.vdim, plan)
+        return {"q": (B * L * m.heads * round_up(m.dim, 32), self.T), "attn_ws": (ws // 4, F32)}
 
     def run(self, y, out, rows, bufs, call, plan):
         m = self.m

@@ -900,11 +900,17 @@ def mix_ws_bytes(B, Lq, H, vdim, n_split):
     return int(L.lib().p3v_attn_mix_ws_bytes(B, Lq, H, vdim, n_split)) if n_split > 0 else 0
 
 
+def mix_prompt_ws_bytes(B, Lq, H, G, dim, vdim, n_keys, dtype):
+    """Workspace of p3v_attn_mix_prompt; 0: not for this call (n_keys = past + L)."""
+    return int(L.lib().p3v_attn_mix_prompt_ws_bytes(B, Lq, H, G, dim, vdim, int(n_keys), int(dtype == F32)))
+
+
 def attention_mixed(qkv, q, k, v, out, norms, talk, sink, B, Lq, H, G, dim, vdim, eps, scale, past, v_first=None, vmix=0.0, pad_len=None,
                     d_past=None, ws=None, n_split=0):
     """Head split + whole-projection q / k norms + value mixing + cache append + attention with mixed heads, sink and output gate
     (include/p3v.h: p3v_mix_args_t).  qkv [B*L, >= H dim + G dim + G vdim + H] (bf16 or fp32), caches k / v as LayeredCacheState keeps
-    them, out [B*L, H vdim]; v_first [B*L, >= G vdim] view: the first value-mixing layer's own values of these tokens."""
+    them, out [B*L, H vdim]; v_first [B*L, >= G vdim] view: the first value-mixing layer's own values of these tokens.  n_split from
+    mix_plan; -1: p3v_attn_mix_prompt, ws of mix_prompt_ws_bytes."""
     f32 = qkv.dtype == F32
     for t, n in ((qkv, "qkv"), (q, "q"), (k, "k"), (v, "v"), (out, "out")):
         _chk(t, F32 if f32 else BF16, n)
@@ -922,6 +928,10 @@ def attention_mixed(qkv, q, k, v, out, norms, talk, sink, B, Lq, H, G, dim, vdim
         raise ValueError("attention_mixed: workspace smaller than mix_ws_bytes")
     if d_past is None and past + Lq > Tp:
         raise ValueError(f"attention_mixed: columns {past} + {Lq} > {Tp}")
+    prompt = n_split < 0
+    if prompt and d_past is not None:
+        raise ValueError("attention_mixed: a prompt's position is a host value")
+    n_split = max(n_split, 0)
     gate = qkv[:, n_qkv:]
     args = L.MixArgs(_p(qkv), _p(norms[0]), _p(norms[1]), _p(v_first), _p(q), _p(k), _p(v), _p(talk), _p(sink), _p(gate), _p(out), _p(ws),
                      _p(pad_len), _p(d_past), float(eps), float(vmix), float(scale), B, Lq, H, G, dim, vdim, dimp, vdimp, ld,
@@ -933,7 +943,10 @@ def attention_mixed(qkv, q, k, v, out, norms, talk, sink, B, Lq, H, G, dim, vdim
             return out
         args.n_split = 1
     L.check(L.lib().p3v_qkv_heads(C.byref(args), _stream()), "qkv_heads")
-    L.check(L.lib().p3v_attn_mix(C.byref(args), _stream()), "attn_mix")
+    if prompt:
+        L.check(L.lib().p3v_attn_mix_prompt(C.byref(args), _p(ws), 0 if ws is None else ws.numel() * ws.element_size(), _stream()), "attn_mix_prompt")
+    else:
+        L.check(L.lib().p3v_attn_mix(C.byref(args), _stream()), "attn_mix")
     return out
 
 

@@ -352,6 +352,53 @@ def test_mixed_attention_key_splits(H, G, dim, vdim, n_split):
         close(got[:, 0], np.stack(want), BF16)
 
 
+@pytest.mark.parametrize("H,G,dim,vdim,B,L,past,pads,scale", [
+    (32, 32, 96, 96, 1, 16, 0, None, None), (32, 32, 96, 96, 2, 33, 0, [0, 20], None), (17, 17, 40, 24, 1, 127, 5, [3], None), (20, 4, 64, 128, 2, 130, 37, [0, 50], None),
+    (32, 16, 128, 7, 1, 260, 64, [100], -0.1), (24, 24, 32, 36, 3, 64, 0, [0, 40, 63], 4.0), (32, 32, 96, 96, 1, 200, 1000, None, 3.0), (32, 32, 64, 64, 1, 1100, 0, [17], None)])
+def test_mixed_attention_of_a_prompt_with_workspace(H, G, dim, vdim, B, L, past, pads, scale):
+    """Two launches: tiles with padding, a position inside a tile, heads that fill no 16, groups, uneven value widths, a negative scale, and
+    scores so far apart (scale 3 and 4) that tiles of one row have different references.  Against float64, and against the one launch."""
+    from phi_3_vision_mlx_amd import ops
+    m = Mix(H, G, dim, vdim, B, (past + L + 31) // 32 * 32, BF16, seed=L, scale=scale)
+    raw = dev(m.r.normal(0, 1, (B, past + L, m.ld)), BF16)
+    if past:
+        m.run(raw[:, :past].contiguous().view(B * past, -1), past, 0, pads, plan=1)
+    x = raw[:, past:].contiguous().view(B * L, -1)
+    one = m.run(x, L, past, pads, plan=1)
+    n = ops.mix_prompt_ws_bytes(B, L, H, G, dim, vdim, past + L, BF16)
+    assert n > 0
+    ws = torch.full((n // 4,), float("nan"), dtype=F32, device=DEV)
+    q, out = torch.zeros(B * H * L * m.k.shape[3], dtype=BF16, device=DEV), torch.full((B * L, H * vdim), float("nan"), dtype=BF16, device=DEV)
+    kw = dict(pad_len=None if pads is None else torch.tensor(pads, dtype=I32, device=DEV), n_split=-1)
+    args = (x, q, m.k, m.v, out, (dev(m.qn), dev(m.kn)), dev(m.talk), dev(m.sink), B, L, H, G, dim, vdim, m.eps, m.scale, past)
+    with pytest.raises(RuntimeError):
+        ops.attention_mixed(*args, ws=ws[:-4], **kw)
+    with pytest.raises(ValueError):
+        ops.attention_mixed(*args, ws=ws, d_past=torch.tensor([past], dtype=I32, device=DEV), **kw)
+    ops.attention_mixed(*args, ws=ws, **kw)
+    got = host(out).reshape(B, L, H, vdim)
+    for b in range(B):
+        lo = max(0, (pads[b] if pads else 0) - past)
+        close(got[b, lo:], one[b, lo:], BF16)
+        if scale is None or abs(scale) < 1:
+            close(got[b, lo:], m.oracle(host(raw)[b], pads[b] if pads else 0)[past + lo:], BF16)
+
+
+def test_mixed_attention_of_a_long_prompt_on_key_fragments():
+    """A prompt whose scores do not go through memory: the planned launch, from fragments of the keys -- the same bits as from rows."""
+    from phi_3_vision_mlx_amd import ops
+    H, L = 32, 2600
+    m = Mix(H, H, 96, 96, 1, 2624, BF16, seed=1)
+    x = dev(m.r.normal(0, 1, (L, m.ld)), BF16)
+    want = m.run(x, L, 0)
+    n = ops.mix_prompt_ws_bytes(1, L, H, H, 96, 96, L, BF16)
+    assert n < 400 << 20
+    ws = torch.full((n // 4,), float("nan"), dtype=F32, device=DEV)
+    q, out = torch.zeros(H * L * 96, dtype=BF16, device=DEV), torch.empty((L, H * 96), dtype=BF16, device=DEV)
+    ops.attention_mixed(x, q, m.k, m.v, out, (dev(m.qn), dev(m.kn)), dev(m.talk), dev(m.sink), 1, L, H, H, 96, 96, m.eps, m.scale, 0, ws=ws, n_split=-1)
+    assert np.array_equal(host(out).reshape(1, L, H, 96), want)
+
+
 @pytest.mark.parametrize("B,L,past,pads", [(1, 16, 300, None), (1, 700, 0, None), (2, 333, 31, [0, 40]), (3, 1025, 0, [0, 64, 1000]), (1, 1500, 545, [7]),
                                               (1, 2048, 0, None), (2, 1200, 3, [5, 700])])
 def test_mixed_attention_runs_by_length(B, L, past, pads):
