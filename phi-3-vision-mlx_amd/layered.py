@@ -72,6 +72,7 @@ class _Layer:
 
 class LayeredModel(DecoderModel):
     x_dtype = F32
+    TAIL_MIN_L = 1024                                            # prompts whose final attention computes the last rows alone (shorter ones may be captured)
 
     def __init__(self, cfg, weights, device="cuda:0"):
         self._init_decoder(cfg, device)
@@ -157,12 +158,14 @@ class LayeredModel(DecoderModel):
             y = bufs["y_first" if i == self.first_v else "y"][:M * mx.w_in.shape[0]].view(M, -1)
             shift = {} if ly.shift is None else dict(shift=ly.shift, hist=st.shift[i], past=past, d_past=d_past, pad_len=st.pad_len)
             ly.norm1.project(x, mx.w_in, h, out=y, B=B, Lq=L, **shift)
-            mx.run(y, o, st.mix[i], bufs, call, bufs["plans"][i])
+            tail = last_only and L > 1 and i == len(self.stack) - 1
+            call.tail = tail and L >= self.TAIL_MIN_L
+            last = mx.run(y, o, st.mix[i], bufs, call, bufs["plans"][i])
             if i == self.first_v:
                 call.v_first = mx.values(y)
             rows = M
-            if last_only and L > 1 and i == len(self.stack) - 1:
-                o, x, rows = o.view(B, L, -1)[:, -1].contiguous(), x.view(B, L, -1)[:, -1].contiguous(), B
+            if tail:
+                o, x, rows = o.view(B, L, -1)[:, -1].contiguous() if last is None else last, x.view(B, L, -1)[:, -1].contiguous(), B
             ops.project(o, mx.o, EPI_SCALE_RESID_F32, resid=x, col_scale=ly.ls1, out=x)
             if ly.mlp:
                 ff = ly.spec.mlp.ff

@@ -9,6 +9,8 @@ projection of the layer's input:
     plan(B, L, n_keys)       what a call's launches are planned for (a one-token call: the cache capacity, so that eager and captured
                              steps run alike)
     run(y, out, rows, bufs, call, plan)
+                             call.tail: only the outputs of each sequence's last token are read; a mixer that saves work by it returns these
+                             rows, else None
 """
 from dataclasses import dataclass
 from typing import Any
@@ -31,6 +33,7 @@ class Call:
     d_past: Any = None
     pad_len: Any = None
     v_first: Any = None
+    tail: bool = False
 
 
 def packed(mats):
@@ -61,14 +64,19 @@ class MixedHeads:
 
     def buffers(self, B, L, n_keys):
         m, plan = self.m, self.plan(B, L, n_keys)
-        ws = ops.mix_prompt_ws_bytes(B, L, m.heads, m.kv_heads, m.dim, m.vdim, n_keys, self.T) if plan < 0 else ops.mix_ws_bytes(B, L, m.heads, m.vdim, plan)
+        if plan < 0:                                             # (of the whole prompt, and of its last tile: Call.tail)
+            ws = max(ops.mix_prompt_ws_bytes(B, n, m.heads, m.kv_heads, m.dim, m.vdim, n_keys, self.T) for n in (L, ops.MIX_TAIL))
+        else:
+            ws = ops.mix_ws_bytes(B, L, m.heads, m.vdim, plan)
         return {"q": (B * L * m.heads * round_up(m.dim, 32), self.T), "attn_ws": (ws // 4, F32)}
 
     def run(self, y, out, rows, bufs, call, plan):
         m = self.m
-        ops.attention_mixed(y, bufs["q"], rows.k, rows.v, out, self.norms, self.talk, self.sink, call.B, call.L, m.heads, m.kv_heads, m.dim, m.vdim,
-                            self.eps, m.scale, call.past, v_first=call.v_first if m.v_mix else None, vmix=self.vmix, pad_len=call.pad_len,
-                            d_past=call.d_past, ws=bufs["attn_ws"], n_split=plan)
+        tail = call.tail and plan < 0
+        got = ops.attention_mixed(y, bufs["q"], rows.k, rows.v, out, self.norms, self.talk, self.sink, call.B, call.L, m.heads, m.kv_heads, m.dim,
+                                  m.vdim, self.eps, m.scale, call.past, v_first=call.v_first if m.v_mix else None, vmix=self.vmix,
+                                  pad_len=call.pad_len, d_past=call.d_past, ws=bufs["attn_ws"], n_split=plan, tail=tail)
+        return got if tail else None
 
     def values(self, y):
         return y[:, self.v_col:self.v_col + self.m.kv_heads * self.m.vdim]

@@ -487,8 +487,8 @@ class Phi3VModel(DecoderModel):
         """Phi3DecoderLayer stack (phi.py:473-485).  `d_past` (device int32) makes every
         position-dependent kernel read the cache length from HBM -> graph-replayable.
         last_only: the caller reads the LAST position only (prefill of generate / choose, Q8): the final layer still builds
-        K / V for every position, but its o_proj and MLP run on the B last rows alone (0.4 ms of a 30 ms prefill);
-        returns [B, H] then."""
+        K / V for every position, but its o_proj and MLP run on the B last rows alone (0.4 ms of a 30 ms prefill), and so does its
+        attention behind TAIL_MIN_L tokens; returns [B, H] then."""
         cfg, w = self.cfg, self.w
         nh, nkv, hd, eps = cfg.num_attention_heads, cfg.num_key_value_heads, self.hd, cfg.rms_norm_eps
         M = B * L
@@ -570,8 +570,11 @@ class Phi3VModel(DecoderModel):
                     if not fused_qkv:
                         ops.rope_kv_append(qkv, st.cos, st.sin, q, st.k_tmp, st.v_tmp, B, L, nh, nkv, hd, past, st.Tp, True, st.T, 1,
                                            q_scale=scale * ops.Q_PRESCALE)
-                    ops.attention(q, o, B, L, nh, nkv, hd, scale, True, past=past, k_past=st.k_tmp, v_past=st.v_tmp,
-                                  past_t=st.Tp, pad_len=st.pad_len, new_is_cache=True, q_prescaled=True)
+                    if last_only and i == cfg.num_hidden_layers - 1 and L >= self.TAIL_MIN_L:
+                        o = self._attend_last(q, st.k_tmp, st.v_tmp, B, L, past, st, scale)
+                    else:
+                        ops.attention(q, o, B, L, nh, nkv, hd, scale, True, past=past, k_past=st.k_tmp, v_past=st.v_tmp,
+                                      past_t=st.Tp, pad_len=st.pad_len, new_is_cache=True, q_prescaled=True)
                     ops.kv_quantize(st.k_tmp, st.v_tmp, st.k8[i], st.v8[i], st.ks[i], st.vs[i], past, L)
             elif n_beam > 1:
                 ops.rope_kv_append(qkv, st.cos, st.sin, q, k_new, v_new, B, L, nh, nkv, hd, past, Lp, False, st.T, n_beam)
@@ -604,12 +607,15 @@ class Phi3VModel(DecoderModel):
                 if not fused_qkv:
                     ops.rope_kv_append(qkv, st.cos, st.sin, q, st.k[i], st.v[i], B, L, nh, nkv, hd, past, st.Tp, True, st.T, 1,
                                        q_scale=scale * ops.Q_PRESCALE)
-                ops.attention(q, o, B, L, nh, nkv, hd, scale, True, past=past, k_past=st.k[i], v_past=st.v[i],
-                              past_t=st.Tp, pad_len=st.pad_len, new_is_cache=True, q_prescaled=True)
+                if last_only and i == cfg.num_hidden_layers - 1 and L >= self.TAIL_MIN_L:
+                    o = self._attend_last(q, st.k[i], st.v[i], B, L, past, st, scale)
+                else:
+                    ops.attention(q, o, B, L, nh, nkv, hd, scale, True, past=past, k_past=st.k[i], v_past=st.v[i],
+                                  past_t=st.Tp, pad_len=st.pad_len, new_is_cache=True, q_prescaled=True)
             if mlx4_first:                                      # this layer attended on the exact keys (phi.py:533); from now on: the codes
                 self._mlx4_quantize(st, i, L, qkv, nh)          # (keys from their exact fp32 values: recomputed from `qkv`)
             if last_only and i == cfg.num_hidden_layers - 1 and L > 1:
-                o = o.view(B, L, -1)[:, -1].contiguous()
+                o = o if o.shape[0] == B else o.view(B, L, -1)[:, -1].contiguous()
                 x = x.view(B, L, -1)[:, -1].contiguous()
                 a, h = a[:B], h[:B]
             # Short prompts and decode batches (9 .. 256 rows): o_proj and down_proj run as K slices, and the launch that adds the slices also writes the
@@ -638,6 +644,21 @@ class Phi3VModel(DecoderModel):
         if mlx4_first:
             st.mlx4_tokens = L
         return x
+
+    # The final layer's attention of the last rows alone, key ranges side by side.  us, all rows : the last of 32 heads x 96: 1024 tokens 26 : 14 (29
+    # when the host waits for nothing else), 2531 55 : 14, 8192 446 : 34, 32768 5414 : 109.  Shorter prompts gain less than its three launches
+    # cost, and may be captured, where nothing is allocated.
+    TAIL_MIN_L = 1024
+
+    def _attend_last(self, q, k, v, B, L, past, st, scale):
+        """Attention outputs [B, heads * hd] of each sequence's last position, q [B, heads, L, hd] scaled and rotated, k / v holding every column."""
+        nh, nkv, hd = self.cfg.num_attention_heads, self.cfg.num_key_value_heads, self.hd
+        n_split = min(64, (past + L + 127) // 128)
+        ws = torch.empty(ops.attention_ws_bytes(B, 1, nh, hd, n_split) // 4, dtype=F32, device=self.device)
+        o = torch.empty((B, nh * hd), dtype=BF16, device=self.device)
+        q = q.view(-1)[:B * nh * L * hd].view(B, nh, L, hd)[:, :, -1].contiguous()
+        return ops.attention(q, o, B, 1, nh, nkv, hd, scale, True, past=past + L - 1, k_past=k, v_past=v, past_t=st.Tp, pad_len=st.pad_len,
+                             new_is_cache=True, q_prescaled=True, ws=ws, n_split=n_split)
 
     def _mlx4_quantize(self, st, i, L, qkv, nh):
         if st.k4.shape[3] != L:                                 # (first call shorter than the state was sized for)

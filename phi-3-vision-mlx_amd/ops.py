@@ -900,17 +900,21 @@ def mix_ws_bytes(B, Lq, H, vdim, n_split):
     return int(L.lib().p3v_attn_mix_ws_bytes(B, Lq, H, vdim, n_split)) if n_split > 0 else 0
 
 
+MIX_TAIL = 16                                                    # rows p3v_attn_mix_prompt computes when only the last is read
+
+
 def mix_prompt_ws_bytes(B, Lq, H, G, dim, vdim, n_keys, dtype):
     """Workspace of p3v_attn_mix_prompt; 0: not for this call (n_keys = past + L)."""
     return int(L.lib().p3v_attn_mix_prompt_ws_bytes(B, Lq, H, G, dim, vdim, int(n_keys), int(dtype == F32)))
 
 
 def attention_mixed(qkv, q, k, v, out, norms, talk, sink, B, Lq, H, G, dim, vdim, eps, scale, past, v_first=None, vmix=0.0, pad_len=None,
-                    d_past=None, ws=None, n_split=0):
+                    d_past=None, ws=None, n_split=0, tail=False):
     """Head split + whole-projection q / k norms + value mixing + cache append + attention with mixed heads, sink and output gate
     (include/p3v.h: p3v_mix_args_t).  qkv [B*L, >= H dim + G dim + G vdim + H] (bf16 or fp32), caches k / v as LayeredCacheState keeps
     them, out [B*L, H vdim]; v_first [B*L, >= G vdim] view: the first value-mixing layer's own values of these tokens.  n_split from
-    mix_plan; -1: p3v_attn_mix_prompt, ws of mix_prompt_ws_bytes."""
+    mix_plan; -1: p3v_attn_mix_prompt, ws of mix_prompt_ws_bytes; then with `tail` the new keys and values are appended, but outputs are made of
+    each sequence's last token alone and returned, [B, H vdim]."""
     f32 = qkv.dtype == F32
     for t, n in ((qkv, "qkv"), (q, "q"), (k, "k"), (v, "v"), (out, "out")):
         _chk(t, F32 if f32 else BF16, n)
@@ -943,6 +947,14 @@ def attention_mixed(qkv, q, k, v, out, norms, talk, sink, B, Lq, H, G, dim, vdim
             return out
         args.n_split = 1
     L.check(L.lib().p3v_qkv_heads(C.byref(args), _stream()), "qkv_heads")
+    if prompt and tail:                                          # the last tile of 16 queries, as a prompt of its own behind the rest
+        n = MIX_TAIL
+        rows = qkv.view(B, Lq, ld)[:, -n:].contiguous().view(B * n, ld)
+        q16 = q[:B * H * Lq * dimp].view(B, H, Lq, dimp)[:, :, -n:].contiguous()
+        out = torch.empty((B * n, H * vdim), dtype=out.dtype, device=out.device)
+        args.q, args.gate, args.out, args.L, args.past = _p(q16), _p(rows[:, n_qkv:]), _p(out), n, int(past) + Lq - n
+        L.check(L.lib().p3v_attn_mix_prompt(C.byref(args), _p(ws), ws.numel() * ws.element_size(), _stream()), "attn_mix_prompt")
+        return out.view(B, n, -1)[:, -1].contiguous()
     if prompt:
         L.check(L.lib().p3v_attn_mix_prompt(C.byref(args), _p(ws), 0 if ws is None else ws.numel() * ws.element_size(), _stream()), "attn_mix_prompt")
     else:

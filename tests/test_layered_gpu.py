@@ -384,6 +384,26 @@ def test_mixed_attention_of_a_prompt_with_workspace(H, G, dim, vdim, B, L, past,
             close(got[b, lo:], m.oracle(host(raw)[b], pads[b] if pads else 0)[past + lo:], BF16)
 
 
+@pytest.mark.parametrize("B,L,past,pads", [(1, 40, 0, None), (2, 50, 16, [3, 30])])
+def test_mixed_attention_of_a_prompts_last_tokens(B, L, past, pads):
+    """`tail`: the last tokens' rows and the cache of the whole call."""
+    from phi_3_vision_mlx_amd import ops
+    H, res = 32, []
+    for tail in (False, True):
+        m = Mix(H, H, 96, 48, B, 96, BF16, seed=7)
+        raw = dev(m.r.normal(0, 1, (B, past + L, m.ld)), BF16)
+        if past:
+            m.run(raw[:, :past].contiguous().view(B * past, -1), past, 0, pads, plan=1)
+        n = max(ops.mix_prompt_ws_bytes(B, r, H, H, 96, 48, past + L, BF16) for r in (L, ops.MIX_TAIL))
+        ws = torch.full((n // 4,), float("nan"), dtype=F32, device=DEV)
+        q, out = torch.zeros(B * H * L * 96, dtype=BF16, device=DEV), torch.full((B * L, H * 48), float("nan"), dtype=BF16, device=DEV)
+        o = ops.attention_mixed(raw[:, past:].contiguous().view(B * L, -1), q, m.k, m.v, out, (dev(m.qn), dev(m.kn)), dev(m.talk), dev(m.sink), B, L, H, H, 96, 48,
+                                m.eps, m.scale, past, pad_len=None if pads is None else torch.tensor(pads, dtype=I32, device=DEV), ws=ws, n_split=-1, tail=tail)
+        res.append((host(o) if tail else host(o).reshape(B, L, -1)[:, -1], host(m.k), host(m.v)))
+    assert np.array_equal(res[0][1], res[1][1]) and np.array_equal(res[0][2], res[1][2])
+    close(res[1][0], res[0][0], BF16)
+
+
 def test_mixed_attention_of_a_long_prompt_on_key_fragments():
     """A prompt whose scores do not go through memory: the planned launch, from fragments of the keys -- the same bits as from rows."""
     from phi_3_vision_mlx_amd import ops

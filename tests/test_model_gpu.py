@@ -332,6 +332,29 @@ def test_split_merge_launch_is_a_tested_fallback_of_the_in_launch_merge(text, mo
     assert_logits(runs["1"][1].flatten(0, 1), runs["0"][1].flatten(0, 1), "merge in launch vs merge launch", rel_atol=1e-2)
 
 
+@pytest.mark.parametrize("kw", [{}, dict(use_quantized_cache=True)])
+def test_last_rows_attention_of_a_prompt(kw, monkeypatch):
+    """The final layer's attention of the last rows alone gives the logits and the cache of all rows: one row and rows of unequal padding, a
+    prompt behind a cached one."""
+    from phi_3_vision_mlx_amd.api import load_synthetic
+    model, _ = load_synthetic(blind_model=True, tiny=True, seed=3, std_scale=4.0, device="cuda:0", **kw)
+    ids = np.concatenate([rand_ids(200, 1), rand_ids(200, 2)])
+    mask = np.ones_like(ids)
+    mask[1, :70] = 0
+    pids = np.maximum(np.cumsum(mask, 1) - 1, 0)
+    got = {}
+    for n in (10 ** 9, 40):
+        monkeypatch.setattr(type(model), "TAIL_MIN_L", n)
+        one, c1 = model(input_ids=ids[:1, :130], max_tokens=90)
+        more, _ = model(input_ids=ids[:1, 130:], cache=c1)
+        two, c2 = model(input_ids=ids, pids=pids, mask=mask, max_tokens=4)
+        st = c2[0].state
+        got[n] = [one, more, two] + [t.clone() for t in ((st.k8[..., :200, :], st.v8[..., :200]) if st.quantized else (st.k[..., :200, :], st.v[..., :200]))]
+    for a, b in zip(got[40][:3], got[10 ** 9][:3]):
+        assert_logits(a, b)
+    assert all(torch.equal(a, b) for a, b in zip(got[40][3:], got[10 ** 9][3:]))
+
+
 def test_batched_left_pad(text):
     model, proc, oracle = text
     inputs = proc(["a", "hello world, this is a longer prompt", "mid size"])
