@@ -1548,6 +1548,27 @@ def _dequant(u8, sc, axis):
     return (u8.float() - 128.0) * sc.unsqueeze(axis)
 
 
+@pytest.mark.parametrize("n,t0,scale", [(1, 0, 1.0), (63, 0, 1e-3), (64, 8, 1e30), (65, 16, 1.0), (300, 0, 1e-36)])
+def test_kv_quantize_codes(ops, n, t0, scale):
+    """Codes and scales of the vectorised quantiser, bit for bit: rint(x * (1 / s)) for keys, rint(x / s) for values, s = amax / 127; a token of
+    zeros, scales whose reciprocal overflows, tokens that fill no tile of 64."""
+    B, nh, T = 1, 3, 384
+    k, v = g((B, nh, T, 96), 61, scale), g((B, nh, T, 96), 62, scale)
+    v[:, :, t0] = 0
+    k8, v8 = torch.zeros((B, nh, T, 96), dtype=torch.uint8, device="cuda"), torch.zeros((B, nh, 96, T), dtype=torch.uint8, device="cuda")
+    ks, vs = torch.zeros((B, nh, T), device="cuda"), torch.zeros((B, nh, T), device="cuda")
+    ops.kv_quantize(k.cuda(), v.transpose(2, 3).contiguous().cuda(), k8, v8, ks, vs, t0, n)
+    for x, codes, s, key in ((k, k8, ks, True), (v, v8.transpose(2, 3), vs, False)):
+        x = x[:, :, t0:t0 + n].float()
+        amax = x.abs().amax(-1)
+        want_s = torch.where(amax > 0, amax / 127.0, torch.ones_like(amax))
+        q = torch.round(x * (1.0 / want_s)[..., None] if key else x / want_s[..., None]) + 128
+        assert torch.equal(s.cpu()[:, :, t0:t0 + n], want_s)
+        if not key or scale > 1e-30:                             # (1 / s overflows for keys there, on both sides; the host's codes of NaN are its own)
+            assert torch.equal(codes.cpu()[:, :, t0:t0 + n].float(), q)
+        assert not codes.cpu()[:, :, t0 + n:].any()
+
+
 @pytest.mark.parametrize("past,L,n_split,fused", [(200, 1, 3, False), (200, 1, 4, False), (190, 3, 4, False), (62, 5, 4, False),
                                                    (200, 1, 4, True), (62, 5, 4, True),
                                                    (200, 1, 2, False), (200, 1, 2, True), (126, 5, 2, True), (30, 16, 2, False)])
