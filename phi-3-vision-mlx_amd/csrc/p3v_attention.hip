@@ -30,6 +30,7 @@ struct AttnP {
   int B, L, nh, nkv, past, past_t, past_div, new_t, pad_div, causal, split_mode, n_split, new_is_cache;
   float scale;
   int head_group;              // k_attn_prefill_dma / _pp: heads whose query blocks are interleaved in launch order
+  int any_order;               // keys may be summed in parts
   int cu_blocks;               // k_attn_prefill_dma: query blocks of all heads that give each CU one workgroup, or 0 (query_block)
   float sc2;                   // what S = Q.K^T is multiplied by before exp2: scale * log2(e), or 1 when Q arrives pre-scaled
   int q_prescaled;
@@ -1248,6 +1249,15 @@ constexpr int P3V_ATTN_PP_MIN_L = 3072;                          // tools/attn_s
 // 22.2 : 21.0, 8 (640) 28.2 : 30.3.
 static bool dma_half_blocks(int pairs, int L) { return (long)pairs * p3v_cdiv(L, 128) <= 512; }
 
+// 128 queries on two groups of waves that take every other key tile (k_attn_prefill_il<.., 2>), one workgroup a CU: while that is one round of
+// them -- one row: and a little more -- and there are keys to share.  us, as below : so (32 heads x 96, causal): 576 tokens 15.0 : 14.5, 704 16.9 : 15.7,
+// 1024 23.4 : 19.4, 1152 25.2 : 22.4, 1408 28.9 : 26.9, but 1500 28.9 : 29.1, 2531 50.1 : 58.6; 200 behind 2000 38.6 : 28.6, 400 behind 4000 72.0 : 49.0,
+// 1024 behind 3000 64.1 : 51.0; two rows of 400 behind 1000 32.9 : 24.9, of 512 15.4 : 15.0, but of 640 (320 workgroups) 19.5 : 22.2.
+static bool il_two_groups(const AttnP& p) {
+  const long wgs = (long)p.nh * p.B * p3v_cdiv(p.L, 128);
+  return p.causal && p.past + p.L >= 576 && wgs <= (p.B == 1 ? 352 : 256);
+}
+
 template <int HD>
 static int launch_attn_prefill(const AttnP& p, hipStream_t s) {
   constexpr int LDS = 2 * (64 * (HD * 2 + 16) + HD * (64 * 2 + 16));
@@ -1285,20 +1295,32 @@ static int launch_attn_prefill(const AttnP& p, hipStream_t s) {
     // -> long prompts: 256-query workgroups (half the L2 -> LDS bytes per flop); ONE row of a few thousand tokens: 128-query
     //    workgroups of the interleaved kernel (best balance, two workgroups per CU); several rows: the 128-query kernel up to ~3500 tokens.
     const bool il_auto = p.L >= 6144 || (p.B == 1 ? p.L >= 768 : p.L >= 3584);
+    const bool pin = il >= 0 || pp >= 0 || p3v_tuning().attn_dma_u >= 0 || p3v_tuning().attn_il_waves >= 0;
+    if (p.q_prescaled && (p3v_tuning().attn_il_waves == 42 || (p.any_order && !pin && il_two_groups(p)))) {
+      constexpr int LDS4 = 2 * (3 * 64 * HD * 2 + 3 * HD * 128);
+      static bool attr42_set = false;
+      if (!attr42_set) {
+        if (hipFuncSetAttribute((const void*)k_attn_prefill_il<HD, 4, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS4) != hipSuccess) return P3V_ERR_HIP;
+        attr42_set = true;
+      }
+      hipLaunchKernelGGL((k_attn_prefill_il<HD, 4, 2>), dim3(p.nh * p3v_cdiv(p.L, 128), 1, p.B), dim3(512), LDS4, s, q);
+      P3V_CHECK_LAUNCH();
+      return P3V_OK;
+    }
     if (p.q_prescaled && (il > 0 || (il < 0 && pp != 0 && il_auto))) {   // (pp = 0 pins the dma kernel)
       constexpr int LDS4 = 3 * 64 * HD * 2 + 3 * HD * 128;
       static bool attr4_set = false;
       if (!attr4_set) {
-        if (hipFuncSetAttribute((const void*)k_attn_prefill_il<HD, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS4) != hipSuccess ||
-            hipFuncSetAttribute((const void*)k_attn_prefill_il<HD, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS4) != hipSuccess)
+        if (hipFuncSetAttribute((const void*)k_attn_prefill_il<HD, 8, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS4) != hipSuccess ||
+            hipFuncSetAttribute((const void*)k_attn_prefill_il<HD, 4, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS4) != hipSuccess)
           return P3V_ERR_HIP;
         attr4_set = true;
       }
       // 128-query workgroups (two per CU) while 256-query ones would leave the launch bounded by its longest block
       const int nw = p3v_tuning().attn_il_waves;
       const bool small = nw == 4 || (nw < 0 && p.L < (p.B == 1 ? 2816 : 6144));
-      if (small) hipLaunchKernelGGL((k_attn_prefill_il<HD, 4>), dim3(p.nh * p3v_cdiv(p.L, 128), 1, p.B), dim3(256), LDS4, s, q);
-      else hipLaunchKernelGGL((k_attn_prefill_il<HD, 8>), dim3(p.nh * p3v_cdiv(p.L, 256), 1, p.B), dim3(512), LDS4, s, q);
+      if (small) hipLaunchKernelGGL((k_attn_prefill_il<HD, 4, 1>), dim3(p.nh * p3v_cdiv(p.L, 128), 1, p.B), dim3(256), LDS4, s, q);
+      else hipLaunchKernelGGL((k_attn_prefill_il<HD, 8, 1>), dim3(p.nh * p3v_cdiv(p.L, 256), 1, p.B), dim3(512), LDS4, s, q);
       P3V_CHECK_LAUNCH();
       return P3V_OK;
     }
@@ -1350,6 +1372,7 @@ extern "C" int p3v_attention(const p3v_attn_args_t* a, void* stream) {
   p.past_div = a->past_div > 0 ? a->past_div : 1; p.new_t = a->new_t; p.pad_div = a->pad_div > 0 ? a->pad_div : 1;
   p.causal = a->causal; p.scale = a->scale;
   p.q_prescaled = a->q_prescaled != 0;
+  p.any_order = a->any_order != 0;
   p.sc2 = p.q_prescaled ? 1.f : a->scale * 1.4426950408889634f;
   p.n_split = a->n_split;
   p.split_mode = (a->L <= P3V_DECODE_MAX_L && a->n_split > 1) ? 1 : 0;

@@ -52,16 +52,21 @@ extern "C" int p3v_ildbg_read(unsigned long long* out) {
 // 72 KB of rings -- for prompts of a few thousand tokens, where 256-query blocks leave the launch bounded by its longest block:
 // 2531 tokens are 10 blocks of 4..40 tiles per head, 320 workgroups for 256 CUs).  The price of NW = 4: every tile is fetched
 // per 128 queries, twice the DMA pieces per wave.
-template <int HD, int NW>
-__global__ void __launch_bounds__(64 * NW, 8 / NW) k_attn_prefill_il(AttnP p) {
+// KG = 2 (NW = 4): two groups of four waves share the 128 queries and take every other tile, each through rings of its own; their sums meet in LDS.
+// A tile is 1.25 - 1.4 us of a workgroup's time however idle the chip, so a short prompt's launch was its last queries' tiles one after
+// the other.  (il_two_groups: where, and what it measured.)
+template <int HD, int NW, int KG>
+__global__ void __launch_bounds__(64 * NW * KG, 8 / (NW * KG)) k_attn_prefill_il(AttnP p) {
   constexpr int KROW = HD * 2, VROW = 128, NKS = HD / 32, NDT = HD / 16, CPR = HD / 8;
   constexpr int KTILE = 64 * KROW, VTILE = HD * VROW, RING = 3;
   constexpr int NK = KTILE / 1024, NV = VTILE / 1024, NPW = (NK + NV) / NW, QB = 32 * NW;   // DMA pieces per tile (K, V^T); per wave and batch
   constexpr float THR = 8.f;
   static_assert((NK + NV) % NW == 0 && (NW == 4 || NW == 8), "pieces must divide over the waves");
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];   // K ring [3][KTILE] | V^T ring [3][VTILE]
+  static_assert(KG == 1 || KG * NW == 8, "two groups of four waves");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem_all[];   // a group: K ring [3][KTILE] | V^T ring [3][VTILE]
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, qi = lane & 15;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) % NW, grp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6) / NW;
+  unsigned char* const smem = smem_all + grp * RING * (KTILE + VTILE);
   const int nqb = (p.L + QB - 1) / QB, per_group = p.head_group * nqb;
   const int hgrp = blockIdx.x / per_group, within = blockIdx.x - hgrp * per_group;
   const int qblk = nqb - 1 - within / p.head_group;             // longest (last) query blocks first
@@ -72,7 +77,8 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) k_attn_prefill_il(AttnP p) {
   const int qb0 = qblk * QB, q0 = qb0 + wave * 32;
   const int kv_end = p.causal ? min(total, past + qb0 + QB) : total;
   const int kv_begin = min(pad & ~63, kv_end);
-  const int NT = (kv_end - kv_begin + 63) >> 6;
+  const int NT = (kv_end - kv_begin + 63) >> 6;             // tiles; a group's j-th is tile KG j + grp of them
+  const int NTG = (NT + KG - 1) / KG;                       // turns (a group's last one may have no tile: no key of it is visible)
   const bool active = q0 < p.L;
   const int wave_last = p.causal ? past + q0 + 31 : total;  // last key position this wave can see
   // interior tiles of this wave: kv0 >= pad, kv0 + 64 <= kv_end, (causal) kv0 + 63 <= past + q0, and no padded query rows
@@ -140,7 +146,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) k_attn_prefill_il(AttnP p) {
 #ifdef P3V_IL_NODMA                                              // timing experiment: tiles never move
     return;
 #endif
-    const int lag = p_lag[i], t = min(kt - lag, NT - 1);
+    const int lag = p_lag[i], t = min(KG * (kt - lag) + grp, NT - 1);
     const int so = p_base[i] + t * p_stride[i];
     const unsigned vo = poff[i];                             // (a builtin called on an element of a dependent-size array: hipcc 7.2
     const __amdgpu_buffer_rsrc_t rs = p_rs[i];               //  silently drops the kernel's HOST stub -- link error, no diagnostic)
@@ -191,7 +197,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) k_attn_prefill_il(AttnP p) {
 
   // ---- pieces of a slot.  u = the half whose softmax is in work (VALU), uu = 1 - u the half on the matrix pipe.
   auto mask_half = [&](int u, int j) __attribute__((always_inline)) {                      // (rare) tile j of half u has invisible keys: -inf in place
-    const int kv0 = kv_begin + 64 * j;
+    const int kv0 = kv_begin + 64 * (KG * j + grp);
     const float ninf = -INFINITY;
 #pragma unroll
     for (int st = 0; st < 4; ++st)
@@ -241,7 +247,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) k_attn_prefill_il(AttnP p) {
   }
   auto slot = [&](int u, int j, bool refill, const unsigned char* Vn, const unsigned char* Kn, int dma_kt = -1, int dma_sk = 0, int dma_sv = 0) __attribute__((always_inline)) {
     const int uu = 1 - u;
-    const bool interior = j >= j_int_lo && j <= j_int_hi;
+    const bool interior = KG * j + grp >= j_int_lo && KG * j + grp <= j_int_hi && j >= 0;
     if (!interior) mask_half(u, j);
     __builtin_amdgcn_sched_barrier(0);
 #if P3V_IL_DMA_FRONT == 1
@@ -377,7 +383,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) k_attn_prefill_il(AttnP p) {
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  const int NTw = active ? max(0, min(NT, ((wave_last - kv_begin) >> 6) + 1)) : 0;   // tiles this wave works on (0 .. NTw-1)
+  const int NTw = active ? (max(0, min(NT, ((wave_last - kv_begin) >> 6) + 1)) + KG - 1 - grp) / KG : 0;   // turns this wave works on (0 .. NTw-1)
   if (NT > 0) {
     issue(0, 0, false);                                      // K(0) alone
     issue(1, 0, true);                                       // batch 0 = K(1), V^T(0)
@@ -417,13 +423,44 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) k_attn_prefill_il(AttnP p) {
         pv_tail(1);
         ++j;
       }
-      for (; j <= NT; ++j) {                                 // done (or never had rows): DMA share + barriers only
+      for (; j <= NTG; ++j) {                                // done (or never had rows): DMA share + barriers only
         issue(j + 2, 0, true);
         step_barrier();
       }
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if constexpr (KG == 2) {                                   // the second group's sums to the first, through the rings
+    float* x = (float*)smem_all + wave * 64 + lane;
+    constexpr int ST = 64 * NW, U = 4 * (NDT + 1) + 1;
+    asm volatile("s_barrier" ::: "memory");                  // (every piece of every wave has landed)
+    if (grp == 1) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        x[u * U * ST] = (unset[u] >> lane) & 1 ? -INFINITY : m_run[u];
+#pragma unroll
+        for (int d = 0; d <= NDT; ++d)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) x[(u * U + 1 + 4 * d + r) * ST] = d < NDT ? o[u][d][r] : ol[u][r];
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    asm volatile("s_barrier" ::: "memory");
+    if (grp == 1) return;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {                            // (a group that has seen no key has no reference: its sums are 0)
+      const float m0 = (unset[u] >> lane) & 1 ? -INFINITY : m_run[u], m1 = x[u * U * ST], mx = fmaxf(fmaxf(m0, m1), -1e30f);
+      const float f0 = __builtin_amdgcn_exp2f(m0 - mx), f1 = __builtin_amdgcn_exp2f(m1 - mx);
+#pragma unroll
+      for (int d = 0; d <= NDT; ++d)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float other = x[(u * U + 1 + 4 * d + r) * ST];
+          if (d < NDT) o[u][d][r] = o[u][d][r] * f0 + other * f1;
+          else ol[u][r] = ol[u][r] * f0 + other * f1;
+        }
+    }
+  }
   const float l_fin[2] = {rows_sum(ol[0][0]), rows_sum(ol[1][0])};   // the sum sits in the g = 0 lane of the query's column (all lanes take part)
 #pragma unroll
   for (int u = 0; u < 2; ++u) {

@@ -611,7 +611,7 @@ class Phi3VModel(DecoderModel):
                     o = self._attend_last(q, st.k[i], st.v[i], B, L, past, st, scale)
                 else:
                     ops.attention(q, o, B, L, nh, nkv, hd, scale, True, past=past, k_past=st.k[i], v_past=st.v[i],
-                                  past_t=st.Tp, pad_len=st.pad_len, new_is_cache=True, q_prescaled=True)
+                                  past_t=st.Tp, pad_len=st.pad_len, new_is_cache=True, q_prescaled=True, any_order=not self.w8)
             if mlx4_first:                                      # this layer attended on the exact keys (phi.py:533); from now on: the codes
                 self._mlx4_quantize(st, i, L, qkv, nh)          # (keys from their exact fp32 values: recomputed from `qkv`)
             if last_only and i == cfg.num_hidden_layers - 1 and L > 1:

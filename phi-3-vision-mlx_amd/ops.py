@@ -527,13 +527,14 @@ Q_PRESCALE = 1.4426950408889634          # log2(e): q_scale = Q_PRESCALE * softm
 
 def attention(q, out, B, Lq, nh, nkv, hd, scale, causal, k_new=None, v_new=None, new_t=0, past=0, k_past=None, v_past=None,
               past_t=0, past_div=1, pad_len=None, pad_div=1, d_past=None, ws=None, n_split=0, new_is_cache=False,
-              q_prescaled=False):
+              q_prescaled=False, any_order=False):
     """softmax((q*scale) k^T + mask) v (phi.py:454-457 / phi.py:148), mask never materialised.
     K tensors are [B, nkv, t, hd]; V tensors are TRANSPOSED [B, nkv, hd, t] (t = past_t / new_t).
-    q_prescaled: q already carries scale * log2(e) (rope_kv_append's q_scale = Q_PRESCALE * scale)."""
+    q_prescaled: q already carries scale * log2(e) (rope_kv_append's q_scale = Q_PRESCALE * scale).  any_order: keys may be summed in
+    parts (include/p3v.h)."""
     args = L.AttnArgs(_p(q), _p(k_past), _p(v_past), _p(k_new), _p(v_new), _p(out), _p(pad_len), _p(d_past), _p(ws),
                       B, Lq, nh, nkv, hd, int(past), past_t, past_div, new_t, pad_div, int(causal), float(scale), n_split, int(new_is_cache),
-                      int(bool(q_prescaled)))
+                      int(bool(q_prescaled)), int(bool(any_order)))
     L.check(L.lib().p3v_attention(C.byref(args), _stream()), "attention")
     return out
 

@@ -616,6 +616,17 @@ def test_attention_prefill_kernels(ops, orc, B, L, past, hd, nh, causal, pads, p
         _prefill_case(ops, orc, B, L, past, hd, nh, causal, pads, prescaled, pp, il_waves=4)      # 128-query workgroups
 
 
+@pytest.mark.parametrize("B,L,past,hd,nh,causal,pads,spike", [
+    (1, 64, 0, 96, 2, True, None, None), (1, 17, 0, 96, 1, True, None, None),     # one tile: the second group has none
+    (1, 129, 0, 96, 2, True, None, (0, 128, 70)), (1, 700, 0, 96, 2, True, None, (0, 650, 90)), (1, 1100, 0, 96, 1, True, None, (0, 1000, 999)),
+    (2, 300, 0, 96, 2, True, [0, 77], (1, 299, 150)), (2, 33, 100, 96, 1, True, [3, 100], None),      # row 1: every past key is padding
+    (1, 300, 3000, 96, 8, True, [1000], (0, 20, 1500)), (1, 577, 0, 64, 2, False, None, None)])
+def test_attention_prefill_two_key_groups(ops, orc, B, L, past, hd, nh, causal, pads, spike):
+    """Every other key tile to a second group of waves, the two sums merged: odd and even numbers of tiles, a query whose one high score the
+    other group does not see, padding that leaves a group no visible key, keys far larger than the rings."""
+    _prefill_case(ops, orc, B, L, past, hd, nh, causal, pads, True, 2, il_waves=42, spike=spike)
+
+
 @pytest.mark.parametrize("prescaled", [True, False], ids=["prescaled", "plain"])
 @pytest.mark.parametrize("B,L,past,hd,nh,causal,pads", [
     (1, 128, 0, 96, 2, True, None), (1, 65, 0, 96, 2, True, None), (1, 17, 0, 96, 1, True, None), (2, 200, 0, 96, 2, True, [0, 131]),
