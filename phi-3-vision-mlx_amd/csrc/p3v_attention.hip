@@ -1250,12 +1250,13 @@ constexpr int P3V_ATTN_PP_MIN_L = 3072;                          // tools/attn_s
 static bool dma_half_blocks(int pairs, int L) { return (long)pairs * p3v_cdiv(L, 128) <= 512; }
 
 // 128 queries on two groups of waves that take every other key tile (k_attn_prefill_il<.., 2>), one workgroup a CU: while that is one round of
-// them -- one row: and a little more -- and there are keys to share.  us, as below : so (32 heads x 96, causal): 576 tokens 15.0 : 14.5, 704 16.9 : 15.7,
-// 1024 23.4 : 19.4, 1152 25.2 : 22.4, 1408 28.9 : 26.9, but 1500 28.9 : 29.1, 2531 50.1 : 58.6; 200 behind 2000 38.6 : 28.6, 400 behind 4000 72.0 : 49.0,
+// them -- one row: and a little more -- and there are keys to share.  us, as below : so (32 heads x 96, causal): 704 tokens 16.9 : 15.7,
+// 1024 23.4 : 19.4, 1152 25.2 : 22.4, but 1500 28.9 : 29.1, 2531 50.1 : 58.6 (576 15.0 : 14.5 and 1408 28.9 : 26.9 alone, inside a prompt of 600 and
+// 1300 tokens 0.4 and 0.2 % slower: 800 0.8 % faster, 1024 1.4); 200 behind 2000 38.6 : 28.6, 400 behind 4000 72.0 : 49.0,
 // 1024 behind 3000 64.1 : 51.0; two rows of 400 behind 1000 32.9 : 24.9, of 512 15.4 : 15.0, but of 640 (320 workgroups) 19.5 : 22.2.
 static bool il_two_groups(const AttnP& p) {
   const long wgs = (long)p.nh * p.B * p3v_cdiv(p.L, 128);
-  return p.causal && p.past + p.L >= 576 && wgs <= (p.B == 1 ? 352 : 256);
+  return p.causal && p.past + p.L >= 704 && wgs <= (p.B == 1 ? 288 : 256);
 }
 
 template <int HD>
