@@ -2052,17 +2052,6 @@ __device__ __forceinline__ void fo_project(const FoP f, const int o_wl, unsigned
     }
     __syncthreads();
     timeout = o_timeout != 0;
-    float* xsum = (float*)(lds + 6144);
-    if (Q4) {                                                  // k_gemv3_q4<1, 3>: X = sum of a piece's 16 activations
-      if (tid < 192) {
-        const u32x4_t a = ((const u32x4_t*)xs)[2 * tid], b = ((const u32x4_t*)xs)[2 * tid + 1];
-        float t = 0.f;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) t += (bf16lo(a[j]) + bf16hi(a[j])) + (bf16lo(b[j]) + bf16hi(b[j]));
-        xsum[tid] = t;
-      }
-      __syncthreads();
-    }
 #pragma unroll
     for (int k = 0; k < NU; ++k) {
       if (k == 1 && !two) continue;
@@ -2072,13 +2061,9 @@ __device__ __forceinline__ void fo_project(const FoP f, const int o_wl, unsigned
         for (int j = 0; j < 3; ++j) {
           const int pc = j * 64 + lane;
           const u32x4_t xa = ((const u32x4_t*)xs)[2 * pc], xb = ((const u32x4_t*)xs)[2 * pc + 1];
-          const float X = xsum[pc], X128 = 128.f * X;
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const float D = dot8_q4(oq[k][h][j][1], xb, dot8_q4(oq[k][h][j][0], xa, 0.f));
-            const float c = bf16lo(osb[k][h][j]) * (D - X128) + bf16hi(osb[k][h][j]) * X;
-            if (h == 0) a0 += c; else a1 += c;
-          }
+          const float X = sum8_q4(xb, sum8_q4(xa, 0.f));
+          a0 = piece_q4(oq[k][0][j][0], oq[k][0][j][1], osb[k][0][j], xa, xb, X, a0);
+          a1 = piece_q4(oq[k][1][j][0], oq[k][1][j][1], osb[k][1][j], xa, xb, X, a1);
         }
         if (k == 0) TMARK(13);
         a0 = wave_sum(a0);

@@ -25,3 +25,20 @@ __device__ __forceinline__ float dot8_q4(uint32_t r, u32x4_t x, float acc) {
   return acc;
 }
 
+// += the sum of 8 activations (the pair of ones goes through a register: as a constant hipcc may encode it as an inline 1.0, which is one bf16 only)
+__device__ __forceinline__ float sum8_q4(u32x4_t x, float acc) {
+  const q4_oct_t xv = __builtin_bit_cast(q4_oct_t, x);
+  uint32_t ones = 0x3F803F80u;
+  asm("" : "+v"(ones));
+  const q4_pair_t o = __builtin_bit_cast(q4_pair_t, ones);
+  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(xv, xv, 0, 1), o, acc, false);
+  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(xv, xv, 2, 3), o, acc, false);
+  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(xv, xv, 4, 5), o, acc, false);
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(xv, xv, 6, 7), o, acc, false);
+}
+
+// one 16-weight piece of a row: acc + scale sum_k x_k q_k + bias X, X = sum_k x_k (the - 128 X of the pairs 128 + q opens the chain)
+__device__ __forceinline__ float piece_q4(uint32_t w0, uint32_t w1, uint32_t sb, u32x4_t xa, u32x4_t xb, float X, float acc) {
+  const float S = dot8_q4(w1, xb, dot8_q4(w0, xa, -128.f * X));
+  return fmaf(bf16lo(sb), S, fmaf(bf16hi(sb), X, acc));
+}

@@ -8,14 +8,14 @@
 //      is the bf16 PAIR (128 + q[2j], 128 + q[2j+1]) -- 0x4300 | q is exactly 128 + q in bf16 -- ready for v_dot2c_f32_bf16
 //      against the activation pair (x[2j], x[2j+1]);
 //   SB [N, K/64] u32: scale (bf16) | bias (bf16) << 16.
-// Per 16-weight piece p of a row, with D = sum_k x_k (128 + q_k) and X = sum_k x_k (16 activations, shared by all rows,
-// precomputed in LDS):   contribution = scale * (D - 128 X) + bias * X.
-// One row (k_gemv3_q4): x (+RMSNorm) staged in LDS while the weights of the wave's first U row pairs are on their way, their sums and their
+// Per 16-weight piece p of a row, with X = sum_k x_k (16 activations; each lane sums its own pieces, once for all its rows):
+//   S = - 128 X + sum_k x_k (128 + q_k),   contribution = scale * S + bias * X.
+// One row (k_gemv3_q4): x (+RMSNorm) staged in LDS while the weights of the wave's first row pair are on their way, the sums of U pairs and their
 // epilogue together at the end.  The bytes (N*K/2 + N*K/16) are a quarter of the bf16 kernel's for as many products, so its instructions count as much as
-// its bytes: 11 per 8 weights, 6 per piece, and one reduction and epilogue per U pairs instead of one each (gate_up: 880 vector instructions a
-// wave, 3 of its 8 us; 1180 before).  16 waves per CU: with attention and o_proj as two launches 4.08 ms per four steps of the 32-layer decoder at 128
-// columns (8 waves 4.11, 12 4.14, 20 4.12; before 4.52; 3.9 with the two as one, k_attn_rows_o):
-// per launch gate_up 9.0 -> 8.1 us, qkv 7.2 -> 6.6, down 7.1 -> 5.9.
+// its bytes: 11 per 8 weights, 4 per piece, one reduction and epilogue per U pairs, and a norm whose steps all four waves share alike.  What else
+// bounds it is where the requests stand (see the pipeline below).  8 waves per CU (6, 10, 16 with the rows of 16384 / 9216: 9.2 / 5.6, 7.8 / 6.2,
+// 8.8 / 6.2 us against 7.8 / 5.6).  Per launch (weights from memory): gate_up 8.9 -> 7.8 us, qkv 6.85 -> 5.6, down 6.2 -> 5.7; four steps of the
+// 32-layer decoder at 128 columns 3.91 -> 3.61 ms.
 #include <stdlib.h>
 
 #include <type_traits>
@@ -34,6 +34,12 @@ typedef std::integral_constant<int, 1> QC1;
 template <int I, int N, class F>
 __device__ __forceinline__ void q4_each(F&& f) {          // f(integral_constant I .. N - 1), unrolled
   if constexpr (I < N) { f(std::integral_constant<int, I>{}); q4_each<I + 1, N>(f); }
+}
+// + the squares of a bf16 pair, fp32
+__device__ __forceinline__ float sumsq_pair(uint32_t x, float acc) {
+  asm("" : "+v"(x));                                    // (hipcc folds bit_casts of loaded words: see dot8)
+  const q4_pair_t v = __builtin_bit_cast(q4_pair_t, x);
+  return __builtin_amdgcn_fdot2_f32_bf16(v, v, acc, false);
 }
 // one addition of a wave reduction for two values at once: a's in the lower half (even rows of 16 lanes), b's in the upper (odd rows)
 __device__ __forceinline__ float swap32_add(float a, float b) {
@@ -54,18 +60,20 @@ template <int NST, int NP, int DEPTH, bool ONE, int STEP>
 __device__ __forceinline__ void gemv3_q4_body(const GemvQ4P& p, int units_per_wave, int wpw, unsigned char* smem, float* red, const GemvStepP* sp) {
   constexpr int PIECES = NST * NP * 64;                 // 16-weight pieces per row
   constexpr int K = PIECES * 16, XCH = K / 8;           // 16-byte x chunks
-  constexpr int XC = (XCH + 255) / 256;
+  // x is staged in steps that all four waves share alike: 16 bytes a thread, 8 where 256 threads x 16 bytes do not divide the row
+  constexpr int XW = XCH % 256 ? 2 : 4, XC = K / 2 / (256 * XW);
+  static_assert(XC * 256 * XW * 2 == K, "whole steps");
+  typedef uint32_t xw_t __attribute__((ext_vector_type(XW)));
   static_assert(DEPTH % NST == 0 && DEPTH / NST <= 4, "whole row pairs, at most four");
   constexpr int U = DEPTH / NST, LU = U == 3 ? 4 : U;   // row pairs requested together; lanes are dealt to LU of them
   u32x4_t* xs = (u32x4_t*)smem;                         // [K] bf16 x (normalised)
-  float* xsum = (float*)(smem + K * 2);                 // [PIECES] sum of the 16 activations of a piece
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool silu = p.epi == P3V_EPI_SILU_MUL, has_res = p.epi == P3V_EPI_RESID_BF16;
   const int u_begin = wave < wpw ? min(p.units, ((int)blockIdx.x * wpw + wave) * units_per_wave) : p.units;   // (wpw: see p3v_gemv_wpw)
   const int u_end = min(p.units, u_begin + units_per_wave);
   const int n_st = (u_end - u_begin) * NST;
 
-  u32x4_t xv[XC], gv[XC];
+  xw_t xv[XC], gv[XC];
   const bf16_t* xrow[1] = {p.x};
   if (STEP == STEP_BEGIN) {
     int id = sp->tok[0];                                // (uniform: a scalar load)
@@ -74,9 +82,9 @@ __device__ __forceinline__ void gemv3_q4_body(const GemvQ4P& p, int units_per_wa
   }
 #pragma unroll
   for (int k = 0; k < XC; ++k) {
-    const int c = min(tid + k * 256, XCH - 1);
-    xv[k] = ((const u32x4_t*)xrow[0])[c];
-    gv[k] = ((const u32x4_t*)(p.norm_w ? p.norm_w : xrow[0]))[c];
+    const int c = tid + k * 256;
+    xv[k] = ((const xw_t*)xrow[0])[c];
+    gv[k] = ((const xw_t*)(p.norm_w ? p.norm_w : xrow[0]))[c];
   }
   u32x2_t wbuf[DEPTH][2][NP];
   uint32_t sbuf[DEPTH][2][NP];
@@ -98,16 +106,14 @@ __device__ __forceinline__ void gemv3_q4_body(const GemvQ4P& p, int units_per_wa
     }
     __builtin_amdgcn_sched_barrier(0);                   // stage by stage: they are waited for in this order
   };
-  auto stage_x = [&]() {                                 // x (normalised) and its piece sums into LDS: all waves of the workgroup
+  auto stage_x = [&]() {                                 // x (normalised) into LDS: all waves of the workgroup
     float r = 1.f;
     if (p.norm_w) {
       float ss = 0.f;
 #pragma unroll
       for (int k = 0; k < XC; ++k)
-        if (tid + k * 256 < XCH) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) { const float a = bf16lo(xv[k][j]), b = bf16hi(xv[k][j]); ss += a * a + b * b; }
-        }
+        for (int j = 0; j < XW; ++j) ss = sumsq_pair(xv[k][j], ss);
       ss = wave_sum(ss);
       if (lane == 0) red[wave] = ss;
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -116,20 +122,12 @@ __device__ __forceinline__ void gemv3_q4_body(const GemvQ4P& p, int units_per_wa
     }
 #pragma unroll
     for (int k = 0; k < XC; ++k) {
-      const int c = tid + k * 256;
-      if (c < XCH) {                                       // (wave-uniform: XCH is a multiple of 64)
-        u32x4_t o = xv[k];
-        if (p.norm_w) {
+      xw_t o = xv[k];
+      if (p.norm_w) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            o[j] = rms_pair(xv[k][j], r, gv[k][j]);
-        }
-        xs[c] = o;
-        float t = 0.f;                                     // X of the piece whose halves lie in lanes 2 i and 2 i + 1, from the (rounded) activations the dots see
-#pragma unroll
-        for (int j = 0; j < 4; ++j) { const float h = bf16lo(o[j]) + bf16hi(o[j]); t += h + P3V_DPP_F32(h, 0xB1); }
-        if (!(tid & 1)) xsum[c >> 1] = t;
+        for (int j = 0; j < XW; ++j) o[j] = rms_pair(xv[k][j], r, gv[k][j]);
       }
+      ((xw_t*)xs)[tid + k * 256] = o;
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -150,13 +148,19 @@ __device__ __forceinline__ void gemv3_q4_body(const GemvQ4P& p, int units_per_wa
   auto resid_of = [&](int gs) {                                  // (an unconditional load: x where there is no residual)
     return *(const uint32_t*)(has_res ? p.resid + 2 * min(u_begin + gs / NST + unit_of, u_end - 1) : xrow[0]);
   };
-  q4_each<0, DEPTH>([&](auto d) { issue(d, d); });
+  // A load that finds its CU's queue of outstanding lines full (some 28 KB: the CU's share of the memory rate for one latency) holds its wave, so
+  // a wave that requests all its rows first comes to x, which has long been there, only when most of the CU's weights are: the norm and the
+  // products were done behind the stream (9216 rows: last wave past its requests at 3.1 us, its norm at 4.5, end 5.5).  One stage before x, one
+  // after it, the others as stages are consumed: 8 waves x 3 KB fill the queue.
+  constexpr int AHEAD = ONE && DEPTH > 2 ? 2 : DEPTH;
+  issue(0, QC0{});
   rbuf = resid_of(0);
   stage_x();
+  q4_each<1, AHEAD>([&](auto d) { issue(d, d); });
 
   // A group of U row pairs: their sums stay in the lanes until all are there, the last two steps of the reduction serve two pairs
   // each (the additions of wave_sum, in its order), and the epilogue runs once, lane unit_of * 64 / LU holding pair unit_of.
-  float acc[U][2];
+  float acc[U][2], xsum[NST * NP];
   auto compute = [&](auto dc) {
     constexpr int d = decltype(dc)::value, un = d / NST, s = d % NST;
     if constexpr (s == 0) acc[un][0] = acc[un][1] = 0.f;
@@ -164,14 +168,10 @@ __device__ __forceinline__ void gemv3_q4_body(const GemvQ4P& p, int units_per_wa
     for (int j = 0; j < NP; ++j) {
       const int pc = (s * NP + j) * 64 + lane;
       const u32x4_t xa = xs[2 * pc], xb = xs[2 * pc + 1];
-      const float X = xsum[pc], X128 = 128.f * X;
+      if constexpr (un == 0) xsum[s * NP + j] = sum8_q4(xb, sum8_q4(xa, 0.f));      // (the same for every row)
+      const float X = xsum[s * NP + j];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const u32x2_t w = wbuf[d][h][j];
-        const float D = dot8_q4(w[1], xb, dot8_q4(w[0], xa, 0.f));
-        const uint32_t sb = sbuf[d][h][j];
-        acc[un][h] += bf16lo(sb) * (D - X128) + bf16hi(sb) * X;
-      }
+      for (int h = 0; h < 2; ++h) acc[un][h] = piece_q4(wbuf[d][h][j][0], wbuf[d][h][j][1], sbuf[d][h][j], xa, xb, X, acc[un][h]);
     }
   };
   auto finish = [&](int u0) {
@@ -216,7 +216,11 @@ __device__ __forceinline__ void gemv3_q4_body(const GemvQ4P& p, int units_per_wa
     finish(u_begin + gs / NST);
     rbuf = next;
   }
-  q4_each<0, DEPTH>([&](auto d) { compute(d); });
+  q4_each<0, DEPTH>([&](auto d) {
+    compute(d);
+    constexpr int next = decltype(d)::value + AHEAD;
+    if constexpr (next < DEPTH) issue(gs + next, std::integral_constant<int, next>{});
+  });
   finish(u_begin + gs / NST);
   if (STEP == STEP_END && LU > 1) {                              // the lanes that finished a pair: their candidates meet in lane 0
 #pragma unroll
@@ -286,7 +290,7 @@ static int launch_gemv3_q4(const GemvQ4P& p, hipStream_t s, const GemvStepP* sp 
   int wpw = p3v_gemv_wpw(waves, n_cu, p3v_tuning().gemv_wpw);
   if (STEP != STEP_NONE && p3v_cdiv(waves, wpw) > P3V_GEMV_STEP_MAX_WG) wpw = 4;
   const dim3 grid(p3v_cdiv(waves, wpw));
-  const size_t lds = (size_t)p.K * 2 + (size_t)p.K / 4;
+  const size_t lds = (size_t)p.K * 2;
   if (STEP != STEP_NONE && (int)grid.x > P3V_GEMV_STEP_MAX_WG) return P3V_ERR_UNSUPPORTED;   // (amax_ws holds one candidate per workgroup)
   const int pairs = upw <= 4 / NST ? upw : NST == 1 && upw % 4 && upw % 3 == 0 ? 3 : 4 / NST;
   auto launch = [&](auto d) {
