@@ -111,9 +111,11 @@ __device__ __forceinline__ void gemv3_f8_body(const GemvF8P& p, int units_per_wa
     step_tail();
     return;
   }
+  // (one step ahead of x, not two: a load that finds its CU's queue of outstanding lines full holds its wave, which then reaches its norm only
+  //  when the CU's weights are nearly all there.  9216 rows 7.25 -> 6.3 us, 16384 rows 10.6 -> 10.0, 32064 rows 17.8 -> 17.3)
   issue(0, IC0{});
-  if constexpr (NS != 1) issue(1, IC1{});
   stage_x();
+  if constexpr (NS != 1) issue(1, IC1{});
 
   float a0 = 0.f, a1 = 0.f;
   auto compute = [&](int gs, auto bufc) {
@@ -484,9 +486,12 @@ static int launch_gemv3_f8(const GemvF8P& p, hipStream_t s, const GemvStepP* sp 
     if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&pr, dev) != hipSuccess) return P3V_ERR_HIP;
     n_cu = pr.multiProcessorCount;
   }
-  const int wpc = p3v_tuning().gemv_f8_wpc;   // waves per CU (a stage is half the bytes of the bf16 kernel's: twice the waves keep as many in flight; 8: 1.321, 16: 1.301, 24: 1.333 ms/step)
-  int upw = p3v_cdiv(p.units, n_cu * wpc);
-  if (upw < 1) upw = 1;
+  // Waves per CU: 8 x 6 KB fill the CU's queue of outstanding lines, and a norm is then done by two workgroups of it instead of four (9216 rows 6.3 us
+  // against 6.8 with 16 waves, 16384 rows 10.0 : 10.2) -- but 16 where 8 would hold more row pairs than the straight-line code takes (32064 rows
+  // 18.6 : 17.3).
+  const int forced = p3v_tuning().gemv_f8_wpc;
+  auto pairs_of = [&](int wpc) { return p3v_cdiv(p.units, n_cu * wpc); };
+  const int upw = forced > 0 ? pairs_of(forced) : pairs_of(8) * NST <= 4 ? pairs_of(8) : pairs_of(16);
   const int waves = p3v_cdiv(p.units, upw);
   const int wpw = p3v_gemv_wpw(waves, n_cu, p3v_tuning().gemv_wpw);
   const dim3 grid(p3v_cdiv(waves, wpw));
