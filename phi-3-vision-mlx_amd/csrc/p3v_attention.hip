@@ -1966,14 +1966,19 @@ __host__ __device__ __forceinline__ FoMap fo_map(int L, int n_split, int nh, int
 // else uses any more.
 enum { FO_NONE = 0, FO_BF16 = 1, FO_F8 = 2, FO_Q4 = 3 };
 struct FoP { const void* o_w; const void* o_scale; bf16_t* o_x; const bf16_t* out; int nh; };
-template <int KIND, int NU = 1>                                // NU = 2: the workgroup may carry a SECOND unit (o_wl2 >= 0): two row pairs per wave
+// A workgroup may carry a SECOND unit (o_wl2 >= 0): as two row pairs per wave (NU = 2), or, where nobody else needs its CU (NW = 8), by four
+// more waves -- a wave alone on its SIMD issues a vector instruction per 8 - 10 cycles, two share it without loss.
+template <int KIND, int NU = 1, int NW = 4>
 __device__ __forceinline__ void fo_project(const FoP f, const int o_wl, unsigned char* lds, const int o_wl2 = -1) {
   constexpr bool F8 = KIND == FO_F8, Q4 = KIND == FO_Q4;
   constexpr int HD = 96, NJ = KIND == FO_BF16 ? 6 : 3;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int Kd = f.nh * HD;
   const size_t row_bytes = (size_t)Kd * (Q4 ? 1 : F8 ? 2 : 4) / 2;
+  static_assert(NW == 4 || (NW == 8 && NU == 1), "one row pair per wave of eight");
   const bool two = NU > 1 && o_wl2 >= 0;                       // workgroup-uniform
+  const bool mine = NW == 4 || wave < 4 || o_wl2 >= 0;         // (a wave without rows requests the first unit's and stores nothing)
+  const int unit = NW == 8 && wave >= 4 && o_wl2 >= 0 ? o_wl2 : o_wl;
   int o_u[NU];                                                 // row pair (2 o_u, 2 o_u + 1) of unit k
   u32x4_t ow[NU][2][Q4 ? 1 : NJ];                              // bf16 / e4m3: 16-byte chunks
   u32x2_t oq[NU][2][Q4 ? 3 : 1];                               // 4-bit: 16-weight pieces (8 bytes) + their scale | bias words
@@ -1982,7 +1987,7 @@ __device__ __forceinline__ void fo_project(const FoP f, const int o_wl, unsigned
   float osc[NU][2];
 #pragma unroll
   for (int k = 0; k < NU; ++k) {
-    o_u[k] = (k == 0 ? o_wl : o_wl2) * 4 + wave;
+    o_u[k] = (k == 0 ? unit : o_wl2) * 4 + (wave & 3);
     if (k == 1 && !two) continue;
     const unsigned char* r0p = (const unsigned char*)f.o_w + (size_t)(2 * o_u[k]) * row_bytes;
     if (Q4) {
@@ -2030,24 +2035,24 @@ __device__ __forceinline__ void fo_project(const FoP f, const int o_wl, unsigned
     }
     TMARK(12);
     __syncthreads();
-    // every wave fetches a quarter of the vector (6 words per lane) into LDS, re-fetching the rare straggler word
+    // every wave fetches its share of the vector (6 words per lane of four waves) into LDS, re-fetching the rare straggler word
     uint32_t* xs = (uint32_t*)lds;                              // the K/V tiles are dead by now (barrier above)
     bool timeout = o_timeout != 0;
     {
-      const int NW = f.nh * HD / 2 / 4;                        // words per wave: 384
-      uint32_t xv[6];
+      constexpr int NX = 24 / NW;                              // words per lane of a wave's share
+      uint32_t xv[NX];
       for (unsigned tries = 0; !timeout; ++tries) {
         bool bad = false;
 #pragma unroll
-        for (int j = 0; j < 6; ++j) xv[j] = __hip_atomic_load(src + wave * NW + j * 64 + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int j = 0; j < NX; ++j) xv[j] = __hip_atomic_load(src + wave * (NX * 64) + j * 64 + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-        for (int j = 0; j < 6; ++j) bad |= (xv[j] & 0xffffu) == 0xffffu || (xv[j] >> 16) == 0xffffu;
+        for (int j = 0; j < NX; ++j) bad |= (xv[j] & 0xffffu) == 0xffffu || (xv[j] >> 16) == 0xffffu;
         if (!__any(bad)) break;
         if (tries >= (1u << 12)) timeout = true;
         __builtin_amdgcn_s_sleep(2);
       }
 #pragma unroll
-      for (int j = 0; j < 6; ++j) xs[wave * NW + j * 64 + lane] = xv[j];
+      for (int j = 0; j < NX; ++j) xs[wave * (NX * 64) + j * 64 + lane] = xv[j];
       if (timeout && lane == 0) o_timeout = 1;
     }
     __syncthreads();
@@ -2089,7 +2094,7 @@ __device__ __forceinline__ void fo_project(const FoP f, const int o_wl, unsigned
         a0 = wave_sum(a0);
         a1 = wave_sum(a1);
       }
-      if (lane == 0) {
+      if (lane == 0 && mine) {
         const float v0 = bf16lo(ores[k]) + bf16_round(a0), v1 = bf16hi(ores[k]) + bf16_round(a1);
         *(uint32_t*)(f.o_x + 2 * o_u[k]) = timeout ? 0x7fc07fc0u : pack_bf16x2(v0, v1);     // NaN: loud (api._rows raises)
       }
@@ -2783,13 +2788,15 @@ __global__ void __launch_bounds__(256, 2) k_attn_decode_rows(AttnDecP p) {
 // o_proj + residual as k_attn_combine_o's do: their rows of W_o are requested at once and wait in registers for the heads' words.  No split
 // partials, so one hand-over through memory where attention, merge launch and merge had two and a launch boundary.  224 workgroups,
 // all resident at once.  What bounds it: launch, new rows, hand-over and dot 6.5 us, then one CU's share of the keys at 28-30 KB/us (eight
-// waves a head instead of four: no faster).  4-bit / bf16 weights, 60 keys 9.84 / 9.78 -> 7.91 / 7.54 us, 130 keys 9.98 / 10.0 -> 9.24 / 9.39.
+// waves a head instead of four: no faster).  4-bit / bf16 weights, 60 keys 9.84 / 9.78 -> 7.91 / 7.54 us, 130 keys 9.98 / 10.0 -> 9.24 / 9.39; eight
+// projecting waves with a row pair each instead of four with two: 4-bit 0.3 us less.
 template <int KIND>
-__global__ void __launch_bounds__(256) k_attn_rows_o(AttnDecP p, int n_units) {
+__global__ void __launch_bounds__(512) k_attn_rows_o(AttnDecP p, int n_units) {
   __shared__ RowsLds lds;
   static_assert(sizeof(lds.tiles) >= 7 * 1024 + 768, "the projection's share");
   const int u = (int)blockIdx.x - p.nh;
   if (u < 0) {
+    if (threadIdx.x >= 256) return;                            // (a head takes four waves, two units eight)
     if (blockIdx.x == 0) {                                     // re-arm the other layer parity's buffer (nobody reads it in this launch)
       uint32_t* ra = (uint32_t*)p.o_rearm;
       for (int i = threadIdx.x; i < p.nh * 96 / 2; i += 256) ra[i] = 0xffffffffu;
@@ -2798,24 +2805,23 @@ __global__ void __launch_bounds__(256) k_attn_rows_o(AttnDecP p, int n_units) {
     return;
   }
   const int n_uw = (int)gridDim.x - p.nh;
-  fo_project<KIND, 2>(FoP{p.o_w, p.o_sb, p.o_x, p.out, p.nh}, u, lds.tiles[0], u + n_uw < n_units ? u + n_uw : -1);
+  fo_project<KIND, 1, 8>(FoP{p.o_w, p.o_sb, p.o_x, p.out, p.nh}, u, lds.tiles[0], u + n_uw < n_units ? u + n_uw : -1);
 }
 
 
-// merge split-KV partials: one block of G = 4 or 8 64-lane groups per (b, head, query): thread (grp, d) loads
+// merge split-KV partials: one block of G = 4, 8 or 16 64-lane groups (combine_threads) per (b, head, query): thread (grp, d) loads
 // (m, l, o[d]) of its share of the splits (batches of 4 independent loads), reduces them against its own
 // running max, and the groups are merged through LDS.
 // (the body is shared with k_attn_combine_o below: WT = the row goes out as 48 packed words with write-through stores, for
 //  consumers polling them in the same launch; the value of every element is computed by the same expression either way)
 template <bool WT>
-__device__ __forceinline__ void combine_rows(const float* __restrict__ ws, bf16_t* __restrict__ out, int L, int nh, int hd, int n_split, int block) {
+__device__ __forceinline__ void combine_rows(const float* __restrict__ ws, bf16_t* __restrict__ out, int L, int nh, int hd, int n_split, int block, int G) {
   __shared__ float pm[CMB_G], pl[CMB_G];
   __shared__ float part[CMB_G][128];
   const int qi = block % L, head = (block / L) % nh, b = block / (L * nh);
   const float* base = ws + (((size_t)b * nh + head) * n_split * 16 + qi) * (hd + 2);
   const size_t sstr = (size_t)16 * (hd + 2);
   const int t = threadIdx.x, grp = t >> 6, d0 = t & 63;       // G groups x 64 lanes; lane handles d0 and d0+64
-  const int G = blockDim.x >> 6;                              // 4, 8 or 16 (combine_threads)
   const int per = (n_split + G - 1) / G, s0 = grp * per, s1 = min(n_split, s0 + per);
   const bool two = d0 + 64 < hd;
   float m = -INFINITY, l = 0.f, a0 = 0.f, a1 = 0.f;
@@ -2867,7 +2873,7 @@ __device__ __forceinline__ void combine_rows(const float* __restrict__ ws, bf16_
 
 __global__ void __launch_bounds__(64 * CMB_G) k_attn_combine2(const float* __restrict__ ws, bf16_t* __restrict__ out, int L,
                                                               int nh, int hd, int n_split) {
-  combine_rows<false>(ws, out, L, nh, hd, n_split, (int)blockIdx.x);
+  combine_rows<false>(ws, out, L, nh, hd, n_split, (int)blockIdx.x, (int)(blockDim.x >> 6));
 }
 
 // Long contexts (the split-KV plans whose partials are merged by a launch of their own: more than 48 tiles of 128 keys, i.e.
@@ -2878,19 +2884,19 @@ __global__ void __launch_bounds__(64 * CMB_G) k_attn_combine2(const float* __res
 // 32k keys: combine 4.9 us + o_proj 5.0 us -> one launch.
 template <int KIND>
 __global__ void __launch_bounds__(512) k_attn_combine_o(const float* __restrict__ ws, bf16_t* __restrict__ out, bf16_t* __restrict__ o_rearm,
-                                                        const void* o_w, const void* o_sb, bf16_t* o_x, int nh, int n_split, int n_units) {
+                                                        const void* o_w, const void* o_sb, bf16_t* o_x, int nh, int n_split, int n_units, int G) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[7 * 1024 + 768];
   if ((int)blockIdx.x < nh) {
+    if ((int)threadIdx.x >= 64 * G) return;                    // (a head takes G waves, two units eight)
     if (blockIdx.x == 0) {                                     // re-arm the other layer parity's buffer (nobody reads it in this launch)
       uint32_t* ra = (uint32_t*)o_rearm;
-      for (int i = threadIdx.x; i < nh * 96 / 2; i += blockDim.x) ra[i] = 0xffffffffu;
+      for (int i = threadIdx.x; i < nh * 96 / 2; i += 64 * G) ra[i] = 0xffffffffu;
     }
-    combine_rows<true>(ws, out, 1, nh, 96, n_split, (int)blockIdx.x);
+    combine_rows<true>(ws, out, 1, nh, 96, n_split, (int)blockIdx.x, G);
     return;
   }
-  if (threadIdx.x >= 256) return;                              // (the merging workgroups use all 64 x G threads, a unit four waves)
   const int n_uw = (int)gridDim.x - nh, u = (int)blockIdx.x - nh;
-  fo_project<KIND, 2>(FoP{o_w, o_sb, o_x, out, nh}, u, lds, u + n_uw < n_units ? u + n_uw : -1);
+  fo_project<KIND, 1, 8>(FoP{o_w, o_sb, o_x, out, nh}, u, lds, u + n_uw < n_units ? u + n_uw : -1);
 }
 
 // B = L = 1, 32 x 96: one workgroup per head + one per two row-pair quartets, all resident at once (one per CU, 8 CUs of head-room)
@@ -2906,8 +2912,8 @@ template <int KIND>
 static int launch_combine_o(const float* ws, void* out, void* o_rearm, const void* o_w, const void* o_sb, void* o_x, int n_heads, int n_split,
                             int o_n, hipStream_t s) {
   const int n_units = o_n / 8, grid_o = n_heads + (n_units + 1) / 2;
-  hipLaunchKernelGGL(k_attn_combine_o<KIND>, dim3(grid_o), dim3(combine_threads(n_split)), 0, s, ws, (bf16_t*)out, (bf16_t*)o_rearm, o_w, o_sb,
-                     (bf16_t*)o_x, n_heads, n_split, n_units);
+  hipLaunchKernelGGL(k_attn_combine_o<KIND>, dim3(grid_o), dim3(512), 0, s, ws, (bf16_t*)out, (bf16_t*)o_rearm, o_w, o_sb, (bf16_t*)o_x, n_heads,
+                     n_split, n_units, combine_threads(n_split) / 64);
   P3V_CHECK_LAUNCH();
   return P3V_OK;
 }
@@ -3047,8 +3053,8 @@ extern "C" int p3v_attention_decode(const p3v_attn_decode_args_t* a, void* strea
   if (fuse_form == 2 && row1) {                                // attention + o_proj + residual in one launch, without split partials
     const int n_units = a->o_n / 8;
     const dim3 grid_o(a->n_heads + (n_units + 1) / 2);
-    if (a->o_proj_sb) hipLaunchKernelGGL(k_attn_rows_o<FO_Q4>, grid_o, dim3(256), 0, s, p, n_units);
-    else hipLaunchKernelGGL(k_attn_rows_o<FO_BF16>, grid_o, dim3(256), 0, s, p, n_units);
+    if (a->o_proj_sb) hipLaunchKernelGGL(k_attn_rows_o<FO_Q4>, grid_o, dim3(512), 0, s, p, n_units);
+    else hipLaunchKernelGGL(k_attn_rows_o<FO_BF16>, grid_o, dim3(512), 0, s, p, n_units);
     P3V_CHECK_LAUNCH();
     return P3V_OK;
   }
