@@ -11,6 +11,10 @@
 //             27.7, qkv 26 -> 24.3, but down 22.6 -> 25.4; the weights lie unpadded, as the other kernels and the loader have them.
 //             128 x 128 tiles (W x 2 staged, half the workgroups) in one pass or with partials in memory were not faster on any shape; where
 //             the K slices that fill the chip again are summed inside the launch they are (p3v_gemm_merge, at the end).
+//             Plain partials of a long K: 128 x 96 tiles in 8 slices where that is a workgroup for more CUs than 64 columns reach (3072 columns:
+//             256 against 192), each of which then asks for less (448 against 768 KB of 8192; the requests alone 16.5 -> 11.5 us).  With the
+//             reduction, 3072 x 8192: 128 rows 24.2 -> 21.8 us, 64 rows 19.9 -> 17.3, 40 rows 18.4 -> 16.3; x 6144 (12 K-tiles a slice) 21.6 -> 20.4;
+//             x 3072 would have 6 K-tiles a slice: 15.5 -> 16.6, so slices of fewer than 12 stay on 64 columns.
 //   staging   LDS-DMA into a ring of 6 stages (A 16 KiB + W 8 KiB each), 5 in flight behind a counted vmcnt; one workgroup per CU
 //             (<= 64 rows: 64-row tiles, A 8 KiB per stage -- a third less staged per K-tile, the same sums bit for bit: 60 -> 53 us
 //             per decoder layer at 17 rows)
@@ -26,7 +30,7 @@
 
 #define SK_BM 128
 #define SK_BK 64
-#define SK_TN 64                    // tile width of the one-pass and partial-sum forms (MERGE: 128)
+#define SK_TN 64                    // tile width of the one-pass form and of most partial-sum forms (else 96, see sk_plan; MERGE: 128)
 #ifndef SK_ABL
 #define SK_ABL 0                    // timing experiments: 1 = A always K-tile 0 (one L2/L1-hot tile), 2 = W likewise, 3 = no MFMAs after K-tile 0
 #endif
@@ -35,34 +39,24 @@
 typedef __attribute__((address_space(3))) void* lptr_t;
 
 template <int TN, int TM = SK_BM> struct SkCfg {
-  static_assert(TM == 128 || (TM == 64 && TN == 64), "64-row tiles: prompts / batches of <= 64 rows, 64-column tiles");
-  static constexpr int NS = TN == 64 ? 6 : 4;                  // ring stages (NS - 1 ahead)
+  static_assert(TM == 128 || (TM == 64 && TN <= 96), "64-row tiles: prompts / batches of <= 64 rows, 64- and 96-column tiles");
+  static constexpr int NS = TN == 64 ? 6 : TN == 96 ? 5 : 4;   // ring stages (NS - 1 ahead)
   static constexpr int A_BYTES = TM * SK_BK * 2, W_BYTES = TN * SK_BK * 2, STAGE = A_BYTES + W_BYTES, LDS = NS * STAGE;
   static constexpr int AQ = TM / 32, WQ = TN / 32;             // A / W pieces (8 rows x 128 B) per producer wave and stage
   static constexpr int PER = AQ + WQ;                          // DMA instructions per producer wave and stage
-  static constexpr int NI = TN == 64 ? TM / 64 : 4;            // 16-row blocks per consumer wave (its 64 columns: 4 blocks)
+  static constexpr int NI = TN == 128 ? 4 : TM / 64;           // 16-row blocks per consumer wave ...
+  static constexpr int NJ = TN == 96 ? 6 : 4;                  // ... and 16-column blocks
 };
 
-// s_waitcnt vmcnt(PER * n) for a uniform run-time n = stages that may stay in flight (PER = 6 or 8 DMA instructions per stage)
-#define SK_WAIT_CASE(k, c) case k: asm volatile("s_waitcnt vmcnt(" #c ")" ::: "memory"); break;
+// s_waitcnt vmcnt(PER * n) for a uniform run-time n = stages that may stay in flight (PER: DMA instructions per stage)
 template <int PER>
 __device__ __forceinline__ void sk_wait_stages(int n) {
-  if (PER == 6) {
-    switch (n) {
-      SK_WAIT_CASE(1, 6) SK_WAIT_CASE(2, 12) SK_WAIT_CASE(3, 18) SK_WAIT_CASE(4, 24)
-      default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-  } else if (PER == 4) {
-    switch (n) {
-      SK_WAIT_CASE(1, 4) SK_WAIT_CASE(2, 8) SK_WAIT_CASE(3, 12) SK_WAIT_CASE(4, 16)
-      default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-  } else {
-    static_assert(PER == 4 || PER == 6 || PER == 8, "");
-    switch (n) {
-      SK_WAIT_CASE(1, 8) SK_WAIT_CASE(2, 16) SK_WAIT_CASE(3, 24) SK_WAIT_CASE(4, 32)
-      default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
+  switch (n) {
+    case 1: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory"); break;
+    case 2: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER) : "memory"); break;
+    case 3: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * PER) : "memory"); break;
+    case 4: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * PER < 63 ? 4 * PER : 63) : "memory"); break;
+    default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
 }
 
@@ -86,7 +80,8 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
   static_assert(TM == SK_BM || EPI != P3V_EPI_QKV, "the qkv epilogue's V tiles are 128 dimensions tall");
   static_assert(!MERGE || (!PART && TN == 128), "merged slices: 128-column tiles");
   constexpr bool SILU = P3V_GATED(EPI);
-  constexpr int NS = C::NS, NI = C::NI;
+  constexpr int NS = C::NS, NI = C::NI, NJ = C::NJ;
+  static_assert(TN != 96 || (PART && !P3V_GATED(EPI)), "96-column tiles: plain partial sums");
   static_assert(NS - 2 <= 4 && (NS - 2) * C::PER < 64, "sk_wait_stages covers 4 stages in flight");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -190,12 +185,12 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
   }
 
   // ---- CONSUMERS: wave (wr, wc) owns NI x 16 rows from wr * NI * 16 and the 64 columns of group wc
-  const int wr = TN == 64 ? wave : wave >> 1, wc = TN == 64 ? 0 : wave & 1;
-  f32x4_t acc[NI][4];
+  const int wr = TN == 128 ? wave >> 1 : wave, wc = TN == 128 ? wave & 1 : 0;
+  f32x4_t acc[NI][NJ];
 #pragma unroll
   for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NJ; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   const int frow = lane & 15, fchunk = lane >> 4;
   {
     int slot = 0;
@@ -203,7 +198,7 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
       __builtin_amdgcn_s_barrier();                             // K-tile kt is in LDS (every producer waited for its pieces)
       const unsigned char* ta = smem + slot * C::STAGE;
       const unsigned char* tb = ta + C::A_BYTES;
-      bf16x8_t af[2][NI], bfr[2][4];
+      bf16x8_t af[2][NI], bfr[2][NJ];
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
 #pragma unroll
@@ -212,7 +207,7 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
           af[kk][i] = *(const bf16x8_t*)(ta + r * 128 + (((kk * 4 + fchunk) ^ (r & 7)) << 4));
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < NJ; ++j) {
           const int r = wc * 64 + j * 16 + frow;
           bfr[kk][j] = *(const bf16x8_t*)(tb + r * 128 + (((kk * 4 + fchunk) ^ (r & 7)) << 4));
         }
@@ -223,7 +218,7 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
 #pragma unroll
         for (int i = 0; i < NI; ++i)
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
+          for (int j = 0; j < NJ; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[kk][j], af[kk][i], acc[i][j], 0, 0, 0);   // W first: transposed block
       slot = slot == NS - 1 ? 0 : slot + 1;
     }
@@ -305,7 +300,7 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
     for (int i = 0; i < NI; ++i) {
       const int m = mrow0 + i * 16;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < NJ; ++j) {
         const int nn = SILU ? n0 + wc * 32 + (j & 1) * 16 + fq * 4 : n0 + wc * 64 + j * 16 + fq * 4;
         if (m < p.M && nn < p.N)
           *(float4*)(part + (size_t)m * ldp + nn + (SILU ? (j >> 1) * p.N : 0)) = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
@@ -387,24 +382,45 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
 // One workgroup per CU: the largest S <= 8 whose tiles * S still fit one round of the chip (slices of >= 6 K-tiles).
 extern "C" int p3v_gemm_rows_slices(int M, int N, int K, int epilogue);            // p3v_gemm_rows.hip: 9 .. 32 rows, weights straight to registers
 int p3v_gemm_rows_launch(const p3v_gemm_args_t* a, float* part, hipStream_t s);
+struct SkPlan { int S, tn; };
 static int sk_slices(int M, int N, int K, int epilogue);
 int p3v_gemm_skinny_slices(int M, int N, int K, int epilogue) {
   const int rs = p3v_gemm_rows_slices(M, N, K, epilogue);
   return rs ? rs : sk_slices(M, N, K, epilogue);
 }
-static int sk_slices(int M, int N, int K, int epilogue) {
+static SkPlan sk_plan(int M, int N, int K, int epilogue) {
   const P3vTuning& t = p3v_tuning();
   const bool silu = P3V_GATED(epilogue);
-  if (t.gemm_no_skinny || M <= 8 || M > t.gemm_skinny_max_m || K % SK_BK || N % (silu ? 32 : 64)) return 0;
-  if (epilogue != P3V_EPI_NONE && epilogue != P3V_EPI_RESID_BF16 && epilogue != P3V_EPI_SCALE_RESID_F32 && !silu) return 0;
-  const int tiles = p3v_cdiv(M, SK_BM) * ((silu ? 2 * N : N) / SK_TN);
-  if (t.gemm_skinny_s > 0) return K % (t.gemm_skinny_s * SK_BK) ? 1 : t.gemm_skinny_s;
-  int best = 1;
-  for (int S = 2; S <= 8; ++S)
-    if (K % (S * SK_BK) == 0 && K / S >= 6 * SK_BK && tiles * S <= t.gemm_splitk_wgs) best = S;
-  return best;
+  if (t.gemm_no_skinny || M <= 8 || M > t.gemm_skinny_max_m || K % SK_BK || N % (silu ? 32 : 64)) return {0, SK_TN};
+  if (epilogue != P3V_EPI_NONE && epilogue != P3V_EPI_RESID_BF16 && epilogue != P3V_EPI_SCALE_RESID_F32 && !silu) return {0, SK_TN};
+  const int mt = p3v_cdiv(M, SK_BM), tiles = mt * ((silu ? 2 * N : N) / SK_TN);
+  if (t.gemm_skinny_s > 0) return {K % (t.gemm_skinny_s * SK_BK) ? 1 : t.gemm_skinny_s, SK_TN};
+  auto slices = [&](int n) {
+    int best = 1;
+    for (int S = 2; S <= 8; ++S)
+      if (K % (S * SK_BK) == 0 && K / S >= 6 * SK_BK && n * S <= t.gemm_splitk_wgs) best = S;
+    return best;
+  };
+  const int S = slices(tiles);
+  if (S == 1 || silu || mt > 1 || N % 96) return {S, SK_TN};
+  const int S96 = slices(N / 96);
+  return S96 > 1 && N / 96 * S96 > tiles * S && K / S96 >= 12 * SK_BK ? SkPlan{S96, 96} : SkPlan{S, SK_TN};
 }
+static int sk_slices(int M, int N, int K, int epilogue) { return sk_plan(M, N, K, epilogue).S; }
 
+// 96-column tiles: plain partial sums
+template <int TM>
+static int launch_skinny96(const SkinnyP& p, int S, hipStream_t s) {
+  typedef SkCfg<96, TM> C;
+  static bool attr_set = false;
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)k_gemm_skinny<P3V_EPI_NONE, true, 96, TM>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS) != hipSuccess) return P3V_ERR_HIP;
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((k_gemm_skinny<P3V_EPI_NONE, true, 96, TM>), dim3(p.N / 96, p3v_cdiv(p.M, TM), S), dim3(512), C::LDS, s, p);
+  P3V_CHECK_LAUNCH();
+  return P3V_OK;
+}
 template <int EPI, int TM>
 static int launch_skinny_tm(const SkinnyP& p, int S, hipStream_t s) {
   typedef SkCfg<SK_TN, TM> C;
@@ -442,11 +458,13 @@ int p3v_gemm_skinny_partials(const p3v_gemm_args_t* a, int* S_out, hipStream_t s
     return p3v_gemm_rows_launch(a, (float*)a->ws, s);
   }
   if (RS == 1) return P3V_ERR_UNSUPPORTED;                       // (runs in one pass: no partials)
-  const int S = sk_slices(a->M, a->N, a->K, a->epilogue);
+  const SkPlan pl = sk_plan(a->M, a->N, a->K, a->epilogue);
+  const int S = pl.S;
   if (S <= 1 || !a->ws || a->ws_bytes < (int64_t)S * a->M * w_rows * 4) return P3V_ERR_UNSUPPORTED;
   if ((uintptr_t)a->ws & 15) return P3V_ERR_ARG;
   *S_out = S;
   const SkinnyP p = {a->A, a->W, a->ws, a->resid, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, a->col_scale, a->K / S, {}, nullptr, nullptr, 0, 0};
+  if (pl.tn == 96) return a->M <= 64 && !p3v_tuning().gemm_skinny_tm128 ? launch_skinny96<64>(p, S, s) : launch_skinny96<SK_BM>(p, S, s);
   if (silu) return launch_skinny<P3V_EPI_SILU_MUL>(p, S, s);                       // (partials: the activation is the reduction's)
   if (a->epilogue == P3V_EPI_RESID_BF16) return launch_skinny<P3V_EPI_RESID_BF16>(p, S, s);
   return launch_skinny<P3V_EPI_NONE>(p, S, s);

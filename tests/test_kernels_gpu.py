@@ -288,6 +288,32 @@ def test_gemm_resid_norm_is_the_two_calls(ops, M, N, K):
     assert bool((sentinel == 7.0).all())
 
 
+@pytest.mark.parametrize("M", [33, 64, 65, 127, 128])
+@pytest.mark.parametrize("N,K", [(3072, 8192), (2304, 8192), (3072, 6144)])
+def test_gemm_partials_on_96_columns(ops, M, N, K):
+    """Rows short of a full chip of 64-column tiles in K slices: 96-column tiles in eight slices, rows up to and across both tile heights,
+    neighbours of the output untouched.  Against fp64: the fp32 sums of eight slices (K products each within K 2^-24 of sum |a w|, far below the
+    bf16 result's half step 2^-9 of its value, twice where the residual sum rounds again); the two tile heights agree bit for bit."""
+    from phi_3_vision_mlx_amd import _lib
+    assert _lib.lib().p3v_gemm_ws_bytes(M, N, K, ops.EPI_RESID_BF16) == 8 * M * N * 4
+    a, w, r = g((M, K), 80).cuda(), g((N, K), 81, 1.0 / math.sqrt(K)).cuda(), g((M + 1, N), 82).cuda()
+    prod, mag = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    for epi in (ops.EPI_NONE, ops.EPI_RESID_BF16):
+        buf = torch.full((M + 1, N), 7.0, dtype=BF16, device="cuda")
+        kw = dict(resid=r[:M]) if epi == ops.EPI_RESID_BF16 else {}
+        ops.gemm(a, w, epi, out=buf[:M], **kw)
+        assert bool((buf[M] == 7.0).all())
+        ref = prod + r[:M].double() if kw else prod
+        tol = 2.0 ** -8 * ref.abs() + (2.0 ** -8 * prod.abs() if kw else 0) + K * 2.0 ** -24 * mag
+        assert bool(((buf[:M].double() - ref).abs() <= tol).all()), (buf[:M].double() - ref).abs().max()
+        if M <= 64:
+            old = ops.set_tuning("gemm_skinny_tm128", 1)
+            try:
+                assert torch.equal(ops.gemm(a, w, epi, **kw), buf[:M])
+            finally:
+                ops.set_tuning("gemm_skinny_tm128", old)
+
+
 @pytest.mark.parametrize("M,N,K,pin,kind", [(300, 3072, 8192, -1, "norm"), (200, 3072, 8192, -1, "norm"), (1023, 3072, 3072, -1, "norm"), (257, 384, 192, 343, "norm"),
                                             (129, 768, 448, 344, "norm"), (161, 256, 1024, 1654, "norm"), (1, 512, 704, 554, "norm"), (641, 1536, 320, 244, "norm"),
                                             (577, 1024, 4096, -1, "bias"), (2308, 1024, 4096, -1, "bias"), (33, 192, 256, 443, "bias"),
