@@ -107,6 +107,9 @@ int p3v_gemm(const p3v_gemm_args_t* args /* host */, void* stream);
 int p3v_gemm_plan(int M, int N, int K, int epilogue);
 int p3v_gemm_tile(int M, int N, int K, int epilogue);
 int64_t p3v_gemm_ws_bytes(int M, int N, int K, int epilogue);
+/* p3v_gemm, p3v_gemm_resid_norm: the largest workspace that either makes use of, never below p3v_gemm_ws_bytes.  Where it is above (33 .. 128 rows, a
+ * long K, few columns), a workspace of this size has the shape run in more slices: faster, the same results up to fp32 summation order. */
+int64_t p3v_gemm_ws_most_bytes(int M, int N, int K, int epilogue);
 /* 9 .. 32 rows of A on bf16 weights with K = 3072 or 8192 (a 9 .. 32-sequence decode batch; the reference's batched benchmark
  * runs 15, phi_3_vision_mlx.py:1226-1243) take a register-streaming kernel inside p3v_gemm / p3v_gemm_resid_norm (weights HBM ->
  * registers in whole lines, A resident as MFMA fragments): this query says how -- 0 = not that kernel's shape, 1 = one pass,

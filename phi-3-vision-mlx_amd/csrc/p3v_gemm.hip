@@ -581,6 +581,12 @@ extern "C" int64_t p3v_gemm_ws_bytes(int M, int N, int K, int epilogue) {
   if (S == 1) return 0;
   return (int64_t)S * M * (P3V_GATED(epilogue) ? 2 * N : N) * 4;
 }
+int p3v_gemm_skinny_most_slices(int M, int N, int K, int epilogue);   // p3v_gemm_skinny.hip: with a workspace for its 96-column tiles
+extern "C" int64_t p3v_gemm_ws_most_bytes(int M, int N, int K, int epilogue) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const int sk = p3v_gemm_skinny_most_slices(M, N, K, epilogue);
+  return sk > 1 ? (int64_t)sk * M * (P3V_GATED(epilogue) ? 2 * N : N) * 4 : p3v_gemm_ws_bytes(M, N, K, epilogue);
+}
 
 // ---- out = resid + bf16(A W^T) and normed = RMSNorm(out) (include/p3v.h): only where the projection runs as K slices anyway
 int p3v_gemm_skinny_partials(const p3v_gemm_args_t* a, int* S_out, hipStream_t s);   // p3v_gemm_skinny.hip

@@ -383,12 +383,14 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
 extern "C" int p3v_gemm_rows_slices(int M, int N, int K, int epilogue);            // p3v_gemm_rows.hip: 9 .. 32 rows, weights straight to registers
 int p3v_gemm_rows_launch(const p3v_gemm_args_t* a, float* part, hipStream_t s);
 struct SkPlan { int S, tn; };
-static int sk_slices(int M, int N, int K, int epilogue);
+static SkPlan sk_plan(int M, int N, int K, int epilogue, bool wide);
+static int sk_slices(int M, int N, int K, int epilogue) { return sk_plan(M, N, K, epilogue, false).S; }
 int p3v_gemm_skinny_slices(int M, int N, int K, int epilogue) {
   const int rs = p3v_gemm_rows_slices(M, N, K, epilogue);
   return rs ? rs : sk_slices(M, N, K, epilogue);
 }
-static SkPlan sk_plan(int M, int N, int K, int epilogue) {
+// wide: whether the caller's workspace holds the partials of 96-column tiles too (p3v_gemm_ws_most_bytes)
+static SkPlan sk_plan(int M, int N, int K, int epilogue, bool wide) {
   const P3vTuning& t = p3v_tuning();
   const bool silu = P3V_GATED(epilogue);
   if (t.gemm_no_skinny || M <= 8 || M > t.gemm_skinny_max_m || K % SK_BK || N % (silu ? 32 : 64)) return {0, SK_TN};
@@ -402,11 +404,14 @@ static SkPlan sk_plan(int M, int N, int K, int epilogue) {
     return best;
   };
   const int S = slices(tiles);
-  if (S == 1 || silu || mt > 1 || N % 96) return {S, SK_TN};
+  if (!wide || S == 1 || silu || mt > 1 || N % 96) return {S, SK_TN};
   const int S96 = slices(N / 96);
   return S96 > 1 && N / 96 * S96 > tiles * S && K / S96 >= 12 * SK_BK ? SkPlan{S96, 96} : SkPlan{S, SK_TN};
 }
-static int sk_slices(int M, int N, int K, int epilogue) { return sk_plan(M, N, K, epilogue).S; }
+int p3v_gemm_skinny_most_slices(int M, int N, int K, int epilogue) {
+  const int rs = p3v_gemm_rows_slices(M, N, K, epilogue);
+  return rs ? rs : sk_plan(M, N, K, epilogue, true).S;
+}
 
 // 96-column tiles: plain partial sums
 template <int TM>
@@ -458,7 +463,8 @@ int p3v_gemm_skinny_partials(const p3v_gemm_args_t* a, int* S_out, hipStream_t s
     return p3v_gemm_rows_launch(a, (float*)a->ws, s);
   }
   if (RS == 1) return P3V_ERR_UNSUPPORTED;                       // (runs in one pass: no partials)
-  const SkPlan pl = sk_plan(a->M, a->N, a->K, a->epilogue);
+  SkPlan pl = sk_plan(a->M, a->N, a->K, a->epilogue, true);
+  if (pl.tn == 96 && a->ws_bytes < (int64_t)pl.S * a->M * w_rows * 4) pl = sk_plan(a->M, a->N, a->K, a->epilogue, false);
   const int S = pl.S;
   if (S <= 1 || !a->ws || a->ws_bytes < (int64_t)S * a->M * w_rows * 4) return P3V_ERR_UNSUPPORTED;
   if ((uintptr_t)a->ws & 15) return P3V_ERR_ARG;

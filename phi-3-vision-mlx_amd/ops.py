@@ -192,7 +192,7 @@ def gemm(a, w, epilogue=EPI_NONE, bias=None, resid=None, out=None, n_out=None, p
     f32_out = epilogue in (EPI_BIAS_RESID_F32, EPI_PATCH, EPI_F32, EPI_SCALE_RESID_F32)
     if out is None:
         out = torch.empty((M, N), dtype=F32 if f32_out else BF16, device=a.device)
-    ws_bytes = L.lib().p3v_gemm_ws_bytes(M, N, K, epilogue)
+    ws_bytes = L.lib().p3v_gemm_ws_most_bytes(M, N, K, epilogue)
     ws = _gemm_workspace(a.device, ws_bytes) if ws_bytes else None
     args = L.GemmArgs(_p(a), _p(w), _p(out), _p(bias), _p(resid), _p(pos), M, N, K, a.stride(0), w.stride(0),
                       ldo if ldo is not None else N, epilogue, patches_per_img, _p(ws), ws.numel() if ws is not None else 0, _p(col_scale))
@@ -211,7 +211,7 @@ def gemm_resid_norm(a, w, resid, norm_w, eps, normed, out=None):
         raise ValueError(f"gemm_resid_norm: shapes {a.shape} x {w.shape}, resid {resid.shape}, normed {normed.shape}")
     if out is None:
         out = torch.empty((M, N), dtype=BF16, device=a.device)
-    ws_bytes = L.lib().p3v_gemm_ws_bytes(M, N, K, EPI_RESID_BF16)
+    ws_bytes = L.lib().p3v_gemm_ws_most_bytes(M, N, K, EPI_RESID_BF16)
     if not ws_bytes:
         return False
     ws = _gemm_workspace(a.device, ws_bytes)
@@ -974,7 +974,7 @@ def latent_ws_bytes(m, B, Lq, n_split):
 
 def _gemm_rows(a, w, out, M, N, K, lda, ldw):
     """out[M, N] = a w^T of raw row pointers (bf16), rows of a and w lda / ldw elements apart."""
-    ws_bytes = L.lib().p3v_gemm_ws_bytes(M, N, K, EPI_NONE)
+    ws_bytes = L.lib().p3v_gemm_ws_most_bytes(M, N, K, EPI_NONE)
     ws = _gemm_workspace(out.device, ws_bytes) if ws_bytes else None
     args = L.GemmArgs(a, w, _p(out), 0, 0, 0, M, N, K, lda, ldw, N, EPI_NONE, 0, _p(ws), ws.numel() if ws is not None else 0, 0)
     L.check(L.lib().p3v_gemm(C.byref(args), _stream()), "gemm")

@@ -295,7 +295,7 @@ def test_gemm_partials_on_96_columns(ops, M, N, K):
     neighbours of the output untouched.  Against fp64: the fp32 sums of eight slices (K products each within K 2^-24 of sum |a w|, far below the
     bf16 result's half step 2^-9 of its value, twice where the residual sum rounds again); the two tile heights agree bit for bit."""
     from phi_3_vision_mlx_amd import _lib
-    assert _lib.lib().p3v_gemm_ws_bytes(M, N, K, ops.EPI_RESID_BF16) == 8 * M * N * 4
+    assert _lib.lib().p3v_gemm_ws_most_bytes(M, N, K, ops.EPI_RESID_BF16) == 8 * M * N * 4 > _lib.lib().p3v_gemm_ws_bytes(M, N, K, ops.EPI_RESID_BF16) > 0
     a, w, r = g((M, K), 80).cuda(), g((N, K), 81, 1.0 / math.sqrt(K)).cuda(), g((M + 1, N), 82).cuda()
     prod, mag = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
     for epi in (ops.EPI_NONE, ops.EPI_RESID_BF16):
