@@ -110,6 +110,8 @@ int64_t p3v_gemm_ws_bytes(int M, int N, int K, int epilogue);
 /* p3v_gemm, p3v_gemm_resid_norm: the largest workspace that either makes use of, never below p3v_gemm_ws_bytes.  Where it is above (33 .. 128 rows, a
  * long K, few columns), a workspace of this size has the shape run in more slices: faster, the same results up to fp32 summation order. */
 int64_t p3v_gemm_ws_most_bytes(int M, int N, int K, int epilogue);
+/* 1: p3v_gemm is faster without the workspace of p3v_gemm_ws_bytes (257 .. 384 rows whose 128 x 128 tiles fill one round of the chip) */
+int p3v_gemm_one_pass_pays(int M, int N, int K, int epilogue);
 /* 9 .. 32 rows of A on bf16 weights with K = 3072 or 8192 (a 9 .. 32-sequence decode batch; the reference's batched benchmark
  * runs 15, phi_3_vision_mlx.py:1226-1243) take a register-streaming kernel inside p3v_gemm / p3v_gemm_resid_norm (weights HBM ->
  * registers in whole lines, A resident as MFMA fragments): this query says how -- 0 = not that kernel's shape, 1 = one pass,
@@ -234,6 +236,8 @@ typedef struct {
   float q_scale;
 } p3v_qkv_split_t;
 int p3v_gemm_qkv(const p3v_gemm_args_t* gemm /* host */, const p3v_qkv_split_t* split /* host */, void* stream);
+/* the same where p3v_gemm_one_pass_pays: p3v_gemm without a workspace + p3v_rope_kv_append, bit for bit, in one launch (P3V_ERR_UNSUPPORTED elsewhere) */
+int p3v_gemm_qkv_one_pass(const p3v_gemm_args_t* gemm /* host */, const p3v_qkv_split_t* split /* host */, void* stream);
 /* The tile p3v_gemm_qkv runs on more than 256 rows (host query; n_q, n_kv: rows of W per region): mb for 32 mb rows x 256 columns, 1: 128 x 128, the value that the knob
  * "gemm_qkv_flat" pins it with; 0: one of the kernels for few rows, 128 x 128 tiles of regions that are no whole 256 columns, or P3V_ERR_UNSUPPORTED */
 int p3v_gemm_qkv_tile(int M, int n_q, int n_kv, int K);

@@ -130,6 +130,7 @@ SIGNATURES = {
     "p3v_gemm": (i32, [C.POINTER(GemmArgs), vp]),
     "p3v_gemm_ws_bytes": (i64, [i32, i32, i32, i32]),
     "p3v_gemm_ws_most_bytes": (i64, [i32, i32, i32, i32]),
+    "p3v_gemm_one_pass_pays": (i32, [i32, i32, i32, i32]),
     "p3v_gemm_rows_slices": (i32, [i32, i32, i32, i32]),
     "p3v_gemv": (i32, [C.POINTER(GemvArgs), vp]),
     "p3v_gemv_step": (i32, [C.POINTER(GemvArgs), C.POINTER(GemvStep), vp]),
@@ -149,6 +150,7 @@ SIGNATURES = {
     "p3v_kv_quantize": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]),
     "p3v_kv_dequantize": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]),
     "p3v_gemm_qkv": (i32, [vp, vp, vp]),
+    "p3v_gemm_qkv_one_pass": (i32, [vp, vp, vp]),
     "p3v_gemm_qkv_merge": (i32, [vp, vp, vp, i64, vp]),
     "p3v_gemm_merge": (i32, [C.POINTER(GemmArgs), vp, i64, vp]),
     "p3v_gemm_merge_ws_bytes": (i64, [i32, i32, i32, i32, i32]),

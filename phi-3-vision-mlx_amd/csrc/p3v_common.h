@@ -215,7 +215,7 @@ struct P3vTuning {
   int gemm_tile;            // 10 mb + nb: pin the tile of the large GEMM (32 mb x 64 nb); -1: cost model
   int gemm_no_splitk, gemm_splitk_max_m, gemm_splitk_max_s, gemm_splitk_wgs, gemm_128, gemm_persistent;
   int gemm_rows;            // 1: 9 .. 32 rows on the register-streaming kernel (p3v_gemm_rows.hip), 0: on the 64-row tiles of p3v_gemm_skinny.hip
-  int gemm_no_skinny, gemm_skinny_max_m, gemm_skinny_s, gemm_skinny_tm128, gemm_no_merge;   // the 128 x 64-tile weight-streaming kernel for 17 .. max_m rows (p3v_gemm_skinny.hip)
+  int gemm_no_skinny, gemm_skinny_max_m, gemm_skinny_s, gemm_skinny_tm128, gemm_skinny_tn, gemm_no_merge;   // the 128 x 64-tile weight-streaming kernel for 17 .. max_m rows (p3v_gemm_skinny.hip)
   int gemm_merge_polls;     // p3v_gemm_merge, p3v_gemm_qkv_merge: looks at a counter before a wait is given up; -1: 2^22 (seconds); tests: 0
   int gemm_slices;          // p3v_gemm_slices: -1: by shape, 0: never, 100 S + 10 mb + nb: S slices of K on tiles of 32 mb x 64 nb
   int gemm_qkv_flat;        // p3v_gemm_qkv on tiles of 32 x gemm_qkv_flat rows (2 .. 8; 1: 128 x 128): -1: by shape, 0: by the kernels for few rows or 128 x 128 tiles

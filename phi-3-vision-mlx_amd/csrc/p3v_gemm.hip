@@ -572,7 +572,10 @@ static int splitk_slices(int M, int N, int K, int epilogue) {
   return S;
 }
 
+int p3v_splitk_slices(int M, int N, int K, int epilogue) { return splitk_slices(M, N, K, epilogue); }
+
 int p3v_gemm_skinny_try(const p3v_gemm_args_t* a, hipStream_t s);
+int p3v_gemm_skinny_tall(const p3v_gemm_args_t* a, hipStream_t s);
 
 extern "C" int64_t p3v_gemm_ws_bytes(int M, int N, int K, int epilogue) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
@@ -730,7 +733,8 @@ extern "C" int p3v_gemm(const p3v_gemm_args_t* a, void* stream) {
     if (rc != P3V_ERR_UNSUPPORTED) return rc;
   }
   {
-    const int rc = gemm_splitk(a, s);
+    int rc = gemm_splitk(a, s);
+    if (rc == P3V_ERR_UNSUPPORTED) rc = p3v_gemm_skinny_tall(a, s);
     if (rc != P3V_ERR_UNSUPPORTED) return rc;
   }
   const bool big_tiles = !p3v_tuning().gemm_128;
@@ -778,7 +782,7 @@ static int gemm128(const p3v_gemm_args_t* a, hipStream_t s) {
 }
 
 // ---- the qkv projection with the head split, the rotation and the KV append in its epilogue (p3v_gemm_qkv.h)
-int p3v_gemm_skinny_qkv(const p3v_gemm_args_t* a, const QkvP& q, hipStream_t s);   // p3v_gemm_skinny.hip
+int p3v_gemm_skinny_qkv(const p3v_gemm_args_t* a, const QkvP& q, bool tall, hipStream_t s);   // p3v_gemm_skinny.hip
 
 int p3v_gemm_skinny_qkv_merge(const p3v_gemm_args_t* a, const QkvP& q, void* ws, int64_t ws_bytes, hipStream_t s);   // p3v_gemm_skinny.hip
 int p3v_qkv_flat_tiles(const QkvP& q, int M, int mb);                                        // p3v_gemm_pc.hip
@@ -834,7 +838,7 @@ extern "C" int p3v_gemm_qkv_tile(int M, int n_q, int n_kv, int K) {
   return qkv_tile_plan(&a, q);
 }
 
-static int gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* merge_ws, int64_t merge_bytes, void* stream) {
+static int gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* merge_ws, int64_t merge_bytes, bool tall, void* stream) {
   if (!a || !sp || !a->A || !a->W || !sp->q_out || !sp->k_dst || !sp->v_dst || (!sp->cos_t) != (!sp->sin_t)) return P3V_ERR_ARG;
   if (a->epilogue != P3V_EPI_NONE && a->epilogue != P3V_EPI_BIAS) return P3V_ERR_ARG;
   if (a->epilogue == P3V_EPI_BIAS && !a->bias) return P3V_ERR_ARG;
@@ -854,14 +858,16 @@ static int gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* m
   QkvP q = {sp->cos_t, sp->sin_t, sp->q_out, sp->k_dst, sp->v_dst, sp->L, nh, nkv, hd, sp->past, dpos0, sp->dst_t, sp->tab_t, sp->tab_div,
             sp->q_scale};
   if (merge_ws) return p3v_gemm_skinny_qkv_merge(a, q, merge_ws, merge_bytes, s);
+  if (tall) return p3v_gemm_skinny_qkv(a, q, true, s);
   const int mb = qkv_tile_plan(a, q);
   if (mb > 1) return p3v_gemm256_flat_qkv(a, q, mb, s);
-  if (!mb && a->M < 1024) return p3v_gemm_skinny_qkv(a, q, s);  // 17 .. 256 rows: the weight-streaming kernel (or "unsupported")
+  if (!mb && a->M < 1024) return p3v_gemm_skinny_qkv(a, q, false, s);  // 17 .. 256 rows: the weight-streaming kernel (or "unsupported")
   if ((nh * hd) % BN || (nkv * hd) % BN || p3v_tuning().gemm_128) return P3V_ERR_UNSUPPORTED;
   const GemmP p = {a->A, a->W, nullptr, a->bias, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0, 0, 0, q};
   return launch_gemm<P3V_EPI_QKV>(p, s);
 }
-extern "C" int p3v_gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* stream) { return gemm_qkv(a, sp, nullptr, 0, stream); }
+extern "C" int p3v_gemm_qkv(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* stream) { return gemm_qkv(a, sp, nullptr, 0, false, stream); }
+extern "C" int p3v_gemm_qkv_one_pass(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* stream) { return gemm_qkv(a, sp, nullptr, 0, true, stream); }
 extern "C" int p3v_gemm_qkv_merge(const p3v_gemm_args_t* a, const p3v_qkv_split_t* sp, void* ws, int64_t ws_bytes, void* stream) {
-  return ws ? gemm_qkv(a, sp, ws, ws_bytes, stream) : P3V_ERR_ARG;
+  return ws ? gemm_qkv(a, sp, ws, ws_bytes, false, stream) : P3V_ERR_ARG;
 }

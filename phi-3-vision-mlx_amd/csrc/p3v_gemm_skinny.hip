@@ -9,12 +9,17 @@
 //             HBM, and in one CU the two add up -- the same requests without any compute take as long as gate_up, 30 us at 128
 //             rows (rows 6144 bytes apart; weights alone 18.5, both packed 25.9: profiles/lds_dma_probe.txt).  Rows of A and W 128 bytes further apart: gate_up 30.2 ->
 //             27.7, qkv 26 -> 24.3, but down 22.6 -> 25.4; the weights lie unpadded, as the other kernels and the loader have them.
-//             128 x 128 tiles (W x 2 staged, half the workgroups) in one pass or with partials in memory were not faster on any shape; where
-//             the K slices that fill the chip again are summed inside the launch they are (p3v_gemm_merge, at the end).
-//             Plain partials of a long K: 128 x 96 tiles in 8 slices where that is a workgroup for more CUs than 64 columns reach (3072 columns:
-//             256 against 192), each of which then asks for less (448 against 768 KB of 8192; the requests alone 16.5 -> 11.5 us).  With the
-//             reduction, 3072 x 8192: 128 rows 24.2 -> 21.8 us, 64 rows 19.9 -> 17.3, 40 rows 18.4 -> 16.3; x 6144 (12 K-tiles a slice) 21.6 -> 20.4;
-//             x 3072 would have 6 K-tiles a slice: 15.5 -> 16.6, so slices of fewer than 12 stay on 64 columns.
+//             128 x 128 tiles (W x 2 staged, half the workgroups) in one pass are not faster up to 128 rows; where the K slices that fill the
+//             chip again are summed inside the launch they are (p3v_gemm_merge, at the end).  Beyond 128 rows they are wherever 64 columns take two
+//             rounds of the chip and 128 one: gate_up of 129 / 192 / 256 rows 45.5 -> 30.4, 44.5 -> 32.6, 45.3 -> 36.2 us, qkv 34.7 -> 27.2, 35.9 -> 30.9,
+//             40.4 -> 36.2 (6144 columns, one round either way: 18.2 against 23.3).  257 .. 384 rows whose tiles are more than half a round and no more than
+//             one (sk_tall): 9216 x 3072 37.6 -> 25.6 at 266, 41.2 -> 33.0 at 384, qkv 42.3 -> 28.1, 46.6 -> 35.8 (slices of K before); gated ones would
+//             take two rounds (44.7 against 54.6).
+//             Plain partials of a long K: 128 x 96 tiles in up to 8 slices where that is a workgroup for more CUs than 64 columns reach (3072 columns:
+//             256 against 192), each of which then asks for less (448 against 768 KB of 8192 at 128 rows; the requests alone 16.5 -> 11.5 us).  With the
+//             reduction, 3072 x 8192: 128 rows 24.2 -> 21.8 us, 64 rows 19.9 -> 17.3, 40 rows 18.4 -> 16.3, 160 rows 28.5 -> 23.3, 200 30.3 -> 24.9, 256 34.7 ->
+//             28.0 (four slices); x 6144 at 100 rows (12 K-tiles a slice) 19.8 -> 18.0, at 200 25.3 -> 21.8; x 4096 at 200 (16) 19.0 -> 17.3; x 3072 would have 6
+//             K-tiles a slice up to 128 rows (15.5 -> 16.6) and 12 beyond (15.4 -> 15.8): slices of fewer than 12 and 16 stay on 64 columns.
 //   staging   LDS-DMA into a ring of 6 stages (A 16 KiB + W 8 KiB each), 5 in flight behind a counted vmcnt; one workgroup per CU
 //             (<= 64 rows: 64-row tiles, A 8 KiB per stage -- a third less staged per K-tile, the same sums bit for bit: 60 -> 53 us
 //             per decoder layer at 17 rows)
@@ -30,7 +35,7 @@
 
 #define SK_BM 128
 #define SK_BK 64
-#define SK_TN 64                    // tile width of the one-pass form and of most partial-sum forms (else 96, see sk_plan; MERGE: 128)
+#define SK_TN 64                    // tile width, but 96 for partial sums of a long K (sk_plan), 128 for MERGE and one pass of many rows (sk_one_pass_tn, sk_tall)
 #ifndef SK_ABL
 #define SK_ABL 0                    // timing experiments: 1 = A always K-tile 0 (one L2/L1-hot tile), 2 = W likewise, 3 = no MFMAs after K-tile 0
 #endif
@@ -382,13 +387,29 @@ __global__ void __launch_bounds__(512, 1) k_gemm_skinny(SkinnyP p) {
 // One workgroup per CU: the largest S <= 8 whose tiles * S still fit one round of the chip (slices of >= 6 K-tiles).
 extern "C" int p3v_gemm_rows_slices(int M, int N, int K, int epilogue);            // p3v_gemm_rows.hip: 9 .. 32 rows, weights straight to registers
 int p3v_gemm_rows_launch(const p3v_gemm_args_t* a, float* part, hipStream_t s);
-struct SkPlan { int S, tn; };
+struct SkPlan { int S, tn; };                                     // slices, tile columns
 static SkPlan sk_plan(int M, int N, int K, int epilogue, bool wide);
 static int sk_slices(int M, int N, int K, int epilogue) { return sk_plan(M, N, K, epilogue, false).S; }
 int p3v_gemm_skinny_slices(int M, int N, int K, int epilogue) {
   const int rs = p3v_gemm_rows_slices(M, N, K, epilogue);
   return rs ? rs : sk_slices(M, N, K, epilogue);
 }
+// Columns of a one-pass tile: rounds of the chip times what a K-tile asks for, 32 KB on 128 columns and 24 on 64 (the header's figures)
+static int sk_one_pass_tn(int M, int rows) {
+  const int pin = p3v_tuning().gemm_skinny_tn, mt = p3v_cdiv(M, SK_BM);
+  if (M <= 64 || rows % 128) return SK_TN;
+  if (pin > 0) return pin == 128 ? 128 : SK_TN;
+  return p3v_cdiv(mt * (rows / 128), 256) * 4 < p3v_cdiv(mt * (rows / 64), 256) * 3 ? 128 : SK_TN;
+}
+// Rows beyond the knob's: one round of 128 x 128 tiles in one pass, where p3v_gemm would run slices of K through a workspace
+int p3v_splitk_slices(int M, int N, int K, int epilogue);            // p3v_gemm.hip
+static bool sk_tall(int M, int N, int K, int epilogue) {
+  const P3vTuning& t = p3v_tuning();
+  if (t.gemm_no_skinny || t.gemm_skinny_tn == SK_TN || M <= t.gemm_skinny_max_m || M > 3 * SK_BM || epilogue != P3V_EPI_NONE || N % 128 || K % SK_BK) return false;
+  const int tiles = p3v_cdiv(M, SK_BM) * (N / 128);
+  return tiles > 128 && tiles <= 256 && p3v_splitk_slices(M, N, K, epilogue) > 1;
+}
+extern "C" int p3v_gemm_one_pass_pays(int M, int N, int K, int epilogue) { return M > 0 && N > 0 && K > 0 && sk_tall(M, N, K, epilogue); }
 // wide: whether the caller's workspace holds the partials of 96-column tiles too (p3v_gemm_ws_most_bytes)
 static SkPlan sk_plan(int M, int N, int K, int epilogue, bool wide) {
   const P3vTuning& t = p3v_tuning();
@@ -404,9 +425,10 @@ static SkPlan sk_plan(int M, int N, int K, int epilogue, bool wide) {
     return best;
   };
   const int S = slices(tiles);
-  if (!wide || S == 1 || silu || mt > 1 || N % 96) return {S, SK_TN};
-  const int S96 = slices(N / 96);
-  return S96 > 1 && N / 96 * S96 > tiles * S && K / S96 >= 12 * SK_BK ? SkPlan{S96, 96} : SkPlan{S, SK_TN};
+  if (S == 1) return {1, sk_one_pass_tn(M, silu ? 2 * N : N)};
+  if (!wide || silu || N % 96 || t.gemm_skinny_tn == SK_TN) return {S, SK_TN};
+  const int tiles96 = mt * (N / 96), S96 = slices(tiles96);
+  return S96 > 1 && tiles96 * S96 > tiles * S && K / S96 >= (mt > 1 ? 16 : 12) * SK_BK ? SkPlan{S96, 96} : SkPlan{S, SK_TN};
 }
 int p3v_gemm_skinny_most_slices(int M, int N, int K, int epilogue) {
   const int rs = p3v_gemm_rows_slices(M, N, K, epilogue);
@@ -423,6 +445,18 @@ static int launch_skinny96(const SkinnyP& p, int S, hipStream_t s) {
     attr_set = true;
   }
   hipLaunchKernelGGL((k_gemm_skinny<P3V_EPI_NONE, true, 96, TM>), dim3(p.N / 96, p3v_cdiv(p.M, TM), S), dim3(512), C::LDS, s, p);
+  P3V_CHECK_LAUNCH();
+  return P3V_OK;
+}
+// 128-column tiles in one pass
+template <int EPI>
+static int launch_skinny128(const SkinnyP& p, int grid_x, int grid_y, hipStream_t s) {
+  static bool attr_set = false;
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)k_gemm_skinny<EPI, false, 128>, hipFuncAttributeMaxDynamicSharedMemorySize, SkCfg<128>::LDS) != hipSuccess) return P3V_ERR_HIP;
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((k_gemm_skinny<EPI, false, 128>), dim3(grid_x, grid_y), dim3(512), SkCfg<128>::LDS, s, p);
   P3V_CHECK_LAUNCH();
   return P3V_OK;
 }
@@ -446,6 +480,7 @@ static int launch_skinny_tm(const SkinnyP& p, int S, hipStream_t s) {
 // <= 64 rows: 64-row tiles (the A panel is two thirds of what a 128-row tile stages per K-tile; half of it would be clamped copies)
 template <int EPI>
 static int launch_skinny(const SkinnyP& p, int S, hipStream_t s) {
+  if (const int rows = P3V_GATED(EPI) ? 2 * p.N : p.N; S == 1 && sk_one_pass_tn(p.M, rows) == 128) return launch_skinny128<EPI>(p, rows / 128, p3v_cdiv(p.M, SK_BM), s);
   return p.M <= 64 && !p3v_tuning().gemm_skinny_tm128 ? launch_skinny_tm<EPI, 64>(p, S, s) : launch_skinny_tm<EPI, SK_BM>(p, S, s);
 }
 
@@ -497,20 +532,30 @@ int p3v_gemm_skinny_try(const p3v_gemm_args_t* a, hipStream_t s) {
   return launch_skinny<P3V_EPI_NONE>(p, 1, s);
 }
 
+// p3v_gemm without the workspace of its slices
+int p3v_gemm_skinny_tall(const p3v_gemm_args_t* a, hipStream_t s) {
+  if (a->bias || !sk_tall(a->M, a->N, a->K, a->epilogue)) return P3V_ERR_UNSUPPORTED;
+  const SkinnyP p = {a->A, a->W, a->out, a->resid, a->M, a->N, a->K, a->lda, a->ldw, a->ldo, a->col_scale, 0, {}, nullptr, nullptr, 0, 0};
+  return launch_skinny128<P3V_EPI_NONE>(p, a->N / 128, p3v_cdiv(a->M, SK_BM), s);
+}
+
 // ---- the qkv projection of a short prompt with the head split, the rotation and the KV append in the epilogue (p3v_gemm_qkv's
 // 17 .. 256-row case): one pass (the epilogue needs whole sums), Q / K tiles + V tiles in a one-dimensional grid.
 // P3V_ERR_UNSUPPORTED (nothing launched) where the shape is not this kernel's.
-int p3v_gemm_skinny_qkv(const p3v_gemm_args_t* a, const QkvP& q, hipStream_t s) {
+int p3v_gemm_skinny_qkv(const p3v_gemm_args_t* a, const QkvP& q, bool tall, hipStream_t s) {
   const P3vTuning& t = p3v_tuning();
-  if (t.gemm_no_skinny || a->M <= 8 || a->M > t.gemm_skinny_max_m || a->K % SK_BK || a->bias) return P3V_ERR_UNSUPPORTED;
+  if (tall && (!sk_tall(a->M, a->N, a->K, P3V_EPI_NONE) || (q.nh * q.hd) % 128 || (q.nkv * q.hd) % 128)) return P3V_ERR_UNSUPPORTED;
+  if (t.gemm_no_skinny || a->M <= 8 || (a->M > t.gemm_skinny_max_m && !tall) || a->K % SK_BK || a->bias) return P3V_ERR_UNSUPPORTED;
   if ((q.nh * q.hd) % 64 || (q.nkv * q.hd) % SK_BM) return P3V_ERR_UNSUPPORTED;   // whole Q / K tiles of 32 pairs, whole V tiles of 128 dims
+  const SkinnyP p = {a->A, a->W, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0, nullptr, 0, q, nullptr, nullptr, 0, 0};
+  if ((q.nh * q.hd) % 128 == 0 && (q.nkv * q.hd) % 128 == 0 && (tall || sk_one_pass_tn(a->M, a->N) == 128))
+    return launch_skinny128<P3V_EPI_QKV>(p, a->N / 128 * p3v_cdiv(a->M, SK_BM), 1, s);
   static bool attr_set = false;
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)k_gemm_skinny<P3V_EPI_QKV, false, SK_TN>, hipFuncAttributeMaxDynamicSharedMemorySize, SkCfg<SK_TN>::LDS) != hipSuccess)
       return P3V_ERR_HIP;
     attr_set = true;
   }
-  const SkinnyP p = {a->A, a->W, nullptr, nullptr, a->M, a->N, a->K, a->lda, a->ldw, 0, nullptr, 0, q, nullptr, nullptr, 0, 0};
   const int mt = p3v_cdiv(a->M, SK_BM), tiles = ((q.nh + q.nkv) * q.hd / 64) * mt + (q.nkv * q.hd / SK_BM) * p3v_cdiv(a->M, 64);
   hipLaunchKernelGGL((k_gemm_skinny<P3V_EPI_QKV, false, SK_TN>), dim3(tiles), dim3(512), SkCfg<SK_TN>::LDS, s, p);
   P3V_CHECK_LAUNCH();

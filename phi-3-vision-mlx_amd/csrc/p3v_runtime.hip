@@ -45,6 +45,7 @@ const Knob kKnobs[] = {
     {"gemv_q4_rows8", &P3vTuning::gemv_q4_rows8, 1},
     {"gemm_no_skinny", &P3vTuning::gemm_no_skinny, 0},      {"gemm_skinny_max_m", &P3vTuning::gemm_skinny_max_m, 256},
     {"gemm_skinny_s", &P3vTuning::gemm_skinny_s, 0},            {"gemm_skinny_tm128", &P3vTuning::gemm_skinny_tm128, 0},
+    {"gemm_skinny_tn", &P3vTuning::gemm_skinny_tn, 0},
     {"gemm_no_merge", &P3vTuning::gemm_no_merge, 0},        {"gemm_slices", &P3vTuning::gemm_slices, -1},
     {"gemm_merge_polls", &P3vTuning::gemm_merge_polls, -1}, {"gemm_qkv_flat", &P3vTuning::gemm_qkv_flat, -1},
     {"gemm_rows", &P3vTuning::gemm_rows, 1},              {"gemm_tile", &P3vTuning::gemm_tile, -1},

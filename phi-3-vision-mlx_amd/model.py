@@ -172,9 +172,10 @@ class Phi3VModel(DecoderModel):
             x = ops.rmsnorm(x, norm_w, eps, out=h)
         if epilogue == EPI_SILU_MUL and 104 < M <= 128 and out is not None and not self.serving and ops.gemm_merge(x, w, epilogue, out):
             return out
-        if epilogue == EPI_RESID_BF16 and out is not None and ops.gemm_slices(x, w, epilogue, resid, out):
+        if (epilogue == EPI_RESID_BF16 and out is not None and not ops.gemm_few_rows(M, w.shape[0], K, epilogue)
+                and ops.gemm_slices(x, w, epilogue, resid, out)):
             return out
-        return ops.gemm(x, w, epilogue, resid=resid, out=out)
+        return ops.gemm(x, w, epilogue, resid=resid, out=out, slices="most")
 
     def _proj_resid_norm(self, o, key, x, norm_w, h):
         """x += bf16(o @ W^T) and h = RMSNorm(x) * norm_w from the projection's own launches (ops.gemm_slices, ops.gemm_resid_norm); False -- nothing
@@ -184,7 +185,8 @@ class Phi3VModel(DecoderModel):
                 or os.environ.get("P3V_RESID_NORM_FUSE", "1") == "0"):
             return False
         w, eps = self.w[key], self.cfg.rms_norm_eps
-        return ops.gemm_slices(o, w, EPI_RESID_BF16, x, x, norm=(norm_w, eps, h[:M])) or ops.gemm_resid_norm(o, w, x, norm_w, eps, h[:M], out=x)
+        return (not ops.gemm_few_rows(M, w.shape[0], o.shape[1], EPI_RESID_BF16) and ops.gemm_slices(o, w, EPI_RESID_BF16, x, x, norm=(norm_w, eps, h[:M]))
+                ) or ops.gemm_resid_norm(o, w, x, norm_w, eps, h[:M], out=x, slices="most")
 
     def _proj_resid_scaled(self, o, key, x, norm_w, h, sq, next_key):
         """x += bf16(o @ W^T), h = bf16(x * norm_w) and the rows' sums of squares (ops.gemm_rows_resid), for the projection `next_key` that
@@ -524,7 +526,8 @@ class Phi3VModel(DecoderModel):
                     normed_in = True                            # (`h` holds the normalised input now, whatever the fused call answers)
                     qkv_args = (hn, w[k_w], st.cos, st.sin, q, kd, vd, B, L, nh, nkv, hd, past, st.Tp, True, st.T, 1)
                     fused_qkv = (M <= 128 and not self.serving and ops.gemm_qkv_merge(*qkv_args, q_scale=scale * ops.Q_PRESCALE)
-                                 or ops.gemm_qkv(*qkv_args, q_scale=scale * ops.Q_PRESCALE))
+                                 or ops.gemm_qkv(*qkv_args, q_scale=scale * ops.Q_PRESCALE)
+                                 or ops.gemm_qkv(*qkv_args, q_scale=scale * ops.Q_PRESCALE, one_pass=True))
             f8_w = self.w8.get(k_w)                             # the same on e4m3 weights and quantised rows
             if (f8_w is not None and L > ops.L.DECODE_MAX_L and n_beam == 1 and k_w not in self.adapters and not mlx4_first and self.fp8_act
                     and ops.gemm_fp8_ok(M, f8_w[0].shape[0], cfg.hidden_size, EPI_NONE) and os.environ.get("P3V_QKV_FUSE", "1") != "0"

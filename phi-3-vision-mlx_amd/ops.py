@@ -181,9 +181,16 @@ def gemm_merge(a, w, epilogue, out):
     return True
 
 
+def _slices_bytes(M, N, K, epilogue, slices):
+    if not slices:
+        return 0
+    return (L.lib().p3v_gemm_ws_most_bytes if slices == "most" else L.lib().p3v_gemm_ws_bytes)(M, N, K, epilogue)
+
+
 def gemm(a, w, epilogue=EPI_NONE, bias=None, resid=None, out=None, n_out=None, pos=None, patches_per_img=0, ldo=None,
-         col_scale=None):
-    """nn.Linear / patch conv: out[M,N] = a[M,K] @ w[N,K]^T (+ epilogue), bf16 MFMA."""
+         col_scale=None, slices=True):
+    """nn.Linear / patch conv: out[M,N] = a[M,K] @ w[N,K]^T (+ epilogue), bf16 MFMA.  slices: with a workspace for slices of K (True), for as
+    many as the library makes use of ("most"), or without one (False)."""
     _chk(a, BF16, "a"), _chk(w, BF16, "w")
     M, K = a.shape
     N = n_out if n_out is not None else (w.shape[0] // 2 if epilogue in GATED else w.shape[0])
@@ -192,15 +199,15 @@ def gemm(a, w, epilogue=EPI_NONE, bias=None, resid=None, out=None, n_out=None, p
     f32_out = epilogue in (EPI_BIAS_RESID_F32, EPI_PATCH, EPI_F32, EPI_SCALE_RESID_F32)
     if out is None:
         out = torch.empty((M, N), dtype=F32 if f32_out else BF16, device=a.device)
-    ws_bytes = L.lib().p3v_gemm_ws_most_bytes(M, N, K, epilogue)
+    ws_bytes = _slices_bytes(M, N, K, epilogue, slices)
     ws = _gemm_workspace(a.device, ws_bytes) if ws_bytes else None
     args = L.GemmArgs(_p(a), _p(w), _p(out), _p(bias), _p(resid), _p(pos), M, N, K, a.stride(0), w.stride(0),
-                      ldo if ldo is not None else N, epilogue, patches_per_img, _p(ws), ws.numel() if ws is not None else 0, _p(col_scale))
+                      ldo if ldo is not None else N, epilogue, patches_per_img, _p(ws), ws_bytes, _p(col_scale))     # (not the buffer's size: results do not follow what it once grew to)
     L.check(L.lib().p3v_gemm(C.byref(args), _stream()), "gemm")
     return out
 
 
-def gemm_resid_norm(a, w, resid, norm_w, eps, normed, out=None):
+def gemm_resid_norm(a, w, resid, norm_w, eps, normed, out=None, slices=True):
     """out = resid + bf16(a @ w^T) and normed = RMSNorm(out) * norm_w from the projection's own launch sequence (the K-slice GEMM +
     ONE reduction launch that also normalises).  Returns False, nothing launched, where the library does not split the shape
     (P3V_ERR_UNSUPPORTED): the caller runs gemm(..., EPI_RESID_BF16) and rmsnorm."""
@@ -211,17 +218,23 @@ def gemm_resid_norm(a, w, resid, norm_w, eps, normed, out=None):
         raise ValueError(f"gemm_resid_norm: shapes {a.shape} x {w.shape}, resid {resid.shape}, normed {normed.shape}")
     if out is None:
         out = torch.empty((M, N), dtype=BF16, device=a.device)
-    ws_bytes = L.lib().p3v_gemm_ws_most_bytes(M, N, K, EPI_RESID_BF16)
+    ws_bytes = _slices_bytes(M, N, K, EPI_RESID_BF16, slices)
     if not ws_bytes:
         return False
     ws = _gemm_workspace(a.device, ws_bytes)
     args = L.GemmArgs(_p(a), _p(w), _p(out), None, _p(resid), None, M, N, K, a.stride(0), w.stride(0), out.stride(0), EPI_RESID_BF16, 0,
-                      _p(ws), ws.numel())
+                      _p(ws), ws_bytes)
     rc = L.lib().p3v_gemm_resid_norm(C.byref(args), _p(norm_w), float(eps), _p(normed), _stream())
     if rc == L.ERR_UNSUPPORTED:
         return False
     L.check(rc, "gemm_resid_norm")
     return True
+
+
+def gemm_few_rows(M, N, K, epilogue):
+    """Whether slices of K on the tiles for few rows (gemm, gemm_resid_norm) go before gemm_slices: a long K of up to 256 rows on 96-column tiles.
+    3072 x 8192 with the norm, us: 200 rows 24.9 (gemm_slices 29.6), 256 rows 28.0 (29.5)."""
+    return M <= 256 and L.lib().p3v_gemm_ws_most_bytes(M, N, K, epilogue) > L.lib().p3v_gemm_ws_bytes(M, N, K, epilogue)
 
 
 def gemm_slices(a, w, epilogue, resid, out, bias=None, col_scale=None, norm=None):
@@ -462,17 +475,18 @@ def rope_kv_append(qkv, cos_t, sin_t, q_out, k_dst, v_dst, B, Lq, nh, nkv, hd, p
 
 
 def gemm_qkv(a, w, cos_t, sin_t, q_out, k_dst, v_dst, B, Lq, nh, nkv, hd, past, dst_t, dst_off_is_past, tab_t=0, tab_div=1,
-             q_scale=1.0, bias=None):
+             q_scale=1.0, bias=None, one_pass=False):
     """qkv projection + head split + _rotate_half + KVCache append in the GEMM's own launches (include/p3v.h: p3v_gemm_qkv) ==
     gemm(a, w[, bias]) followed by rope_kv_append(...), bit for bit.  Returns False -- nothing launched -- when the library does not
-    take the shape (short prompts, unaligned append offsets, ...): the caller then runs the two calls."""
+    take the shape (short prompts, unaligned append offsets, ...): the caller then runs the two calls.  one_pass: for the sizes where gemm
+    without slices pays (p3v_gemm_qkv_one_pass), == that gemm followed by rope_kv_append."""
     _chk(a, BF16, "a"), _chk(w, BF16, "w")
     M, K = a.shape
     g = L.GemmArgs(_p(a), _p(w), 0, _p(bias), 0, 0, M, w.shape[0], K, a.stride(0), w.stride(0), w.shape[0],
                    EPI_BIAS if bias is not None else EPI_NONE, 0, 0, 0)
     sp = L.QkvSplit(_p(cos_t), _p(sin_t), _p(q_out), _p(k_dst), _p(v_dst), B, Lq, nh, nkv, hd, int(past), dst_t, int(dst_off_is_past),
                     tab_t, tab_div, float(q_scale))
-    rc = L.lib().p3v_gemm_qkv(C.byref(g), C.byref(sp), _stream())
+    rc = (L.lib().p3v_gemm_qkv_one_pass if one_pass else L.lib().p3v_gemm_qkv)(C.byref(g), C.byref(sp), _stream())
     if rc == L.ERR_UNSUPPORTED:
         return False
     L.check(rc, "gemm_qkv")
@@ -884,9 +898,10 @@ def project(x, w, epilogue=EPI_NONE, resid=None, col_scale=None, out=None, alone
         if K % 64 == 0 and N % 8 == 0:
             if alone and epilogue in GATED and 104 < M <= 128 and gemm_merge(x, w, epilogue, out):
                 return out
-            if scaled and gemm_slices(x, w, epilogue, resid, out, col_scale=col_scale):
+            if scaled and not gemm_few_rows(M, N, K, epilogue) and gemm_slices(x, w, epilogue, resid, out, col_scale=col_scale):
                 return out
-            return gemm(x, w, epilogue, resid=resid, out=out, col_scale=col_scale)
+            return gemm(x, w, epilogue, resid=resid, out=out, col_scale=col_scale,
+                        slices=False if L.lib().p3v_gemm_one_pass_pays(M, N, K, epilogue) else "most")
     args = L.GemmArgs(_p(x), _p(w), _p(out), 0, _p(resid), 0, M, N, K, x.stride(0), w.stride(0), out.stride(0), epilogue, 0, 0, 0, _p(col_scale))
     L.check(L.lib().p3v_gemm_any(C.byref(args), int(f32), _stream()), "gemm_any")
     return out
@@ -974,9 +989,9 @@ def latent_ws_bytes(m, B, Lq, n_split):
 
 def _gemm_rows(a, w, out, M, N, K, lda, ldw):
     """out[M, N] = a w^T of raw row pointers (bf16), rows of a and w lda / ldw elements apart."""
-    ws_bytes = L.lib().p3v_gemm_ws_most_bytes(M, N, K, EPI_NONE)
+    ws_bytes = _slices_bytes(M, N, K, EPI_NONE, "most")
     ws = _gemm_workspace(out.device, ws_bytes) if ws_bytes else None
-    args = L.GemmArgs(a, w, _p(out), 0, 0, 0, M, N, K, lda, ldw, N, EPI_NONE, 0, _p(ws), ws.numel() if ws is not None else 0, 0)
+    args = L.GemmArgs(a, w, _p(out), 0, 0, 0, M, N, K, lda, ldw, N, EPI_NONE, 0, _p(ws), ws_bytes, 0)
     L.check(L.lib().p3v_gemm(C.byref(args), _stream()), "gemm")
 
 

@@ -288,20 +288,21 @@ def test_gemm_resid_norm_is_the_two_calls(ops, M, N, K):
     assert bool((sentinel == 7.0).all())
 
 
-@pytest.mark.parametrize("M", [33, 64, 65, 127, 128])
+@pytest.mark.parametrize("M", [33, 64, 65, 127, 128, 129, 191, 256])
 @pytest.mark.parametrize("N,K", [(3072, 8192), (2304, 8192), (3072, 6144)])
 def test_gemm_partials_on_96_columns(ops, M, N, K):
-    """Rows short of a full chip of 64-column tiles in K slices: 96-column tiles in eight slices, rows up to and across both tile heights,
+    """Rows short of a full chip of 64-column tiles in K slices: 96-column tiles in eight slices, rows up to and across both tile heights
+    (beyond 128 rows: four),
     neighbours of the output untouched.  Against fp64: the fp32 sums of eight slices (K products each within K 2^-24 of sum |a w|, far below the
     bf16 result's half step 2^-9 of its value, twice where the residual sum rounds again); the two tile heights agree bit for bit."""
     from phi_3_vision_mlx_amd import _lib
-    assert _lib.lib().p3v_gemm_ws_most_bytes(M, N, K, ops.EPI_RESID_BF16) == 8 * M * N * 4 > _lib.lib().p3v_gemm_ws_bytes(M, N, K, ops.EPI_RESID_BF16) > 0
+    assert _lib.lib().p3v_gemm_ws_most_bytes(M, N, K, ops.EPI_RESID_BF16) == (8 if M <= 128 else 4) * M * N * 4 > _lib.lib().p3v_gemm_ws_bytes(M, N, K, ops.EPI_RESID_BF16) > 0
     a, w, r = g((M, K), 80).cuda(), g((N, K), 81, 1.0 / math.sqrt(K)).cuda(), g((M + 1, N), 82).cuda()
     prod, mag = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
     for epi in (ops.EPI_NONE, ops.EPI_RESID_BF16):
         buf = torch.full((M + 1, N), 7.0, dtype=BF16, device="cuda")
         kw = dict(resid=r[:M]) if epi == ops.EPI_RESID_BF16 else {}
-        ops.gemm(a, w, epi, out=buf[:M], **kw)
+        ops.gemm(a, w, epi, out=buf[:M], slices="most", **kw)
         assert bool((buf[M] == 7.0).all())
         ref = prod + r[:M].double() if kw else prod
         tol = 2.0 ** -8 * ref.abs() + (2.0 ** -8 * prod.abs() if kw else 0) + K * 2.0 ** -24 * mag
@@ -309,9 +310,46 @@ def test_gemm_partials_on_96_columns(ops, M, N, K):
         if M <= 64:
             old = ops.set_tuning("gemm_skinny_tm128", 1)
             try:
-                assert torch.equal(ops.gemm(a, w, epi, **kw), buf[:M])
+                assert torch.equal(ops.gemm(a, w, epi, slices="most", **kw), buf[:M])
             finally:
                 ops.set_tuning("gemm_skinny_tm128", old)
+
+
+@pytest.mark.parametrize("M", [129, 200, 256, 257, 300, 384])
+@pytest.mark.parametrize("K,heads", [(512, 32), (1024, 24)])
+def test_gemm_one_pass_on_128_columns(ops, M, K, heads):
+    """Two or three tiles of 128 rows in one round of 128 x 128 tiles: up to 256 rows the same bits as on 64 columns (every sum runs through K
+    in order), gated ones too; beyond, without a workspace, within the fp32 sums of K products of fp64 (K 2^-24 of sum |a w|, below the result's
+    half step); the qkv epilogue has the bits of the product and p3v_rope_kv_append behind it, caches and neighbours untouched elsewhere."""
+    N = heads * 96 * 3
+    a, w = g((M, K), 90).cuda(), g((N, K), 91, 1.0 / math.sqrt(K)).cuda()
+    assert ops.L.lib().p3v_gemm_one_pass_pays(M, N, K, ops.EPI_NONE) == (M > 256)
+    buf = torch.full((M + 1, N), 7.0, dtype=BF16, device="cuda")
+    ops.gemm(a, w, out=buf[:M], slices=False)
+    assert bool((buf[M] == 7.0).all())
+    prod = a.double() @ w.double().t()
+    tol = 2.0 ** -8 * prod.abs() + K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t())
+    assert bool(((buf[:M].double() - prod).abs() <= tol).all())
+    if M <= 256:
+        wg = g((16384, K), 92, 1.0 / math.sqrt(K)).cuda()
+        gated = ops.gemm(a, wg, ops.EPI_SILU_MUL)
+        old = ops.set_tuning("gemm_skinny_tn", 64)
+        try:
+            assert torch.equal(ops.gemm(a, w), buf[:M]) and torch.equal(ops.gemm(a, wg, ops.EPI_SILU_MUL), gated)
+        finally:
+            ops.set_tuning("gemm_skinny_tn", old)
+    T = 8 + M + 3
+    Tp = (T + 127) // 128 * 128
+    cos, sin = torch.rand((1, T, 48), device="cuda"), torch.rand((1, T, 48), device="cuda")
+    outs = []
+    for fused in (False, True):
+        q, k, v = torch.full((1, heads, M, 96), 7.0, dtype=BF16, device="cuda"), g((1, heads, Tp, 96), 93).cuda(), g((1, heads, 96, Tp), 94).cuda()
+        if fused:
+            assert ops.gemm_qkv(a, w, cos, sin, q, k, v, 1, M, heads, heads, 96, 8, Tp, True, T, 1, q_scale=1.3, one_pass=M > 256)
+        else:
+            ops.rope_kv_append(buf[:M], cos, sin, q, k, v, 1, M, heads, heads, 96, 8, Tp, True, T, 1, q_scale=1.3)
+        outs.append((q, k, v))
+    assert all(torch.equal(x, y) for x, y in zip(*outs))
 
 
 @pytest.mark.parametrize("M,N,K,pin,kind", [(300, 3072, 8192, -1, "norm"), (200, 3072, 8192, -1, "norm"), (1023, 3072, 3072, -1, "norm"), (257, 384, 192, 343, "norm"),
