@@ -11,11 +11,11 @@
 //             twice the bf16 rate on this chip (the unscaled 16x16x32 fp8 MFMA runs at the bf16 rate).  A lane holds 32
 //             k bytes of its row (lane & 15) for k-block lane >> 4 -- the SAME bytes for A and B, so which k they are
 //             does not matter (the kernel takes 16-byte chunks fchunk and fchunk + 4: bank-conflict-free reads).
-//   tile      chosen by time (f8_tile_plan).  Flat ones, 128 or 160(M) x 256 / 192 / 128(N) x 128(K): 768
+//   tile      chosen by time (f8_tile_plan).  Flat ones, 128 or 160(M) x 256 / 192 / 128(N) x 128(K), and small ones: 768
 //             threads: 8 CONSUMER waves as 2(M) x 4(N), ONE MFMA per 16 x 16 block and K-tile, and 4 PRODUCER waves that only
 //             request K-tiles by LDS-DMA (as p3v_gemm_pc.hip): rows of 128 BYTES, 16-byte chunk c of row r stored at chunk
-//             c ^ (r & 7), swizzled on the source address; three buffers of a K-tile (four from 128 x 192 down: what 160 KiB
-//             hold), so a request has two or three K-tiles' time to land.  Tall ones, 192, 224 or 256 x 256, on FOUR waves that request and
+//             c ^ (r & 7), swizzled on the source address; three buffers of a K-tile (four from 128 x 192 down, up to eight of small ones: what
+//             160 KiB hold), so a request has two or three K-tiles' time to land.  Tall ones, 192, 224 or 256 x 256, on FOUR waves that request and
 //             multiply (k_gemm_f8_w4).
 //             What bounds it: the requests, 60 ns per four 1-KiB pieces of a CU with the weights from memory, 40 with all of it in the L2s
 //             (a K-tile of 192 x 256, 0.64 us of MFMAs, takes 0.81 - 0.85 and 0.73 where 12 - 60 CUs are at it), and, with all CUs at it, the
@@ -24,6 +24,11 @@
 //             122 -> 93, 2531 124 -> 106, 4096 198 -> 164, 8192 367 -> 327 (2.5 PFLOP/s); 9216 x 3072 2531 rows 71 -> 61, 4096 106 -> 97; 3072 x 8192
 //             3500 92 -> 69, 4096 99 -> 79; 3072 x 3072 4096 50 -> 37.  One round of flat tiles that fills the chip stays ahead of one of tall ones
 //             that does not: 3072 x 8192 at 2531 rows 59 (128 rows), 62 (192).
+//             Some hundred rows leave most CUs without a 128 x 128 tile, and no slices of K can bring them in (another order of the sums would reach the next
+//             row quantiser).  Tiles of 32 x 64, 64 x 64, 64 x 128 and 96 x 128 do: a K-tile of 12 - 28 KB is 0.23 - 0.45 us of a CU's requests instead of
+//             0.5, with up to eight buffers of it in flight.  us, 128 x 128 -> the small one: 3072 x 8192 137 rows 31.0 -> 18.0 (32 x 64), 276 31.2 -> 21.5
+//             (64 x 64), 512 39.3 -> 30.1 (64 x 128), 803 33.2 -> 32.9 (96 x 128); 3072 x 3072 137 rows 15.1 -> 9.1, 276 15.5 -> 11.2; 9216 x 3072 137 rows 15.9
+//             -> 14.2; gate | up 128 rows 23.0 -> 20.1.  Tiles of 96 x 64 and 128 x 64 are hardly ever the fastest, by 3 % then.
 //   epilogue  scales, then none / residual add / SiLU(gate) * up, bf16 out, straight from the accumulators (p3v_gemm256_epi.h).
 #include <stdlib.h>
 
@@ -48,7 +53,19 @@ struct PlaceF8 { int m0, n0, swapped, is_k, row0; };             // P3V_EPI_QKV:
 struct TileF8 { int a_off[8], b_off[8]; __amdgpu_buffer_rsrc_t rs_a, rs_b; };   // where the requests of an output tile's K-tiles come from
 
 #define F8_BUF(mb, nb) ((32 * (mb) + 64 * (nb)) * TKB)
-#define F8_STAGES(mb, nb) (160 * 1024 / F8_BUF(mb, nb) < 4 ? 160 * 1024 / F8_BUF(mb, nb) : 4)
+#define F8_STAGES(mb, nb) f8_stages(160 * 1024 / F8_BUF(mb, nb), F8_BUF(mb, nb))
+constexpr int f8_stages(int fit, int buf) { return buf >= 32 * 1024 ? (fit < 4 ? fit : 4) : fit < 8 ? fit : 8; }
+
+// s_waitcnt vmcnt(PER n): all but the n youngest K-tiles of PER requests each have landed
+template <int PER>
+__device__ __forceinline__ void f8_wait(int n) {
+#define F8_WAIT(k) case k: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(k * PER < 63 ? k * PER : 63) : "memory"); break;
+  switch (n) {
+    F8_WAIT(1) F8_WAIT(2) F8_WAIT(3) F8_WAIT(4) F8_WAIT(5) F8_WAIT(6) F8_WAIT(7)
+    default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+#undef F8_WAIT
+}
 
 // A wave's 16 MB x 16 NB sums at rows mrow0 - fc .., outputs from column nw on, straight from the accumulators: lane (fc = lane & 15, fq = lane >> 4)
 // holds columns 4 fq .. 4 fq + 3 of block row fc; lanes q and q ^ 1 trade packed halves of two neighbouring column blocks: 16-byte stores.
@@ -126,7 +143,7 @@ __global__ void __launch_bounds__(768, 1) k_gemm_f8(GemmF8P p) {
   constexpr int HB = SILU ? NB / 2 : NB;                           // column blocks of outputs of a wave
   constexpr int TM = 32 * MB, TN = 64 * NB, A_BYTES = TM * TKB, BUF_BYTES = F8_BUF(MB, NB);
   constexpr int S = F8_STAGES(MB, NB), PER = MB + 2 * NB;          // LDS buffers; requests of a producer wave per K-tile
-  static_assert(S >= 3 && (S - 1) * PER < 64, "");
+  static_assert(S >= 3 && S <= 8 && (S - 1) * PER < 64, "f8_wait");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr int n_out_tile = SILU ? TN / 2 : TN;
@@ -214,11 +231,7 @@ __global__ void __launch_bounds__(768, 1) k_gemm_f8(GemmF8P p) {
     for (int g = 0; g < min(S, total); ++g) request();
     for (int g = 0; g < total; ++g) {
       // K-tile g has landed when only the younger ones' requests are out: S - 1 of them at first, then S - 2, fewer at the end
-      const int young = min(g == 0 ? S - 1 : S - 2, total - 1 - g);
-      if (young >= 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S > 3 ? 3 : 0) * PER) : "memory");
-      else if (young == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER) : "memory");
-      else if (young == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      f8_wait<PER>(min(g == 0 ? S - 1 : S - 2, total - 1 - g));
       __builtin_amdgcn_s_barrier();                               // K-tile g is there; K-tile g - 1 is in the consumers' registers
       if (g > 0 && g - 1 + S < total) request();
     }
@@ -617,13 +630,17 @@ static int launch_f8_v(const GemmF8P& p, hipStream_t s) {
 // names is 0.2 % slower than the fastest of the seven on average over those 360 sizes, 6.8 % at most (with each projection's own times left out of the
 // fit: the same).  The fit to K = 3072 and 8192 alone that this one replaces: 1.4 %, 20 % at most, at short K (4096 x 384, 1300 rows 9.8 -> 8.9 us; 9216 x 3072,
 // 1024 rows 31.3 -> 29.9); rounds alone: 7.7 % at K = 3072 and 8192.
+// The four small tiles are fitted to 14 heights, 64 .. 1300 rows, of the same projections (the second table there): what the plan names is 0.8 % slower than
+// the fastest of eleven on average, 25 % at most (803 x 9216 x 640 as before them), and 17.5 % faster than the fastest of seven (3 % slower at most).
 static int f8_cus() { const int n = p3v_gemm256_cus(); return n ? n : 256; }     // (no device: host queries)
 struct F8Tile { int mb, nb; float once, f, gated, resid, c, fill, out; };
 static float f8_tile_plan(int M, int N, int K, int ldo, int epilogue, int& mb, int& nb) {
   static const F8Tile tiles[] = {{4, 4, 4.82f, 0.1f, 1.75f, 1.45f, 0.779f, 0.023f, 2.48f},  {5, 4, 5.01f, 0.71f, 2.18f, 1.85f, 0.804f, 0.103f, 2.57f},
                                  {4, 3, 5.72f, 0.42f, 0.f, 1.64f, 0.569f, 0.054f, 1.86f},   {4, 2, 3.87f, 0.21f, 0.76f, 0.72f, 0.492f, 0.017f, 1.44f},
                                  {8, 4, 5.02f, 3.29f, 1.82f, 2.34f, 0.98f, 0.269f, 2.46f},  {7, 4, 5.18f, 2.09f, 1.69f, 1.88f, 0.897f, 0.2f, 2.45f},
-                                 {6, 4, 4.97f, 1.57f, 1.4f, 1.25f, 0.847f, 0.141f, 2.36f}};
+                                 {6, 4, 4.97f, 1.57f, 1.4f, 1.25f, 0.847f, 0.141f, 2.36f},
+                                 {3, 2, 3.395f, 0.f, 0.869f, 0.236f, 0.42f, 0.108f, 1.499f}, {2, 2, 3.051f, 0.f, 0.679f, 0.014f, 0.431f, 0.021f, 0.975f},
+                                 {2, 1, 2.443f, 0.888f, 0.f, 0.103f, 0.293f, 0.f, 0.475f},   {1, 1, 2.35f, 0.602f, 0.f, 0.227f, 0.234f, 0.f, 0.138f}};
   const int n_cu = f8_cus(), pin = p3v_tuning().gemm_f8_narrow;
   const bool silu = epilogue == P3V_EPI_SILU_MUL, resid = epilogue == P3V_EPI_RESID_BF16;
   const float kt = (float)(K / TKB);
@@ -635,7 +652,7 @@ static float f8_tile_plan(int M, int N, int K, int ldo, int epilogue, int& mb, i
     const long n = (long)(N / n_tile) * p3v_cdiv(M, 32 * t.mb);
     const float rounds = (float)p3v_cdiv(n, (long)n_cu), used = (float)n / (float)n_cu;
     float c = t.once + rounds * (t.f + (silu ? t.gated : resid ? t.resid : 0.f) + t.c * kt) + used * (t.fill * kt + t.out);
-    if (pin == 10 * t.mb + t.nb || (pin == 0 && t.mb == 4 && t.nb == 4) || (pin == 1 && t.nb == 2)) c = 0.f;
+    if (pin == 10 * t.mb + t.nb || (pin == 0 && t.mb == 4 && t.nb == 4) || (pin == 1 && t.mb == 4 && t.nb == 2)) c = 0.f;
     if (best < 0.f || c < best) best = c, mb = t.mb, nb = t.nb;
   }
   return best;
@@ -647,7 +664,9 @@ static int launch_f8(const GemmF8P& p, hipStream_t s) {
   f8_tile_plan(p.M, p.N, p.K, p.ldo, EPI, mb, nb);
   if constexpr (EPI != P3V_EPI_SILU_MUL)
     if (nb == 3) return launch_f8_v<EPI, 4, 3>(p, s);
-  if (nb == 2) return launch_f8_v<EPI, 4, 2>(p, s);
+  if constexpr (EPI != P3V_EPI_SILU_MUL)
+    if (nb == 1) return mb == 1 ? launch_f8_v<EPI, 1, 1>(p, s) : launch_f8_v<EPI, 2, 1>(p, s);
+  if (nb == 2) return mb == 2 ? launch_f8_v<EPI, 2, 2>(p, s) : mb == 3 ? launch_f8_v<EPI, 3, 2>(p, s) : launch_f8_v<EPI, 4, 2>(p, s);
   if (mb == 8) return launch_f8_w4<EPI, 8>(p, s);
   if (mb == 7) return launch_f8_w4<EPI, 7>(p, s);
   if (mb == 6) return launch_f8_w4<EPI, 6>(p, s);

@@ -2344,6 +2344,30 @@ def test_gemm_fp8_tiles_agree(ops, request, epi, M, N, K):
 
 
 @pytest.mark.parametrize("epi", ["none", "resid", "silu"])
+@pytest.mark.parametrize("M,N,K", [(1, 256, 128), (31, 256, 256), (33, 768, 896), (64, 384, 1024), (65, 256, 1152), (97, 768, 2176), (2049, 3072, 256), (160, 3072, 3072)])
+def test_gemm_fp8_small_tiles(ops, request, epi, M, N, K):
+    """Tiles of 32 x 64, 64 x 64, 64 x 128 and 96 x 128 against the 128 x 128 one: the same bits.  1 .. 9 and 17 K-tiles against five to eight buffers, rows at and past
+    a tile's, a K-tile stream that crosses from one output tile of a workgroup to the next (2049 x 3072), the row behind the last untouched."""
+    EPI = {"none": ops.EPI_NONE, "resid": ops.EPI_RESID_BF16, "silu": ops.EPI_SILU_MUL}[epi]
+    rows = 2 * N if epi == "silu" else N
+    a8, w8 = _e4m3(g((M, K), 65, 1.0, F32)).view(torch.uint8).cuda(), _e4m3(g((rows, K), 66, 1.0, F32)).view(torch.uint8).cuda()
+    gen = torch.Generator().manual_seed(67)
+    sa, sw = (torch.rand((M,), generator=gen) + 0.5).cuda(), ((torch.rand((rows,), generator=gen) + 0.5) / K).cuda()
+    x = g((M + 1, N), 68, 1.0).cuda()
+    old = ops.set_tuning("gemm_f8_narrow", -1)
+    request.addfinalizer(lambda: ops.set_tuning("gemm_f8_narrow", old))
+    outs = []
+    for tile in (42, 32, 22) + (() if epi == "silu" else (21, 11)):
+        ops.set_tuning("gemm_f8_narrow", tile)
+        assert ops.L.lib().p3v_gemm_fp8_tile(M, N, K, EPI) == tile
+        out = x.clone()
+        ops.gemm_fp8(a8, sa, w8, sw, EPI, resid=out[:M] if epi == "resid" else None, out=out[:M])
+        assert torch.equal(out[M], x[M]), tile
+        outs.append(out[:M])
+    assert all(torch.equal(o, outs[0]) for o in outs) and torch.isfinite(outs[0].float()).all() and not torch.equal(outs[0], x[:M])
+
+
+@pytest.mark.parametrize("epi", ["none", "resid", "silu"])
 @pytest.mark.parametrize("M,cols,K", [(1, 1, 256), (192, 1, 512), (193, 3, 256), (225, 2, 1024), (257, 1, 3072), (4301, 12, 256), (2531, 24, 512),
                                       (257, 2, 384), (193, 1, 640), (4301, 24, 256), (4301, 24, 384), (4301, 24, 768), (8449, 24, 640), (8449, 24, 256), (300, 3, 128), (8449, 24, 128)])
 def test_gemm_fp8_tall_tiles(ops, request, epi, M, cols, K):

@@ -88,7 +88,7 @@ def sweep_bf16(rows):
 
 
 def sweep_fp8(rows):
-    tiles = [44, 54, 43, 42, 64, 74, 84]
+    tiles = [44, 54, 43, 42, 64, 74, 84, 32, 22, 21, 11]
     print("N x K (epilogue)                 M  choice" + "".join(f"{t:>8}" for t in tiles))
 
     def codes(n, k):
@@ -105,7 +105,7 @@ def sweep_fp8(rows):
                 for i, x in enumerate(w):
                     ops.gemm_fp8(a[i % 2], sa, x, ws, e, resid=r if epi == "resid" else None, out=out)
                 return _lib.lib().p3v_gemm_fp8_tile(M, N, K, e) in tiles
-            usable = [t for t in tiles if N % (32 * (t % 10) if epi == "silu" else 64 * (t % 10)) == 0 and not (epi == "silu" and t == 43)]
+            usable = [t for t in tiles if N % (32 * (t % 10) if epi == "silu" else 64 * (t % 10)) == 0 and not (epi == "silu" and t % 2)]
             times = dict(zip(usable, in_turn("gemm_f8_narrow", usable, run, len(w) * 2.0 * M * wn * K, 2e15)))
             row(f"{N}{'(x2)' if epi == 'silu' else ''} x {K} {epi}", M, _lib.lib().p3v_gemm_fp8_tile(M, N, K, e), [times.get(t) for t in tiles], len(w))
 
