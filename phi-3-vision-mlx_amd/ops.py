@@ -108,6 +108,16 @@ def owned_gemm_workspace(holder, frozen):
         _ws_owner.now = prev
 
 
+def _owned_scratch(name, n, dtype, device):
+    holder, frozen = _ws_owner.now
+    buf = holder.get(name)
+    if buf is None or buf.numel() < n:
+        if frozen:
+            raise RuntimeError(f"scratch {name} of {n} elements requested under graph capture (warm-up sized {0 if buf is None else buf.numel()})")
+        buf = holder[name] = torch.empty((n,), dtype=dtype, device=device)
+    return buf
+
+
 def _gemm_workspace(device, nbytes):
     """The library never allocates (include/p3v.h): the caller owns the split-K workspace.  One grow-only torch buffer per
     (device, stream): it is live only between the two launches of one p3v_gemm call, so launches on one stream share it."""
@@ -419,9 +429,13 @@ def dequant_fp8(w8, w_scale, out=None):
 
 def quant_fp8_rows(x, norm_w=None, norm_eps=0.0, out=None, scale=None):
     """bf16 rows -> (e4m3 bytes [M, K], fp32 scale [M]), one scale per row = max|h| / 448; with `norm_w` h is the
-    RMSNorm of x (the fused activation quantiser of the W8A8 prefill projections)."""
+    RMSNorm of x (the fused activation quantiser of the W8A8 prefill projections).  Inside owned_gemm_workspace what is not given is the
+    owner's scratch, good until the next call: a graph keeps writing to it."""
     _chk(x, BF16, "x")
     M, K = x.shape
+    if _ws_owner.now is not None:
+        out = _owned_scratch("a8", M * K, torch.uint8, x.device)[:M * K].view(M, K) if out is None else out
+        scale = _owned_scratch("a8_scale", M, F32, x.device)[:M] if scale is None else scale
     out = torch.empty((M, K), dtype=torch.uint8, device=x.device) if out is None else out
     scale = torch.empty((M,), dtype=F32, device=x.device) if scale is None else scale
     L.check(L.lib().p3v_quant_fp8_rows(_p(x), _p(norm_w), float(norm_eps), _p(out), _p(scale), M, K, _stream()), "quant_fp8_rows")

@@ -282,6 +282,38 @@ def test_captured_short_prompt_prefill_with_4bit_weights_equals_eager(monkeypatc
     assert len(model._prefill_graphs) == 1
 
 
+@pytest.mark.parametrize("kw", [dict(quantized_fp8=True, use_quantized_cache=True), dict(quantized_fp8=True), dict(use_quantized_cache=True),
+                                dict(quantized_fp8=True, use_quantized_cache=True, fp8_activations=False)])
+@pytest.mark.parametrize("n", [57, 200])
+def test_captured_prefill_with_8bit_weights_and_cache_equals_eager(monkeypatch, kw, n):
+    """The same for e4m3 weights (the activation quantiser's rows belong to the graph) and the int8 cache: two prompts in turn, decode steps, eager
+    work of other sizes and synchronisations between the replays, every one bit-identical to the eager path, cache rows too."""
+    from phi_3_vision_mlx_amd import ops
+    from phi_3_vision_mlx_amd.api import load_synthetic
+    model, _ = load_synthetic(blind_model=True, tiny=False, seed=0, device="cuda:0", num_hidden_layers=2, **kw)
+    ids = [rand_ids(n, 44 + i) for i in range(2)]
+    quantised = kw.get("use_quantized_cache", False)
+
+    def one(i):
+        lg, cache = model(input_ids=ids[i], max_tokens=6)
+        st = cache[0].state
+        rows = [t[..., :n].clone() for t in ((st.v8, st.ks, st.vs) if quantised else (st.v,))] + [(st.k8 if quantised else st.k)[:, :, :, :n].clone()]
+        t, toks = ops.argmax(lg[:, -1, :].contiguous())[:, None], []
+        for _ in range(3):
+            _, t = model.greedy_step(t, cache)
+            toks.append(t.clone())
+        return [lg.clone(), torch.cat(toks, 1)] + rows
+    monkeypatch.setenv("P3V_PREFILL_GRAPH", "0")
+    ref = [one(0), one(1)]
+    monkeypatch.setenv("P3V_PREFILL_GRAPH", "1")
+    for rep in range(6):
+        got = one(rep & 1)
+        assert all(torch.equal(a, b) for a, b in zip(got, ref[rep & 1])), rep
+        model(input_ids=rand_ids(90 + rep, 50 + rep), max_tokens=2)     # (another length, eager: its scratch is its own)
+        torch.cuda.synchronize()
+    assert len(model._prefill_graphs) == 1
+
+
 def test_graph_decode_with_more_than_16_rows(text):
     """B = 20 rows: the decode projections are split-K GEMMs (M > 16), whose workspace the captured graph must own (
     no allocation under capture, no dangling pointer after a regrow).  Graph replays == eager steps, bit for bit, also after
