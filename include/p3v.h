@@ -255,6 +255,8 @@ int p3v_gemm_qkv_merge(const p3v_gemm_args_t* gemm /* host */, const p3v_qkv_spl
  * (hd / 2) % 16 == 0, whole 256-column tiles per region, an 8-aligned append offset and dst_t, and B == 1 or L >= 7. */
 int p3v_gemm_qkv_fp8(const p3v_gemm_fp8_args_t* gemm /* host */, const p3v_qkv_split_t* split /* host */, void* stream);
 int p3v_gemm_qkv_fp8_pays(int M, int n_q, int n_kv, int K);      /* 1: faster than the two calls (n_q, n_kv: rows of W per region) */
+/* the same where p3v_rope_kv_quantize takes the place of p3v_rope_kv_append and the keys' and values' quantiser */
+int p3v_gemm_qkv_fp8_stored_pays(int M, int n_q, int n_kv, int K);
 
 /* ---- attention, phi.py:454-457 (decoder, causal + left-pad, Mask4D phi.py:550-563)
  * and phi.py:148 (CLIP, no mask).  q [B, nh, L, hd]; keys/values come from two
@@ -347,6 +349,11 @@ int p3v_stage_rope(const float* cos_t, const float* sin_t, int past, const int32
  * p3v_kv_quantize converts rows [t0, t0+n_tok) of a bf16 K [BH, src_t, hd] / V^T [BH, hd, src_t] pair. */
 int p3v_kv_quantize(const uint16_t* k, const uint16_t* vt, uint8_t* k8, uint8_t* v8t, float* k_scale, float* v_scale,
                     int BH, int hd, int src_t, int dst_t, int t0, int n_tok, void* stream);
+/* p3v_rope_kv_append (rotated, at columns past ..) and p3v_kv_quantize of the appended tokens into int8 caches of the same dst_t columns, bit for bit, in one
+ * launch.  P3V_ERR_UNSUPPORTED, nothing launched: hd != 96, L < 32, past % 8, dst_t % 8, rows off 16 bytes, codes off 8: the two calls. */
+int p3v_rope_kv_quantize(const uint16_t* qkv, const float* cos_t, const float* sin_t, uint16_t* q_out, uint16_t* k_dst, uint16_t* v_dst, uint8_t* k8,
+                         uint8_t* v8t, float* k_scale, float* v_scale, int B, int L, int n_heads, int n_kv, int hd, int past, int dst_t, int tab_t,
+                         int tab_div, float q_scale, void* stream);
 /* p3v_attention_decode on the int8 cache: same contract; the step's own new rows are quantised,
  * appended, and attended in their quantised form (one representation per key, whenever it is read). */
 /* the inverse, tokens [0, n_tok) of every (batch row, kv head): bf16 K [BH, dst_t, hd] / V^T [BH, hd, dst_t] = (code - 128) * scale.

@@ -147,6 +147,7 @@ SIGNATURES = {
     "p3v_attention_decode_can_fuse_oproj": (i32, [i32, i32, i32, i32, i32, i32, i32, i32]),
     "p3v_attention_decode_rows_fit": (i32, [i32, i32, i32, i32, i32]),
     "p3v_attention_decode_fused_role": (i32, [i32, i32, i32, i32, i32, C.POINTER(i32)]),
+    "p3v_rope_kv_quantize": (i32, [vp] * 10 + [i32] * 9 + [f32, vp]),
     "p3v_kv_quantize": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]),
     "p3v_kv_dequantize": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]),
     "p3v_gemm_qkv": (i32, [vp, vp, vp]),
@@ -160,6 +161,7 @@ SIGNATURES = {
     "p3v_gemm_qkv_tile": (i32, [i32, i32, i32, i32]),
     "p3v_gemm_qkv_fp8": (i32, [C.POINTER(GemmF8Args), C.POINTER(QkvSplit), vp]),
     "p3v_gemm_qkv_fp8_pays": (i32, [i32, i32, i32, i32]),
+    "p3v_gemm_qkv_fp8_stored_pays": (i32, [i32, i32, i32, i32]),
     "p3v_gemm_slices": (i32, [C.POINTER(GemmArgs), vp, f32, vp, vp]),
     "p3v_gemm_slices_ws_bytes": (i64, [i32, i32, i32, i32]),
     "p3v_gemm_resid_norm": (i32, [C.POINTER(GemmArgs), vp, f32, vp, vp]),

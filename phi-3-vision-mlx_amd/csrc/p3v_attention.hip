@@ -3249,6 +3249,145 @@ extern "C" int p3v_kv_quantize(const uint16_t* k, const uint16_t* vt, uint8_t* k
   return P3V_OK;
 }
 
+// p3v_rope_kv_append, then p3v_kv_quantize of what it appended, in one launch: the same values and codes.  First the V tiles, a workgroup per 64
+// tokens of a head: 16 lanes hold a token's 96 dimensions (12 of them work), so its maximum is known before the transpose, and LDS carries value and code in one
+// word.  Then a workgroup per token for its query and key rows, 8 lanes a row (6 work): a lane rotates chunk c and the one 48 dimensions on.  What bounds it:
+// launch and one trip for some hundred tokens, the traffic beyond (43 KB a token of 32 heads; the 12 KB of keys and values are not read again): 2531
+// tokens 20.6 us, 5.3 TB/s.  Behind the projection, launch behind launch, us a layer of 32 heads, two launches -> this: 137 tokens 8.9 -> 4.6, 276 10.2 -> 5.3, 803
+// 13.6 -> 7.6, 2531 31.5 -> 20.6, 8192 111 -> 98.
+struct RopeQ8P {
+  const bf16_t* qkv; const float* cos_t; const float* sin_t; bf16_t* q_out; bf16_t* k_dst; bf16_t* v_dst; uint8_t* k8; uint8_t* v8; float* ksc; float* vsc;
+  int B, L, nh, nkv, past, dst_t, tab_t, tab_div, nx;             // nx: 64-token tiles of a row
+  float q_scale;
+};
+__global__ void __launch_bounds__(256) k_rope_kv_q8(RopeQ8P p) {
+  constexpr int HD = 96, HALF = 48, LD = HD + 1;
+  __shared__ uint32_t tile[64 * LD];                              // value | code << 16 of (token, dim)
+  const int tid = threadIdx.x, row_w = (p.nh + 2 * p.nkv) * HD, n_v = p.nx * p.nkv * p.B;
+  if ((int)blockIdx.x < n_v) {
+    const int l0 = (int)blockIdx.x % p.nx * 64, head = (int)blockIdx.x / p.nx % p.nkv, b = (int)blockIdx.x / (p.nx * p.nkv);
+    const size_t bh = (size_t)b * p.nkv + head;
+    const int t0 = p.past + l0, c = tid & 15, r16 = tid >> 4;
+    const bf16_t* src = p.qkv + ((size_t)b * p.L + l0) * row_w + (p.nh + p.nkv + head) * HD + min(c, 11) * 8;
+    u32x4_t vv[4];
+#pragma unroll
+    for (int pass = 0; pass < 4; ++pass) vv[pass] = *(const u32x4_t*)(src + (size_t)min(pass * 16 + r16, p.L - 1 - l0) * row_w);
+#pragma unroll
+    for (int pass = 0; pass < 4; ++pass) {
+      const int r = pass * 16 + r16;
+      float x[8], amax = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = e & 1 ? bf16hi(vv[pass][e >> 1]) : bf16lo(vv[pass][e >> 1]), amax = fmaxf(amax, fabsf(x[e]));
+      amax = fmaxf(amax, P3V_DPP_F32(amax, 0xB1));
+      amax = fmaxf(amax, P3V_DPP_F32(amax, 0x4E));
+      amax = fmaxf(amax, P3V_DPP_F32(amax, 0x124));
+      amax = fmaxf(amax, P3V_DPP_F32(amax, 0x128));
+      const float sc = amax > 0.f ? amax / 127.f : 1.f, inv = 1.f / sc;
+      int q[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float y = x[e] * inv;
+        q[e] = (int)rintf(fmaf(fmaf(-y, sc, x[e]), inv, y));
+      }
+      if (sc < 1e-30f)                                            // (a scale whose reciprocal may overflow: the division itself)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) q[e] = (int)rintf(x[e] / sc);
+      if (c < 12) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) tile[r * LD + c * 8 + e] = (vv[pass][e >> 1] >> (16 * (e & 1)) & 0xffffu) | (uint32_t)(q[e] + 128) << 16;
+      }
+      if (c == 0 && l0 + r < p.L) p.vsc[bh * p.dst_t + t0 + r] = sc;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int i = j * 256 + tid, d = i >> 3, tc = i & 7, n_ok = min(8, p.L - (l0 + tc * 8));
+      if (n_ok <= 0) continue;
+      uint32_t w[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) w[e] = tile[(tc * 8 + e) * LD + d];
+      const size_t at = (bh * HD + d) * p.dst_t + t0 + tc * 8;
+      if (n_ok == 8) {
+        u32x4_t v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = __builtin_amdgcn_perm(w[2 * e + 1], w[2 * e], 0x05040100u);
+        *(u32x4_t*)(p.v_dst + at) = v;
+        u32x2_t o;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          o[h] = __builtin_amdgcn_perm(w[4 * h + 1], w[4 * h], 0x0c0c0602u) | __builtin_amdgcn_perm(w[4 * h + 3], w[4 * h + 2], 0x0c0c0602u) << 16;
+        *(u32x2_t*)(p.v8 + at) = o;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (e < n_ok) p.v_dst[at + e] = (bf16_t)w[e], p.v8[at + e] = (uint8_t)(w[e] >> 16);
+      }
+    }
+    return;
+  }
+  const int tok = (int)blockIdx.x - n_v, b = tok / p.L, l = tok - b * p.L, pos = p.past + l;
+  const int c = min(tid & 7, 5), r32 = tid >> 3, n_rows = p.nh + p.nkv;
+  const bool live = (tid & 7) < 6;
+  const bf16_t* row = p.qkv + (size_t)tok * row_w + c * 8;
+  const size_t trow = ((size_t)(b / p.tab_div) * p.tab_t + pos) * HALF + c * 8;
+  const float4 c0 = *(const float4*)(p.cos_t + trow), c1 = *(const float4*)(p.cos_t + trow + 4), s0 = *(const float4*)(p.sin_t + trow), s1 = *(const float4*)(p.sin_t + trow + 4);
+  const float cs[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w}, sn[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+  for (int h = r32; h < n_rows; h += 32) {
+    const u32x4_t lo = *(const u32x4_t*)(row + h * HD), hi = *(const u32x4_t*)(row + h * HD + HALF);
+    const bool is_k = h >= p.nh;
+    const float qs = is_k ? 1.f : p.q_scale;
+    u32x4_t olo, ohi;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float x0, y0, x1, y1;
+      p3v_rope_pair(bf16lo(lo[j]), bf16lo(hi[j]), cs[2 * j], sn[2 * j], qs, x0, y0);
+      p3v_rope_pair(bf16hi(lo[j]), bf16hi(hi[j]), cs[2 * j + 1], sn[2 * j + 1], qs, x1, y1);
+      olo[j] = pack_bf16x2(x0, x1), ohi[j] = pack_bf16x2(y0, y1);
+    }
+    if (!is_k) {
+      bf16_t* dst = p.q_out + (((size_t)b * p.nh + h) * p.L + l) * HD + c * 8;
+      if (live) *(u32x4_t*)dst = olo, *(u32x4_t*)(dst + HALF) = ohi;
+      continue;
+    }
+    float amax = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) amax = fmaxf(fmaxf(fmaxf(amax, fabsf(bf16lo(olo[j]))), fmaxf(fabsf(bf16hi(olo[j])), fabsf(bf16lo(ohi[j])))), fabsf(bf16hi(ohi[j])));
+    amax = fmaxf(amax, P3V_DPP_F32(amax, 0xB1));
+    amax = fmaxf(amax, P3V_DPP_F32(amax, 0x4E));
+    amax = fmaxf(amax, P3V_DPP_F32(amax, 0x141));                 // row_half_mirror: the other four lanes of the row's eight
+    const float sc = amax > 0.f ? amax / 127.f : 1.f, inv = 1.f / sc;
+    const size_t at = ((size_t)b * p.nkv + h - p.nh) * p.dst_t + pos;
+    if (live) {
+      *(u32x4_t*)(p.k_dst + at * HD + c * 8) = olo, *(u32x4_t*)(p.k_dst + at * HD + c * 8 + HALF) = ohi;
+      u32x2_t o, o2;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        o[e] = pack_codes((int)rintf(bf16lo(olo[2 * e]) * inv), (int)rintf(bf16hi(olo[2 * e]) * inv), (int)rintf(bf16lo(olo[2 * e + 1]) * inv),
+                          (int)rintf(bf16hi(olo[2 * e + 1]) * inv));
+        o2[e] = pack_codes((int)rintf(bf16lo(ohi[2 * e]) * inv), (int)rintf(bf16hi(ohi[2 * e]) * inv), (int)rintf(bf16lo(ohi[2 * e + 1]) * inv),
+                           (int)rintf(bf16hi(ohi[2 * e + 1]) * inv));
+      }
+      *(u32x2_t*)(p.k8 + at * HD + c * 8) = o, *(u32x2_t*)(p.k8 + at * HD + c * 8 + HALF) = o2;
+    }
+    if ((tid & 7) == 0) p.ksc[at] = sc;
+  }
+}
+
+extern "C" int p3v_rope_kv_quantize(const uint16_t* qkv, const float* cos_t, const float* sin_t, uint16_t* q_out, uint16_t* k_dst, uint16_t* v_dst, uint8_t* k8,
+                                    uint8_t* v8t, float* k_scale, float* v_scale, int B, int L, int n_heads, int n_kv, int hd, int past, int dst_t, int tab_t,
+                                    int tab_div, float q_scale, void* stream) {
+  if (!qkv || !cos_t || !sin_t || !q_out || !k_dst || !v_dst || !k8 || !v8t || !k_scale || !v_scale || !(q_scale > 0.f)) return P3V_ERR_ARG;
+  if (B <= 0 || L <= 0 || n_heads <= 0 || n_kv <= 0 || tab_div <= 0 || past < 0 || past > dst_t - L) return P3V_ERR_ARG;
+  if (hd != 96 || L < 32 || past % 8 || dst_t % 8 || (((uintptr_t)qkv | (uintptr_t)cos_t | (uintptr_t)sin_t | (uintptr_t)q_out | (uintptr_t)k_dst | (uintptr_t)v_dst) & 15) ||
+      (((uintptr_t)k8 | (uintptr_t)v8t) & 7))
+    return P3V_ERR_UNSUPPORTED;
+  const int nx = p3v_cdiv(L, 64);
+  const RopeQ8P p = {qkv, cos_t, sin_t, q_out, k_dst, v_dst, k8, v8t, k_scale, v_scale, B, L, n_heads, n_kv, past, dst_t, tab_t, tab_div, nx, q_scale};
+  hipLaunchKernelGGL(k_rope_kv_q8, dim3(nx * n_kv * B + B * L), dim3(256), 0, (hipStream_t)stream, p);
+  P3V_CHECK_LAUNCH();
+  return P3V_OK;
+}
+
 // int8 caches -> bf16 K [BH, dst_t, hd] / V^T [BH, hd, dst_t], tokens [0, n_tok): (code - 128) * scale, rounded once.
 // Used by cached calls with more than 16 new tokens on the quantised cache (constrain() with a long constraint text):
 // they attend through the prefill kernel on a dequantised copy of the layer (the reference re-dequantises the whole

@@ -707,15 +707,20 @@ extern "C" int p3v_gemm_fp8(const p3v_gemm_fp8_args_t* a, void* stream) {
 // way by 13 us.)  us a layer, two - one, in a prompt: 768 tokens 5, 2531 13, 4096 37, 6000 16, but 256 -5, 1024 -7, 1800 -10, 2700 -11, where tiles of
 // other heights fill their rounds; 8192 -15, where the rule says one (launch behind launch: +30).
 // (Tiles of 192 and 224 rows on four waves under this epilogue, with one wave per SIMD to run it: no faster than the faster of the two at any size.)
-extern "C" int p3v_gemm_qkv_fp8_pays(int M, int n_q, int n_kv, int K) {
-  if (M <= 0 || K <= 0 || n_q <= 0 || n_kv <= 0 || n_q % 256 || n_kv % 256) return 0;
+static float qkv_fp8_gain(int M, int n_q, int n_kv, int K) {       // us that one launch saves
   int mb, nb;
   const int N = n_q + 2 * n_kv, n_cu = f8_cus();
   const float kt = (float)(K / TKB), out = (float)M * (float)N;
   const long tiles = (long)(n_q + n_kv) / 256 * p3v_cdiv(M, 128) + (long)n_kv / 128 * p3v_cdiv(M, 256);
   const float one = 6.66f + p3v_cdiv(tiles, (long)n_cu) * (1.73f + 0.62f * kt) + (float)tiles / (float)n_cu * (0.2f * kt + 4.23f);
-  return one < f8_tile_plan(M, N, K, N, P3V_EPI_NONE, mb, nb) + 3.5f + 9.5e-7f * out + 4e-7f * fmaxf(out - 2e7f, 0.f);
+  return f8_tile_plan(M, N, K, N, P3V_EPI_NONE, mb, nb) + 3.5f + 9.5e-7f * out + 4e-7f * fmaxf(out - 2e7f, 0.f) - one;
 }
+static bool qkv_fp8_sizes(int M, int n_q, int n_kv, int K) { return M > 0 && K > 0 && n_q > 0 && n_kv > 0 && n_q % 256 == 0 && n_kv % 256 == 0; }
+extern "C" int p3v_gemm_qkv_fp8_pays(int M, int n_q, int n_kv, int K) { return qkv_fp8_sizes(M, n_q, n_kv, K) && qkv_fp8_gain(M, n_q, n_kv, K) > 0.f; }
+// With an int8 cache behind it the split + rotation store the codes too (p3v_rope_kv_quantize), and a quantiser's launch goes with them: one launch has to
+// gain 5 us more.  us a layer in whole prompts, two - one: 400 tokens -5.0, 577 -5.0, 680 -1.6, 2300 -10.2, 2531 +1.2, 3500 -7.0 (the rule says one), 3800 -1.2,
+// 4096 +25, 6000 +3.1, 7000 +1.5, 8000 +20; 7600 -15 and 8192 -52, where it says one.
+extern "C" int p3v_gemm_qkv_fp8_stored_pays(int M, int n_q, int n_kv, int K) { return qkv_fp8_sizes(M, n_q, n_kv, K) && qkv_fp8_gain(M, n_q, n_kv, K) > 5.f; }
 
 // p3v_gemm_fp8 (epilogue NONE) + p3v_rope_kv_append in one launch, bit for bit, on 128 x 256 tiles: the projection's 47 MB (2531 rows) are
 // neither written nor read again.

@@ -531,7 +531,7 @@ class Phi3VModel(DecoderModel):
             f8_w = self.w8.get(k_w)                             # the same on e4m3 weights and quantised rows
             if (f8_w is not None and L > ops.L.DECODE_MAX_L and n_beam == 1 and k_w not in self.adapters and not mlx4_first and self.fp8_act
                     and ops.gemm_fp8_ok(M, f8_w[0].shape[0], cfg.hidden_size, EPI_NONE) and os.environ.get("P3V_QKV_FUSE", "1") != "0"
-                    and ops.gemm_qkv_fp8_pays(M, nh * hd, nkv * hd, cfg.hidden_size)
+                    and ops.gemm_qkv_fp8_pays(M, nh * hd, nkv * hd, cfg.hidden_size, stored=bool(st.quantized))
                     and not (st.quantized and past > 0 and not getattr(st, "fresh_rows", False))):
                 kd, vd = (st.k_tmp, st.v_tmp) if st.quantized else (st.k[i], st.v[i])
                 a8, sa = ops.quant_fp8_rows(h if normed_in else x, None if normed_in else w[p + "input_layernorm.weight"], eps)
@@ -570,7 +570,9 @@ class Phi3VModel(DecoderModel):
                 else:                                           # prefill: exact attention, quantised copy stored
                     if past > 0 and not getattr(st, "fresh_rows", False):   # long cached call (constrain with > 16 tokens): attend on a
                         ops.kv_dequantize(st.k8[i], st.v8[i], st.ks[i], st.vs[i], st.k_tmp, st.v_tmp, past)   # dequantised copy
-                    if not fused_qkv:
+                    stored = not fused_qkv and ops.rope_kv_quantize(qkv, st.cos, st.sin, q, st.k_tmp, st.v_tmp, st.k8[i], st.v8[i], st.ks[i], st.vs[i], B, L,
+                                                                    nh, nkv, hd, past, st.Tp, st.T, 1, q_scale=scale * ops.Q_PRESCALE)
+                    if not fused_qkv and not stored:
                         ops.rope_kv_append(qkv, st.cos, st.sin, q, st.k_tmp, st.v_tmp, B, L, nh, nkv, hd, past, st.Tp, True, st.T, 1,
                                            q_scale=scale * ops.Q_PRESCALE)
                     if last_only and i == cfg.num_hidden_layers - 1 and L >= self.TAIL_MIN_L:
@@ -578,7 +580,8 @@ class Phi3VModel(DecoderModel):
                     else:
                         ops.attention(q, o, B, L, nh, nkv, hd, scale, True, past=past, k_past=st.k_tmp, v_past=st.v_tmp,
                                       past_t=st.Tp, pad_len=st.pad_len, new_is_cache=True, q_prescaled=True)
-                    ops.kv_quantize(st.k_tmp, st.v_tmp, st.k8[i], st.v8[i], st.ks[i], st.vs[i], past, L)
+                    if not stored:
+                        ops.kv_quantize(st.k_tmp, st.v_tmp, st.k8[i], st.v8[i], st.ks[i], st.vs[i], past, L)
             elif n_beam > 1:
                 ops.rope_kv_append(qkv, st.cos, st.sin, q, k_new, v_new, B, L, nh, nkv, hd, past, Lp, False, st.T, n_beam)
                 ops.attention(q, o, B, L, nh, nkv, hd, scale, True, k_new=k_new, v_new=v_new, new_t=Lp, past=past,

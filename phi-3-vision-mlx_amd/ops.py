@@ -545,9 +545,10 @@ def gemm_qkv_fp8(a8, a_scale, w8, w_scale, cos_t, sin_t, q_out, k_dst, v_dst, B,
     return True
 
 
-def gemm_qkv_fp8_pays(M, n_q, n_kv, K):
-    """Whether gemm_qkv_fp8 is faster than the two calls it stands for (n_q, n_kv: weight rows per region)."""
-    return bool(L.lib().p3v_gemm_qkv_fp8_pays(M, n_q, n_kv, K))
+def gemm_qkv_fp8_pays(M, n_q, n_kv, K, stored=False):
+    """Whether gemm_qkv_fp8 is faster than the two calls it stands for (n_q, n_kv: weight rows per region).  stored: than gemm_fp8 and
+    rope_kv_quantize, where it would need kv_quantize behind it."""
+    return bool((L.lib().p3v_gemm_qkv_fp8_stored_pays if stored else L.lib().p3v_gemm_qkv_fp8_pays)(M, n_q, n_kv, K))
 
 
 Q_PRESCALE = 1.4426950408889634          # log2(e): q_scale = Q_PRESCALE * softmax scale for q_prescaled attention
@@ -612,6 +613,17 @@ def kv_quantize(k, vt, k8, v8t, k_scale, v_scale, t0, n_tok):
     B, nkv, src_t, hd = k.shape
     L.check(L.lib().p3v_kv_quantize(_p(k), _p(vt), _p(k8), _p(v8t), _p(k_scale), _p(v_scale), B * nkv, hd, src_t,
                                     k8.shape[2], int(t0), int(n_tok), _stream()), "kv_quantize")
+
+
+def rope_kv_quantize(qkv, cos_t, sin_t, q_out, k_dst, v_dst, k8, v8t, k_scale, v_scale, B, Lq, nh, nkv, hd, past, dst_t, tab_t=0, tab_div=1, q_scale=1.0):
+    """rope_kv_append at columns past .. and kv_quantize of those tokens in one launch; False -- nothing launched -- for a shape the library does not
+    take (include/p3v.h: p3v_rope_kv_quantize)."""
+    rc = L.lib().p3v_rope_kv_quantize(_p(qkv), _p(cos_t), _p(sin_t), _p(q_out), _p(k_dst), _p(v_dst), _p(k8), _p(v8t), _p(k_scale), _p(v_scale), B, Lq, nh,
+                                      nkv, hd, int(past), dst_t, tab_t, tab_div, float(q_scale), _stream())
+    if rc == L.ERR_UNSUPPORTED:
+        return False
+    L.check(rc, "rope_kv_quantize")
+    return True
 
 
 def kv_quantize_mlx4(k, vt, k4, v4, k_sb, v_sb, n_tok, qkv=None, cos_t=None, sin_t=None, nh=0, past=0, tab_t=0, tab_div=1):

@@ -2276,6 +2276,31 @@ def test_rmsnorm_widths(ops, orc, rows, H):
     test_rmsnorm(ops, orc, rows, H)
 
 
+@pytest.mark.parametrize("B,L,nh,nkv,past", [(1, 32, 32, 32, 0), (1, 63, 8, 2, 8), (2, 64, 5, 5, 0), (3, 65, 4, 1, 64), (1, 137, 32, 32, 0), (2, 200, 33, 3, 16)])
+def test_rope_kv_quantize_is_the_two_calls(ops, B, L, nh, nkv, past):
+    """p3v_rope_kv_quantize against p3v_rope_kv_append + p3v_kv_quantize: queries, appended rows, codes and scales bit for bit, everything else in both
+    caches untouched; token tiles short of, at and past 64, heads that do not fill a pass of rows, rows of zeros, of tiny and of huge values."""
+    Tp, T = (past + L + 9 + 63) // 64 * 64, past + L + 5
+    qkv = g((B * L, (nh + 2 * nkv) * 96), 700).cuda()
+    qkv[0], qkv[1], qkv[2], qkv[3, ::7] = 0, qkv[1] * 1e-36, qkv[2] * 1e36, 300.0
+    cos, sin = torch.rand((B, T, 48), device="cuda"), torch.rand((B, T, 48), device="cuda")
+
+    def fresh():
+        return [torch.full((B, nh, L, 96), 7.0, dtype=BF16, device="cuda"), g((B, nkv, Tp, 96), 701).cuda(), g((B, nkv, 96, Tp), 702).cuda(),
+                torch.full((B, nkv, Tp, 96), 9, dtype=torch.uint8, device="cuda"), torch.full((B, nkv, 96, Tp), 9, dtype=torch.uint8, device="cuda"),
+                torch.full((B, nkv, Tp), 5.0, device="cuda"), torch.full((B, nkv, Tp), 5.0, device="cuda")]
+    two, one = fresh(), fresh()
+    ops.rope_kv_append(qkv, cos, sin, *two[:3], B, L, nh, nkv, 96, past, Tp, True, T, 1, q_scale=1.3)
+    ops.kv_quantize(*two[1:], past, L)
+    assert ops.rope_kv_quantize(qkv, cos, sin, *one, B, L, nh, nkv, 96, past, Tp, T, 1, q_scale=1.3)
+    for i, (a, b) in enumerate(zip(one, two)):
+        assert torch.equal(a, b), (i, (a != b).sum())
+    kept = [t.clone() for t in one]
+    assert not ops.rope_kv_quantize(qkv, cos, sin, *one, 1, 31, nh, nkv, 96, past, Tp, T, 1)      # few tokens, an odd column: nothing is launched
+    assert not ops.rope_kv_quantize(qkv, cos, sin, *one, B, L, nh, nkv, 96, past + 4, Tp, T, 1)
+    assert all(torch.equal(a, b) for a, b in zip(one, kept))
+
+
 @pytest.mark.parametrize("narrow", [None, "0", "1"])
 @pytest.mark.parametrize("epi,M,N,K", [("none", 300, 512, 384), ("none", 2531, 9216, 3072), ("resid", 2531, 3072, 8192),
                                        ("silu", 700, 1024, 3072), ("resid", 17, 256, 128), ("none", 513, 384, 256)])
