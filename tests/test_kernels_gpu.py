@@ -1874,6 +1874,31 @@ def test_argmax_logsoftmax_topk(ops, orc):
     assert tk.tolist() == orc.top3_candidates(x, 3).tolist()
 
 
+@pytest.mark.parametrize("n", [8, 16, 1000, 8184, 8192, 8200, 32064, 32768, 40008, 65544])
+def test_argmax_by_pieces(ops, n):
+    """Rows of fewer pieces of 8 than threads, exactly four a thread, and several turns of four: the largest at either end and anywhere, ties (a neighbour, another
+    piece of the same thread, another turn) to the first, zeros of both signs, a row of -inf, one of NaNs and one behind the largest."""
+    rng = np.random.default_rng(n)
+    rows, want = [], []
+    for at in [0, n - 1] + [int(v) for v in rng.integers(0, n, 6)]:
+        x = g((n,), 78 + at).clamp(-3, 3)
+        x[at] = 4.0
+        rows.append(x), want.append(at)
+        for gap in (1, 8192, 32768):
+            if at + gap < n:
+                y = x.clone()
+                y[at + gap] = 4.0
+                rows.append(y), want.append(at)
+    zero = torch.zeros(n, dtype=BF16)
+    zero[: n // 2] = -0.0
+    rows += [zero, torch.full((n,), float("-inf"), dtype=BF16), torch.full((n,), float("nan"), dtype=BF16)]
+    want += [0, 0, -1]
+    bad = rows[0].clone()
+    bad[n - 1] = float("nan")
+    rows.append(bad), want.append(-1)
+    assert ops.argmax(torch.stack(rows).cuda()).tolist() == want
+
+
 def test_argmax_reports_nan_rows(ops):
     """A NaN anywhere in a row makes its arg-max -1 (the host loops raise on it), other rows are unaffected."""
     from phi_3_vision_mlx_amd.api import _rows
