@@ -1698,6 +1698,35 @@ def test_kv_quantize_and_q8_decode(ops, orc, past, L, n_split, fused):
     assert (v8.cpu()[:, :, :, past].float() - (torch.round(x[:, 2 * nh:, 0].float() / (x[:, 2 * nh:, 0].float().abs().amax(-1, keepdim=True) / 127)) + 128)).abs().max() <= 1
 
 
+@pytest.mark.parametrize("B,cap,past,L,q8", [(1, 6272, 6100, 1, True), (1, 16384, 16300, 1, True), (3, 4224, 4095, 2, True), (16, 640, 511, 1, True),
+                                             (1, 6272, 6271, 1, False), (1, 8192, 8064, 3, False)])
+def test_decode_attention_with_a_tile_of_128_keys_each_on_long_caches(ops, B, cap, past, L, q8):
+    """As many splits as tiles of 128 keys, up to the 128 a call may have, merged by a launch and -- up to 48 -- inside, against the walking kernel
+    on few splits: the same output within the rounding of its probabilities (the maxima they are rounded against differ), the same appended rows."""
+    nh, hd = 4, 96
+    rng = torch.Generator("cuda").manual_seed(past)
+    qkv = g((B * L, 3 * nh * hd), 190).cuda()
+    cos, sin = torch.rand((B, L, hd // 2), device="cuda", generator=rng), torch.rand((B, L, hd // 2), device="cuda", generator=rng)
+    pad = torch.tensor([0, 700, 131] * 6, dtype=torch.int32)[:B].clamp(max=past // 2).cuda()
+
+    def caches():
+        r = torch.Generator("cuda").manual_seed(7)
+        if q8:
+            return [torch.randint(1, 256, s, dtype=torch.uint8, device="cuda", generator=r) for s in ((B, nh, cap, hd), (B, nh, hd, cap))] + \
+                   [torch.rand((B, nh, cap), device="cuda", generator=r) * 0.01 + 0.01 for _ in range(2)]
+        return [torch.randn(s, device="cuda", generator=r).to(BF16) for s in ((B, nh, cap, hd), (B, nh, hd, cap))]
+    outs = []
+    for n_split, fused in [(5, False), (cap // 128, False)] + ([(cap // 128, True)] if cap // 128 <= 48 else []):
+        c, out, ws = caches(), torch.full((B, L, nh * hd), float("nan"), dtype=BF16, device="cuda"), ops.attention_ws(B, L, nh, hd, n_split, "cuda")
+        (ops.attention_decode_q8 if q8 else ops.attention_decode)(qkv, cos, sin, L, *c, out, B, L, nh, nh, hd, hd ** -0.5, past, cap, ws, n_split, pad_len=pad,
+                                                                  merge_in_launch=fused)
+        assert (ws.view(torch.int32) == -1).all()
+        outs.append((out, c))
+    for out, c in outs[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(c, outs[0][1]))
+        close(out, outs[0][0], rtol=2 ** -6, atol=2 ** -6 * outs[0][0].float().abs().max().item())
+
+
 @pytest.mark.parametrize("past,cap,dev_past", [(2531, 2688, True), (300, 1664, False)])
 def test_attention_decode_with_fused_4bit_oproj_is_bit_identical_to_two_launches(ops, past, cap, dev_past):
     """k_attn_decode128_o4: the fused launch on MLX 4-bit group-64 o_proj weights (the reference's quantize_model format, device
