@@ -452,14 +452,15 @@ class Phi3VModel(DecoderModel):
             # next 24 KB tile in flight) walking several tiles
             tiles = -(-T // 64)
             tiles128 = T // 128 if T % 128 == 0 else 0           # T is the cache CAPACITY when the plan is for a captured graph
-            if tiles128 and (tiles128 <= 128 and (tiles > 16 or B * nh * tiles > 4096) if quantized else tiles > 16 and tiles128 <= 64 and B * nh * tiles128 <= 2048) \
+            if tiles128 and (tiles128 <= 128 and (tiles > 16 or B * nh * tiles > 4096) if quantized else tiles > 16 and tiles128 <= 48 and B * nh * tiles128 <= 2048) \
                     and os.environ.get("P3V_ATTN_TILE128", "1") != "0":
                 # one 128-key tile per workgroup (k_attn_decode128): half the partials of 64-key ones to merge; short caches keep 64-key tiles
                 # (more workgroups than CUs matters more).  Four steps, us, this plan : the one behind it (64-key tiles up to 8192 columns, then
-                # the walking kernel).  bf16 cache, one row: 6100 keys 7966 : 8116 (4-bit weights 5486 : 5605), 7000 8130 : 8447, but 8064 8458 : 8367 and
-                # 12000 9465 : 9238 -- up to 64 tiles.  int8 cache, whose walking kernel takes its bytes through registers: 6100 5523 : 6840, 7000 5613 : 7113,
-                # 8064 5818 : 6117, 16000 7174 : 8192; 2 rows 4000 8655 : 9071, 4 rows 2000 8803 : 9446, 8 rows 1000 8541 : 9061, 2500 10381 : 11162,
-                # 16 rows 500 11007 : 11799.  (Merged by a launch of its own beyond 48 splits or 4096 workgroups.)
+                # the walking kernel).  int8 cache, whose walking kernel takes its bytes through registers: 6100 keys 5523 : 6840, 7000 5613 : 7113, 8064 5818 :
+                # 6117, 16000 7174 : 8192; 2 rows 4000 8655 : 9071, 4 rows 2000 8803 : 9446, 8 rows 1000 8541 : 9061, 2500 10381 : 11162, 16 rows 500 11007 : 11799,
+                # the same error against 64 bits.  bf16 cache beyond 48 tiles: 7000 keys 8130 : 8447 (8064 8458 : 8367), but 64-key tiles, whose maxima
+                # carry more of the probabilities exactly, are 3 % nearer to 64 bits (0.00174 : 0.00179).  (Merged by a launch of its own beyond 48 splits or, of more
+                # than 4, 4096 workgroups.)
                 n_split = tiles128
             elif tiles <= 128 and B * nh * tiles <= 4096:
                 n_split = tiles
@@ -476,7 +477,7 @@ class Phi3VModel(DecoderModel):
             # layer, the in-launch merge 0.5; with 24 splits at B = 1 / 32k the one merging workgroup per head is the slower
             # way: +1.6 % per step, +4.5 % at 8k)
             mode = os.environ.get("P3V_ATTN_FUSED_MERGE", "1")
-            fused = (n_split in (tiles, tiles128) or n_split <= 4 or mode == "2") and n_split <= 48 and B * nh * n_split <= 4096 and mode != "0"
+            fused = (n_split in (tiles, tiles128) or n_split <= 4 or mode == "2") and n_split <= 48 and (n_split <= 4 or B * nh * n_split <= 4096) and mode != "0"
             # The merging workgroup of a (row, head) waits -- bounded, NaN-poisoned on expiry -- for partials of workgroups that
             # the hardware dispatches before it (linear order; observed, not documented).  When the whole grid is resident at once
             # (128-key tiles: 3 workgroups per CU, 64-key: 5) nothing depends on that order.  A server takes the separate merge
