@@ -284,10 +284,12 @@ typedef struct {
   int new_is_cache;         /* 1: (k_new,v_new) ignored, rows [past,past+L) are read from (k_past,v_past) too --
                                used with d_past, when the append offset is only known on the device */
   int q_prescaled;          /* 1: q already carries scale * log2(e) (p3v_rope_kv_append's q_scale); `scale` is then unused */
-  int any_order;            /* 1: a query's keys may be summed in parts (prompts of few workgroups): as exact, rounded otherwise.  For callers whose
-                               next projection does not quantise its activations: 8-bit steps carry such a rounding to per cents of a logit */
 } p3v_attn_args_t;
 int p3v_attention(const p3v_attn_args_t* args /* host */, void* stream);
+/* the same where a query's keys may be summed in parts (prompts of few workgroups): as exact, rounded otherwise.  For callers whose next projection does
+ * not quantise its activations: 8-bit steps carry such a rounding to per cents of a logit.  (An entry point, not a field: the struct ends as callers
+ * built against earlier headers have it, and its last four bytes are padding in their hands.) */
+int p3v_attention_any_order(const p3v_attn_args_t* args /* host */, void* stream);
 /* bytes of workspace p3v_attention needs for the decode (L<=P3V_DECODE_MAX_L) path */
 int64_t p3v_attention_ws_bytes(int B, int L, int n_heads, int hd, int n_split);
 #define P3V_DECODE_MAX_L 16

@@ -67,7 +67,7 @@ class AttnArgs(C.Structure):
                 ("pad_len", vp), ("d_past", vp), ("ws", vp),
                 ("B", i32), ("L", i32), ("n_heads", i32), ("n_kv", i32), ("hd", i32),
                 ("past", i32), ("past_t", i32), ("past_div", i32), ("new_t", i32), ("pad_div", i32),
-                ("causal", i32), ("scale", f32), ("n_split", i32), ("new_is_cache", i32), ("q_prescaled", i32), ("any_order", i32)]
+                ("causal", i32), ("scale", f32), ("n_split", i32), ("new_is_cache", i32), ("q_prescaled", i32)]
 
 
 class GemvQ4Args(C.Structure):
@@ -143,6 +143,7 @@ SIGNATURES = {
     "p3v_rope_table": (i32, [vp, vp, f32, vp, vp, i32, i32, vp]),
     "p3v_rope_kv_append": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp, i32, i32, i32, i32, f32, vp]),
     "p3v_attention": (i32, [C.POINTER(AttnArgs), vp]),
+    "p3v_attention_any_order": (i32, [C.POINTER(AttnArgs), vp]),
     "p3v_attention_decode": (i32, [C.POINTER(AttnDecArgs), vp]),
     "p3v_attention_decode_can_fuse_oproj": (i32, [i32, i32, i32, i32, i32, i32, i32, i32]),
     "p3v_attention_decode_rows_fit": (i32, [i32, i32, i32, i32, i32]),

@@ -1358,7 +1358,7 @@ extern "C" int64_t p3v_attention_ws_bytes(int B, int L, int n_heads, int hd, int
   return (int64_t)B * n_heads * n_split * 16 * (hd + 2) * 4;
 }
 
-extern "C" int p3v_attention(const p3v_attn_args_t* a, void* stream) {
+static int attention(const p3v_attn_args_t* a, int any_order, void* stream) {
   if (!a || !a->q || !a->out) return P3V_ERR_ARG;
   if (a->new_is_cache ? (!a->k_past || !a->v_past) : (!a->k_new || !a->v_new)) return P3V_ERR_ARG;
   if (a->hd != 64 && a->hd != 96) return P3V_ERR_UNSUPPORTED;
@@ -1373,7 +1373,7 @@ extern "C" int p3v_attention(const p3v_attn_args_t* a, void* stream) {
   p.past_div = a->past_div > 0 ? a->past_div : 1; p.new_t = a->new_t; p.pad_div = a->pad_div > 0 ? a->pad_div : 1;
   p.causal = a->causal; p.scale = a->scale;
   p.q_prescaled = a->q_prescaled != 0;
-  p.any_order = a->any_order != 0;
+  p.any_order = any_order;
   p.sc2 = p.q_prescaled ? 1.f : a->scale * 1.4426950408889634f;
   p.n_split = a->n_split;
   p.split_mode = (a->L <= P3V_DECODE_MAX_L && a->n_split > 1) ? 1 : 0;
@@ -1393,6 +1393,8 @@ extern "C" int p3v_attention(const p3v_attn_args_t* a, void* stream) {
   }
   return P3V_OK;
 }
+extern "C" int p3v_attention(const p3v_attn_args_t* a, void* stream) { return attention(a, 0, stream); }
+extern "C" int p3v_attention_any_order(const p3v_attn_args_t* a, void* stream) { return attention(a, 1, stream); }
 
 // =====================================================================================
 // Fused decode step attention (L <= 16 new tokens, n_beam == 1):

@@ -560,11 +560,11 @@ def attention(q, out, B, Lq, nh, nkv, hd, scale, causal, k_new=None, v_new=None,
     """softmax((q*scale) k^T + mask) v (phi.py:454-457 / phi.py:148), mask never materialised.
     K tensors are [B, nkv, t, hd]; V tensors are TRANSPOSED [B, nkv, hd, t] (t = past_t / new_t).
     q_prescaled: q already carries scale * log2(e) (rope_kv_append's q_scale = Q_PRESCALE * scale).  any_order: keys may be summed in
-    parts (include/p3v.h)."""
+    parts (include/p3v.h: p3v_attention_any_order)."""
     args = L.AttnArgs(_p(q), _p(k_past), _p(v_past), _p(k_new), _p(v_new), _p(out), _p(pad_len), _p(d_past), _p(ws),
                       B, Lq, nh, nkv, hd, int(past), past_t, past_div, new_t, pad_div, int(causal), float(scale), n_split, int(new_is_cache),
-                      int(bool(q_prescaled)), int(bool(any_order)))
-    L.check(L.lib().p3v_attention(C.byref(args), _stream()), "attention")
+                      int(bool(q_prescaled)))
+    L.check((L.lib().p3v_attention_any_order if any_order else L.lib().p3v_attention)(C.byref(args), _stream()), "attention")
     return out
 
 

@@ -691,6 +691,39 @@ def test_attention_prefill_two_key_groups(ops, orc, B, L, past, hd, nh, causal, 
     _prefill_case(ops, orc, B, L, past, hd, nh, causal, pads, True, 2, il_waves=42, spike=spike)
 
 
+def _attention_rows(ops, B, L, past, nh, causal, fn="p3v_attention", tail=0):
+    """p3v_attention of pre-scaled queries on a cache of random keys, through the C entry `fn`; tail: the byte in the struct's last four, behind its last field."""
+    import ctypes
+    lib, Tp = ops.L, (past + L + 63) // 64 * 64
+    q, k, v = g((B, nh, L, 96), 140, 0.2).cuda(), g((B, nh, Tp, 96), 141).cuda(), g((B, nh, 96, Tp), 142).cuda()
+    out = torch.full((B, L, nh * 96), float("nan"), dtype=BF16, device="cuda")
+    a = lib.AttnArgs(q.data_ptr(), k.data_ptr(), v.data_ptr(), None, None, out.data_ptr(), None, None, None, B, L, nh, nh, 96, past, Tp, 1, 0, 1, int(causal), 1.0, 0, 1, 1)
+    end = lib.AttnArgs.q_prescaled.offset + 4
+    assert ctypes.sizeof(a) == end + 4
+    ctypes.memset(ctypes.addressof(a) + end, tail, 4)
+    lib.check(getattr(lib.lib(), fn)(ctypes.byref(a), torch.cuda.current_stream().cuda_stream), fn)
+    return out
+
+
+def test_attention_reads_nothing_behind_its_arguments_last_field(ops):
+    """The four bytes behind q_prescaled are padding to a caller whose struct ends there: what they hold changes nothing, not even the order of a sum."""
+    assert torch.equal(_attention_rows(ops, 1, 800, 0, 8, True), _attention_rows(ops, 1, 800, 0, 8, True, tail=0xff))
+
+
+@pytest.mark.parametrize("B,L,past,nh,causal,two", [
+    (1, 640, 63, 8, True, False), (1, 640, 64, 8, True, True), (1, 704, 0, 8, True, True),                  # from 704 keys on
+    (1, 1152, 0, 32, True, True), (1, 1153, 0, 32, True, False), (2, 512, 200, 32, True, True), (2, 513, 200, 32, True, False),      # workgroups: 288 of one row, 256 of several
+    (1, 800, 0, 8, False, False)])
+def test_which_prompts_attend_by_two_key_groups(ops, request, B, L, past, nh, causal, two):
+    """p3v_attention_any_order inside the limits: the bits of the pinned kernel with two key groups; outside them, and p3v_attention anywhere: its own."""
+    own, free = _attention_rows(ops, B, L, past, nh, causal), _attention_rows(ops, B, L, past, nh, causal, "p3v_attention_any_order")
+    old = ops.set_tuning("attn_il_waves", 42)
+    request.addfinalizer(lambda: ops.set_tuning("attn_il_waves", old))
+    pinned = _attention_rows(ops, B, L, past, nh, causal)
+    assert torch.isfinite(own.float()).all() and not torch.equal(own, pinned)
+    assert torch.equal(free, pinned if two else own)
+
+
 @pytest.mark.parametrize("prescaled", [True, False], ids=["prescaled", "plain"])
 @pytest.mark.parametrize("B,L,past,hd,nh,causal,pads", [
     (1, 128, 0, 96, 2, True, None), (1, 65, 0, 96, 2, True, None), (1, 17, 0, 96, 1, True, None), (2, 200, 0, 96, 2, True, [0, 131]),
