@@ -135,6 +135,13 @@ class Phi3VModel(DecoderModel):
         ops.lora_down(x, a, out=t)
         return ops.lora_up(y, t, b, scale, epilogue, resid=resid, out=out)
 
+    def _quantises_rows(self, key, M, epilogue=EPI_NONE):
+        """Whether the projection `key` of M rows quantises them first (W8A8 on the fp8 matrix cores)."""
+        if key not in self.w8 or not self.fp8_act:
+            return False
+        N, K = self.w8[key][0].shape
+        return not (M <= 8 or (M <= ops.GEMV_MAX_M and K % 512 == 0)) and ops.gemm_fp8_ok(M, N, K, epilogue)
+
     def _proj_frozen(self, x, key, epilogue=EPI_NONE, resid=None, norm_w=None, out=None, h=None):
         """Weight-streaming kernel for skinny x, MFMA GEMM otherwise; bf16 or fp8 weights."""
         eps = self.cfg.rms_norm_eps
@@ -156,7 +163,7 @@ class Phi3VModel(DecoderModel):
             return ops.gemv_q4(x, q4[0], q4[1], epilogue, resid=resid, norm_w=norm_w, norm_eps=eps, out=out)
         if q is not None and skinny and K in (3072, 8192):
             return ops.gemv_fp8(x, q[0], q[1], epilogue, resid=resid, norm_w=norm_w, norm_eps=eps, out=out)
-        if q is not None and not skinny and self.fp8_act and ops.gemm_fp8_ok(M, q[0].shape[0], K, epilogue):
+        if self._quantises_rows(key, M, epilogue):
             # prompt-sized input: W8A8 on the fp8 matrix cores, activations quantised per token row (fused with the norm)
             a8, sa = ops.quant_fp8_rows(x, norm_w, eps)
             return ops.gemm_fp8(a8, sa, q[0], q[1], epilogue, resid=resid, out=out)
@@ -495,7 +502,7 @@ class Phi3VModel(DecoderModel):
         position-dependent kernel read the cache length from HBM -> graph-replayable.
         last_only: the caller reads the LAST position only (prefill of generate / choose, Q8): the final layer still builds
         K / V for every position, but its o_proj and MLP run on the B last rows alone (0.4 ms of a 30 ms prefill), and so does its
-        attention behind TAIL_MIN_L tokens; returns [B, H] then."""
+        attention behind TAIL_MIN_L tokens where no projection of theirs quantises its rows; returns [B, H] then."""
         cfg, w = self.cfg, self.w
         nh, nkv, hd, eps = cfg.num_attention_heads, cfg.num_key_value_heads, self.hd, cfg.rms_norm_eps
         M = B * L
@@ -517,6 +524,10 @@ class Phi3VModel(DecoderModel):
             k_new = torch.empty((B, nkv, Lp, hd), dtype=BF16, device=self.device)
             v_new = torch.zeros((B, nkv, hd, Lp), dtype=BF16, device=self.device)
         normed_in = False                                       # `h` already holds the layer's normalised input
+        # (the last rows' keys are summed in parts: not in front of a row quantiser, see p3v_attention_any_order)
+        end = f"model.layers.{cfg.num_hidden_layers - 1}."
+        tail = last_only and L >= self.TAIL_MIN_L and not any(
+            self._quantises_rows(end + k, B, e) for k, e in (("self_attn.o_proj.weight", EPI_RESID_BF16), ("mlp.gate_up_proj.weight", EPI_SILU_MUL), ("mlp.down_proj.weight", EPI_RESID_BF16)))
         for i in range(cfg.num_hidden_layers):
             p = f"model.layers.{i}."
             # Prompt-sized calls on bf16 weights: the qkv projection writes rotated Q, the K cache rows and the V^T cache columns from
@@ -580,7 +591,7 @@ class Phi3VModel(DecoderModel):
                     if not fused_qkv and not stored:
                         ops.rope_kv_append(qkv, st.cos, st.sin, q, st.k_tmp, st.v_tmp, B, L, nh, nkv, hd, past, st.Tp, True, st.T, 1,
                                            q_scale=scale * ops.Q_PRESCALE)
-                    if last_only and i == cfg.num_hidden_layers - 1 and L >= self.TAIL_MIN_L:
+                    if tail and i == cfg.num_hidden_layers - 1:
                         o = self._attend_last(q, st.k_tmp, st.v_tmp, B, L, past, st, scale)
                     else:
                         ops.attention(q, o, B, L, nh, nkv, hd, scale, True, past=past, k_past=st.k_tmp, v_past=st.v_tmp,
@@ -618,7 +629,7 @@ class Phi3VModel(DecoderModel):
                 if not fused_qkv:
                     ops.rope_kv_append(qkv, st.cos, st.sin, q, st.k[i], st.v[i], B, L, nh, nkv, hd, past, st.Tp, True, st.T, 1,
                                        q_scale=scale * ops.Q_PRESCALE)
-                if last_only and i == cfg.num_hidden_layers - 1 and L >= self.TAIL_MIN_L:
+                if tail and i == cfg.num_hidden_layers - 1:
                     o = self._attend_last(q, st.k[i], st.v[i], B, L, past, st, scale)
                 else:
                     ops.attention(q, o, B, L, nh, nkv, hd, scale, True, past=past, k_past=st.k[i], v_past=st.v[i],

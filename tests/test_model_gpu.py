@@ -387,6 +387,23 @@ def test_last_rows_attention_of_a_prompt(kw, monkeypatch):
     assert all(torch.equal(a, b) for a, b in zip(got[40][3:], got[10 ** 9][3:]))
 
 
+@pytest.mark.parametrize("B,quantised", [(2, False), (16, False), (17, True)])
+def test_last_rows_attention_stays_out_of_8bit_projections(B, quantised, monkeypatch):
+    """e4m3 weights: while the last rows' projections stream the weights they attend alone, the same logits; from 17 rows on these projections quantise their
+    rows, whose attention is then that of all rows, bit for bit."""
+    from phi_3_vision_mlx_amd.api import load_synthetic
+    model, _ = load_synthetic(blind_model=True, tiny=False, seed=3, device="cuda:0", num_hidden_layers=2, quantized_fp8=True)
+    ids, got, calls = np.concatenate([rand_ids(140, 60 + i) for i in range(B)]), {}, []
+    own = type(model)._attend_last
+    monkeypatch.setattr(type(model), "_attend_last", lambda self, *a: calls.append(1) or own(self, *a))
+    for n in (10 ** 9, 40):
+        monkeypatch.setattr(type(model), "TAIL_MIN_L", n)
+        got[n] = model(input_ids=ids, max_tokens=4)[0]
+    assert len(calls) == (0 if quantised else 1)
+    assert_logits(got[40], got[10 ** 9])
+    assert not quantised or torch.equal(got[40], got[10 ** 9])
+
+
 def test_batched_left_pad(text):
     model, proc, oracle = text
     inputs = proc(["a", "hello world, this is a longer prompt", "mid size"])
