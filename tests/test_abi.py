@@ -314,6 +314,11 @@ def test_which_tile_runs_an_fp8_projection():
         for M, n_q, n_kv, K, want in ((256, 3072, 3072, 3072, 0), (577, 3072, 3072, 3072, 1), (768, 3072, 3072, 3072, 1), (1024, 3072, 3072, 3072, 0), (1800, 3072, 3072, 3072, 0), (2048, 3072, 3072, 3072, 0),
                                       (2531, 3072, 3072, 3072, 1), (2700, 3072, 3072, 3072, 0), (4096, 3072, 3072, 3072, 1), (6000, 3072, 3072, 3072, 1), (8192, 3072, 3072, 3072, 1), (16384, 3072, 3072, 3072, 1), (2531, 1024, 1024, 1024, 1), (1536, 768, 768, 384, 1)):
             assert l.p3v_gemm_qkv_fp8_pays(M, n_q, n_kv, K) == want, (M, n_q, n_kv, K)
+        # (in front of p3v_rope_kv_quantize: the faster side of whole prompts run either way, by 5 us a layer or more)
+        for M, want in ((137, 0), (276, 0), (803, 0), (1024, 0), (1800, 0), (2300, 0), (2700, 0), (3300, 0), (3900, 0), (4050, 1), (4096, 1), (4500, 0), (4700, 0), (5200, 1),
+                        (6500, 0), (7300, 0), (7600, 0), (7800, 0), (8000, 1), (8192, 0), (10000, 0), (65536, 0), (0, 0)):
+            assert l.p3v_gemm_qkv_fp8_stored_pays(M, 3072, 3072, 3072) == want, M
+        assert l.p3v_gemm_qkv_fp8_stored_pays(4096, 3000, 3072, 3072) == 0
         for M, N, K, epi in ((0, 256, 256, ops.EPI_NONE), (1, 100, 256, ops.EPI_NONE), (1, 256, 64, ops.EPI_NONE), (1, 256, 256, ops.EPI_GELU_MUL)):
             assert l.p3v_gemm_fp8_tile(M, N, K, epi) == 0
     finally:
