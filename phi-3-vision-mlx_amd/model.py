@@ -459,13 +459,16 @@ class Phi3VModel(DecoderModel):
             # next 24 KB tile in flight) walking several tiles
             tiles = -(-T // 64)
             tiles128 = T // 128 if T % 128 == 0 else 0           # T is the cache CAPACITY when the plan is for a captured graph
-            if tiles128 and (tiles128 <= 128 and (tiles > 16 or B * nh * tiles > 4096) if quantized else tiles > 16 and tiles128 <= 48 and B * nh * tiles128 <= 2048) \
+            if tiles128 and (tiles128 <= 128 and B * nh * tiles128 <= 65536 and (tiles > 16 or B * nh * tiles > 4096) if quantized else tiles > 16 and tiles128 <= 48 and B * nh * tiles128 <= 2048) \
                     and os.environ.get("P3V_ATTN_TILE128", "1") != "0":
                 # one 128-key tile per workgroup (k_attn_decode128): half the partials of 64-key ones to merge; short caches keep 64-key tiles
                 # (more workgroups than CUs matters more).  Four steps, us, this plan : the one behind it (64-key tiles up to 8192 columns, then
                 # the walking kernel).  int8 cache, whose walking kernel takes its bytes through registers: 6100 keys 5523 : 6840, 7000 5613 : 7113, 8064 5818 :
-                # 6117, 16000 7174 : 8192; 2 rows 4000 8655 : 9071, 4 rows 2000 8803 : 9446, 8 rows 1000 8541 : 9061, 2500 10381 : 11162, 16 rows 500 11007 : 11799,
-                # the same error against 64 bits.  bf16 cache beyond 48 tiles: 7000 keys 8130 : 8447 (8064 8458 : 8367), but 64-key tiles, whose maxima
+                # 6117, 16000 7174 : 8192; 2 rows 4000 8655 : 9071, 4 rows 2000 8803 : 9446, 8 rows 1000 8541 : 9061, 2500 10381 : 11162, 16 rows 500 11007 : 11799.
+                # Attention and merge of one layer, launch behind launch, up to the 65536 workgroups where the rule ends: 4 rows of 8000 49 : 57, 16000 87 : 114; 8 of
+                # 4000 50 : 57, 16000 163 : 220; 16 of 1000 32 : 43, 4000 91 : 134, 16000 324 : 547; 32 of 600 44 : 54, 2500 114 : 150; 64 of 500 63 : 72, 1000 103 : 124;
+                # none of 33 sizes slower.  Its partials take 6 KB a workgroup -- 0.8 % of 32 layers' cache, 389 MB for 16 rows of 16000 where the walking kernel's take
+                # 9.  Error against 64 bits: the walking kernel's or less (16 rows of 16000 0.00167 : 0.00173).  bf16 cache beyond 48 tiles: 7000 keys 8130 : 8447 (8064 8458 : 8367), but 64-key tiles, whose maxima
                 # carry more of the probabilities exactly, are 3 % nearer to 64 bits (0.00174 : 0.00179).  (Merged by a launch of its own beyond 48 splits or, of more
                 # than 4, 4096 workgroups.)
                 n_split = tiles128

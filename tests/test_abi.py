@@ -357,6 +357,19 @@ def test_which_decode_batches_run_one_workgroup_per_row_and_head():
         assert fit(*no) == 0, no
 
 
+@pytest.mark.parametrize("B,T,n_split", [(1, 6272, 49), (1, 16384, 128), (1, 16512, 40), (8, 2688, 21), (16, 16256, 127), (32, 8064, 63), (32, 8192, 64), (64, 4096, 32), (64, 4224, 1),
+                                         (32, 8320, 2), (64, 16256, 1), (512, 640, 1)])
+def test_how_many_workgroups_attend_an_int8_cache(monkeypatch, B, T, n_split):
+    """A 128-key tile a workgroup as far as that was measured, 65536 workgroups and their partials; the walking kernel's few splits beyond, however many rows."""
+    from types import SimpleNamespace
+    from phi_3_vision_mlx_amd import model, ops
+    monkeypatch.delenv("P3V_ATTN_NSPLIT", raising=False), monkeypatch.delenv("P3V_ATTN_TILE128", raising=False)
+    monkeypatch.setattr(ops, "attention_ws", lambda B, L, nh, hd, n, dev: ops.attention_ws_bytes(B, L, nh, hd, n))
+    bufs = {}
+    model.Phi3VModel._split_plan(SimpleNamespace(cfg=SimpleNamespace(num_attention_heads=32), hd=96, device="cpu"), bufs, B, 1, T, quantized=True)
+    assert bufs["n_split"] == n_split and bufs["ws"] <= 65536 * 16 * 98 * 4
+
+
 def test_fused_qkv_projections_decline_several_rows_of_fewer_than_seven_tokens():
     """The V^T epilogue's runs of eight tokens cross the end of one batch row at most.  Everything else about these calls is taken, so
     the answer comes from that check (no kernel starts: declined on the host)."""
