@@ -297,10 +297,10 @@ def test_which_tile_runs_an_fp8_projection():
     assert l.p3v_get_tuning(b"gemm_f8_narrow", ctypes.byref(v)) == 0
     try:
         for K in (256, 384, 640, 3200):
-            for tile in (44, 54, 42, 43, 64, 74, 84):
+            for tile in (44, 54, 42, 43, 64, 74, 84, 32, 22, 21, 11):
                 assert l.p3v_set_tuning(b"gemm_f8_narrow", tile) == 0
                 assert l.p3v_gemm_fp8_tile(1300, 9216, K, ops.EPI_NONE) == tile, (K, tile)
-                if tile != 43:
+                if tile % 2 == 0:
                     assert l.p3v_gemm_fp8_tile(1300, 8192, K, ops.EPI_SILU_MUL) == tile, (K, tile)
         assert l.p3v_set_tuning(b"gemm_f8_narrow", 43) == 0
         free = l.p3v_gemm_fp8_tile(1300, 4096, 384, ops.EPI_NONE)
@@ -309,7 +309,10 @@ def test_which_tile_runs_an_fp8_projection():
         for M, N, K, epi, want in ((1300, 4096, 384, ops.EPI_NONE, 44), (768, 9216, 640, ops.EPI_NONE, 44), (1300, 9216, 640, ops.EPI_NONE, 64), (1300, 9216, 3200, ops.EPI_NONE, 64),
                                    (1024, 9216, 3072, ops.EPI_NONE, 54), (320, 9216, 3072, ops.EPI_NONE, 42), (2531, 9216, 3072, ops.EPI_NONE, 64),
                                    (2531, 8192, 3072, ops.EPI_SILU_MUL, 74), (2048, 8192, 2944, ops.EPI_SILU_MUL, 84), (2531, 3072, 8192, ops.EPI_RESID_BF16, 44),
-                                   (4096, 3072, 3072, ops.EPI_RESID_BF16, 74)):
+                                   (4096, 3072, 3072, ops.EPI_RESID_BF16, 74),
+                                   (137, 3072, 8192, ops.EPI_RESID_BF16, 11), (276, 3072, 8192, ops.EPI_RESID_BF16, 21), (512, 3072, 8192, ops.EPI_RESID_BF16, 22),
+                                   (803, 3072, 8192, ops.EPI_RESID_BF16, 32), (137, 3072, 3072, ops.EPI_RESID_BF16, 11), (137, 9216, 3072, ops.EPI_NONE, 22),
+                                   (276, 9216, 3072, ops.EPI_NONE, 32), (128, 8192, 3072, ops.EPI_SILU_MUL, 22), (257, 8192, 3072, ops.EPI_SILU_MUL, 44)):
             assert l.p3v_gemm_fp8_tile(M, N, K, epi) == want, (M, N, K, epi, l.p3v_gemm_fp8_tile(M, N, K, epi))
         for M, n_q, n_kv, K, want in ((256, 3072, 3072, 3072, 0), (577, 3072, 3072, 3072, 1), (768, 3072, 3072, 3072, 1), (1024, 3072, 3072, 3072, 0), (1800, 3072, 3072, 3072, 0), (2048, 3072, 3072, 3072, 0),
                                       (2531, 3072, 3072, 3072, 1), (2700, 3072, 3072, 3072, 0), (4096, 3072, 3072, 3072, 1), (6000, 3072, 3072, 3072, 1), (8192, 3072, 3072, 3072, 1), (16384, 3072, 3072, 3072, 1), (2531, 1024, 1024, 1024, 1), (1536, 768, 768, 384, 1)):
@@ -323,6 +326,21 @@ def test_which_tile_runs_an_fp8_projection():
             assert l.p3v_gemm_fp8_tile(M, N, K, epi) == 0
     finally:
         l.p3v_set_tuning(b"gemm_f8_narrow", v.value)
+
+
+def test_which_projections_pay_in_one_pass_and_which_ask_for_more_slices():
+    """p3v_gemm_one_pass_pays: 257 .. 384 rows, more than 128 and at most 256 tiles of 128 x 128, where K slices would run otherwise.  p3v_gemm_ws_most_bytes: up to 256 rows,
+    whole 96 columns, slices of 12 K-tiles, 16 beyond 128 rows; p3v_gemm_ws_bytes where the kernel for 9 .. 32 rows or another takes the shape."""
+    from phi_3_vision_mlx_amd import _lib, ops
+    l = _lib.lib()
+    for M, tiles, K, epi, want in ((300, 42, 3072, ops.EPI_NONE, 0), (300, 43, 3072, ops.EPI_NONE, 1), (300, 85, 3072, ops.EPI_NONE, 1), (300, 86, 3072, ops.EPI_NONE, 0),
+                                   (256, 72, 3072, ops.EPI_NONE, 0), (257, 72, 3072, ops.EPI_NONE, 1), (384, 72, 512, ops.EPI_NONE, 1), (385, 72, 3072, ops.EPI_NONE, 0),
+                                   (300, 72, 3072, ops.EPI_RESID_BF16, 0), (300, 72.5, 3072, ops.EPI_NONE, 0), (300, 72, 3136, ops.EPI_NONE, 0), (0, 72, 3072, ops.EPI_NONE, 0)):
+        assert l.p3v_gemm_one_pass_pays(M, int(tiles * 128), K, epi) == want, (M, tiles, K, epi)
+    for M, N, K, few, most in ((9, 3072, 8192, 4, 4), (32, 3072, 8192, 4, 4), (20, 3072, 6144, 4, 8), (33, 3072, 8192, 4, 8), (128, 3072, 6144, 4, 8), (129, 3072, 8192, 2, 4),
+                               (256, 3072, 8192, 2, 4), (257, 3072, 8192, 4, 4), (200, 3072, 4096, 2, 4), (100, 3072, 4096, 4, 4), (200, 3072, 3072, 2, 2), (128, 3000, 8192, 0, 0)):
+        got = [f(M, N, K, ops.EPI_RESID_BF16) / (4 * M * N) for f in (l.p3v_gemm_ws_bytes, l.p3v_gemm_ws_most_bytes)]
+        assert got == [few, most], (M, N, K, got)
 
 
 def test_which_tile_runs_a_qkv_projection():

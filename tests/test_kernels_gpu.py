@@ -352,6 +352,25 @@ def test_gemm_one_pass_on_128_columns(ops, M, K, heads):
     assert all(torch.equal(x, y) for x, y in zip(*outs))
 
 
+@pytest.mark.parametrize("B,L", [(2, 65), (2, 100), (3, 43), (12, 21), (36, 7), (2, 129), (3, 100), (4, 96), (48, 8), (5, 75)])
+def test_gemm_qkv_one_pass_of_several_rows(ops, B, L):
+    """Several short prompts on 128 x 128 tiles: token tiles that cross from one row into the next (and, of 7 and 8 tokens, over up to 19 of them), up to 256 rows
+    through p3v_gemm_qkv, beyond through its one-pass call.  The bits of the product and p3v_rope_kv_append, queries, keys, values and what lies beside them."""
+    M, K, nh, nkv, past = B * L, 512, 32, 32, 8
+    N, T = (nh + 2 * nkv) * 96, past + L + 3
+    Tp = (T + 127) // 128 * 128
+    a, w = g((M, K), 190).cuda(), g((N, K), 191, 1.0 / math.sqrt(K)).cuda()
+    cos, sin = torch.rand((B, T, 48), device="cuda"), torch.rand((B, T, 48), device="cuda")
+
+    def fresh():
+        return torch.full((B, nh, L, 96), 7.0, dtype=BF16, device="cuda"), g((B, nkv, Tp, 96), 193).cuda(), g((B, nkv, 96, Tp), 194).cuda()
+    two, one = fresh(), fresh()
+    rest = (B, L, nh, nkv, 96, past, Tp, True, T, 1)
+    ops.rope_kv_append(ops.gemm(a, w, slices=False), cos, sin, *two, *rest, q_scale=1.3)
+    assert ops.gemm_qkv(a, w, cos, sin, *one, *rest, q_scale=1.3, one_pass=M > 256)
+    assert all(torch.equal(x, y) for x, y in zip(one, two))
+
+
 @pytest.mark.parametrize("M,N,K,pin,kind", [(300, 3072, 8192, -1, "norm"), (200, 3072, 8192, -1, "norm"), (1023, 3072, 3072, -1, "norm"), (257, 384, 192, 343, "norm"),
                                             (129, 768, 448, 344, "norm"), (161, 256, 1024, 1654, "norm"), (1, 512, 704, 554, "norm"), (641, 1536, 320, 244, "norm"),
                                             (577, 1024, 4096, -1, "bias"), (2308, 1024, 4096, -1, "bias"), (33, 192, 256, 443, "bias"),
