@@ -107,8 +107,10 @@ int p3v_gemm(const p3v_gemm_args_t* args /* host */, void* stream);
 int p3v_gemm_plan(int M, int N, int K, int epilogue);
 int p3v_gemm_tile(int M, int N, int K, int epilogue);
 int64_t p3v_gemm_ws_bytes(int M, int N, int K, int epilogue);
-/* p3v_gemm, p3v_gemm_resid_norm: the largest workspace that either makes use of, never below p3v_gemm_ws_bytes.  Where it is above (33 .. 128 rows, a
- * long K, few columns), a workspace of this size has the shape run in more slices: faster, the same results up to fp32 summation order. */
+/* p3v_gemm, p3v_gemm_resid_norm: the largest workspace that either makes use of, never below p3v_gemm_ws_bytes.  Where it is above, a workspace of this size
+ * has the shape run in more slices on tiles of 96 columns: faster, the same results up to fp32 summation order.  That is up to 256 rows of the ungated
+ * epilogues with N a multiple of 96, where the larger tiles make more workgroups and a slice keeps 12 K-tiles of 64 (16 beyond 128 rows); not where
+ * p3v_gemm_rows_slices takes the shape (9 .. 32 rows, K = 3072 or 8192).  3072 x 8192: 33 .. 256 rows. */
 int64_t p3v_gemm_ws_most_bytes(int M, int N, int K, int epilogue);
 /* 1: p3v_gemm is faster without the workspace of p3v_gemm_ws_bytes (257 .. 384 rows whose 128 x 128 tiles fill one round of the chip) */
 int p3v_gemm_one_pass_pays(int M, int N, int K, int epilogue);
