@@ -58,7 +58,11 @@ class MixedHeads:
 
     def plan(self, B, L, n_keys):
         m = self.m
-        if ops.mix_prompt_ws_bytes(B, L, m.heads, m.kv_heads, m.dim, m.vdim, n_keys, self.T):
+        # (a single tile of 32 keys does not pay for the fragments' launch and the scores' way through memory, but where wide heads fill the one
+        #  launch's registers.  us of head split and attention, one launch : two, 16, 32 and, two tiles, 33 tokens: 32 heads x 96 24.5 : 25.5, 25.0 : 26.0, 28.1 : 26.9;
+        #  24 x 64 19.7 : 20.4, 19.9 : 21.2, 24.3 : 21.4; 18 x 96 / 48 16.9 : 20.1, 17.3 : 21.1, 22.0 : 21.9; 32 x 128 36.3 : 27.7.  Whole prompts of 17 .. 32 tokens 2.5 % faster, captured, and 4 .. 6
+        #  where the host is what they wait for; a few tokens behind earlier ones are two tiles: 16 behind 32 30.9 : 26.2)
+        if (n_keys > 32 or round_up(m.dim, 32) + round_up(m.vdim, 32) > 192) and ops.mix_prompt_ws_bytes(B, L, m.heads, m.kv_heads, m.dim, m.vdim, n_keys, self.T):
             return -1
         return ops.mix_plan(B, L, m.heads, m.kv_heads, m.dim, m.vdim, n_keys, self.T)
 

@@ -221,6 +221,17 @@ def test_launch_planning_and_struct_layouts():
         assert names == [f for f, _ in cls._fields_], cname
 
 
+@pytest.mark.parametrize("H,G,dim,vdim,one", [(32, 32, 96, 96, True), (24, 24, 64, 64, True), (18, 6, 96, 48, True), (32, 16, 128, 128, False), (32, 8, 96, 96, None), (16, 16, 96, 96, None)])
+def test_which_prompts_mix_heads_in_two_launches(H, G, dim, vdim, one):
+    """From 16 tokens on, but not over one tile of 32 keys unless the heads are wide; never four heads of a key head or up to 16 heads (None)."""
+    from types import SimpleNamespace
+    from phi_3_vision_mlx_amd import mixers, ops
+    mx = SimpleNamespace(m=SimpleNamespace(heads=H, kv_heads=G, dim=dim, vdim=vdim), T=ops.BF16)
+    for B in (1, 3):
+        for L, n_keys, two in ((15, 15, False), (15, 900, False), (16, 16, not one), (32, 32, not one), (16, 33, True), (33, 33, True), (40, 1000, True)):
+            assert (mixers.MixedHeads.plan(mx, B, L, n_keys) < 0) == (two and one is not None), (B, L, n_keys)
+
+
 def test_launchers_reject_what_their_kernels_do_not_take():
     """Argument checks come before any launch: they run without a GPU."""
     import ctypes as C
