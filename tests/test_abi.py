@@ -388,6 +388,29 @@ def test_how_many_workgroups_attend_an_int8_cache(monkeypatch, B, T, n_split):
     assert bufs["n_split"] == n_split and bufs["ws"] <= 65536 * 16 * 98 * 4
 
 
+@pytest.mark.parametrize("held", ["bf16", "q4", "fp8"])
+def test_which_prompt_projections_ask_for_the_most_slices(monkeypatch, held):
+    """Weights that lie in memory: up to 256 rows; weights expanded into the scratch in front of the product: 129 .. 256."""
+    from types import SimpleNamespace
+    import torch
+    from phi_3_vision_mlx_amd import model, ops
+    seen, w = [], torch.empty((3072, 8192), dtype=torch.bfloat16, device="meta")
+    monkeypatch.setattr(ops, "gemm", lambda *a, **k: seen.append(("gemm", k["slices"])))
+    monkeypatch.setattr(ops, "gemm_slices", lambda *a, **k: seen.append("slices"))
+    for f in ("dequant_q4", "dequant_fp8"):
+        monkeypatch.setattr(ops, f, lambda *a, **k: w)
+    me = SimpleNamespace(cfg=SimpleNamespace(rms_norm_eps=1e-5), fp8_act=False, serving=False, w={"k": w}, _deq=torch.empty(3072 * 8192, device="meta"),
+                         w8={"k": (w, None)} if held == "fp8" else {}, w4={"k": (torch.empty((3072, 1024), device="meta"), None)} if held == "q4" else {})
+    me._quantises_rows = lambda *a: model.Phi3VModel._quantises_rows(me, *a)
+    for M in (33, 128, 129, 256, 257):
+        most = M <= 256 and (M > 128 or held == "bf16")
+        for epi in (ops.EPI_NONE, ops.EPI_RESID_BF16):
+            seen.clear()
+            x = torch.empty((M, 8192), device="meta")
+            model.Phi3VModel._proj_frozen(me, x, "k", epi, resid=x, out=x)
+            assert seen == (["slices"] if epi == ops.EPI_RESID_BF16 and not most else []) + [("gemm", "most" if most else True)], (M, epi, seen)
+
+
 def test_fused_qkv_projections_decline_several_rows_of_fewer_than_seven_tokens():
     """The V^T epilogue's runs of eight tokens cross the end of one batch row at most.  Everything else about these calls is taken, so
     the answer comes from that check (no kernel starts: declined on the host)."""
