@@ -125,11 +125,13 @@ class LayeredModel(DecoderModel):
         need = {"h": (M * cfg.hidden_size, T), "y": (M * max(m.w_in.shape[0] for m in mixers), T), "o": (M * max(m.n_out for m in mixers), T), "a": (M * ff, T)}
         if self.first_v is not None:                             # its values stay readable through the stack
             need["y_first"] = (M * mixers[self.first_v].w_in.shape[0], T)
-        for m in {id(m): m for m in mixers}.values():
+        alike = {m.m: m for m in mixers}                         # (sizes and plans follow the mixer's sizes alone: asked for once each)
+        for m in alike.values():
             for k, (n, dt) in m.buffers(B, L, n_keys).items():
                 need[k] = (max(n, need.get(k, (0, dt))[0]), dt)
         bufs = {k: torch.zeros(n, dtype=dt, device=dev) if k == "q" else torch.empty(n, dtype=dt, device=dev) for k, (n, dt) in need.items()}
-        bufs["plans"] = [m.plan(B, L, n_keys) for m in mixers]
+        plans = {spec: m.plan(B, L, n_keys) for spec, m in alike.items()}
+        bufs["plans"] = [plans[m.m] for m in mixers]
         return bufs
 
     # ------------------------------------------------------------------ layers

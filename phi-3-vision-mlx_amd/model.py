@@ -163,7 +163,7 @@ class Phi3VModel(DecoderModel):
             return ops.gemv_q4(x, q4[0], q4[1], epilogue, resid=resid, norm_w=norm_w, norm_eps=eps, out=out)
         if q is not None and skinny and K in (3072, 8192):
             return ops.gemv_fp8(x, q[0], q[1], epilogue, resid=resid, norm_w=norm_w, norm_eps=eps, out=out)
-        if self._quantises_rows(key, M, epilogue):
+        if q is not None and self._quantises_rows(key, M, epilogue):
             # prompt-sized input: W8A8 on the fp8 matrix cores, activations quantised per token row (fused with the norm)
             a8, sa = ops.quant_fp8_rows(x, norm_w, eps)
             return ops.gemm_fp8(a8, sa, q[0], q[1], epilogue, resid=resid, out=out)
@@ -182,8 +182,7 @@ class Phi3VModel(DecoderModel):
         # Weights just expanded into the scratch come out of the caches, where more slices of them only add partial sums up to 128 rows.  4-bit prompts, the most
         # slices : as many as without them: 33 tokens 4122 : 4087 us, 64 4199 : 4165, 128 4701 : 4631, but 129 5237 : 5335, 200 5279 : 5436.
         most = M <= 256 and (M > 128 or (q is None and q4 is None))
-        if (epilogue == EPI_RESID_BF16 and out is not None and not (most and ops.gemm_few_rows(M, w.shape[0], K, epilogue))
-                and ops.gemm_slices(x, w, epilogue, resid, out)):
+        if epilogue == EPI_RESID_BF16 and out is not None and ops.gemm_slices(x, w, epilogue, resid, out, few_rows=most):
             return out
         return ops.gemm(x, w, epilogue, resid=resid, out=out, slices="most" if most else True)
 
@@ -195,8 +194,7 @@ class Phi3VModel(DecoderModel):
                 or os.environ.get("P3V_RESID_NORM_FUSE", "1") == "0"):
             return False
         w, eps = self.w[key], self.cfg.rms_norm_eps
-        return (not ops.gemm_few_rows(M, w.shape[0], o.shape[1], EPI_RESID_BF16) and ops.gemm_slices(o, w, EPI_RESID_BF16, x, x, norm=(norm_w, eps, h[:M]))
-                ) or ops.gemm_resid_norm(o, w, x, norm_w, eps, h[:M], out=x, slices="most")
+        return ops.gemm_slices(o, w, EPI_RESID_BF16, x, x, norm=(norm_w, eps, h[:M]), few_rows=True) or ops.gemm_resid_norm(o, w, x, norm_w, eps, h[:M], out=x, slices="most")
 
     def _proj_resid_scaled(self, o, key, x, norm_w, h, sq, next_key):
         """x += bf16(o @ W^T), h = bf16(x * norm_w) and the rows' sums of squares (ops.gemm_rows_resid), for the projection `next_key` that

@@ -247,13 +247,14 @@ def gemm_few_rows(M, N, K, epilogue):
     return M <= 256 and L.lib().p3v_gemm_ws_most_bytes(M, N, K, epilogue) > L.lib().p3v_gemm_ws_bytes(M, N, K, epilogue)
 
 
-def gemm_slices(a, w, epilogue, resid, out, bias=None, col_scale=None, norm=None):
+def gemm_slices(a, w, epilogue, resid, out, bias=None, col_scale=None, norm=None, few_rows=False):
     """gemm with a residual epilogue as slices of K (include/p3v.h: p3v_gemm_slices); norm = (weight, eps, normed): and normed = RMSNorm(out)
-    from the launch that adds the slices (EPI_RESID_BF16).  False -- nothing launched -- where the library does not take the shape that way."""
+    from the launch that adds the slices (EPI_RESID_BF16).  False -- nothing launched -- where the library does not take the shape that way or, with
+    few_rows, where gemm_few_rows goes before it."""
     M, K = a.shape
     N = w.shape[0]
     n = L.lib().p3v_gemm_slices_ws_bytes(M, N, K, epilogue)
-    if not n:
+    if not n or (few_rows and gemm_few_rows(M, N, K, epilogue)):
         return False
     stream = F32 if epilogue in (EPI_BIAS_RESID_F32, EPI_SCALE_RESID_F32) else BF16
     _chk(a, BF16, "a"), _chk(w, BF16, "w"), _chk(resid, stream, "resid"), _chk(out, stream, "out")
@@ -924,10 +925,10 @@ def project(x, w, epilogue=EPI_NONE, resid=None, col_scale=None, out=None, alone
         if K % 64 == 0 and N % 8 == 0:
             if alone and epilogue in GATED and 104 < M <= 128 and gemm_merge(x, w, epilogue, out):
                 return out
-            if scaled and not gemm_few_rows(M, N, K, epilogue) and gemm_slices(x, w, epilogue, resid, out, col_scale=col_scale):
+            if scaled and gemm_slices(x, w, epilogue, resid, out, col_scale=col_scale, few_rows=True):
                 return out
             return gemm(x, w, epilogue, resid=resid, out=out, col_scale=col_scale,
-                        slices=False if L.lib().p3v_gemm_one_pass_pays(M, N, K, epilogue) else "most")
+                        slices="most" if M <= 256 else M > 384 or not L.lib().p3v_gemm_one_pass_pays(M, N, K, epilogue))
     args = L.GemmArgs(_p(x), _p(w), _p(out), 0, _p(resid), 0, M, N, K, x.stride(0), w.stride(0), out.stride(0), epilogue, 0, 0, 0, _p(col_scale))
     L.check(L.lib().p3v_gemm_any(C.byref(args), int(f32), _stream()), "gemm_any")
     return out

@@ -396,7 +396,7 @@ def test_which_prompt_projections_ask_for_the_most_slices(monkeypatch, held):
     from phi_3_vision_mlx_amd import model, ops
     seen, w = [], torch.empty((3072, 8192), dtype=torch.bfloat16, device="meta")
     monkeypatch.setattr(ops, "gemm", lambda *a, **k: seen.append(("gemm", k["slices"])))
-    monkeypatch.setattr(ops, "gemm_slices", lambda *a, **k: seen.append("slices"))
+    monkeypatch.setattr(ops, "gemm_slices", lambda *a, **k: seen.append(("slices", k["few_rows"])))
     for f in ("dequant_q4", "dequant_fp8"):
         monkeypatch.setattr(ops, f, lambda *a, **k: w)
     me = SimpleNamespace(cfg=SimpleNamespace(rms_norm_eps=1e-5), fp8_act=False, serving=False, w={"k": w}, _deq=torch.empty(3072 * 8192, device="meta"),
@@ -408,7 +408,7 @@ def test_which_prompt_projections_ask_for_the_most_slices(monkeypatch, held):
             seen.clear()
             x = torch.empty((M, 8192), device="meta")
             model.Phi3VModel._proj_frozen(me, x, "k", epi, resid=x, out=x)
-            assert seen == (["slices"] if epi == ops.EPI_RESID_BF16 and not most else []) + [("gemm", "most" if most else True)], (M, epi, seen)
+            assert seen == ([("slices", most)] if epi == ops.EPI_RESID_BF16 else []) + [("gemm", "most" if most else True)], (M, epi, seen)
 
 
 def test_fused_qkv_projections_decline_several_rows_of_fewer_than_seven_tokens():
