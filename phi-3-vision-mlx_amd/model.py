@@ -547,7 +547,7 @@ class Phi3VModel(DecoderModel):
                     qkv_args = (hn, w[k_w], st.cos, st.sin, q, kd, vd, B, L, nh, nkv, hd, past, st.Tp, True, st.T, 1)
                     fused_qkv = (M <= 128 and not self.serving and ops.gemm_qkv_merge(*qkv_args, q_scale=scale * ops.Q_PRESCALE)
                                  or ops.gemm_qkv(*qkv_args, q_scale=scale * ops.Q_PRESCALE)
-                                 or ops.gemm_qkv(*qkv_args, q_scale=scale * ops.Q_PRESCALE, one_pass=True))
+                                 or 256 < M <= 384 and ops.gemm_qkv(*qkv_args, q_scale=scale * ops.Q_PRESCALE, one_pass=True))     # (elsewhere it declines)
             f8_w = self.w8.get(k_w)                             # the same on e4m3 weights and quantised rows
             if (f8_w is not None and L > ops.L.DECODE_MAX_L and n_beam == 1 and k_w not in self.adapters and not mlx4_first and self.fp8_act
                     and ops.gemm_fp8_ok(M, f8_w[0].shape[0], cfg.hidden_size, EPI_NONE) and os.environ.get("P3V_QKV_FUSE", "1") != "0"
@@ -590,8 +590,8 @@ class Phi3VModel(DecoderModel):
                 else:                                           # prefill: exact attention, quantised copy stored
                     if past > 0 and not getattr(st, "fresh_rows", False):   # long cached call (constrain with > 16 tokens): attend on a
                         ops.kv_dequantize(st.k8[i], st.v8[i], st.ks[i], st.vs[i], st.k_tmp, st.v_tmp, past)   # dequantised copy
-                    stored = not fused_qkv and ops.rope_kv_quantize(qkv, st.cos, st.sin, q, st.k_tmp, st.v_tmp, st.k8[i], st.v8[i], st.ks[i], st.vs[i], B, L,
-                                                                    nh, nkv, hd, past, st.Tp, st.T, 1, q_scale=scale * ops.Q_PRESCALE)
+                    stored = not fused_qkv and L >= 32 and past % 8 == 0 and ops.rope_kv_quantize(     # (elsewhere it declines)
+                        qkv, st.cos, st.sin, q, st.k_tmp, st.v_tmp, st.k8[i], st.v8[i], st.ks[i], st.vs[i], B, L, nh, nkv, hd, past, st.Tp, st.T, 1, q_scale=scale * ops.Q_PRESCALE)
                     if not fused_qkv and not stored:
                         ops.rope_kv_append(qkv, st.cos, st.sin, q, st.k_tmp, st.v_tmp, B, L, nh, nkv, hd, past, st.Tp, True, st.T, 1,
                                            q_scale=scale * ops.Q_PRESCALE)

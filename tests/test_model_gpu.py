@@ -404,6 +404,31 @@ def test_last_rows_attention_stays_out_of_8bit_projections(B, quantised, monkeyp
     assert not quantised or torch.equal(got[40], got[10 ** 9])
 
 
+@pytest.mark.parametrize("kw,B,L,past,asked", [({}, 2, 60, 0, False), ({}, 2, 150, 0, True), ({}, 2, 200, 0, False), (dict(use_quantized_cache=True, quantized_fp8=True), 3, 20, 0, False),
+                                               (dict(use_quantized_cache=True, quantized_fp8=True), 3, 40, 0, True), (dict(use_quantized_cache=True), 1, 40, 100, False)])
+def test_launches_that_decline_a_size_are_not_asked(monkeypatch, kw, B, L, past, asked):
+    """A declined call costs the host as much as one that runs: the one-pass qkv is asked for at 257 .. 384 rows, the launch that rotates and quantises from 32 tokens on
+    at a whole 8 columns -- and then they answer."""
+    from phi_3_vision_mlx_amd import ops
+    from phi_3_vision_mlx_amd.api import load_synthetic
+    model, _ = load_synthetic(blind_model=True, tiny=False, seed=0, device="cuda:0", num_hidden_layers=2, **kw)
+    cache = model(input_ids=np.concatenate([rand_ids(past, 3)] * B), max_tokens=L + 4)[1] if past else None
+    got, qkv, quantise = [], ops.gemm_qkv, ops.rope_kv_quantize
+
+    def watch(f, when):
+        def call(*a, **k):
+            r = f(*a, **k)
+            if when(k):
+                got.append(r)
+            return r
+        return call
+    monkeypatch.setattr(ops, "gemm_qkv", watch(qkv, lambda k: k.get("one_pass")))
+    monkeypatch.setattr(ops, "rope_kv_quantize", watch(quantise, lambda k: True))
+    ids = np.concatenate([rand_ids(L, 70 + i) for i in range(B)])
+    model(input_ids=ids, cache=cache) if past else model(input_ids=ids, max_tokens=4)
+    assert got == [True] * (2 if asked else 0)
+
+
 def test_batched_left_pad(text):
     model, proc, oracle = text
     inputs = proc(["a", "hello world, this is a longer prompt", "mid size"])
