@@ -720,14 +720,14 @@ extern "C" int p3v_gemm_qkv_fp8_pays(int M, int n_q, int n_kv, int K) { return q
 // With an int8 cache behind it the split + rotation store the codes too (p3v_rope_kv_quantize), and a quantiser's launch goes with them: one launch has to
 // gain 5 us more, and more than that the longer both take: the chip is then at its power limit, where 128 x 256 tiles on twelve waves cost more than their time
 // (8192 tokens: the two pairs of launches are equal, but gate_up and attention beside the pair are 2 and 5 % faster).  The threshold is fitted to whole prompts of 137 .. 14000
-// tokens at the decoder's widths, 85 lengths run either way, 31 of them on two to four machines: it names the slower side by 9 us a layer at most (4150 .. 4300 tokens on
+// tokens at the decoder's widths, 95 lengths run either way, 35 of them on two to five machines: it names the slower side by 9 us a layer at most (4150 .. 4300 tokens on
 // one machine, 8130 on another; 1.3 % of the prompt), elsewhere by no more than the runs of one side differ.  us a layer, two - one: 400 tokens -4.6, 577 -3.7, 768 0.4, 803 -19, 1800
-// -16, 2300 -10, 2531 0 .. 3, 2670 2, 3300 -7 and -18, 3500 0 and -7, 3900 -8.4, 4000 2 and 6, 4050 28, 4096 13 .. 30, 4150 -9 and -5, 4300 -5 and 3, 4500 -15, 5200 6, 6000 -2 and 4, 6500 -15 and -5,
+// -16, 2300 -10, 2531 -5 .. 3, 2670 2, 3300 -7 and -18, 3500 0 and -7, 3900 -8.4, 4000 2 and 6, 4050 28, 4096 13 .. 30, 4150 -9 and -5, 4300 -5 and 3, 4500 -15, 5150 1, 5170 4, 5200 6, 6000 -2 and 4, 6100 -1 and 8, 6500 -15 and -5,
 // 6750 41, 7000 0, 7300 -25 .. -37, 7800 -32, 8000 1 .. 20, 8192 -52, -40, -22 and 9, 10000 -14 and -8, 12288 0.
 extern "C" int p3v_gemm_qkv_fp8_stored_pays(int M, int n_q, int n_kv, int K) {
   if (!qkv_fp8_sizes(M, n_q, n_kv, K)) return 0;
   const float out = (float)M * (float)(n_q + 2 * n_kv);
-  return out <= 7.5e7f && qkv_fp8_gain(M, n_q, n_kv, K) > 5.f + 3.3e-7f * fmaxf(out - 2.4e7f, 0.f);
+  return out <= 7.5e7f && qkv_fp8_gain(M, n_q, n_kv, K) > 5.f + 3.2e-7f * fmaxf(out - 2.4e7f, 0.f);
 }
 
 // p3v_gemm_fp8 (epilogue NONE) + p3v_rope_kv_append in one launch, bit for bit, on 128 x 256 tiles: the projection's 47 MB (2531 rows) are
