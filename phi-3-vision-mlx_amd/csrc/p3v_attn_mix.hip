@@ -48,6 +48,8 @@ __device__ __forceinline__ float* ws_o(float* ws, const AttnMixP& p, size_t rows
 //   P  [heads][16 q][32 keys] bf16,  AL [heads][16 q] rescale factors,  MM [heads][16 q] running maxima
 // The softmax's sum rides in the second product as one more value dimension (a row of ones).  The value fragments of a tile are
 // requested ahead of its mixing and the next tile's key fragments ahead of the second product; the barriers wait for LDS only.
+// KX: keys as fragments (k_mix_keys), else rows of the cache -- apart, since the steps between a key's pieces are then constants of the loads (12 rows behind 6500 keys
+// of 32 heads x 96: 155 us with one kernel for both, 146 so).
 // SHARED: the heads of a wave share one key / value head (else every head loads its own fragments, one head ahead).
 template <int HW> struct MixCfg {
   static constexpr int HP = 8 * HW, HS = HP + 4, QS = 32 * HS + 4;      // heads padded, S strides (floats): key, query
@@ -57,7 +59,7 @@ template <int HW> struct MixCfg {
   static constexpr int LDS = S_BYTES + P_BYTES + 2 * A_BYTES + HM * 1024 + (HW == 4 ? 8 * 4096 : 0);
 };
 
-template <int HW, int DC, int VC, bool SHARED>
+template <int HW, int DC, int VC, bool SHARED, bool KX>
 __global__ void __launch_bounds__(512, 1) k_attn_mix_prefill(AttnMixP p) {
   typedef MixCfg<HW> C;
   constexpr int NB = SHARED ? 1 : 2;                                     // fragment buffers
@@ -124,27 +126,45 @@ __global__ void __launch_bounds__(512, 1) k_attn_mix_prefill(AttnMixP p) {
     for (int i = tid; i < C::S_BYTES / 4; i += 512) S[i] = 0.f;
   lds_barrier();
 
-  const bf16_t* kb = (p.kx ? p.kx : (const bf16_t*)p.k) + (size_t)b * p.G * (p.kx ? p.kx_rows : p.Tp) * p.dimp;
+  const bf16_t* kb = (KX ? p.kx : (const bf16_t*)p.k) + (size_t)b * p.G * (KX ? p.kx_rows : p.Tp) * p.dimp;
   const bf16_t* vb = (const bf16_t*)p.v + (size_t)b * p.G * p.Tp * p.vdimp;
-  // (rows of the cache, or their fragments: k_mix_keys)
-  const uint32_t k_lane = p.kx ? lane * 16 : (uint32_t)(lc * p.dimp + lg * 8) * 2, kc = p.kx ? 1024 : 64, k_rows = p.kx ? p.kx_rows : p.Tp;
-  const uint32_t v_lane = (uint32_t)(((lg >> 1) * p.vdimp + lc) * 16 + (lg & 1) * 8) * 2;
+  // AS_GLOBAL: keys and values by pointers to device memory (gload), else by generic ones.  Which is faster follows the registers that are left: us, generic : device,
+  // 2048 rows of 32 x 96 on 8 key heads 119 : 114, 18 x 96 / 48 123 : 118, 24 x 64 146 : 141, but 32 x 128 on 8 226 : 240, 16 x 96 110 : 111, and 12 rows behind 6500 keys of
+  // 32 x 96 146 : 155.
+  constexpr bool AS_GLOBAL = KX || (HW == 4 && DC + VC <= (SHARED ? 6 : 5));
+  constexpr uint32_t kc = KX ? 512 : 32;                                 // elements from one 32-dimension piece of a key's fragment or row to the next
+  const uint32_t k_lane = KX ? lane * 8 : (uint32_t)(lc * p.dimp + lg * 8);
+  const int k_rows = KX ? p.kx_rows : p.Tp;
+  const uint32_t v_lane = (uint32_t)(((lg >> 1) * p.vdimp + lc) * 16 + (lg & 1) * 8);
   const bool active = wave * HW < p.H;
   bf16x8_t kf[NB][2][DC], vf[NB][NV];
   auto load_k = [&](int t, int i) {
     const int g = min(wave * HW + i, p.H - 1) / per, bf = SHARED ? 0 : i & 1;
-    gptr_t k0 = (gptr_t)(kb + ((size_t)g * k_rows + t * 32) * p.dimp), k1 = k0 + (size_t)32 * p.dimp;
-    asm volatile("" : "+s"(k0), "+s"(k1));                               // (scalar bases + one 32-bit lane offset: no 64-bit lane addresses)
+    const bf16_t *k0 = kb + ((size_t)g * k_rows + t * 32) * p.dimp, *k1 = k0 + (size_t)16 * p.dimp;
+    if constexpr (AS_GLOBAL) {
+      gptr_t a = (gptr_t)k0, b_ = (gptr_t)k1;
+      asm volatile("" : "+s"(a), "+s"(b_));                               // (scalar bases + one 32-bit lane offset: no 64-bit lane addresses)
 #pragma unroll
-    for (int c = 0; c < DC; ++c) kf[bf][0][c] = gload<bf16x8_t>(k0 + c * kc, k_lane), kf[bf][1][c] = gload<bf16x8_t>(k1 + c * kc, k_lane);
+      for (int c = 0; c < DC; ++c) kf[bf][0][c] = gload<bf16x8_t>(a + c * kc * 2, k_lane * 2), kf[bf][1][c] = gload<bf16x8_t>(b_ + c * kc * 2, k_lane * 2);
+    } else {
+      asm volatile("" : "+s"(k0), "+s"(k1));
+#pragma unroll
+      for (int c = 0; c < DC; ++c) kf[bf][0][c] = *(const bf16x8_t*)(k0 + k_lane + c * kc), kf[bf][1][c] = *(const bf16x8_t*)(k1 + k_lane + c * kc);
+    }
   };
   auto load_v = [&](int t, int i) {
     const int g = min(wave * HW + i, p.H - 1) / per, bf = SHARED ? 0 : i & 1;
-    gptr_t vr = (gptr_t)(vb + ((size_t)g * (p.Tp >> 4) + t * 2) * p.vdimp * 16);
-    asm volatile("" : "+s"(vr));
+    const bf16_t* vr = vb + ((size_t)g * (p.Tp >> 4) + t * 2) * p.vdimp * 16;
+    if constexpr (AS_GLOBAL) {
+      gptr_t a = (gptr_t)vr;
+      asm volatile("" : "+s"(a));
 #pragma unroll
-    for (int d = 0; d < NV; ++d)
-      vf[bf][d] = gload<bf16x8_t>(vr + d * 512, v_lane);
+      for (int d = 0; d < NV; ++d) vf[bf][d] = gload<bf16x8_t>(a + d * 512, v_lane * 2);
+    } else {
+      asm volatile("" : "+s"(vr));
+#pragma unroll
+      for (int d = 0; d < NV; ++d) vf[bf][d] = *(const bf16x8_t*)(vr + v_lane + d * 256);
+    }
   };
   if (active && t0 < t1) load_k(t0, 0);
 
@@ -655,35 +675,35 @@ static int mix_combine(const AttnMixP& p, hipStream_t s) {
   return P3V_OK;
 }
 
-template <int HW, int DC, int VC, bool SHARED>
+template <int HW, int DC, int VC, bool SHARED, bool KX>
 static int launch_prefill(const AttnMixP& p, hipStream_t s) {
   static bool attr_set = false;
   if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)k_attn_mix_prefill<HW, DC, VC, SHARED>, hipFuncAttributeMaxDynamicSharedMemorySize, MixCfg<HW>::LDS) != hipSuccess) return P3V_ERR_HIP;
+    if (hipFuncSetAttribute((const void*)k_attn_mix_prefill<HW, DC, VC, SHARED, KX>, hipFuncAttributeMaxDynamicSharedMemorySize, MixCfg<HW>::LDS) != hipSuccess) return P3V_ERR_HIP;
     attr_set = true;
   }
   dim3 grid(p3v_cdiv(p.L, 16), p.n_split, p.B);
   if (p.runs) grid = dim3(p.runs);
-  hipLaunchKernelGGL((k_attn_mix_prefill<HW, DC, VC, SHARED>), grid, dim3(512), MixCfg<HW>::LDS, s, p);
+  hipLaunchKernelGGL((k_attn_mix_prefill<HW, DC, VC, SHARED, KX>), grid, dim3(512), MixCfg<HW>::LDS, s, p);
   P3V_CHECK_LAUNCH();
   return p.n_split > 1 ? mix_combine(p, s) : P3V_OK;
 }
-template <int HW, bool SHARED, int DC>
+template <int HW, bool SHARED, bool KX, int DC>
 static int prefill_vc(const AttnMixP& p, hipStream_t s) {
   switch (p.vdimp / 32) {
-    case 1: return launch_prefill<HW, DC, 1, SHARED>(p, s);
-    case 2: return launch_prefill<HW, DC, 2, SHARED>(p, s);
-    case 3: return launch_prefill<HW, DC, 3, SHARED>(p, s);
-    default: return launch_prefill<HW, DC, 4, SHARED>(p, s);
+    case 1: return launch_prefill<HW, DC, 1, SHARED, KX>(p, s);
+    case 2: return launch_prefill<HW, DC, 2, SHARED, KX>(p, s);
+    case 3: return launch_prefill<HW, DC, 3, SHARED, KX>(p, s);
+    default: return launch_prefill<HW, DC, 4, SHARED, KX>(p, s);
   }
 }
-template <int HW, bool SHARED>
+template <int HW, bool SHARED, bool KX = false>
 static int prefill_dc(const AttnMixP& p, hipStream_t s) {
   switch (p.dimp / 32) {
-    case 1: return prefill_vc<HW, SHARED, 1>(p, s);
-    case 2: return prefill_vc<HW, SHARED, 2>(p, s);
-    case 3: return prefill_vc<HW, SHARED, 3>(p, s);
-    default: return prefill_vc<HW, SHARED, 4>(p, s);
+    case 1: return prefill_vc<HW, SHARED, KX, 1>(p, s);
+    case 2: return prefill_vc<HW, SHARED, KX, 2>(p, s);
+    case 3: return prefill_vc<HW, SHARED, KX, 3>(p, s);
+    default: return prefill_vc<HW, SHARED, KX, 4>(p, s);
   }
 }
 
@@ -703,6 +723,7 @@ int mix_prefill(AttnMixP p, int n_keys, hipStream_t s) {
   const int per = p.H / p.G;                                             // query heads of a key / value head
   if (p.H <= 8) return prefill_dc<1, true>(p, s);
   if (p.H <= 16) return per % 2 ? prefill_dc<2, false>(p, s) : prefill_dc<2, true>(p, s);
+  if (p.kx) return prefill_dc<4, false, true>(p, s);                     // (mixp_two: the only heads whose keys are copied)
   return per % 4 ? prefill_dc<4, false>(p, s) : prefill_dc<4, true>(p, s);
 }
 
