@@ -136,7 +136,7 @@ class Phi3VModel(DecoderModel):
         return ops.lora_up(y, t, b, scale, epilogue, resid=resid, out=out)
 
     def _quantises_rows(self, key, M, epilogue=EPI_NONE):
-        """Whether the projection `key` of M rows quantises them first (W8A8 on the fp8 matrix cores)."""
+        """Whether the projection `key` of M rows quantises them first (W8A8 on the fp8 matrix cores): what _proj_frozen does."""
         if key not in self.w8 or not self.fp8_act:
             return False
         N, K = self.w8[key][0].shape
@@ -163,7 +163,7 @@ class Phi3VModel(DecoderModel):
             return ops.gemv_q4(x, q4[0], q4[1], epilogue, resid=resid, norm_w=norm_w, norm_eps=eps, out=out)
         if q is not None and skinny and K in (3072, 8192):
             return ops.gemv_fp8(x, q[0], q[1], epilogue, resid=resid, norm_w=norm_w, norm_eps=eps, out=out)
-        if q is not None and self._quantises_rows(key, M, epilogue):
+        if q is not None and not skinny and self.fp8_act and ops.gemm_fp8_ok(M, q[0].shape[0], K, epilogue):
             # prompt-sized input: W8A8 on the fp8 matrix cores, activations quantised per token row (fused with the norm)
             a8, sa = ops.quant_fp8_rows(x, norm_w, eps)
             return ops.gemm_fp8(a8, sa, q[0], q[1], epilogue, resid=resid, out=out)

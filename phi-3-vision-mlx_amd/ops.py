@@ -192,9 +192,7 @@ def gemm_merge(a, w, epilogue, out):
 
 
 def _slices_bytes(M, N, K, epilogue, slices):
-    if not slices:
-        return 0
-    return (L.lib().p3v_gemm_ws_most_bytes if slices == "most" else L.lib().p3v_gemm_ws_bytes)(M, N, K, epilogue)
+    return L.lib().p3v_gemm_ws_bytes(M, N, K, epilogue) if slices is True else L.lib().p3v_gemm_ws_most_bytes(M, N, K, epilogue) if slices else 0
 
 
 def gemm(a, w, epilogue=EPI_NONE, bias=None, resid=None, out=None, n_out=None, pos=None, patches_per_img=0, ldo=None,

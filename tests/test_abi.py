@@ -401,7 +401,6 @@ def test_which_prompt_projections_ask_for_the_most_slices(monkeypatch, held):
         monkeypatch.setattr(ops, f, lambda *a, **k: w)
     me = SimpleNamespace(cfg=SimpleNamespace(rms_norm_eps=1e-5), fp8_act=False, serving=False, w={"k": w}, _deq=torch.empty(3072 * 8192, device="meta"),
                          w8={"k": (w, None)} if held == "fp8" else {}, w4={"k": (torch.empty((3072, 1024), device="meta"), None)} if held == "q4" else {})
-    me._quantises_rows = lambda *a: model.Phi3VModel._quantises_rows(me, *a)
     for M in (33, 128, 129, 256, 257):
         most = M <= 256 and (M > 128 or held == "bf16")
         for epi in (ops.EPI_NONE, ops.EPI_RESID_BF16):
