@@ -58,11 +58,17 @@ class MixedHeads:
 
     def plan(self, B, L, n_keys):
         m = self.m
-        # (a single tile of 32 keys does not pay for the fragments' launch and the scores' way through memory, but where wide heads fill the one
-        #  launch's registers.  us of head split and attention, one launch : two, 16, 32 and, two tiles, 33 tokens: 32 heads x 96 24.5 : 25.5, 25.0 : 26.0, 28.1 : 26.9;
-        #  24 x 64 19.7 : 20.4, 19.9 : 21.2, 24.3 : 21.4; 18 x 96 / 48 16.9 : 20.1, 17.3 : 21.1, 22.0 : 21.9; 32 x 128 36.3 : 27.7.  Whole prompts of 17 .. 32 tokens 2.5 % faster, captured, and 4 .. 6
-        #  where the host is what they wait for; a few tokens behind earlier ones are two tiles: 16 behind 32 30.9 : 26.2)
-        if (n_keys > 32 or round_up(m.dim, 32) + round_up(m.vdim, 32) > 192) and ops.mix_prompt_ws_bytes(B, L, m.heads, m.kv_heads, m.dim, m.vdim, n_keys, self.T):
+        # Two launches on fragments of the keys, or one on their rows.  Wide heads fill the one launch's registers: two.  Else
+        # - a single tile of 32 keys does not pay for the fragments' launch and the scores' way through memory.  us of head split and attention, one launch : two, 16, 32 and,
+        #   two tiles, 33 tokens: 32 heads x 96 24.5 : 25.5, 25.0 : 26.0, 28.1 : 26.9; 24 x 64 19.7 : 20.4, 19.9 : 21.2, 24.3 : 21.4; 18 x 96 / 48 16.9 : 20.1, 17.3 : 21.1, 22.0 : 21.9; 32 x
+        #   128 36.3 : 27.7.  Whole prompts of 17 .. 32 tokens 2.5 % faster, captured, and 4 .. 6 where the host is what they wait for; a few tokens behind earlier ones
+        #   are two tiles: 16 behind 32 30.9 : 26.2.
+        # - few new tokens of many rows behind long caches do not pay for the copy of all keys, once they fill the chip in one launch: 12 rows of 96 behind 2000 234 : 293, 8 of 40 behind
+        #   3000 179 : 205, 6 of 40 behind 3000 144 : 159, but 4 of 128 behind 4000 1.23x faster in two, 2 of 24 behind 16000 1.51x.  The line is fitted to 1506 sizes of 1 .. 16 rows of 24 ..
+        #   600 tokens behind 0 .. 16000 at 32 x 96 and 24 x 64: 0.4 % behind the faster form on average (two launches always: 0.9 %, 41 % at most), 17 % at most.
+        narrow, copied = round_up(m.dim, 32) + round_up(m.vdim, 32) <= 192, 2e-6 * B * m.kv_heads * n_keys * round_up(m.dim, 32)      # MB of keys
+        one = narrow and (n_keys <= 32 or (n_keys > L and B * -(-L // 16) >= 10 and copied >= 80 + 0.5 * L))
+        if not one and ops.mix_prompt_ws_bytes(B, L, m.heads, m.kv_heads, m.dim, m.vdim, n_keys, self.T):
             return -1
         return ops.mix_plan(B, L, m.heads, m.kv_heads, m.dim, m.vdim, n_keys, self.T)
 

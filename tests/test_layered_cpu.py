@@ -232,6 +232,17 @@ def test_which_prompts_mix_heads_in_two_launches(H, G, dim, vdim, one):
             assert (mixers.MixedHeads.plan(mx, B, L, n_keys) < 0) == (two and one is not None), (B, L, n_keys)
 
 
+@pytest.mark.parametrize("B,L,past,two", [(12, 96, 2000, False), (8, 40, 3000, False), (6, 40, 2000, True), (6, 40, 3000, False), (12, 16, 1500, False), (9, 16, 8000, True), (1, 24, 16000, True),
+                                          (1, 600, 16000, True), (1, 160, 32000, False), (16, 900, 0, True), (4, 128, 2000, True)])
+def test_few_new_tokens_behind_long_caches_read_the_keys_rows(B, L, past, two):
+    """Ten query tiles in all and 80 MB of keys, half a MB more a new token: then one launch on the keys' rows, which nobody copies; wide heads in two whatever there is."""
+    from types import SimpleNamespace
+    from phi_3_vision_mlx_amd import mixers, ops
+    for dim, want in ((96, two), (128, True)):
+        mx = SimpleNamespace(m=SimpleNamespace(heads=32, kv_heads=32, dim=dim, vdim=dim), T=ops.BF16)
+        assert (mixers.MixedHeads.plan(mx, B, L, past + L) < 0) == want, dim
+
+
 def test_launchers_reject_what_their_kernels_do_not_take():
     """Argument checks come before any launch: they run without a GPU."""
     import ctypes as C
