@@ -1253,10 +1253,14 @@ static bool dma_half_blocks(int pairs, int L) { return (long)pairs * p3v_cdiv(L,
 // them -- one row: and a little more -- and there are keys to share.  us, as below : so (32 heads x 96, causal): 704 tokens 16.9 : 15.7,
 // 1024 23.4 : 19.4, 1152 25.2 : 22.4, but 1500 28.9 : 29.1, 2531 50.1 : 58.6 (576 15.0 : 14.5 and 1408 28.9 : 26.9 alone, inside a prompt of 600 and
 // 1300 tokens 0.4 and 0.2 % slower: 800 0.8 % faster, 1024 1.4); 200 behind 2000 38.6 : 28.6, 400 behind 4000 72.0 : 49.0,
-// 1024 behind 3000 64.1 : 51.0; two rows of 400 behind 1000 32.9 : 24.9, of 512 15.4 : 15.0, but of 640 (320 workgroups) 19.5 : 22.2.
+// 1024 behind 3000 64.1 : 51.0; two rows of 400 behind 1000 32.9 : 24.9, of 512 15.4 : 15.0, but of 640 (320 workgroups) 19.5 : 22.2.  Behind a cache the few workgroups
+// beyond one round are as long as the others: one round there (1100 behind 704 33.5 : 38.1, behind 3008 73.9 : 78.5, but 1024 behind 3008 1.25x faster so), and from 896 keys on where 64-query
+// workgroups of the other kernel fill the chip or a query block is short of keys (640 behind 64 17.7 : 18.6, 128 behind 704 18.0 : 18.5, 8 rows of 33 behind 704 18.1 : 19.4; 200 behind 704
+// 1.02x, 33 behind 704 1.08x faster so).  Of 296 sizes behind caches of 64 .. 30016 keys the slowest is then 4 % behind.
 static bool il_two_groups(const AttnP& p) {
   const long wgs = (long)p.nh * p.B * p3v_cdiv(p.L, 128);
-  return p.causal && p.past + p.L >= 704 && wgs <= (p.B == 1 ? 288 : 256);
+  const bool behind = p.past > 0;
+  return p.causal && p.past + p.L >= (behind && (p.L > 64 || wgs > 192) ? 896 : 704) && wgs <= (p.B == 1 && !behind ? 288 : 256);
 }
 
 template <int HD>

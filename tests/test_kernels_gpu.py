@@ -730,8 +730,10 @@ def test_attention_reads_nothing_behind_its_arguments_last_field(ops):
 
 
 @pytest.mark.parametrize("B,L,past,nh,causal,two", [
-    (1, 640, 63, 8, True, False), (1, 640, 64, 8, True, True), (1, 704, 0, 8, True, True),                  # from 704 keys on
-    (1, 1152, 0, 32, True, True), (1, 1153, 0, 32, True, False), (2, 512, 200, 32, True, True), (2, 513, 200, 32, True, False),      # workgroups: 288 of one row, 256 of several
+    (1, 703, 0, 8, True, False), (1, 704, 0, 8, True, True), (1, 64, 639, 8, True, False), (1, 64, 640, 8, True, True),      # from 704 keys on, more than 64 new or a fuller
+    (1, 65, 830, 8, True, False), (1, 65, 831, 8, True, True), (7, 33, 862, 32, True, False), (7, 33, 863, 32, True, True),    # chip behind a cache: from 896
+    (1, 1152, 0, 32, True, True), (1, 1153, 0, 32, True, False), (1, 1024, 8, 32, True, True), (1, 1025, 8, 32, True, False),  # workgroups: 288 of one row, 256 behind a cache
+    (2, 512, 400, 32, True, True), (2, 513, 400, 32, True, False),                                                              # ... and of several
     (1, 800, 0, 8, False, False)])
 def test_which_prompts_attend_by_two_key_groups(ops, request, B, L, past, nh, causal, two):
     """p3v_attention_any_order inside the limits: the bits of the pinned kernel with two key groups; outside them, and p3v_attention anywhere: its own."""
