@@ -14,7 +14,7 @@
 // epilogue together at the end.  The bytes (N*K/2 + N*K/16) are a quarter of the bf16 kernel's for as many products, so its instructions count as much as
 // its bytes: 11 per 8 weights, 4 per piece, one reduction and epilogue per U pairs, and a norm whose steps all four waves share alike.  What else
 // bounds it is where the requests stand (see the pipeline below).  8 waves per CU (6, 10, 16 with the rows of 16384 / 9216: 9.2 / 5.6, 7.8 / 6.2,
-// 8.8 / 6.2 us against 7.8 / 5.6).  Per launch (weights from memory): gate_up 8.9 -> 7.8 us, qkv 6.85 -> 5.6, down 6.2 -> 5.7; four steps of the
+// 8.8 / 6.2 us against 7.8 / 5.6; 16 where the launch's rule says).  Per launch (weights from memory): gate_up 8.9 -> 7.8 us, qkv 6.85 -> 5.6, down 6.2 -> 5.7; four steps of the
 // 32-layer decoder at 128 columns 3.91 -> 3.61 ms.
 #include <stdlib.h>
 
@@ -283,8 +283,13 @@ static int launch_gemv3_q4(const GemvQ4P& p, hipStream_t s, const GemvStepP* sp 
     if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&pr, dev) != hipSuccess) return P3V_ERR_HIP;
     n_cu = pr.multiProcessorCount;
   }
-  const int wpc = p3v_tuning().gemv_q4_wpc;   // waves per CU
-  int upw = p3v_cdiv(p.units, n_cu * wpc);
+  // Waves per CU: 8, so that a norm is done by two workgroups of it instead of four -- but 16 where 8 would hold one row pair more than a turn takes, a second turn for
+  // it alone (us with the norm, 8 : 16, 18000 x 3072 11.2 : 7.9, 20000 12.1 : 9.8, 9216 x 8192 14.1 : 11.5, 12288 15.7 : 14.4), or, without a norm, a second turn at all (24576
+  // x 3072 9.8 : 9.2, 32064 12.1 : 11.6, 16384 x 8192 16.7 : 15.4).  Two and more turns with a norm: 28000 x 3072 12.4 : 13.4, 32064 12.6 : 13.2, 24576 x 8192 22.5 : 28.7.
+  const int forced = p3v_tuning().gemv_q4_wpc, turn = 4 / NST;
+  auto pairs_of = [&](int wpc) { return p3v_cdiv(p.units, n_cu * wpc); };
+  int upw = pairs_of(forced > 0 ? forced : 8);
+  if (forced <= 0 && upw > turn && (upw == turn + 1 || (!p.norm_w && upw <= 2 * turn))) upw = pairs_of(16);
   if (upw < 1) upw = 1;
   const int waves = p3v_cdiv(p.units, upw);
   int wpw = p3v_gemv_wpw(waves, n_cu, p3v_tuning().gemv_wpw);

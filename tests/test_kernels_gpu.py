@@ -2279,6 +2279,27 @@ def test_gemm_rows_resid_refuses(ops):
         assert torch.all(s == 7.0) and torch.all(sq == 7.0) and torch.all(o == 7.0)
 
 
+@pytest.mark.parametrize("N,K", [(16384, 3072), (16386, 3072), (20480, 3072), (20482, 3072), (32768, 3072), (32770, 3072), (8192, 8192), (8194, 8192), (12288, 8192), (12290, 8192), (16386, 8192)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_gemv_q4_waves_by_rows(ops, request, N, K, norm):
+    """One row at the edges of the waves' rule -- a turn of row pairs, one pair more, two turns and beyond: the bits that 8, 16 and 3 waves a CU give; without a norm,
+    the product in 64 bits within test_gemv_q4_row_groups' bound and the rounding of the bf16 result."""
+    from phi_3_vision_mlx_amd.weights import mlx_dequantize, mlx_quantize, q4_repack
+    packed, sc, bi = mlx_quantize(g((N, K), 415, 0.03))
+    w4, sb = (t.cuda() for t in q4_repack(packed, sc, bi))
+    x, nw = g((1, K), 416).cuda(), (g((K,), 417) * 0.1 + 1).cuda() if norm else None
+    got = ops.gemv_q4(x, w4, sb, norm_w=nw, norm_eps=1e-5)
+    request.addfinalizer(lambda old=ops.set_tuning("gemv_q4_wpc", 0): ops.set_tuning("gemv_q4_wpc", old))
+    for waves in (8, 16, 3):
+        ops.set_tuning("gemv_q4_wpc", waves)
+        assert torch.equal(ops.gemv_q4(x, w4, sb, norm_w=nw, norm_eps=1e-5), got), waves
+    if not norm:
+        wd = mlx_dequantize(packed, sc, bi).cuda()
+        y = x.double() @ wd.double().t()
+        tol = 2.0 ** -15 * wd.abs().max() * x.double().abs().sum() + 2.0 ** -8 * y.abs()
+        assert bool(((got.double() - y).abs() <= tol).all()), ((got.double() - y).abs() / tol).max()
+
+
 @pytest.mark.parametrize("M", [2, 5, 8, 15, 16])
 @pytest.mark.parametrize("N,K,epi", [(9216, 3072, "none"), (3072, 3072, "resid"), (8192, 3072, "silu"), (3072, 8192, "resid"), (32064, 3072, "none")])
 def test_gemv_q4_rows_2_to_16(ops, N, K, epi, M):
